@@ -1,0 +1,100 @@
+"""Product kernels at the sizes where they can go wrong -- tile edges, remainders, the shortest loops -- against float64."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import ug_amd
+from gpu_calls import BF16, GLU, NONE, SWIGLU, Gpu, Product, close, get, p, rand, view
+from test_gpu_parity import _raw_matmul
+from ug_amd import rng
+
+pytestmark = pytest.mark.gpu
+
+RING = {"10": "256x128", "6": "128x128", "7": "64x128", "9": "64x64"}  # GEMM_SHAPE -> tile
+
+
+def rounded(dtype, v):
+    return rng.bf16_round(v) if dtype == "bf16" else v.astype(np.float16).astype(np.float32)
+
+
+# 4 .. 9 K tiles: the ring's first and last rounds alone, then odd and even counts of steady ones
+@pytest.mark.parametrize("bmnk", [(1, 300, 264, 256), (2, 257, 136, 320), (3, 9, 8, 384), (1, 63, 392, 448), (1, 128, 128, 512), (1, 65, 1000, 576)])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
+def test_ring_tiles(hip, tune, bmnk, dtype, rhs_nk):
+    """Every tile of the ring on rows and columns that hang over it: the bound of an f32 sum rounded once, and small integers exactly."""
+    b, m, n, k = bmnk
+    dt = ug_amd.BF16 if dtype == "bf16" else ug_amd.F16
+    a, w = rounded(dtype, rng.uniform_pm1(1, b * m * k)).reshape(b, m, k), rounded(dtype, rng.uniform_pm1(2, b * k * n)).reshape(b, k, n)
+    exact = np.matmul(a.astype(np.float64), w.astype(np.float64))
+    bound = (2.0 ** -8 if dtype == "bf16" else 2.0 ** -11) * np.abs(exact) + k * np.finfo(np.float32).eps * np.matmul(np.abs(a).astype(np.float64), np.abs(w).astype(np.float64))
+    ai, wi = np.floor(a * 4), np.floor(w * 4)
+    whole = rounded(dtype, np.matmul(ai, wi).ravel()).reshape(exact.shape)  # (sums below 2^24)
+    for shape, tile in RING.items():
+        if shape == "9" and not rhs_nk:
+            continue  # the transposing reads want 128 columns
+        tune.setenv("UGHIP_GEMM_SHAPE", shape)
+        print("ring", dtype, bmnk, "NT" if rhs_nk else "NN", tile, flush=True)
+        got = _raw_matmul(hip, dt, a, w, rhs_nk)
+        assert ug_amd.last_kernel() == f"gemm_dma4<{dtype},{'NT' if rhs_nk else 'NN'},{tile},512t,ring>"
+        assert np.all(np.abs(got - exact) <= bound * 1.001 + 1e-7)
+        np.testing.assert_array_equal(_raw_matmul(hip, dt, ai, wi, rhs_nk), whole)
+
+
+@pytest.mark.parametrize("m, n, k, groups", [(17, 72, 256, 0), (70, 136, 320, 0), (300, 264, 384, 0), (301, 40, 448, 5), (40, 136, 576, 3)])
+@pytest.mark.parametrize("act", [NONE, SWIGLU, GLU])
+def test_ring_rows(hip, tune, m, n, k, groups, act):
+    """Products of rows on every tile of the ring: bias, gated units, rows gathered and sorted by matrix (one matrix without any)."""
+    gpu, rows, mats = Gpu(hip), n if act == NONE else 2 * n, max(1, groups)
+    x, w, bias = rand(1, m, k), rand(2, mats, rows, k, std=k ** -0.5), rand(3, rows, std=0.5)
+    if groups:
+        gen = np.random.default_rng(4)
+        end = np.sort(gen.integers(0, m + 1, groups)).astype(np.int32)
+        end[0], end[-1] = 0, m
+        src, bias = gen.integers(0, m, m).astype(np.int32), 0 * bias
+        of = np.searchsorted(end, np.arange(m), side="right")
+        y = np.stack([w[of[i]] @ x[src[i]] for i in range(m)])
+    else:
+        y = x @ w[0].T + bias
+    if act != NONE:
+        limit, alpha, shift = (1.5, 1.702, 1.0) if act == GLU else (1e9, 1.0, 0.0)
+        g, u = np.minimum(y[:, :n], limit), np.clip(y[:, n:], -limit, limit)
+        y = g / (1 + np.exp(-alpha * g)) * (u + shift)
+    dx, dw, db = gpu.up(x, bf16=True), gpu.up(w, bf16=True), gpu.up(bias)
+    idx = (gpu.up(src), gpu.up(end)) if groups else (None, None)
+    for shape, tile in RING.items():
+        tune.setenv("UGHIP_GEMM_SHAPE", shape)
+        dst = gpu.out(m * n + 8)
+        q = Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), bias=None if groups else db.raw(), m=m, n=n, k=k, product=BF16, act=act, row_index=idx[0].raw() if groups else None,
+                    group_end=idx[1].raw() if groups else None, groups=groups, x_rows=m if groups else 0, act_alpha=1.702 if act == GLU else 0, act_shift=1.0 if act == GLU else 0,
+                    act_limit=1.5 if act == GLU else 0)
+        print("ring rows", m, n, k, groups, act, tile, flush=True)
+        gpu.call("ughip_product_rows", C.byref(q))
+        assert f"{tile},512t,ring,rows" in ug_amd.last_kernel()
+        out = get(dst, m * n + 8)
+        assert np.all(np.isnan(out[m * n :])), "wrote past the end"
+        close(out[: m * n].reshape(m, n), y, 2e-5)
+
+
+@pytest.mark.parametrize("m, n, k", [(385, 264, 256), (400, 136, 448)])
+def test_ring_planes(hip, tune, m, n, k):
+    """Three bf16 terms on the ring's tiles, with a K split where it divides: the bound of an f32 sum."""
+    gpu, Z = Gpu(hip), C.c_size_t
+    x, w, r = rng.normal(1, m * k).reshape(m, k), rand(2, n, k, std=k ** -0.5), rng.normal(3, m * n).reshape(m, n)
+    want = x.astype(np.float64) @ w.T + r
+    bound = k * np.finfo(np.float32).eps * (np.abs(x).astype(np.float64) @ np.abs(w).T) + 4 * np.finfo(np.float32).eps * np.abs(want) + 1e-7
+    dx, dw, dr = gpu.up(x), gpu.up(w, bf16=True), gpu.up(r)
+    for shape, tile in RING.items():
+        if shape == "10":
+            continue  # not a tile of this product
+        for split in ("1", "2"):
+            if split == "2" and (k // 64) % 2:
+                continue
+            tune.setenv("UGHIP_X3_DMA", shape)
+            tune.setenv("UGHIP_X3_SPLIT", split)
+            dst = gpu.out(m * n)
+            print("ring planes", m, n, k, tile, split, flush=True)
+            gpu.call("ughip_linear_add_rows", p(dx), p(dw), p(dr), p(dst), Z(m), Z(n), Z(k), 1)
+            assert f"{tile},512t,ring,3 planes" in ug_amd.last_kernel()
+            assert np.all(np.abs(get(dst, (m, n)) - want) <= bound)

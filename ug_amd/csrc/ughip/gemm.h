@@ -45,7 +45,8 @@ double gemm_tiled_cost_us(int dtype, const MMArgs& p, size_t batch);
 
 // 16-bit types, one wave per SIMD: 256 x 256, 256 x 128 or 128 x 128 tiles (tile codes 256, 128, 64), 4 waves laid out
 // 2 x 2 with the accumulators in the accumulation registers, loads that write LDS directly, rhs [n, k]- or [k, n]-major
-// (gemm_dma.hip).  Any M, N % 8 == 0, K % 64 == 0 and K >= 256, 16-byte aligned rows, contiguous [batch, M, N] result.
+// (gemm_dma.hip), and a ring of four or three stages under eight waves with 256 x 128, 128 x 128, 64 x 128 and 64 x 64 tiles (codes 129, 65, 48,
+// 32; gemm_ring.hip).  Any M, N % 8 == 0, K % 64 == 0 and K >= 256, 16-byte aligned rows, contiguous [batch, M, N] result.
 bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile);
 hipError_t gemm_dma_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, int tile);
 // The tile code this kernel should take the problem with, 0 when another kernel should.
@@ -58,8 +59,10 @@ hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile
 // f32 operands as three bf16 planes each (rows of 3 k elements, the planes of every 64 elements of k side by side; p.K = 6 k):
 // the product as six bf16 terms with an f32 result, on either rhs layout.
 bool gemm_dma_planes6_supported(const MMArgs& p, size_t batch, int tile);
+void gemm_dma_planes3_name(int tile, int nsplit, const char* tail, char* out, size_t out_len);
 void gemm_dma_planes6_name(const MMArgs& p, int tile, char* out, size_t out_len);
 hipError_t gemm_dma_launch_planes6(hipStream_t stream, const MMArgs& p, size_t batch, int tile);
+int gemm_dma_forced_tile(long long shape);  // (tuning aid) the tile code that a value of GEMM_SHAPE or X3_DMA names, 0: none
 bool gemm_dma_planes3_split_ok(const MMArgs& p, int nsplit);
 // c = fold of nsplit f32 slabs [m, n] in slab order, then the epilogue: NONE, ADD (+ residual[m, n]) or SWIGLU
 // (c[m, n / 2] = silu(sum[:, :n / 2]) * sum[:, n / 2:]); n % 8 == 0.

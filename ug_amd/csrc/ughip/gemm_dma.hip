@@ -29,39 +29,13 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "gemm.h"
+#include "gemm_dma.h"
 #include "internal.h"
 #include "ughip.h"
 
 namespace ughip {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ floatx4 mma16(__bf16, const u32x4& a, const u32x4& b, const floatx4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ floatx4 mma16(_Float16, const u32x4& a, const u32x4& b, const floatx4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-// s_waitcnt vmcnt(n) alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (((N >> 4) & 3) << 14) | (7 << 4) | (15 << 8));
-}
-__device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(0xc07f); }
-
-// Every lane's 16 bytes at base + voff go to LDS at lds_byte_addr + lane * 16.  The compiler does not see the load
-// (it would wait for all of them before any LDS read): the waits are explicit.
-__device__ __forceinline__ void dma16(const void* base, unsigned voff, unsigned lds_byte_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_byte_addr), "v"(voff), "s"(base) : "memory", "m0");
-}
 // The same in two halves with an MFMA between them as the wait state that the write of M0 needs.  The first half names M0
 // as clobbered; nothing can tell the compiler that the second half reads it, so nothing it emits between the two may
 // write M0.  This kernel has no instruction that would (no LDS instruction of gfx950 needs M0); the build is held to that
@@ -72,21 +46,6 @@ __device__ __forceinline__ void dma16_m0(unsigned lds_byte_addr, unsigned stage_
   asm volatile("s_add_u32 m0, %0, %1" : : "s"(lds_byte_addr), "s"(stage_offset) : "memory", "scc", "m0");
 }
 __device__ __forceinline__ void dma16_go(const void* base, unsigned voff) { asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base) : "memory"); }
-
-constexpr int BK = 64;
-
-// k-contiguous operand tile ([rows][64] 16-bit): 128-byte rows of 8 chunks, chunk' = chunk ^ ((row / 2) & 7)
-__device__ __forceinline__ int kc_idx(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }  // in 16-byte units
-
-// n-contiguous rhs tile ([64 k][BN n] 16-bit): rows of BN / 16 pieces of 32 bytes, piece' = piece ^ h(k) with
-// h(k) = (k & 3) | ((k >> 3) & 1) << 2.  A transposing read names, per half wave, 8 rows (k = 8 g + e: e = 0..3 and two values
-// of g) and 32 bytes of each; h sends those rows to 8 different pieces, i.e. to all 64 banks once.  (With 64-byte segments
-// swizzled by k & 7 the two g of a half wave met in the same banks: 4096^3 95.5 -> 94.2 us on one box.)
-__device__ __forceinline__ int kn_h(int k) { return (k & 3) | (((k >> 3) & 1) << 2); }
-template <int BN>
-__device__ __forceinline__ int kn_byte(int k, int n) {
-  return k * (BN * 2) + (((n >> 4) ^ kn_h(k)) << 5) + (n & 15) * 2;
-}
 
 // Lane l feeds row / column l % 16, k = 8 (l / 16) .. + 7 of a step of 32.  TWO: the schedule with two barriers per K tile.
 // F32OUT: the result leaves as f32 straight from the accumulators (+ residual when given) instead of as T through LDS.
@@ -205,27 +164,10 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
     }
   }
   const long long a_step = BK * 2, b_step = B_KN ? (long long)BK * ldb * 2 : BK * 2;
-  // which K tile of the lhs and of the rhs in memory the loop's K tile `tile` reads (scalar arithmetic)
-  auto a_tile = [&](int tile) -> int {
-    if constexpr (BDIV == 6) {
-      const int g = tile / 6, r = tile - 6 * g;
-      return 3 * g + ((0x010120 >> (4 * r)) & 3);  // planes 0, 2, 1, 0, 1, 0
-    } else {
-      return tile;
-    }
-  };
-  auto b_tile = [&](int tile) -> int {
-    if constexpr (BDIV == 6) {
-      const int g = tile / 6, r = tile - 6 * g;
-      return 3 * g + ((0x001102 >> (4 * r)) & 3);  // planes 2, 0, 1, 1, 0, 0
-    } else {
-      return tile / BDIV;
-    }
-  };
   auto dma = [&](int tile, int idx) {  // idx: compile-time after unrolling
     const unsigned st = lds_addr + (tile & 1) * STAGE_BYTES;
-    if (idx < NDA) dma16(Ab + a_tile(tile) * a_step, voff[idx], st + (idx * 4 + wave) * 1024);
-    else dma16(Bb + b_tile(tile) * b_step, voff[idx], st + A_BYTES + ((idx - NDA) * 4 + wave) * 1024);
+    if (idx < NDA) dma16(Ab + lhs_k_tile<BDIV>(tile) * a_step, voff[idx], st + (idx * 4 + wave) * 1024);
+    else dma16(Bb + rhs_k_tile<BDIV>(tile) * b_step, voff[idx], st + A_BYTES + ((idx - NDA) * 4 + wave) * 1024);
   };
   auto dma_m0 = [&](int tile, int idx) {
     const unsigned in_stage = lds_addr + (idx < NDA ? (idx * 4 + wave) * 1024 : A_BYTES + ((idx - NDA) * 4 + wave) * 1024);  // loop invariant
@@ -235,8 +177,8 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
     __builtin_amdgcn_sched_barrier(0);
   };
   auto dma_go = [&](int tile, int idx) {
-    if (idx < NDA) dma16_go(Ab + a_tile(tile) * a_step, voff[idx]);
-    else dma16_go(Bb + b_tile(tile) * b_step, voff[idx]);
+    if (idx < NDA) dma16_go(Ab + lhs_k_tile<BDIV>(tile) * a_step, voff[idx]);
+    else dma16_go(Bb + rhs_k_tile<BDIV>(tile) * b_step, voff[idx]);
   };
 
   floatx4 acc[NI][NJ];
@@ -509,15 +451,34 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 }  // namespace
 
 namespace {
-// tile codes of the entry points below: 256 = 256 x 256, 128 = 256 x 128, 64 = 128 x 128
+// tile codes of the entry points below: 256 = 256 x 256, 128 = 256 x 128, 64 = 128 x 128; on gemm_ring 129 = 256 x 128, 65 = 128 x 128, 48 = 64 x 128,
+// 32 = 64 x 64 ([n, k]-major rhs only)
 bool tile_dims(int tile, int* bm, int* bn) {
   if (tile == 256) *bm = 256, *bn = 256;
-  else if (tile == 128) *bm = 256, *bn = 128;
-  else if (tile == 64) *bm = 128, *bn = 128;
+  else if (tile == 128 || tile == 129) *bm = 256, *bn = 128;
+  else if (tile == 64 || tile == 65) *bm = 128, *bn = 128;
+  else if (tile == 48) *bm = 64, *bn = 128;
+  else if (tile == 32) *bm = 64, *bn = 64;
   else return false;
   return true;
 }
 }  // namespace
+
+static bool ring_tile(int tile) { return tile == 129 || tile == 65 || tile == 48 || tile == 32; }
+static const char* waves_name(int tile) { return ring_tile(tile) ? "512t,ring" : "256t"; }  // in the names of these kernels
+// (tuning aid) the tile code that GEMM_SHAPE names, 0: none
+int gemm_dma_forced_tile(long long shape) {
+  switch (shape) {
+    case 3: return 256;
+    case 4: return 128;
+    case 5: return 64;
+    case 6: return 65;
+    case 7: return 48;
+    case 9: return 32;
+    case 10: return 129;
+  }
+  return 0;
+}
 
 bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
   if (dtype != UGHIP_BF16 && dtype != UGHIP_F16) return false;
@@ -526,13 +487,27 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < 4 * BK || batch == 0) return false;
   if (p.a_cs != 1 || p.a_rs % 8 || (batch > 1 && (p.a_bs % 8 || p.b_bs % 8 || p.c_bs % 8))) return false;
   const bool nn = p.b_cs == 1 && p.b_rs != 1, nt = p.b_rs == 1 && p.b_cs != 1;
-  if (nn == nt) return false;
+  if (nn == nt || (nn && tile == 32)) return false;
   const long long ldb = nn ? p.b_rs : p.b_cs;
   if (ldb % 8) return false;
   // per-lane offsets are 32-bit: the furthest row of a tile has to stay below 4 GiB from the tile's first byte
   if ((unsigned long long)p.a_rs * 2 * bm >= (1ull << 32) || (unsigned long long)ldb * 2 * (nn ? BK : bn) >= (1ull << 32)) return false;
   if (!aligned16(p.a) || !aligned16(p.b) || !aligned16(p.c)) return false;
   return batch * (size_t)((p.M + bm - 1) / bm) * (size_t)((p.N + bn - 1) / bn) < (1u << 24);
+}
+
+// What `tiles` tiles of the ring kernel take: a fixed part and, per round of 256 tiles, the K tiles.  The time of a K tile is that of its bytes
+// on their way to a CU, some 100 bytes per ns from the memory-side cache and 60 from HBM however many are asked for at once (with the MFMAs or the
+// LDS reads taken out the kernel takes as long), so it goes by where the operands come from: `streamed` is a matrix nobody has read
+// lately, as the weights of a model's next layer are.  Fitted to (m x n x k, us): 2048^2 x 5632 streamed 51 (128 x 128) / 67 (256 x 128), 1024 x 2048 x
+// 5632 streamed 38 (64 x 128), 509 x 2048 x 5632 streamed 26 (64 x 64), 2048 x 11264 x 2048 streamed 89 (256 x 128); 2048^3 19.2 (128 x 128),
+// 1024 x 2048 x 4096 21.1 (64 x 128), 256 x 4096^2 14.7 (64 x 64).
+static double ring_cost_us(size_t tiles, int kt, int tile, bool streamed) {
+  const double t0 = tile == 129 ? 0.64 : tile == 65 ? (streamed ? 0.54 : 0.30) : tile == 48 ? (streamed ? 0.40 : 0.21) : streamed ? 0.255 : 0.11;
+  const double t1 = tile == 129 ? 0.22 : streamed ? 0 : tile == 65 ? 0.17 : tile == 48 ? 0.07 : 0.075;
+  double us = tile == 129 ? 5.0 : tile == 65 ? 4.0 : 3.3;
+  for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (t0 + t1 * (left < 256 ? (double)left : 256.0) / 256.0);
+  return us;
 }
 
 // Which tile this kernel should take the problem with (a tile code), or 0 when the register-staged kernel is expected to
@@ -546,13 +521,14 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
 // (3072 x 4096^2: 131 -> 91 us, 5120^2 x 1024: 77 -> 54, 1280 x 8192 x 2048: 64 -> 47, 2048 x 2560 x 2048: 35 -> 29,
 // 2304^3: 39 -> 35) and leaves those with about 128 tiles where they were (2048^2 x 5632: 56 us against 72).  The
 // 128 x 128 tile (two workgroups per CU) takes what neither fits: 2304^3 35 -> 31 us, 2048 x 2560 x 2048 29 -> 27.
-// UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 0..2 keeps it out (tuning aid).
+// UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 10 / 6 / 7 / 9 the ring's tiles, 0..2 keeps both out (tuning aid).
 double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
   int bm, bn;
   if (!tile_dims(tile, &bm, &bn)) return 1e30;
   const size_t tiles = batch * (size_t)((p.M + bm - 1) / bm) * (size_t)((p.N + bn - 1) / bn);
   const int kt = p.K / BK;
   const bool nn = p.b_cs == 1 && p.b_rs != 1;
+  if (ring_tile(tile)) return ring_cost_us(tiles, kt, tile, false) * (nn ? 1.08 : 1.0) + (double)batch * p.M * p.N * 2 / 6.4e6;
   double us = 4.0 + (double)batch * p.M * p.N * 2 / 6.4e6;
   // (the figures below were fitted to the kernel on 32 x 32 x 16 MFMAs; on 16 x 16 x 32 and with the loads spread behind two
   // barriers every K tile takes 8 % less: 4096^3 97 us, 8 x 1024^3 18.8, 1024 x 4096^2 41 on 128 x 128 tiles)
@@ -576,17 +552,28 @@ double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
 
 int gemm_dma_pick(int dtype, const MMArgs& p, size_t batch) {
   if (long long s; tune_get(TUNE_GEMM_SHAPE, &s)) {
-    const int forced = s == 3 ? 256 : s == 4 ? 128 : s == 5 ? 64 : 0;
+    const int forced = gemm_dma_forced_tile(s);
     return forced && gemm_dma_supported(dtype, p, batch, forced) ? forced : 0;
   }
   int best = 0;
   double best_us = 0;
-  for (int tile : {256, 128, 64}) {
-    if (!gemm_dma_supported(dtype, p, batch, tile)) continue;
+  // The ring where 128 x 128 tiles would leave CUs without one (us by box, best of gemm_dma4 and gemm_tiled -> ring: 1024^3 [k, n]-major
+  // 11.4 -> 7.9, 2048 x 1024^2 10.8 -> 8.2, 1024 x 2048 x 4096 28.7 -> 21.1 and 37.3 -> 24.5, 1536^3 16.2 -> 13.1, 96^2 x 4096 [k, n]-major 33 -> 15.4).  From
+  // there on 2304^3 says 31.0 against 37.1.  An [n, k]-major rhs under a handful of tiles with a short K stays with gemm_tiled and its K split:
+  // the callers that count on that kernel there (the tests among them) keep it, and so do up to 128 rows whose K it splits over workgroups (at 64 x
+  // 2048 x 2048 it takes 11.6 us against 7.7, with N = 256 it is the faster one).
+  const size_t tiles = batch * (size_t)((p.M + 127) / 128) * (size_t)((p.N + 127) / 128);
+  const bool few = tiles < 256 && !(p.b_rs == 1 && tiles <= 64 && p.K <= 1024) && !(p.M <= 128 && gemm_tiled_workspace_bytes(dtype, p, batch) != 0);
+  for (int tile : {256, 128, 64, 65, 48, 32}) {
+    if ((ring_tile(tile) && !few) || !gemm_dma_supported(dtype, p, batch, tile)) continue;
     const double us = gemm_dma_cost_us(p, batch, tile);
     if (!best || us < best_us * 0.97) best = tile, best_us = us;  // the larger tile on a near tie: fewer operand bytes
   }
   if (!best) return 0;
+  if (ring_tile(best)) {
+    const double tiled = gemm_tiled_cost_us(dtype, p, batch);  // (its model is 0-20 % below what [k, n]-major products take)
+    return tiled < 0 || best_us < tiled ? best : 0;
+  }
   // the 128 x 128 tile runs at the register-staged kernel's pace (both are bound by their LDS reads): it has to be
   // clearly cheaper to take the product from it
   const double other = gemm_tiled_cost_us(dtype, p, batch);
@@ -597,7 +584,7 @@ void gemm_dma_name(int dtype, const MMArgs& p, int tile, char* out, size_t out_l
   int bm = 0, bn = 0;
   tile_dims(tile, &bm, &bn);
   const bool nn = p.b_cs == 1 && p.b_rs != 1;
-  snprintf(out, out_len, "gemm_dma4<%s,%s,%dx%d,256t>", dtype == UGHIP_F16 ? "f16" : "bf16", nn ? "NN" : "NT", bm, bn);
+  snprintf(out, out_len, "gemm_dma4<%s,%s,%dx%d,%s>", dtype == UGHIP_F16 ? "f16" : "bf16", nn ? "NN" : "NT", bm, bn, waves_name(tile));
 }
 
 hipError_t gemm_dma_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, int tile) {
@@ -610,6 +597,7 @@ hipError_t gemm_dma_launch(hipStream_t stream, int dtype, const MMArgs& p, size_
     gemm_dma_name(dtype, p, tile, name, sizeof name);
     note_kernel("%s", name);
   }
+  if (ring_tile(tile)) return gemm_ring_launch(stream, dtype, DmaForm::PLAIN, p, batch, tile, nullptr, DmaRows());
 #define UGHIP_DMA_CASE(T)                                                                                                  \
   if (tile == 256) return nn ? launch<T, 256, 256, true>(stream, p, batch) : launch<T, 256, 256, false>(stream, p, batch); \
   if (tile == 128) return nn ? launch<T, 256, 128, true>(stream, p, batch) : launch<T, 256, 128, false>(stream, p, batch); \
@@ -630,6 +618,14 @@ bool gemm_dma_planes3_split_ok(const MMArgs& p, int nsplit) {
   return kts % 3 == 0 && kts >= 4;
 }
 
+void gemm_dma_planes3_name(int tile, int nsplit, const char* tail, char* out, size_t out_len) {
+  int bm = 0, bn = 0;
+  tile_dims(tile, &bm, &bn);
+  char split[24] = "";
+  if (nsplit > 1) snprintf(split, sizeof split, ",splitK=%d", nsplit);
+  snprintf(out, out_len, "gemm_dma4<bf16,NT,%dx%d,%s,3 planes%s,f32 out%s>", bm, bn, waves_name(tile), split, tail ? tail : "");
+}
+
 hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile, int nsplit, const float* residual, const char* note_tail) {
   if (p.b_k_div != 3 || !(p.b_rs == 1 && p.b_cs != 1) || !gemm_dma_planes3_split_ok(p, nsplit) || (nsplit > 1 && residual)) return hipErrorInvalidValue;
   MMArgs q = p;
@@ -639,11 +635,10 @@ hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile
   }
   if (!gemm_dma_supported(UGHIP_BF16, q, (size_t)nsplit, tile)) return hipErrorInvalidValue;
   if (residual && !aligned16(residual)) return hipErrorInvalidValue;
-  int bm = 0, bn = 0;
-  tile_dims(tile, &bm, &bn);
-  char split[24] = "";
-  if (nsplit > 1) snprintf(split, sizeof split, ",splitK=%d", nsplit);
-  note_kernel("gemm_dma4<bf16,NT,%dx%d,256t,3 planes%s,f32 out%s>", bm, bn, split, note_tail ? note_tail : "");
+  char name[160];
+  gemm_dma_planes3_name(tile, nsplit, note_tail, name, sizeof name);
+  note_kernel("%s", name);
+  if (ring_tile(tile)) return gemm_ring_launch(stream, UGHIP_BF16, DmaForm::PLANES3, q, (size_t)nsplit, tile, residual, DmaRows());
   if (tile == 256) return launch<__bf16, 256, 256, false, true, 3>(stream, q, (size_t)nsplit, residual);
   if (tile == 128) return launch<__bf16, 256, 128, false, true, 3>(stream, q, (size_t)nsplit, residual);
   return launch<__bf16, 128, 128, false, true, 3>(stream, q, (size_t)nsplit, residual);
@@ -652,7 +647,7 @@ hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile
 
 bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, bool swiglu, int tile) {
   int bm, bn;
-  if (!tile_dims(tile, &bm, &bn)) return false;
+  if (!tile_dims(tile, &bm, &bn) || (tile != 256 && !ring_tile(tile))) return false;
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < 4 * BK || p.a_cs != 1 || p.a_rs % 8 || p.b_rs != 1 || p.b_cs % 8) return false;
   if (r.n_out <= 0 || r.n_out % 4 || p.N != (swiglu ? 2 * r.n_out : r.n_out) || r.dst_stride % 4 || r.w_group % 8) return false;
   // per-lane offsets are 32-bit: rows of x anywhere, matrix rows of a tile (of the whole matrix with SwiGLU)
@@ -664,31 +659,40 @@ bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, bool swiglu, int
 
 int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, bool swiglu) {
   if (long long s; tune_get(TUNE_GEMM_SHAPE, &s)) {  // tuning aid, as for gemm_dma_pick
-    const int forced = s == 3 ? 256 : s == 4 ? 128 : s == 5 ? 64 : 0;
+    const int forced = gemm_dma_forced_tile(s);
     return forced && gemm_dma_rows_supported(p, r, swiglu, forced) ? forced : 0;
   }
-  // Measured on bf16 rows with K around 2048 (products of a prompt of 2048 positions, dense and by expert): the largest tile
-  // wherever it numbers most of the chip (47 GFLOP over 16 experts 116 us against 139-152), the smallest elsewhere (2048 x 2048 x
-  // 4096: 32 us against 37 and 51); the middle one was never the fastest.
-  const size_t groups = r.groups ? r.groups : 1, m = (p.M + groups - 1) / groups;  // rows as if they were spread evenly
-  const size_t tiles = groups * ((m + 255) / 256) * ((p.N + 255) / 256);
-  if (tiles >= 200 && m > 128 && gemm_dma_rows_supported(p, r, swiglu, 256)) return 256;
-  return gemm_dma_rows_supported(p, r, swiglu, 64) ? 64 : 0;
+  // A model's products: the matrix comes from memory.  256 x 256 tiles of gemm_dma4 and the ring's, by what they are expected to take
+  // (2048 positions: down 74 -> 51 us, gate and up 105 -> 89, output 26 -> 18, attention's input 37 -> 29; 509 positions: state-space output
+  // 53 -> 19, input 43 -> 32, dense gate and up 40 -> 30; 16 experts' gate and up 83 -> 62, down 38 -> 33; 33 rows of 11264 x 2048 31 -> 13).
+  const size_t groups = r.groups ? r.groups : 1;
+  const double m = (double)p.M / groups;  // rows as if they were spread evenly
+  int best = 0;
+  double best_us = 0;
+  for (int tile : {256, 129, 65, 48, 32}) {
+    if (!gemm_dma_rows_supported(p, r, swiglu, tile)) continue;
+    int bm, bn;
+    tile_dims(tile, &bm, &bn);
+    // tile rows: of groups near or above a tile's height every second one takes one more
+    const double rows = groups == 1 ? (p.M + bm - 1) / bm : m < 0.8 * bm ? groups : groups * (m / bm + 0.5);
+    const size_t tiles = (size_t)(rows + 0.5) * ((p.N + bn - 1) / bn);
+    const int kt = p.K / BK;
+    double us = 6.0;
+    if (tile == 256)
+      for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (1.23 + 0.33 * (left < 256 ? (double)left : 256.0) / 256.0);
+    else us = ring_cost_us(tiles, kt, tile, true);
+    if (!best || us < best_us * 0.97) best = tile, best_us = us;  // the larger tile on a near tie
+  }
+  return best;
 }
 
 hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRows& r, bool swiglu, int tile) {
   if (!gemm_dma_rows_supported(p, r, swiglu, tile)) return hipErrorInvalidValue;
   int bm = 0, bn = 0;
   tile_dims(tile, &bm, &bn);
-  note_kernel("gemm_dma4<bf16,NT,%dx%d,256t,rows%s%s>", bm, bn, swiglu ? ",swiglu" : "", r.groups ? ",grouped" : "");
-  if (swiglu) {
-    if (tile == 256) return launch<__bf16, 256, 256, false, false, 1, 2>(stream, p, 1, nullptr, r);
-    if (tile == 128) return launch<__bf16, 256, 128, false, false, 1, 2>(stream, p, 1, nullptr, r);
-    return launch<__bf16, 128, 128, false, false, 1, 2>(stream, p, 1, nullptr, r);
-  }
-  if (tile == 256) return launch<__bf16, 256, 256, false, false, 1, 1>(stream, p, 1, nullptr, r);
-  if (tile == 128) return launch<__bf16, 256, 128, false, false, 1, 1>(stream, p, 1, nullptr, r);
-  return launch<__bf16, 128, 128, false, false, 1, 1>(stream, p, 1, nullptr, r);
+  note_kernel("gemm_dma4<bf16,NT,%dx%d,%s,rows%s%s>", bm, bn, waves_name(tile), swiglu ? ",swiglu" : "", r.groups ? ",grouped" : "");
+  if (ring_tile(tile)) return gemm_ring_launch(stream, UGHIP_BF16, swiglu ? DmaForm::ROWS_GLU : DmaForm::ROWS, p, 1, tile, nullptr, r);
+  return swiglu ? launch<__bf16, 256, 256, false, false, 1, 2>(stream, p, 1, nullptr, r) : launch<__bf16, 256, 256, false, false, 1, 1>(stream, p, 1, nullptr, r);
 }
 
 // Both operands as three bf16 planes per 64 elements of k (p.K = 6 k, rows of 3 k elements), f32 result: see BDIV == 6.

@@ -1,0 +1,334 @@
+// 16-bit MFMA GEMM for products that leave the chip idle or waiting on gemm_dma4's tiles: C = A x B, f32 accumulate, K tile 64.
+//
+//   Eight waves, 4 x 2, each BM / 4 x BN / 2 of the result in 16 x 16 accumulators (v_mfma_f32_16x16x32): a wave's waits are filled by the other
+//   one of its SIMD.  The k order of every sum is that of gemm_dma4 and gemm_tiled, so the results are theirs bit for bit.
+//   A ring of four stages (three for 256 x 128): the loads of a K tile go out (global_load_lds_dwordx4, as in gemm_dma4) when the tile that
+//   many in front of it has been read, so three (two) tiles are on their way while one is multiplied.  One barrier per K tile.
+//
+// What bounds it: the operands' way to a CU.  2048^2 x 5632 on 128 x 128 tiles, one to a CU, takes 0.51 us per K tile of 32 KB with the operands in
+// the memory-side cache and 0.55 with the matrix from HBM (gemm_dma4's two stages: 0.85); the same kernel without its MFMAs takes 0.38 / 0.54,
+// without its loads 0.35-0.39, and a loop of nothing but the loads 0.33 / 0.52: a CU gets some 100 / 60 bytes per ns however many loads it has
+// on their way (deeper rings, loads that bypass the cache and a wave that touches the lines for L2 ahead of the others made nothing faster).
+// So tiles are as large as leaves every CU one, by the model in gemm_dma.hip.
+#include <hip/hip_runtime.h>
+
+#include <atomic>
+#include <type_traits>
+
+#include "gemm_dma.h"
+#include "internal.h"
+#include "ughip.h"
+
+namespace ughip {
+namespace {
+
+constexpr int stages(int bm) { return bm == 256 ? 3 : 4; }
+
+// Template parameters and DmaRows as in gemm_dma4.
+template <typename T, int BM, int BN, bool B_KN, bool F32OUT, int BDIV, int ROWS>
+__global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tiles_m, int tiles_n, const float* __restrict__ residual, DmaRows rw) {
+  static_assert(ROWS == 0 || (BDIV == 1 && !B_KN && !F32OUT), "rows: one plane against an [n, k]-major rhs");
+  static_assert(BDIV == 1 || !B_KN, "planes of the lhs: against an [n, k]-major rhs only");
+  static_assert(!B_KN || BN >= 128, "the swizzle of an n-contiguous tile wants eight 32-byte pieces per row");
+  extern __shared__ u32x4 lds[];
+  constexpr int S = stages(BM);
+  constexpr int NI = BM / 64, NJ = BN / 32, NM = NI * NJ;  // 16-row and 16-column fragments and MFMAs of a wave and step of 32 k
+  constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, STAGE_BYTES = A_BYTES + B_BYTES;
+  constexpr int NDA = BM / 64, NDB = BN / 64, ND = NDA + NDB;   // loads per wave and K tile
+  constexpr int R = NI + NJ;                                      // fragment reads per step
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // XCD-aware order of the tiles: as in gemm_dma4 (the grid is 8 more at least, the runs are of equal length)
+  int tiles = batches * tiles_m * tiles_n;
+  if (ROWS != 0 && rw.groups) {
+    int rows = 0, begin = 0;
+    for (int g = 0; g < rw.groups; ++g) {
+      int end = rw.group_end[g];
+      end = end < begin ? begin : end > p.M ? p.M : end;
+      rows += (end - begin + BM - 1) / BM;
+      begin = end;
+    }
+    tiles_m = rows;
+    tiles = rows * tiles_n;
+  }
+  const int per = (tiles + 7) >> 3;
+  if ((int)blockIdx.x >= 8 * per) return;
+  const int bid = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  if (bid >= tiles) return;
+  const int tpb = tiles_m * tiles_n;
+  const int batch = bid / tpb;
+  const int t_in = bid - batch * tpb;
+  int tm, tn;
+  if ((tiles_m & 3) == 0) {
+    const int sr = t_in / (4 * tiles_n), rem = t_in - sr * 4 * tiles_n;
+    tm = sr * 4 + (rem & 3);
+    tn = rem >> 2;
+  } else {
+    tm = t_in / tiles_n;
+    tn = t_in - tm * tiles_n;
+  }
+  int m0 = tm * BM, m_end = p.M, group = 0;
+  const int n0 = tn * BN;
+  if (ROWS != 0 && rw.groups) {
+    int t = tm, begin = 0;
+    bool found = false;
+    for (int g = 0; g < rw.groups && !found; ++g) {
+      int end = rw.group_end[g];
+      end = end < begin ? begin : end > p.M ? p.M : end;
+      const int tiles = (end - begin + BM - 1) / BM;
+      if (t < tiles) group = g, m0 = begin + t * BM, m_end = end, found = true;
+      else t -= tiles, begin = end;
+    }
+    if (!found) return;  // the same for the whole workgroup
+  }
+  const long long lda = p.a_rs, ldb = B_KN ? p.b_rs : p.b_cs;
+  const char* Ab = reinterpret_cast<const char*>(static_cast<const T*>(p.a) + (size_t)batch * p.a_bs + (ROWS ? 0 : (size_t)m0 * lda));
+  const char* Bb = reinterpret_cast<const char*>(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs + (ROWS ? (size_t)group * rw.w_group : 0) +
+                                                 (ROWS == 2 ? 0 : B_KN ? (size_t)n0 : (size_t)n0 * ldb));
+  const int KT = p.K / BK;
+  const int wm = (wave >> 1) * (BM / 4), wn = (wave & 1) * (BN / 2);
+  const unsigned lds_addr = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds;
+  // per-lane byte offsets of this wave's loads; rows past the end fetch the last row again (their results are not stored)
+  unsigned voff[ND];
+  const int m_last = m_end - 1 - m0, n_left = p.N - n0;
+#pragma unroll
+  for (int i = 0; i < NDA; ++i) {
+    const int row = (i * 8 + wave) * 8 + (lane >> 3), cp = lane & 7;
+    int src = min(row, m_last);
+    if constexpr (ROWS != 0) {
+      src += m0;
+      if (rw.row_index) src = max(0, min(rw.row_index[src], rw.x_rows - 1));
+    }
+    voff[i] = (unsigned)(src * lda * 2 + ((cp ^ ((row >> 1) & 7)) << 4));
+  }
+#pragma unroll
+  for (int i = 0; i < NDB; ++i) {
+    const int g = i * 8 + wave;
+    if (!B_KN) {
+      const int row = g * 8 + (lane >> 3), cp = lane & 7;
+      int src = min(row, n_left - 1);
+      if constexpr (ROWS == 2) {  // a wave's half of the tile: BN / 4 gate columns, then the same columns of up
+        const int q = row % (BN / 2);
+        src = min(tn * (BN / 2) + row / (BN / 2) * (BN / 4) + q % (BN / 4), rw.n_out - 1) + (q >= BN / 4 ? rw.n_out : 0);
+      }
+      voff[NDA + i] = (unsigned)(src * ldb * 2 + ((cp ^ ((row >> 1) & 7)) << 4));
+    } else {
+      constexpr int CPR = BN / 8;  // 16-byte chunks per row of k
+      const int k = g * (64 / CPR) + lane / CPR, cpos = lane % CPR;
+      const int src = (((cpos >> 1) ^ kn_h(k)) << 1) | (cpos & 1);
+      voff[NDA + i] = (unsigned)(k * ldb * 2 + (min(src, n_left / 8 - 1) << 4));  // N % 8 == 0: whole 16-byte chunks
+    }
+  }
+  const long long a_step = BK * 2, b_step = B_KN ? (long long)BK * ldb * 2 : BK * 2;
+  auto dma = [&](int tile, int idx) {  // idx: compile-time after unrolling
+    const unsigned st = lds_addr + (unsigned)tile % S * STAGE_BYTES;
+    if (idx < NDA) dma16(Ab + lhs_k_tile<BDIV>(tile) * a_step, voff[idx], st + (idx * 8 + wave) * 1024);
+    else dma16(Bb + rhs_k_tile<BDIV>(tile) * b_step, voff[idx], st + A_BYTES + ((idx - NDA) * 8 + wave) * 1024);
+  };
+
+  floatx4 acc[NI][NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  u32x4 fa[2][NI], fb[2][NJ];
+  auto read_frag = [&](int tile, int step, int idx, int set) {
+    const int stage = (unsigned)tile % S;
+    if (idx < NI) {
+      fa[set][idx] = lds[stage * (STAGE_BYTES / 16) + kc_idx(wm + idx * 16 + (lane & 15), 4 * step + (lane >> 4))];
+    } else if (!B_KN) {
+      fb[set][idx - NI] = lds[stage * (STAGE_BYTES / 16) + A_BYTES / 16 + kc_idx(wn + (idx - NI) * 16 + (lane & 15), 4 * step + (lane >> 4))];
+    } else {
+      typedef __attribute__((address_space(3))) s16x4 lds_v4;  // transposing reads: as in gemm_dma4
+      const int g = lane >> 4, li = lane & 15, q = li & 3, e = li >> 2;
+      const char __attribute__((address_space(3)))* Bs = (const char __attribute__((address_space(3)))*)lds + stage * STAGE_BYTES + A_BYTES;
+      const int n = wn + (idx - NI) * 16 + 4 * q, k0 = step * 32 + 8 * g + e;
+      const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(Bs + kn_byte<BN>(k0, n))));
+      const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(Bs + kn_byte<BN>(k0 + 4, n))));
+      fb[set][idx - NI] = u32x4{lo.x, lo.y, hi.x, hi.y};
+    }
+  };
+
+  // MFMAs of one step on register set X, the next step's reads (tile rt, step rs: into the other set) and the loads of tile dt dealt over them
+  auto step = [&](auto set, auto reads, int rt, int rs, auto loads, int dt) {
+    constexpr int X = decltype(set)::value;
+#pragma unroll
+    for (int g = 0; g < NM; ++g) {
+      if constexpr (decltype(reads)::value) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (r * NM / R == g) read_frag(rt, rs, r, X ^ 1);
+      }
+      if constexpr (decltype(loads)::value) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+          if (d * NM / ND == g) dma(dt, d);
+      }
+      acc[g / NJ][g % NJ] = mma16(T(), fb[X][g % NJ], fa[X][g / NJ], acc[g / NJ][g % NJ]);  // operands swapped: a lane gets 4 columns of a row
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+  using CS = std::integral_constant<int, S>;
+  using Y = std::true_type;
+  using N_ = std::false_type;
+  // Everybody has read the stage of tile kt, and tile kt + 1 has landed.  A: how many tiles follow kt (S stands for that many or more).
+  auto turn = [&](auto ahead) {
+    constexpr int A = decltype(ahead)::value;
+    if constexpr (A > 0) wait_vmcnt<((A < S ? A : S - 1) - 1) * ND>();
+    wait_lgkmcnt0();
+    __builtin_amdgcn_s_barrier();
+  };
+  // A K tile: the first step's fragments are in set 0, the turn comes between the steps, behind it the tile's stage takes the loads of the tile
+  // S further on.
+  auto body = [&](int kt, auto ahead) {
+    constexpr int A = decltype(ahead)::value;
+    step(C0(), Y(), kt, 1, N_(), 0);
+    turn(ahead);
+    step(C1(), std::bool_constant<(A > 0)>(), kt + 1, 0, std::bool_constant<A == S>(), kt + S);
+  };
+#pragma unroll
+  for (int t = 0; t < S; ++t)
+#pragma unroll
+    for (int d = 0; d < ND; ++d) dma(t, d);
+  wait_vmcnt<(S - 1) * ND>();
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int r = 0; r < R; ++r) read_frag(0, 0, r, 0);
+  const int full = KT - S;
+  for (int kt = 0; kt < full; ++kt) body(kt, CS());
+  if constexpr (S == 4) body(KT - 4, std::integral_constant<int, 3>());
+  body(KT - 3, std::integral_constant<int, 2>());
+  body(KT - 2, C1());
+  body(KT - 1, C0());
+
+  // Register e of lane l of block (i, j): row wm + 16 i + l % 16, column wn + 16 j + 4 (l / 16) + e.
+  if constexpr (ROWS != 0) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    constexpr int NC = ROWS == 2 ? NJ / 2 : NJ;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int col = ROWS == 2 ? tn * (BN / 2) + (wave & 1) * (BN / 4) + j * 16 + (lane >> 4) * 4 : n0 + wn + j * 16 + (lane >> 4) * 4;
+      if (col >= rw.n_out) continue;  // n_out % 4 == 0: a group of 4 columns exists whole or not at all
+      floatx4 b = {0.f, 0.f, 0.f, 0.f}, bu = {0.f, 0.f, 0.f, 0.f};
+      if (rw.bias) {
+        b = *reinterpret_cast<const floatx4*>(rw.bias + col);
+        if (ROWS == 2) bu = *reinterpret_cast<const floatx4*>(rw.bias + rw.n_out + col);
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int row = wm + i * 16 + (lane & 15);
+        if (row > m_last) continue;
+        floatx4 v = acc[i][j] + b;
+        if constexpr (ROWS == 2) {
+          floatx4 u = acc[i][j + NC] + bu;
+          if (rw.glu_limit > 0.f) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              v[e] = v[e] > rw.glu_limit ? rw.glu_limit : v[e];
+              u[e] = u[e] > rw.glu_limit ? rw.glu_limit : u[e] < -rw.glu_limit ? -rw.glu_limit : u[e];
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = v[e] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * rw.glu_alpha * v[e])) * (u[e] + rw.glu_shift);
+        }
+        const size_t at = (size_t)(m0 + row) * rw.dst_stride + col;
+        if (rw.dst_bf16) *reinterpret_cast<u32x2*>(static_cast<T*>(rw.dst) + at) = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
+        else *reinterpret_cast<floatx4*>(static_cast<float*>(rw.dst) + at) = v;
+      }
+    }
+    return;
+  }
+  if constexpr (F32OUT) {
+    float* __restrict__ C = static_cast<float*>(p.c) + (size_t)batch * p.c_bs + (size_t)m0 * p.N + n0;
+    const float* __restrict__ Rz = residual ? residual + (size_t)batch * p.c_bs + (size_t)m0 * p.N + n0 : nullptr;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int row = wm + i * 16 + (lane & 15), col = wn + j * 16 + (lane >> 4) * 4;
+        if (row <= m_last && col < n_left) {  // N % 8 == 0: a group of 4 columns exists whole or not at all
+          floatx4 v = acc[i][j];
+          if (Rz) v += *reinterpret_cast<const floatx4*>(Rz + (size_t)row * p.N + col);
+          *reinterpret_cast<floatx4*>(C + (size_t)row * p.N + col) = v;
+        }
+      }
+    return;
+  }
+  // 16-bit result through LDS, out in 16-byte pieces of whole rows past the cache.
+  constexpr int PITCH = BN * 2 + 8;
+  char __attribute__((address_space(3)))* Cs = (char __attribute__((address_space(3)))*)lds;
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      typedef T tx4 __attribute__((ext_vector_type(4)));
+      tx4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (T)acc[i][j][e];
+      const int row = wm + i * 16 + (lane & 15), col = wn + j * 16 + (lane >> 4) * 4;
+      *(u32x2 __attribute__((address_space(3)))*)(Cs + row * PITCH + col * 2) = __builtin_bit_cast(u32x2, v);
+    }
+  __syncthreads();
+  constexpr int CPR = BN / 8, RPP = 512 / CPR;
+  T* __restrict__ C = static_cast<T*>(p.c) + (size_t)batch * p.c_bs + (size_t)m0 * p.N + n0;
+  const int c = tid % CPR, r0 = tid / CPR;
+#pragma unroll
+  for (int pass = 0; pass < BM / RPP; ++pass) {
+    const int row = pass * RPP + r0;
+    const u32x2 lo = *(const u32x2 __attribute__((address_space(3)))*)(Cs + row * PITCH + c * 16);
+    const u32x2 hi = *(const u32x2 __attribute__((address_space(3)))*)(Cs + row * PITCH + c * 16 + 8);
+    if (row <= m_last && c * 8 < n_left) __builtin_nontemporal_store(u32x4{lo.x, lo.y, hi.x, hi.y}, reinterpret_cast<u32x4*>(C + (size_t)row * p.N + c * 8));
+  }
+}
+
+template <typename T, int BM, int BN, bool B_KN, bool F32OUT, int BDIV, int ROWS>
+hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, const float* residual, const DmaRows& rw) {
+  constexpr int LDS_BYTES = stages(BM) * (BM + BN) * BK * 2;  // the result's rows fit as well
+  static_assert(LDS_BYTES >= BM * (BN * 2 + 8));
+  static std::atomic<unsigned long long> configured{0};  // one bit per device: the attribute is per device
+  auto kernel = gemm_ring<T, BM, BN, B_KN, F32OUT, BDIV, ROWS>;
+  int dev = 0;
+  if (hipError_t e = hipGetDevice(&dev)) return e;
+  const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
+  if (!bit || !(configured.load(std::memory_order_relaxed) & bit)) {
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES)) return e;
+    configured.fetch_or(bit, std::memory_order_relaxed);
+  }
+  const int tiles_m = (p.M + BM - 1) / BM + rw.groups, tiles_n = (p.N + BN - 1) / BN;
+  const size_t total = (batch * (size_t)tiles_m * tiles_n + 7) / 8 * 8 + (rw.groups ? 8 : 0);
+  kernel<<<dim3((unsigned)total), dim3(512), LDS_BYTES, stream>>>(p, (int)batch, tiles_m, tiles_n, residual, rw);
+  return hipGetLastError();
+}
+
+template <typename T, bool F32OUT, int BDIV, int ROWS>
+hipError_t launch_nt(hipStream_t stream, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw) {
+  if (tile == 129) return launch<T, 256, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+  if (tile == 65) return launch<T, 128, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+  if (tile == 48) return launch<T, 64, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+  return launch<T, 64, 64, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+}
+template <typename T>
+hipError_t launch_plain(hipStream_t stream, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw) {
+  if (!(p.b_cs == 1 && p.b_rs != 1)) return launch_nt<T, false, 1, 0>(stream, p, batch, tile, residual, rw);
+  if (tile == 129) return launch<T, 256, 128, true, false, 1, 0>(stream, p, batch, residual, rw);
+  if (tile == 65) return launch<T, 128, 128, true, false, 1, 0>(stream, p, batch, residual, rw);
+  return tile == 48 ? launch<T, 64, 128, true, false, 1, 0>(stream, p, batch, residual, rw) : hipErrorInvalidValue;
+}
+
+}  // namespace
+
+hipError_t gemm_ring_launch(hipStream_t stream, int dtype, DmaForm form, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw) {
+  switch (form) {
+    case DmaForm::ROWS: return launch_nt<__bf16, false, 1, 1>(stream, p, batch, tile, residual, rw);
+    case DmaForm::ROWS_GLU: return launch_nt<__bf16, false, 1, 2>(stream, p, batch, tile, residual, rw);
+    case DmaForm::PLANES3: return launch_nt<__bf16, true, 3, 0>(stream, p, batch, tile, residual, rw);
+    case DmaForm::PLAIN: break;
+  }
+  return dtype == UGHIP_F16 ? launch_plain<_Float16>(stream, p, batch, tile, residual, rw) : launch_plain<__bf16>(stream, p, batch, tile, residual, rw);
+}
+
+}  // namespace ughip

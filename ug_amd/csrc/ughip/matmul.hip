@@ -771,16 +771,16 @@ static RowsRoute rows_route(const MMArgs& p, int dtype, bool x3, GemmEpilogue::K
   // more).  Its result leaves as f32 with the residual added on the way; SwiGLU goes through the scratch block and the fold.
   // (from 384 rows: at 128 and 256 rows the register-staged kernel is as fast or faster for four of the five products of a
   // llama step -- q|k|v 25.2 us against 28.6 at 256 rows -- and the model below does not see that; at 512 rows this kernel is)
-  long long x3_dma = -1, x3_split = 0;  // tuning aids: X3_DMA 0 keeps the register-staged kernel, 3 / 4 / 5 force a tile; X3_SPLIT n a K split
+  long long x3_dma = -1, x3_split = 0;  // tuning aids: X3_DMA 0 keeps the register-staged kernel, values of GEMM_SHAPE force a tile; X3_SPLIT n a K split
   tune_get(TUNE_X3_DMA, &x3_dma);
   tune_get(TUNE_X3_SPLIT, &x3_split);
   if (x3 && m >= 384 && x3_dma != 0) {
     MMArgs q = p;
     q.c = const_cast<void*>(dst);  // alignment of the result as f32
     double best = 0;
-    const int forced_tile = x3_dma == 3 ? 256 : x3_dma == 4 ? 128 : x3_dma == 5 ? 64 : 0;
+    const int forced_tile = x3_dma > 0 ? gemm_dma_forced_tile(x3_dma) : 0;
     const int forced_split = (int)x3_split;
-    for (int tile : {256, 128, 64}) {
+    for (int tile : {256, 128, 65, 64, 48, 32}) {  // (codes 65, 48, 32: gemm_ring; 1900 x 2048 x 2048 64 -> 54 us, 512 x 2048 x 2048 32 -> 26)
       if (forced_tile && tile != forced_tile) continue;
       for (int split : {1, 2, 4, 8}) {
         if (forced_split && split != forced_split) continue;
@@ -1036,11 +1036,7 @@ extern "C" int ughip_linear_rows_plan(int w_dtype, int product, int form, size_t
     rows_x3_name(route.x3, kind, buf, buf_len);
   } else if (route.kind == RowsRoute::DMA_PLANES) {
     const bool fold = route.dma_split > 1 || kind == GemmEpilogue::SWIGLU;
-    int bm = 256, bn = route.dma_tile == 256 ? 256 : 128;
-    if (route.dma_tile == 64) bm = 128;
-    char split[24] = "";
-    if (route.dma_split > 1) snprintf(split, sizeof split, ",splitK=%d", route.dma_split);
-    snprintf(buf, buf_len, "gemm_dma4<bf16,NT,%dx%d,256t,3 planes%s,f32 out%s>", bm, bn, split, dma_planes_tail(kind, fold, form == 1));
+    gemm_dma_planes3_name(route.dma_tile, route.dma_split, dma_planes_tail(kind, fold, form == 1), buf, buf_len);
   } else {
     gemm_tiled_name(dtype, p, 1, mixed, &epi, buf, buf_len);
   }
