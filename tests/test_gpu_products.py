@@ -98,3 +98,32 @@ def test_ring_planes(hip, tune, m, n, k):
             gpu.call("ughip_linear_add_rows", p(dx), p(dw), p(dr), p(dst), Z(m), Z(n), Z(k), 1)
             assert f"{tile},512t,ring,3 planes" in ug_amd.last_kernel()
             assert np.all(np.abs(get(dst, (m, n)) - want) <= bound)
+
+
+# tile edges (64; 128 where that many tiles fill the chip), K steps of 64 / 32 elements: none whole, one, one and a remainder, several; single rows
+# and columns, and fewer than eight of them (another kernel's)
+@pytest.mark.parametrize("bmnk", [(1, 1, 1, 1), (2, 8, 9, 7), (1, 63, 65, 33), (3, 65, 64, 31), (1, 129, 8, 64), (2, 9, 77, 65), (1, 64, 7, 129), (1, 7, 200, 128), (1, 130, 66, 200), (1, 2049, 2001, 70)])
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
+@pytest.mark.parametrize("lhs_mk", [True, False], ids=["rows", "transposed"])
+def test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk):
+    """Any size, operands that start at any element and lie either way: the bound of an f32 sum (rounded once for 16 bits), nothing written past the
+    result, nothing read from behind the operands (not-a-number there)."""
+    b, m, n, k = bmnk
+    dt, enc = {"f32": (ug_amd.F32, lambda v: v), "f16": (ug_amd.F16, lambda v: v.astype(np.float16)), "bf16": (ug_amd.BF16, rng.to_bf16_bits)}[dtype]
+    a, w = rng.uniform_pm1(1, b * m * k), rng.uniform_pm1(2, b * k * n)
+    if dtype != "f32":
+        a, w = rounded(dtype, a), rounded(dtype, w)
+    a, w = a.reshape(b, m, k), w.reshape(b, k, n)
+    nan = np.full(3, np.nan, np.float32)
+    sa = hip.slice_from(enc(np.concatenate([nan, (a if lhs_mk else np.swapaxes(a, 1, 2)).ravel(), nan]).astype(np.float32)))
+    sw = hip.slice_from(enc(np.concatenate([nan, (np.swapaxes(w, 1, 2) if rhs_nk else w).ravel(), nan]).astype(np.float32)))
+    dst = hip.slice_from(enc(np.full(b * m * n + 9, 7.0, np.float32)))
+    print("any size", dtype, bmnk, rhs_nk, lhs_mk, flush=True)
+    hip.matmul(dst, sa, sw, (b, m, n, k), ((b, m, k), (m * k, k, 1) if lhs_mk else (m * k, 1, m), 3), ((b, k, n), (k * n, 1, k) if rhs_nk else (k * n, n, 1), 3))
+    got = dst.to_vec()
+    got = (rng.from_bf16_bits(got) if dtype == "bf16" else got).astype(np.float64)
+    assert np.all(got[b * m * n :] == 7.0), "wrote past the end"
+    exact = np.matmul(a.astype(np.float64), w.astype(np.float64))
+    bound = {"f32": 0, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype] * np.abs(exact) + (k + 1) * np.finfo(np.float32).eps * np.matmul(np.abs(a).astype(np.float64), np.abs(w).astype(np.float64))
+    assert np.all(np.abs(got[: b * m * n].reshape(exact.shape) - exact) <= bound * 1.001 + 1e-7)

@@ -92,6 +92,11 @@ bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, bool swiglu, int
 int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, bool swiglu);  // a tile code, 0: no tile takes it
 hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRows& r, bool swiglu, int tile);
 
+// Any M, N, K and any alignment (gemm_ragged.hip; f32, f16, bf16): operands contiguous along k or along their other dimension, at least eight
+// elements from one k to the next in the latter case.  Contiguous [batch, M, N] result.
+bool gemm_ragged_supported(const MMArgs& p, size_t batch);
+hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch);
+
 // f32, one wave per SIMD: 256 x 128 tiles of v_mfma_f32_32x32x2_f32, loads that write LDS directly, rhs [n, k]- or [k, n]-major
 // (gemm_dma_f32.hip).  Any M, N % 4 == 0, K % 32 == 0 and K >= 64, 16-byte aligned rows, contiguous [batch, M, N] result.
 // _pick: whether this kernel should take the problem ([k, n]-major rhs, whole rounds of 256 tiles or nearly, K >= 512;

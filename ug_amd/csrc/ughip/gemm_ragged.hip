@@ -1,0 +1,251 @@
+// MFMA GEMM for operands that no tuned kernel takes -- any M, N and K, rows that start at any element -- with f32 accumulate: f32, f16, bf16;
+// each operand contiguous along k or along its other dimension.
+//
+//   64 x 64 or 128 x 128 tiles, four waves 2 x 2, 32 x 32 MFMA blocks.  A K step is 128 bytes of a k-contiguous row, 8 chunks of 16 bytes,
+//   fetched by 16-byte loads at whatever address the row has (the hardware takes any) two steps ahead into registers, then written to one of
+//   two LDS buffers: k-contiguous operands as rows of k, the others as they lie, and the waves read those back transposed
+//   (ds_read_b64_tr_b16; f32 element by element).  The last step, K's remainder or a whole one, is loaded element by element with zeros for
+//   what does not exist, and comes first, under the way of the next ones: it holds the only row of a
+//   [k, n]-major operand behind which nothing may be read.
+//
+// What bounds it: the steps' latency on few tiles (0.35 us each in 16 bits, 0.6 in f32), LDS and the f32 matrix pipe on many.  Against element-by-element
+// loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 14.5 us, f32 256 -> 35; 2001^3 f16 265 -> 40, f32 343 -> 155; 3999^2 x
+// 2000 f16 1190 -> 118, f32 1015 -> 513; 100^3 9.4 -> 5.4.  The 128 x 128 tile from 256 of them on: 2001^3 has that many.
+#include <hip/hip_runtime.h>
+
+#include "gemm.h"
+#include "ughip.h"
+
+namespace ughip {
+namespace {
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+// vectors at the address of any element
+typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
+typedef u32x2 u32x2_at2 __attribute__((aligned(2)));
+typedef f32x4 f32x4_at4 __attribute__((aligned(4)));
+__device__ __forceinline__ u32x4 load16(const float* p) { return *reinterpret_cast<const u32x4_at4*>(p); }
+template <typename T>
+__device__ __forceinline__ u32x4 load16(const T* p) {
+  return *reinterpret_cast<const u32x4_at2*>(p);
+}
+__device__ __forceinline__ void store4(float* p, const f32x4& v) { *reinterpret_cast<f32x4_at4*>(p) = v; }
+template <typename T>
+__device__ __forceinline__ void store4(T* p, const f32x4& v) {
+  typedef T tx4 __attribute__((ext_vector_type(4)));
+  *reinterpret_cast<u32x2_at2*>(p) = __builtin_bit_cast(u32x2, __builtin_convertvector(v, tx4));
+}
+
+__device__ __forceinline__ void mma(__bf16, const u32x4& a, const u32x4& b, f32x16& c) {
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ void mma(_Float16, const u32x4& a, const u32x4& b, f32x16& c) {
+  c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ void mma(float, const u32x4& a, const u32x4& b, f32x16& c) {
+  const f32x4 fa = __builtin_bit_cast(f32x4, a), fb = __builtin_bit_cast(f32x4, b);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], c, 0, 0, 0);  // lanes 0-31 the even chunk's k, 32-63 the odd one's
+}
+
+// One operand's share of a workgroup's tile: `rows` (M or N) times k.  KC: contiguous along k.
+template <typename T, int B, bool KC>
+struct Side {
+  static constexpr int E = 16 / sizeof(T), KE = 8 * E;           // elements per chunk, k per step
+  static constexpr int CPR = KC ? 8 : B / E;                     // chunks per row in LDS (a row: of k, or of the operand's rows at one k)
+  static constexpr int PITCH = CPR * 16 + 16, LDS_ROWS = KC ? B : KE, BYTES = LDS_ROWS * PITCH;
+  static constexpr int N = LDS_ROWS * CPR / 256;                 // chunks per thread
+  const T* at[N];
+  long long step;  // elements from one K step to the next
+  int lds_at[N];
+
+  __device__ void place(const T* base, int r0, int rows, long long rs, long long cs, int tid) {
+    step = KC ? KE : KE * cs;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int id = tid + 256 * i, row = id / CPR, c = id % CPR;
+      lds_at[i] = row * PITCH + c * 16;
+      // past the last row: any row (its results are not stored); a chunk that straddles the end runs on into the next k's row
+      if (KC) at[i] = base + min(r0 + row, rows - 1) * rs + c * E;
+      else at[i] = base + (long long)row * cs + (r0 + c * E < rows ? r0 + c * E : 0);
+    }
+  }
+  __device__ u32x4 load(int i, int s) const { return load16(at[i] + s * step); }
+  // step s with `left` elements of k, by element; rows: of the operand behind r0
+  __device__ u32x4 load_last(int i, int s, int left, int r0, int rows, int tid) const {
+    const int id = tid + 256 * i, row = id / CPR, c = id % CPR;
+    T v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int k = KC ? c * E + e : row;
+      long long off = s * step;
+      if (KC) off += k < left ? e : -c * E;
+      else off += (r0 + c * E < rows ? min(e, rows - 1 - r0 - c * E) : 0);
+      const bool there = k < left;
+      const T* p = at[i] + off;
+      if (!KC && !there) p = at[i] - row * (step / KE);  // something that exists: the operand's first k
+      v[e] = there ? *p : (T)0.f;
+    }
+    return __builtin_bit_cast(u32x4, v);
+  }
+  // lane's fragment of block b0 .. b0 + 31, chunk pair c2 (chunks 2 c2 and 2 c2 + 1)
+  __device__ static u32x4 frag(const char* lds, int b0, int c2, int lane) {
+    if constexpr (KC) {
+      return *reinterpret_cast<const u32x4*>(lds + (b0 + (lane & 31)) * PITCH + (2 * c2 + (lane >> 5)) * 16);
+    } else if constexpr (sizeof(T) == 4) {
+      u32x4 v;
+      const char* q = lds + (2 * c2 + (lane >> 5)) * 4 * PITCH + (b0 + (lane & 31)) * 4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = *reinterpret_cast<const unsigned*>(q + e * PITCH);
+      return v;
+    } else {
+      // lane q + 4 e of a 16-lane group names row k0 + e and four columns from 4 q; lane i receives k0 .. k0 + 3 of column i
+      typedef __attribute__((address_space(3))) s16x4 lds_v4;
+      const int g = lane >> 4, li = lane & 15, k0 = c2 * 16 + 8 * (g >> 1) + (li >> 2);
+      const char* q = lds + k0 * PITCH + (b0 + (g & 1) * 16 + 4 * (li & 3)) * 2;
+      const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)q));
+      const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(q + 4 * PITCH)));
+      return u32x4{lo.x, lo.y, hi.x, hi.y};
+    }
+  }
+};
+
+template <typename T, int BT, bool A_KC, bool B_KC>
+__global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int tiles_m, int tiles_n) {
+  typedef Side<T, BT, A_KC> SA;
+  typedef Side<T, BT, B_KC> SB;
+  constexpr int MI = BT / 64, KE = SA::KE;
+  __shared__ __attribute__((aligned(16))) char lds[2][SA::BYTES + SB::BYTES];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // each XCD a contiguous run of tiles (block ids go round-robin over the 8)
+  const int tiles = tiles_m * tiles_n, per = (tiles + 7) >> 3, bid = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if (bid >= tiles) return;
+  const int tm = bid / tiles_n, tn = bid - tm * tiles_n, m0 = tm * BT, n0 = tn * BT;
+  SA a;
+  SB b;
+  a.place(static_cast<const T*>(p.a) + (size_t)blockIdx.y * p.a_bs, m0, p.M, p.a_rs, p.a_cs, tid);
+  b.place(static_cast<const T*>(p.b) + (size_t)blockIdx.y * p.b_bs, n0, p.N, p.b_cs, p.b_rs, tid);
+  const int full = (p.K - 1) / KE, left = p.K - full * KE;  // whole steps, and 1 .. KE elements of k behind them
+  f32x16 acc[MI][MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < MI; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  const int wm = (wave >> 1) * 32 * MI, wn = (wave & 1) * 32 * MI;
+
+  u32x4 ra[2][SA::N], rb[2][SB::N], la[SA::N], lb[SB::N];
+  auto fetch = [&](int d, int s) {
+#pragma unroll
+    for (int i = 0; i < SA::N; ++i) ra[d][i] = a.load(i, s);
+#pragma unroll
+    for (int i = 0; i < SB::N; ++i) rb[d][i] = b.load(i, s);
+  };
+  auto put = [&](char* buf, const u32x4* va, const u32x4* vb) {
+#pragma unroll
+    for (int i = 0; i < SA::N; ++i) *reinterpret_cast<u32x4*>(buf + a.lds_at[i]) = va[i];
+#pragma unroll
+    for (int i = 0; i < SB::N; ++i) *reinterpret_cast<u32x4*>(buf + SA::BYTES + b.lds_at[i]) = vb[i];
+  };
+  auto multiply = [&](const char* buf) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      u32x4 fa[MI], fb[MI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) fa[i] = SA::frag(buf, wm + 32 * i, c, lane), fb[i] = SB::frag(buf + SA::BYTES, wn + 32 * i, c, lane);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < MI; ++j) mma(T(), fb[j], fa[i], acc[i][j]);  // swapped: a lane holds columns of one row
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < SA::N; ++i) la[i] = a.load_last(i, full, left, m0, p.M, tid);
+#pragma unroll
+  for (int i = 0; i < SB::N; ++i) lb[i] = b.load_last(i, full, left, n0, p.N, tid);
+  if (full > 0) {
+    fetch(0, 0);
+    fetch(1, min(1, full - 1));
+  }
+  put(lds[0], la, lb);
+  __syncthreads();
+  multiply(lds[0]);
+  for (int s0 = 0; s0 < full; s0 += 2) {
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const int s = s0 + d;
+      if (s >= full) break;
+      char* buf = lds[d ^ 1];
+      put(buf, ra[d], rb[d]);
+      fetch(d, min(s + 2, full - 1));  // (without a branch, so that a step's loads can be waited for alone)
+      __syncthreads();                 // one barrier a step: the buffer written next was read before it
+      multiply(buf);
+    }
+  }
+
+  // element e of lane l of block (i, j): row l % 32, column 8 (e / 4) + 4 (l / 32) + e % 4
+  T* __restrict__ C = static_cast<T*>(p.c) + (size_t)blockIdx.y * p.c_bs;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int row = m0 + wm + 32 * i + (lane & 31);
+    if (row >= p.M) continue;
+#pragma unroll
+    for (int j = 0; j < MI; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int col = n0 + wn + 32 * j + 8 * g + 4 * (lane >> 5);
+        T* q = C + (size_t)row * p.N + col;
+        if (col + 4 <= p.N) {
+          store4(q, f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]});
+        } else {
+#pragma unroll
+          for (int e = 0; e < 3; ++e)
+            if (col + e < p.N) q[e] = (T)acc[i][j][4 * g + e];
+        }
+      }
+  }
+}
+
+template <typename T, int BT>
+hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch) {
+  const int tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BT - 1) / BT;
+  const dim3 grid((unsigned)(((size_t)tiles_m * tiles_n + 7) / 8 * 8), (unsigned)batch);
+  const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
+  if (ak && bk) gemm_ragged<T, BT, true, true><<<grid, 256, 0, stream>>>(p, tiles_m, tiles_n);
+  else if (ak) gemm_ragged<T, BT, true, false><<<grid, 256, 0, stream>>>(p, tiles_m, tiles_n);
+  else if (bk) gemm_ragged<T, BT, false, true><<<grid, 256, 0, stream>>>(p, tiles_m, tiles_n);
+  else gemm_ragged<T, BT, false, false><<<grid, 256, 0, stream>>>(p, tiles_m, tiles_n);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_type(hipStream_t stream, const MMArgs& p, size_t batch) {
+  const size_t big = batch * (size_t)((p.M + 127) / 128) * (size_t)((p.N + 127) / 128);
+  return big >= 256 ? launch<T, 128>(stream, p, batch) : launch<T, 64>(stream, p, batch);
+}
+
+}  // namespace
+
+bool gemm_ragged_supported(const MMArgs& p, size_t batch) {
+  // an operand that is contiguous along its other dimension: eight elements or more from one k to the next, so that a chunk over the end of a
+  // row stays inside the rows behind it
+  const bool a = p.a_cs == 1 || (p.a_rs == 1 && p.a_cs >= 8 && p.M >= 8), b = p.b_rs == 1 || (p.b_cs == 1 && p.b_rs >= 8 && p.N >= 8);
+  return a && b && p.M > 0 && p.N > 0 && p.K > 0 && p.a_rs >= 0 && p.b_cs >= 0 && batch <= 65535 && (size_t)((p.M + 63) / 64) * ((p.N + 63) / 64) < (1u << 24);
+}
+
+hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch) {
+  if (!gemm_ragged_supported(p, batch)) return hipErrorInvalidValue;
+  if (dtype == UGHIP_F32) return launch_type<float>(stream, p, batch);
+  return dtype == UGHIP_F16 ? launch_type<_Float16>(stream, p, batch) : launch_type<__bf16>(stream, p, batch);
+}
+
+}  // namespace ughip

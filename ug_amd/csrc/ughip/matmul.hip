@@ -605,7 +605,8 @@ static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* l
     dim3 grid((unsigned)((n + 63) / 64), (unsigned)((m + 63) / 64), (unsigned)b);
     if (grid.y > 65535 || b > 65535) return set_error(UGHIP_ERR_INVALID, "matmul: m or batch too large for this kernel");
     note_kernel("gemm_any<%s>", tn);
-    if (f32) gemm_f32_any<<<grid, 256, 0, st>>>(p);
+    if (gemm_ragged_supported(p, b)) UGHIP_HIPCHK(gemm_ragged_launch(st, dst->dtype, p, b));
+    else if (f32) gemm_f32_any<<<grid, 256, 0, st>>>(p);
     else if (dst->dtype == UGHIP_F16) gemm_half_any<_Float16><<<grid, 256, 0, st>>>(p);
     else gemm_half_any<__bf16><<<grid, 256, 0, st>>>(p);
   }
