@@ -1141,6 +1141,13 @@ class Lowering {
     return 1;
   }
 
+  // A row whose length is no multiple of 4 is taken in groups of 4 all the same, the last one moved back so that it ends with the row: its
+  // first elements are the group before's as well (a reduction folds them once, a store writes them twice, with the same value -- what a
+  // kernel stores it never loads).  Same lengths as pick_vec's 4.  The 128-bit accesses then start at any element, which the hardware takes.
+  // By single elements -> so: softmax [16411, 1531], two kernels, 133 -> 82 us, [8000, 4097] 167 -> 105; RMSNorm [16411, 1531] 84 -> 48, [1900, 2049]
+  // 10.7 -> 8.2.  What is left is the rows' way through memory (16 bytes per element of the softmax at 5 TB/s).
+  static bool overlapped(i64 extent, i64 threads) { return extent % 4 != 0 && threads > 64 && extent > (threads - 64) * 4; }
+
   void emit_items(std::ostringstream& o, bool want_cols, uint64_t col_mask, int indent, bool guard_row_stores, int tpr, bool one_thread) const {
     for (const Item& it : items_) {
       bool is_col = (it.deps & col_mask) != 0;
@@ -1157,7 +1164,7 @@ class Lowering {
   }
 
   // Statements of a reduction loop body with the fold redirected to the thread-local partial.
-  void emit_reduce_body(std::ostringstream& o, const Region& r, int indent) const {
+  void emit_reduce_body(std::ostringstream& o, const Region& r, int indent, const char* fold_if = nullptr) const {
     std::string ty = dtype_c_name(vt_[r.acc].dtype);
     std::string fn = reduce_functor(r.op);
     std::string part = "ug_p" + std::to_string(r.acc);
@@ -1170,7 +1177,9 @@ class Lowering {
       if (i == r.fold) {
         const ughip_instr& f = I_[i];
         std::string x = opnd(r.acc_is_lhs ? f.b : f.a);
-        o << pad << part << " = " << fn << "::f(" << part << ", (" << ty << ")(" << x << "));\n";
+        // (a value chosen, not a branch around the fold: the compiler would move the loads into it one by one)
+        if (fold_if) o << pad << part << " = " << fn << "::f(" << part << ", " << fold_if << " ? (" << ty << ")(" << x << ") : " << identity_lit(r.op, vt_[r.acc].dtype) << ");\n";
+        else o << pad << part << " = " << fn << "::f(" << part << ", (" << ty << ")(" << x << "));\n";
         continue;
       }
       std::string s = stmt(i);
@@ -1185,10 +1194,13 @@ class Lowering {
     std::string pad(2 * indent, ' ');
     const LoopInfo& L = loops_[r.loop];
     std::string ty = dtype_c_name(vt_[r.acc].dtype);
-    int vec = pick_vec(L.trip, tpr);
+    const bool over = overlapped(L.trip, tpr);
+    int vec = over ? 4 : pick_vec(L.trip, tpr);
     std::string part = "ug_p" + std::to_string(r.acc);
     o << pad << ty << " " << part << " = " << identity_lit(r.op, vt_[r.acc].dtype) << ";\n";
-    o << pad << "for (int ug_i = ug_t * " << vec << "; ug_i < " << L.trip << "; ug_i += " << tpr * vec << ") {\n";
+    const char* first = over ? "ug_g" : "ug_i";
+    o << pad << "for (int " << first << " = ug_t * " << vec << "; " << first << " < " << L.trip << "; " << first << " += " << tpr * vec << ") {\n";
+    if (over) o << pad << "  const int ug_i = ug_g < " << L.trip - 4 << " ? ug_g : " << L.trip - 4 << ";\n";
     o << pad << "#pragma unroll\n";
     o << pad << "  for (int ug_u = 0; ug_u < " << vec << "; ++ug_u) {\n";
     o << pad << "    const int " << var(L.begin) << " = ";
@@ -1196,7 +1208,7 @@ class Lowering {
     o << "(ug_i + ug_u)";
     if (L.step != 1) o << " * " << L.step;
     o << ";\n";
-    emit_reduce_body(o, r, indent + 2);
+    emit_reduce_body(o, r, indent + 2, over ? "ug_i + ug_u >= ug_g" : nullptr);
     o << pad << "  }\n" << pad << "}\n";
     emit_region_finish(o, r, indent, tpr);
   }
@@ -1382,11 +1394,14 @@ class Lowering {
     for (const Item& it : items_) any_col |= (it.deps & col_mask) != 0;
     if (any_col) {
       i64 inner = cols.empty() ? 1 : loops_[cols.back()].trip;
-      int vec = (inner % 4 == 0 && pick_vec(nc, tpr) == 4) ? 4 : 1;
-      o << "    for (int ug_c = ug_t; ug_c < " << nc / vec << "; ug_c += " << tpr << ") {\n";
+      const bool over = !grid_reduce && cols.size() == 1 && overlapped(nc, tpr);
+      int vec = over || (inner % 4 == 0 && pick_vec(nc, tpr) == 4) ? 4 : 1;
+      o << "    for (int ug_c = ug_t; ug_c < " << (nc + vec - 1) / vec << "; ug_c += " << tpr << ") {\n";
+      if (over) o << "      const int ug_i = ug_c < " << nc / 4 << " ? ug_c * 4 : " << nc - 4 << ";\n";
       o << "#pragma unroll\n";
       o << "      for (int ug_u = 0; ug_u < " << vec << "; ++ug_u) {\n";
-      emit_decode(o, cols, "ug_c", vec, 4);
+      if (over) emit_decode(o, cols, "(ug_i + ug_u)", 1, 4);
+      else emit_decode(o, cols, "ug_c", vec, 4);
       emit_items(o, true, col_mask, 4, false, tpr, false);
       o << "      }\n    }\n";
     }
