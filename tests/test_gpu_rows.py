@@ -1,0 +1,34 @@
+"""Kernels over rows of the listed-layers decoders at the sizes where their vector forms begin and end."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import plain_hybrid as ph
+from gpu_calls import Gpu, View, Z, close, get, p, rand, view
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [4, 1024, 1028, 4096, 4100, 1026])
+@pytest.mark.parametrize("top", [1, 3, 4, 5, 9])
+@pytest.mark.parametrize("second", [False, True])
+def test_routed_rows_join_the_residual(hip, n, top, second):
+    """The weighted sum of routed rows, normed and added: counts around the four rows on their way at a time, places without a row, rows beyond y."""
+    gpu, m, rows, eps = Gpu(hip), 5, 7, 1e-3
+    x, y, w, nxt, weights = rand(1, m, n), rand(2, rows, n), rand(3, n), rand(4, n), rand(5, m, top)
+    slots = np.random.default_rng(6).integers(-1, rows + 1, (m, top)).astype(np.int32)
+    slots[0], slots[1] = 0, -1
+    y[rows - 1] = np.where(np.arange(n) % 2, 50.0, -50.0)
+    want = np.zeros((m, n))
+    for i in range(m):
+        for j in range(top):
+            if 0 <= slots[i, j] < rows:
+                want[i] += weights[i, j] * y[slots[i, j]]
+    want = x + ph.rms(want, eps) * w
+    sx, sy, sw, sn, ss, swt = gpu.up(x), gpu.up(y), gpu.up(w), gpu.up(nxt), gpu.up(slots), gpu.up(weights)
+    dst, copy = gpu.out(m * n), gpu.out(m * n)
+    gpu.call("ughip_add_rms_norm_rows", view(sx, 0, n), view(sy, 0, n), p(ss), p(swt), Z(top), Z(rows), p(sw), C.c_float(eps), View(None, 0, 0), view(dst, 0, n), p(sn) if second else None,
+             p(copy), Z(m), Z(n))
+    close(get(dst, (m, n)), want, 5e-6)
+    close(get(copy, (m, n)), ph.rms(want, eps) * nxt if second else want, 8e-6)
