@@ -46,7 +46,7 @@ double gemm_tiled_cost_us(int dtype, const MMArgs& p, size_t batch);
 // 16-bit types, one wave per SIMD: 256 x 256, 256 x 128 or 128 x 128 tiles (tile codes 256, 128, 64), 4 waves laid out
 // 2 x 2 with the accumulators in the accumulation registers, loads that write LDS directly, rhs [n, k]- or [k, n]-major
 // (gemm_dma.hip), and a ring of four or three stages under eight waves with 256 x 128, 128 x 128, 64 x 128 and 64 x 64 tiles (codes 129, 65, 48,
-// 32; gemm_ring.hip).  Any M, N % 8 == 0, K % 64 == 0 and K >= 256, 16-byte aligned rows, contiguous [batch, M, N] result.
+// 32; gemm_ring.hip).  Any M, N % 8 == 0, K % 64 == 0 (gemm_dma4: K >= 256), 16-byte aligned rows, contiguous [batch, M, N] result.
 bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile);
 hipError_t gemm_dma_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, int tile);
 // The tile code this kernel should take the problem with, 0 when another kernel should.
@@ -86,11 +86,17 @@ struct DmaRows {
   long long w_group = 0, dst_stride = 0;
   int groups = 0, x_rows = 0, n_out = 0;
   bool dst_bf16 = false;
+  const void* table = nullptr;  // (act LOOKUP) the result times element (ids[row], table_col + column) of a table, f32 or bf16
+  const int* ids = nullptr;
+  long long table_stride = 0, table_col = 0;
+  int table_rows = 0;
+  bool table_bf16 = false;
   float glu_alpha = 1.f, glu_shift = 0.f, glu_limit = 0.f;  // the gated unit with swiglu: gate * sigmoid(alpha gate) * (up + shift), both limited (limit > 0)
 };
-bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, bool swiglu, int tile);
-int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, bool swiglu);  // a tile code, 0: no tile takes it
-hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRows& r, bool swiglu, int tile);
+enum class RowsAct { NONE, GLU, LOOKUP };
+bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int tile);
+int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act);  // a tile code, 0: no tile takes it
+hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRows& r, RowsAct act, int tile);
 
 // Any M, N, K and any alignment (gemm_ragged.hip; f32, f16, bf16): operands contiguous along k or along their other dimension, at least eight
 // elements from one k to the next in the latter case.  Contiguous [batch, M, N] result.

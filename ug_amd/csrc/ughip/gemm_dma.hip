@@ -465,6 +465,7 @@ bool tile_dims(int tile, int* bm, int* bn) {
 }  // namespace
 
 static bool ring_tile(int tile) { return tile == 129 || tile == 65 || tile == 48 || tile == 32; }
+static int least_k(int tile) { return ring_tile(tile) ? BK : 4 * BK; }
 static const char* waves_name(int tile) { return ring_tile(tile) ? "512t,ring" : "256t"; }  // in the names of these kernels
 // (tuning aid) the tile code that GEMM_SHAPE names, 0: none
 int gemm_dma_forced_tile(long long shape) {
@@ -484,7 +485,7 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
   if (dtype != UGHIP_BF16 && dtype != UGHIP_F16) return false;
   int bm, bn;
   if (!tile_dims(tile, &bm, &bn)) return false;
-  if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < 4 * BK || batch == 0) return false;
+  if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || batch == 0) return false;
   if (p.a_cs != 1 || p.a_rs % 8 || (batch > 1 && (p.a_bs % 8 || p.b_bs % 8 || p.c_bs % 8))) return false;
   const bool nn = p.b_cs == 1 && p.b_rs != 1, nt = p.b_rs == 1 && p.b_cs != 1;
   if (nn == nt || (nn && tile == 32)) return false;
@@ -645,22 +646,22 @@ hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile
 }
 
 
-bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, bool swiglu, int tile) {
+bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int tile) {
   int bm, bn;
-  if (!tile_dims(tile, &bm, &bn) || (tile != 256 && !ring_tile(tile))) return false;
-  if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < 4 * BK || p.a_cs != 1 || p.a_rs % 8 || p.b_rs != 1 || p.b_cs % 8) return false;
-  if (r.n_out <= 0 || r.n_out % 4 || p.N != (swiglu ? 2 * r.n_out : r.n_out) || r.dst_stride % 4 || r.w_group % 8) return false;
+  if (!tile_dims(tile, &bm, &bn) || (tile != 256 && !ring_tile(tile)) || (tile == 256 && act == RowsAct::LOOKUP)) return false;
+  if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || p.a_cs != 1 || p.a_rs % 8 || p.b_rs != 1 || p.b_cs % 8) return false;
+  if (r.n_out <= 0 || r.n_out % 4 || p.N != (act == RowsAct::GLU ? 2 * r.n_out : r.n_out) || r.dst_stride % 4 || r.w_group % 8) return false;
   // per-lane offsets are 32-bit: rows of x anywhere, matrix rows of a tile (of the whole matrix with SwiGLU)
   const unsigned long long x_rows = r.row_index ? r.x_rows : p.M;
-  if (x_rows * p.a_rs * 2 >= (1ull << 31) || (unsigned long long)p.b_cs * 2 * (swiglu ? p.N : bn) >= (1ull << 31)) return false;
+  if (x_rows * p.a_rs * 2 >= (1ull << 31) || (unsigned long long)p.b_cs * 2 * (act == RowsAct::GLU ? p.N : bn) >= (1ull << 31)) return false;
   if (!aligned16(p.a) || !aligned16(p.b) || !aligned16(r.dst) || (r.bias && !aligned16(r.bias))) return false;
   return ((size_t)(p.M + bm - 1) / bm + r.groups) * (size_t)((p.N + bn - 1) / bn) < (1u << 24);
 }
 
-int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, bool swiglu) {
+int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
   if (long long s; tune_get(TUNE_GEMM_SHAPE, &s)) {  // tuning aid, as for gemm_dma_pick
     const int forced = gemm_dma_forced_tile(s);
-    return forced && gemm_dma_rows_supported(p, r, swiglu, forced) ? forced : 0;
+    return forced && gemm_dma_rows_supported(p, r, act, forced) ? forced : 0;
   }
   // A model's products: the matrix comes from memory.  256 x 256 tiles of gemm_dma4 and the ring's, by what they are expected to take
   // (2048 positions: down 74 -> 51 us, gate and up 105 -> 89, output 26 -> 18, attention's input 37 -> 29; 509 positions: state-space output
@@ -670,7 +671,7 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, bool swiglu) {
   int best = 0;
   double best_us = 0;
   for (int tile : {256, 129, 65, 48, 32}) {
-    if (!gemm_dma_rows_supported(p, r, swiglu, tile)) continue;
+    if (!gemm_dma_rows_supported(p, r, act, tile)) continue;
     int bm, bn;
     tile_dims(tile, &bm, &bn);
     // tile rows: of groups near or above a tile's height every second one takes one more
@@ -686,13 +687,13 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, bool swiglu) {
   return best;
 }
 
-hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRows& r, bool swiglu, int tile) {
-  if (!gemm_dma_rows_supported(p, r, swiglu, tile)) return hipErrorInvalidValue;
+hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRows& r, RowsAct act, int tile) {
+  if (!gemm_dma_rows_supported(p, r, act, tile)) return hipErrorInvalidValue;
   int bm = 0, bn = 0;
   tile_dims(tile, &bm, &bn);
-  note_kernel("gemm_dma4<bf16,NT,%dx%d,%s,rows%s%s>", bm, bn, waves_name(tile), swiglu ? ",swiglu" : "", r.groups ? ",grouped" : "");
-  if (ring_tile(tile)) return gemm_ring_launch(stream, UGHIP_BF16, swiglu ? DmaForm::ROWS_GLU : DmaForm::ROWS, p, 1, tile, nullptr, r);
-  return swiglu ? launch<__bf16, 256, 256, false, false, 1, 2>(stream, p, 1, nullptr, r) : launch<__bf16, 256, 256, false, false, 1, 1>(stream, p, 1, nullptr, r);
+  note_kernel("gemm_dma4<bf16,NT,%dx%d,%s,rows%s%s>", bm, bn, waves_name(tile), act == RowsAct::GLU ? ",swiglu" : act == RowsAct::LOOKUP ? ",lookup" : "", r.groups ? ",grouped" : "");
+  if (ring_tile(tile)) return gemm_ring_launch(stream, UGHIP_BF16, act == RowsAct::GLU ? DmaForm::ROWS_GLU : act == RowsAct::LOOKUP ? DmaForm::ROWS_LOOKUP : DmaForm::ROWS, p, 1, tile, nullptr, r);
+  return act == RowsAct::GLU ? launch<__bf16, 256, 256, false, false, 1, 2>(stream, p, 1, nullptr, r) : launch<__bf16, 256, 256, false, false, 1, 1>(stream, p, 1, nullptr, r);
 }
 
 // Both operands as three bf16 planes per 64 elements of k (p.K = 6 k, rows of 3 k elements), f32 result: see BDIV == 6.

@@ -17,6 +17,7 @@
 
 #include "gemm_dma.h"
 #include "internal.h"
+#include "layers.h"
 #include "ughip.h"
 
 namespace ughip {
@@ -24,7 +25,7 @@ namespace {
 
 constexpr int stages(int bm) { return bm == 256 ? 3 : 4; }
 
-// Template parameters and DmaRows as in gemm_dma4.
+// Template parameters and DmaRows as in gemm_dma4; ROWS 3: rows that leave as gelu(y) times an element of their token's row of a table.
 template <typename T, int BM, int BN, bool B_KN, bool F32OUT, int BDIV, int ROWS>
 __global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tiles_m, int tiles_n, const float* __restrict__ residual, DmaRows rw) {
   static_assert(ROWS == 0 || (BDIV == 1 && !B_KN && !F32OUT), "rows: one plane against an [n, k]-major rhs");
@@ -192,17 +193,21 @@ __global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tile
   };
 #pragma unroll
   for (int t = 0; t < S; ++t)
+    if (t < KT) {
 #pragma unroll
-    for (int d = 0; d < ND; ++d) dma(t, d);
-  wait_vmcnt<(S - 1) * ND>();
+      for (int d = 0; d < ND; ++d) dma(t, d);
+    }
+  if (KT >= S) wait_vmcnt<(S - 1) * ND>();
+  else wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int r = 0; r < R; ++r) read_frag(0, 0, r, 0);
-  const int full = KT - S;
-  for (int kt = 0; kt < full; ++kt) body(kt, CS());
-  if constexpr (S == 4) body(KT - 4, std::integral_constant<int, 3>());
-  body(KT - 3, std::integral_constant<int, 2>());
-  body(KT - 2, C1());
+  for (int kt = 0; kt < KT - S; ++kt) body(kt, CS());
+  if constexpr (S == 4) {
+    if (KT > 3) body(KT - 4, std::integral_constant<int, 3>());
+  }
+  if (KT > 2) body(KT - 3, std::integral_constant<int, 2>());
+  if (KT > 1) body(KT - 2, C1());
   body(KT - 1, C0());
 
   // Register e of lane l of block (i, j): row wm + 16 i + l % 16, column wn + 16 j + 4 (l / 16) + e.
@@ -223,6 +228,15 @@ __global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tile
         const int row = wm + i * 16 + (lane & 15);
         if (row > m_last) continue;
         floatx4 v = acc[i][j] + b;
+        if constexpr (ROWS == 3) {
+          const int id = rw.ids[m0 + row];
+          const size_t at = (size_t)(id >= 0 && id < rw.table_rows ? id : 0) * rw.table_stride + rw.table_col + col;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float f = rw.table_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(rw.table)[at + e]) : static_cast<const float*>(rw.table)[at + e];
+            v[e] = gelu_tanh_f(v[e]) * (id >= 0 && id < rw.table_rows ? f : __uint_as_float(0x7fc00000u));
+          }
+        }
         if constexpr (ROWS == 2) {
           floatx4 u = acc[i][j + NC] + bu;
           if (rw.glu_limit > 0.f) {
@@ -324,6 +338,7 @@ hipError_t launch_plain(hipStream_t stream, const MMArgs& p, size_t batch, int t
 hipError_t gemm_ring_launch(hipStream_t stream, int dtype, DmaForm form, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw) {
   switch (form) {
     case DmaForm::ROWS: return launch_nt<__bf16, false, 1, 1>(stream, p, batch, tile, residual, rw);
+    case DmaForm::ROWS_LOOKUP: return launch_nt<__bf16, false, 1, 3>(stream, p, batch, tile, residual, rw);
     case DmaForm::ROWS_GLU: return launch_nt<__bf16, false, 1, 2>(stream, p, batch, tile, residual, rw);
     case DmaForm::PLANES3: return launch_nt<__bf16, true, 3, 0>(stream, p, batch, tile, residual, rw);
     case DmaForm::PLAIN: break;

@@ -313,9 +313,6 @@ hipError_t launch_types(hipStream_t st, const ProductArgs& a, int act, bool vec)
   return launch_act<CT, XT, WT, UGHIP_ACT_NONE>(st, a, vec);
 }
 
-// below that the few-row tile (64 x 64 of rows_product_kernel) and its longer steps; at 17 rows of 10304 x 2048 the ring takes 12.6 us against 17.6
-constexpr size_t DMA_ROWS_MIN = 17;
-
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
@@ -380,11 +377,21 @@ extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
   a.glu = glu_form(p->act, p->act_alpha, p->act_shift, p->act_limit);
   const bool vec = p->k % 8 == 0 && (p->x.stride * xs) % 16 == 0 && (w_stride * (p->w->dtype == UGHIP_BF16 ? 2 : 4)) % 16 == 0 && aligned16(a.x) && aligned16(a.w);
   const bool xb = p->x.s->dtype == UGHIP_BF16, wb = p->w->dtype == UGHIP_BF16;
+  // one row (the head behind a prompt): the decode kernels, which stream the matrix past f32 values of the row (32000 x 2048 bf16: 22 us against 36 here)
+  if (p->m == 1 && !xb && !a.dst_bf16 && p->act == UGHIP_ACT_NONE && !a.bias && !p->groups && w_stride == p->k && p->k % 4 == 0 && p->k >= 512 && p->x.offset == 0 &&
+      p->dst.offset == 0 && p->dst.s != p->x.s) {
+    const ughip_slice* w = p->w;
+    if (int rc = ughip_gemv_multi(dev, p->x.s, 1, &w, &p->n, p->k, p->dst.s)) return rc;
+    note_kernel("rows_product<%s,one row>", f32 ? "f32" : "bf16");
+    return UGHIP_OK;
+  }
   // few dense rows: products that share their K among workgroups
   if (!f32 && !xb && wb && !a.dst_bf16 && p->act == UGHIP_ACT_NONE && !a.bias && !a.groups && p->x.stride == p->k && p->dst.stride == p->n && w_stride == p->k &&
       few_rows_product_fits(p->w, static_cast<const float*>(a.x), static_cast<const float*>(a.dst), p->m, p->n, p->k))
     return few_rows_product(dev, what, static_cast<const float*>(a.x), p->w, static_cast<float*>(a.dst), p->m, p->n, p->k);
-  if (xb && wb && p->act != UGHIP_ACT_GELU_MUL && p->m >= DMA_ROWS_MIN) {
+  // bf16 rows and matrices: tiles of the kernels whose loads write LDS, from one row up (17 rows of 10304 x 2048 12.6 us against 17.6 here, 5 gated
+  // rows of 11264 x 2048 12.4 against 28.5; 509 rows of 256 x 2048 times a lookup 14.2 against 20.2, 2048 rows of 2048 x 128 8.4 against 12.3)
+  if (xb && wb) {
     MMArgs q;
     q.a = a.x, q.b = a.w, q.c = nullptr;
     q.M = a.m, q.N = (int)w_rows, q.K = a.k;
@@ -394,8 +401,10 @@ extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
     r.row_index = a.row_index, r.group_end = a.group_end, r.bias = a.bias, r.dst = a.dst, r.w_group = (long long)a.w_group, r.dst_stride = (long long)a.dst_stride;
     r.groups = a.groups, r.x_rows = a.x_rows, r.n_out = a.n, r.dst_bf16 = a.dst_bf16;
     r.glu_alpha = a.glu.alpha, r.glu_shift = a.glu.shift, r.glu_limit = a.glu.limit;
-    if (const int tile = gemm_dma_rows_pick(q, r, glu)) {
-      UGHIP_HIPCHK(gemm_dma_launch_rows(dev->stream, q, r, glu, tile));
+    r.table = a.table, r.ids = a.ids, r.table_stride = (long long)a.table_stride, r.table_col = (long long)a.table_col, r.table_rows = a.table_rows, r.table_bf16 = a.table_bf16;
+    const RowsAct form = glu ? RowsAct::GLU : act == UGHIP_ACT_GELU_MUL ? RowsAct::LOOKUP : RowsAct::NONE;
+    if (const int tile = gemm_dma_rows_pick(q, r, form)) {
+      UGHIP_HIPCHK(gemm_dma_launch_rows(dev->stream, q, r, form, tile));
       return UGHIP_OK;
     }
   }
