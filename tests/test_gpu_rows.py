@@ -32,3 +32,19 @@ def test_routed_rows_join_the_residual(hip, n, top, second):
              p(copy), Z(m), Z(n))
     close(get(dst, (m, n)), want, 5e-6)
     close(get(copy, (m, n)), ph.rms(want, eps) * nxt if second else want, 8e-6)
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("t, want", [(40, [39]), (40, [7, 0, 39]), (3, [1, 1]), (2, [1, 0]), (130, list(range(129))), (1, [0])])
+def test_llama_logits_of_some_positions(hip, bf16, t, want):
+    """The head on the wanted rows alone gives what it gives among all of them, and the state behind the step is the same."""
+    import ug_amd
+    cfg = {"model_type": "llama", "hidden_size": 256, "intermediate_size": 512, "max_position_embeddings": 256, "num_attention_heads": 4, "num_key_value_heads": 2, "num_hidden_layers": 2,
+           "rms_norm_eps": 1e-5, "vocab_size": 97}
+    model = ug_amd.Decoder.random(hip, cfg, bf16=bf16, seed=3, std=0.1, norm_mean=1.0)
+    tokens = np.random.default_rng(t).integers(0, 97, t)
+    all_state, state = model.new_state(200), model.new_state(200)
+    full, some = model.step(all_state, tokens, want=np.arange(t)), model.step(state, tokens, want=want)
+    assert some.shape == (len(want), 97)
+    np.testing.assert_allclose(some, full[want], rtol=0, atol=2e-5 * np.abs(full).max())   # the same f32 sums in another order
+    np.testing.assert_array_equal(model.step(state, [5], want=[0]), model.step(all_state, [5], want=[0]))

@@ -92,7 +92,12 @@ std::vector<float> decoder_step(const Decoder& model, DecoderState& state, const
     x.data_vec(v.data(), DType::F32);
     hidden->push_back(std::move(v));
   };
-  LB logits = model.step(ids, pos, state, want.empty() ? nullptr : &rows, hidden ? &keep : nullptr);
+  // Several positions: the hidden state behind every layer is realised as soon as its graph exists, as generate_greedy does with a prompt, so
+  // the device starts on layer 0 while the others' graphs are built (prompts over 6 layers: 2048 positions 2.69 -> 2.48 ms, 509 positions with experts 2.15 -> 1.91).
+  std::vector<std::unique_ptr<CompiledSchedule>> layers;
+  const std::function<void(const LB&)> launch = [&](const LB& x) { layers.push_back(std::make_unique<CompiledSchedule>(Schedule::create_one(x).compile_and_run(cache))); };
+  const bool by_layer = tokens.size() > 1 && dev->runs_async() && !switch_on(SW_NO_LAYER_STEPS);
+  LB logits = model.step(ids, pos, state, want.empty() ? nullptr : &rows, hidden ? &keep : by_layer ? &launch : nullptr);
   CompiledSchedule compiled = Schedule::create_one(logits).compile_and_run(cache);
   state.settle();
   std::vector<float> out;

@@ -1051,7 +1051,7 @@ std::vector<Cache> Model::new_cache() const {
 }
 
 // model.rs:259-269, 365-373
-LB Model::fwd(const LB& tokens, const LB& pos, std::vector<Cache>& cache, const std::function<void(const LB&)>* after_layer, bool last_position_only) const {
+LB Model::fwd(const LB& tokens, const LB& pos, std::vector<Cache>& cache, const std::function<void(const LB&)>* after_layer, bool last_position_only, const LB* rows) const {
   if (cache.size() != layers_.size()) bail("cache/layer count mismatch");
   LB xs = index_select(embedding_, tokens);
   float eps = (float)cfg_.rms_norm_eps;
@@ -1077,6 +1077,9 @@ LB Model::fwd(const LB& tokens, const LB& pos, std::vector<Cache>& cache, const 
     // a prompt whose logits are read at the last position only: one row through the norm and the head (the row-vector kernel
     // streams the head once, as in a decode step) instead of all of them
     if (last_position_only && xs.rank() == 3 && xs.dims()[1] > 1) xs = xs.narrow(1, xs.dims()[1] - 1, 1);
+    // and a step that asks for some positions: those rows alone meet the norm and the head
+    if (rows && xs.rank() == 3 && xs.dims()[0] == 1 && rows->elem_count() < xs.dims()[1])
+      xs = index_select(xs.reshape(Shape({xs.dims()[1], xs.dims()[2]})), *rows).reshape(Shape({1, rows->elem_count(), xs.dims()[2]}));
     return ops_->linear_packed(xs, {head_}, &ln_f_, eps);
   }
   xs = rms_norm(xs, ln_f_, eps);
@@ -1109,9 +1112,9 @@ LB Model::step(const LB& tokens, const LB& pos, DecoderState& state, const LB* r
   LlamaState* s = dynamic_cast<LlamaState*>(&state);
   if (!s) bail("a llama step needs a llama state");
   const size_t t = tokens.dims()[1];
-  LB logits = fwd(tokens, pos, s->cache, after_layer, rows == nullptr);
+  LB logits = fwd(tokens, pos, s->cache, after_layer, rows == nullptr, rows);
   s->len += t;
-  if (!rows) return logits;
+  if (!rows || logits.dims()[logits.rank() - 2] != t) return logits;
   return index_select(logits.reshape(Shape({t, cfg_.vocab_size})), *rows);
 }
 
