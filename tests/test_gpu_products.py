@@ -42,7 +42,7 @@ def test_ring_tiles(hip, tune, bmnk, dtype, rhs_nk):
         np.testing.assert_array_equal(_raw_matmul(hip, dt, ai, wi, rhs_nk), whole)
 
 
-@pytest.mark.parametrize("m, n, k, groups", [(17, 72, 256, 0), (70, 136, 320, 0), (300, 264, 384, 0), (301, 40, 448, 5), (40, 136, 576, 3)])
+@pytest.mark.parametrize("m, n, k, groups", [(1, 8, 64, 0), (17, 72, 128, 0), (193, 392, 192, 0), (70, 136, 320, 0), (300, 264, 384, 0), (301, 40, 448, 5), (40, 136, 576, 3)])
 @pytest.mark.parametrize("act", [NONE, SWIGLU, GLU])
 def test_ring_rows(hip, tune, m, n, k, groups, act):
     """Products of rows on every tile of the ring: bias, gated units, rows gathered and sorted by matrix (one matrix without any)."""
@@ -63,7 +63,7 @@ def test_ring_rows(hip, tune, m, n, k, groups, act):
         y = g / (1 + np.exp(-alpha * g)) * (u + shift)
     dx, dw, db = gpu.up(x, bf16=True), gpu.up(w, bf16=True), gpu.up(bias)
     idx = (gpu.up(src), gpu.up(end)) if groups else (None, None)
-    for shape, tile in RING.items():
+    for shape, tile in {**RING, "11": "192x192"}.items():
         tune.setenv("UGHIP_GEMM_SHAPE", shape)
         dst = gpu.out(m * n + 8)
         q = Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), bias=None if groups else db.raw(), m=m, n=n, k=k, product=BF16, act=act, row_index=idx[0].raw() if groups else None,

@@ -70,7 +70,7 @@ __device__ __forceinline__ int rhs_k_tile(int tile) {
 
 // The products those kernels take, besides plain ones: see gemm_dma4.
 enum class DmaForm { PLAIN, PLANES3, ROWS, ROWS_GLU, ROWS_LOOKUP };
-// gemm_ring.hip: one of its tiles (codes 129, 65, 48, 32: 256 x 128, 128 x 128, 64 x 128, 64 x 64), operands as the _supported functions of gemm_dma.hip check them.
+// gemm_ring.hip: one of its tiles (codes 129, 97, 65, 48, 32: 256 x 128, 192 x 192, 128 x 128, 64 x 128, 64 x 64), operands as the _supported functions of gemm_dma.hip check them.
 hipError_t gemm_ring_launch(hipStream_t stream, int dtype, DmaForm form, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw);
 
 }  // namespace ughip

@@ -452,10 +452,11 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 namespace {
 // tile codes of the entry points below: 256 = 256 x 256, 128 = 256 x 128, 64 = 128 x 128; on gemm_ring 129 = 256 x 128, 65 = 128 x 128, 48 = 64 x 128,
-// 32 = 64 x 64 ([n, k]-major rhs only)
+// 32 = 64 x 64 ([n, k]-major rhs only), 97 = 192 x 192 (rows only)
 bool tile_dims(int tile, int* bm, int* bn) {
   if (tile == 256) *bm = 256, *bn = 256;
   else if (tile == 128 || tile == 129) *bm = 256, *bn = 128;
+  else if (tile == 97) *bm = 192, *bn = 192;
   else if (tile == 64 || tile == 65) *bm = 128, *bn = 128;
   else if (tile == 48) *bm = 64, *bn = 128;
   else if (tile == 32) *bm = 64, *bn = 64;
@@ -464,7 +465,7 @@ bool tile_dims(int tile, int* bm, int* bn) {
 }
 }  // namespace
 
-static bool ring_tile(int tile) { return tile == 129 || tile == 65 || tile == 48 || tile == 32; }
+static bool ring_tile(int tile) { return tile == 129 || tile == 97 || tile == 65 || tile == 48 || tile == 32; }
 static int least_k(int tile) { return ring_tile(tile) ? BK : 4 * BK; }
 static const char* waves_name(int tile) { return ring_tile(tile) ? "512t,ring" : "256t"; }  // in the names of these kernels
 // (tuning aid) the tile code that GEMM_SHAPE names, 0: none
@@ -477,6 +478,7 @@ int gemm_dma_forced_tile(long long shape) {
     case 7: return 48;
     case 9: return 32;
     case 10: return 129;
+    case 11: return 97;
   }
   return 0;
 }
@@ -488,7 +490,7 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || batch == 0) return false;
   if (p.a_cs != 1 || p.a_rs % 8 || (batch > 1 && (p.a_bs % 8 || p.b_bs % 8 || p.c_bs % 8))) return false;
   const bool nn = p.b_cs == 1 && p.b_rs != 1, nt = p.b_rs == 1 && p.b_cs != 1;
-  if (nn == nt || (nn && tile == 32)) return false;
+  if (nn == nt || (nn && tile == 32) || tile == 97) return false;
   const long long ldb = nn ? p.b_rs : p.b_cs;
   if (ldb % 8) return false;
   // per-lane offsets are 32-bit: the furthest row of a tile has to stay below 4 GiB from the tile's first byte
@@ -501,12 +503,13 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
 // on their way to a CU, some 100 bytes per ns from the memory-side cache and 60 from HBM however many are asked for at once (with the MFMAs or the
 // LDS reads taken out the kernel takes as long), so it goes by where the operands come from: `streamed` is a matrix nobody has read
 // lately, as the weights of a model's next layer are.  Fitted to (m x n x k, us): 2048^2 x 5632 streamed 51 (128 x 128) / 67 (256 x 128), 1024 x 2048 x
-// 5632 streamed 38 (64 x 128), 509 x 2048 x 5632 streamed 26 (64 x 64), 2048 x 11264 x 2048 streamed 89 (256 x 128); 2048^3 19.2 (128 x 128),
+// 5632 streamed 38 (64 x 128), 509 x 2048 x 5632 streamed 26 (64 x 64), 2048 x 11264 x 2048 streamed 89 (256 x 128), 700 x
+// 11264 x 2048 streamed 34 and 1500 x 11264 x 2048 68 (192 x 192); 2048^3 19.2 (128 x 128),
 // 1024 x 2048 x 4096 21.1 (64 x 128), 256 x 4096^2 14.7 (64 x 64).
 static double ring_cost_us(size_t tiles, int kt, int tile, bool streamed) {
-  const double t0 = tile == 129 ? 0.64 : tile == 65 ? (streamed ? 0.54 : 0.30) : tile == 48 ? (streamed ? 0.40 : 0.21) : streamed ? 0.255 : 0.11;
-  const double t1 = tile == 129 ? 0.22 : streamed ? 0 : tile == 65 ? 0.17 : tile == 48 ? 0.07 : 0.075;
-  double us = tile == 129 ? 5.0 : tile == 65 ? 4.0 : 3.3;
+  const double t0 = tile == 129 ? 0.64 : tile == 97 ? 0.62 : tile == 65 ? (streamed ? 0.54 : 0.30) : tile == 48 ? (streamed ? 0.40 : 0.21) : streamed ? 0.255 : 0.11;
+  const double t1 = tile == 129 ? 0.22 : tile == 97 ? 0.30 : streamed ? 0 : tile == 65 ? 0.17 : tile == 48 ? 0.07 : 0.075;
+  double us = tile == 129 || tile == 97 ? 5.0 : tile == 65 ? 4.0 : 3.3;
   for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (t0 + t1 * (left < 256 ? (double)left : 256.0) / 256.0);
   return us;
 }
@@ -648,7 +651,7 @@ hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile
 
 bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int tile) {
   int bm, bn;
-  if (!tile_dims(tile, &bm, &bn) || (tile != 256 && !ring_tile(tile)) || (tile == 256 && act == RowsAct::LOOKUP)) return false;
+  if (!tile_dims(tile, &bm, &bn) || (tile != 256 && !ring_tile(tile)) || ((tile == 256 || tile == 97) && act == RowsAct::LOOKUP)) return false;
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || p.a_cs != 1 || p.a_rs % 8 || p.b_rs != 1 || p.b_cs % 8) return false;
   if (r.n_out <= 0 || r.n_out % 4 || p.N != (act == RowsAct::GLU ? 2 * r.n_out : r.n_out) || r.dst_stride % 4 || r.w_group % 8) return false;
   // per-lane offsets are 32-bit: rows of x anywhere, matrix rows of a tile (of the whole matrix with SwiGLU)
@@ -665,13 +668,15 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
   }
   // A model's products: the matrix comes from memory.  256 x 256 tiles of gemm_dma4 and the ring's, by what they are expected to take
   // (2048 positions: down 74 -> 51 us, gate and up 105 -> 89, output 26 -> 18, attention's input 37 -> 29; 509 positions: state-space output
-  // 53 -> 19, input 43 -> 32, dense gate and up 40 -> 30; 16 experts' gate and up 83 -> 62, down 38 -> 33; 33 rows of 11264 x 2048 31 -> 13).
+  // 53 -> 19, input 43 -> 32, dense gate and up 40 -> 30; 16 experts' gate and up 83 -> 62, down 38 -> 33, 700 positions' gate and
+  // up 52 -> 34; 33 rows of 11264 x 2048 31 -> 13).
   const size_t groups = r.groups ? r.groups : 1;
   const double m = (double)p.M / groups;  // rows as if they were spread evenly
   int best = 0;
   double best_us = 0;
-  for (int tile : {256, 129, 65, 48, 32}) {
-    if (!gemm_dma_rows_supported(p, r, act, tile)) continue;
+  for (int tile : {256, 129, 65, 48, 32, 97}) {
+    // (192 x 192 where it saves a round of one matrix's tiles; a model's experts are too uneven: rows past 192 cost the round they were to save)
+    if (!gemm_dma_rows_supported(p, r, act, tile) || (tile == 97 && r.groups)) continue;
     int bm, bn;
     tile_dims(tile, &bm, &bn);
     // tile rows: of groups near or above a tile's height every second one takes one more
@@ -682,7 +687,7 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
     if (tile == 256)
       for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (1.23 + 0.33 * (left < 256 ? (double)left : 256.0) / 256.0);
     else us = ring_cost_us(tiles, kt, tile, true);
-    if (!best || us < best_us * 0.97) best = tile, best_us = us;  // the larger tile on a near tie
+    if (!best || us < best_us * (tile == 97 ? 0.9 : 0.97)) best = tile, best_us = us;  // the larger tile on a near tie
   }
   return best;
 }

@@ -2,7 +2,8 @@
 //
 //   Eight waves, 4 x 2, each BM / 4 x BN / 2 of the result in 16 x 16 accumulators (v_mfma_f32_16x16x32): a wave's waits are filled by the other
 //   one of its SIMD.  The k order of every sum is that of gemm_dma4 and gemm_tiled, so the results are theirs bit for bit.
-//   A ring of four stages (three for 256 x 128): the loads of a K tile go out (global_load_lds_dwordx4, as in gemm_dma4) when the tile that
+//   192 x 192 for rows only: 700 rows against 11264 x 2048 are 236 of them, one round (52 us with 256 x 256, 54 with 256 x 128, 34 so).
+//   A ring of four stages (three for the two largest tiles): the loads of a K tile go out (global_load_lds_dwordx4, as in gemm_dma4) when the tile that
 //   many in front of it has been read, so three (two) tiles are on their way while one is multiplied.  One barrier per K tile.
 //
 // What bounds it: the operands' way to a CU.  2048^2 x 5632 on 128 x 128 tiles, one to a CU, takes 0.51 us per K tile of 32 KB with the operands in
@@ -23,7 +24,7 @@
 namespace ughip {
 namespace {
 
-constexpr int stages(int bm) { return bm == 256 ? 3 : 4; }
+constexpr int stages(int bm) { return bm >= 192 ? 3 : 4; }
 
 // Template parameters and DmaRows as in gemm_dma4; ROWS 3: rows that leave as gelu(y) times an element of their token's row of a table.
 template <typename T, int BM, int BN, bool B_KN, bool F32OUT, int BDIV, int ROWS>
@@ -321,6 +322,9 @@ hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, const float
 template <typename T, bool F32OUT, int BDIV, int ROWS>
 hipError_t launch_nt(hipStream_t stream, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw) {
   if (tile == 129) return launch<T, 256, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+  if constexpr (ROWS == 1 || ROWS == 2) {
+    if (tile == 97) return launch<T, 192, 192, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+  }
   if (tile == 65) return launch<T, 128, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
   if (tile == 48) return launch<T, 64, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
   return launch<T, 64, 64, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
