@@ -813,7 +813,7 @@ def llama_pieces(dev, steps, warmup):
     # occupy the vector ALU): TFLOP/s and frac_mfma_f32 are the f32 products the op stands for against the f32 peak,
     # frac_mfma_bf16 prices the six-fold flops it actually issues against the bf16 peak.
     out["c4_attention_cached_t512"] = {"us": round(sec * 1e6, 2), "TFLOP/s": round(flop / sec / 1e12, 2), "frac_mfma_f32": round(flop / sec / 1e12 / MFMA_F32_PEAK_TF, 4),
-                                       "frac_mfma_bf16": round(6 * flop / sec / 1e12 / MFMA_BF16_PEAK_TF, 4), "kernel": "att_planes_kernel + attention_prefill_x6_kernel<2>",
+                                       "frac_mfma_bf16": round(6 * flop / sec / 1e12 / MFMA_BF16_PEAK_TF, 4), "kernel": "att_planes_kernel + attention_prefill_x6_kernel",
                                        "algorithmic_bytes": int(nbytes), "verified": True,
                                        "replaces": "c4_rope_q + c4_qk_t + c4_causal_softmax_fused + c4_att_v + 2 repeats + 2 transposes"}
     # the same op over a prompt of 2048 positions (a full cache), and with the f32 products it had before

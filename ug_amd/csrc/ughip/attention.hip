@@ -744,6 +744,7 @@ typedef __bf16 att_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float att_f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned att_u32x4 __attribute__((ext_vector_type(4)));
 constexpr int ATT_PLANE_BLOCK = 1536;  // 16-byte units per block of 32 keys: 2 x 3 planes x 4 operands x 64 lanes
+constexpr int ATT_MERGE_ROW = 66;      // floats from one register's 64 lanes to the next: four registers on, 8 banks on
 
 // (x0, x1) -> three words of two bf16 each (x0 in the low half); remainders are exact f32 subtractions.  An infinity or a
 // NaN stays whole in the first term (FINITE: the caller knows there is no infinity, e.g. among the exponentials of a softmax;
@@ -816,33 +817,35 @@ __device__ __forceinline__ att_f32x16 att_mma_bf16(const att_u32x4& a, const att
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf16x8, a), __builtin_bit_cast(att_bf16x8, b), c, 0, 0, 0);
 }
 
-// Same work split, statistics, merge and output as attention_prefill_kernel<64, GROUPS>; q is scaled before it is split
-// (scores come out of the MFMAs scaled, and in units of log 2).  planes: what att_planes_kernel wrote for these caches, n_kb blocks per kv head.
+// A workgroup takes 32 queries of a head, its four waves every fourth block of keys, as attention_prefill_kernel<64, 1> does; the
+// four partial results meet in LDS.  q is scaled before it is split (scores come out of the MFMAs scaled, and in units of log 2).
+// planes: what att_planes_kernel wrote for these caches, n_kb blocks per kv head.
 // dst_planes != nullptr: the result goes there as the three bf16 planes of rows of nh * 64 elements (what a product of
 // these rows on the bf16 matrix pipe reads) and dst is not written.
-template <int GROUPS>
-__global__ void __launch_bounds__(256 * GROUPS, 2) attention_prefill_x6_kernel(const float* __restrict__ q, const att_u32x4* __restrict__ planes, float* __restrict__ dst,
-                                                                               uint16_t* __restrict__ dst_planes, int nh, int nkv, int t, int s, int n_kb, size_t q_row_stride, float scale,
-                                                                               const float* __restrict__ cos_t, const float* __restrict__ sin_t,
-                                                                               const int* __restrict__ pos, size_t table_len, int interleaved) {
+// Grid (b * nh, blocks of queries over y and z): the longest rows of every head first, two workgroups to a CU that start and end
+// apart, so that one's loop covers the other's first loads and its merge.  Neighbours in x, which go to the chip's eight parts in
+// turn, have different key heads: a part's cache holds the planes of one or a few (24 KB per 32 keys and head).  1900 positions, 32
+// heads on 4: 145 us with a long and a short row of queries sharing a workgroup of eight waves whose first wave merged and stored
+// alone, 113 us so; its MFMAs alone are 37 us, its vector instructions another 21.
+__global__ void __launch_bounds__(256, 2) attention_prefill_x6_kernel(const float* __restrict__ q, const att_u32x4* __restrict__ planes, float* __restrict__ dst,
+                                                                      uint16_t* __restrict__ dst_planes, int nh, int nkv, int t, int s, int n_kb, size_t q_row_stride, float scale,
+                                                                      const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+                                                                      const int* __restrict__ pos, size_t table_len, int interleaved) {
   constexpr int D = 64, H = D / 2, DB = D / 32;
-  __shared__ float merge_ml_all[GROUPS][3][2][64];
-  __shared__ float merge_o_all[GROUPS][3][DB * 16][64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3, group = tid >> 8;
+  __shared__ float merge_ml[4][2][64];
+  __shared__ float merge_o[4][DB * 16][ATT_MERGE_ROW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 31, hh = lane >> 5;
-  const int bh = blockIdx.y, b = bh / nh, head = bh % nh, kvh = head / (nh / nkv);
-  const int n_qb = (t + 31) / 32;
-  const int qb = GROUPS == 1 ? n_qb - 1 - (int)blockIdx.x : (group == 0 ? n_qb - 1 - (int)blockIdx.x : (int)blockIdx.x);
-  const bool idle = GROUPS == 2 && group == 1 && qb == n_qb - 1 - qb;
-  float (*merge_ml)[2][64] = merge_ml_all[group];
-  float (*merge_o)[64] = merge_o_all[group][0];
+  const int n_bkv = gridDim.x / (nh / nkv), bkv = blockIdx.x % n_bkv, b = bkv / nkv, kvh = bkv % nkv, head = kvh * (nh / nkv) + blockIdx.x / n_bkv;
+  const int n_qb = (t + 31) / 32, qb = n_qb - 1 - (int)(blockIdx.z * gridDim.y + blockIdx.y);
+  if (qb < 0) return;
   const int q0 = qb * 32;
   const int qi = min(q0 + col, t - 1);
   const int q_pos = s - t + qi;
   const int last_pos = s - t + min(q0 + 31, t - 1);
   const int q_pos_min = s - t + min(q0, t - 1);
   const att_u32x4* pl = planes + ((size_t)b * nkv + kvh) * (size_t)n_kb * ATT_PLANE_BLOCK + lane;
-  const int n_blocks = idle ? 0 : last_pos / 32 + 1;
+  const int n_blocks = last_pos / 32 + 1;
 
   // K operands of this wave's first block set out before the query row is touched
   att_u32x4 kop[3][4], vop[3][DB][2];
@@ -995,47 +998,45 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) attention_prefill_x6_kernel(c
         for (int e = 0; e < DB; ++e) o[e] = att_mma_bf16(vop[TA[term]][e][st], pop[TB[term]][st], o[e]);
   }
 
-  // merge the four waves' partial results in wave order
-  if (wave != 0) {
-    merge_ml[wave - 1][0][lane] = m_run;
-    merge_ml[wave - 1][1][lane] = l_half;
-#pragma unroll
-    for (int e = 0; e < DB; ++e)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) merge_o[(wave - 1) * DB * 16 + e * 16 + r][lane] = o[e][r];
-  }
-  __syncthreads();
-  if (wave != 0 || idle) return;
-  float m_tot = m_run;
-#pragma unroll
-  for (int w = 0; w < 3; ++w) m_tot = fmaxf(m_tot, merge_ml[w][0][lane]);
-  float f = __builtin_amdgcn_exp2f(m_run - m_tot);
-  float l_tot = l_half * f;
+  // The four waves' partial results meet in wave order.  Thread: eight elements of a row, so that a row's stores are one piece.
+  merge_ml[wave][0][lane] = m_run;
+  merge_ml[wave][1][lane] = l_half;
 #pragma unroll
   for (int e = 0; e < DB; ++e)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[e][r] *= f;
+    for (int r = 0; r < 16; ++r) merge_o[wave][e * 16 + r][lane] = o[e][r];
+  __syncthreads();
+  const int row = tid >> 3, d0 = (tid & 7) * 8, r0 = (tid & 7) * 4;  // elements d0 .. + 3 of row `row`: registers r0 .. + 3 of lane `row`; the next four: of lane row + 32
+  float m_tot = merge_ml[0][0][row];
 #pragma unroll
-  for (int w = 0; w < 3; ++w) {
-    f = __builtin_amdgcn_exp2f(merge_ml[w][0][lane] - m_tot);
-    l_tot += merge_ml[w][1][lane] * f;
+  for (int w = 1; w < 4; ++w) m_tot = fmaxf(m_tot, merge_ml[w][0][row]);
+  float l0 = 0.f, l1 = 0.f, y[8];
 #pragma unroll
-    for (int e = 0; e < DB; ++e)
+  for (int i = 0; i < 8; ++i) y[i] = 0.f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) o[e][r] += merge_o[w * DB * 16 + e * 16 + r][lane] * f;
+  for (int w = 0; w < 4; ++w) {
+    const float f = __builtin_amdgcn_exp2f(merge_ml[w][0][row] - m_tot);
+    l0 += merge_ml[w][1][row] * f;
+    l1 += merge_ml[w][1][row + 32] * f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] += merge_o[w][r0 + (i & 3)][row + (i >> 2) * 32] * f;
   }
-  l_tot += __shfl_xor(l_tot, 32, 64);
-  if (q0 + col < t) {
-    const size_t row = (size_t)b * t + qi, width = (size_t)nh * D;
-    float* orow = dst + row * width + (size_t)head * D;
+  if (q0 + row >= t) return;
+  const float l_tot = l0 + l1;
 #pragma unroll
-    for (int e = 0; e < DB; ++e)
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const float y[4] = {o[e][a * 4] / l_tot, o[e][a * 4 + 1] / l_tot, o[e][a * 4 + 2] / l_tot, o[e][a * 4 + 3] / l_tot};
-        if (dst_planes) split3_store4(y, dst_planes + row * 3 * width, (size_t)head * D + e * 32 + a * 8 + hh * 4);
-        else *reinterpret_cast<float4*>(orow + e * 32 + a * 8 + hh * 4) = make_float4(y[0], y[1], y[2], y[3]);
-      }
+  for (int i = 0; i < 8; ++i) y[i] /= l_tot;
+  const size_t width = (size_t)nh * D, to = (size_t)b * t + q0 + row;
+  if (dst_planes) {
+    att_u32x4 hi, mid, lo;
+    att_split8(y, hi, mid, lo);
+    uint16_t* x3 = dst_planes + to * 3 * width + (size_t)head * 3 * D + d0;  // a head is one K tile of the product: its three planes side by side
+    *reinterpret_cast<att_u32x4*>(x3) = hi;
+    *reinterpret_cast<att_u32x4*>(x3 + 64) = mid;
+    *reinterpret_cast<att_u32x4*>(x3 + 128) = lo;
+  } else {
+    float* out = dst + to * width + (size_t)head * D + d0;
+    *reinterpret_cast<float4*>(out) = make_float4(y[0], y[1], y[2], y[3]);
+    *reinterpret_cast<float4*>(out + 4) = make_float4(y[4], y[5], y[6], y[7]);
   }
 }
 
@@ -1349,10 +1350,9 @@ static int attention_prefill_launch(ughip_device* dev, const ughip_slice* q, siz
     att_u32x4* planes = reinterpret_cast<att_u32x4*>(ws);
     att_planes_kernel<<<dim3((unsigned)n_kb, (unsigned)bkv), 256, 0, dev->stream>>>(kp, vp, planes, is, cap);
     UGHIP_HIPCHK(hipGetLastError());
-    if (pair)
-      attention_prefill_x6_kernel<2><<<paired, 512, 0, dev->stream>>>(qp, planes, op, out_planes, inh, inkv, it, is, (int)n_kb, q_row_stride, scale, cp, sp, pp, tl, interleaved);
-    else
-      attention_prefill_x6_kernel<1><<<single, 256, 0, dev->stream>>>(qp, planes, op, out_planes, inh, inkv, it, is, (int)n_kb, q_row_stride, scale, cp, sp, pp, tl, interleaved);
+    const unsigned z = (n_qb + 65534) / 65535;
+    attention_prefill_x6_kernel<<<dim3((unsigned)(b * n_heads), (n_qb + z - 1) / z, z), 256, 0, dev->stream>>>(qp, planes, op, out_planes, inh, inkv, it, is, (int)n_kb, q_row_stride, scale, cp, sp,
+                                                                                                           pp, tl, interleaved);
     UGHIP_HIPCHK(hipGetLastError());
     if (wrote_planes) *wrote_planes = out_planes != nullptr;
     return UGHIP_OK;
