@@ -740,34 +740,17 @@ __global__ void __launch_bounds__(256 * GROUPS) attention_prefill_kernel(const f
 //       from where they are (as in the kernel above).
 // Keys past s are planes of zeros.
 typedef __bf16 att_bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 att_bf16x2 __attribute__((ext_vector_type(2)));
-typedef float att_f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned att_u32x4 __attribute__((ext_vector_type(4)));
 constexpr int ATT_PLANE_BLOCK = 1536;  // 16-byte units per block of 32 keys: 2 x 3 planes x 4 operands x 64 lanes
 constexpr int ATT_MERGE_ROW = 66;      // floats from one register's 64 lanes to the next: four registers on, 8 banks on
 
-// (x0, x1) -> three words of two bf16 each (x0 in the low half); remainders are exact f32 subtractions.  An infinity or a
-// NaN stays whole in the first term (FINITE: the caller knows there is no infinity, e.g. among the exponentials of a softmax;
-// a NaN then gives three NaNs).
-template <bool FINITE = false>
-__device__ __forceinline__ void att_split_pair(float x0, float x1, unsigned& hi, unsigned& mid, unsigned& lo) {
-  const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(att_f32x2{x0, x1}, att_bf16x2));
-  float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
-  if (!FINITE) {
-    if ((h & 0x7f80u) == 0x7f80u) r0 = 0.f;
-    if ((h & 0x7f800000u) == 0x7f800000u) r1 = 0.f;
-  }
-  const unsigned m = __builtin_bit_cast(unsigned, __builtin_convertvector(att_f32x2{r0, r1}, att_bf16x2));
-  const float q0 = r0 - __uint_as_float(m << 16), q1 = r1 - __uint_as_float(m & 0xffff0000u);
-  hi = h, mid = m, lo = __builtin_bit_cast(unsigned, __builtin_convertvector(att_f32x2{q0, q1}, att_bf16x2));
-}
 // eight values -> one operand per plane
 template <bool FINITE = false>
 __device__ __forceinline__ void att_split8(const float (&x)[8], att_u32x4& hi, att_u32x4& mid, att_u32x4& lo) {
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
     unsigned h, md, l;
-    att_split_pair<FINITE>(x[2 * m], x[2 * m + 1], h, md, l);
+    split3_pair<FINITE>(x[2 * m], x[2 * m + 1], h, md, l);
     hi[m] = h, mid[m] = md, lo[m] = l;
   }
 }

@@ -15,28 +15,36 @@ __device__ __forceinline__ uint16_t bf16_rne(float f) {
   if ((x & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((x >> 16) | 0x40u);  // NaN stays NaN
   return (uint16_t)((x + 0x7fffu + ((x >> 16) & 1u)) >> 16);
 }
-// hi + mid + lo of one value
-__device__ __forceinline__ void split3(float x, uint16_t& hi, uint16_t& mid, uint16_t& lo) {
-  hi = bf16_rne(x);
-  const float h = __uint_as_float((uint32_t)hi << 16);
-  // an infinity (given, or reached when |x| rounds up past the largest bf16) or a NaN is all in the first term: the
-  // remainders would be inf - inf, and the product has to give what the f32 pipe gives for such an x
-  const bool fin = (hi & 0x7f80) != 0x7f80;
-  const float r1 = fin ? x - h : 0.f;  // exact: hi shares the leading bits of x
-  mid = bf16_rne(r1);
-  const float r2 = r1 - __uint_as_float((uint32_t)mid << 16);
-  lo = bf16_rne(r2);
+// Two values -> three words of two bf16 each (x0 in the low half); remainders are exact f32 subtractions.  An infinity (given, or
+// reached when |x| rounds up past the largest bf16) or a NaN is all in the first term: the remainders would be inf - inf, and the
+// product has to give what the f32 pipe gives for such an x (FINITE: the caller knows there is no infinity, e.g. among the
+// exponentials of a softmax; a NaN then gives three NaNs).  The conversions round two values at once and branch nowhere: a norm
+// of 1900 rows of 2048 to planes 9.7 -> 7.9 us, a gated fold of 1900 rows of 2 x 5632 36.2 -> 34.8 us against integer rounding with a branch
+// for NaN.
+typedef __bf16 split_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float split_f32x2 __attribute__((ext_vector_type(2)));
+template <bool FINITE = false>
+__device__ __forceinline__ void split3_pair(float x0, float x1, unsigned& hi, unsigned& mid, unsigned& lo) {
+  const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(split_f32x2{x0, x1}, split_bf16x2));
+  float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
+  if (!FINITE) {
+    if ((h & 0x7f80u) == 0x7f80u) r0 = 0.f;
+    if ((h & 0x7f800000u) == 0x7f800000u) r1 = 0.f;
+  }
+  const unsigned m = __builtin_bit_cast(unsigned, __builtin_convertvector(split_f32x2{r0, r1}, split_bf16x2));
+  const float q0 = r0 - __uint_as_float(m << 16), q1 = r1 - __uint_as_float(m & 0xffff0000u);
+  hi = h, mid = m, lo = __builtin_bit_cast(unsigned, __builtin_convertvector(split_f32x2{q0, q1}, split_bf16x2));
 }
 
 // Four consecutive elements of a row of k, split, to their places in the row's planes (x3_row: the row's first element).
 __device__ __forceinline__ void split3_store4(const float in[4], uint16_t* __restrict__ x3_row, size_t col) {
-  uint16_t hi[4], mid[4], lo[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) split3(in[i], hi[i], mid[i], lo[i]);
+  uint2 hi, mid, lo;
+  split3_pair(in[0], in[1], hi.x, mid.x, lo.x);
+  split3_pair(in[2], in[3], hi.y, mid.y, lo.y);
   uint16_t* o = x3_row + (col / 64) * 192 + col % 64;
-  *reinterpret_cast<ushort4*>(o) = make_ushort4(hi[0], hi[1], hi[2], hi[3]);
-  *reinterpret_cast<ushort4*>(o + 64) = make_ushort4(mid[0], mid[1], mid[2], mid[3]);
-  *reinterpret_cast<ushort4*>(o + 128) = make_ushort4(lo[0], lo[1], lo[2], lo[3]);
+  *reinterpret_cast<uint2*>(o) = hi;
+  *reinterpret_cast<uint2*>(o + 64) = mid;
+  *reinterpret_cast<uint2*>(o + 128) = lo;
 }
 
 }  // namespace ughip

@@ -655,13 +655,13 @@ __global__ void __launch_bounds__(256) split3_operands_kernel(const float* __res
   if (lhs || !b_kn) {
     split3_store4(in, x3 + row * 3 * w, col);
   } else {
-    uint16_t hi[4], mid[4], lo[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) split3(in[i], hi[i], mid[i], lo[i]);
+    uint2 hi, mid, lo;
+    split3_pair(in[0], in[1], hi.x, mid.x, lo.x);
+    split3_pair(in[2], in[3], hi.y, mid.y, lo.y);
     uint16_t* o = x3 + ((row / 64) * 192 + row % 64) * w + col;
-    *reinterpret_cast<ushort4*>(o) = make_ushort4(hi[0], hi[1], hi[2], hi[3]);
-    *reinterpret_cast<ushort4*>(o + 64 * w) = make_ushort4(mid[0], mid[1], mid[2], mid[3]);
-    *reinterpret_cast<ushort4*>(o + 128 * w) = make_ushort4(lo[0], lo[1], lo[2], lo[3]);
+    *reinterpret_cast<uint2*>(o) = hi;
+    *reinterpret_cast<uint2*>(o + 64 * w) = mid;
+    *reinterpret_cast<uint2*>(o + 128 * w) = lo;
   }
 }
 
