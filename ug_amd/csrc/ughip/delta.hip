@@ -84,7 +84,7 @@ struct DeltaArgs {
 
 template <int C>
 __host__ __device__ constexpr size_t prepare_lds_floats(int dp) {
-  return (size_t)3 * C * (dp + 4) + (size_t)C * (C + 4) + C;
+  return (size_t)2 * C * (dp + 4) + (size_t)(C / 16) * (C / 16 + 1) / 2 * 256 + 2 * C;
 }
 
 // four elements of a row, zeros from `left` on
@@ -102,53 +102,68 @@ template <int C>
 constexpr int prepare_threads() {
   return C == 64 ? 512 : 256;
 }
+// The queries stay in memory: they are read where they are used, times their rows' factors.  What is left in LDS of 64 rows of 128
+// channels (77 KB) is two workgroups to a CU; bound by vector instructions.  2048 positions of
+// 16 heads: 69 us with one workgroup to a CU, 62 us so.
 template <int C, bool VEC>
-__global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(DeltaArgs a) {
+__global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) delta_prepare_kernel(DeltaArgs a) {
   constexpr int NB = C / 16, NT = prepare_threads<C>(), NW = NT / 64;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int dp = a.dp, ds = dp + 4, chunk = blockIdx.x, h = blockIdx.y, g = h / (a.heads / a.kv_heads), row0 = chunk * C, rows = min(C, a.t - row0), d = a.dim;
   float* K = lds;             // [C][ds]
-  float* Q = K + C * ds;      // [C][ds]
-  float* B = Q + C * ds;      // [C][ds]: log2 of the decays, summed from the start of a block of 16 rows
-  float* A = B + C * ds;      // [C][C + 4]: A, then the inverses of I + A in the diagonal blocks
-  float* beta = A + C * (C + 4);
-  constexpr int as = C + 4;
+  float* B = K + C * ds;      // [C][ds]: log2 of the decays, summed from the start of a block of 16 rows
+  float* A = B + C * ds;      // left operands of A up to the diagonal, then the inverses of I + A in the diagonal blocks
+  float* beta = A + NB * (NB + 1) / 2 * 256;
+  float* unit = beta + C;     // what makes a query a unit vector, scaled; 0 past the last row
   const size_t at = (size_t)chunk * a.heads + h;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, kg = lane >> 4;
   const int d4 = dp / 4;
   const float neg = -expf(a.a_log[h]) * LOG2E;
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  for (int e = threadIdx.x; e < C * d4; e += NT) {
-    const int r = e / d4, c = (e - r * d4) * 4;
-    f32x4_t k = zero, q = zero, l = zero;
-    if (r < rows && c < d) {
-      const float* row = a.qkv + (size_t)(row0 + r) * a.qkv_stride + (size_t)g * d + c;
-      q = four<VEC>(row, d - c), k = four<VEC>(row + (size_t)a.kv_heads * d, d - c);
-      l = four<VEC>(a.a + (size_t)(row0 + r) * a.a_stride + (size_t)h * d + c, d - c);
-      const f32x4_t bias = four<VEC>(a.dt_bias + (size_t)h * d + c, d - c);
+  constexpr int AT_ONCE = 4;  // pieces of a thread on their way together: the decays' logarithms are long, and a load behind them would come late
+  for (int e0 = threadIdx.x; e0 < C * d4; e0 += AT_ONCE * NT) {
+    f32x4_t k[AT_ONCE], l[AT_ONCE], bias[AT_ONCE];
 #pragma unroll
-      for (int x = 0; x < 4; ++x) l[x] = c + x < d ? neg * softplus_f(l[x] + bias[x]) : 0.f;
+    for (int u = 0; u < AT_ONCE; ++u) {
+      const int e = e0 + u * NT, r = e / d4, c = (e - r * d4) * 4, rr = min(r, rows - 1);
+      k[u] = l[u] = bias[u] = zero;
+      if (c < d) {
+        k[u] = four<VEC>(a.qkv + (size_t)(row0 + rr) * a.qkv_stride + (size_t)(a.kv_heads + g) * d + c, d - c);
+        l[u] = four<VEC>(a.a + (size_t)(row0 + rr) * a.a_stride + (size_t)h * d + c, d - c);
+        bias[u] = four<VEC>(a.dt_bias + (size_t)h * d + c, d - c);
+      }
     }
-    *reinterpret_cast<f32x4_t*>(K + r * ds + c) = k;
-    *reinterpret_cast<f32x4_t*>(Q + r * ds + c) = q;
-    *reinterpret_cast<f32x4_t*>(B + r * ds + c) = l;
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u) {
+      const int e = e0 + u * NT, r = e / d4, c = (e - r * d4) * 4;
+      if (e >= C * d4) break;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) l[u][x] = r < rows && c + x < d ? neg * softplus_f(l[u][x] + bias[u][x]) : 0.f;
+      *reinterpret_cast<f32x4_t*>(K + r * ds + c) = r < rows ? k[u] : zero;
+      *reinterpret_cast<f32x4_t*>(B + r * ds + c) = l[u];
+    }
   }
   if (threadIdx.x < C) beta[threadIdx.x] = (int)threadIdx.x < rows ? exact_sigmoid(a.b[(size_t)(row0 + threadIdx.x) * a.b_stride + h]) : 0.f;
   __syncthreads();
+  // a query's four elements from c on, zeros past its last one
+  auto query = [&](int r, int c) {
+    const float* row = a.qkv + (size_t)(row0 + min(r, rows - 1)) * a.qkv_stride + (size_t)g * d;
+    if constexpr (VEC) return c < d ? *reinterpret_cast<const f32x4_t*>(row + c) : zero;
+    else return four<false>(row + c, d - c);
+  };
   // unit vectors: 16 lanes per row
   const float q_scale = 1.f / sqrtf((float)d);
   for (int r = wave * 4 + kg; r < C; r += 4 * NW) {
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      float* row = (m ? Q : K) + r * ds;
-      float ss = 0.f;
-      for (int c = j * 4; c < dp; c += 64) {
-        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(row + c);
-        ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-      }
-      const float f = (m ? q_scale : 1.f) / sqrtf(row_sum16(ss) + UNIT_EPS);
-      for (int c = j * 4; c < dp; c += 64) *reinterpret_cast<f32x4_t*>(row + c) *= f;
+    float* row = K + r * ds;
+    float ss = 0.f, sq = 0.f;
+    for (int c = j * 4; c < dp; c += 64) {
+      const f32x4_t q = query(r, c), v = *reinterpret_cast<const f32x4_t*>(row + c);
+      ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+      sq += q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
     }
+    const float f = 1.f / sqrtf(row_sum16(ss) + UNIT_EPS), fq = q_scale / sqrtf(row_sum16(sq) + UNIT_EPS);
+    for (int c = j * 4; c < dp; c += 64) *reinterpret_cast<f32x4_t*>(row + c) *= f;
+    if (j == 0) unit[r] = r < rows ? fq : 0.f;
   }
   for (int x = threadIdx.x; x < dp * NB; x += NT) {
     float* col = B + (x / dp) * 16 * ds + x % dp;
@@ -160,6 +175,7 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
 
   float* P = a.p + at * C * C;
   auto row4 = [&](const float* m, int r, int c) { return *reinterpret_cast<const f32x4_t*>(m + r * ds + c); };
+  auto tile_a = [&](int I, int J) { return A + (I * (I + 1) / 2 + J) * 256; };
   // a pair of blocks per wave and turn, those of a block with itself first
   for (int n = wave; n < NB * (NB + 1) / 2; n += NW) {
     int I = n, J = n;
@@ -167,6 +183,7 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
       I = 1;
       for (J = n - NB; J >= I; ++I) J -= I;
     }
+    const float uq = unit[16 * I + j];
     if (J < I) {
       f32x4_t acc[4] = {zero, zero, zero, zero};
       for (int c = 4 * kg; c < dp; c += 32) {
@@ -179,7 +196,7 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
           for (int M = J + 1; M < I; ++M) rest += row4(B, 16 * M + 15, cc);
           y[2 * u] = y[2 * u + 1] = row4(K, 16 * J + j, cc) * exp2_4(rest);
           x[2 * u] = row4(K, 16 * I + j, cc) * left;
-          x[2 * u + 1] = row4(Q, 16 * I + j, cc) * left;
+          x[2 * u + 1] = query(16 * I + j, cc) * uq * left;
         }
         mfma16x16_each(x, y, acc);
       }
@@ -187,7 +204,7 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 16 * I + 4 * kg + e;
-        A[i * as + 16 * J + j] = ak[e] * beta[i];
+        tile_a(I, J)[left_at(4 * kg + e, j)] = ak[e] * beta[i];
         P[(I * NB + J) * 256 + left_at(4 * kg + e, j)] = aq[e];
       }
       continue;
@@ -206,7 +223,7 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
           const f32x4_t l = row4(B, 16 * I + j, cc), k = row4(K, 16 * I + j, cc), left = exp2_4(l);
           y[2 * u] = y[2 * u + 1] = k * exp2_4(-l);
           x[2 * u] = k * left;
-          x[2 * u + 1] = row4(Q, 16 * I + j, cc) * left;
+          x[2 * u + 1] = query(16 * I + j, cc) * uq * left;
         }
         mfma16x16_each(x, y, acc);
       }
@@ -214,7 +231,7 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 4 * kg + e, row = 16 * I + i;
-        A[row * as + 16 * I + j] = j < i ? ak[e] * beta[row] : 0.f;
+        tile_a(I, I)[left_at(i, j)] = j < i ? ak[e] * beta[row] : 0.f;
         P[(I * NB + I) * 256 + left_at(i, j)] = j <= i ? aq[e] : 0.f;
       }
       continue;
@@ -223,7 +240,7 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
     float ak[4] = {0.f, 0.f, 0.f, 0.f}, aq[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 2
     for (int c = 0; c < dp; c += 4) {
-      const f32x4_t ki = row4(K, 16 * I + j, c), qi = row4(Q, 16 * I + j, c), bi = row4(B, 16 * I + j, c);
+      const f32x4_t ki = row4(K, 16 * I + j, c), qi = query(16 * I + j, c) * uq, bi = row4(B, 16 * I + j, c);
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         const f32x4_t kj = row4(K, 16 * I + 4 * kg + x, c);
@@ -239,7 +256,7 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       const int jj = 4 * kg + x;
-      A[(16 * I + j) * as + 16 * I + jj] = jj < j ? ak[x] * bt : 0.f;
+      tile_a(I, I)[left_at(j, jj)] = jj < j ? ak[x] * bt : 0.f;
       P[(I * NB + I) * 256 + left_at(j, jj)] = jj <= j ? aq[x] : 0.f;
     }
   }
@@ -247,26 +264,22 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
 
   // the inverses of the diagonal blocks, a column per lane
   if (wave < NB && lane < 16) {
-    float* block = A + 16 * wave * as + 16 * wave;
+    float* block = tile_a(wave, wave);
     float x[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       float v = i == lane ? 1.f : 0.f;
 #pragma unroll
-      for (int m = 0; m < i; ++m) v -= block[i * as + m] * x[m];
+      for (int m = 0; m < i; ++m) v -= block[left_at(i, m)] * x[m];
       x[i] = v;
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) block[i * as + lane] = x[i];
+    for (int i = 0; i < 16; ++i) block[left_at(i, lane)] = x[i];
   }
   __syncthreads();
   // (I + A) X = right-hand side, 16 columns per wave and turn: first the channels of beta G K, then the columns of beta V
   {
-    f32x4_t m[NB][NB];
-#pragma unroll
-    for (int I = 0; I < NB; ++I)
-#pragma unroll
-      for (int J = 0; J <= I; ++J) m[I][J] = *reinterpret_cast<const f32x4_t*>(A + (16 * I + j) * as + 16 * J + 4 * kg);
+    auto m = [&](int I, int J) { return tile_of(A, I * (I + 1) / 2 + J, lane); };
     const float* values = a.qkv + (size_t)row0 * a.qkv_stride + (size_t)2 * a.kv_heads * d + (size_t)h * a.vdim;
     const int kt = dp / 16, all = kt + a.vp / 16;
     f32x4_t ahead[NB];
@@ -274,10 +287,12 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
       if (tile < kt || tile >= all) return;  // uniform over the wave
       const int c = (tile - kt) * 16 + j;
       const float* col = values + (c < a.vdim ? c : 0);
+      size_t stride = a.qkv_stride;
+      asm volatile("" : "+s"(stride));  // (16 rows' addresses held over the loop would not leave registers for two workgroups)
 #pragma unroll
       for (int I = 0; I < NB; ++I)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ahead[I][e] = col[(size_t)min(16 * I + 4 * kg + e, rows - 1) * a.qkv_stride];
+        for (int e = 0; e < 4; ++e) ahead[I][e] = col[(size_t)min(16 * I + 4 * kg + e, rows - 1) * stride];
     };
     fetch(wave);
     for (int tile = wave; tile < all; tile += NW) {
@@ -309,13 +324,17 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
         f32x4_t acc[NB];
 #pragma unroll
         for (int J = 0; J < I; ++J) acc[J] = zero;
+        f32x4_t mi[NB];
+        asm volatile("" ::: "memory");  // (read again for every tile: held over the loop they would not leave registers for two workgroups)
+#pragma unroll
+        for (int J = 0; J <= I; ++J) mi[J] = m(I, J);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int J = 0; J < I; ++J) acc[J] = mfma16(m[I][J][e], x[J][e], acc[J]);
+          for (int J = 0; J < I; ++J) acc[J] = mfma16(mi[J][e], x[J][e], acc[J]);
 #pragma unroll
         for (int J = 0; J < I; ++J) x[I] -= acc[J];
-        x[I] = mfma16x16(m[I][I], x[I], zero);
+        x[I] = mfma16x16(mi[I], x[I], zero);
         if (tile < kt) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) W[(I * kt + tile) * 256 + left_at(4 * kg + e, j)] = x[I][e];
@@ -331,7 +350,7 @@ __global__ void __launch_bounds__((prepare_threads<C>())) delta_prepare_kernel(D
     const int tile = e / 64, r = tile / (dp / 16) * 16 + (e & 15), c = tile % (dp / 16) * 16 + (e >> 4 & 3) * 4;
     f32x4_t l = row4(B, r, c);
     for (int M = 0; M < r / 16; ++M) l += row4(B, 16 * M + 15, c);
-    *reinterpret_cast<f32x4_t*>(QG + 4 * e) = row4(Q, r, c) * exp2_4(l);
+    *reinterpret_cast<f32x4_t*>(QG + 4 * e) = query(r, c) * unit[r] * exp2_4(l);
   }
   float* KD = a.kd + at * C * dp;
   for (int e = threadIdx.x; e < C * d4; e += NT) {
