@@ -269,22 +269,46 @@ __global__ void __launch_bounds__(256) ssm_chunk_scan_kernel(SsmArgs a) {
   a.s[h * per + e] = s;
 }
 
-template <bool VEC>
-__global__ void __launch_bounds__(256) ssm_chunk_out_kernel(SsmArgs a) {
+// NC > 0: states of up to 16 NC rows, whose C a wave holds in registers (its own 16 rows are all that it reads): what is left in LDS at
+// 64 positions and 128 rows is 69 KB, two workgroups to a CU, of which one loads while the other multiplies.  512 positions of 64 heads
+// on 8 groups: 37 us with C in LDS (103 KB) and one workgroup to a CU, 24.3 us so.  0: any state, C in LDS.
+template <bool VEC, int NC>
+__global__ void __launch_bounds__(256, 2) ssm_chunk_out_kernel(SsmArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int q = a.q, chunk = blockIdx.x, row0 = chunk * q, rows = min(q, a.t - row0), N = a.state, ns = row_n(N), np = pad16(N), gs = q + 4, inner = a.heads * a.vdim;
   const HeadWalk hw(a);
   float* cum = lds;
   float* d = lds + 64;
   float* Cs = lds + 128;      // [q][ns]
-  float* Gs = Cs + q * ns;    // [q][gs]: C_i . B_j
+  float* Gs = NC ? Cs : Cs + q * ns;  // [q][gs]: C_i . B_j
   float* Bs = Gs + q * gs;    // [q][ns], then
   float* Xs = Bs;             // [q][PS]
   float* Ss = Xs + q * PS;    // [np][PS]
   const float* xbc0 = a.xbc + (size_t)row0 * a.xbc_stride;
   const float *b_src = xbc0 + inner + (size_t)hw.g * N, *c_src = xbc0 + inner + (size_t)(a.groups + hw.g) * N;
-  const int bt = q * np / 4;
-  if (bt <= 8 * 256) {
+  const int bt = q * np / 4, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, kg = lane >> 4, tq = q / 16, i0 = wave * 16;
+  f32x4_t cf[NC ? NC : 1];  // elements 16 n + 4 kg .. of C's row i0 + j
+  if constexpr (NC > 0) {
+    static_assert(NC <= 8, "B in one piece");
+    TileRegs<8, VEC> b;
+    b.load(b_src, a.xbc_stride, rows, N, np / 4, bt);
+    const bool there = i0 + j < rows;
+    const float* row = c_src + (size_t)(there ? i0 + j : 0) * a.xbc_stride;
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      const int k = 16 * n + 4 * kg;
+      if (VEC) {  // every lane loads
+        cf[n] = *reinterpret_cast<const f32x4_t*>(row + (k < N ? k : 0));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cf[n][e] = k + e < N ? row[k + e] : 0.f;
+      }
+    }
+    b.store(Bs, ns, np / 4, bt);
+#pragma unroll
+    for (int n = 0; n < NC; ++n)
+      if (!there || 16 * n + 4 * kg >= N) cf[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  } else if (bt <= 8 * 256) {
     TileRegs<8, VEC> b, c;  // both on their way at once
     b.load(b_src, a.xbc_stride, rows, N, np / 4, bt);
     c.load(c_src, a.xbc_stride, rows, N, np / 4, bt);
@@ -294,7 +318,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_out_kernel(SsmArgs a) {
     tile_to_lds<VEC>(Bs, ns, b_src, a.xbc_stride, rows, N, np / 4, bt);
     tile_to_lds<VEC>(Cs, ns, c_src, a.xbc_stride, rows, N, np / 4, bt);
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, kg = lane >> 4, tq = q / 16, i0 = wave * 16, xt = q * PB / 4, st = np * PB / 4;
+  const int xt = q * PB / 4, st = np * PB / 4;
   TileRegs<4, VEC> x;
   TileRegs<8, VEC> s;
   float decays = 0.f;  // A of row `lane` (first wave), d of it (second)
@@ -304,15 +328,25 @@ __global__ void __launch_bounds__(256) ssm_chunk_out_kernel(SsmArgs a) {
     x.load(xbc0 + (size_t)hw.head(i) * a.vdim + hw.col(i), a.xbc_stride, rows, pw, PB / 4, xt);
     s.load(a.chunk_s + ((size_t)chunk * a.heads + hw.head(i)) * N * a.vdim + hw.col(i), a.vdim, N, pw, PB / 4, st);
   };
+  auto each_c = [&](auto f) {
+    if constexpr (NC > 0) {
+#pragma unroll
+      for (int n = 0; n < NC; ++n) {
+        if (16 * n >= np) break;
+        f(16 * n + 4 * kg, cf[n]);
+      }
+    } else {
+#pragma unroll 2
+      for (int k = 4 * kg; k < np; k += 16) f(k, *reinterpret_cast<const f32x4_t*>(Cs + (i0 + j) * ns + k));
+    }
+  };
   if (hw.items) fetch(0);
   __syncthreads();
   if (wave < tq) {
     f32x4_t acc[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) acc[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int k = 4 * kg; k < np; k += 16) {  // k four elements per lane at a time: 16-byte reads
-      const f32x4_t c = *reinterpret_cast<const f32x4_t*>(Cs + (i0 + j) * ns + k);
+    each_c([&](int k, const f32x4_t& c) {  // k four elements per lane at a time: 16-byte reads
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         if (u > wave) break;  // columns past the row tile are not used
@@ -322,7 +356,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_out_kernel(SsmArgs a) {
         acc[u] = mfma16(c.z, b.z, acc[u]);
         acc[u] = mfma16(c.w, b.w, acc[u]);
       }
-    }
+    });
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (u < tq)
@@ -352,9 +386,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_out_kernel(SsmArgs a) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) in_chunk[u] = mfma16(m, Xs[k * PS + u * 16 + j], in_chunk[u]);
     }
-#pragma unroll 2
-    for (int k = 4 * kg; k < np; k += 16) {
-      const f32x4_t c = *reinterpret_cast<const f32x4_t*>(Cs + (i0 + j) * ns + k);
+    each_c([&](int k, const f32x4_t& c) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         from_s[u] = mfma16(c.x, Ss[k * PS + u * 16 + j], from_s[u]);
@@ -362,7 +394,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_out_kernel(SsmArgs a) {
         from_s[u] = mfma16(c.z, Ss[(k + 2) * PS + u * 16 + j], from_s[u]);
         from_s[u] = mfma16(c.w, Ss[(k + 3) * PS + u * 16 + j], from_s[u]);
       }
-    }
+    });
     const float skip = a.skip[h];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -540,7 +572,8 @@ extern "C" int ughip_ssm_rows(ughip_device* dev, ughip_view xbc, ughip_view dt, 
   static const hipError_t attr = [] {
     hipError_t e = hipSuccess;
     for (const void* f : {reinterpret_cast<const void*>(ssm_chunk_state_kernel<true>), reinterpret_cast<const void*>(ssm_chunk_state_kernel<false>),
-                          reinterpret_cast<const void*>(ssm_chunk_out_kernel<true>), reinterpret_cast<const void*>(ssm_chunk_out_kernel<false>)})
+                          reinterpret_cast<const void*>(ssm_chunk_out_kernel<true, 8>), reinterpret_cast<const void*>(ssm_chunk_out_kernel<false, 8>),
+                          reinterpret_cast<const void*>(ssm_chunk_out_kernel<true, 0>), reinterpret_cast<const void*>(ssm_chunk_out_kernel<false, 0>)})
       if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     return e;
   }();
@@ -550,8 +583,14 @@ extern "C" int ughip_ssm_rows(ughip_device* dev, ughip_view xbc, ughip_view dt, 
   if (vec) ssm_chunk_state_kernel<true><<<grid, 256, lds_s, dev->stream>>>(a);
   else ssm_chunk_state_kernel<false><<<grid, 256, lds_s, dev->stream>>>(a);
   ssm_chunk_scan_kernel<<<dim3((unsigned)((elems + 255) / 256), (unsigned)heads), 256, 0, dev->stream>>>(a);
-  if (vec) ssm_chunk_out_kernel<true><<<grid, 256, lds_o, dev->stream>>>(a);
-  else ssm_chunk_out_kernel<false><<<grid, 256, lds_o, dev->stream>>>(a);
+  const size_t lds_c = (size_t)q * row_n((int)state) * sizeof(float);  // C's part of lds_o
+  if (state <= 128) {
+    if (vec) ssm_chunk_out_kernel<true, 8><<<grid, 256, lds_o - lds_c, dev->stream>>>(a);
+    else ssm_chunk_out_kernel<false, 8><<<grid, 256, lds_o - lds_c, dev->stream>>>(a);
+  } else {
+    if (vec) ssm_chunk_out_kernel<true, 0><<<grid, 256, lds_o, dev->stream>>>(a);
+    else ssm_chunk_out_kernel<false, 0><<<grid, 256, lds_o, dev->stream>>>(a);
+  }
   UGHIP_HIPCHK(hipGetLastError());
   return UGHIP_OK;
 }
