@@ -38,9 +38,16 @@ __device__ __forceinline__ void split3_pair(float x0, float x1, unsigned& hi, un
 
 // Four consecutive elements of a row of k, split, to their places in the row's planes (x3_row: the row's first element).
 __device__ __forceinline__ void split3_store4(const float in[4], uint16_t* __restrict__ x3_row, size_t col) {
+  // the terms of the f32 value, as if it had been stored: a product in front of this must not be fused into the first remainder
+  float x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = in[i];
+    asm("" : "+v"(x[i]));
+  }
   uint2 hi, mid, lo;
-  split3_pair(in[0], in[1], hi.x, mid.x, lo.x);
-  split3_pair(in[2], in[3], hi.y, mid.y, lo.y);
+  split3_pair(x[0], x[1], hi.x, mid.x, lo.x);
+  split3_pair(x[2], x[3], hi.y, mid.y, lo.y);
   uint16_t* o = x3_row + (col / 64) * 192 + col % 64;
   *reinterpret_cast<uint2*>(o) = hi;
   *reinterpret_cast<uint2*>(o + 64) = mid;

@@ -525,7 +525,7 @@ static double ring_cost_us(size_t tiles, int kt, int tile, bool streamed) {
 // (3072 x 4096^2: 131 -> 91 us, 5120^2 x 1024: 77 -> 54, 1280 x 8192 x 2048: 64 -> 47, 2048 x 2560 x 2048: 35 -> 29,
 // 2304^3: 39 -> 35) and leaves those with about 128 tiles where they were (2048^2 x 5632: 56 us against 72).  The
 // 128 x 128 tile (two workgroups per CU) takes what neither fits: 2304^3 35 -> 31 us, 2048 x 2560 x 2048 29 -> 27.
-// UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 10 / 6 / 7 / 9 the ring's tiles, 0..2 keeps both out (tuning aid).
+// UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 10 / 11 / 6 / 7 / 9 the ring's tiles, 0..2 keeps both out (tuning aid).
 double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
   int bm, bn;
   if (!tile_dims(tile, &bm, &bn)) return 1e30;
