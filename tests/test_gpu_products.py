@@ -127,3 +127,30 @@ def test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk):
     exact = np.matmul(a.astype(np.float64), w.astype(np.float64))
     bound = {"f32": 0, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype] * np.abs(exact) + (k + 1) * np.finfo(np.float32).eps * np.matmul(np.abs(a).astype(np.float64), np.abs(w).astype(np.float64))
     assert np.all(np.abs(got[: b * m * n].reshape(exact.shape) - exact) <= bound * 1.001 + 1e-7)
+
+
+# products of one tile, of several, of tiles of both sizes, in batches; f32 on both sides of one step by element
+@pytest.mark.parametrize("b, m, n, k, dtype, kernel", [(300, 33, 17, 40, "f32", "gemm_any<f32>"), (17, 9, 70, 65, "f16", "gemm_any<f16>"), (9, 65, 129, 130, "bf16", "gemm_any<bf16>"),
+                                                       (3, 1155, 1155, 130, "bf16", "gemm_any<bf16,128x128>"), (5, 70, 130, 16, "f32", "gemm_any<f32,by element>"),
+                                                       (5, 70, 131, 17, "f32", "gemm_any<f32>"), (2, 20, 7, 100, "f16", "gemm_any<f16,by element>")])
+@pytest.mark.parametrize("shared", [False, True], ids=["batched", "one lhs"])
+def test_batches_of_products_of_any_size(hip, b, m, n, k, dtype, kernel, shared):
+    """Batches, a left operand with padded rows that is each product's own or all products' (batch stride 0), and the kernel by its name."""
+    gap = 3
+    a, w = rng.uniform_pm1(1, b * m * k), rng.uniform_pm1(2, b * k * n)
+    dt, enc = {"f32": (ug_amd.F32, lambda v: v), "f16": (ug_amd.F16, lambda v: v.astype(np.float16)), "bf16": (ug_amd.BF16, rng.to_bf16_bits)}[dtype]
+    if dtype != "f32":
+        a, w = rounded(dtype, a), rounded(dtype, w)
+    a, w = a.reshape(b, m, k)[: 1 if shared else b], w.reshape(b, k, n)
+    padded = np.full((a.shape[0], m, k + gap), np.nan, np.float32)
+    padded[:, :, :k] = a
+    sa, sw, dst = hip.slice_from(enc(padded.ravel())), hip.slice_from(enc(w.ravel())), hip.slice_from(enc(np.full(b * m * n + 9, 7.0, np.float32)))
+    print("batches", dtype, b, m, n, k, shared, flush=True)
+    hip.matmul(dst, sa, sw, (b, m, n, k), ((b, m, k), (0 if shared else m * (k + gap), k + gap, 1), 0), ((b, k, n), (k * n, n, 1), 0))
+    assert ug_amd.last_kernel() == kernel
+    got = dst.to_vec()
+    got = (rng.from_bf16_bits(got) if dtype == "bf16" else got).astype(np.float64)
+    assert np.all(got[b * m * n :] == 7.0), "wrote past the end"
+    exact = np.matmul(a.astype(np.float64), w.astype(np.float64))
+    bound = {"f32": 0, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype] * np.abs(exact) + (k + 1) * np.finfo(np.float32).eps * np.matmul(np.abs(a).astype(np.float64), np.abs(w).astype(np.float64))
+    assert np.all(np.abs(got[: b * m * n].reshape(exact.shape) - exact) <= bound * 1.001 + 1e-7)

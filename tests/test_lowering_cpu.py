@@ -365,3 +365,27 @@ def test_kernel_choice_for_the_baseline_shapes_is_pinned():
         assert "6 terms" not in _plan(F, F, 1, 1024, 1024, 1000, 1)
         assert "6 terms" not in _plan(B, B, 1, 4096, 4096, 4096, 1)
     assert "6 terms" not in _plan(F, F, 8, 1024, 1024, 1024, 0)
+
+
+def test_plans_of_products_of_any_size():
+    """Which tile takes a product that no tuned kernel does: the large one where it is mostly full and pays for its prologue, f32 products of one
+    short step by element, and so what gemm_ragged cannot read."""
+    F, H, B = ug_amd.F32, ug_amd.F16, ug_amd.BF16
+    want = {
+        (F, F, 300, 33, 17, 129, 0): "gemm_any<f32>",
+        (H, H, 300, 33, 17, 129, 0): "gemm_any<f16>",                  # 300 tiles of 128 x 128, nine tenths of them padding
+        (H, H, 100, 9, 700, 333, 0): "gemm_any<f16>",
+        (H, H, 1, 2001, 2001, 1001, 0): "gemm_any<f16,128x128>",
+        (B, B, 200, 70, 130, 333, 0): "gemm_any<bf16,128x128>",        # a quarter padding
+        (B, B, 1, 2001, 2001, 65, 0): "gemm_any<bf16,128x128>",
+        (B, B, 1, 2001, 2001, 63, 0): "gemm_any<bf16,128x128>",        # one full round
+        (B, B, 1, 3001, 3001, 63, 0): "gemm_any<bf16>",
+        (F, F, 1, 2001, 2001, 1001, 0): "gemm_any<f32>",
+        (F, F, 1, 3501, 3501, 1101, 0): "gemm_any<f32>",
+        (F, F, 1, 3999, 3999, 2001, 0): "gemm_any<f32,128x128>",
+        (F, F, 1, 2001, 2001, 17, 0): "gemm_any<f32>",
+        (F, F, 1, 2001, 2001, 15, 0): "gemm_any<f32,by element>",
+        (H, H, 1, 20, 7, 100, 0): "gemm_any<f16,by element>",          # rows of k shorter than a chunk
+    }
+    got = {key: _plan(*key) for key in want}
+    assert got == want

@@ -99,9 +99,10 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act);  // a ti
 hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRows& r, RowsAct act, int tile);
 
 // Any M, N, K and any alignment (gemm_ragged.hip; f32, f16, bf16): operands contiguous along k or along their other dimension, at least eight
-// elements from one k to the next in the latter case.  Contiguous [batch, M, N] result.
-bool gemm_ragged_supported(const MMArgs& p, size_t batch);
-hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch);
+// elements from one k to the next in the latter case.  Contiguous [batch, M, N] result.  The tile it takes a product with, 64 or 128; 0: the
+// kernels that go by element should.
+int gemm_ragged_tile(int dtype, const MMArgs& p, size_t batch);
+hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, int tile);
 
 // f32, one wave per SIMD: 256 x 128 tiles of v_mfma_f32_32x32x2_f32, loads that write LDS directly, rhs [n, k]- or [k, n]-major
 // (gemm_dma_f32.hip).  Any M, N % 4 == 0, K % 32 == 0 and K >= 64, 16-byte aligned rows, contiguous [batch, M, N] result.

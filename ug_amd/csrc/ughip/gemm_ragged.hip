@@ -9,8 +9,8 @@
 //   [k, n]-major operand behind which nothing may be read.
 //
 // What bounds it: the steps' latency on few tiles (0.35 us each in 16 bits, 0.6 in f32), LDS and the f32 matrix pipe on many.  Against element-by-element
-// loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 14.5 us, f32 256 -> 35; 2001^3 f16 265 -> 40, f32 343 -> 155; 3999^2 x
-// 2000 f16 1190 -> 118, f32 1015 -> 513; 100^3 9.4 -> 5.4.  The 128 x 128 tile from 256 of them on: 2001^3 has that many.
+// loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 14.6 us, f32 256 -> 34; 2001^3 f16 270 -> 37, f32 340 -> 135; 3999^2 x
+// 2000 f16 1204 -> 103, f32 1014 -> 520; 100^3 9.4 -> 5.4.  Which tile takes what: gemm_ragged_tile.
 #include <hip/hip_runtime.h>
 
 #include "gemm.h"
@@ -119,20 +119,21 @@ struct Side {
 };
 
 template <typename T, int BT, bool A_KC, bool B_KC>
-__global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int tiles_m, int tiles_n) {
+__global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int tiles_m, int tiles_n) {
   typedef Side<T, BT, A_KC> SA;
   typedef Side<T, BT, B_KC> SB;
   constexpr int MI = BT / 64, KE = SA::KE;
   __shared__ __attribute__((aligned(16))) char lds[2][SA::BYTES + SB::BYTES];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // each XCD a contiguous run of tiles (block ids go round-robin over the 8)
-  const int tiles = tiles_m * tiles_n, per = (tiles + 7) >> 3, bid = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  // each XCD a contiguous run of all products' tiles (block ids go round-robin over the 8): with the runs dealt product by product a batch
+  // of products of one tile would be one XCD's work (300 of 33 x 17 x 129 in f32: 32 us that way, 8.9 so, 16 in the kernel by element)
+  const int tpb = tiles_m * tiles_n, tiles = batches * tpb, per = (tiles + 7) >> 3, bid = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if (bid >= tiles) return;
-  const int tm = bid / tiles_n, tn = bid - tm * tiles_n, m0 = tm * BT, n0 = tn * BT;
+  const int batch = bid / tpb, in_batch = bid - batch * tpb, tm = in_batch / tiles_n, tn = in_batch - tm * tiles_n, m0 = tm * BT, n0 = tn * BT;
   SA a;
   SB b;
-  a.place(static_cast<const T*>(p.a) + (size_t)blockIdx.y * p.a_bs, m0, p.M, p.a_rs, p.a_cs, tid);
-  b.place(static_cast<const T*>(p.b) + (size_t)blockIdx.y * p.b_bs, n0, p.N, p.b_cs, p.b_rs, tid);
+  a.place(static_cast<const T*>(p.a) + (size_t)batch * p.a_bs, m0, p.M, p.a_rs, p.a_cs, tid);
+  b.place(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs, n0, p.N, p.b_cs, p.b_rs, tid);
   const int full = (p.K - 1) / KE, left = p.K - full * KE;  // whole steps, and 1 .. KE elements of k behind them
   f32x16 acc[MI][MI];
 #pragma unroll
@@ -193,7 +194,7 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int tiles_m, int ti
   }
 
   // element e of lane l of block (i, j): row l % 32, column 8 (e / 4) + 4 (l / 32) + e % 4
-  T* __restrict__ C = static_cast<T*>(p.c) + (size_t)blockIdx.y * p.c_bs;
+  T* __restrict__ C = static_cast<T*>(p.c) + (size_t)batch * p.c_bs;
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int row = m0 + wm + 32 * i + (lane & 31);
@@ -218,34 +219,44 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int tiles_m, int ti
 template <typename T, int BT>
 hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch) {
   const int tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BT - 1) / BT;
-  const dim3 grid((unsigned)(((size_t)tiles_m * tiles_n + 7) / 8 * 8), (unsigned)batch);
+  const unsigned grid = (unsigned)((batch * tiles_m * tiles_n + 7) / 8 * 8);
   const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
-  if (ak && bk) gemm_ragged<T, BT, true, true><<<grid, 256, 0, stream>>>(p, tiles_m, tiles_n);
-  else if (ak) gemm_ragged<T, BT, true, false><<<grid, 256, 0, stream>>>(p, tiles_m, tiles_n);
-  else if (bk) gemm_ragged<T, BT, false, true><<<grid, 256, 0, stream>>>(p, tiles_m, tiles_n);
-  else gemm_ragged<T, BT, false, false><<<grid, 256, 0, stream>>>(p, tiles_m, tiles_n);
+  if (ak && bk) gemm_ragged<T, BT, true, true><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n);
+  else if (ak) gemm_ragged<T, BT, true, false><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n);
+  else if (bk) gemm_ragged<T, BT, false, true><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n);
+  else gemm_ragged<T, BT, false, false><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n);
   return hipGetLastError();
-}
-
-template <typename T>
-hipError_t launch_type(hipStream_t stream, const MMArgs& p, size_t batch) {
-  const size_t big = batch * (size_t)((p.M + 127) / 128) * (size_t)((p.N + 127) / 128);
-  return big >= 256 ? launch<T, 128>(stream, p, batch) : launch<T, 64>(stream, p, batch);
 }
 
 }  // namespace
 
-bool gemm_ragged_supported(const MMArgs& p, size_t batch) {
+static bool supported(const MMArgs& p, size_t batch) {
   // an operand that is contiguous along its other dimension: eight elements or more from one k to the next, so that a chunk over the end of a
   // row stays inside the rows behind it
   const bool a = p.a_cs == 1 || (p.a_rs == 1 && p.a_cs >= 8 && p.M >= 8), b = p.b_rs == 1 || (p.b_cs == 1 && p.b_rs >= 8 && p.N >= 8);
-  return a && b && p.M > 0 && p.N > 0 && p.K > 0 && p.a_rs >= 0 && p.b_cs >= 0 && batch <= 65535 && (size_t)((p.M + 63) / 64) * ((p.N + 63) / 64) < (1u << 24);
+  return a && b && p.M > 0 && p.N > 0 && p.K > 0 && p.a_rs >= 0 && p.b_cs >= 0 && batch <= 65535 && batch * ((p.M + 63) / 64) * ((p.N + 63) / 64) < (1u << 24);
 }
 
-hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch) {
-  if (!gemm_ragged_supported(p, batch)) return hipErrorInvalidValue;
-  if (dtype == UGHIP_F32) return launch_type<float>(stream, p, batch);
-  return dtype == UGHIP_F16 ? launch_type<_Float16>(stream, p, batch) : launch_type<__bf16>(stream, p, batch);
+// Where each tile is the faster one, measured (us, by element / 64 x 64 / 128 x 128); the large one from 256 of them on, one round of the chip, where no
+// more than a quarter of them is padding (100 f16 products of 9 x 700 x 1001, half of it padding: 261 / 42 / 52):
+//   f32 up to K = 16, one step of the kernel by element, is its store: 3001 x 3003 x 16 13.8 / 15.4 / 20.6, 2001^2 x 8 8.0 / 9.0 / 10.1; at K = 17 17.7 /
+//   15.4 / 20.8.  The f32 matrix pipe is busy on small tiles already (2001^2 x 129 28.4 / 17.1 / 19.9, 7 x 512 x 1219 x 333 70 / 36 / 52, 3501^2 x 1001 205 small, 263
+//   large), but for long sums in three rounds or more whose last is nearly full: 3999^2 x 2000 1014 / 520 / 510, 4095^3 1048 small, 1028 large.
+//   16 bits: the large tile's prologue wants more than one step to pay for it, or a single full round: 2001^2 x 8 8.3 / 7.7 / 8.3, x 33 10.0 / 9.0 / 8.5, x 127 18.1 /
+//   14.3 / 11.9, x 1001 141 / 31.2 / 23.5, 7 x 512 x 1219 x 63 19.6 / 13.1 / 15.4, x 129 37.8 / 13.1 / 15.0, x 1001 283 / 37.5 / 35.0.
+int gemm_ragged_tile(int dtype, const MMArgs& p, size_t batch) {
+  if (!supported(p, batch) || (dtype == UGHIP_F32 && p.K <= 16)) return 0;
+  const size_t big = batch * ((p.M + 127) / 128) * ((p.N + 127) / 128), small = batch * ((p.M + 63) / 64) * ((p.N + 63) / 64);
+  if (big < 256 || 3 * big > small) return 64;
+  if (dtype == UGHIP_F32) return big >= 768 && (big + 64) % 256 <= 64 && p.K >= 1024 ? 128 : 64;
+  return p.K > 64 || (big == 256 && p.K > 8) ? 128 : 64;
+}
+
+hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, int tile) {
+  if (!supported(p, batch) || (tile != 64 && tile != 128)) return hipErrorInvalidValue;
+  if (dtype == UGHIP_F32) return tile == 128 ? launch<float, 128>(stream, p, batch) : launch<float, 64>(stream, p, batch);
+  if (dtype == UGHIP_F16) return tile == 128 ? launch<_Float16, 128>(stream, p, batch) : launch<_Float16, 64>(stream, p, batch);
+  return tile == 128 ? launch<__bf16, 128>(stream, p, batch) : launch<__bf16, 64>(stream, p, batch);
 }
 
 }  // namespace ughip

@@ -500,6 +500,9 @@ static Route matmul_route(int dtype, bool mixed, const MMArgs& p, size_t b, size
   return gemm_tiled_supported(dtype, p, b, mixed) ? ROUTE_TILED : ROUTE_ANY;
 }
 
+// The kernels behind ROUTE_ANY, in names: gemm_ragged's 64 x 64 and 128 x 128 tiles (gemm_ragged_tile), and the ones that go by element.
+static const char* any_tail(int tile) { return tile == 128 ? ",128x128" : tile ? "" : ",by element"; }
+
 static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* lhs, const ughip_slice* rhs, size_t b, size_t m, size_t n, size_t k,
                        size_t rank, const size_t* lhs_dims, const size_t* lhs_strides, size_t lhs_offset, const size_t* rhs_dims, const size_t* rhs_strides,
                        size_t rhs_offset, bool no_alloc) {
@@ -604,8 +607,9 @@ static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* l
   } else {
     dim3 grid((unsigned)((n + 63) / 64), (unsigned)((m + 63) / 64), (unsigned)b);
     if (grid.y > 65535 || b > 65535) return set_error(UGHIP_ERR_INVALID, "matmul: m or batch too large for this kernel");
-    note_kernel("gemm_any<%s>", tn);
-    if (gemm_ragged_supported(p, b)) UGHIP_HIPCHK(gemm_ragged_launch(st, dst->dtype, p, b));
+    const int tile = gemm_ragged_tile(dst->dtype, p, b);
+    note_kernel("gemm_any<%s%s>", tn, any_tail(tile));
+    if (tile) UGHIP_HIPCHK(gemm_ragged_launch(st, dst->dtype, p, b, tile));
     else if (f32) gemm_f32_any<<<grid, 256, 0, st>>>(p);
     else if (dst->dtype == UGHIP_F16) gemm_half_any<_Float16><<<grid, 256, 0, st>>>(p);
     else gemm_half_any<__bf16><<<grid, 256, 0, st>>>(p);
@@ -1003,7 +1007,7 @@ extern "C" int ughip_matmul_plan(int dtype, int rhs_dtype, size_t b, size_t m, s
       break;
     }
     case ROUTE_TILED: gemm_tiled_name(dtype, p, b, mixed, nullptr, buf, buf_len); break;
-    default: snprintf(buf, buf_len, "gemm_any<%s>", tn); break;
+    default: snprintf(buf, buf_len, "gemm_any<%s%s>", tn, any_tail(gemm_ragged_tile(dtype, p, b))); break;
   }
   return UGHIP_OK;
 }
