@@ -154,3 +154,35 @@ def test_batches_of_products_of_any_size(hip, b, m, n, k, dtype, kernel, shared)
     exact = np.matmul(a.astype(np.float64), w.astype(np.float64))
     bound = {"f32": 0, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype] * np.abs(exact) + (k + 1) * np.finfo(np.float32).eps * np.matmul(np.abs(a).astype(np.float64), np.abs(w).astype(np.float64))
     assert np.all(np.abs(got[: b * m * n].reshape(exact.shape) - exact) <= bound * 1.001 + 1e-7)
+
+
+# one group, a wave's 64 and one more, several rounds of them; groups without rows, ends in front of their predecessors' and behind the rows
+@pytest.mark.parametrize("groups", [1, 2, 63, 64, 65, 128, 300])
+@pytest.mark.parametrize("rows", [0, 3, 700])
+def test_rows_by_group(hip, tune, groups, rows):
+    """Which matrix a row meets, on every tile of rows: against the same product with each row's matrix looked up."""
+    gpu, n, k, m = Gpu(hip), 24, 256, max(1, rows)
+    gen = np.random.default_rng(groups + rows)
+    x, w = rand(1, m, k), rand(2, groups, n, k, std=k ** -0.5)
+    end = np.sort(gen.integers(0, rows + 1, groups)).astype(np.int32)
+    end[-1] = rows
+    said = end.copy()
+    if groups > 2:
+        said[1:-1:7] = -5              # an empty group, whatever is behind it
+        end = np.maximum.accumulate(np.maximum(said, 0)).astype(np.int32)
+    if rows == 700:
+        said[-1] = rows + 1000
+    src, of = gen.integers(0, m, m).astype(np.int32), np.searchsorted(end, np.arange(rows), side="right")
+    y = np.stack([w[of[i]] @ x[src[i]] for i in range(rows)]) if rows else np.zeros((0, n))
+    dx, dw, di, de = gpu.up(x, bf16=True), gpu.up(w, bf16=True), gpu.up(src), gpu.up(said)
+    for shape in (None, "0", "3", *RING, "11"):
+        if shape is not None:
+            tune.setenv("UGHIP_GEMM_SHAPE", shape)
+        dst = gpu.out(m * n + 8)
+        print("rows by group", groups, rows, shape, flush=True)
+        gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=BF16, act=NONE, row_index=di.raw(), group_end=de.raw(),
+                                                       groups=groups, x_rows=m)))
+        out = get(dst, m * n + 8)
+        assert np.all(np.isnan(out[rows * n :])), "wrote what belongs to no group"
+        if rows:
+            close(out[: rows * n].reshape(rows, n), y, 2e-5)

@@ -68,6 +68,60 @@ __device__ __forceinline__ int rhs_k_tile(int tile) {
   }
 }
 
+// Inclusive scans over the lanes of a wave, all active; of values from 0 up.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int scan_move(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);  // 0 where there is no lane to read from
+}
+template <typename F>
+__device__ __forceinline__ int wave_scan(int v, F f) {
+  v = f(v, scan_move<0x111, 0xf>(v));  // within rows of 16 lanes: from 1, 2, 4 and 8 lanes below
+  v = f(v, scan_move<0x112, 0xf>(v));
+  v = f(v, scan_move<0x114, 0xf>(v));
+  v = f(v, scan_move<0x118, 0xf>(v));
+  v = f(v, scan_move<0x142, 0xa>(v));  // the last lane of rows 0 and 2 to rows 1 and 3
+  return f(v, scan_move<0x143, 0xc>(v));  // lane 31 to rows 2 and 3
+}
+
+// Rows sorted by group, ceil(rows / BM) tile rows to each: a lane per group, 64 at a time.  Every workgroup asks for it before its first load, one
+// that finds no tile of its own too, and mostly has its CU to itself: read one after the other by scalar loads the ends took it 0.1-0.15 us each
+// (64 groups, n = 2 x 552, k = 128, 1638 rows: 49 us so, on 64 x 128 tiles, 12.8 with a lane per group; 18.9 in rows_product).
+template <int BM>
+struct GroupTiles {
+  const int* group_end;
+  int groups, m, lane;
+  int begin = 0, end = 0, upto = 0;  // lane's group: its rows, and the tile rows of all groups up to it
+  int rows = 0, tiles = 0;           // of the groups read so far
+
+  __device__ __forceinline__ void read(int base) {
+    int e = base + lane < groups ? group_end[base + lane] : 0;
+    e = wave_scan(max(min(e, m), rows), [](int a, int b) { return max(a, b); });  // (an end in front of its predecessor's: an empty group)
+    begin = __builtin_amdgcn_update_dpp(rows, e, 0x138, 0xf, 0xf, false);         // from one lane below, lane 0 the groups in front
+    end = e;
+    upto = tiles + wave_scan((e - begin + BM - 1) / BM, [](int a, int b) { return a + b; });
+    rows = __builtin_amdgcn_readlane(e, 63), tiles = __builtin_amdgcn_readlane(upto, 63);
+  }
+  __device__ __forceinline__ int count() {
+    rows = tiles = 0;
+    for (int base = 0; base < groups; base += 64) read(base);
+    return tiles;
+  }
+  // behind count(): group and rows [m0, m_end) of a tile row below it
+  __device__ __forceinline__ bool find(int tile, int& group, int& m0, int& m_end) {
+    if (groups > 64) rows = tiles = 0;
+    for (int base = 0; base < groups; base += 64) {
+      if (groups > 64) read(base);
+      const unsigned long long behind = __ballot(upto > tile);
+      if (!behind) continue;
+      const int l = __builtin_ctzll(behind), first = __builtin_amdgcn_readlane(begin, l);
+      group = base + l, m_end = __builtin_amdgcn_readlane(end, l);
+      m0 = first + (tile - __builtin_amdgcn_readlane(upto, l) + (m_end - first + BM - 1) / BM) * BM;
+      return true;
+    }
+    return false;
+  }
+};
+
 // The products those kernels take, besides plain ones: see gemm_dma4.
 enum class DmaForm { PLAIN, PLANES3, ROWS, ROWS_GLU, ROWS_LOOKUP };
 // gemm_ring.hip: one of its tiles (codes 129, 97, 65, 48, 32: 256 x 128, 192 x 192, 128 x 128, 64 x 128, 64 x 64), operands as the _supported functions of gemm_dma.hip check them.

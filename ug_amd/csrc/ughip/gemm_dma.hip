@@ -73,16 +73,11 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   // tiles, and tiles are numbered in super-rows of 4 tile rows, column by column inside, so that such a run is a 4-row
   // block: its workgroups share few A and B panels in their XCD's L2.
   int bid = blockIdx.x;
+  GroupTiles<BM> by_group{rw.group_end, rw.groups, p.M, lane};
   if constexpr (ROWS != 0) {
     if (rw.groups) {
       // how many tile rows there are is known here only: the workgroups past them leave before the runs are dealt
-      int rows = 0, begin = 0;
-      for (int g = 0; g < rw.groups; ++g) {
-        int end = rw.group_end[g];
-        end = end < begin ? begin : end > p.M ? p.M : end;
-        rows += (end - begin + BM - 1) / BM;
-        begin = end;
-      }
+      const int rows = by_group.count();
       const int tiles = rows * tiles_n, per = (tiles + 7) >> 3;
       if (bid >= 8 * per) return;
       bid = (bid & 7) * per + (bid >> 3);
@@ -106,21 +101,7 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   }
   int m0 = tm * BM, m_end = p.M, group = 0;
   const int n0 = tn * BN;
-  if constexpr (ROWS != 0) {
-    if (rw.groups) {
-      // groups take ceil(rows / BM) tile rows each, in order
-      int t = tm, begin = 0;
-      bool found = false;
-      for (int g = 0; g < rw.groups && !found; ++g) {
-        int end = rw.group_end[g];
-        end = end < begin ? begin : end > p.M ? p.M : end;
-        const int tiles = (end - begin + BM - 1) / BM;
-        if (t < tiles) group = g, m0 = begin + t * BM, m_end = end, found = true;
-        else t -= tiles, begin = end;
-      }
-      if (!found) return;  // the same for the whole workgroup
-    }
-  }
+  if (ROWS != 0 && rw.groups && !by_group.find(tm, group, m0, m_end)) return;  // the same for the whole workgroup
   const long long lda = p.a_rs, ldb = B_KN ? p.b_rs : p.b_cs;
   const char* Ab = reinterpret_cast<const char*>(static_cast<const T*>(p.a) + (size_t)batch * p.a_bs + (ROWS ? 0 : (size_t)m0 * lda));
   const char* Bb = reinterpret_cast<const char*>(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs + (ROWS ? (size_t)group * rw.w_group : 0) +
@@ -668,15 +649,17 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
   }
   // A model's products: the matrix comes from memory.  256 x 256 tiles of gemm_dma4 and the ring's, by what they are expected to take
   // (2048 positions: down 74 -> 51 us, gate and up 105 -> 89, output 26 -> 18, attention's input 37 -> 29; 509 positions: state-space output
-  // 53 -> 19, input 43 -> 32, dense gate and up 40 -> 30; 16 experts' gate and up 83 -> 62, down 38 -> 33, 700 positions' gate and
-  // up 52 -> 34; 33 rows of 11264 x 2048 31 -> 13).
+  // 53 -> 19, input 43 -> 32, dense gate and up 40 -> 30; 700 positions' gate and up 52 -> 34; 33 rows of 11264 x 2048 31 -> 13).
+  // By group, how the rows are spread is not known here; the model takes them as even.  16 experts' gate and up (n = 2 x 1408, k = 2048) whose shares
+  // of the rows differ by 40 %, 256 x 256 / 256 x 128 / 192 x 192 / 128 x 128: 1000 rows 56 / 65 / 46 / 54 us, 2036 59 / 68 / 46 / 66, 2800 59 / 73 / 75 / 74, 4096
+  // 103 / 91 / 74 / 89; a router whose groups of 2036 rows run from 60 to 260 takes 52 to 72 on 192 x 192 (rows past 192 are a second round) and 70
+  // on 256 x 256.
   const size_t groups = r.groups ? r.groups : 1;
   const double m = (double)p.M / groups;  // rows as if they were spread evenly
   int best = 0;
   double best_us = 0;
   for (int tile : {256, 129, 65, 48, 32, 97}) {
-    // (192 x 192 where it saves a round of one matrix's tiles; a model's experts are too uneven: rows past 192 cost the round they were to save)
-    if (!gemm_dma_rows_supported(p, r, act, tile) || (tile == 97 && r.groups)) continue;
+    if (!gemm_dma_rows_supported(p, r, act, tile)) continue;
     int bm, bn;
     tile_dims(tile, &bm, &bn);
     // tile rows: of groups near or above a tile's height every second one takes one more
@@ -687,7 +670,8 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
     if (tile == 256)
       for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (1.23 + 0.33 * (left < 256 ? (double)left : 256.0) / 256.0);
     else us = ring_cost_us(tiles, kt, tile, true);
-    if (!best || us < best_us * (tile == 97 ? 0.9 : 0.97)) best = tile, best_us = us;  // the larger tile on a near tie
+    // the larger tile on a near tie; 192 x 192 last: for one matrix where it clearly saves a round, by group from the same margin on as the others
+    if (!best || us < best_us * (tile == 97 && groups == 1 ? 0.9 : 0.97)) best = tile, best_us = us;
   }
   return best;
 }

@@ -43,16 +43,10 @@ __global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tile
 
   // XCD-aware order of the tiles: as in gemm_dma4 (the grid is 8 more at least, the runs are of equal length)
   int tiles = batches * tiles_m * tiles_n;
+  GroupTiles<BM> by_group{rw.group_end, rw.groups, p.M, lane};
   if (ROWS != 0 && rw.groups) {
-    int rows = 0, begin = 0;
-    for (int g = 0; g < rw.groups; ++g) {
-      int end = rw.group_end[g];
-      end = end < begin ? begin : end > p.M ? p.M : end;
-      rows += (end - begin + BM - 1) / BM;
-      begin = end;
-    }
-    tiles_m = rows;
-    tiles = rows * tiles_n;
+    tiles_m = by_group.count();
+    tiles = tiles_m * tiles_n;
   }
   const int per = (tiles + 7) >> 3;
   if ((int)blockIdx.x >= 8 * per) return;
@@ -72,18 +66,7 @@ __global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tile
   }
   int m0 = tm * BM, m_end = p.M, group = 0;
   const int n0 = tn * BN;
-  if (ROWS != 0 && rw.groups) {
-    int t = tm, begin = 0;
-    bool found = false;
-    for (int g = 0; g < rw.groups && !found; ++g) {
-      int end = rw.group_end[g];
-      end = end < begin ? begin : end > p.M ? p.M : end;
-      const int tiles = (end - begin + BM - 1) / BM;
-      if (t < tiles) group = g, m0 = begin + t * BM, m_end = end, found = true;
-      else t -= tiles, begin = end;
-    }
-    if (!found) return;  // the same for the whole workgroup
-  }
+  if (ROWS != 0 && rw.groups && !by_group.find(tm, group, m0, m_end)) return;  // the same for the whole workgroup
   const long long lda = p.a_rs, ldb = B_KN ? p.b_rs : p.b_cs;
   const char* Ab = reinterpret_cast<const char*>(static_cast<const T*>(p.a) + (size_t)batch * p.a_bs + (ROWS ? 0 : (size_t)m0 * lda));
   const char* Bb = reinterpret_cast<const char*>(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs + (ROWS ? (size_t)group * rw.w_group : 0) +
