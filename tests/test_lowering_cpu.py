@@ -389,3 +389,16 @@ def test_plans_of_products_of_any_size():
     }
     got = {key: _plan(*key) for key in want}
     assert got == want
+
+
+def test_narrow_products_with_a_long_k_take_the_kernel_that_splits_it():
+    """Few 64 x 64 tiles with a long K each: the register-staged kernel's K split is the faster one; where the tiles fill the chip, the ring."""
+    B = ug_amd.BF16
+    for shape in [(1, 584, 360, 6656, 1), (1, 583, 264, 5248, 1), (5, 220, 352, 7488, 1), (1, 3978, 16, 4992, 1), (4, 320, 64, 2496, 0), (7, 2512, 64, 5952, 1)]:
+        assert _plan(B, B, *shape).startswith("gemm_tiled<bf16") and "splitK" in _plan(B, B, *shape), shape
+    for shape in [(1, 2462, 232, 7360, 1), (1, 469, 688, 5376, 1), (3, 1240, 512, 7680, 1), (4, 3760, 64, 8000, 1)]:
+        assert "ring" in _plan(B, B, *shape), shape
+    for m, n, k in [(1011, 280, 2112), (740, 512, 2368), (402, 464, 1600)]:
+        assert _rows_plan(B, 1, 0, m, n, k).startswith("gemm_tiled"), (m, n, k)
+    for m, n, k in [(505, 136, 4352), (396, 160, 512)]:
+        assert "ring,3 planes" in _rows_plan(B, 1, 0, m, n, k), (m, n, k)

@@ -446,6 +446,10 @@ bool tile_dims(int tile, int* bm, int* bn) {
 }
 }  // namespace
 
+static size_t tile_count(const MMArgs& p, size_t batch, int tile) {  // 0: no such tile
+  int bm, bn;
+  return tile_dims(tile, &bm, &bn) ? batch * (size_t)((p.M + bm - 1) / bm) * (size_t)((p.N + bn - 1) / bn) : 0;
+}
 static bool ring_tile(int tile) { return tile == 129 || tile == 97 || tile == 65 || tile == 48 || tile == 32; }
 static int least_k(int tile) { return ring_tile(tile) ? BK : 4 * BK; }
 static const char* waves_name(int tile) { return ring_tile(tile) ? "512t,ring" : "256t"; }  // in the names of these kernels
@@ -480,16 +484,19 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
   return batch * (size_t)((p.M + bm - 1) / bm) * (size_t)((p.N + bn - 1) / bn) < (1u << 24);
 }
 
-// What `tiles` tiles of the ring kernel take: a fixed part and, per round of 256 tiles, the K tiles.  The time of a K tile is that of its bytes
-// on their way to a CU, some 100 bytes per ns from the memory-side cache and 60 from HBM however many are asked for at once (with the MFMAs or the
-// LDS reads taken out the kernel takes as long), so it goes by where the operands come from: `streamed` is a matrix nobody has read
-// lately, as the weights of a model's next layer are.  Fitted to (m x n x k, us): 2048^2 x 5632 streamed 51 (128 x 128) / 67 (256 x 128), 1024 x 2048 x
-// 5632 streamed 38 (64 x 128), 509 x 2048 x 5632 streamed 26 (64 x 64), 2048 x 11264 x 2048 streamed 89 (256 x 128), 700 x
-// 11264 x 2048 streamed 34 and 1500 x 11264 x 2048 68 (192 x 192); 2048^3 19.2 (128 x 128),
-// 1024 x 2048 x 4096 21.1 (64 x 128), 256 x 4096^2 14.7 (64 x 64).
-static double ring_cost_us(size_t tiles, int kt, int tile, bool streamed) {
-  const double t0 = tile == 129 ? 0.64 : tile == 97 ? 0.62 : tile == 65 ? (streamed ? 0.54 : 0.30) : tile == 48 ? (streamed ? 0.40 : 0.21) : streamed ? 0.255 : 0.11;
-  const double t1 = tile == 129 ? 0.22 : tile == 97 ? 0.30 : streamed ? 0 : tile == 65 ? 0.17 : tile == 48 ? 0.07 : 0.075;
+// What `tiles` tiles of the ring kernel take: a fixed part and, per round of 256 tiles, the K tiles.  The time of a K tile is mostly that of its
+// bytes on their way to a CU, some 100 bytes per ns from the memory-side cache and 60 from HBM however many are asked for at once (operands from
+// HBM: the kernel takes as long without its MFMAs), so it goes by where the operands come from.  MEMORY is a matrix nobody has read lately,
+// as the weights of a model's next layer are; CACHE what a product finds whose operands were written or read just before; PLANES an lhs of three
+// planes.  Fitted to (m x n x k, us): 2048^2 x 5632 from memory 51 (128 x 128) / 67 (256 x 128), 1024 x 2048 x
+// 5632 from memory 38 (64 x 128), 509 x 2048 x 5632 from memory 26 (64 x 64), 2048 x 11264 x 2048 from memory 89 (256 x 128), 700 x
+// 11264 x 2048 from memory 34 and 1500 x 11264 x 2048 68 (192 x 192); 2048^3 19.2 (128 x 128),
+// 1024 x 2048 x 4096 21.1 (64 x 128), 256 x 4096^2 14.7 (64 x 64), 584 x 360 x 6656 20.9 and 9 x 64 x 4416 13.2 (64 x 64).
+enum class Operands { MEMORY, CACHE, PLANES };
+static double ring_cost_us(size_t tiles, int kt, int tile, Operands from) {
+  const bool memory = from == Operands::MEMORY, planes = from == Operands::PLANES;
+  const double t0 = tile == 129 ? 0.64 : tile == 97 ? 0.62 : tile == 65 ? (memory ? 0.54 : 0.30) : tile == 48 ? (memory ? 0.40 : 0.21) : memory ? 0.255 : planes ? 0.11 : 0.14;
+  const double t1 = tile == 129 ? 0.22 : tile == 97 ? 0.30 : memory ? 0 : tile == 65 ? 0.17 : tile == 48 ? 0.07 : planes ? 0.075 : 0.045;
   double us = tile == 129 || tile == 97 ? 5.0 : tile == 65 ? 4.0 : 3.3;
   for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (t0 + t1 * (left < 256 ? (double)left : 256.0) / 256.0);
   return us;
@@ -508,12 +515,12 @@ static double ring_cost_us(size_t tiles, int kt, int tile, bool streamed) {
 // 128 x 128 tile (two workgroups per CU) takes what neither fits: 2304^3 35 -> 31 us, 2048 x 2560 x 2048 29 -> 27.
 // UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 10 / 11 / 6 / 7 / 9 the ring's tiles, 0..2 keeps both out (tuning aid).
 double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
-  int bm, bn;
-  if (!tile_dims(tile, &bm, &bn)) return 1e30;
-  const size_t tiles = batch * (size_t)((p.M + bm - 1) / bm) * (size_t)((p.N + bn - 1) / bn);
+  const size_t tiles = tile_count(p, batch, tile);
+  if (!tiles) return 1e30;
   const int kt = p.K / BK;
   const bool nn = p.b_cs == 1 && p.b_rs != 1;
-  if (ring_tile(tile)) return ring_cost_us(tiles, kt, tile, false) * (nn ? 1.08 : 1.0) + (double)batch * p.M * p.N * 2 / 6.4e6;
+  if (ring_tile(tile))
+    return ring_cost_us(tiles, kt, tile, p.b_k_div == 3 ? Operands::PLANES : Operands::CACHE) * (nn ? 1.1 : 1.0) + (double)batch * p.M * p.N * 2 / 6.4e6;
   double us = 4.0 + (double)batch * p.M * p.N * 2 / 6.4e6;
   // (the figures below were fitted to the kernel on 32 x 32 x 16 MFMAs; on 16 x 16 x 32 and with the loads spread behind two
   // barriers every K tile takes 8 % less: 4096^3 97 us, 8 x 1024^3 18.8, 1024 x 4096^2 41 on 128 x 128 tiles)
@@ -556,8 +563,13 @@ int gemm_dma_pick(int dtype, const MMArgs& p, size_t batch) {
   }
   if (!best) return 0;
   if (ring_tile(best)) {
-    const double tiled = gemm_tiled_cost_us(dtype, p, batch);  // (its model is 0-20 % below what [k, n]-major products take)
-    return tiled < 0 || best_us < tiled ? best : 0;
+    // What gemm_tiled is priced at: 0-20 % below what [k, n]-major products take, up to a quarter above what those take whose K it splits (5 x 220 x 352
+    // x 7488 18.8 us there, 23.0 here).  Operands that the memory-side cache cannot hold come from memory: 7 x 2512 x 64 x 5952, 215 MB, 51 us there, 64
+    // here; 4 x 3760 x 64 x 8000, one round of tiles, 55 and 50.
+    const double tiled = gemm_tiled_cost_us(dtype, p, batch);
+    const bool memory = 2.0 * batch * p.K * ((double)p.M + p.N) > 192e6;
+    if (memory) best_us = ring_cost_us(tile_count(p, batch, best), p.K / BK, best, Operands::MEMORY);
+    return tiled < 0 || best_us < tiled * (!memory && gemm_tiled_workspace_bytes(dtype, p, batch) ? 0.945 : 1.0) ? best : 0;
   }
   // the 128 x 128 tile runs at the register-staged kernel's pace (both are bound by their LDS reads): it has to be
   // clearly cheaper to take the product from it
@@ -669,7 +681,7 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
     double us = 6.0;
     if (tile == 256)
       for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (1.23 + 0.33 * (left < 256 ? (double)left : 256.0) / 256.0);
-    else us = ring_cost_us(tiles, kt, tile, true);
+    else us = ring_cost_us(tiles, kt, tile, Operands::MEMORY);
     // the larger tile on a near tie; 192 x 192 last: for one matrix where it clearly saves a round, by group from the same margin on as the others
     if (!best || us < best_us * (tile == 97 && groups == 1 ? 0.9 : 0.97)) best = tile, best_us = us;
   }

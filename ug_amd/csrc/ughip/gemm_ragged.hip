@@ -242,14 +242,15 @@ static bool supported(const MMArgs& p, size_t batch) {
 //   f32 up to K = 16, one step of the kernel by element, is its store: 3001 x 3003 x 16 13.8 / 15.4 / 20.6, 2001^2 x 8 8.0 / 9.0 / 10.1; at K = 17 17.7 /
 //   15.4 / 20.8.  The f32 matrix pipe is busy on small tiles already (2001^2 x 129 28.4 / 17.1 / 19.9, 7 x 512 x 1219 x 333 70 / 36 / 52, 3501^2 x 1001 205 small, 263
 //   large), but for long sums in three rounds or more whose last is nearly full: 3999^2 x 2000 1014 / 520 / 510, 4095^3 1048 small, 1028 large.
-//   16 bits: the large tile's prologue wants more than one step to pay for it, or a single full round: 2001^2 x 8 8.3 / 7.7 / 8.3, x 33 10.0 / 9.0 / 8.5, x 127 18.1 /
-//   14.3 / 11.9, x 1001 141 / 31.2 / 23.5, 7 x 512 x 1219 x 63 19.6 / 13.1 / 15.4, x 129 37.8 / 13.1 / 15.0, x 1001 283 / 37.5 / 35.0.
+//   16 bits: the large tile's prologue wants more than one step to pay for it, or a last round that is nearly full: 2001^2 x 8 8.3 / 7.7 / 8.3, x 33 10.0 / 9.0 / 8.5, x 127
+//   18.1 / 14.3 / 11.9, x 1001 141 / 31.2 / 23.5, 3187 x 2088 x 64 16.3 small, 14.5 large, 7 x 512 x 1219 x 63 19.6 / 13.1 / 15.4, x 129 37.8 / 13.1 / 15.0, x 1001 283 /
+//   37.5 / 35.0.
 int gemm_ragged_tile(int dtype, const MMArgs& p, size_t batch) {
   if (!supported(p, batch) || (dtype == UGHIP_F32 && p.K <= 16)) return 0;
   const size_t big = batch * ((p.M + 127) / 128) * ((p.N + 127) / 128), small = batch * ((p.M + 63) / 64) * ((p.N + 63) / 64);
   if (big < 256 || 3 * big > small) return 64;
   if (dtype == UGHIP_F32) return big >= 768 && (big + 64) % 256 <= 64 && p.K >= 1024 ? 128 : 64;
-  return p.K > 64 || (big == 256 && p.K > 8) ? 128 : 64;
+  return p.K > 64 || (p.K > 8 && big * 5 >= (big + 255) / 256 * 256 * 4) ? 128 : 64;
 }
 
 hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, int tile) {

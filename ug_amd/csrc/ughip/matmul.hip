@@ -801,6 +801,9 @@ static RowsRoute rows_route(const MMArgs& p, int dtype, bool x3, GemmEpilogue::K
       }
     }
     const double other = gemm_tiled_cost_us(dtype, p, 1);
+    // 64 x 64 tiles (code 32) whose long K is not split leave most CUs without one, and the others wait longer for each K tile than the model says: 1011 x 280
+    // x 2112 31.7 us, 25.2 on gemm_tiled; 740 x 512 x 2368 33.5 and 29.0; 3954 x 96 x 2368 43.7 and 39.5
+    if (r.dma_tile == 32 && r.dma_split == 1 && q.K >= 4096) best += 0.07 * (q.K / 64);
     if (r.dma_tile && !forced_tile && other >= 0 && other < best * 1.05) r.dma_tile = 0;  // it has to be clearly cheaper: its model is the rougher one
   }
   if (r.dma_tile) r.kind = RowsRoute::DMA_PLANES;
