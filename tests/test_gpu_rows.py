@@ -48,3 +48,30 @@ def test_llama_logits_of_some_positions(hip, bf16, t, want):
     assert some.shape == (len(want), 97)
     np.testing.assert_allclose(some, full[want], rtol=0, atol=2e-5 * np.abs(full).max())   # the same f32 sums in another order
     np.testing.assert_array_equal(model.step(state, [5], want=[0]), model.step(all_state, [5], want=[0]))
+
+
+# more chunks and heads than the chip has CUs, and half the heads of them at a time: two forms of the preparation, with 16-byte loads and without
+@pytest.mark.parametrize("d, vd", [(64, 16), (100, 32), (99, 17), (128, 128)])
+def test_delta_rows_of_many_heads_and_of_half_of_them(hip, d, vd):
+    """The rows of a head are the same bits whichever form prepares its chunks (and those of a few heads are held to float64 elsewhere)."""
+    from gpu_calls import Delta
+    gpu, H, T, eps = Gpu(hip), 172, 100, 1e-5
+    q, k, v, a, z = (rand(i, T, H, n) for i, n in enumerate((d, d, vd, d, vd)))
+    b, a_log, dt_bias, norm = rand(6, T, H), rand(7, H), rand(8, H, d), rand(9, vd) + 1
+
+    def rows(heads):
+        n = heads.stop - heads.start
+        s = {"qkv": np.concatenate([x[:, heads].reshape(T, -1) for x in (q, k, v)], 1), "b": b[:, heads], "a": a[:, heads], "z": z[:, heads], "a_log": a_log[heads], "dt": dt_bias[heads], "norm": norm}
+        s = {name: gpu.up(np.ascontiguousarray(x)) for name, x in s.items()}
+        S, dst = gpu.out(n * d * vd), gpu.out(T * n * vd)
+        print("delta rows", n, d, vd, flush=True)
+        gpu.call("ughip_delta_rows", C.byref(Delta(t=T, pos=0, heads=n, kv_heads=n, dim=d, vdim=vd, a_log=s["a_log"].raw(), dt_bias=s["dt"].raw(), norm=s["norm"].raw(), s=S.raw(), eps=eps,
+                                                   qkv=view(s["qkv"], 0, n * (2 * d + vd)), b=view(s["b"], 0, n), a=view(s["a"], 0, n * d), z=view(s["z"], 0, n * vd), dst=view(dst, 0, n * vd))))
+        return get(dst, (T, n, vd)), get(S, (n, d, vd))
+
+    whole, state = rows(slice(0, H))
+    assert np.all(np.isfinite(whole)) and np.all(np.isfinite(state))
+    for heads in (slice(0, 86), slice(86, 172)):
+        part, part_state = rows(heads)
+        np.testing.assert_array_equal(whole[:, heads], part)
+        np.testing.assert_array_equal(state[heads], part_state)

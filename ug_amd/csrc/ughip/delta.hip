@@ -82,9 +82,9 @@ struct DeltaArgs {
   float* gam;    // G_C of every channel
 };
 
-template <int C>
+template <int C, bool PAIR>
 __host__ __device__ constexpr size_t prepare_lds_floats(int dp) {
-  return (size_t)2 * C * (dp + 4) + (size_t)(C / 16) * (C / 16 + 1) / 2 * 256 + 2 * C;
+  return (size_t)(PAIR ? 2 : 3) * C * (dp + 4) + (size_t)(C / 16) * (C / 16 + 1) / 2 * 256 + 2 * C;
 }
 
 // four elements of a row, zeros from `left` on
@@ -102,11 +102,12 @@ template <int C>
 constexpr int prepare_threads() {
   return C == 64 ? 512 : 256;
 }
-// The queries stay in memory: they are read where they are used, times their rows' factors.  What is left in LDS of 64 rows of 128
-// channels (77 KB) is two workgroups to a CU; bound by vector instructions.  2048 positions of
-// 16 heads: 69 us with one workgroup to a CU, 62 us so.
-template <int C, bool VEC>
-__global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) delta_prepare_kernel(DeltaArgs a) {
+// PAIR: two workgroups to a CU.  The queries stay in memory, read where they are used, times their rows' factors (77 KB are left in LDS of 64 rows of
+// 128 channels), and A is read again for every tile of the solve; bound by vector instructions.  2048 positions of 16 heads: 69 us with
+// one workgroup to a CU, 62 us so.  Up to one workgroup per CU the queries lie in LDS and A in registers; all three launches of the rows with it, against
+// PAIR there: 989 positions of 4 heads 86.8 and 90.0 us, 898 of 16 (100 channels) 71.9 and 74.8, 3 of 16 (vdim 64) 22.2 and 23.0.
+template <int C, bool VEC, bool PAIR>
+__global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_prepare_kernel(DeltaArgs a) {
   constexpr int NB = C / 16, NT = prepare_threads<C>(), NW = NT / 64;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int dp = a.dp, ds = dp + 4, chunk = blockIdx.x, h = blockIdx.y, g = h / (a.heads / a.kv_heads), row0 = chunk * C, rows = min(C, a.t - row0), d = a.dim;
@@ -114,7 +115,8 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
   float* B = K + C * ds;      // [C][ds]: log2 of the decays, summed from the start of a block of 16 rows
   float* A = B + C * ds;      // left operands of A up to the diagonal, then the inverses of I + A in the diagonal blocks
   float* beta = A + NB * (NB + 1) / 2 * 256;
-  float* unit = beta + C;     // what makes a query a unit vector, scaled; 0 past the last row
+  float* unit = beta + C;     // PAIR: what makes a query a unit vector, scaled; 0 past the last row
+  float* Q = unit + C;        // else: [C][ds]
   const size_t at = (size_t)chunk * a.heads + h;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, kg = lane >> 4;
   const int d4 = dp / 4;
@@ -122,12 +124,14 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   constexpr int AT_ONCE = 4;  // pieces of a thread on their way together: the decays' logarithms are long, and a load behind them would come late
   for (int e0 = threadIdx.x; e0 < C * d4; e0 += AT_ONCE * NT) {
-    f32x4_t k[AT_ONCE], l[AT_ONCE], bias[AT_ONCE];
+    f32x4_t k[AT_ONCE], l[AT_ONCE], bias[AT_ONCE], q[PAIR ? 1 : AT_ONCE];
 #pragma unroll
     for (int u = 0; u < AT_ONCE; ++u) {
       const int e = e0 + u * NT, r = e / d4, c = (e - r * d4) * 4, rr = min(r, rows - 1);
       k[u] = l[u] = bias[u] = zero;
+      if constexpr (!PAIR) q[u] = zero;
       if (c < d) {
+        if constexpr (!PAIR) q[u] = four<VEC>(a.qkv + (size_t)(row0 + rr) * a.qkv_stride + (size_t)g * d + c, d - c);
         k[u] = four<VEC>(a.qkv + (size_t)(row0 + rr) * a.qkv_stride + (size_t)(a.kv_heads + g) * d + c, d - c);
         l[u] = four<VEC>(a.a + (size_t)(row0 + rr) * a.a_stride + (size_t)h * d + c, d - c);
         bias[u] = four<VEC>(a.dt_bias + (size_t)h * d + c, d - c);
@@ -141,12 +145,14 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
       for (int x = 0; x < 4; ++x) l[u][x] = r < rows && c + x < d ? neg * softplus_f(l[u][x] + bias[u][x]) : 0.f;
       *reinterpret_cast<f32x4_t*>(K + r * ds + c) = r < rows ? k[u] : zero;
       *reinterpret_cast<f32x4_t*>(B + r * ds + c) = l[u];
+      if constexpr (!PAIR) *reinterpret_cast<f32x4_t*>(Q + r * ds + c) = r < rows ? q[u] : zero;
     }
   }
   if (threadIdx.x < C) beta[threadIdx.x] = (int)threadIdx.x < rows ? exact_sigmoid(a.b[(size_t)(row0 + threadIdx.x) * a.b_stride + h]) : 0.f;
   __syncthreads();
   // a query's four elements from c on, zeros past its last one
   auto query = [&](int r, int c) {
+    if constexpr (!PAIR) return *reinterpret_cast<const f32x4_t*>(Q + r * ds + c);
     const float* row = a.qkv + (size_t)(row0 + min(r, rows - 1)) * a.qkv_stride + (size_t)g * d;
     if constexpr (VEC) return c < d ? *reinterpret_cast<const f32x4_t*>(row + c) : zero;
     else return four<false>(row + c, d - c);
@@ -162,8 +168,11 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
       sq += q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
     }
     const float f = 1.f / sqrtf(row_sum16(ss) + UNIT_EPS), fq = q_scale / sqrtf(row_sum16(sq) + UNIT_EPS);
-    for (int c = j * 4; c < dp; c += 64) *reinterpret_cast<f32x4_t*>(row + c) *= f;
-    if (j == 0) unit[r] = r < rows ? fq : 0.f;
+    for (int c = j * 4; c < dp; c += 64) {
+      *reinterpret_cast<f32x4_t*>(row + c) *= f;
+      if constexpr (!PAIR) *reinterpret_cast<f32x4_t*>(Q + r * ds + c) *= fq;
+    }
+    if (PAIR && j == 0) unit[r] = r < rows ? fq : 0.f;
   }
   for (int x = threadIdx.x; x < dp * NB; x += NT) {
     float* col = B + (x / dp) * 16 * ds + x % dp;
@@ -173,6 +182,12 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
   }
   __syncthreads();
 
+  // of a unit query
+  auto unit_query = [&](int r, int c, float f) {
+    f32x4_t q = query(r, c);
+    if constexpr (PAIR) q *= f;
+    return q;
+  };
   float* P = a.p + at * C * C;
   auto row4 = [&](const float* m, int r, int c) { return *reinterpret_cast<const f32x4_t*>(m + r * ds + c); };
   auto tile_a = [&](int I, int J) { return A + (I * (I + 1) / 2 + J) * 256; };
@@ -183,7 +198,7 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
       I = 1;
       for (J = n - NB; J >= I; ++I) J -= I;
     }
-    const float uq = unit[16 * I + j];
+    const float uq = PAIR ? unit[16 * I + j] : 1.f;
     if (J < I) {
       f32x4_t acc[4] = {zero, zero, zero, zero};
       for (int c = 4 * kg; c < dp; c += 32) {
@@ -196,7 +211,7 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
           for (int M = J + 1; M < I; ++M) rest += row4(B, 16 * M + 15, cc);
           y[2 * u] = y[2 * u + 1] = row4(K, 16 * J + j, cc) * exp2_4(rest);
           x[2 * u] = row4(K, 16 * I + j, cc) * left;
-          x[2 * u + 1] = query(16 * I + j, cc) * uq * left;
+          x[2 * u + 1] = unit_query(16 * I + j, cc, uq) * left;
         }
         mfma16x16_each(x, y, acc);
       }
@@ -223,7 +238,7 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
           const f32x4_t l = row4(B, 16 * I + j, cc), k = row4(K, 16 * I + j, cc), left = exp2_4(l);
           y[2 * u] = y[2 * u + 1] = k * exp2_4(-l);
           x[2 * u] = k * left;
-          x[2 * u + 1] = query(16 * I + j, cc) * uq * left;
+          x[2 * u + 1] = unit_query(16 * I + j, cc, uq) * left;
         }
         mfma16x16_each(x, y, acc);
       }
@@ -240,7 +255,7 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
     float ak[4] = {0.f, 0.f, 0.f, 0.f}, aq[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 2
     for (int c = 0; c < dp; c += 4) {
-      const f32x4_t ki = row4(K, 16 * I + j, c), qi = query(16 * I + j, c) * uq, bi = row4(B, 16 * I + j, c);
+      const f32x4_t ki = row4(K, 16 * I + j, c), qi = unit_query(16 * I + j, c, uq), bi = row4(B, 16 * I + j, c);
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         const f32x4_t kj = row4(K, 16 * I + 4 * kg + x, c);
@@ -280,6 +295,13 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
   // (I + A) X = right-hand side, 16 columns per wave and turn: first the channels of beta G K, then the columns of beta V
   {
     auto m = [&](int I, int J) { return tile_of(A, I * (I + 1) / 2 + J, lane); };
+    f32x4_t held[PAIR ? 1 : NB][PAIR ? 1 : NB];
+    if constexpr (!PAIR) {
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int J = 0; J <= I; ++J) held[I][J] = m(I, J);
+    }
     const float* values = a.qkv + (size_t)row0 * a.qkv_stride + (size_t)2 * a.kv_heads * d + (size_t)h * a.vdim;
     const int kt = dp / 16, all = kt + a.vp / 16;
     f32x4_t ahead[NB];
@@ -288,7 +310,7 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
       const int c = (tile - kt) * 16 + j;
       const float* col = values + (c < a.vdim ? c : 0);
       size_t stride = a.qkv_stride;
-      asm volatile("" : "+s"(stride));  // (16 rows' addresses held over the loop would not leave registers for two workgroups)
+      if constexpr (PAIR) asm volatile("" : "+s"(stride));  // (16 rows' addresses held over the loop would not leave registers for two workgroups)
 #pragma unroll
       for (int I = 0; I < NB; ++I)
 #pragma unroll
@@ -325,9 +347,11 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
 #pragma unroll
         for (int J = 0; J < I; ++J) acc[J] = zero;
         f32x4_t mi[NB];
-        asm volatile("" ::: "memory");  // (read again for every tile: held over the loop they would not leave registers for two workgroups)
+        if constexpr (PAIR) asm volatile("" ::: "memory");  // (read again for every tile: held over the loop they would not leave registers for two workgroups)
 #pragma unroll
-        for (int J = 0; J <= I; ++J) mi[J] = m(I, J);
+        for (int J = 0; J <= I; ++J)
+          if constexpr (PAIR) mi[J] = m(I, J);
+          else mi[J] = held[I][J];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -350,7 +374,7 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (C == 64 ? 4 : 1)) del
     const int tile = e / 64, r = tile / (dp / 16) * 16 + (e & 15), c = tile % (dp / 16) * 16 + (e >> 4 & 3) * 4;
     f32x4_t l = row4(B, r, c);
     for (int M = 0; M < r / 16; ++M) l += row4(B, 16 * M + 15, c);
-    *reinterpret_cast<f32x4_t*>(QG + 4 * e) = query(r, c) * unit[r] * exp2_4(l);
+    *reinterpret_cast<f32x4_t*>(QG + 4 * e) = unit_query(r, c, PAIR ? unit[r] : 1.f) * exp2_4(l);
   }
   float* KD = a.kd + at * C * dp;
   for (int e = threadIdx.x; e < C * d4; e += NT) {
@@ -792,12 +816,12 @@ int check_delta(const ughip_device* dev, const ughip_delta* p, const char* what)
   return check_buf(dev, p->s, p->heads * p->dim * p->vdim, UGHIP_F32, what);
 }
 
-template <int C, bool VEC>
+template <int C, bool VEC, bool PAIR>
 int prepare(ughip_device* dev, const DeltaArgs& a) {
-  const size_t bytes = prepare_lds_floats<C>(a.dp) * sizeof(float);
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(delta_prepare_kernel<C, VEC>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  const size_t bytes = prepare_lds_floats<C, PAIR>(a.dp) * sizeof(float);
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(delta_prepare_kernel<C, VEC, PAIR>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   UGHIP_HIPCHK(attr);
-  delta_prepare_kernel<C, VEC><<<dim3((unsigned)a.chunks, (unsigned)a.heads), prepare_threads<C>(), bytes, dev->stream>>>(a);
+  delta_prepare_kernel<C, VEC, PAIR><<<dim3((unsigned)a.chunks, (unsigned)a.heads), prepare_threads<C>(), bytes, dev->stream>>>(a);
   UGHIP_HIPCHK(hipGetLastError());
   return UGHIP_OK;
 }
@@ -813,7 +837,10 @@ int scan_out(ughip_device* dev, const DeltaArgs& a) {
 }
 template <int C>
 int run_chunks(ughip_device* dev, const DeltaArgs& a, bool vec) {
-  if (int rc = vec ? prepare<C, true>(dev, a) : prepare<C, false>(dev, a)) return rc;
+  int rc = UGHIP_OK;
+  if (C == 64 && a.chunks * a.heads > dev->num_cus) rc = vec ? prepare<C, true, C == 64>(dev, a) : prepare<C, false, C == 64>(dev, a);
+  else rc = vec ? prepare<C, true, false>(dev, a) : prepare<C, false, false>(dev, a);
+  if (rc) return rc;
   return a.dp == 64 ? scan_out<C, 4>(dev, a) : a.dp == 128 ? scan_out<C, 8>(dev, a) : a.dp == 192 ? scan_out<C, 12>(dev, a) : scan_out<C, 16>(dev, a);
 }
 
