@@ -10,7 +10,7 @@ from gpu_calls import Gpu, View, Z, close, get, p, rand, view
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [4, 1024, 1028, 4096, 4100, 1026])
+@pytest.mark.parametrize("n", [4, 64, 68, 1024, 1028, 2048, 2052, 4096, 4100, 1026])
 @pytest.mark.parametrize("top", [1, 3, 4, 5, 9])
 @pytest.mark.parametrize("second", [False, True])
 def test_routed_rows_join_the_residual(hip, n, top, second):

@@ -90,12 +90,14 @@ __global__ void __launch_bounds__(256) add_rms_norm_kernel(AddNormArgs a) {
 // The same for up to 4096 elements, a multiple of 4, held in registers.  ROUTED: with slots, four of a row's rows of y on their way at a time,
 // added in order as above.  Everything that is read is asked for before the first sum, the norms' weights too: what bounds it on few rows is the
 // chain of loads and sums (509 rows of 2048 from four routed rows each: 20.8 us element by element, 7.0 so), on many the rows' way through
-// memory (2048 rows of 2048: 58 MB in 12.9 us; 13.4 with the weights asked for behind the sums).
-template <bool ROUTED>
+// memory (2048 rows of 2048 from one routed row each: 50 MB in 9.5 us).  U: groups of four elements of a thread, no more than
+// the row has; with registers for 4096 elements a CU held too few rows of any width (4096 rows of 120 from four routed rows 15.8 us, 7.2 element by
+// element, 7.0 so; without routed rows 8.1, 6.0 and 6.6).  Routed rows of up to 64 elements go element by element (4096 of 64 from eight: 9.7 here, 7.2).
+template <bool ROUTED, int U>
 __global__ void __launch_bounds__(256) add_rms_norm4_kernel(AddNormArgs a) {
   __shared__ float red[2][4];
   const size_t i = blockIdx.x;
-  f32x4_t v[4], x[4], e[4], w[4], nx[4];
+  f32x4_t v[U], x[U], e[U], w[U], nx[U];
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   float ss = 0.f;
   auto square = [](const f32x4_t& q) { return q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w; };
@@ -104,7 +106,7 @@ __global__ void __launch_bounds__(256) add_rms_norm4_kernel(AddNormArgs a) {
     return c < a.n && p ? *reinterpret_cast<const f32x4_t*>(p + at + c) : zero;
   };
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < U; ++u) {
     v[u] = ROUTED ? zero : get(a.y, i * a.y_stride, u);
     x[u] = get(a.x, i * a.x_stride, u);
     e[u] = get(a.extra, i * a.extra_stride, u);
@@ -113,7 +115,7 @@ __global__ void __launch_bounds__(256) add_rms_norm4_kernel(AddNormArgs a) {
   }
   if constexpr (ROUTED) {
     for (int j0 = 0; j0 < a.top; j0 += 4) {
-      f32x4_t t[4][4];
+      f32x4_t t[4][U];
       float by[4];
       bool there[4];
 #pragma unroll
@@ -122,17 +124,17 @@ __global__ void __launch_bounds__(256) add_rms_norm4_kernel(AddNormArgs a) {
         by[j] = a.weights[i * a.top + at];
         there[j] = j0 + j < a.top && r >= 0 && r < a.y_rows;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) t[j][u] = there[j] ? get(a.y, (size_t)r * a.y_stride, u) : zero;
+        for (int u = 0; u < U; ++u) t[j][u] = there[j] ? get(a.y, (size_t)r * a.y_stride, u) : zero;
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (there[j])
 #pragma unroll
-          for (int u = 0; u < 4; ++u) v[u] += by[j] * t[j][u];
+          for (int u = 0; u < U; ++u) v[u] += by[j] * t[j][u];
     }
   }
 #pragma unroll
-  for (int u = 0; u < 4; ++u) ss += square(v[u]);
+  for (int u = 0; u < U; ++u) ss += square(v[u]);
   ss = block_sum<4>(ss, red[0]);
   const float inv = 1.f / sqrtf(ss / (float)a.n + a.eps);
   auto put4 = [](void* dst, bool bf16, size_t at, const f32x4_t& q) {
@@ -141,7 +143,7 @@ __global__ void __launch_bounds__(256) add_rms_norm4_kernel(AddNormArgs a) {
   };
   ss = 0.f;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int c = (u * 256 + (int)threadIdx.x) * 4;
     if (c >= a.n) continue;
     if (a.y) v[u] = v[u] * inv * w[u] + x[u] + e[u];
@@ -154,7 +156,7 @@ __global__ void __launch_bounds__(256) add_rms_norm4_kernel(AddNormArgs a) {
   ss = block_sum<4>(ss, red[1]);
   const float inv2 = 1.f / sqrtf(ss / (float)a.n + a.eps);
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int c = (u * 256 + (int)threadIdx.x) * 4;
     if (c < a.n) put4(a.copy, a.copy_bf16, i * a.n + c, v[u] * inv2 * nx[u]);
   }
@@ -279,9 +281,10 @@ extern "C" int ughip_add_rms_norm_rows(ughip_device* dev, ughip_view x, ughip_vi
   AddNormArgs a{view_ptr<float>(x), view_ptr<float>(y), buf_ptr<float>(w), d, copy_at, view_ptr<float>(extra), buf_ptr<float>(next), x.stride, y.stride, dst.stride, extra.stride,
                 buf_ptr<int>(slots), buf_ptr<float>(weights), (int)top, (int)y_rows, (int)n, eps, bf16, copy_bf16};
   auto rows4 = [](const void* q, size_t stride) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0 && (!q || stride % 4 == 0); };
-  if (n % 4 == 0 && n <= 4096 && rows4(a.x, a.x_stride) && rows4(a.y, a.y_stride) && rows4(a.extra, a.extra_stride) && rows4(d, a.dst_stride)) {
-    if (slots) add_rms_norm4_kernel<true><<<(unsigned)m, 256, 0, dev->stream>>>(a);
-    else add_rms_norm4_kernel<false><<<(unsigned)m, 256, 0, dev->stream>>>(a);
+  if (n % 4 == 0 && n <= 4096 && (!slots || n > 64) && rows4(a.x, a.x_stride) && rows4(a.y, a.y_stride) && rows4(a.extra, a.extra_stride) && rows4(d, a.dst_stride)) {
+    auto go = [&](auto kernel) { kernel<<<(unsigned)m, 256, 0, dev->stream>>>(a); };
+    if (slots) n <= 1024 ? go(add_rms_norm4_kernel<true, 1>) : n <= 2048 ? go(add_rms_norm4_kernel<true, 2>) : go(add_rms_norm4_kernel<true, 4>);
+    else n <= 1024 ? go(add_rms_norm4_kernel<false, 1>) : n <= 2048 ? go(add_rms_norm4_kernel<false, 2>) : go(add_rms_norm4_kernel<false, 4>);
     UGHIP_HIPCHK(hipGetLastError());
     return UGHIP_OK;
   }
