@@ -11,7 +11,7 @@ from ug_amd import rng
 
 pytestmark = pytest.mark.gpu
 
-RING = {"10": "256x128", "6": "128x128", "7": "64x128", "9": "64x64"}  # GEMM_SHAPE -> tile
+RING = {"10": "256x128", "12": "128x128", "13": "64x128", "9": "64x64"}  # GEMM_SHAPE -> tile
 
 
 def rounded(dtype, v):
@@ -186,3 +186,15 @@ def test_rows_by_group(hip, tune, groups, rows):
         assert np.all(np.isnan(out[rows * n :])), "wrote what belongs to no group"
         if rows:
             close(out[: rows * n].reshape(rows, n), y, 2e-5)
+
+
+@pytest.mark.parametrize("shape, kernel", [("3", "gemm_dma4<bf16,NT,256x256,256t,rows>"), ("4", "gemm_dma4<bf16,NT,256x128,512t,ring,rows>"), ("5", "gemm_dma4<bf16,NT,128x128,512t,ring,rows>"),
+                                           ("0", "rows_product<bf16,none>"), ("6", "rows_product<bf16,none>"), ("7", "rows_product<bf16,none>")])
+def test_forced_tiles_of_rows(hip, tune, shape, kernel):
+    gpu, m, n, k = Gpu(hip), 70, 136, 320
+    x, w = rand(1, m, k), rand(2, n, k, std=k ** -0.5)
+    dx, dw, dst = gpu.up(x, bf16=True), gpu.up(w, bf16=True), gpu.out(m * n)
+    tune.setenv("UGHIP_GEMM_SHAPE", shape)
+    gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=BF16, act=NONE)))
+    assert ug_amd.last_kernel() == kernel
+    close(get(dst, (m, n)), x @ w.T, 2e-5)

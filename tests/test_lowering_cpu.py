@@ -402,3 +402,27 @@ def test_narrow_products_with_a_long_k_take_the_kernel_that_splits_it():
         assert _rows_plan(B, 1, 0, m, n, k).startswith("gemm_tiled"), (m, n, k)
     for m, n, k in [(505, 136, 4352), (396, 160, 512)]:
         assert "ring,3 planes" in _rows_plan(B, 1, 0, m, n, k), (m, n, k)
+
+
+def test_forced_tiles_are_the_ones_that_their_numbers_name():
+    """UGHIP_GEMM_SHAPE and UGHIP_X3_DMA: 0..2, 6 and 7 the register-staged kernel's tiles, for 16-bit products too; 3..5 gemm_dma4's, 9..13 the ring's."""
+    B, F = ug_amd.BF16, ug_amd.F32
+    staged = {0: "256x128", 1: "128x128", 2: "128x64", 6: "64x128", 7: "32x128"}
+    lds = {3: "256x256,256t", 4: "256x128,256t", 5: "128x128,256t", 10: "256x128,512t,ring", 12: "128x128,512t,ring", 13: "64x128,512t,ring", 9: "64x64,512t,ring"}
+    for shape, tile in staged.items():
+        with ug_amd.tuning(GEMM_SHAPE=shape):
+            m = 60 if shape > 2 else 512  # (at most two of the small tiles' rows)
+            assert _plan(B, B, 1, m, 1024, 512, 1).startswith(f"gemm_tiled<bf16,NT,{tile},"), shape
+            assert _plan(F, F, 1, m, 1024, 512, 1).startswith(f"gemm_tiled<f32,NT,{tile},"), shape
+    for shape, tile in lds.items():
+        with ug_amd.tuning(GEMM_SHAPE=shape):
+            assert _plan(B, B, 1, 512, 1024, 512, 1) == f"gemm_dma4<bf16,NT,{tile}>", shape
+    auto = _rows_plan(B, 1, 0, 1900, 2048, 2048)
+    for shape in (3, 4, 5, 9, 12, 13):
+        with ug_amd.tuning(X3_DMA=shape, X3_SPLIT=1):
+            assert _rows_plan(B, 1, 0, 1900, 2048, 2048) == f"gemm_dma4<bf16,NT,{lds[shape]},3 planes,f32 out>", shape
+    for shape in (6, 7, 10, 11, 99):  # no tile of this product: as if not set
+        with ug_amd.tuning(X3_DMA=shape):
+            assert _rows_plan(B, 1, 0, 1900, 2048, 2048) == auto, shape
+    with ug_amd.tuning(X3_DMA=0):
+        assert _rows_plan(B, 1, 0, 1900, 2048, 2048).startswith("gemm_tiled")

@@ -453,17 +453,17 @@ static size_t tile_count(const MMArgs& p, size_t batch, int tile) {  // 0: no su
 static bool ring_tile(int tile) { return tile == 129 || tile == 97 || tile == 65 || tile == 48 || tile == 32; }
 static int least_k(int tile) { return ring_tile(tile) ? BK : 4 * BK; }
 static const char* waves_name(int tile) { return ring_tile(tile) ? "512t,ring" : "256t"; }  // in the names of these kernels
-// (tuning aid) the tile code that GEMM_SHAPE names, 0: none
+// (tuning aid) the tile code that GEMM_SHAPE names, 0: none of these kernels'
 int gemm_dma_forced_tile(long long shape) {
   switch (shape) {
     case 3: return 256;
     case 4: return 128;
     case 5: return 64;
-    case 6: return 65;
-    case 7: return 48;
     case 9: return 32;
     case 10: return 129;
     case 11: return 97;
+    case 12: return 65;
+    case 13: return 48;
   }
   return 0;
 }
@@ -513,7 +513,7 @@ static double ring_cost_us(size_t tiles, int kt, int tile, Operands from) {
 // (3072 x 4096^2: 131 -> 91 us, 5120^2 x 1024: 77 -> 54, 1280 x 8192 x 2048: 64 -> 47, 2048 x 2560 x 2048: 35 -> 29,
 // 2304^3: 39 -> 35) and leaves those with about 128 tiles where they were (2048^2 x 5632: 56 us against 72).  The
 // 128 x 128 tile (two workgroups per CU) takes what neither fits: 2304^3 35 -> 31 us, 2048 x 2560 x 2048 29 -> 27.
-// UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 10 / 11 / 6 / 7 / 9 the ring's tiles, 0..2 keeps both out (tuning aid).
+// UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 10 / 12 / 13 / 9 the ring's 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64, 0..2, 6 and 7 keep both out (tuning aid).
 double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
   const size_t tiles = tile_count(p, batch, tile);
   if (!tiles) return 1e30;
@@ -656,7 +656,7 @@ bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int
 
 int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
   if (long long s; tune_get(TUNE_GEMM_SHAPE, &s)) {  // tuning aid, as for gemm_dma_pick
-    const int forced = gemm_dma_forced_tile(s);
+    const int tile = gemm_dma_forced_tile(s), forced = tile == 128 ? 129 : tile == 64 ? 65 : tile;  // (256 x 128 and 128 x 128 tiles of rows are the ring's)
     return forced && gemm_dma_rows_supported(p, r, act, forced) ? forced : 0;
   }
   // A model's products: the matrix comes from memory.  256 x 256 tiles of gemm_dma4 and the ring's, by what they are expected to take

@@ -304,13 +304,15 @@ hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, const float
 
 template <typename T, bool F32OUT, int BDIV, int ROWS>
 hipError_t launch_nt(hipStream_t stream, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw) {
-  if (tile == 129) return launch<T, 256, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+  if constexpr (BDIV == 1) {
+    if (tile == 129) return launch<T, 256, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+  }
   if constexpr (ROWS == 1 || ROWS == 2) {
     if (tile == 97) return launch<T, 192, 192, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
   }
   if (tile == 65) return launch<T, 128, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
   if (tile == 48) return launch<T, 64, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
-  return launch<T, 64, 64, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+  return tile == 32 ? launch<T, 64, 64, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw) : hipErrorInvalidValue;
 }
 template <typename T>
 hipError_t launch_plain(hipStream_t stream, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw) {

@@ -75,13 +75,13 @@ const char* dtype_name(int dt);
 // through ughip_set_tuning: dispatch reads an atomic, never the environment, so a launch thread and a test that
 // flips a switch do not meet in getenv / setenv.
 enum TuneKey {
-  TUNE_GEMM_SHAPE,          // 0..2: a gemm_tiled tile (keeps gemm_dma4 out); 3 / 4 / 5: gemm_dma4 with 256x256 / 256x128 / 128x128; 10 / 11 / 6 / 7 / 9: gemm_ring with 256x128 / 192x192 (rows) / 128x128 / 64x128 / 64x64; 8: gemm_dma_f32 for f32 products
+  TUNE_GEMM_SHAPE,          // 0..2, 6, 7: a gemm_tiled tile (keeps gemm_dma4 and gemm_ring out); 3 / 4 / 5: gemm_dma4 with 256x256 / 256x128 / 128x128 (products of rows: gemm_ring's of the latter two); 10 / 11 / 12 / 13 / 9: gemm_ring with 256x128 / 192x192 (rows) / 128x128 / 64x128 / 64x64; 8: gemm_dma_f32 for f32 products
   TUNE_GEMM_SPLIT,          // K split of gemm_tiled
   TUNE_GEMM_4WAVES,         // (set at all) the 256-thread form of the 256x128 tile
   TUNE_GEMV_KS,             // waves per output column of the GEMV family: 1, 2 or 4
   TUNE_GEMV_ROWS,           // rows per workgroup of fused_gemv_bf16_rows: 1, 2, 4 or 8
   TUNE_GEMV_BF16_ROWS,      // 0: bf16 matrices take the f32 kernels' lane layout
-  TUNE_X3_DMA,              // three-term bf16 products: 0 keeps gemm_tiled, values of GEMM_SHAPE force a tile
+  TUNE_X3_DMA,              // three-term bf16 products: 0 keeps gemm_tiled; 3 / 4 / 5, 12 / 13 / 9 force the tile that GEMM_SHAPE names so; others: as if not set
   TUNE_X3_SPLIT,            // K split of the three-term product on gemm_dma4
   TUNE_X3_ROWS,             // three-term bf16 products of 65 .. 128 rows: 0 keeps the kernels that take planes, n > 0 forces n units per workgroup of rows_x3
   TUNE_ATT_SPLIT,           // key ranges per head of single-query attention
