@@ -32,10 +32,13 @@ int ughip_gather_rows(ughip_device* dev, const ughip_slice* table, size_t table_
 /* ---- products of rows ---------------------------------------------------------------------------------------------------
  * dst = act(x w^T + bias), any m, n, k.  `product`:
  *   UGHIP_PRODUCT_F32   x and w F32, the f32 matrix pipe;
- *   UGHIP_PRODUCT_BF16  x and w rounded to (or stored as) bf16, the bf16 matrix pipe, f32 accumulation.  (2 .. 128 dense F32 rows
- *                       against a BF16 matrix of regular sizes keep their F32 values: the kernels of ughip_linear_rows.)
- * x, w and dst may each be F32 or BF16 (F32 only for UGHIP_PRODUCT_F32).  BF16 rows and matrices of regular sizes take the
- * one-wave-per-SIMD kernel of ughip_matmul, the rest one that takes any size (ughip_last_kernel names it).
+ *   UGHIP_PRODUCT_BF16  x and w rounded to (or stored as) bf16, the bf16 matrix pipe, f32 accumulation.  (Some dense F32 rows without bias
+ *                       or act keep their F32 values: 2 .. 128 against a BF16 matrix of regular sizes, by the kernels of
+ *                       ughip_linear_rows; one with k >= 512, k % 4 == 0, x and dst different slices at offset 0 and rows of w k
+ *                       elements apart, by ughip_gemv_multi, which keeps those of an F32 matrix too.)
+ * x, w and dst may each be F32 or BF16 (F32 only for UGHIP_PRODUCT_F32).  BF16 rows and matrices with k % 64 == 0 and 16-byte aligned
+ * rows take the 16-bit kernels of ughip_matmul whose loads write LDS (256 x 256 tiles, or the ring of stages with smaller ones), the
+ * rest one that takes any size (ughip_last_kernel names it).
  * `act`:
  *   UGHIP_ACT_NONE      dst[m, n] = y;
  *   UGHIP_ACT_SWIGLU    w is [2 n, k], gate rows then up rows (and bias 2 n values): dst = silu(y_gate) * y_up;

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import ug_amd
-from gpu_calls import BF16, GLU, NONE, SWIGLU, Gpu, Product, close, get, p, rand, view
+from gpu_calls import BF16, F32, GELU_MUL, GLU, NONE, SWIGLU, Gpu, Product, close, get, p, rand, view
 from test_gpu_parity import _raw_matmul
 from ug_amd import rng
 
@@ -198,3 +198,100 @@ def test_forced_tiles_of_rows(hip, tune, shape, kernel):
     gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=BF16, act=NONE)))
     assert ug_amd.last_kernel() == kernel
     close(get(dst, (m, n)), x @ w.T, 2e-5)
+
+
+def _random_products():
+    gen = np.random.default_rng(17)
+    out = [(1, 130, 136, 64, "bf16", True), (2, 65, 264, 128, "f16", False), (1, 300, 72, 192, "bf16", False), (1, 257, 392, 64, "f16", False), (3, 9, 8, 128, "bf16", False), (1, 64, 64, 192, "f16", True)]
+    for _ in range(18):
+        b, m, n, kt = int(gen.integers(1, 4)), int(gen.integers(9, 600)), 8 * int(gen.integers(1, 60)), int(gen.integers(1, 12))
+        out.append((b, m, n, 64 * kt, ("bf16", "f16")[int(gen.integers(2))], bool(gen.integers(2))))
+    return out
+
+
+# one to three K tiles, where only the tail of the loop runs, in both layouts and types, and sizes as they come
+@pytest.mark.parametrize("b, m, n, k, dtype, rhs_nk", _random_products())
+def test_ring_tiles_give_the_other_kernels_bits(hip, tune, b, m, n, k, dtype, rhs_nk):
+    """Every tile of the ring sums in the order of the register-staged kernel (without a K split): the same bits, on values that any other order would
+    round otherwise."""
+    dt = ug_amd.BF16 if dtype == "bf16" else ug_amd.F16
+    a, w = rounded(dtype, rng.normal(1, b * m * k)).reshape(b, m, k), rounded(dtype, rng.normal(2, b * k * n)).reshape(b, k, n)
+    tune.setenv("UGHIP_GEMM_SPLIT", "1")
+    ref = None
+    if rhs_nk or n % 128 == 0:  # (whole column tiles for a [k, n]-major rhs)
+        tune.setenv("UGHIP_GEMM_SHAPE", "1")
+        ref = _raw_matmul(hip, dt, a, w, rhs_nk)
+        assert ug_amd.last_kernel().startswith("gemm_tiled<")
+    elif k >= 256:
+        tune.setenv("UGHIP_GEMM_SHAPE", "5")
+        ref = _raw_matmul(hip, dt, a, w, rhs_nk)
+        assert ug_amd.last_kernel().startswith("gemm_dma4<") and "ring" not in ug_amd.last_kernel()
+    exact = np.matmul(a.astype(np.float64), w.astype(np.float64))
+    bound = (2.0 ** -8 if dtype == "bf16" else 2.0 ** -11) * np.abs(exact) + k * np.finfo(np.float32).eps * np.matmul(np.abs(a).astype(np.float64), np.abs(w).astype(np.float64))
+    for shape, tile in RING.items():
+        if shape == "9" and not rhs_nk:
+            continue
+        tune.setenv("UGHIP_GEMM_SHAPE", shape)
+        print("ring bits", dtype, b, m, n, k, "NT" if rhs_nk else "NN", tile, flush=True)
+        got = _raw_matmul(hip, dt, a, w, rhs_nk)
+        assert ug_amd.last_kernel() == f"gemm_dma4<{dtype},{'NT' if rhs_nk else 'NN'},{tile},512t,ring>"
+        assert np.all(np.abs(got - exact) <= bound * 1.001 + 1e-7)
+        if ref is None:
+            ref = got  # (neither of the others takes it: the tiles among themselves)
+        np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("m, n, k", [(1, 8, 64), (70, 136, 320), (193, 72, 192), (300, 264, 128)])
+@pytest.mark.parametrize("table_bf16", [True, False])
+@pytest.mark.parametrize("out_bf16", [True, False])
+def test_ring_rows_times_a_lookup(hip, tune, m, n, k, table_bf16, out_bf16):
+    """gelu(y) times an element of a table row, on every tile that has the form: tables and results of either type, ids outside the table."""
+    gpu, rows, col = Gpu(hip), 13, 4
+    x, w, bias, table = rand(1, m, k), rand(2, n, k, std=k ** -0.5), rand(3, n, std=0.5), rand(4, rows, n + 6)
+    ids = (np.arange(m) * 5 % rows).astype(np.int32)
+    ids[m // 2], ids[m - 1] = (-1, rows) if m > 1 else (rows, rows)
+    y = x @ w.T + bias
+    inside = (ids >= 0) & (ids < rows)
+    want = 0.5 * y * (1 + np.tanh(np.sqrt(2 / np.pi) * (y + 0.044715 * y ** 3))) * table[np.where(inside, ids, 0)][:, col : col + n]
+    dx, dw, db, dt, di = gpu.up(x, bf16=True), gpu.up(w, bf16=True), gpu.up(bias), gpu.up(table, bf16=table_bf16), gpu.up(ids)
+    for shape in (None, "10", "12", "13", "9"):
+        if shape:
+            tune.setenv("UGHIP_GEMM_SHAPE", shape)
+        dst = gpu.out(m * n + 8, bf16=out_bf16)
+        print("lookup rows", m, n, k, table_bf16, out_bf16, shape, flush=True)
+        gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), bias=db.raw(), m=m, n=n, k=k, product=BF16, act=GELU_MUL, table=dt.raw(), ids=di.raw(),
+                                                       table_rows=rows, table_stride=n + 6, table_col=col)))
+        assert ",512t,ring,rows,lookup>" in ug_amd.last_kernel() and (shape is None or RING[shape] in ug_amd.last_kernel())
+        out = get(dst, m * n + 8)
+        assert np.all(np.isnan(out[m * n :])), "wrote past the end"
+        out = out[: m * n].reshape(m, n)
+        assert np.all(np.isnan(out[~inside]))
+        if inside.any():
+            close(out[inside], want[inside], 2e-5, rel=2.0 ** -8 if out_bf16 else 0.0)
+
+
+@pytest.mark.parametrize("k", [512, 516, 2048, 9000])
+@pytest.mark.parametrize("n", [1, 77, 2000])
+@pytest.mark.parametrize("w_bf16, mode", [(True, BF16), (False, BF16), (False, F32)])
+def test_one_row_keeps_its_f32_values(hip, n, k, w_bf16, mode):
+    """One dense f32 row goes to the decode kernels: neither it nor an F32 matrix is rounded to bf16, whatever the product is called."""
+    gpu, eps = Gpu(hip), np.finfo(np.float32).eps
+    x, w = rng.normal(1, k).astype(np.float64), (rand(2, n, k, std=k ** -0.5) if w_bf16 else rng.normal(2, n * k, k ** -0.5).reshape(n, k).astype(np.float64))
+    dx, dw, dst = gpu.up(np.concatenate([x, np.full(8, np.nan)])), gpu.up(w, bf16=w_bf16), gpu.out(n + 8)
+    gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k + 8), dst=view(dst, 0, n), w=dw.raw(), m=1, n=n, k=k, product=mode, act=NONE)))
+    assert ug_amd.last_kernel() == f"rows_product<{'f32' if mode == F32 else 'bf16'},one row>"
+    out = get(dst, n + 8)
+    assert np.all(np.isnan(out[n:])), "wrote past the end"
+    assert np.all(np.abs(out[:n] - w @ x) <= k * eps * (np.abs(w) @ np.abs(x)))
+
+
+@pytest.mark.parametrize("k, bias, offset", [(256, False, 0), (511, False, 0), (512, True, 0), (512, False, 4)])
+def test_one_row_elsewhere_is_rounded(hip, k, bias, offset):
+    """A row with a bias, at an offset, or short: rounded to bf16 in front of the product, as several rows are."""
+    gpu, n = Gpu(hip), 40
+    x, w, b = rng.normal(1, k), rand(2, n, k, std=k ** -0.5), rand(3, n)
+    want = w @ rng.bf16_round(x).astype(np.float64) + (b if bias else 0)
+    dx, dw, db, dst = gpu.up(np.concatenate([np.zeros(offset), x])), gpu.up(w, bf16=True), gpu.up(b), gpu.out(n)
+    gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, offset, k), dst=view(dst, 0, n), w=dw.raw(), bias=db.raw() if bias else None, m=1, n=n, k=k, product=BF16, act=NONE)))
+    assert "one row" not in ug_amd.last_kernel()
+    close(get(dst, n), want, 2e-5)

@@ -550,10 +550,11 @@ int gemm_dma_pick(int dtype, const MMArgs& p, size_t batch) {
   int best = 0;
   double best_us = 0;
   // The ring where 128 x 128 tiles would leave CUs without one (us by box, best of gemm_dma4 and gemm_tiled -> ring: 1024^3 [k, n]-major
-  // 11.4 -> 7.9, 2048 x 1024^2 10.8 -> 8.2, 1024 x 2048 x 4096 28.7 -> 21.1 and 37.3 -> 24.5, 1536^3 16.2 -> 13.1, 96^2 x 4096 [k, n]-major 33 -> 15.4).  From
-  // there on 2304^3 says 31.0 against 37.1.  An [n, k]-major rhs under a handful of tiles with a short K stays with gemm_tiled and its K split:
-  // the callers that count on that kernel there (the tests among them) keep it, and so do up to 128 rows whose K it splits over workgroups (at 64 x
-  // 2048 x 2048 it takes 11.6 us against 7.7, with N = 256 it is the faster one).
+  // 11.4 -> 7.9, 2048 x 1024^2 10.8 -> 8.2, 1024 x 2048 x 4096 28.7 -> 21.1 and 37.3 -> 24.5, 1536^3 16.2 -> 13.1, 96^2 x 4096 [k, n]-major 33 -> 15.4).
+  // Past one round 2304^3 takes 29.2 in place of the ring's 33.4.  Three kinds of product keep their plans, which callers hold them to, though the
+  // ring is the faster one for most of them (us there / ring): exactly one round of tiles (2048^3 23.5 / 20.0, 2048^2 x 5632 54.5 / 42.8, 4 x 1024^3 13.1 / 9.9);
+  // [n, k]-major, up to 64 tiles, K up to 1024 (1024^3 10.3 / 6.3, 512^3 6.5 / 5.6, 64^2 x 1024 8.7 / 5.6, 64^2 x 128 6.2 / 5.6); up to 128 rows
+  // whose K gemm_tiled splits (64 x 2048^2 10.8 / 7.7, 128 x 256 x 2048 9.8 / 7.8; 64 x 256 x 4096 11.5 / 12.5, 64 x 2048 x 4096 12.6 / 13.5).
   const size_t tiles = batch * (size_t)((p.M + 127) / 128) * (size_t)((p.N + 127) / 128);
   const bool few = tiles < 256 && !(p.b_rs == 1 && tiles <= 64 && p.K <= 1024) && !(p.M <= 128 && gemm_tiled_workspace_bytes(dtype, p, batch) != 0);
   for (int tile : {256, 128, 64, 65, 48, 32}) {

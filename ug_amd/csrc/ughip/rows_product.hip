@@ -379,7 +379,7 @@ extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
   const bool xb = p->x.s->dtype == UGHIP_BF16, wb = p->w->dtype == UGHIP_BF16;
   // one row (the head behind a prompt): the decode kernels, which stream the matrix past f32 values of the row (32000 x 2048 bf16: 22 us against 36 here)
   if (p->m == 1 && !xb && !a.dst_bf16 && p->act == UGHIP_ACT_NONE && !a.bias && !p->groups && w_stride == p->k && p->k % 4 == 0 && p->k >= 512 && p->x.offset == 0 &&
-      p->dst.offset == 0 && p->dst.s != p->x.s) {
+      p->dst.offset == 0 && p->dst.s != p->x.s && p->dst.s != p->w) {
     const ughip_slice* w = p->w;
     if (int rc = ughip_gemv_multi(dev, p->x.s, 1, &w, &p->n, p->k, p->dst.s)) return rc;
     note_kernel("rows_product<%s,one row>", f32 ? "f32" : "bf16");
