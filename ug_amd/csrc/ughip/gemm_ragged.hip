@@ -8,7 +8,7 @@
 //   what does not exist, and comes first, under the way of the next ones: it holds the only row of a
 //   [k, n]-major operand behind which nothing may be read.
 //
-// What bounds it: the steps' latency on few tiles (0.35 us each in 16 bits, 0.6 in f32), LDS and the f32 matrix pipe on many.  Against element-by-element
+// What bounds it: the steps' latency on few tiles (0.4 us each in 16 bits, 0.6 in f32), LDS and the f32 matrix pipe on many.  Against element-by-element
 // loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 14.6 us, f32 256 -> 34; 2001^3 f16 270 -> 37, f32 340 -> 135; 3999^2 x
 // 2000 f16 1204 -> 103, f32 1014 -> 520; 100^3 9.4 -> 5.4.  Which tile takes what: gemm_ragged_tile.
 #include <hip/hip_runtime.h>

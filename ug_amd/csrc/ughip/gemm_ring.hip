@@ -6,9 +6,9 @@
 //   A ring of four stages (three for the two largest tiles): the loads of a K tile go out (global_load_lds_dwordx4, as in gemm_dma4) when the tile that
 //   many in front of it has been read, so three (two) tiles are on their way while one is multiplied.  One barrier per K tile.
 //
-// What bounds it: the operands' way to a CU.  2048^2 x 5632 on 128 x 128 tiles, one to a CU, takes 0.51 us per K tile of 32 KB with the operands in
-// the memory-side cache and 0.55 with the matrix from HBM (gemm_dma4's two stages: 0.85); the same kernel without its MFMAs takes 0.38 / 0.54,
-// without its loads 0.35-0.39, and a loop of nothing but the loads 0.33 / 0.52: a CU gets some 100 / 60 bytes per ns however many loads it has
+// What bounds it: the operands' way to a CU.  2048^2 x 5632 on 128 x 128 tiles, one to a CU, takes 42 us, 0.44 per K tile of 32 KB, with the operands in
+// the memory-side cache (matrix pipes busy 61 % of the time) and 54 us, 0.57, with both from HBM (42 %); gemm_dma4's two stages 58 and 75.  From HBM
+// it takes as long without its MFMAs, and a loop of nothing but the loads takes 0.33 / 0.52 us: a CU gets some 100 / 60 bytes per ns however many it has
 // on their way (deeper rings, loads that bypass the cache and a wave that touches the lines for L2 ahead of the others made nothing faster).
 // So tiles are as large as leaves every CU one, by the model in gemm_dma.hip.
 #include <hip/hip_runtime.h>
