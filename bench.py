@@ -7,8 +7,9 @@ is one run of the compiled schedule (one kernel launch) with a and b resident in
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--headline-only]
 
-The other single-GPU configs (softmax sweep, batched matmul, llama pieces, llama decode) are
-reported under "extras" of the same line; --headline-only (or --no-extras / --no-llama) leaves
+The JSON line is the last one and short: the headline, its roofline and one figure per config.  Everything
+else (each config in full, the softmax sweep, batched matmul, llama pieces, llama decode) is printed ahead of
+it, a line per entry that starts with "detail " and the entry's name; --headline-only (or --no-extras / --no-llama) leaves
 them out, which is what the profiler runs use.  Only one GPU is ever used.
 """
 import argparse
@@ -1126,6 +1127,41 @@ def config_summary(line):
     return out
 
 
+SHORT_CONFIGS = (("c1_softmax_lazy_32x1024", "us_per_softmax"), ("c3_bmm_f32_8x1024^3", "TFLOP/s"), ("c3_bmm_bf16_8x1024^3", "TFLOP/s"), ("mm_bf16_nt_4096^3", "TFLOP/s"),
+                 ("c4_rms_norm_512x2048", "us"), ("c4_softmax_lazy_1x32x512x512", "us"), ("c4_attention_cached_t512", "us"),
+                 ("c5_decode_f32_fused_level3", "tok/s"), ("c5_decode_bf16_matrices_level3", "tok/s"), ("c5_unit_norms_prompt1900_bf16_matrices_prefill_bf16x3", "prefill_ms"))
+SHORT_ROOFLINE = ("bound", "achieved", "peak", "unit", "frac", "step_us", "kernel_us", "kernel_frac", "fold_kernel_us", "sustained_frac", "traffic", "traffic_source")
+
+
+def details(line):
+    """(name, value) of everything the run measured: the entries of `extras` and of `roofline.configs` one by one."""
+    for key, value in line.items():
+        if key == "extras" and isinstance(value, dict):
+            yield from ((f"extras.{k}", v) for k, v in value.items())
+        elif key == "roofline":
+            yield key, {k: v for k, v in value.items() if k != "configs"}
+            yield from ((f"roofline.configs.{k}", v) for k, v in value.get("configs", {}).items())
+        elif isinstance(value, (dict, list)):
+            yield key, value
+
+
+def short_line(line):
+    """The line that a program reads: under 2000 characters, so that a log which keeps only its end still holds it."""
+    out = {k: v for k, v in line.items() if not isinstance(v, (dict, list))}
+    out["config"] = line["config"]
+    rf = line["roofline"]
+    out["roofline"] = {k: rf[k] for k in SHORT_ROOFLINE if k in rf}
+    if isinstance(line.get("cpu_baseline"), dict):
+        out["cpu_baseline"] = {**line["cpu_baseline"], "sample": line["cpu_baseline"].get("sample", "").split(" (")[0]}
+    configs = rf.get("configs", {})
+    # a config that failed says so here: its message is with the details
+    out["configs"] = {f"{k} {unit}": configs[k][unit] if unit in configs[k] else "error" for k, unit in SHORT_CONFIGS if k in configs}
+    failed = [k for k, v in line.get("extras", {}).items() if k == "error" or (isinstance(v, dict) and "error" in v)]
+    if failed:
+        out["failed"] = failed[:4]
+    return out
+
+
 def decode_launch_floor_model(ex):
     """A decode step as a chain of dependent launches: launches x the measured time of one dependent launch + the weights at
     the rate a read-only stream beyond the caches reaches on this box.  measured / model says how much of the miss against the
@@ -1182,7 +1218,7 @@ def main():
 
     # The timed region (W warm-up steps, then exactly K steps between synchronisations) is run three times and the
     # median run is the one reported: K = 200 steps are 4 ms of GPU time, and one scheduler hiccup on the host
-    # moves a single run's wall clock by 20 %.  All three are kept in the line ("runs").
+    # moves a single run's wall clock by 20 %.  All three are reported ("runs").
     runs = sorted((timed(dev, cs.run, args.steps, args.warmup) for _ in range(3)), key=lambda t: t[0])
     wall, ev_ms = runs[1]
     ms_per_step = wall * 1e3 / args.steps
@@ -1291,7 +1327,9 @@ def main():
     model = decode_launch_floor_model(line.get("extras", {}))
     if model:
         line["roofline"]["launch_floor_model"] = model
-    print(json.dumps(line), flush=True)
+    for name, entry in details(line):
+        print(f"detail {name} {json.dumps(entry)}")
+    print(json.dumps(short_line(line)), flush=True)
 
 
 if __name__ == "__main__":
