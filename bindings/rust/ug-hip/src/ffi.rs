@@ -114,6 +114,29 @@ extern "C" {
         name: *const c_char,
         out: *mut *mut UghipFunc,
     ) -> c_int;
+    pub fn ughip_compile_rows_pair(
+        dev: *mut UghipDevice,
+        first: *const UghipSsa,
+        second: *const UghipSsa,
+        names: *const *const c_char,
+        shared: *const c_int,
+        n_shared: usize,
+        link: c_int,
+        keep: c_int,
+        out: *mut *mut UghipFunc,
+    ) -> c_int;
+    pub fn ughip_codegen_rows_pair(
+        first: *const UghipSsa,
+        second: *const UghipSsa,
+        names: *const *const c_char,
+        shared: *const c_int,
+        n_shared: usize,
+        link: c_int,
+        keep: c_int,
+        buf: *mut c_char,
+        buf_len: usize,
+        out_len: *mut usize,
+    ) -> c_int;
     pub fn ughip_func_release(f: *mut UghipFunc) -> c_int;
     pub fn ughip_run(dev: *mut UghipDevice, f: *mut UghipFunc, args: *const *mut UghipSlice, n_args: usize) -> c_int;
     pub fn ughip_run_part(

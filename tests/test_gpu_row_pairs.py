@@ -1,0 +1,114 @@
+"""Row kernels that hold their rows in registers, and two of them as one launch: widths around the groups of four, the waves and the rows per
+workgroup, what somebody else can see of the buffer between the two, and neighbours that must stay two launches."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import ug_amd
+from ug_amd import LazyBuffer as LB
+from ug_amd import Schedule
+
+EPS32 = 2.0 ** -24
+
+
+def _x(seed, *shape):
+    return np.random.default_rng(seed).standard_normal(shape).astype(np.float32)
+
+
+def _softmax(x):
+    e = np.exp(x.astype(np.float64) - x.max(-1, keepdims=True))
+    return e / e.sum(-1, keepdims=True)
+
+
+def _parts(x, weight=None, dev=None):
+    """The softmax in steps, so that the buffer between its kernels has a name here: (exponentials, result)."""
+    wide = lambda r: r.broadcast(x.shape)  # noqa: E731
+    lx = LB.copy(x, x.shape, dev)
+    e = lx.binary("sub", wide(lx.reduce("max", len(x.shape) - 1))).unary("exp")
+    out = e.binary("div", wide(e.reduce("sum", len(x.shape) - 1)))
+    return e, out if weight is None else out.binary("mul", wide(LB.copy(weight, (1,) * (len(x.shape) - 1) + weight.shape, dev)))
+
+
+def _joined(lb, keep=0):
+    """The source of the first two items of a graph as one launch, '' where they stay two; needs no device."""
+    s = Schedule.create_one(lb)
+    ka, kb = s.item_ssa(0), s.item_ssa(1)
+    a, b, lib = ka.wire(), kb.wire(), ug_amd.ughip_lib()
+    names, n = (C.c_char_p * 2)(b"first", b"second"), C.c_size_t()
+    shared = (C.c_int * b.n_args)(*([a.n_args - 1] + [-1] * (b.n_args - 1)))
+    args = (C.byref(a), C.byref(b), names, shared, C.c_size_t(b.n_args), C.c_int(a.n_args - 1), C.c_int(keep))
+    assert lib.ughip_codegen_rows_pair(*args, None, C.c_size_t(0), C.byref(n)) == 0, lib.ughip_last_error()
+    buf = C.create_string_buffer(n.value + 1)
+    assert lib.ughip_codegen_rows_pair(*args, buf, C.c_size_t(n.value + 1), C.byref(n)) == 0
+    return buf.value.decode()
+
+
+def test_which_neighbours_are_joined(cpu):
+    kernel = lambda src: src[src.index("__global__"):]  # noqa: E731
+    for shape in [(1, 4), (7, 333), (5, 256), (3, 8192), (2, 3, 49152)]:
+        src = kernel(_joined(_parts(_x(1, *shape), dev=cpu)[1]))
+        assert "ug_link" in src and src.count("__restrict__") == 2, shape  # what lies between is no argument
+        assert kernel(_joined(_parts(_x(1, *shape), dev=cpu)[1], keep=1)).count("__restrict__") == 3
+    assert _joined(_parts(_x(1, 2, 3), dev=cpu)[1]) == ""  # rows shorter than a group
+    assert _joined(_parts(_x(1, 2, 49153), dev=cpu)[1]) == ""  # more than a thread holds
+    e, _ = _parts(_x(1, 64, 64), dev=cpu)
+    t = e.transpose(0, 1)
+    assert _joined(t.binary("div", t.reduce("sum", 1).broadcast((64, 64)))) == ""  # another row's elements
+
+
+WIDTHS = [4, 5, 7, 63, 64, 65, 128, 255, 256, 257, 259, 260, 767, 768, 769, 1020, 1023, 1531, 4095, 4096, 4097, 8191, 8193, 16380, 49151, 49152, 49153]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", WIDTHS)
+@pytest.mark.parametrize("rows", [1, 3, 9])
+def test_softmax_and_norm_of_any_width(hip, width, rows):
+    x, w = 3 * _x(width, rows, width), 1 + 0.1 * _x(5, width)
+    got = ug_amd.llama.softmax(LB.copy(x, x.shape, hip)).data_vec().reshape(x.shape)
+    # an exponential is 2 ulp of its argument's rounding off (|x - max| up to some 30), a sum of n terms in a tree at most log2(n) roundings
+    np.testing.assert_allclose(got, _softmax(x), rtol=(40 + np.log2(width)) * 2 * EPS32, atol=1e-30)
+    got = ug_amd.llama.rms_norm(LB.copy(x, x.shape, hip), LB.copy(w, w.shape, hip), 1e-5).data_vec().reshape(x.shape)
+    want = x / np.sqrt((x.astype(np.float64) ** 2).mean(-1, keepdims=True) + 1e-5) * w
+    np.testing.assert_allclose(got, want, rtol=(10 + width / 1024 + np.log2(width)) * EPS32, atol=1e-30)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(3, 5), (9, 130), (4, 3, 257), (33, 2052)])
+def test_what_others_see_of_the_buffer_between(hip, shape):
+    """Held by a handle it is written, and the same as ever; held by nobody it is never realised; both give the result's same bits."""
+    x, w = _x(2, *shape), _x(3, shape[-1])
+    e, out = _parts(x, w, dev=hip)
+    Schedule.create_one(out).compile().run()
+    assert e.realized()
+    np.testing.assert_allclose(e.data_vec().reshape(shape), np.exp(x.astype(np.float64) - x.max(-1, keepdims=True)), rtol=40 * EPS32)
+    kept = out.data_vec()
+    e, out = _parts(x, w, dev=hip)
+    del e
+    Schedule.create_one(out).compile().run()
+    assert np.array_equal(kept, out.data_vec())
+    np.testing.assert_allclose(kept.reshape(shape), _softmax(x) * w, rtol=60 * EPS32, atol=1e-30)
+    # both at once: the buffer is an output itself
+    e, out = _parts(x, w, dev=hip)
+    Schedule.create([e, out]).compile().run()
+    assert np.array_equal(kept, out.data_vec()) and e.realized()
+
+
+@pytest.mark.gpu
+def test_neighbours_that_stay_two_launches(hip):
+    x = _x(4, 64, 64)
+    e, _ = _parts(x, dev=hip)
+    t = e.transpose(0, 1)
+    out = t.binary("div", t.reduce("sum", 1).broadcast((64, 64)))
+    del e, t
+    want = np.exp(x.astype(np.float64) - x.max(-1, keepdims=True)).T
+    np.testing.assert_allclose(out.data_vec().reshape(64, 64), want / want.sum(-1, keepdims=True), rtol=60 * EPS32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("row", [[np.inf, 1, 2, 3, 4], [-np.inf, 1, 2, 3, 4], [np.nan, 1, 2, 3, 4], [-3.4028235e38] * 5, [3.4028235e38, 1, 2, 3, -3.4028235e38]])
+def test_extreme_rows(hip, cpu, row):
+    """Infinities, NaN and the lowest value give what the oracle's two kernels give."""
+    x = np.array([row * 70, [0.5] * (5 * 70)], np.float32)
+    got, want = (ug_amd.llama.softmax(LB.copy(x, x.shape, d)).data_vec().reshape(x.shape) for d in (hip, cpu))
+    np.testing.assert_allclose(got, want, rtol=1e-5, atol=1e-30)

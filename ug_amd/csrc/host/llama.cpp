@@ -1200,7 +1200,7 @@ std::vector<int32_t> generate_greedy_queued(const Decoder& model, const std::vec
     if (run_now) {
       st.compiled = std::make_unique<CompiledSchedule>(schedule.compile_and_run(ccache));
     } else {
-      st.compiled = std::make_unique<CompiledSchedule>(schedule.compile_with_cache(ccache));
+      st.compiled = std::make_unique<CompiledSchedule>(schedule.compile_with_cache(ccache, false));
       st.compiled->allocate_all();
     }
     st.n_items += schedule.items().size();
@@ -1321,7 +1321,7 @@ std::vector<int32_t> generate_greedy(const Decoder& model, const std::vector<int
     auto t1 = clock::now();
     Schedule schedule = Schedule::create_one(st.logits);
     auto t2 = clock::now();
-    st.compiled = std::make_unique<CompiledSchedule>(schedule.compile_with_cache(ccache));
+    st.compiled = std::make_unique<CompiledSchedule>(schedule.compile_with_cache(ccache, false));
     // Buffers are taken from the pool here, on the preparing thread, so that the launches of this
     // step (possibly issued from another thread) do not allocate.
     st.compiled->allocate_all();

@@ -39,6 +39,7 @@ class LazyBuffer {
   size_t elem_count() const { return shape().num_elements(); }
   const DevicePtr& device() const;
   const std::shared_ptr<DataCell>& data() const;
+  long use_count() const { return p_.use_count(); }
 
   bool in_place_op() const;                // lazy_buffer.rs:130-144
   bool realized() const;                   // :146-154
@@ -141,6 +142,7 @@ struct ScheduleItem {
 // cache.rs:74-101
 struct CompilationCache {
   std::unordered_map<std::string, std::shared_ptr<Func>> op_cache, ssa_cache;
+  std::unordered_map<std::string, std::shared_ptr<Func>> pair_cache;  // null: these two kernels do not run as one
 };
 
 // schedule.rs:210-306
@@ -152,6 +154,9 @@ struct CompiledFunc {
   size_t b = 0, m = 0, n = 0, k = 0;
   bool transpose = false;
   CustomF f;
+  // This kernel and the next as one launch (Device::compile_rows_pair): what run() dispatches in place of both.
+  std::shared_ptr<Func> pair;
+  Args pair_args;
 };
 
 struct CompiledSchedule {
@@ -174,7 +179,8 @@ class Schedule {
     CompilationCache c;
     return compile_with_cache(c);
   }
-  CompiledSchedule compile_with_cache(CompilationCache& cache) const;
+  // pairs: neighbouring row kernels are joined where the device can.
+  CompiledSchedule compile_with_cache(CompilationCache& cache, bool pairs = true) const;
   // The same, and every item is dispatched as soon as it is compiled: on a device that queues work the first kernels
   // execute while the later items are still being looked up.  The result is as after compile_with_cache + run().
   CompiledSchedule compile_and_run(CompilationCache& cache) const;
@@ -182,6 +188,8 @@ class Schedule {
 
  private:
   CompiledFunc compile_item(const ScheduleItem& item, CompilationCache& cache) const;
+  std::shared_ptr<Func> compile_pair(size_t first, CompilationCache& cache, Args* args) const;
+  bool only_between(const LazyBuffer& b, size_t first) const;
   std::vector<ScheduleItem> items_;
   std::map<size_t, LazyBuffer> per_arg_id_;
   DevicePtr device_;

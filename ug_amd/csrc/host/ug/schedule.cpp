@@ -248,11 +248,99 @@ const LazyBuffer& Schedule::get_arg_id(ArgId id) const {
 }
 
 // schedule.rs:115-207
-CompiledSchedule Schedule::compile_with_cache(CompilationCache& cache) const {
+CompiledSchedule Schedule::compile_with_cache(CompilationCache& cache, bool pairs) const {
   CompiledSchedule out;
   out.device = device_;
-  for (const ScheduleItem& item : items_) out.funcs.push_back(compile_item(item, cache));
+  for (size_t i = 0; i < items_.size(); ++i) {
+    Args args;
+    std::shared_ptr<Func> pair = pairs && device_->joins_rows() && i + 1 < items_.size() ? compile_pair(i, cache, &args) : nullptr;
+    out.funcs.push_back(compile_item(items_[i], cache));
+    if (!pair) continue;
+    out.funcs.back().pair = std::move(pair);
+    out.funcs.back().pair_args = std::move(args);
+    out.funcs.push_back(compile_item(items_[++i], cache));
+  }
   return out;
+}
+
+// Whether nothing but items `first` and `first + 1` can ever ask for what is in `b`: no other item, no other buffer on the same storage, and
+// every holder of the handle is this schedule or the graph it was made from.  (Handles are only ever copied from handles, so nobody can come
+// by one later.)
+bool Schedule::only_between(const LazyBuffer& b, size_t first) const {
+  if (b.data().use_count() != 1) return false;
+  const LazyBufferInner* wanted = &b.inner();
+  long known = 0;
+  std::vector<const LazyBuffer*> todo;
+  std::set<const LazyBufferInner*> seen;
+  auto note = [&](const LazyBuffer& x) {
+    if (!x.valid()) return;
+    if (&x.inner() == wanted) ++known;
+    if (seen.insert(&x.inner()).second) todo.push_back(&x);
+  };
+  for (size_t i = 0; i < items_.size(); ++i) {
+    const ScheduleItem& it = items_[i];
+    const long before = known;
+    for (const auto& a : it.kernel.args) note(a.second);
+    for (const auto& a : it.args) note(a.second);
+    for (const LazyBuffer* x : {&it.kernel.dst.second, &it.dst, &it.lhs, &it.rhs}) note(*x);
+    if (known != before && i != first && i != first + 1) return false;
+  }
+  for (const auto& a : per_arg_id_) note(a.second);
+  while (!todo.empty()) {
+    const Op& op = todo.back()->inner().op;
+    todo.pop_back();
+    note(op.arg);
+    note(op.arg2);
+    for (const LazyBuffer& a : op.args) note(a);
+  }
+  return b.use_count() == known;
+}
+
+std::shared_ptr<Func> Schedule::compile_pair(size_t first, CompilationCache& cache, Args* args) const {
+  const ScheduleItem &x = items_[first], &y = items_[first + 1];
+  if (x.kind != ScheduleItem::Kernel || y.kind != ScheduleItem::Kernel || x.kernel.has_dst_layout || y.kernel.has_dst_layout) return nullptr;
+  const LazyBuffer& between = x.kernel.dst.second;
+  if (between.elem_count() != y.kernel.dst.second.elem_count() || between.in_place_op() || y.kernel.dst.second.in_place_op()) return nullptr;
+  // arguments by storage; a kernel that names one storage twice is refused when it runs, as ever
+  std::vector<const DataCell*> cells;
+  int link = -1;
+  for (const auto& a : x.kernel.args) {
+    const DataCell* c = a.second.data().get();
+    if (std::find(cells.begin(), cells.end(), c) != cells.end()) return nullptr;
+    if (c == between.data().get()) link = (int)cells.size();
+    cells.push_back(c);
+  }
+  const size_t n_first = cells.size();
+  std::vector<int> shared;
+  bool linked = false;
+  for (const auto& a : y.kernel.args) {
+    const DataCell* c = a.second.data().get();
+    const size_t at = std::find(cells.begin(), cells.end(), c) - cells.begin();
+    if (at < cells.size() && at >= n_first) return nullptr;
+    shared.push_back(at < n_first ? (int)at : -1);
+    linked |= (int)at == link;
+    if (at == cells.size()) cells.push_back(c);
+  }
+  if (link < 0 || !linked) return nullptr;
+  const bool keep = !only_between(between, first);
+  op::Kernel a = x.kernel.kernel(), b = y.kernel.kernel();
+  const std::string key_a = normalized_kernel_key(a), key_b = normalized_kernel_key(b);
+  std::string key = key_a + "\n" + key_b + "\n" + (keep ? "k" : "") + std::to_string(link);
+  for (int s : shared) key += "," + std::to_string(s);
+  auto it = cache.pair_cache.find(key);
+  if (it == cache.pair_cache.end()) {
+    const std::array<std::string, 2> names{a.ops[0].name(), b.ops[0].name()};
+    auto funcs = device_->compile_rows_pair(a.optimize().lower(op::Opts()), b.optimize().lower(op::Opts()), names, shared, link, keep);
+    cache.op_cache.emplace(key_a, funcs[1]);
+    cache.op_cache.emplace(key_b, funcs[2]);
+    it = cache.pair_cache.emplace(key, funcs[0]).first;
+  }
+  if (!it->second) return nullptr;
+  for (size_t k = 0; k < n_first; ++k)
+    if (keep || (int)k != link) args->push_back({x.kernel.args[k].first, get_arg_id(x.kernel.args[k].first)});
+  for (size_t k = 0; k < shared.size(); ++k)
+    if (shared[k] < 0) args->push_back({y.kernel.args[k].first, get_arg_id(y.kernel.args[k].first)});
+  return it->second;
 }
 
 CompiledSchedule Schedule::compile_and_run(CompilationCache& cache) const {
@@ -331,8 +419,12 @@ CompiledFunc Schedule::compile_item(const ScheduleItem& item, CompilationCache& 
 }
 
 void CompiledSchedule::allocate_all() const {
-  for (const CompiledFunc& f : funcs) {
-    if (f.kind == CompiledFunc::MatMul) {
+  for (size_t i = 0; i < funcs.size(); ++i) {
+    const CompiledFunc& f = funcs[i];
+    if (f.pair) {
+      for (const auto& a : f.pair_args) a.second.maybe_allocate_uninit();
+      ++i;
+    } else if (f.kind == CompiledFunc::MatMul) {
       f.dst.maybe_allocate_uninit();
       f.lhs.maybe_allocate_uninit();
       f.rhs.maybe_allocate_uninit();
@@ -343,8 +435,30 @@ void CompiledSchedule::allocate_all() const {
 }
 
 // schedule.rs:234-305
+// The slices of a launch's arguments, allocated where that is left to do.
+static void borrow(const Args& args, std::vector<Slice*>& bs) {
+  bs.clear();
+  for (const auto& a : args) {
+    a.second.maybe_allocate_uninit();
+    // RefCell::try_borrow_mut: a cell may appear once.
+    Slice* s = a.second.data()->slice.get();
+    for (Slice* seen : bs)
+      if (seen == s) bail("already borrowed: BorrowMutError");
+    bs.push_back(s);
+  }
+}
+
 void CompiledSchedule::run() const {
-  for (const CompiledFunc& f : funcs) run_one(f);
+  thread_local std::vector<Slice*> bs;
+  for (size_t i = 0; i < funcs.size(); ++i) {
+    if (!funcs[i].pair) {
+      run_one(funcs[i]);
+      continue;
+    }
+    borrow(funcs[i].pair_args, bs);
+    device->run(*funcs[i].pair, bs);
+    ++i;
+  }
 }
 
 void CompiledSchedule::run_one(const CompiledFunc& f) const {
@@ -353,15 +467,7 @@ void CompiledSchedule::run_one(const CompiledFunc& f) const {
     switch (f.kind) {
       case CompiledFunc::Kernel:
       case CompiledFunc::Custom: {
-        bs.clear();
-        for (const auto& a : f.args) {
-          a.second.maybe_allocate_uninit();
-          // RefCell::try_borrow_mut: a cell may appear once.
-          Slice* s = a.second.data()->slice.get();
-          for (Slice* seen : bs)
-            if (seen == s) bail("already borrowed: BorrowMutError");
-          bs.push_back(s);
-        }
+        borrow(f.args, bs);
         if (f.kind == CompiledFunc::Kernel) device->run(*f.func, bs);
         else (*f.f)(bs);
         break;

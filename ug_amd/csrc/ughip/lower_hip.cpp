@@ -233,6 +233,7 @@ class Lowering {
   int n_;
   std::string entry_;
   bool as_written_ = false;
+  std::map<int, std::string> held_;  // loads whose element is in a register already, and what it is called
   mutable bool nt_loads_ = false;  // loads of the region being emitted bypass cache allocation
   bool nt_stores_ = false;         // stores to kernel arguments go past the cache (set while an elementwise kernel is emitted)
   Lowered out_;
@@ -702,7 +703,8 @@ class Lowering {
   }
 
   // ---- text emission -----------------------------------------------------------------------
-  static std::string var(int i) { return "v" + std::to_string(i); }
+  std::string vp_ = "v";  // first letter of this kernel's values: two kernels may share a source
+  std::string var(int i) const { return vp_ + std::to_string(i); }
 
   static std::string f32_lit(float f) {
     if (std::isinf(f)) return f > 0 ? "__builtin_inff()" : "(-__builtin_inff())";
@@ -822,7 +824,8 @@ class Lowering {
       case UGHIP_I_END_IF: o << "}"; break;
       case UGHIP_I_IF: o << "if (" << opnd(in.a) << ") {"; break;
       case UGHIP_I_LOAD:
-        if (nt_loads_) o << ty << " " << var(i) << " = __builtin_nontemporal_load(&" << var((int)in.v) << "[" << opnd(in.a) << "]);";
+        if (auto at = held_.find(i); at != held_.end()) o << ty << " " << var(i) << " = " << at->second << ";";
+        else if (nt_loads_) o << ty << " " << var(i) << " = __builtin_nontemporal_load(&" << var((int)in.v) << "[" << opnd(in.a) << "]);";
         else o << ty << " " << var(i) << " = " << var((int)in.v) << "[" << opnd(in.a) << "];";
         break;
       case UGHIP_I_ASSIGN: o << var((int)in.v) << " = " << opnd(in.a) << ";"; break;
@@ -1112,14 +1115,15 @@ class Lowering {
   void emit_decode(std::ostringstream& o, const std::vector<int>& ls, const std::string& group, int vec, int indent) const {
     std::string pad(2 * indent, ' ');
     if (ls.empty()) return;
-    o << pad << "int ug_r = " << group << ";\n";
+    const std::string left = "ug_r" + vp_;
+    o << pad << "int " << left << " = " << group << ";\n";
     for (int k = (int)ls.size() - 1; k >= 0; --k) {
       const LoopInfo& L = loops_[ls[k]];
       bool inner = k == (int)ls.size() - 1;
       i64 radix = inner ? L.trip / vec : L.trip;
       // one spelling of the radix per loop, so the % and / below share it (one parameter slot)
       std::string rs = !k ? "" : (parametric_ ? kparam(radix) : std::to_string(radix));
-      std::string digit = k == 0 ? "ug_r" : "(ug_r % " + rs + ")";
+      std::string digit = k == 0 ? left : "(" + left + " % " + rs + ")";
       if (inner && vec > 1) digit = "(" + digit + " * " + std::to_string(vec) + " + ug_u)";
       o << pad << "const int " << var(L.begin) << " = ";
       if (parametric_) {
@@ -1130,7 +1134,7 @@ class Lowering {
         if (L.step != 1) o << " * " << L.step;
       }
       o << ";\n";
-      if (k) o << pad << "ug_r /= " << rs << ";\n";
+      if (k) o << pad << left << " /= " << rs << ";\n";
     }
   }
 
@@ -1145,7 +1149,7 @@ class Lowering {
   // first elements are the group before's as well (a reduction folds them once, a store writes them twice, with the same value -- what a
   // kernel stores it never loads).  Same lengths as pick_vec's 4.  The 128-bit accesses then start at any element, which the hardware takes.
   // By single elements -> so: softmax [16411, 1531], two kernels, 133 -> 82 us, [8000, 4097] 167 -> 105; RMSNorm [16411, 1531] 84 -> 48, [1900, 2049]
-  // 10.7 -> 8.2.  What is left is the rows' way through memory (16 bytes per element of the softmax at 5 TB/s).
+  // 10.7 -> 8.2.
   static bool overlapped(i64 extent, i64 threads) { return extent % 4 != 0 && threads > 64 && extent > (threads - 64) * 4; }
 
   void emit_items(std::ostringstream& o, bool want_cols, uint64_t col_mask, int indent, bool guard_row_stores, int tpr, bool one_thread) const {
@@ -1310,6 +1314,13 @@ class Lowering {
     int rows_per_block = tpr == 64 ? 4 : 1;
     if (nr < rows_per_block) rows_per_block = 1;
     int block = tpr * rows_per_block;
+    if (!grid_reduce) {
+      find_rows_form(rows, cols, nr, nc, tpr, rows_per_block);
+      if (rows_ok_) {
+        emit_rows();
+        return;
+      }
+    }
     std::ostringstream o;
     o << kPrelude << "\nextern \"C\" __global__ void __launch_bounds__(" << block << ") " << entry_ << "(" << signature(grid_reduce) << ") {\n";
     o << "  const int ug_t = (int)threadIdx.x % " << tpr << ";\n";
@@ -1412,6 +1423,244 @@ class Lowering {
     out_.grid = grid_reduce ? (unsigned)(nr * nb) : (unsigned)((nr + rows_per_block - 1) / rows_per_block);
   }
 
+  // ---- rows held in registers -----------------------------------------------------------------
+  // A row kernel whose reductions and column loop all run over the same W elements: thread t owns the groups of `vec` consecutive elements
+  // t, t + tpr, .. in every one of them, so what it loads for one loop serves the others, and the elements another kernel stored for the same
+  // row (`link`) need not go through memory.  Everything is asked for ahead of the first reduction.  As in `overlapped`, the last group is
+  // moved back to end with the row; a group past the end is the last one again, folded and stored by nobody.
+  // What bounds it: HBM for many rows, the launch for few.  Re-reading each loop's operands (and the softmax's exponentials through memory,
+  // two launches) -> so: softmax [32, 1024] 6.3 -> 3.4 us, [16411, 1531] 77.3 -> 42.3 (4.7 TB/s of its 200 MB), [1472, 4113] 22.1 -> 13.8, [9994, 256] 8.4 -> 5.3;
+  // RMSNorm [1900, 2048] 7.3 -> 6.5.  At most 48 elements a thread are held (rows of 49152); longer rows go through memory as before.
+ public:
+  struct Held {  // a load's place: argument, offset = c + sum row[k] * (digit of row loop k) + unit * (index along the row)
+    int arg = 0, unit = 0;
+    i64 c = 0;
+    std::vector<i64> row;
+    bool operator==(const Held& o) const { return arg == o.arg && unit == o.unit && c == o.c && row == o.row; }
+  };
+  struct RowsForm {
+    std::vector<i64> trips;  // of the row loops, outermost first (those with one trip left out)
+    i64 nr = 0, width = 0;
+    int tpr = 0, vec = 0, per = 0, rows_per_block = 0;
+  };
+
+  // nullptr: not of this form.
+  const RowsForm* rows_form() const { return rows_ok_ ? &form_ : nullptr; }
+  const std::vector<char>& written() const { return out_.arg_written; }
+  const Lowered& lowered() const { return out_; }
+  void rename(const std::string& prefix) { vp_ = prefix; }
+  // The one store of argument `arg` as a place; false: there are several, or it is not one element per column.
+  bool stored_at(int arg, Held* at) const {
+    int found = -1;
+    for (int i = 0; i < n_; ++i)
+      if (I_[i].op == UGHIP_I_STORE && arg_of_[I_[i].v] == arg) {
+        if (found >= 0) return false;
+        found = i;
+      }
+    return found >= 0 && place_of(found, cols_[0], at);
+  }
+  // Every load of argument `arg` is of place `at` (in that argument's own numbering).
+  bool loaded_only_at(int arg, const Held& at) const {
+    bool any = false;
+    for (int i = 0; i < n_; ++i) {
+      if (I_[i].op != UGHIP_I_LOAD || arg_of_[I_[i].v] != arg) continue;
+      Held h;
+      if (encl_[i] < 0 || !place_of(i, encl_[i], &h)) return false;
+      h.arg = at.arg;
+      if (!(h == at)) return false;
+      any = true;
+    }
+    return any;
+  }
+
+  // Registers shared by the kernels of a source: the places in them, by the argument numbers of the source.
+  struct Registers {
+    std::vector<Held> at;
+    std::vector<int> dtype;
+    int floats_left = 48;  // per thread: at 1024 threads the compiler has 128
+  };
+  // Row decoding and the loads of everything that is held; link: this kernel's argument that is not loaded but found in ug_link.
+  void emit_rows_head(std::ostringstream& o, Registers& regs, const std::vector<int>& arg_number, int link) {
+    emit_decode(o, rows_, "ug_row", 1, 1);
+    for (int i = 0; i < n_; ++i) {
+      if (I_[i].op != UGHIP_I_LOAD || arg_of_[I_[i].v] < 0 || encl_[i] < 0) continue;
+      if (arg_of_[I_[i].v] == link) {
+        held_[i] = "ug_link[ug_it][ug_u]";
+        continue;
+      }
+      Held h;
+      if (!place_of(i, encl_[i], &h)) continue;
+      h.arg = arg_number[h.arg];
+      size_t k = std::find(regs.at.begin(), regs.at.end(), h) - regs.at.begin();
+      const std::string name = "ug_h" + std::to_string(k);
+      if (k == regs.at.size()) {
+        if (regs.floats_left < form_.per * form_.vec) continue;
+        regs.floats_left -= form_.per * form_.vec;
+        regs.at.push_back(h);
+        regs.dtype.push_back(I_[i].dtype);
+        o << "  " << dtype_c_name(I_[i].dtype) << " " << name << "[" << form_.per << "][" << form_.vec << "];\n";
+        const Aff a = aff_of(I_[i].a);
+        o << "#pragma unroll\n  for (int ug_it = 0; ug_it < " << form_.per << "; ++ug_it) {\n";
+        emit_group(o, 2);
+        o << "#pragma unroll\n    for (int ug_u = 0; ug_u < " << form_.vec << "; ++ug_u) " << name << "[ug_it][ug_u] = " << var((int)I_[i].v) << "[" << a.c;
+        for (const auto& kv : a.t) {
+          if (kv.first == encl_[i]) o << " + " << loops_[kv.first].lo * kv.second << " + (ug_i + ug_u)";
+          else o << " + " << var(loops_[kv.first].begin) << " * " << kv.second;
+        }
+        o << "];\n  }\n";
+      } else if (regs.dtype[k] != I_[i].dtype) {
+        continue;
+      }
+      held_[i] = name + "[ug_it][ug_u]";
+    }
+  }
+  // The rest.  link: the argument whose store goes to ug_link (-1: none), kept: and to memory as well.
+  void emit_rows_body(std::ostringstream& o, int link, bool kept) {
+    const bool masked = form_.width % ((i64)form_.vec * form_.tpr) != 0;
+    uint64_t col_mask = 1ull << cols_[0];
+    for (const Item& it : items_) {
+      if (it.deps & col_mask) continue;
+      if (it.kind == 1) {
+        const Region& r = regions_[it.region];
+        const LoopInfo& L = loops_[r.loop];
+        o << "  " << dtype_c_name(vt_[r.acc].dtype) << " ug_p" << r.acc << " = " << identity_lit(r.op, vt_[r.acc].dtype) << ";\n";
+        o << "#pragma unroll\n  for (int ug_it = 0; ug_it < " << form_.per << "; ++ug_it) {\n";
+        emit_group(o, 2);
+        o << "#pragma unroll\n    for (int ug_u = 0; ug_u < " << form_.vec << "; ++ug_u) {\n";
+        o << "      const int " << var(L.begin) << " = " << L.lo << " + (ug_i + ug_u) * " << L.step << ";\n";
+        emit_reduce_body(o, r, 3, masked ? "ug_i + ug_u >= ug_g" : nullptr);
+        o << "    }\n  }\n";
+        emit_region_finish(o, r, 1, form_.tpr);
+      } else {
+        emit_range(o, it.idx, it.end, 1);
+      }
+    }
+    o << "#pragma unroll\n  for (int ug_it = 0; ug_it < " << form_.per << "; ++ug_it) {\n";
+    emit_group(o, 2);
+    std::vector<int> stores;
+    for (const Item& it : items_)
+      if ((it.deps & col_mask) && I_[it.idx].op == UGHIP_I_STORE && (kept || arg_of_[I_[it.idx].v] != link)) stores.push_back(it.idx);
+    for (int st : stores) {
+      const std::string n = std::to_string(st);
+      o << "    int ug_o" << n << "[" << form_.vec << "];\n    " << dtype_c_name(I_[st].dtype) << " ug_s" << n << "[" << form_.vec << "];\n";
+    }
+    o << "#pragma unroll\n    for (int ug_u = 0; ug_u < " << form_.vec << "; ++ug_u) {\n";
+    emit_decode(o, cols_, "(ug_i + ug_u)", 1, 3);
+    for (const Item& it : items_) {
+      if (!(it.deps & col_mask)) continue;
+      if (it.kind == 0 && I_[it.idx].op == UGHIP_I_STORE) {
+        const ughip_instr& in = I_[it.idx];
+        if (arg_of_[in.v] == link) o << "      ug_link[ug_it][ug_u] = " << opnd(in.b) << ";\n";
+        if (!kept && arg_of_[in.v] == link) continue;
+        const std::string n = std::to_string(it.idx);
+        o << "      ug_o" << n << "[ug_u] = " << opnd(in.a) << ";\n      ug_s" << n << "[ug_u] = " << opnd(in.b) << ";\n";
+      } else {
+        emit_range(o, it.idx, it.end, 3);
+      }
+    }
+    o << "    }\n";
+    for (int st : stores) {
+      const std::string n = std::to_string(st);
+      o << "    " << (masked ? "if (ug_g < " + std::to_string(form_.width) + ") " : std::string()) << "{\n#pragma unroll\n      for (int ug_u = 0; ug_u < " << form_.vec << "; ++ug_u) " << var((int)I_[st].v)
+        << "[ug_o" << n << "[ug_u]] = ug_s" << n << "[ug_u];\n    }\n";
+    }
+    o << "  }\n";
+  }
+  static void emit_rows_prologue(std::ostringstream& o, const std::string& entry, const std::string& sig, const RowsForm& f) {
+    o << kPrelude << "\nextern \"C\" __global__ void __launch_bounds__(" << f.tpr * f.rows_per_block << ") " << entry << "(" << sig << ") {\n";
+    o << "  const int ug_t = (int)threadIdx.x % " << f.tpr << ";\n";
+    o << "  const int ug_row = (int)blockIdx.x * " << f.rows_per_block << " + (int)threadIdx.x / " << f.tpr << ";\n";
+    if (f.rows_per_block > 1) o << "  if (ug_row >= " << f.nr << ") return;\n";
+  }
+  std::string declare(size_t a) const {
+    return (out_.arg_written[a] ? "" : "const ") + std::string(dtype_c_name(s_.args[a].dtype)) + "* __restrict__ " + var((int)s_.args[a].var);
+  }
+  std::string arg_name(size_t a) const { return var((int)s_.args[a].var); }
+  std::string arg_type(size_t a) const { return (out_.arg_written[a] ? "" : "const ") + std::string(dtype_c_name(s_.args[a].dtype)) + "*"; }
+
+ private:
+  bool rows_ok_ = false;
+  RowsForm form_;
+  std::vector<int> rows_, cols_;
+
+  // `int ug_g` (the group's place in the row as dealt out) and `int ug_i` (where its elements are)
+  void emit_group(std::ostringstream& o, int indent) const {
+    const std::string pad(2 * indent, ' ');
+    o << pad << "const int ug_g = (ug_t + ug_it * " << form_.tpr << ") * " << form_.vec << ";\n";
+    if (form_.width % ((i64)form_.vec * form_.tpr) != 0) o << pad << "const int ug_i = ug_g < " << form_.width - form_.vec << " ? ug_g : " << form_.width - form_.vec << ";\n";
+    else o << pad << "const int ug_i = ug_g;\n";
+  }
+
+  // The place of a load or store inside loop `l` that runs along the row; false: it does not step by one element there, or depends on other loops.
+  bool place_of(int i, int l, Held* h) const {
+    const Aff a = aff_of(I_[i].a);
+    if (!a.ok || guarded_[i]) return false;
+    h->arg = arg_of_[I_[i].v];
+    h->c = a.c;
+    h->row.clear();
+    h->unit = 0;
+    for (const auto& kv : a.t) {
+      if (kv.first == l) {
+        if (kv.second * loops_[l].step != 1 || kv.second != 1) return false;
+        h->unit = 1, h->c += kv.second * loops_[l].lo;
+      } else if (std::find(rows_.begin(), rows_.end(), kv.first) == rows_.end()) {
+        return false;
+      }
+    }
+    if (!h->unit) return false;
+    for (int r : rows_) {
+      if (loops_[r].trip <= 1) {
+        auto it = a.t.find(r);
+        if (it != a.t.end()) h->c += it->second * loops_[r].lo;
+        continue;
+      }
+      auto it = a.t.find(r);
+      const i64 k = it == a.t.end() ? 0 : it->second;
+      h->c += k * loops_[r].lo;
+      h->row.push_back(k * loops_[r].step);
+    }
+    return true;
+  }
+
+  void find_rows_form(const std::vector<int>& rows, const std::vector<int>& cols, i64 nr, i64 nc, int tpr, int rows_per_block) {
+    if (cols.size() != 1 || regions_.empty() || nc < 4) return;
+    for (const Item& it : items_) {
+      if (it.kind == 2) return;
+      if (it.kind == 1 && ((it.deps >> cols[0]) & 1)) return;
+    }
+    for (const Region& r : regions_) {
+      if (r.trip != nc) return;
+      for (int i = r.range + 1; i < r.end; ++i)
+        if (I_[i].op == UGHIP_I_RANGE || I_[i].op == UGHIP_I_STORE) return;
+    }
+    for (int i = 0; i < n_; ++i)
+      if (I_[i].op == UGHIP_I_STORE && encl_[i] != cols[0]) return;
+    rows_ = rows, cols_ = cols;
+    form_.nr = nr, form_.width = nc, form_.tpr = tpr, form_.rows_per_block = rows_per_block;
+    form_.vec = tpr > 64 || nc == 256 ? 4 : 1;
+    form_.per = (int)(((nc + form_.vec - 1) / form_.vec + tpr - 1) / tpr);
+    form_.trips.clear();
+    for (int r : rows)
+      if (loops_[r].trip > 1) form_.trips.push_back(loops_[r].trip);
+    rows_ok_ = form_.per * form_.vec <= 48;
+  }
+
+  void emit_rows() {
+    std::ostringstream o;
+    emit_rows_prologue(o, entry_, signature(false), form_);
+    std::vector<int> number;
+    for (size_t a = 0; a < s_.n_args; ++a) number.push_back((int)a);
+    Registers regs;
+    emit_rows_head(o, regs, number, -1);
+    emit_rows_body(o, -1, true);
+    o << "}\n";
+    held_.clear();
+    out_.source = o.str();
+    out_.strategy = UGHIP_STRAT_ROW_BLOCK;
+    out_.block = (unsigned)(form_.tpr * form_.rows_per_block);
+    out_.grid = (unsigned)((form_.nr + form_.rows_per_block - 1) / form_.rows_per_block);
+  }
+
   // First stage of a grid-wide reduction: workgroup `ug_blk` of `nb` takes every nb-th slab.
   void emit_region_partial(std::ostringstream& o, const Region& r, int indent, int tpr, unsigned nb) const {
     std::string pad(2 * indent, ' ');
@@ -1448,6 +1697,76 @@ class Lowering {
 };
 
 }  // namespace
+
+bool lower_rows_pair(const ughip_ssa& first, const ughip_ssa& second, const std::string entries[3], const int* shared, int link, bool keep, Lowered* out, Lowered parts[2]) {
+  for (const ughip_ssa* ssa : {&first, &second})
+    if (!ssa->instrs || (!ssa->args && ssa->n_args)) throw std::runtime_error("ssa lowering: null instrs/args");
+  Lowering a(first, entries[1], false), b(second, entries[2], false);
+  parts[0] = a.run(), parts[1] = b.run();
+  const Lowered &la = parts[0], &lb = parts[1];
+  const std::string& entry = entries[0];
+  b.rename("w");
+  const Lowering::RowsForm *fa = a.rows_form(), *fb = b.rows_form();
+  if (!fa || !fb || fa->nr != fb->nr || fa->width != fb->width || fa->trips != fb->trips || link < 0 || link >= (int)first.n_args || !la.arg_written[link]) return false;
+  int link_b = -1;
+  for (size_t k = 0; k < second.n_args; ++k) {
+    if (shared[k] < 0) continue;
+    if (shared[k] >= (int)first.n_args || first.args[shared[k]].dtype != second.args[k].dtype || lb.arg_written[k]) return false;
+    if (shared[k] == link) {
+      if (link_b >= 0) return false;
+      link_b = (int)k;
+    } else if (la.arg_written[shared[k]]) {
+      return false;
+    }
+  }
+  for (size_t k = 0; k < first.n_args; ++k)
+    if (la.arg_written[k] && (int)k != link) return false;
+  Lowering::Held at;
+  if (link_b < 0 || !a.stored_at(link, &at) || !b.loaded_only_at(link_b, at)) return false;
+
+  Lowered r;
+  r.entry = entry;
+  std::string sig;
+  std::vector<int> number_a(first.n_args, -1), number_b(second.n_args, -1);
+  auto take = [&](const Lowering& l, const Lowered& low, const ughip_ssa& ssa, size_t k) {
+    sig += (sig.empty() ? "" : ", ") + l.declare(k);
+    r.arg_dtype.push_back(ssa.args[k].dtype);
+    r.min_len.push_back(low.min_len[k]);
+    r.arg_written.push_back(low.arg_written[k]);
+    return (int)r.arg_dtype.size() - 1;
+  };
+  for (size_t k = 0; k < first.n_args; ++k)
+    if (keep || (int)k != link) number_a[k] = take(a, la, first, k);
+  std::string aliases;
+  for (size_t k = 0; k < second.n_args; ++k) {
+    if (shared[k] < 0) {
+      number_b[k] = take(b, lb, second, k);
+    } else if ((int)k != link_b) {
+      number_b[k] = number_a[shared[k]];
+      r.min_len[number_b[k]] = std::max(r.min_len[number_b[k]], lb.min_len[k]);
+      if (la.min_len[shared[k]] < 0 || lb.min_len[k] < 0) r.min_len[number_b[k]] = -1;
+      aliases += "  " + b.arg_type(k) + " " + b.arg_name(k) + " = " + a.arg_name(shared[k]) + ";\n";
+    }
+  }
+  std::ostringstream o;
+  Lowering::emit_rows_prologue(o, entry, sig, *fa);
+  o << aliases << "  " << dtype_c_name(first.args[link].dtype) << " ug_link[" << fa->per << "][" << fa->vec << "];\n";
+  Lowering::Registers regs;
+  regs.floats_left -= fa->per * fa->vec;
+  a.emit_rows_head(o, regs, number_a, -1);
+  b.emit_rows_head(o, regs, number_b, link_b);
+  o << "  {\n";
+  a.emit_rows_body(o, link, keep);
+  o << "  }\n  {\n";
+  b.emit_rows_body(o, -1, true);
+  o << "  }\n}\n";
+  r.source = o.str();
+  r.strategy = UGHIP_STRAT_ROW_BLOCK;
+  r.block = (unsigned)(fa->tpr * fa->rows_per_block);
+  r.grid = (unsigned)((fa->nr + fa->rows_per_block - 1) / fa->rows_per_block);
+  *out = r;
+  return true;
+}
 
 Lowered lower_ssa(const ughip_ssa& ssa, const std::string& entry, bool as_written) {
   if (!ssa.instrs || (!ssa.args && ssa.n_args)) throw std::runtime_error("ssa lowering: null instrs/args");
