@@ -89,7 +89,7 @@ enum TuneKey {
   TUNE_NO_NT_LOADS,         // (set at all) the grid-wide reduction reads with ordinary loads
   TUNE_GRID_REDUCE_BLOCKS,  // workgroups of the grid-wide reduction's first stage
   TUNE_GRID_REDUCE_THREADS, // threads per workgroup there: 64, 128, 256, 512 or 1024
-  TUNE_NO_NT_STORES,        // (set at all) generated elementwise kernels store through the cache
+  TUNE_NO_NT_STORES,        // (set at all) generated elementwise and row kernels store through the cache
   TUNE_SOFTMAX_STREAM,      // ughip_softmax_rows: 0 never takes the resident wave-per-row kernel, n > 0 forces it onto n workgroups
   TUNE_ATT_X6,              // attention over several query positions, head size 64: 0 keeps the f32 products, 1 takes six bf16 terms for any count
   TUNE_MATMUL_X6,           // f32 products of ughip_matmul: 1 takes those of contiguous operands with k % 64 == 0, n % 8 == 0 as six bf16 terms on the bf16 matrix pipe

@@ -1240,7 +1240,7 @@ class Lowering {
     kparams_.clear();
     // Whole 128-bit groups are stored past the cache: nothing in the launch reads them back (stored buffers are never loaded
     // here), and the next kernel would find them in another XCD's L2 at best.  SwiGLU [512, 5632]: 4.6 -> 3.6 us, [16384, 5632]
-    // 184 -> 179 us.  Not for the row kernels: their stores do not merge under the hint (RMSNorm [8192, 2048]: 20.8 -> 31.6 us).
+    // 184 -> 179 us.
     nt_stores_ = vec == 4 && !ughip::tune_on(ughip::TUNE_NO_NT_STORES);
     std::ostringstream b;
     b << "  const int ug_g = (int)blockIdx.x * " << block << " + (int)threadIdx.x;\n";
@@ -1429,7 +1429,7 @@ class Lowering {
   // row (`link`) need not go through memory.  Everything is asked for ahead of the first reduction.  As in `overlapped`, the last group is
   // moved back to end with the row; a group past the end is the last one again, folded and stored by nobody.
   // What bounds it: HBM for many rows, the launch for few.  Re-reading each loop's operands (and the softmax's exponentials through memory,
-  // two launches) -> so: softmax [32, 1024] 6.3 -> 3.4 us, [16411, 1531] 77.3 -> 42.3 (4.7 TB/s of its 200 MB), [1472, 4113] 22.1 -> 13.8, [9994, 256] 8.4 -> 5.3;
+  // two launches) -> so, with stores through the cache: softmax [32, 1024] 6.3 -> 3.4 us, [16411, 1531] 77.3 -> 42.3 (4.7 TB/s of its 200 MB), [1472, 4113] 22.1 -> 13.8, [9994, 256] 8.4 -> 5.3;
   // RMSNorm [1900, 2048] 7.3 -> 6.5.  At most 48 elements a thread are held (rows of 49152); longer rows go through memory as before.
  public:
   struct Held {  // a load's place: argument, offset = c + sum row[k] * (digit of row loop k) + unit * (index along the row)
@@ -1561,7 +1561,18 @@ class Lowering {
     o << "    }\n";
     for (int st : stores) {
       const std::string n = std::to_string(st);
-      o << "    " << (masked ? "if (ug_g < " + std::to_string(form_.width) + ") " : std::string()) << "{\n#pragma unroll\n      for (int ug_u = 0; ug_u < " << form_.vec << "; ++ug_u) " << var((int)I_[st].v)
+      const std::string guard = masked ? "if (ug_g < " + std::to_string(form_.width) + ") " : "";
+      Held h;
+      if (form_.vec == 4 && dtype_size(I_[st].dtype) == 4 && !ughip::tune_on(ughip::TUNE_NO_NT_STORES) && place_of(st, cols_[0], &h)) {
+        // A whole group past the cache, as one vector at whatever element it starts (element by element the hint keeps the stores from
+        // merging): the next kernel would find it in another XCD's L2 at best.  Softmax [16411, 1531] 43.1 -> 40.7 us, [957, 6560] 11.8 -> 9.8,
+        // [11392, 448] 9.7 -> 8.3; RMSNorm [1900, 2048] 6.5 -> 5.9; rows that fit a few workgroups as before.
+        const std::string ty = dtype_c_name(I_[st].dtype), v = "ug_s" + n;
+        o << "    " << guard << "{\n      typedef " << ty << " ug_4 __attribute__((ext_vector_type(4), aligned(4)));\n      __builtin_nontemporal_store(ug_4{" << v << "[0], " << v << "[1], " << v << "[2], " << v
+          << "[3]}, (ug_4*)&" << var((int)I_[st].v) << "[ug_o" << n << "[0]]);\n    }\n";
+        continue;
+      }
+      o << "    " << guard << "{\n#pragma unroll\n      for (int ug_u = 0; ug_u < " << form_.vec << "; ++ug_u) " << var((int)I_[st].v)
         << "[ug_o" << n << "[ug_u]] = ug_s" << n << "[ug_u];\n    }\n";
     }
     o << "  }\n";
