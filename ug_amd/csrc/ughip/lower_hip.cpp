@@ -154,6 +154,22 @@ template <typename Op, typename T> UG_DEV T ug_block_reduce_dyn(T v) {
 )HIP";
 
 // ---------------------------------------------------------------------------------------
+// Source text as it grows.  (A stream of the standard library costs half a microsecond to construct, and a statement is a text of its own: a
+// lazy graph's kernel 16 -> 6 us.)
+class Text {
+ public:
+  Text& operator<<(const std::string& s) { return t_ += s, *this; }
+  Text& operator<<(const char* s) { return t_ += s, *this; }
+  template <typename N, typename = std::enable_if_t<std::is_integral_v<N>>>
+  Text& operator<<(N n) {
+    return t_ += std::to_string(n), *this;
+  }
+  const std::string& str() const { return t_; }
+
+ private:
+  std::string t_;
+};
+
 struct VType {
   bool valid = false, ptr = false, local = false;
   int dtype = UGHIP_F32;
@@ -767,7 +783,7 @@ class Lowering {
   std::string stmt(int i) const {
     const ughip_instr& in = I_[i];
     std::string ty = vt_[i].valid && !vt_[i].ptr ? dtype_c_name(vt_[i].dtype) : "";
-    std::ostringstream o;
+    Text o;
     switch (in.op) {
       case UGHIP_I_DEFINE_GLOBAL: return "";
       case UGHIP_I_DEFINE_LOCAL: o << "__shared__ " << dtype_c_name(in.dtype) << " " << var(i) << "[" << in.n << "];"; break;
@@ -850,7 +866,7 @@ class Lowering {
   }
 
   std::string signature(bool scratch) const {
-    std::ostringstream o;
+    Text o;
     for (size_t a = 0; a < s_.n_args; ++a) {
       if (a) o << ", ";
       o << (out_.arg_written[a] ? "" : "const ") << dtype_c_name(s_.args[a].dtype) << "* __restrict__ " << var((int)s_.args[a].var);
@@ -862,7 +878,7 @@ class Lowering {
     return o.str();
   }
 
-  void emit_range(std::ostringstream& o, int from, int to, int indent) const {
+  void emit_range(Text& o, int from, int to, int indent) const {
     int depth = indent;
     for (int i = from; i <= to; ++i) {
       int op = I_[i].op;
@@ -875,7 +891,7 @@ class Lowering {
 
   void emit_literal(unsigned grid, unsigned block) {
     if (block > 1024) fail("block_dim > 1024");
-    std::ostringstream o;
+    Text o;
     o << kPrelude << "\nextern \"C\" __global__ void __launch_bounds__(" << block << ") " << entry_ << "(" << signature(false) << ") {\n";
     emit_range(o, 0, n_ - 1, 1);
     o << "}\n";
@@ -1112,7 +1128,7 @@ class Lowering {
   // `const int v<loop> = lo + digit * step;` for each loop of `ls`.  `group` counts groups of
   // `vec` consecutive iterations of the innermost (fastest) loop; `ug_u` selects inside the group,
   // which keeps the addresses of the unrolled copies visibly consecutive for the compiler.
-  void emit_decode(std::ostringstream& o, const std::vector<int>& ls, const std::string& group, int vec, int indent) const {
+  void emit_decode(Text& o, const std::vector<int>& ls, const std::string& group, int vec, int indent) const {
     std::string pad(2 * indent, ' ');
     if (ls.empty()) return;
     const std::string left = "ug_r" + vp_;
@@ -1152,7 +1168,7 @@ class Lowering {
   // 10.7 -> 8.2.
   static bool overlapped(i64 extent, i64 threads) { return extent % 4 != 0 && threads > 64 && extent > (threads - 64) * 4; }
 
-  void emit_items(std::ostringstream& o, bool want_cols, uint64_t col_mask, int indent, bool guard_row_stores, int tpr, bool one_thread) const {
+  void emit_items(Text& o, bool want_cols, uint64_t col_mask, int indent, bool guard_row_stores, int tpr, bool one_thread) const {
     for (const Item& it : items_) {
       bool is_col = (it.deps & col_mask) != 0;
       if (is_col != want_cols) continue;
@@ -1168,7 +1184,7 @@ class Lowering {
   }
 
   // Statements of a reduction loop body with the fold redirected to the thread-local partial.
-  void emit_reduce_body(std::ostringstream& o, const Region& r, int indent, const char* fold_if = nullptr) const {
+  void emit_reduce_body(Text& o, const Region& r, int indent, const char* fold_if = nullptr) const {
     std::string ty = dtype_c_name(vt_[r.acc].dtype);
     std::string fn = reduce_functor(r.op);
     std::string part = "ug_p" + std::to_string(r.acc);
@@ -1194,7 +1210,7 @@ class Lowering {
 
   // Cooperative reduction by the `tpr` threads that share a row; afterwards every one of them
   // holds the folded accumulator in v<acc>.
-  void emit_region(std::ostringstream& o, const Region& r, int indent, int tpr) const {
+  void emit_region(Text& o, const Region& r, int indent, int tpr) const {
     std::string pad(2 * indent, ' ');
     const LoopInfo& L = loops_[r.loop];
     std::string ty = dtype_c_name(vt_[r.acc].dtype);
@@ -1217,7 +1233,7 @@ class Lowering {
     emit_region_finish(o, r, indent, tpr);
   }
 
-  void emit_region_finish(std::ostringstream& o, const Region& r, int indent, int tpr) const {
+  void emit_region_finish(Text& o, const Region& r, int indent, int tpr) const {
     std::string pad(2 * indent, ' ');
     std::string ty = dtype_c_name(vt_[r.acc].dtype);
     std::string fn = reduce_functor(r.op);
@@ -1242,7 +1258,7 @@ class Lowering {
     // here), and the next kernel would find them in another XCD's L2 at best.  SwiGLU [512, 5632]: 4.6 -> 3.6 us, [16384, 5632]
     // 184 -> 179 us.
     nt_stores_ = vec == 4 && !ughip::tune_on(ughip::TUNE_NO_NT_STORES);
-    std::ostringstream b;
+    Text b;
     b << "  const int ug_g = (int)blockIdx.x * " << block << " + (int)threadIdx.x;\n";
     b << "  if (ug_g >= " << (parametric_ ? kparam(groups) : std::to_string(groups)) << ") return;\n";
     // Items that depend on no loop are computed once per thread, ahead of the unrolled part.
@@ -1253,7 +1269,7 @@ class Lowering {
     emit_decode(b, chain_, "ug_g", vec, 2);
     emit_items(b, true, all, 2, false, 1, true);
     b << "  }\n}\n";
-    std::ostringstream o;
+    Text o;
     o << kPrelude << "\n";
     std::string sig = signature(false);
     if (parametric_) {
@@ -1274,7 +1290,7 @@ class Lowering {
     const int block = 256;
     uint64_t col_mask = 0;
     for (int l : cols) col_mask |= 1ull << l;
-    std::ostringstream o;
+    Text o;
     o << kPrelude << "\nextern \"C\" __global__ void __launch_bounds__(" << block << ") " << entry_ << "(" << signature(false) << ") {\n";
     o << "  const int ug_row = (int)blockIdx.x * " << block << " + (int)threadIdx.x;\n";
     o << "  if (ug_row >= " << nr << ") return;\n";
@@ -1321,7 +1337,7 @@ class Lowering {
         return;
       }
     }
-    std::ostringstream o;
+    Text o;
     o << kPrelude << "\nextern \"C\" __global__ void __launch_bounds__(" << block << ") " << entry_ << "(" << signature(grid_reduce) << ") {\n";
     o << "  const int ug_t = (int)threadIdx.x % " << tpr << ";\n";
     unsigned nb = 1;
@@ -1480,7 +1496,7 @@ class Lowering {
     int floats_left = 48;  // per thread: at 1024 threads the compiler has 128
   };
   // Row decoding and the loads of everything that is held; link: this kernel's argument that is not loaded but found in ug_link.
-  void emit_rows_head(std::ostringstream& o, Registers& regs, const std::vector<int>& arg_number, int link) {
+  void emit_rows_head(Text& o, Registers& regs, const std::vector<int>& arg_number, int link) {
     emit_decode(o, rows_, "ug_row", 1, 1);
     for (int i = 0; i < n_; ++i) {
       if (I_[i].op != UGHIP_I_LOAD || arg_of_[I_[i].v] < 0 || encl_[i] < 0) continue;
@@ -1515,7 +1531,7 @@ class Lowering {
     }
   }
   // The rest.  link: the argument whose store goes to ug_link (-1: none), kept: and to memory as well.
-  void emit_rows_body(std::ostringstream& o, int link, bool kept) {
+  void emit_rows_body(Text& o, int link, bool kept) {
     const bool masked = form_.width % ((i64)form_.vec * form_.tpr) != 0;
     uint64_t col_mask = 1ull << cols_[0];
     for (const Item& it : items_) {
@@ -1577,7 +1593,7 @@ class Lowering {
     }
     o << "  }\n";
   }
-  static void emit_rows_prologue(std::ostringstream& o, const std::string& entry, const std::string& sig, const RowsForm& f) {
+  static void emit_rows_prologue(Text& o, const std::string& entry, const std::string& sig, const RowsForm& f) {
     o << kPrelude << "\nextern \"C\" __global__ void __launch_bounds__(" << f.tpr * f.rows_per_block << ") " << entry << "(" << sig << ") {\n";
     o << "  const int ug_t = (int)threadIdx.x % " << f.tpr << ";\n";
     o << "  const int ug_row = (int)blockIdx.x * " << f.rows_per_block << " + (int)threadIdx.x / " << f.tpr << ";\n";
@@ -1595,7 +1611,7 @@ class Lowering {
   std::vector<int> rows_, cols_;
 
   // `int ug_g` (the group's place in the row as dealt out) and `int ug_i` (where its elements are)
-  void emit_group(std::ostringstream& o, int indent) const {
+  void emit_group(Text& o, int indent) const {
     const std::string pad(2 * indent, ' ');
     o << pad << "const int ug_g = (ug_t + ug_it * " << form_.tpr << ") * " << form_.vec << ";\n";
     if (form_.width % ((i64)form_.vec * form_.tpr) != 0) o << pad << "const int ug_i = ug_g < " << form_.width - form_.vec << " ? ug_g : " << form_.width - form_.vec << ";\n";
@@ -1657,7 +1673,7 @@ class Lowering {
   }
 
   void emit_rows() {
-    std::ostringstream o;
+    Text o;
     emit_rows_prologue(o, entry_, signature(false), form_);
     std::vector<int> number;
     for (size_t a = 0; a < s_.n_args; ++a) number.push_back((int)a);
@@ -1673,7 +1689,7 @@ class Lowering {
   }
 
   // First stage of a grid-wide reduction: workgroup `ug_blk` of `nb` takes every nb-th slab.
-  void emit_region_partial(std::ostringstream& o, const Region& r, int indent, int tpr, unsigned nb) const {
+  void emit_region_partial(Text& o, const Region& r, int indent, int tpr, unsigned nb) const {
     std::string pad(2 * indent, ' ');
     const LoopInfo& L = loops_[r.loop];
     std::string ty = dtype_c_name(vt_[r.acc].dtype);
@@ -1759,7 +1775,7 @@ bool lower_rows_pair(const ughip_ssa& first, const ughip_ssa& second, const std:
       aliases += "  " + b.arg_type(k) + " " + b.arg_name(k) + " = " + a.arg_name(shared[k]) + ";\n";
     }
   }
-  std::ostringstream o;
+  Text o;
   Lowering::emit_rows_prologue(o, entry, sig, *fa);
   o << aliases << "  " << dtype_c_name(first.args[link].dtype) << " ug_link[" << fa->per << "][" << fa->vec << "];\n";
   Lowering::Registers regs;
