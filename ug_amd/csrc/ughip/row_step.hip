@@ -1,13 +1,13 @@
 // Products of one row with their neighbours folded in (ughip_product_row): a decode step of the layers in ughip_layers.h.
 //
-// A workgroup of four waves takes 4 R columns, R per wave.  It asks for everything the input row is made of (PV 16-byte pieces per
-// thread and vector), then every wave for the first NB batches of four runs of 512 elements of its matrix rows (eight elements per
-// lane and run);
-// the row -- residual add with the norm of the sublayer in front, gate, norm -- is made in LDS in the shadow of the matrix, and
-// every wave multiplies, asking for batch b + NB where batch b was.  The input row costs a few cache reads per workgroup and spares the launches that would make it; the
-// first workgroup stores the new residual.  PLAIN: the row is x as it is (or, routed, times the experts' weights).  PV = 0: rows of any
-// length and alignment, element by element.
+// row_wide_kernel: the whole workgroup on every matrix row, the input row -- residual add with the norm of the sublayer in front, gate,
+// norm -- made in registers in every workgroup while the matrix is on its way.  It costs a workgroup a few cache reads and spares the
+// launches that would make it; the first one stores the new residual.  PLAIN: the row is x as it is (or, routed, times the experts' weights).
+// row_step_kernel: rows of any length and alignment.  A workgroup of four waves takes 4 R columns, R per wave: runs of 512 elements of the
+// matrix rows (eight elements per lane and run), four to a batch, batch b + NB asked for where batch b was; the input row in LDS.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "layers.h"
 #include "route.h"
@@ -94,40 +94,39 @@ struct Eight<float> {
   }
 };
 
+// What becomes of column `col`'s sum (with NM 2: the gate's and the up row's).
+template <int NM>
+__device__ __forceinline__ float finished(const RowArgs& a, int col, const float (&sums)[NM]) {
+  float v = sums[0];
+  if (a.bias) v += a.bias[col];
+  if constexpr (NM == 2) {
+    float u = sums[1];
+    if (a.bias) u += a.bias[a.n + col];
+    return glu_f(v, u, a.glu);
+  }
+  if (a.table) {
+    const int id = a.ids[0];
+    float t = __uint_as_float(0x7fc00000u);
+    if (id >= 0 && id < a.table_rows) {
+      const size_t at = (size_t)id * a.table_stride + a.table_col + col;
+      t = a.table_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(a.table)[at]) : static_cast<const float*>(a.table)[at];
+    }
+    v = gelu_tanh_f(v) * t;
+  }
+  return v;
+}
+
 // R columns of NM matrices per wave; VEC: rows are 16-byte aligned and a multiple of 8 long.  ROUTE as in ughip_row_step: with 2 a
 // column's row is the chosen experts' rows one after the other, each from a batch of its own on.
-template <typename WT, int R, int NM, int ROUTE, bool VEC, int NB, int PV, bool PLAIN>
+template <typename WT, int R, int NM, int ROUTE, bool VEC, int NB>
 __global__ void __launch_bounds__(256) row_step_kernel(RowArgs a) {
   extern __shared__ __attribute__((aligned(16))) float in[];  // the row (segments `padded` apart), then ROUTE 1: logits and work space
   __shared__ float red[4][4];
-  __shared__ float part_sum[4 * (PV ? PV : 1)];
   __shared__ int s_ids[64];
   __shared__ float s_wts[64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int padded = (a.k + RUN - 1) / RUN * RUN, bps = (padded / RUN + PRE - 1) / PRE, batches = (ROUTE == 2 ? a.segs : 1) * bps;
   const int col0 = (blockIdx.x * 4 + wave) * R;
-  constexpr int NP = PV ? PV : 1;
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  const int total = (ROUTE == 2 ? a.segs : 1) * a.k;
-  f32x4_t px[NP], py[NP], pyn[NP], pn[NP], pe[NP];  // x, y or the gate, the two norms' weights, and what joins x besides
-  if constexpr (PV != 0 && PLAIN) {
-#pragma unroll
-    for (int u = 0; u < PV; ++u) {
-      const int i = (u * 256 + (int)threadIdx.x) * 4;
-      px[u] = i < total ? *reinterpret_cast<const f32x4_t*>(a.x + i) : zero;
-    }
-  } else if constexpr (PV != 0) {
-#pragma unroll
-    for (int u = 0; u < PV; ++u) {
-      const int i = (u * 256 + (int)threadIdx.x) * 4;
-      const bool ok = i < a.k;  // a multiple of 4
-      px[u] = ok ? *reinterpret_cast<const f32x4_t*>(a.x + i) : zero;
-      py[u] = ok && (a.y || a.gate) ? *reinterpret_cast<const f32x4_t*>((a.y ? a.y : a.gate) + i) : zero;
-      pyn[u] = ok && a.y ? *reinterpret_cast<const f32x4_t*>(a.y_norm + i) : zero;
-      pn[u] = ok && a.norm ? *reinterpret_cast<const f32x4_t*>(a.norm + i) : zero;
-      pe[u] = ok && a.extra ? *reinterpret_cast<const f32x4_t*>(a.extra + i) : zero;
-    }
-  }
   if constexpr (ROUTE == 1) {  // which experts' matrices: before anything of them can be asked for
     float* lg = in + padded;
     for (int e = threadIdx.x; e < a.route.experts; e += 256) lg[e] = a.logits[e];
@@ -193,89 +192,10 @@ __global__ void __launch_bounds__(256) row_step_kernel(RowArgs a) {
 
   // the input row
   float ss = 0.f;
-  if constexpr (PV != 0 && PLAIN) {
-#pragma unroll
-    for (int u = 0; u < PV; ++u) {
-      const int i = (u * 256 + (int)threadIdx.x) * 4;
-      if constexpr (ROUTE == 2) {
-        // (i + 1/2) / k is never within a rounding of a whole number
-        const int j = (int)(((float)i + 0.5f) * a.inv_k);
-        if (i < total) *reinterpret_cast<f32x4_t*>(in + j * padded + (i - j * a.k)) = px[u] * s_wts[j];
-      } else {
-        if (i < padded) *reinterpret_cast<f32x4_t*>(in + i) = px[u];
-      }
-    }
-    if constexpr (ROUTE == 2)
-      for (int j = 0; j < a.segs; ++j)
-        for (int i = a.k + (int)threadIdx.x; i < padded; i += 256) in[j * padded + i] = 0.f;
-  } else if constexpr (ROUTE == 2) {
+  if constexpr (ROUTE == 2) {
     for (int j = 0; j < a.segs; ++j) {
       const float w = s_wts[j];
       for (int i = threadIdx.x; i < padded; i += 256) in[j * padded + i] = i < a.k ? a.x[j * a.k + i] * w : 0.f;
-    }
-  } else if constexpr (PV != 0) {
-    auto square = [](const f32x4_t& v) { return v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; };
-    if (a.y) {
-#pragma unroll
-      for (int u = 0; u < PV; ++u) ss += square(py[u]);
-      ss = block_sum<4>(ss, red[0]);
-      const float inv = 1.f / sqrtf(ss / (float)a.k + a.eps);
-#pragma unroll
-      for (int u = 0; u < PV; ++u) {
-        px[u] = px[u] + py[u] * inv * pyn[u] + pe[u];
-        const int i = (u * 256 + (int)threadIdx.x) * 4;
-        if (a.x_out && blockIdx.x == 0 && i < a.k) *reinterpret_cast<f32x4_t*>(a.x_out + i) = px[u];
-      }
-    } else if (a.gate && !a.gate_after) {
-#pragma unroll
-      for (int u = 0; u < PV; ++u)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) px[u][e] *= silu_f(py[u][e]);
-    }
-    if (a.norm && a.norm_groups == 1) {
-      ss = 0.f;
-#pragma unroll
-      for (int u = 0; u < PV; ++u) ss += square(px[u]);
-      ss = block_sum<4>(ss, red[1]);
-      const float inv = 1.f / sqrtf(ss / (float)a.k + a.eps);
-#pragma unroll
-      for (int u = 0; u < PV; ++u) px[u] = px[u] * inv * pn[u];
-    } else if (a.norm && a.k < 256 * a.norm_groups) {
-      // parts inside a wave's piece: 4, 8, .. or 128 elements (the host checks)
-      const int part = a.k / a.norm_groups;
-#pragma unroll
-      for (int u = 0; u < PV; ++u) {
-        float s = square(px[u]);
-        for (int d = part >> 3; d; d >>= 1) s += __shfl_xor(s, d, 64);
-        px[u] = px[u] * (1.f / sqrtf(s / (float)part + a.eps)) * pn[u];
-      }
-    } else if (a.norm) {
-      // parts of whole runs of 256 elements (the host checks): one wave's pieces each
-      const int runs = a.k / a.norm_groups / 256;
-#pragma unroll
-      for (int u = 0; u < PV; ++u) {
-        const float s = wave_sum(square(px[u]));
-        if (lane == 0) part_sum[u * 4 + wave] = s;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < PV; ++u) {
-        const int first = (u * 4 + wave) / runs * runs;
-        float s = 0.f;
-        for (int i = 0; i < runs && first + i < 4 * PV; ++i) s += part_sum[first + i];
-        px[u] = px[u] * (1.f / sqrtf(s / (float)(runs * 256) + a.eps)) * pn[u];
-      }
-    }
-    if (a.gate && a.gate_after) {
-#pragma unroll
-      for (int u = 0; u < PV; ++u)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) px[u][e] *= sigmoid_f(py[u][e]);
-    }
-#pragma unroll
-    for (int u = 0; u < PV; ++u) {
-      const int i = (u * 256 + (int)threadIdx.x) * 4;
-      if (i < padded) *reinterpret_cast<f32x4_t*>(in + i) = px[u];
     }
   } else {
     for (int i = threadIdx.x; i < padded; i += 256) {
@@ -357,66 +277,229 @@ __global__ void __launch_bounds__(256) row_step_kernel(RowArgs a) {
     for (int m = 0; m < NM; ++m) acc[m][r] = wave_sum(acc[m][r]);
     if (lane != 0 || !live[r]) continue;
     const int col = col0 + r;
-    float v = acc[0][r];
-    if (a.bias) v += a.bias[col];
-    if (NM == 2) {
-      float u = acc[NM - 1][r];
-      if (a.bias) u += a.bias[a.n + col];
-      v = glu_f(v, u, a.glu);
-    } else if (a.table) {
-      const int id = a.ids[0];
-      float t = __uint_as_float(0x7fc00000u);
-      if (id >= 0 && id < a.table_rows) {
-        const size_t at = (size_t)id * a.table_stride + a.table_col + col;
-        t = a.table_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(a.table)[at]) : static_cast<const float*>(a.table)[at];
-      }
-      v = gelu_tanh_f(v) * t;
-    }
-    a.dst[col] = v;
+    float u[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) u[m] = acc[m][r];
+    a.dst[col] = finished<NM>(a, col, u);
   }
 }
 
-template <typename WT, int R, int NM, int ROUTE, bool VEC, int NB, int PV, bool PLAIN>
+// The sum over the NW waves of a workgroup, NW up to 16 and known when it runs; `red` holds 16 floats of which those past NW are zero.
+__device__ __forceinline__ float any_block_sum(float v, float* red) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return row_sum16(red[threadIdx.x & 15]);
+}
+
+// The same product with the whole workgroup on every matrix row: thread t holds elements 8 t .. 8 t + 7 of the input row in registers (of
+// ROUTE 2: of the chosen experts' rows one after the other), as many waves as that takes, and the workgroup walks B batches of R columns, two
+// batches on their way.
+template <typename WT, int NM, int R, int B, int ROUTE, bool PLAIN>
+__global__ void __launch_bounds__(1024) row_wide_kernel(RowArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float route_work[];  // ROUTE 1: logits and work space
+  __shared__ float red[3][16];
+  __shared__ float part[NM * B * R][17];
+  __shared__ int s_ids[64];
+  __shared__ float s_wts[64];
+  constexpr int NB = B < 2 ? B : 2;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), waves = blockDim.x >> 6, e0 = t * 8;
+  const int total = (ROUTE == 2 ? a.segs : 1) * a.k;
+  const bool ok = e0 < total;
+  const int at0 = ok ? e0 : 0;  // (a lane past the end reads the row's first elements and multiplies them with zeros)
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t v[2], y[2], yn[2], nm[2], ex[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    v[i] = *reinterpret_cast<const f32x4_t*>(a.x + at0 + 4 * i);
+    if constexpr (!PLAIN) {
+      if (a.y || a.gate) y[i] = *reinterpret_cast<const f32x4_t*>((a.y ? a.y : a.gate) + at0 + 4 * i);
+      if (a.y) yn[i] = *reinterpret_cast<const f32x4_t*>(a.y_norm + at0 + 4 * i);
+      if (a.norm) nm[i] = *reinterpret_cast<const f32x4_t*>(a.norm + at0 + 4 * i);
+      if (a.extra) ex[i] = *reinterpret_cast<const f32x4_t*>(a.extra + at0 + 4 * i);
+    }
+  }
+  if constexpr (!PLAIN)
+    if (t < 48) red[t >> 4][t & 15] = 0.f;
+  if constexpr (ROUTE == 1) {  // which experts' matrices: before anything of them can be asked for
+    float* lg = route_work;
+    for (int e = t; e < a.route.experts; e += blockDim.x) lg[e] = a.logits[e];
+    __syncthreads();
+    if (wave == 0) {
+      float* work = lg + a.route.experts;
+      int* ids = reinterpret_cast<int*>(work + route_lds_floats(a.route.experts, a.route.groups));
+      float* wts = reinterpret_cast<float*>(ids + a.route.top);
+      route_choose(lg, a.route, work, ids, wts);
+      if (lane < a.route.top) s_ids[lane] = ids[lane];
+      if (blockIdx.x == 0 && lane < a.route.top) a.route_ids[lane] = ids[lane], a.route_weights[lane] = wts[lane];
+    }
+    __syncthreads();
+  }
+  int seg = 0;
+  if constexpr (ROUTE == 2) {
+    if (t < a.segs) {
+      const int e = a.route_ids[t];
+      s_ids[t] = e >= 0 && e < a.route.experts ? e : 0;
+      s_wts[t] = a.route_weights[t];
+    }
+    __syncthreads();
+    seg = (int)(((float)at0 + 0.5f) * a.inv_k);  // never within a rounding of a whole number
+  }
+  const int col0 = blockIdx.x * (B * R);
+  const WT* mine = static_cast<const WT*>(a.w) + (ROUTE == 2 ? (size_t)s_ids[seg] * a.w_group + (size_t)(at0 - seg * a.k) : (size_t)at0);
+  Eight<WT> held[NB][NM][R];
+  auto fetch = [&](int b, Eight<WT>(&to)[NM][R]) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int col = min(col0 + b * R + r, a.cols - 1);
+      size_t at = (size_t)col * a.k;
+      if (ROUTE == 1) {
+        const int j = col / a.n;
+        at = (size_t)__builtin_amdgcn_readfirstlane(s_ids[j]) * a.w_group + (size_t)(col - j * a.n) * a.k;
+      }
+#pragma unroll
+      for (int m = 0; m < NM; ++m) to[m][r].load(mine + at + (m ? (size_t)a.n * a.k : 0));
+    }
+  };
+#pragma unroll
+  for (int b = 0; b < NB; ++b) fetch(b, held[b]);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // the input row
+  if (!ok) v[0] = v[1] = zero;
+  if constexpr (ROUTE == 2) {
+    const float w = s_wts[seg];
+    v[0] *= w, v[1] *= w;
+  }
+  if constexpr (!PLAIN) {
+    auto square = [](const f32x4_t& p, const f32x4_t& q) { return p.x * p.x + p.y * p.y + p.z * p.z + p.w * p.w + (q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w); };
+    __syncthreads();  // (`red` is clear)
+    if (a.y) {
+      const float ss = any_block_sum(ok ? square(y[0], y[1]) : 0.f, red[0]), inv = 1.f / sqrtf(ss / (float)a.k + a.eps);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        v[i] = v[i] + y[i] * inv * yn[i];
+        if (a.extra) v[i] += ex[i];
+        if (a.x_out && blockIdx.x == 0 && ok) *reinterpret_cast<f32x4_t*>(a.x_out + e0 + 4 * i) = v[i];
+      }
+    } else if (a.gate && !a.gate_after) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[i][e] *= silu_f(y[i][e]);
+    }
+    if (!ok) v[0] = v[1] = zero;
+    if (a.norm) {
+      float ss = square(v[0], v[1]);
+      const int part = a.k / a.norm_groups;
+      if (a.norm_groups == 1) {
+        ss = any_block_sum(ss, red[1]);
+      } else if (part < 512) {  // 1, 2, 4, .. or 32 lanes (the host checks)
+        for (int d = part >> 4; d; d >>= 1) ss += __shfl_xor(ss, d, 64);
+      } else {  // whole waves (the host checks)
+        ss = wave_sum(ss);
+        if (lane == 0) red[2][wave] = ss;
+        __syncthreads();
+        const int run = part >> 9, first = wave / run * run;
+        ss = 0.f;
+        for (int i = 0; i < run; ++i) ss += red[2][first + i];
+      }
+      const float inv = 1.f / sqrtf(ss / (float)part + a.eps);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) v[i] = v[i] * inv * nm[i];
+      if (!ok) v[0] = v[1] = zero;
+    }
+    if (a.gate && a.gate_after) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[i][e] *= sigmoid_f(y[i][e]);
+      if (!ok) v[0] = v[1] = zero;
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float s = wave_sum(held[b % NB][m][r].dot(v[0], v[1], 0.f));
+        if (lane == 0) part[(m * B + b) * R + r][wave] = s;
+      }
+    if (b + NB < B) fetch(b + NB, held[b % NB]);
+  }
+  __syncthreads();
+  const int col = col0 + t;
+  if (t >= B * R || col >= a.cols) return;
+  float u[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    u[m] = 0.f;
+    for (int w = 0; w < waves; ++w) u[m] += part[m * B * R + t][w];
+  }
+  a.dst[col] = finished<NM>(a, col, u);
+}
+
+template <typename WT, int R, int NM, int ROUTE, bool VEC>
 hipError_t launch_one(hipStream_t st, const RowArgs& a, size_t lds) {
   const unsigned grid = (unsigned)((a.cols + 4 * R - 1) / (4 * R));
-  auto kernel = row_step_kernel<WT, R, NM, ROUTE, VEC, NB, PV, PLAIN>;
+  auto kernel = row_step_kernel<WT, R, NM, ROUTE, VEC, VEC ? 2 : 1>;
   if (lds > 60 * 1024)
     if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); e != hipSuccess) return e;
   kernel<<<grid, 256, lds, st>>>(a);
   return hipGetLastError();
 }
 
-// pieces: the input row is read 16 bytes at a time
 template <typename WT, int R, int NM, int ROUTE>
-hipError_t launch_vec(hipStream_t st, const RowArgs& a, size_t lds, bool vec, bool pieces) {
-  if (!vec) return launch_one<WT, R, NM, ROUTE, false, 1, 0, false>(st, a, lds);
-  const int total = (ROUTE == 2 ? a.segs : 1) * a.k;
-  if (pieces && !a.y && !a.gate && !a.norm && total <= 8192) {
-    if constexpr (ROUTE != 2)
-      if (total <= 2048) return launch_one<WT, R, NM, ROUTE, true, 1, 2, true>(st, a, lds);
-    return launch_one<WT, R, NM, ROUTE, true, 2, 8, true>(st, a, lds);
-  }
-  if constexpr (ROUTE != 2) {
-    if (pieces && a.k <= 2048) return launch_one<WT, R, NM, ROUTE, true, 1, 2, false>(st, a, lds);
-    if (pieces && a.k <= 4096) return launch_one<WT, R, NM, ROUTE, true, 2, 4, false>(st, a, lds);
-  }
-  return launch_one<WT, R, NM, ROUTE, true, 2, 0, false>(st, a, lds);
+hipError_t launch_vec(hipStream_t st, const RowArgs& a, size_t lds, bool vec) {
+  return vec ? launch_one<WT, R, NM, ROUTE, true>(st, a, lds) : launch_one<WT, R, NM, ROUTE, false>(st, a, lds);
 }
 
 template <typename WT, int NM, int ROUTE>
-hipError_t launch_rows(hipStream_t st, const RowArgs& a, size_t lds, bool vec, bool pieces) {
+hipError_t launch_rows(hipStream_t st, const RowArgs& a, size_t lds, bool vec) {
   // enough workgroups for the chip first, then more columns for each of them to share the input row
   const int r = a.cols >= 8192 && NM == 1 ? 4 : a.cols >= 2048 ? 2 : 1;
   if constexpr (NM == 1)
-    if (r == 4) return launch_vec<WT, 4, NM, ROUTE>(st, a, lds, vec, pieces);
-  return r >= 2 ? launch_vec<WT, 2, NM, ROUTE>(st, a, lds, vec, pieces) : launch_vec<WT, 1, NM, ROUTE>(st, a, lds, vec, pieces);
+    if (r == 4) return launch_vec<WT, 4, NM, ROUTE>(st, a, lds, vec);
+  return r >= 2 ? launch_vec<WT, 2, NM, ROUTE>(st, a, lds, vec) : launch_vec<WT, 1, NM, ROUTE>(st, a, lds, vec);
 }
 
 template <typename WT>
-hipError_t launch_any(hipStream_t st, const RowArgs& a, int route, bool up, size_t lds, bool vec, bool pieces) {
-  if (route == 1) return up ? launch_rows<WT, 2, 1>(st, a, lds, vec, pieces) : hipErrorInvalidValue;
-  if (route == 2) return launch_rows<WT, 1, 2>(st, a, lds, vec, pieces);
-  return up ? launch_rows<WT, 2, 0>(st, a, lds, vec, pieces) : launch_rows<WT, 1, 0>(st, a, lds, vec, pieces);
+hipError_t launch_any(hipStream_t st, const RowArgs& a, int route, bool up, size_t lds, bool vec) {
+  if (route == 1) return up ? launch_rows<WT, 2, 1>(st, a, lds, vec) : hipErrorInvalidValue;
+  if (route == 2) return launch_rows<WT, 1, 2>(st, a, lds, vec);
+  return up ? launch_rows<WT, 2, 0>(st, a, lds, vec) : launch_rows<WT, 1, 0>(st, a, lds, vec);
+}
+
+constexpr int WIDE_MAX = 8192;  // elements of the input row: eight to a thread
+
+// Columns per workgroup: the more, the fewer times the input row is read and made, but every CU wants a workgroup and some six waves to keep
+// enough of the matrix on its way (and past 16 matrix rows the last ones wait).  bf16, us by columns per workgroup 1 / 2 / 4 / 8 / 16, in a token's sequence:
+//   1024 of 1024 3.5 / 3.6 / 3.5 / 4.1 / 5.2, 3336 of 1024 6.5 / 5.9 / 5.0 / 5.2 / 6.2, gated 2816 of 1024 6.6 / 6.2 / 5.4 / 6.3 / 8.2, 1024 of 2816 3.6 / 3.7 / 3.7 / 4.3 / 5.3,
+//   6416 of 2048 15.4 / 11.5 / 9.9 / 9.1 / 8.1, gated 5632 of 2048 17.6 / 13.6 / 12.1 / 11.0 / 12.2, 2048 of 5632 7.4 / 6.4 / 6.0 / 6.0 / 7.2,
+//   32000 of 1024 28.6 / 17.4 / 13.5 / 12.5 / 13.8, of 2048 60 / 41 / 31 / 25 / 23
+int wide_columns(int cols, int threads, int matrices) {
+  int most = 16 / matrices;
+  while (most > 1 && ((cols + most - 1) / most < 256 || (cols + most - 1) / most * (threads / 64) < 1400)) most /= 2;
+  return most;
+}
+
+template <typename WT, int NM, int ROUTE, bool PLAIN>
+hipError_t launch_wide(hipStream_t st, const RowArgs& a, size_t lds) {
+  const int total = (ROUTE == 2 ? a.segs : 1) * a.k, threads = (total / 8 + 63) / 64 * 64;
+  auto go = [&](auto kernel, int columns) {
+    kernel<<<(unsigned)((a.cols + columns - 1) / columns), threads, lds, st>>>(a);
+    return hipGetLastError();
+  };
+  switch (wide_columns(a.cols, threads, NM)) {
+    case 1: return go(row_wide_kernel<WT, NM, 1, 1, ROUTE, PLAIN>, 1);
+    case 2: return go(row_wide_kernel<WT, NM, 2, 1, ROUTE, PLAIN>, 2);
+    case 4: return go(row_wide_kernel<WT, NM, 2, 2, ROUTE, PLAIN>, 4);
+    case 8: return go(row_wide_kernel<WT, NM, 2, 4, ROUTE, PLAIN>, 8);
+    default:
+      if constexpr (NM == 1) return go(row_wide_kernel<WT, NM, 4, 4, ROUTE, PLAIN>, 16);
+      return hipErrorInvalidValue;
+  }
 }
 
 constexpr size_t ROW_MAX = 16000;
@@ -512,9 +595,21 @@ extern "C" int ughip_product_row(ughip_device* dev, const ughip_row_step* p) {
   const bool vec = p->k % 8 == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15) == 0;
   auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   const size_t part = p->k / norm_groups;
-  const bool parts_fit = !p->norm || norm_groups == 1 || part % 256 == 0 || (part >= 4 && part < 256 && (part & (part - 1)) == 0);
-  const bool pieces = p->k % 4 == 0 && parts_fit && a16(a.x) && a16(a.y) && a16(a.gate) && a16(a.x_out) && a16(a.extra);
-  UGHIP_HIPCHK(p->w->dtype == UGHIP_BF16 ? launch_any<uint16_t>(dev->stream, a, p->route, glu, lds, vec, pieces)
-                                         : launch_any<float>(dev->stream, a, p->route, glu, lds, vec, pieces));
+  // pieces of eight elements, a thread each, and normed parts of whole waves or of whole powers of two of lanes
+  const bool parts_fit = !p->norm || norm_groups == 1 || part % 512 == 0 || (part >= 8 && part < 512 && (part & (part - 1)) == 0);
+  if (vec && total <= (size_t)WIDE_MAX && parts_fit && a16(a.x) && a16(a.y) && a16(a.gate) && a16(a.x_out) && a16(a.extra)) {
+    const size_t work = p->route == 1 ? (p->experts + (size_t)route_lds_floats(a.route.experts, a.route.groups) + 2 * p->top) * sizeof(float) : 0;
+    const bool plain = !a.y && !a.gate && !a.norm;
+    auto go = [&](auto type) {
+      using WT = decltype(type);
+      if (p->route == 1) return launch_wide<WT, 2, 1, true>(dev->stream, a, work);
+      if (p->route == 2) return launch_wide<WT, 1, 2, true>(dev->stream, a, 0);
+      if (glu) return plain ? launch_wide<WT, 2, 0, true>(dev->stream, a, 0) : launch_wide<WT, 2, 0, false>(dev->stream, a, 0);
+      return plain ? launch_wide<WT, 1, 0, true>(dev->stream, a, 0) : launch_wide<WT, 1, 0, false>(dev->stream, a, 0);
+    };
+    UGHIP_HIPCHK(p->w->dtype == UGHIP_BF16 ? go(uint16_t()) : go(float()));
+    return UGHIP_OK;
+  }
+  UGHIP_HIPCHK(p->w->dtype == UGHIP_BF16 ? launch_any<uint16_t>(dev->stream, a, p->route, glu, lds, vec) : launch_any<float>(dev->stream, a, p->route, glu, lds, vec));
   return UGHIP_OK;
 }
