@@ -570,9 +570,12 @@ __global__ void __launch_bounds__(C * 4) delta_out_kernel(DeltaArgs a) {
 
 // ---- one position -------------------------------------------------------------------------------------------------------------
 // A workgroup takes a head and COLS columns of its state: it convolves those columns and the head's q and k (again in every workgroup:
-// a few hundred channels), makes the head's decays, then 8 threads per column walk the state.  The ring's slot of this position is one
+// a few hundred channels), makes the head's decays, then GROUPS threads per column walk the state.  The ring's slot of this position is one
 // that no tap of this position reads, so the rows go in while other workgroups still convolve.
-constexpr int COLS = 32, GROUPS = 8, HELD = 16;
+// What bounds it: its chain of phases, each a trip to memory or LDS (the state of 8 heads is 0.5 MB).  8 threads per column with bounds checks on
+// every row they hold and sums over eight lanes through LDS 8.4 us, 16 threads, no checks where none are needed and the sums in registers 4.9
+// (8 or 16 heads of 128; a launch that streams 2 MB takes 2.6).
+constexpr int COLS = 32, GROUPS = 16, HELD = 8, STEP_THREADS = COLS * GROUPS;
 struct DeltaStepArgs {
   const float* qkv;  // this position's inputs of the convolution
   const float* b;
@@ -663,11 +666,18 @@ __device__ __forceinline__ float row_part(const WT* row, const float* x, int k0,
   return s;
 }
 
-constexpr int ROUNDS = 5, PIECES = 2;  // of the decays' and gates' rows, asked for before anything else: 160 rows of up to 128 elements
-template <typename WT, bool V8, int TAPS>
-__global__ void __launch_bounds__(256) delta_step_kernel(DeltaStepArgs a) {
+// The sum over the eight lanes that share all bits of their number but the last three.
+__device__ __forceinline__ float sum8(float v) {
+  v += dpp_move<0xB1>(v);         // quad_perm: lane ^ 1
+  v += dpp_move<0x4E>(v);         // quad_perm: lane ^ 2
+  return v + dpp_move<0x141>(v);  // row_half_mirror: 7 - lane, one of the other four
+}
+constexpr int ROUND_ROWS = STEP_THREADS / 8, ROUNDS = (160 + ROUND_ROWS - 1) / ROUND_ROWS, PIECES = 2;  // of the decays' and gates' rows, asked for before anything else: 160 rows of up to 128 elements
+// WHOLE: heads of GROUPS * HELD elements, values in whole runs of COLS: every thread holds its part of the state, and all of it.
+template <typename WT, bool V8, int TAPS, bool WHOLE>
+__global__ void __launch_bounds__(STEP_THREADS) delta_step_kernel(DeltaStepArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int d = a.dim, h = blockIdx.x, p0 = blockIdx.y * COLS, per = a.heads / a.kv_heads, g = h / per, gd = a.kv_heads * d;
+  const int d = WHOLE ? GROUPS * HELD : a.dim, h = blockIdx.x, p0 = blockIdx.y * COLS, per = a.heads / a.kv_heads, g = h / per, gd = a.kv_heads * d;
   float* q = lds;
   float* k = q + d;
   float* decay = k + d;
@@ -682,18 +692,18 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaStepArgs a) {
     return gate ? static_cast<const WT*>(a.w_z) + (size_t)(h * a.vdim + p0 + r - d) * a.z_rank : static_cast<const WT*>(a.w_a) + (size_t)(h * d + r) * a.a_rank;
   };
   Piece8<WT> pre[V8 ? ROUNDS : 1][PIECES];
-  const int r_mine = row8 + 32 * l8;  // the row whose decay (or gate) this lane finishes
+  const int r_mine = row8 + ROUND_ROWS * l8;  // the row whose decay (or gate) this lane finishes
   const float bias = a.dt_bias[h * d + min(r_mine, d - 1)];
   if constexpr (V8) {
 #pragma unroll
     for (int u = 0; u < ROUNDS; ++u) {
-      const int r = min(row8 + 32 * u, d + mine - 1), n = r >= d ? a.z_rank : a.a_rank;
+      const int r = min(row8 + ROUND_ROWS * u, d + mine - 1), n = r >= d ? a.z_rank : a.a_rank;
 #pragma unroll
       for (int b = 0; b < PIECES; ++b) pre[u][b].load(row_of(r) + (b * 64 + l8 * 8 < n ? b * 64 + l8 * 8 : 0));
     }
   }
   float* S = a.s + (size_t)h * d * a.vdim + p;
-  const bool there = p < a.vdim;
+  const bool there = WHOLE || p < a.vdim;
   float held[HELD];  // the first of the state's rows (lanes without a place in it load another's)
   {
     const float* Sl = a.s + (size_t)h * d * a.vdim + (there ? p : 0);
@@ -703,7 +713,7 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaStepArgs a) {
   __builtin_amdgcn_sched_barrier(0);
   float* slot = a.ring + (size_t)a.slot * a.channels;
   const bool first = h % per == 0 && blockIdx.y == 0;  // stores the key head's rows
-  for (int i = tid; i < 2 * d; i += 256) {
+  for (int i = tid; i < 2 * d; i += STEP_THREADS) {
     const int c = (i < d ? 0 : gd - d) + g * d + i;
     lds[i] = conv_one<TAPS>(a, c);
     if (first) slot[c] = a.qkv[c];
@@ -713,8 +723,8 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaStepArgs a) {
     vs[tid] = conv_one<TAPS>(a, c);
     slot[c] = a.qkv[c];
   }
-  for (int i = tid; i < a.a_rank; i += 256) a_in[i] = a.a_in[i];
-  for (int i = tid; i < a.z_rank; i += 256) z_in[i] = a.z_in[i];
+  for (int i = tid; i < a.a_rank; i += STEP_THREADS) a_in[i] = a.a_in[i];
+  for (int i = tid; i < a.z_rank; i += STEP_THREADS) z_in[i] = a.z_in[i];
   if (a.fresh) {  // nothing is known of the state's memory
 #pragma unroll
     for (int u = 0; u < HELD; ++u) held[u] = 0.f;
@@ -728,11 +738,6 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaStepArgs a) {
     ss = wave_sum(ss);
     if (lane == 0) scale[wave] = 1.f / sqrtf(ss + UNIT_EPS) * (wave ? 1.f : 1.f / sqrtf((float)d));
   }
-  auto over8 = [&](float s) {
-    s += __shfl_xor(s, 4, 64);
-    s += __shfl_xor(s, 2, 64);
-    return s + __shfl_xor(s, 1, 64);
-  };
   auto finish = [&](int r, float s, float b) {
     if (r >= d + mine) return;
     if (r >= d) a.out[(size_t)a.heads * a.vdim + h * a.vdim + p0 + r - d] = s;
@@ -742,21 +747,21 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaStepArgs a) {
     float s_mine = 0.f;
 #pragma unroll
     for (int u = 0; u < ROUNDS; ++u) {
-      const int rr = min(row8 + 32 * u, d + mine - 1), n = rr >= d ? a.z_rank : a.a_rank;
+      const int rr = min(row8 + ROUND_ROWS * u, d + mine - 1), n = rr >= d ? a.z_rank : a.a_rank;
       const float* x = rr >= d ? z_in : a_in;
       float s = 0.f;
 #pragma unroll
       for (int b = 0; b < PIECES; ++b)
         if (b * 64 + l8 * 8 < n) s += pre[u][b].dot(x + b * 64 + l8 * 8);
       if (n > PIECES * 64) s += row_part<WT, V8>(row_of(rr), x, PIECES * 64, n, l8);
-      s = over8(s);
+      s = sum8(s);
       if (l8 == u) s_mine = s;
     }
     if (l8 < ROUNDS) finish(r_mine, s_mine, bias);
   }
-  for (int r = row8 + (V8 ? 32 * ROUNDS : 0); r < d + mine; r += 32) {  // a row's eight lanes stay together
+  for (int r = row8 + (V8 ? ROUND_ROWS * ROUNDS : 0); r < d + mine; r += ROUND_ROWS) {  // a row's eight lanes stay together
     const bool gate = r >= d;
-    const float s = over8(row_part<WT, V8>(row_of(r), gate ? z_in : a_in, 0, gate ? a.z_rank : a.a_rank, l8));
+    const float s = sum8(row_part<WT, V8>(row_of(r), gate ? z_in : a_in, 0, gate ? a.z_rank : a.a_rank, l8));
     if (l8 == 0) finish(r, s, gate ? 0.f : a.dt_bias[h * d + r]);
   }
   __syncthreads();
@@ -765,11 +770,11 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaStepArgs a) {
 #pragma unroll
   for (int u = 0; u < HELD; ++u) {
     const int c = grp + GROUPS * u;
-    if (c >= d) break;
+    if (!WHOLE && c >= d) break;
     held[u] *= decay[c];
     sk += held[u] * (k[c] * ks);
   }
-  if (there && !a.fresh)
+  if (!WHOLE && there && !a.fresh)
     for (int c = grp + GROUPS * HELD; c < d; c += GROUPS) sk += S[(size_t)c * a.vdim] * decay[c] * (k[c] * ks);
   part[grp][col] = sk;
   __syncthreads();
@@ -782,12 +787,12 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaStepArgs a) {
 #pragma unroll
   for (int u = 0; u < HELD; ++u) {
     const int c = grp + GROUPS * u;
-    if (c >= d) break;
+    if (!WHOLE && c >= d) break;
     const float v = held[u] + k[c] * ks * u_new;
     if (there) S[(size_t)c * a.vdim] = v;
     o += v * (q[c] * qs);
   }
-  if (there)
+  if (!WHOLE && there)
     for (int c = grp + GROUPS * HELD; c < d; c += GROUPS) {
       float v = k[c] * ks * u_new;
       if (!a.fresh) v += S[(size_t)c * a.vdim] * decay[c];
@@ -920,12 +925,13 @@ extern "C" int ughip_delta_step(ughip_device* dev, const ughip_delta* p) {
                   (int)(p->pos < p->n_taps ? p->pos : p->n_taps), (int)(p->pos % p->n_taps), (int)p->n_taps, (int)H, (int)G, (int)d, (int)vd, (int)p->a_rank, (int)p->z_rank, (int)ch, p->pos == 0};
   const bool v8 = p->a_rank % 8 == 0 && p->z_rank % 8 == 0 && (reinterpret_cast<uintptr_t>(a.w_a) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.w_z) & 15) == 0;
   const size_t lds = (3 * d + p->a_rank + p->z_rank) * sizeof(float);
-  auto go = [&](auto kernel) { kernel<<<dim3((unsigned)H, (unsigned)((vd + COLS - 1) / COLS)), 256, lds, dev->stream>>>(a); };
-  const bool bf = p->w_a->dtype == UGHIP_BF16;
-  auto taps = [&](auto type, auto whole) {
+  auto go = [&](auto kernel) { kernel<<<dim3((unsigned)H, (unsigned)((vd + COLS - 1) / COLS)), STEP_THREADS, lds, dev->stream>>>(a); };
+  const bool bf = p->w_a->dtype == UGHIP_BF16, whole = d == GROUPS * HELD && vd % COLS == 0;
+  auto taps = [&](auto type, auto pieces) {
     using WT = decltype(type);
-    constexpr bool V8 = decltype(whole)::value;
-    p->n_taps == 4 ? go(delta_step_kernel<WT, V8, 4>) : p->n_taps == 3 ? go(delta_step_kernel<WT, V8, 3>) : p->n_taps == 2 ? go(delta_step_kernel<WT, V8, 2>) : go(delta_step_kernel<WT, V8, 0>);
+    constexpr bool V8 = decltype(pieces)::value;
+    if (V8 && whole && p->n_taps == 4) return go(delta_step_kernel<WT, V8, 4, V8>);
+    p->n_taps == 4 ? go(delta_step_kernel<WT, V8, 4, false>) : p->n_taps == 3 ? go(delta_step_kernel<WT, V8, 3, false>) : p->n_taps == 2 ? go(delta_step_kernel<WT, V8, 2, false>) : go(delta_step_kernel<WT, V8, 0, false>);
   };
   if (bf) v8 ? taps(uint16_t(), std::true_type{}) : taps(uint16_t(), std::false_type{});
   else v8 ? taps(float(), std::true_type{}) : taps(float(), std::false_type{});
