@@ -138,35 +138,38 @@ struct SplitArgs {
   float* acc;  // [splits][kv_heads rows][vdim]
   float* ml;   // [splits][kv_heads rows][2]
   size_t dst_stride;
-  int rows, row_blocks, splits, window;  // rows: (position, head) pairs per key head
+  int rows, row_blocks, splits, window, per;  // rows: (position, head) pairs per key head; per: heads per key head
   bool dst_bf16;
 };
 constexpr int SK = 32;
 
-// NW waves.  APPEND: one position, whose key and value come from the projected row.
-template <typename T, int DQ, int DV, int NW, bool APPEND>
+// NW waves; W value elements of its heads (DV, or 32: other workgroups take the rest and make the scores again).  APPEND: one position, whose
+// key and value come from the projected row.  VEC as for `turned`.
+template <typename T, int DQ, int DV, int NW, bool APPEND, bool VEC, int W>
 __global__ void __launch_bounds__(64 * NW) attention_split_kernel(SplitArgs a) {
   constexpr int E = 16 / sizeof(T), QC = DQ / E, NV = sizeof(T) == 2 ? 2 : 4;  // NV: 16-byte value operands of a tile and 32 value elements
   constexpr bool BF = sizeof(T) == 2;
-  constexpr int Q_ROW = DQ + E;
+  constexpr int Q_ROW = DQ + E, VB = W / 32, ACROSS = DV / W;
   extern __shared__ __attribute__((aligned(16))) float parts[];
   const GroupedArgs& g = a.g;
-  const int kv = blockIdx.x % g.kv_heads, rb = blockIdx.x / g.kv_heads, split = blockIdx.y, per = g.heads / g.kv_heads;
+  const int kv = blockIdx.x, split = blockIdx.y, per = a.per, rb = blockIdx.z / ACROSS, v0 = blockIdx.z % ACROSS * W;
+  if (ACROSS > 1 && v0 >= g.vdim) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 31, hf = lane >> 5;
-  const int r_last = min(a.rows, rb * 32 + 32) - 1, r_mine = min(rb * 32 + col, r_last), p_mine = g.pos + r_mine / per;
-  const int first = g.pos + rb * 32 / per, last = g.pos + r_last / per, s_all = g.pos + g.t;
-  const int tile0 = a.window ? max(0, first - a.window + 1) / SK : 0, tiles = last / SK + 1 - tile0, share = (tiles + a.splits - 1) / a.splits;
+  const int r_last = min(a.rows, rb * 32 + 32) - 1, r_mine = min(rb * 32 + col, r_last), p_mine = g.pos + (APPEND ? 0 : r_mine / per);
+  const int first = g.pos + (APPEND ? 0 : rb * 32 / per), last = g.pos + (APPEND ? 0 : r_last / per), s_all = g.pos + g.t;
+  const int tile0 = a.window ? max(0, first - a.window + 1) / SK : 0, tiles = last / SK + 1 - tile0, share = a.splits == 1 ? tiles : (tiles + a.splits - 1) / a.splits;
   const int k_stop = min(tile0 + tiles, tile0 + (split + 1) * share) * SK, oldest = a.window ? p_mine - a.window : -1;
   const T* keys = static_cast<const T*>(g.kc) + (size_t)kv * g.cap * DQ;
-  const T* values = static_cast<const T*>(g.vc) + (size_t)kv * g.vdim * g.cap;
-  u32x4_t kf[QC / 2], vf[DV / 32][NV];
+  const T* values = static_cast<const T*>(g.vc) + ((size_t)kv * g.vdim + v0) * g.cap;
+  const int v_left = g.vdim - v0;
+  u32x4_t kf[QC / 2], vf[VB][NV];
   auto fetch = [&](int k0) {  // (the caches hold whole tiles)
 #pragma unroll
     for (int c = 0; c < QC / 2; ++c) kf[c] = *reinterpret_cast<const u32x4_t*>(keys + (size_t)(k0 + col) * DQ + (2 * c + hf) * E);
 #pragma unroll
-    for (int i = 0; i < DV / 32; ++i) {
+    for (int i = 0; i < VB; ++i) {
       const int v = i * 32 + col;
-      const T* row = values + (size_t)(v < g.vdim ? v : 0) * g.cap + k0 + 4 * hf;
+      const T* row = values + (size_t)(v < v_left ? v : 0) * g.cap + k0 + 4 * hf;
 #pragma unroll
       for (int u = 0; u < NV; ++u) {
         if constexpr (BF) {
@@ -186,36 +189,67 @@ __global__ void __launch_bounds__(64 * NW) attention_split_kernel(SplitArgs a) {
   T* q_lo = q_hi + (size_t)live * Q_ROW;  // (bf16 only)
   T* k_new = q_hi + (size_t)live * Q_ROW * (BF ? 2 : 1);
   T* v_new = k_new + DQ;
-  for (int x = threadIdx.x; x < (live + (APPEND ? 1 : 0)) * (DQ / 2); x += 64 * NW) {
-    const int r = x / (DQ / 2), d = x % (DQ / 2) * 2, row = min(rb * 32 + r, r_last);
-    const bool query = r < live;
-    const float* head = g.qkv + (size_t)(row / per) * g.row + (size_t)(query ? kv * per + row % per : g.heads + kv) * g.dim;
-    float v[2];
-    turned<2>(head, d, g.dim, turn_of(g, g.pos + row / per, query), v);
-    T* to = query ? q_hi + r * Q_ROW + d : k_new + d;
-    to[0] = to_elem<T>(v[0]), to[1] = to_elem<T>(v[1]);
-    if constexpr (BF) {
-      if (query) {
-        q_lo[r * Q_ROW + d] = to_elem<T>(v[0] - bf16_to_f32(to[0]));
-        q_lo[r * Q_ROW + d + 1] = to_elem<T>(v[1] - bf16_to_f32(to[1]));
+  auto place_of = [&](int r, const float*& head, int& pos) {
+    const int row = APPEND ? r : min(rb * 32 + r, r_last), at = APPEND ? 0 : row / per, of = APPEND ? rb * 32 + r : row - at * per;
+    head = g.qkv + (size_t)at * g.row + (size_t)(r < live ? kv * per + of : g.heads + kv) * g.dim;
+    pos = g.pos + at;
+  };
+  if constexpr (VEC) {
+    constexpr int N = 8;
+    for (int x = threadIdx.x; x < (live + (APPEND ? 1 : 0)) * (DQ / N); x += 64 * NW) {
+      const int r = x / (DQ / N), d = x % (DQ / N) * N;
+      const float* head;
+      int pos;
+      place_of(r, head, pos);
+      float v[N];
+      turned<N, true>(head, d, g.dim, turn_of(g, pos, r < live), v);
+      T hi[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) hi[e] = to_elem<T>(v[e]);
+      __builtin_memcpy(__builtin_assume_aligned(r < live ? q_hi + r * Q_ROW + d : k_new + d, 16), hi, sizeof hi);
+      if constexpr (BF) {
+        if (r < live) {
+#pragma unroll
+          for (int e = 0; e < N; ++e) hi[e] = to_elem<T>(v[e] - bf16_to_f32(hi[e]));
+          __builtin_memcpy(__builtin_assume_aligned(q_lo + r * Q_ROW + d, 16), hi, sizeof hi);
+        }
+      }
+    }
+  } else {
+    for (int x = threadIdx.x; x < (live + (APPEND ? 1 : 0)) * (DQ / 2); x += 64 * NW) {
+      const int r = x / (DQ / 2), d = x % (DQ / 2) * 2;
+      const bool query = r < live;
+      const float* head;
+      int pos;
+      place_of(r, head, pos);
+      float v[2];
+      turned<2>(head, d, g.dim, turn_of(g, pos, query), v);
+      T* to = query ? q_hi + r * Q_ROW + d : k_new + d;
+      to[0] = to_elem<T>(v[0]), to[1] = to_elem<T>(v[1]);
+      if constexpr (BF) {
+        if (query) {
+          q_lo[r * Q_ROW + d] = to_elem<T>(v[0] - bf16_to_f32(to[0]));
+          q_lo[r * Q_ROW + d + 1] = to_elem<T>(v[1] - bf16_to_f32(to[1]));
+        }
       }
     }
   }
-  if constexpr (APPEND)
-    for (int v = threadIdx.x; v < DV; v += 64 * NW) v_new[v] = to_elem<T>(v < g.vdim ? g.qkv[(size_t)(g.heads + g.kv_heads) * g.dim + (size_t)kv * g.vdim + v] : 0.f);
+  if constexpr (APPEND)  // (the last threads: the first ones have the queries)
+    if (const int v = 64 * NW - 1 - (int)threadIdx.x; v < W) v_new[v] = to_elem<T>(v < v_left ? g.qkv[(size_t)(g.heads + g.kv_heads) * g.dim + (size_t)kv * g.vdim + v0 + v] : 0.f);
   __syncthreads();
   const int q_at = (r_mine - rb * 32) * Q_ROW + hf * E;  // chunk 2 c + hf of row `col`: 2 c E further
   if constexpr (APPEND) {
     // the workgroup that meets the new key leaves it in the caches
     if ((tile0 + split * share) * SK <= g.pos && g.pos < k_stop) {
       T* krow = static_cast<T*>(g.kc) + ((size_t)kv * g.cap + g.pos) * DQ;
-      for (int x = threadIdx.x; x < QC; x += 64 * NW) *reinterpret_cast<u32x4_t*>(krow + x * E) = *reinterpret_cast<const u32x4_t*>(k_new + x * E);
-      for (int v = threadIdx.x; v < g.vdim; v += 64 * NW) static_cast<T*>(g.vc)[((size_t)kv * g.vdim + v) * g.cap + g.pos] = v_new[v];
+      if (v0 == 0)
+        for (int x = threadIdx.x; x < QC; x += 64 * NW) *reinterpret_cast<u32x4_t*>(krow + x * E) = *reinterpret_cast<const u32x4_t*>(k_new + x * E);
+      if (const int v = 64 * NW - 1 - (int)threadIdx.x; v < W && v < v_left) static_cast<T*>(g.vc)[((size_t)kv * g.vdim + v0 + v) * g.cap + g.pos] = v_new[v];
     }
   }
-  f32x16 o[DV / 32];
+  f32x16 o[VB];
 #pragma unroll
-  for (int i = 0; i < DV / 32; ++i)
+  for (int i = 0; i < VB; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
   float mx = -INFINITY, sum = 0.f;
@@ -229,24 +263,26 @@ __global__ void __launch_bounds__(64 * NW) attention_split_kernel(SplitArgs a) {
           kf[c] = mine ? piece : kf[c];
         }
 #pragma unroll
-        for (int i = 0; i < DV / 32; ++i) {
+        for (int i = 0; i < VB; ++i) {
           const T now = v_new[i * 32 + col];
 #pragma unroll
-          for (int u = 0; u < NV; ++u) {
-            T e[E];
-            __builtin_memcpy(e, &vf[i][u], 16);
+          for (int u = 0; u < NV; ++u)
 #pragma unroll
-            for (int x = 0; x < E; ++x) {
-              const int p = k0 + (BF ? 16 * u + 8 * (x >> 2) : 8 * u) + 4 * hf + (x & 3);
-              e[x] = p < g.pos ? e[x] : p == g.pos ? now : T(0);
+            for (int w = 0; w < 4; ++w) {
+              // the word's first position; what it keeps of the cache and where the new value goes
+              const int p = k0 + (BF ? 16 * u + 8 * (w >> 1) + 2 * (w & 1) : 8 * u + w) + 4 * hf;
+              if constexpr (BF) {
+                const unsigned kept = (p < g.pos ? 0xffffu : 0) | (p + 1 < g.pos ? 0xffff0000u : 0), here = p == g.pos ? (unsigned)now : p + 1 == g.pos ? (unsigned)now << 16 : 0u;
+                vf[i][u][w] = (vf[i][u][w] & kept) | here;
+              } else {
+                vf[i][u][w] = p < g.pos ? vf[i][u][w] : p == g.pos ? __builtin_bit_cast(unsigned, now) : 0u;
+              }
             }
-            __builtin_memcpy(&vf[i][u], e, 16);
-          }
         }
       }
     } else if (k0 + SK > s_all) {  // places past the last position were never written
 #pragma unroll
-      for (int i = 0; i < DV / 32; ++i)
+      for (int i = 0; i < VB; ++i)
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
           T e[E];
@@ -284,7 +320,7 @@ __global__ void __launch_bounds__(64 * NW) attention_split_kernel(SplitArgs a) {
     }
     sum = sum * alpha + part + __shfl_xor(part, 32, 64);
 #pragma unroll
-    for (int i = 0; i < DV / 32; ++i)
+    for (int i = 0; i < VB; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
 #pragma unroll
@@ -297,13 +333,13 @@ __global__ void __launch_bounds__(64 * NW) attention_split_kernel(SplitArgs a) {
           lo[e] = (__bf16)(s[8 * u + e] - (float)hi[e]);
         }
 #pragma unroll
-        for (int i = 0; i < DV / 32; ++i) {
+        for (int i = 0; i < VB; ++i) {
           o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[i][u]), hi, o[i], 0, 0, 0);
           o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[i][u]), lo, o[i], 0, 0, 0);
         }
       } else {
 #pragma unroll
-        for (int i = 0; i < DV / 32; ++i) {
+        for (int i = 0; i < VB; ++i) {
           const f32x4_t v = __builtin_bit_cast(f32x4_t, vf[i][u]);
 #pragma unroll
           for (int x = 0; x < 4; ++x) o[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[x], s[4 * u + x], o[i], 0, 0, 0);
@@ -312,21 +348,22 @@ __global__ void __launch_bounds__(64 * NW) attention_split_kernel(SplitArgs a) {
     }
     if (k0 + NW * SK < k_stop) fetch(k0 + NW * SK);
   }
-  // the waves' parts: [wave][row][DV + 4], then every wave's maximum and sum per row
+  // the waves' parts: [wave][row][W + 4], then every wave's maximum and sum per row
   __syncthreads();  // (what was staged there has been read)
-  constexpr int P = DV + 4;
+  constexpr int P = W + 4;
   float* ml = parts + (size_t)NW * live * P;
   if (col < live) {
     float* mine = parts + ((size_t)wave * live + col) * P;
 #pragma unroll
-    for (int i = 0; i < DV / 32; ++i)
+    for (int i = 0; i < VB; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) *reinterpret_cast<f32x4_t*>(mine + i * 32 + 8 * q + 4 * hf) = f32x4_t{o[i][4 * q], o[i][4 * q + 1], o[i][4 * q + 2], o[i][4 * q + 3]};
     if (hf == 0) ml[(wave * live + col) * 2] = mx, ml[(wave * live + col) * 2 + 1] = sum;
   }
   __syncthreads();
-  for (int x = threadIdx.x; x < live * g.vdim; x += 64 * NW) {
-    const int r = x / g.vdim, v = x - r * g.vdim, row = rb * 32 + r;
+  for (int x = threadIdx.x; x < live * W; x += 64 * NW) {
+    const int r = x / W, v = x % W, row = rb * 32 + r;
+    if (v >= v_left) continue;
     float m[NW], top = -INFINITY;
 #pragma unroll
     for (int w = 0; w < NW; ++w) top = fmaxf(top, m[w] = ml[(w * live + r) * 2]);
@@ -339,13 +376,14 @@ __global__ void __launch_bounds__(64 * NW) attention_split_kernel(SplitArgs a) {
       val += f * parts[((size_t)w * live + r) * P + v];
     }
     if (a.splits == 1) {
-      const size_t at = (size_t)(row / per) * a.dst_stride + (size_t)(kv * per + row % per) * g.vdim + v;
+      const int pos = APPEND ? 0 : row / per;
+      const size_t at = (size_t)pos * a.dst_stride + (size_t)(kv * per + row - pos * per) * g.vdim + v0 + v;
       if (a.dst_bf16) static_cast<uint16_t*>(a.dst)[at] = bf16_rne(val / l);
       else static_cast<float*>(a.dst)[at] = val / l;
     } else {
       const size_t at = (size_t)split * g.kv_heads * a.rows + (size_t)kv * a.rows + row;
-      a.acc[at * g.vdim + v] = val;
-      if (v == 0) a.ml[at * 2] = top, a.ml[at * 2 + 1] = l;
+      a.acc[at * g.vdim + v0 + v] = val;
+      if (v0 + v == 0) a.ml[at * 2] = top, a.ml[at * 2 + 1] = l;
     }
   }
 }
@@ -399,15 +437,16 @@ int with_sizes(const Built& b, F&& f) {
   return f(integral_constant<int, 256>{}, integral_constant<int, 256>{});
 }
 
+// Whether the projected rows can be read (and turned) eight elements at a time: the VEC of the kernels.
+bool pieces_of_eight(const GroupedArgs& g) { return g.dim % 8 == 0 && g.rot % 8 == 0 && g.row % 4 == 0 && (reinterpret_cast<uintptr_t>(g.qkv) & 15) == 0; }
+
 template <typename T, int DQ>
 int place(ughip_device* dev, const GroupedArgs& g) {
   const size_t pieces = (size_t)(g.q_rows > g.t ? g.q_rows : g.t) * (DQ * sizeof(T) / 16), tiles = ((size_t)g.t + VT - 1) / VT;
   const size_t x = (pieces + 255) / 256 > tiles ? (pieces + 255) / 256 : tiles;
   const int y = (g.q_rows ? g.heads : 0) + g.kv_heads + g.kv_heads * ((g.vdim + VT - 1) / VT);
   if (y > 65535) return set_error(UGHIP_ERR_UNSUPPORTED, "grouped_attention: too many heads");
-  auto whole = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-  const bool vec = g.dim % 8 == 0 && g.rot % 8 == 0 && g.row % 4 == 0 && whole(g.qkv);
-  if (vec) attention_place_kernel<T, DQ, true><<<dim3((unsigned)x, (unsigned)y), 256, 0, dev->stream>>>(g);
+  if (pieces_of_eight(g)) attention_place_kernel<T, DQ, true><<<dim3((unsigned)x, (unsigned)y), 256, 0, dev->stream>>>(g);
   else attention_place_kernel<T, DQ, false><<<dim3((unsigned)x, (unsigned)y), 256, 0, dev->stream>>>(g);
   UGHIP_HIPCHK(hipGetLastError());
   return UGHIP_OK;
@@ -434,7 +473,8 @@ int attend_few(ughip_device* dev, SplitArgs a) {
   const GroupedArgs& g = a.g;
   if (g.t > 1)
     if (int rc = place<T, DQ>(dev, g)) return rc;
-  a.rows = g.t * (g.heads / g.kv_heads), a.row_blocks = (a.rows + 31) / 32;
+  a.per = g.heads / g.kv_heads;
+  a.rows = g.t * a.per, a.row_blocks = (a.rows + 31) / 32;
   const int groups = g.kv_heads * a.row_blocks;
   int seen = g.pos + g.t;
   if (a.window && seen > a.window + g.t - 1) seen = a.window + g.t - 1;
@@ -451,16 +491,24 @@ int attend_few(ughip_device* dev, SplitArgs a) {
     if (int rc = rows_scratch(dev, (n_ml + rows * g.vdim) * sizeof(float), &ws)) return rc;
     a.ml = static_cast<float*>(ws), a.acc = a.ml + n_ml;
   }
+  // One position: the values over several workgroups while the chip has CUs for them.  (Few key heads and short caches leave it empty, and a
+  // CU reads no more than 60 bytes per ns: 8 heads on 2, us behind 100 / 160 / 220 positions 8.6 / 10.2 / 10.7 -> 6.3 / 6.7 / 6.9.)
+  const int across = g.t == 1 && groups * splits * (DV / 32) <= dev->num_cus ? DV / 32 : 1;
   const int live = a.rows < 32 ? a.rows : 32;
-  const size_t staged = ((size_t)live * (DQ + 16 / sizeof(T)) * (sizeof(T) == 2 ? 2 : 1) + DQ + DV) * sizeof(T), met = (size_t)NW * live * (DV + 4 + 2) * sizeof(float);
+  const size_t staged = ((size_t)live * (DQ + 16 / sizeof(T)) * (sizeof(T) == 2 ? 2 : 1) + DQ + DV) * sizeof(T), met = (size_t)NW * live * (DV / across + 4 + 2) * sizeof(float);
   const size_t lds = staged > met ? staged : met;
   auto go = [&](auto kernel) {
     if (lds > 60 * 1024)
       if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); e != hipSuccess) return e;
-    kernel<<<dim3((unsigned)groups, (unsigned)splits), 64 * NW, lds, dev->stream>>>(a);
+    kernel<<<dim3((unsigned)g.kv_heads, (unsigned)splits, (unsigned)(a.row_blocks * across)), 64 * NW, lds, dev->stream>>>(a);
     return hipGetLastError();
   };
-  UGHIP_HIPCHK(g.t == 1 ? go(attention_split_kernel<T, DQ, DV, NW, true>) : go(attention_split_kernel<T, DQ, DV, NW, false>));
+  auto with_vec = [&](auto v) {
+    constexpr bool VEC = decltype(v)::value;
+    if (g.t > 1) return go(attention_split_kernel<T, DQ, DV, NW, false, VEC, DV>);
+    return across > 1 ? go(attention_split_kernel<T, DQ, DV, NW, true, VEC, 32>) : go(attention_split_kernel<T, DQ, DV, NW, true, VEC, DV>);
+  };
+  UGHIP_HIPCHK(pieces_of_eight(g) ? with_vec(std::true_type()) : with_vec(std::false_type()));
   if (splits > 1) {
     attention_merge_kernel<<<(unsigned)(g.kv_heads * a.rows), 256, 0, dev->stream>>>(a);
     UGHIP_HIPCHK(hipGetLastError());
