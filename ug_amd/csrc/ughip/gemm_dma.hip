@@ -1,6 +1,6 @@
 // 16-bit MFMA GEMM for gfx950 with one wave per SIMD: C[b] = A[b] x B[b], f32 accumulate, bf16 or f16.
 //
-//   block tile BM x BN (256 x 256, 256 x 128 or 128 x 128), K tile 64, 4 waves laid out 2 x 2, each owning BM/2 x BN/2 of the result
+//   block tile BM x BN (256 x 256, 256 x 192, 256 x 128 or 128 x 128), K tile 64, 4 waves laid out 2 x 2, each owning BM/2 x BN/2 of the result
 //   (any M, N a multiple of 8: a last tile hangs over the end, reads the last row again and stores what exists):
 //   (BM / 32) x (BN / 32) accumulators of 16 x 16 (v_mfma_f32_16x16x32: 4 registers each) live in the accumulation
 //   registers -- all 256 of them for the largest tile, which a lone wave per SIMD can have -- and leave the
@@ -60,6 +60,7 @@ template <typename T, int BM, int BN, bool B_KN, bool TWO, bool F32OUT = false, 
 __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tiles_n, const float* __restrict__ residual, DmaRows rw) {
   static_assert(ROWS == 0 || (BDIV == 1 && !B_KN && !F32OUT), "rows: one plane against an [n, k]-major rhs");
   static_assert(BDIV == 1 || BDIV == 6 || !B_KN, "planes of the lhs alone: against an [n, k]-major rhs only");
+  static_assert(BN != 192 || (!B_KN && F32OUT), "192 columns: neither the swizzle of an n-contiguous tile nor the way out through LDS divides them");
   extern __shared__ u32x4 lds[];
   constexpr int NI = BM / 32, NJ = BN / 32;            // 16-row and 16-column fragments per wave
   constexpr int NM = NI * NJ;                          // MFMAs per k32 step
@@ -432,10 +433,11 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 }  // namespace
 
 namespace {
-// tile codes of the entry points below: 256 = 256 x 256, 128 = 256 x 128, 64 = 128 x 128; on gemm_ring 129 = 256 x 128, 65 = 128 x 128, 48 = 64 x 128,
+// tile codes of the entry points below: 256 = 256 x 256, 192 = 256 x 192 (three planes only), 128 = 256 x 128, 64 = 128 x 128; on gemm_ring 129 = 256 x 128, 65 = 128 x 128, 48 = 64 x 128,
 // 32 = 64 x 64 ([n, k]-major rhs only), 97 = 192 x 192 (rows only)
 bool tile_dims(int tile, int* bm, int* bn) {
   if (tile == 256) *bm = 256, *bn = 256;
+  else if (tile == 192) *bm = 256, *bn = 192;
   else if (tile == 128 || tile == 129) *bm = 256, *bn = 128;
   else if (tile == 97) *bm = 192, *bn = 192;
   else if (tile == 64 || tile == 65) *bm = 128, *bn = 128;
@@ -464,6 +466,7 @@ int gemm_dma_forced_tile(long long shape) {
     case 11: return 97;
     case 12: return 65;
     case 13: return 48;
+    case 14: return 192;
   }
   return 0;
 }
@@ -475,7 +478,7 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || batch == 0) return false;
   if (p.a_cs != 1 || p.a_rs % 8 || (batch > 1 && (p.a_bs % 8 || p.b_bs % 8 || p.c_bs % 8))) return false;
   const bool nn = p.b_cs == 1 && p.b_rs != 1, nt = p.b_rs == 1 && p.b_cs != 1;
-  if (nn == nt || (nn && tile == 32) || tile == 97) return false;
+  if (nn == nt || (nn && tile == 32) || tile == 97 || (tile == 192 && p.b_k_div != 3)) return false;
   const long long ldb = nn ? p.b_rs : p.b_cs;
   if (ldb % 8) return false;
   // per-lane offsets are 32-bit: the furthest row of a tile has to stay below 4 GiB from the tile's first byte
@@ -513,6 +516,9 @@ static double ring_cost_us(size_t tiles, int kt, int tile, Operands from) {
 // (3072 x 4096^2: 131 -> 91 us, 5120^2 x 1024: 77 -> 54, 1280 x 8192 x 2048: 64 -> 47, 2048 x 2560 x 2048: 35 -> 29,
 // 2304^3: 39 -> 35) and leaves those with about 128 tiles where they were (2048^2 x 5632: 56 us against 72).  The
 // 128 x 128 tile (two workgroups per CU) takes what neither fits: 2304^3 35 -> 31 us, 2048 x 2560 x 2048 29 -> 27.
+// 256 x 192, for three planes: what leaves 256 x 256 tiles a round and a half or a split.  Gate and up of a llama layer (k 2048, n 2 x 5632, with
+// the fold), us at 384 / 512 / 700 / 1024 / 1500 / 1900 / 2048 rows: 92 / 82 / 131 / 140 / 234 / 254 / 255 -> 76 / 74 / 116 / 126 / 205 / 238 / 240; k 1024, n 2 x 2816: 1500
+// 87 -> 68, 1900 92 -> 74; q | k | v of 1900 rows 80 -> 74 in two splits.  One plane of rows gains nothing (2048 x 11264 x 2048 from memory 97.6, 96.2 so).
 // UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 10 / 12 / 13 / 9 the ring's 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64, 0..2, 6 and 7 keep both out (tuning aid).
 double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
   const size_t tiles = tile_count(p, batch, tile);
@@ -530,11 +536,13 @@ double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
     // 0.47 + 0.16 x busy, the next 256 fill the second slots (2048^3 24.7 us, 2304^3 31.3, 2816^3 45.5, 5120^2 x 1024 61)
     us += kt * 0.88 * (double)(tiles / 512) * layout;
     const size_t left = tiles % 512;
-    if (left > 256) us += kt * (0.63 + 0.25 * (double)(left - 256) / 256.0) * layout;
+    // (unsplit planes take as long with a few second slots filled as with most: 1900 x 2560 x 2048, 300 tiles, 78 us; 600 x 11264 x 2048, 440, 80)
+    if (left > 256) us += kt * (p.b_k_div == 3 && batch == 1 ? 0.82 : 0.63 + 0.25 * (double)(left - 256) / 256.0) * layout;
     else if (left) us += kt * (0.47 + 0.16 * (double)left / 256.0) * layout;
     return us;
   }
-  const double t0 = tile == 256 ? 0.9 : 0.62, t1 = tile == 256 ? 0.6 : 0.2;
+  // (256 x 128 with unsplit planes: 1900 x 2560 x 2048 81.5 us, and 74.5 in two splits of 256 x 192)
+  const double t0 = tile == 256 ? 0.9 : tile == 192 ? 0.76 : p.b_k_div == 3 && batch == 1 ? 0.68 : 0.62, t1 = tile == 256 ? 0.6 : tile == 192 ? 0.4 : 0.2;
   for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) {
     const double busy = (left < 256 ? (double)left : 256.0) / 256.0;
     us += kt * (t0 + t1 * busy) * layout;
@@ -638,6 +646,7 @@ hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile
   note_kernel("%s", name);
   if (ring_tile(tile)) return gemm_ring_launch(stream, UGHIP_BF16, DmaForm::PLANES3, q, (size_t)nsplit, tile, residual, DmaRows());
   if (tile == 256) return launch<__bf16, 256, 256, false, true, 3>(stream, q, (size_t)nsplit, residual);
+  if (tile == 192) return launch<__bf16, 256, 192, false, true, 3>(stream, q, (size_t)nsplit, residual);
   if (tile == 128) return launch<__bf16, 256, 128, false, true, 3>(stream, q, (size_t)nsplit, residual);
   return launch<__bf16, 128, 128, false, true, 3>(stream, q, (size_t)nsplit, residual);
 }

@@ -81,7 +81,7 @@ enum TuneKey {
   TUNE_GEMV_KS,             // waves per output column of the GEMV family: 1, 2 or 4
   TUNE_GEMV_ROWS,           // rows per workgroup of fused_gemv_bf16_rows: 1, 2, 4 or 8
   TUNE_GEMV_BF16_ROWS,      // 0: bf16 matrices take the f32 kernels' lane layout
-  TUNE_X3_DMA,              // three-term bf16 products: 0 keeps gemm_tiled; 3 / 4 / 5, 12 / 13 / 9 force the tile that GEMM_SHAPE names so; others: as if not set
+  TUNE_X3_DMA,              // three-term bf16 products: 0 keeps gemm_tiled; 3 / 4 / 5, 12 / 13 / 9 force the tile that GEMM_SHAPE names so, 14 gemm_dma4's 256x192; others: as if not set
   TUNE_X3_SPLIT,            // K split of the three-term product on gemm_dma4
   TUNE_X3_ROWS,             // three-term bf16 products of 65 .. 128 rows: 0 keeps the kernels that take planes, n > 0 forces n units per workgroup of rows_x3
   TUNE_ATT_SPLIT,           // key ranges per head of single-query attention

@@ -776,7 +776,7 @@ static RowsRoute rows_route(const MMArgs& p, int dtype, bool x3, GemmEpilogue::K
   // more).  Its result leaves as f32 with the residual added on the way; SwiGLU goes through the scratch block and the fold.
   // (from 384 rows: at 128 and 256 rows the register-staged kernel is as fast or faster for four of the five products of a
   // llama step -- q|k|v 25.2 us against 28.6 at 256 rows -- and the model below does not see that; at 512 rows this kernel is)
-  long long x3_dma = -1, x3_split = 0;  // tuning aids: X3_DMA 0 keeps the register-staged kernel, 3, 4, 5, 9, 12 and 13 force a tile as GEMM_SHAPE does; X3_SPLIT n a K split
+  long long x3_dma = -1, x3_split = 0;  // tuning aids: X3_DMA 0 keeps the register-staged kernel, 3, 4, 5, 9, 12, 13 and 14 force a tile as GEMM_SHAPE does; X3_SPLIT n a K split
   tune_get(TUNE_X3_DMA, &x3_dma);
   tune_get(TUNE_X3_SPLIT, &x3_split);
   if (x3 && m >= 384 && x3_dma != 0) {
@@ -785,7 +785,7 @@ static RowsRoute rows_route(const MMArgs& p, int dtype, bool x3, GemmEpilogue::K
     double best = 0;
     const int named = x3_dma > 0 ? gemm_dma_forced_tile(x3_dma) : 0, forced_tile = named == 129 || named == 97 ? 0 : named;
     const int forced_split = (int)x3_split;
-    for (int tile : {256, 128, 65, 64, 48, 32}) {  // (codes 65, 48, 32: gemm_ring; 1900 x 2048 x 2048 64 -> 54 us, 512 x 2048 x 2048 32 -> 26)
+    for (int tile : {256, 128, 65, 64, 48, 32, 192}) {  // (codes 65, 48, 32: gemm_ring; 1900 x 2048 x 2048 64 -> 54 us, 512 x 2048 x 2048 32 -> 26)
       if (forced_tile && tile != forced_tile) continue;
       for (int split : {1, 2, 4, 8}) {
         if (forced_split && split != forced_split) continue;
