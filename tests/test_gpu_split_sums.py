@@ -1,0 +1,37 @@
+"""Products of any size whose K several workgroups share, and the rules for the larger tile: what each plan leaves, against the bound of an f32 sum."""
+import numpy as np
+import pytest
+
+import test_gpu_products as products
+import test_zz_no_alloc as no_alloc
+import ug_amd
+
+pytestmark = pytest.mark.gpu
+
+
+# the fewest steps of K that are split, a whole last step and one element of one, uneven slabs, a tile over the edge, slabs of 1, 2 and 3 elements behind the last four,
+# as many slabs as there may be, tiles times slabs on either side of a round of the chip; a product in a batch
+@pytest.mark.parametrize("bmnk", [(1, 9, 9, 1600), (1, 9, 9, 1601), (1, 65, 67, 1407), (1, 21, 11, 4096), (1, 63, 65, 3000), (3, 70, 9, 2050), (1, 705, 700, 2001), (1, 500, 1001, 2001)])
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
+@pytest.mark.parametrize("lhs_mk", [True, False], ids=["rows", "transposed"])
+def test_split_sums(hip, bmnk, dtype, rhs_nk, lhs_mk):
+    products.test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk)
+    if bmnk[1] < 100 and bmnk[3] % 64:
+        assert ",splitK=" in ug_amd.last_kernel(), ug_amd.last_kernel()
+
+
+# 16 bits, fewer than 256 large tiles: four small ones and three to a CU, on both sides of the sums that pay for the large one
+@pytest.mark.parametrize("bmnk, large", [((1, 1729, 1729, 257), True), ((1, 1729, 1729, 255), False), ((1, 1601, 1601, 1537), True), ((1, 1601, 1601, 1535), False)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_three_and_four_tiles_to_a_cu(hip, bmnk, large, dtype):
+    products.test_products_of_any_size(hip, bmnk, dtype, True, True)
+    assert ug_amd.last_kernel() == f"gemm_any<{dtype}{',128x128' if large else ''}>"
+
+
+@pytest.mark.parametrize("dtype", [ug_amd.F32, ug_amd.BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("bmnk", [(1, 70, 65, 3001), (2, 33, 9, 2047)])
+def test_the_call_that_may_not_allocate(hip, dtype, bmnk):
+    ref, got, kernel = no_alloc._both(hip, dtype, bmnk, True, 91)
+    assert ",splitK=" in kernel
+    np.testing.assert_array_equal(got, ref)

@@ -99,10 +99,15 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act);  // a ti
 hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRows& r, RowsAct act, int tile);
 
 // Any M, N, K and any alignment (gemm_ragged.hip; f32, f16, bf16): operands contiguous along k or along their other dimension, at least eight
-// elements from one k to the next in the latter case.  Contiguous [batch, M, N] result.  The tile it takes a product with, 64 or 128; 0: the
-// kernels that go by element should.
-int gemm_ragged_tile(int dtype, const MMArgs& p, size_t batch);
-hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, int tile);
+// elements from one k to the next in the latter case.  Contiguous [batch, M, N] result.  The plan it takes a product with; tile 0: the kernels
+// that go by element should.
+struct RaggedPlan {
+  int tile = 0, nsplit = 1;  // 64 or 128; nsplit > 1: workgroups share a tile's K and leave slabs in the workspace, which a second launch adds up
+  size_t ws_bytes = 0;
+  static constexpr size_t MAX_WS = (size_t)32 << 20;
+};
+RaggedPlan gemm_ragged_plan(int dtype, const MMArgs& p, size_t batch);
+hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, const RaggedPlan& plan, float* workspace);
 
 // f32, one wave per SIMD: 256 x 128 tiles of v_mfma_f32_32x32x2_f32, loads that write LDS directly, rhs [n, k]- or [k, n]-major
 // (gemm_dma_f32.hip).  Any M, N % 4 == 0, K % 32 == 0 and K >= 64, 16-byte aligned rows, contiguous [batch, M, N] result.

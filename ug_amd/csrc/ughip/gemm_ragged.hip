@@ -8,9 +8,10 @@
 //   what does not exist, and comes first, under the way of the next ones: it holds the only row of a
 //   [k, n]-major operand behind which nothing may be read.
 //
-// What bounds it: the steps' latency on few tiles (0.4 us each in 16 bits, 0.6 in f32), LDS and the f32 matrix pipe on many.  Against element-by-element
+// What bounds it: the steps of K on few tiles (0.3 us each in 16 bits, 0.6 in f32, the f32 matrix pipe two thirds of that; deeper prefetch changes nothing), LDS and the f32
+// matrix pipe on many.  Against element-by-element
 // loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 14.6 us, f32 256 -> 34; 2001^3 f16 270 -> 37, f32 340 -> 135; 3999^2 x
-// 2000 f16 1204 -> 103, f32 1014 -> 520; 100^3 9.4 -> 5.4.  Which tile takes what: gemm_ragged_tile.
+// 2000 f16 1204 -> 103, f32 1014 -> 520; 100^3 9.4 -> 5.4.  Which tile takes what and where K is split: gemm_ragged_plan.
 #include <hip/hip_runtime.h>
 
 #include "gemm.h"
@@ -118,8 +119,14 @@ struct Side {
   }
 };
 
-template <typename T, int BT, bool A_KC, bool B_KC>
-__global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int tiles_m, int tiles_n) {
+template <typename T, bool SPLIT>
+struct Result { typedef T type; };
+template <typename T>
+struct Result<T, true> { typedef float type; };
+
+// SPLIT: slab s of nsplit has the steps per * s .. per * (s + 1) - 1 of K, the last one the remainder, and leaves its sums in ws, slab_elems apart.
+template <typename T, int BT, bool A_KC, bool B_KC, bool SPLIT>
+__global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int tiles_m, int tiles_n, int nsplit, int per, float* __restrict__ ws, size_t slab_elems) {
   typedef Side<T, BT, A_KC> SA;
   typedef Side<T, BT, B_KC> SB;
   constexpr int MI = BT / 64, KE = SA::KE;
@@ -127,14 +134,20 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // each XCD a contiguous run of all products' tiles (block ids go round-robin over the 8): with the runs dealt product by product a batch
   // of products of one tile would be one XCD's work (300 of 33 x 17 x 129 in f32: 32 us that way, 8.9 so, 16 in the kernel by element)
-  const int tpb = tiles_m * tiles_n, tiles = batches * tpb, per = (tiles + 7) >> 3, bid = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  const int tpb = tiles_m * tiles_n, tiles = batches * tpb * (SPLIT ? nsplit : 1), run = (tiles + 7) >> 3;
+  int bid = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
   if (bid >= tiles) return;
+  const int slab = SPLIT ? bid / (batches * tpb) : 0;  // (slab by slab: tiles of one slab that share rows are neighbours)
+  if (SPLIT) bid -= slab * batches * tpb;
   const int batch = bid / tpb, in_batch = bid - batch * tpb, tm = in_batch / tiles_n, tn = in_batch - tm * tiles_n, m0 = tm * BT, n0 = tn * BT;
   SA a;
   SB b;
   a.place(static_cast<const T*>(p.a) + (size_t)batch * p.a_bs, m0, p.M, p.a_rs, p.a_cs, tid);
   b.place(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs, n0, p.N, p.b_cs, p.b_rs, tid);
   const int full = (p.K - 1) / KE, left = p.K - full * KE;  // whole steps, and 1 .. KE elements of k behind them
+  // the steps behind the first one: that is K's remainder, or in front of the last slab the slab's first
+  const bool with_left = !SPLIT || slab == nsplit - 1;
+  const int begin = SPLIT ? slab * per + (with_left ? 0 : 1) : 0, end = with_left ? full : (slab + 1) * per;
   f32x16 acc[MI][MI];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -169,32 +182,40 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
         for (int j = 0; j < MI; ++j) mma(T(), fb[j], fa[i], acc[i][j]);  // swapped: a lane holds columns of one row
     }
   };
+  if (with_left) {
 #pragma unroll
-  for (int i = 0; i < SA::N; ++i) la[i] = a.load_last(i, full, left, m0, p.M, tid);
+    for (int i = 0; i < SA::N; ++i) la[i] = a.load_last(i, full, left, m0, p.M, tid);
 #pragma unroll
-  for (int i = 0; i < SB::N; ++i) lb[i] = b.load_last(i, full, left, n0, p.N, tid);
-  if (full > 0) {
-    fetch(0, 0);
-    fetch(1, min(1, full - 1));
+    for (int i = 0; i < SB::N; ++i) lb[i] = b.load_last(i, full, left, n0, p.N, tid);
+  } else {
+#pragma unroll
+    for (int i = 0; i < SA::N; ++i) la[i] = a.load(i, begin - 1);
+#pragma unroll
+    for (int i = 0; i < SB::N; ++i) lb[i] = b.load(i, begin - 1);
+  }
+  if (end > begin) {
+    fetch(0, begin);
+    fetch(1, min(begin + 1, end - 1));
   }
   put(lds[0], la, lb);
   __syncthreads();
   multiply(lds[0]);
-  for (int s0 = 0; s0 < full; s0 += 2) {
+  for (int s0 = begin; s0 < end; s0 += 2) {
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
       const int s = s0 + d;
-      if (s >= full) break;
+      if (s >= end) break;
       char* buf = lds[d ^ 1];
       put(buf, ra[d], rb[d]);
-      fetch(d, min(s + 2, full - 1));  // (without a branch, so that a step's loads can be waited for alone)
+      fetch(d, min(s + 2, end - 1));  // (without a branch, so that a step's loads can be waited for alone)
       __syncthreads();                 // one barrier a step: the buffer written next was read before it
       multiply(buf);
     }
   }
 
   // element e of lane l of block (i, j): row l % 32, column 8 (e / 4) + 4 (l / 32) + e % 4
-  T* __restrict__ C = static_cast<T*>(p.c) + (size_t)batch * p.c_bs;
+  typedef typename Result<T, SPLIT>::type R;
+  R* __restrict__ C = (SPLIT ? reinterpret_cast<R*>(ws + slab * slab_elems) : static_cast<R*>(p.c)) + (size_t)batch * p.c_bs;
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int row = m0 + wm + 32 * i + (lane & 31);
@@ -204,28 +225,51 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int col = n0 + wn + 32 * j + 8 * g + 4 * (lane >> 5);
-        T* q = C + (size_t)row * p.N + col;
+        R* q = C + (size_t)row * p.N + col;
         if (col + 4 <= p.N) {
           store4(q, f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]});
         } else {
 #pragma unroll
           for (int e = 0; e < 3; ++e)
-            if (col + e < p.N) q[e] = (T)acc[i][j][4 * g + e];
+            if (col + e < p.N) q[e] = (R)acc[i][j][4 * g + e];
         }
       }
   }
 }
 
-template <typename T, int BT>
-hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch) {
-  const int tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BT - 1) / BT;
-  const unsigned grid = (unsigned)((batch * tiles_m * tiles_n + 7) / 8 * 8);
+// c = the slabs' sum, in their order
+template <typename T>
+__global__ void __launch_bounds__(256) gemm_ragged_fold(const float* __restrict__ ws, T* __restrict__ c, size_t elems, size_t slab_elems, int nsplit) {
+  const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (at >= elems) return;
+  f32x4 s = *reinterpret_cast<const f32x4*>(ws + at);
+  for (int k = 1; k < nsplit; ++k) s += *reinterpret_cast<const f32x4*>(ws + k * slab_elems + at);
+  if (at + 4 <= elems) {
+    store4(c + at, s);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (at + e < elems) c[at + e] = (T)s[e];
+  }
+}
+
+template <typename T, int BT, bool SPLIT>
+hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, int nsplit, float* ws) {
+  const int tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BT - 1) / BT, ke = 128 / (int)sizeof(T), steps = (p.K + ke - 1) / ke, per = (steps + nsplit - 1) / nsplit;
+  const unsigned grid = (unsigned)((batch * tiles_m * tiles_n * nsplit + 7) / 8 * 8);
+  const size_t elems = batch * p.M * p.N, slab = (elems + 3) / 4 * 4;
   const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
-  if (ak && bk) gemm_ragged<T, BT, true, true><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n);
-  else if (ak) gemm_ragged<T, BT, true, false><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n);
-  else if (bk) gemm_ragged<T, BT, false, true><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n);
-  else gemm_ragged<T, BT, false, false><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n);
+  if (ak && bk) gemm_ragged<T, BT, true, true, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  else if (ak) gemm_ragged<T, BT, true, false, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  else if (bk) gemm_ragged<T, BT, false, true, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  else gemm_ragged<T, BT, false, false, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  if (SPLIT) gemm_ragged_fold<T><<<(unsigned)((elems + 1023) / 1024), 256, 0, stream>>>(ws, static_cast<T*>(p.c), elems, slab, nsplit);
   return hipGetLastError();
+}
+template <typename T>
+hipError_t launch_plan(hipStream_t stream, const MMArgs& p, size_t batch, const RaggedPlan& pl, float* ws) {
+  if (pl.nsplit > 1) return launch<T, 64, true>(stream, p, batch, pl.nsplit, ws);
+  return pl.tile == 128 ? launch<T, 128, false>(stream, p, batch, 1, nullptr) : launch<T, 64, false>(stream, p, batch, 1, nullptr);
 }
 
 }  // namespace
@@ -245,19 +289,53 @@ static bool supported(const MMArgs& p, size_t batch) {
 //   16 bits: the large tile's prologue wants more than one step to pay for it, or a last round that is nearly full: 2001^2 x 8 8.3 / 7.7 / 8.3, x 33 10.0 / 9.0 / 8.5, x 127
 //   18.1 / 14.3 / 11.9, x 1001 141 / 31.2 / 23.5, 3187 x 2088 x 64 16.3 small, 14.5 large, 7 x 512 x 1219 x 63 19.6 / 13.1 / 15.4, x 129 37.8 / 13.1 / 15.0, x 1001 283 /
 //   37.5 / 35.0.
-int gemm_ragged_tile(int dtype, const MMArgs& p, size_t batch) {
-  if (!supported(p, batch) || (dtype == UGHIP_F32 && p.K <= 16)) return 0;
-  const size_t big = batch * ((p.M + 127) / 128) * ((p.N + 127) / 128), small = batch * ((p.M + 63) / 64) * ((p.N + 63) / 64);
-  if (big < 256 || 3 * big > small) return 64;
+//   16 bits, fewer than 256 large ones: 64 x 64 tiles that share a CU wait for its loads, so four of them and a long sum (1216 x 3200 x 1652 44.3 small, 27.2 large,
+//   1489 x 2130 x 932 24.7 / 19.2, 1215 x 2795 x 593 22.6 / 17.0; 2893 x 1238 x 202 10.5 / 10.3) or three and a longer one (1613 x 1568 x 3947 71.5 / 58.3, 3038 x 886 x 1694 27.4 /
+//   24.8; 2415 x 1244 x 861 18.3 / 19.2) are better off as one; two are not (2020 x 1018 x 2436 24.7 / 30.7).
+static int tile_of(int dtype, const MMArgs& p, size_t big, size_t small) {
+  if (3 * big > small) return 64;
   if (dtype == UGHIP_F32) return big >= 768 && (big + 64) % 256 <= 64 && p.K >= 1024 ? 128 : 64;
+  if (big < 256) return (small > 768 && p.K > 256) || (small > 600 && p.K >= 1536) ? 128 : 64;
   return p.K > 64 || (p.K > 8 && big * 5 >= (big + 255) / 256 * 256 * 4) ? 128 : 64;
 }
 
-hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, int tile) {
-  if (!supported(p, batch) || (tile != 64 && tile != 128)) return hipErrorInvalidValue;
-  if (dtype == UGHIP_F32) return tile == 128 ? launch<float, 128>(stream, p, batch) : launch<float, 64>(stream, p, batch);
-  if (dtype == UGHIP_F16) return tile == 128 ? launch<_Float16, 128>(stream, p, batch) : launch<_Float16, 64>(stream, p, batch);
-  return tile == 128 ? launch<__bf16, 128>(stream, p, batch) : launch<__bf16, 64>(stream, p, batch);
+// Small tiles that leave CUs idle, or one round of the f32 matrix pipe nearly half empty, share a long sum: slabs of K in the workspace and a launch that adds them.
+// Priced by what a step takes alone on its CU (0.28 us, f32 0.58) or beside another tile (0.45, 1.1), the second launch (2.5 and 0.12 a slab) and
+// the slabs' way to memory and back.  Measured, us whole / as split: f32 1056 x 65 x 3317 63 / 17 (six), 26 x 777 x 2040 41 / 11 (sixteen), 139 x 2791 x 2962 58 / 40
+// (three), 511 x 1309 x 2341 48 / 35 (three), 1000 x 777 x 1531 32.6 / 33.9 (two: stays whole); f16 397 x 112 x 3459 19.4 / 9.0 (eight), 282 x 1004 x 2989 22.4 / 12.8 (three), 171 x
+// 2075 x 3227 23.9 / 17.2 (two), 443 x 498 x 784 7.1 / 7.5 (two: stays whole).  At most 32 MB of slabs, the least that the block of partial tiles
+// holds.
+static int split_of(int dtype, const MMArgs& p, size_t batch, size_t tiles) {
+  const bool f32 = dtype == UGHIP_F32;
+  const int ke = f32 ? 32 : 64, steps = (p.K + ke - 1) / ke;
+  const double alone = f32 ? 0.58 : 0.28, shared = f32 ? 1.1 : 0.45;
+  const size_t slab_bytes = (batch * p.M * p.N + 3) / 4 * 16;
+  if (tiles >= 256) return 1;
+  int best = 1;
+  double best_us = steps * alone * 0.95;
+  for (int ns = 2; ns <= 32 && ns * 2 <= steps && tiles * ns <= 512 && ns * slab_bytes <= RaggedPlan::MAX_WS; ++ns) {
+    const int per = (steps + ns - 1) / ns;
+    if ((steps + per - 1) / per != ns) continue;  // a slab would have no steps
+    const double us = per * (tiles * ns <= 256 ? alone : shared) + 2.5 + 0.12 * ns + (double)(ns + 1) * slab_bytes / 5e6;
+    if (us < best_us) best = ns, best_us = us;
+  }
+  return best;
+}
+
+RaggedPlan gemm_ragged_plan(int dtype, const MMArgs& p, size_t batch) {
+  RaggedPlan pl;
+  if (!supported(p, batch) || (dtype == UGHIP_F32 && p.K <= 16)) return pl;
+  const size_t big = batch * ((p.M + 127) / 128) * ((p.N + 127) / 128), small = batch * ((p.M + 63) / 64) * ((p.N + 63) / 64);
+  pl.tile = tile_of(dtype, p, big, small);
+  if (pl.tile == 64) pl.nsplit = split_of(dtype, p, batch, small);
+  if (pl.nsplit > 1) pl.ws_bytes = pl.nsplit * ((batch * p.M * p.N + 3) / 4 * 16);
+  return pl;
+}
+
+hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, const RaggedPlan& pl, float* ws) {
+  if (!supported(p, batch) || (pl.tile != 64 && pl.tile != 128) || pl.nsplit < 1 || (pl.nsplit > 1 && (pl.tile != 64 || !ws))) return hipErrorInvalidValue;
+  if (dtype == UGHIP_F32) return launch_plan<float>(stream, p, batch, pl, ws);
+  return dtype == UGHIP_F16 ? launch_plan<_Float16>(stream, p, batch, pl, ws) : launch_plan<__bf16>(stream, p, batch, pl, ws);
 }
 
 }  // namespace ughip

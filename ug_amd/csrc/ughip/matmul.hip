@@ -500,8 +500,11 @@ static Route matmul_route(int dtype, bool mixed, const MMArgs& p, size_t b, size
   return gemm_tiled_supported(dtype, p, b, mixed) ? ROUTE_TILED : ROUTE_ANY;
 }
 
-// The kernels behind ROUTE_ANY, in names: gemm_ragged's 64 x 64 and 128 x 128 tiles (gemm_ragged_tile), and the ones that go by element.
-static const char* any_tail(int tile) { return tile == 128 ? ",128x128" : tile ? "" : ",by element"; }
+// The kernels behind ROUTE_ANY, in names: gemm_ragged's 64 x 64 and 128 x 128 tiles (gemm_ragged_plan), and the ones that go by element.
+static void any_name(const char* tn, const RaggedPlan& pl, char* out, size_t out_len) {
+  if (pl.nsplit > 1) snprintf(out, out_len, "gemm_any<%s,splitK=%d>", tn, pl.nsplit);
+  else snprintf(out, out_len, "gemm_any<%s%s>", tn, pl.tile == 128 ? ",128x128" : pl.tile ? "" : ",by element");
+}
 
 static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* lhs, const ughip_slice* rhs, size_t b, size_t m, size_t n, size_t k,
                        size_t rank, const size_t* lhs_dims, const size_t* lhs_strides, size_t lhs_offset, const size_t* rhs_dims, const size_t* rhs_strides,
@@ -607,9 +610,20 @@ static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* l
   } else {
     dim3 grid((unsigned)((n + 63) / 64), (unsigned)((m + 63) / 64), (unsigned)b);
     if (grid.y > 65535 || b > 65535) return set_error(UGHIP_ERR_INVALID, "matmul: m or batch too large for this kernel");
-    const int tile = gemm_ragged_tile(dst->dtype, p, b);
-    note_kernel("gemm_any<%s%s>", tn, any_tail(tile));
-    if (tile) UGHIP_HIPCHK(gemm_ragged_launch(st, dst->dtype, p, b, tile));
+    RaggedPlan pl = gemm_ragged_plan(dst->dtype, p, b);
+    static_assert(RaggedPlan::MAX_WS <= UGHIP_MATMUL_NOALLOC_SCRATCH_BYTES, "a product that could be taken whole is not refused for its slabs");
+    float* ws = static_cast<float*>(dev->static_scratch);
+    if (pl.nsplit > 1 && !no_alloc) {
+      if (grow_gemm_ws(dev, pl.ws_bytes)) {  // no memory for the slabs: whole
+        (void)hipGetLastError();
+        pl.nsplit = 1;
+      }
+      ws = static_cast<float*>(dev->gemm_ws);
+    }
+    char name[64];
+    any_name(tn, pl, name, sizeof name);
+    note_kernel("%s", name);
+    if (pl.tile) UGHIP_HIPCHK(gemm_ragged_launch(st, dst->dtype, p, b, pl, ws));
     else if (f32) gemm_f32_any<<<grid, 256, 0, st>>>(p);
     else if (dst->dtype == UGHIP_F16) gemm_half_any<_Float16><<<grid, 256, 0, st>>>(p);
     else gemm_half_any<__bf16><<<grid, 256, 0, st>>>(p);
@@ -1010,7 +1024,7 @@ extern "C" int ughip_matmul_plan(int dtype, int rhs_dtype, size_t b, size_t m, s
       break;
     }
     case ROUTE_TILED: gemm_tiled_name(dtype, p, b, mixed, nullptr, buf, buf_len); break;
-    default: snprintf(buf, buf_len, "gemm_any<%s%s>", tn, any_tail(gemm_ragged_tile(dtype, p, b))); break;
+    default: any_name(tn, gemm_ragged_plan(dtype, p, b), buf, buf_len); break;
   }
   return UGHIP_OK;
 }
