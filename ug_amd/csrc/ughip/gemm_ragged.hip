@@ -8,7 +8,7 @@
 //   what does not exist, and comes first, under the way of the next ones: it holds the only row of a
 //   [k, n]-major operand behind which nothing may be read.
 //
-// What bounds it: the steps of K on few tiles (0.3 us each in 16 bits, 0.6 in f32, the f32 matrix pipe two thirds of that; deeper prefetch changes nothing), LDS and the f32
+// What bounds it: the steps of K on few tiles (0.3 us each in 16 bits, a CU's share of the caches; 0.6 in f32, the f32 matrix pipe two thirds of that; four steps ahead or more waves per tile change nothing), LDS and the f32
 // matrix pipe on many.  Against element-by-element
 // loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 14.6 us, f32 256 -> 34; 2001^3 f16 270 -> 37, f32 340 -> 135; 3999^2 x
 // 2000 f16 1204 -> 103, f32 1014 -> 520; 100^3 9.4 -> 5.4.  Which tile takes what and where K is split: gemm_ragged_plan.
@@ -195,23 +195,24 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
   }
   if (end > begin) {
     fetch(0, begin);
+    __builtin_amdgcn_sched_barrier(0);  // (in this order: the loop counts on it)
     fetch(1, min(begin + 1, end - 1));
   }
   put(lds[0], la, lb);
   __syncthreads();
   multiply(lds[0]);
-  for (int s0 = begin; s0 < end; s0 += 2) {
-#pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      const int s = s0 + d;
-      if (s >= end) break;
-      char* buf = lds[d ^ 1];
-      put(buf, ra[d], rb[d]);
-      fetch(d, min(s + 2, end - 1));  // (without a branch, so that a step's loads can be waited for alone)
-      __syncthreads();                 // one barrier a step: the buffer written next was read before it
-      multiply(buf);
-    }
-  }
+  auto step = [&](int d, int s) {
+    char* buf = lds[d ^ 1];
+    put(buf, ra[d], rb[d]);
+    fetch(d, min(s + 2, end - 1));  // (without a branch, so that a step's loads can be waited for alone)
+    __syncthreads();                // one barrier a step: the buffer written next was read before it
+    multiply(buf);
+  };
+  // Two steps a turn and no way out between them: from there the compiler sees one back to the loop's head on which the loads wanted there are the latest,
+  // and waits for all of them there.  f16 900 x 1000 x 4001 29.2 -> 24.4 us, 1000 x 777 x 1531 14.2 -> 12.8; f32 497 x 391 x 2100 whole 45.3 -> 43.6.
+  int s = begin;
+  for (; s + 2 <= end; s += 2) step(0, s), step(1, s + 1);
+  if (s < end) step(0, s);
 
   // element e of lane l of block (i, j): row l % 32, column 8 (e / 4) + 4 (l / 32) + e % 4
   typedef typename Result<T, SPLIT>::type R;
