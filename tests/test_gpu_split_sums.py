@@ -35,3 +35,13 @@ def test_the_call_that_may_not_allocate(hip, dtype, bmnk):
     ref, got, kernel = no_alloc._both(hip, dtype, bmnk, True, 91)
     assert ",splitK=" in kernel
     np.testing.assert_array_equal(got, ref)
+
+
+# K of a step less one, a step, one and a bit, two less one: the step in front of K's end overlaps the one before by nothing to all but one; columns and rows that end
+# inside a piece of 16 bytes, at its first element and at its last
+@pytest.mark.parametrize("bmnk", [(1, 9, 9, 31), (1, 66, 71, 32), (2, 67, 65, 33), (1, 71, 66, 63), (1, 12, 79, 64), (2, 77, 12, 65), (1, 73, 9, 95), (3, 9, 10, 127), (1, 68, 95, 128)])
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
+@pytest.mark.parametrize("lhs_mk", [True, False], ids=["rows", "transposed"])
+def test_last_step(hip, bmnk, dtype, rhs_nk, lhs_mk):
+    products.test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk)

@@ -4,9 +4,9 @@
 //   64 x 64 or 128 x 128 tiles, four waves 2 x 2, 32 x 32 MFMA blocks.  A K step is 128 bytes of a k-contiguous row, 8 chunks of 16 bytes,
 //   fetched by 16-byte loads at whatever address the row has (the hardware takes any) two steps ahead into registers, then written to one of
 //   two LDS buffers: k-contiguous operands as rows of k, the others as they lie, and the waves read those back transposed
-//   (ds_read_b64_tr_b16; f32 element by element).  The last step, K's remainder or a whole one, is loaded element by element with zeros for
-//   what does not exist, and comes first, under the way of the next ones: it holds the only row of a
-//   [k, n]-major operand behind which nothing may be read.
+//   (ds_read_b64_tr_b16; f32 element by element).  The last step, K's remainder or a whole one, comes first, under the way of the next ones: the
+//   elements in front of K's end by vectors, with zeros for those that belong to the step before (a K of less than one step: element by element). It
+//   holds the only row of a [k, n]-major operand behind which nothing may be read.
 //
 // What bounds it: the steps of K on few tiles (0.3 us each in 16 bits, a CU's share of the caches; 0.6 in f32, the f32 matrix pipe two thirds of that; four steps ahead or more waves per tile change nothing), LDS and the f32
 // matrix pipe on many.  Against element-by-element
@@ -97,6 +97,27 @@ struct Side {
     }
     return __builtin_bit_cast(u32x4, v);
   }
+  // The same for K >= KE, by vectors: the KE elements of k in front of K's end, of which `trimmed` keeps those that step s - 1 has not had.  (32 loads of
+  // an element per thread kept a CU's address unit busy for a microsecond: f16 1000 x 777 x 1531 12.8 -> 12.2 us.)
+  __device__ u32x4 load_end(int i, int s, int left, int r0, int rows, int tid) const {
+    const int id = tid + 256 * i, row = id / CPR, c = id % CPR, x = r0 + c * E < rows ? r0 + c * E : 0;
+    if (KC) return load16(at[i] + s * step - (KE - left));
+    const T* q = at[i] + s * step - (KE - left) * (step / KE);
+    if (row < KE - 1 || x + E <= rows) return load16(q);
+    T t[E];  // behind the last row nothing may be read
+#pragma unroll
+    for (int e = 0; e < E; ++e) t[e] = q[min(e, rows - 1 - x)];
+    return __builtin_bit_cast(u32x4, t);
+  }
+  __device__ static u32x4 trimmed(u32x4 v, int i, int left, int tid) {
+    const int id = tid + 256 * i, row = id / CPR, c = id % CPR, had = KE - left;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int n = KC ? had - c * E - w * (E / 4) : row < had ? 2 : 0;  // of this word's elements and those behind it
+      v[w] = n >= E / 4 ? 0u : n > 0 ? v[w] & 0xffff0000u : v[w];
+    }
+    return v;
+  }
   // lane's fragment of block b0 .. b0 + 31, chunk pair c2 (chunks 2 c2 and 2 c2 + 1)
   __device__ static u32x4 frag(const char* lds, int b0, int c2, int lane) {
     if constexpr (KC) {
@@ -182,7 +203,12 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
         for (int j = 0; j < MI; ++j) mma(T(), fb[j], fa[i], acc[i][j]);  // swapped: a lane holds columns of one row
     }
   };
-  if (with_left) {
+  if (with_left && full > 0) {
+#pragma unroll
+    for (int i = 0; i < SA::N; ++i) la[i] = a.load_end(i, full, left, m0, p.M, tid);
+#pragma unroll
+    for (int i = 0; i < SB::N; ++i) lb[i] = b.load_end(i, full, left, n0, p.N, tid);
+  } else if (with_left) {
 #pragma unroll
     for (int i = 0; i < SA::N; ++i) la[i] = a.load_last(i, full, left, m0, p.M, tid);
 #pragma unroll
@@ -197,6 +223,12 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
     fetch(0, begin);
     __builtin_amdgcn_sched_barrier(0);  // (in this order: the loop counts on it)
     fetch(1, min(begin + 1, end - 1));
+  }
+  if (with_left && full > 0) {
+#pragma unroll
+    for (int i = 0; i < SA::N; ++i) la[i] = SA::trimmed(la[i], i, left, tid);
+#pragma unroll
+    for (int i = 0; i < SB::N; ++i) lb[i] = SB::trimmed(lb[i], i, left, tid);
   }
   put(lds[0], la, lb);
   __syncthreads();
