@@ -614,12 +614,10 @@ static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* l
     static_assert(RaggedPlan::MAX_WS <= UGHIP_MATMUL_NOALLOC_SCRATCH_BYTES, "a product that could be taken whole is not refused for its slabs");
     float* ws = static_cast<float*>(dev->static_scratch);
     if (pl.nsplit > 1 && !no_alloc) {
-      if (grow_gemm_ws(dev, pl.ws_bytes)) {  // no memory for the slabs: whole
-        (void)hipGetLastError();
-        pl.nsplit = 1;
-      }
+      if (grow_gemm_ws(dev, pl.ws_bytes)) (void)hipGetLastError();
       ws = static_cast<float*>(dev->gemm_ws);
     }
+    if (!ws) pl.nsplit = 1;  // no memory for the slabs: whole
     char name[64];
     any_name(tn, pl, name, sizeof name);
     note_kernel("%s", name);
