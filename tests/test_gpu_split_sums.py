@@ -9,15 +9,15 @@ import ug_amd
 pytestmark = pytest.mark.gpu
 
 
-# the fewest steps of K that are split, a whole last step and one element of one, uneven slabs, a tile over the edge, slabs of 1, 2 and 3 elements behind the last four,
+# sums that are split in 32 bits, the shorter ones on 32 x 32 tiles without a split in 16: a whole last step and one element of one, uneven slabs, a tile over the edge, slabs of 1, 2 and 3 elements behind the last four,
 # as many slabs as there may be, tiles times slabs on either side of a round of the chip; a product in a batch
-@pytest.mark.parametrize("bmnk", [(1, 9, 9, 1600), (1, 9, 9, 1601), (1, 65, 67, 1407), (1, 21, 11, 4096), (1, 63, 65, 3000), (3, 70, 9, 2050), (1, 705, 700, 2001), (1, 500, 1001, 2001)])
+@pytest.mark.parametrize("bmnk", [(1, 9, 9, 1600), (1, 9, 9, 1601), (1, 65, 67, 1407), (1, 21, 11, 4096), (1, 63, 65, 3000), (3, 70, 9, 2050), (1, 150, 500, 4001), (1, 500, 1001, 2001)])
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
 @pytest.mark.parametrize("lhs_mk", [True, False], ids=["rows", "transposed"])
 def test_split_sums(hip, bmnk, dtype, rhs_nk, lhs_mk):
     products.test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk)
-    if bmnk[1] < 100 and bmnk[3] % 64:
+    if dtype == "f32" and bmnk[1] < 100 and bmnk[3] % 64:
         assert ",splitK=" in ug_amd.last_kernel(), ug_amd.last_kernel()
 
 
@@ -30,7 +30,7 @@ def test_three_and_four_tiles_to_a_cu(hip, bmnk, large, dtype):
 
 
 @pytest.mark.parametrize("dtype", [ug_amd.F32, ug_amd.BF16], ids=["f32", "bf16"])
-@pytest.mark.parametrize("bmnk", [(1, 70, 65, 3001), (2, 33, 9, 2047)])
+@pytest.mark.parametrize("bmnk", [(1, 70, 65, 6001), (2, 33, 9, 5999)])
 def test_the_call_that_may_not_allocate(hip, dtype, bmnk):
     ref, got, kernel = no_alloc._both(hip, dtype, bmnk, True, 91)
     assert ",splitK=" in kernel
@@ -44,4 +44,13 @@ def test_the_call_that_may_not_allocate(hip, dtype, bmnk):
 @pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
 @pytest.mark.parametrize("lhs_mk", [True, False], ids=["rows", "transposed"])
 def test_last_step(hip, bmnk, dtype, rhs_nk, lhs_mk):
+    products.test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk)
+
+
+# 32 x 32 tiles, a few and several to a CU: fewer steps of K than waves, as many, one more, uneven parts and a last wave without one; tiles over both edges; batches
+@pytest.mark.parametrize("bmnk", [(1, 100, 100, 65), (1, 33, 65, 120), (1, 300, 300, 300), (2, 31, 97, 257), (1, 330, 9, 350), (1, 625, 319, 353), (15, 19, 18, 640), (1, 23, 148, 1355), (8, 200, 200, 200)])
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
+@pytest.mark.parametrize("lhs_mk", [True, False], ids=["rows", "transposed"])
+def test_small_tiles(hip, bmnk, dtype, rhs_nk, lhs_mk):
     products.test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk)

@@ -102,7 +102,7 @@ hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRo
 // elements from one k to the next in the latter case.  Contiguous [batch, M, N] result.  The plan it takes a product with; tile 0: the kernels
 // that go by element should.
 struct RaggedPlan {
-  int tile = 0, nsplit = 1;  // 64 or 128; nsplit > 1: workgroups share a tile's K and leave slabs in the workspace, which a second launch adds up
+  int tile = 0, nsplit = 1;  // 32, 64 or 128; nsplit > 1, not with 128: workgroups share a tile's K and leave slabs in the workspace, which a second launch adds up
   size_t ws_bytes = 0;
   static constexpr size_t MAX_WS = (size_t)32 << 20;
 };

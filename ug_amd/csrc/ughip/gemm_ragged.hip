@@ -1,7 +1,7 @@
 // MFMA GEMM for operands that no tuned kernel takes -- any M, N and K, rows that start at any element -- with f32 accumulate: f32, f16, bf16;
 // each operand contiguous along k or along its other dimension.
 //
-//   64 x 64 or 128 x 128 tiles, four waves 2 x 2, 32 x 32 MFMA blocks.  A K step is 128 bytes of a k-contiguous row, 8 chunks of 16 bytes,
+//   64 x 64 or 128 x 128 tiles, four waves 2 x 2, 32 x 32 MFMA blocks (and 32 x 32 tiles: gemm_ragged32).  A K step is 128 bytes of a k-contiguous row, 8 chunks of 16 bytes,
 //   fetched by 16-byte loads at whatever address the row has (the hardware takes any) two steps ahead into registers, then written to one of
 //   two LDS buffers: k-contiguous operands as rows of k, the others as they lie, and the waves read those back transposed
 //   (ds_read_b64_tr_b16; f32 element by element).  The last step, K's remainder or a whole one, comes first, under the way of the next ones: the
@@ -13,6 +13,8 @@
 // loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 14.6 us, f32 256 -> 34; 2001^3 f16 270 -> 37, f32 340 -> 135; 3999^2 x
 // 2000 f16 1204 -> 103, f32 1014 -> 520; 100^3 9.4 -> 5.4.  Which tile takes what and where K is split: gemm_ragged_plan.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "gemm.h"
 #include "ughip.h"
@@ -58,12 +60,12 @@ __device__ __forceinline__ void mma(float, const u32x4& a, const u32x4& b, f32x1
 }
 
 // One operand's share of a workgroup's tile: `rows` (M or N) times k.  KC: contiguous along k.
-template <typename T, int B, bool KC>
+template <typename T, int B, bool KC, int THREADS = 256>
 struct Side {
   static constexpr int E = 16 / sizeof(T), KE = 8 * E;           // elements per chunk, k per step
   static constexpr int CPR = KC ? 8 : B / E;                     // chunks per row in LDS (a row: of k, or of the operand's rows at one k)
   static constexpr int PITCH = CPR * 16 + 16, LDS_ROWS = KC ? B : KE, BYTES = LDS_ROWS * PITCH;
-  static constexpr int N = LDS_ROWS * CPR / 256;                 // chunks per thread
+  static constexpr int N = LDS_ROWS * CPR / THREADS;             // chunks per thread
   const T* at[N];
   long long step;  // elements from one K step to the next
   int lds_at[N];
@@ -72,7 +74,7 @@ struct Side {
     step = KC ? KE : KE * cs;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      const int id = tid + 256 * i, row = id / CPR, c = id % CPR;
+      const int id = tid + THREADS * i, row = id / CPR, c = id % CPR;
       lds_at[i] = row * PITCH + c * 16;
       // past the last row: any row (its results are not stored); a chunk that straddles the end runs on into the next k's row
       if (KC) at[i] = base + min(r0 + row, rows - 1) * rs + c * E;
@@ -82,7 +84,7 @@ struct Side {
   __device__ u32x4 load(int i, int s) const { return load16(at[i] + s * step); }
   // step s with `left` elements of k, by element; rows: of the operand behind r0
   __device__ u32x4 load_last(int i, int s, int left, int r0, int rows, int tid) const {
-    const int id = tid + 256 * i, row = id / CPR, c = id % CPR;
+    const int id = tid + THREADS * i, row = id / CPR, c = id % CPR;
     T v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -100,7 +102,7 @@ struct Side {
   // The same for K >= KE, by vectors: the KE elements of k in front of K's end, of which `trimmed` keeps those that step s - 1 has not had.  (32 loads of
   // an element per thread kept a CU's address unit busy for a microsecond: f16 1000 x 777 x 1531 12.8 -> 12.2 us.)
   __device__ u32x4 load_end(int i, int s, int left, int r0, int rows, int tid) const {
-    const int id = tid + 256 * i, row = id / CPR, c = id % CPR, x = r0 + c * E < rows ? r0 + c * E : 0;
+    const int id = tid + THREADS * i, row = id / CPR, c = id % CPR, x = r0 + c * E < rows ? r0 + c * E : 0;
     if (KC) return load16(at[i] + s * step - (KE - left));
     const T* q = at[i] + s * step - (KE - left) * (step / KE);
     if (row < KE - 1 || x + E <= rows) return load16(q);
@@ -110,7 +112,7 @@ struct Side {
     return __builtin_bit_cast(u32x4, t);
   }
   __device__ static u32x4 trimmed(u32x4 v, int i, int left, int tid) {
-    const int id = tid + 256 * i, row = id / CPR, c = id % CPR, had = KE - left;
+    const int id = tid + THREADS * i, row = id / CPR, c = id % CPR, had = KE - left;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const int n = KC ? had - c * E - w * (E / 4) : row < had ? 2 : 0;  // of this word's elements and those behind it
@@ -270,6 +272,115 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
   }
 }
 
+// 32 x 32 tiles, for products of so few larger ones that most CUs would have none.  A wave has a block of its own parts of K, LDS of its own and no barriers
+// in its loop; the four waves' sums meet in LDS.  Part i (of 4 nsplit) has the steps per * i .. per * (i + 1) - 1, of which there may be none.
+// What bounds it: launch and first bytes, then a wave's chain of steps (0.6 us, in 16 bits 8 KB of a CU's share of the caches).  f32 625 x 319 x 353 on 64 x 64 tiles 10.3 us, 6.3 so;
+// what it takes, and more figures: gemm_ragged_plan.
+template <typename T, bool A_KC, bool B_KC, bool SPLIT>
+__global__ void __launch_bounds__(256) gemm_ragged32(MMArgs p, int batches, int tiles_m, int tiles_n, int nsplit, int per, float* __restrict__ ws, size_t slab_elems) {
+  typedef Side<T, 32, A_KC, 64> SA;
+  typedef Side<T, 32, B_KC, 64> SB;
+  constexpr int KE = SA::KE, BUF = SA::BYTES + SB::BYTES;
+  static_assert(BUF >= 4 * 1024);  // a wave's sums go where its operands were
+  __shared__ __attribute__((aligned(16))) char lds[4][BUF];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tpb = tiles_m * tiles_n, tiles = batches * tpb * (SPLIT ? nsplit : 1), run = (tiles + 7) >> 3;
+  int bid = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+  if (bid >= tiles) return;
+  const int slab = SPLIT ? bid / (batches * tpb) : 0;
+  if (SPLIT) bid -= slab * batches * tpb;
+  const int batch = bid / tpb, in_batch = bid - batch * tpb, tm = in_batch / tiles_n, tn = in_batch - tm * tiles_n, m0 = tm * 32, n0 = tn * 32;
+  const int full = (p.K - 1) / KE, left = p.K - full * KE;
+  const int from = (slab * 4 + wave) * per, to = min(from + per, full + 1);
+  const bool with_left = to == full + 1;
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+  char* buf = lds[wave];
+  if (from < to) {
+    SA a;
+    SB b;
+    a.place(static_cast<const T*>(p.a) + (size_t)batch * p.a_bs, m0, p.M, p.a_rs, p.a_cs, lane);
+    b.place(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs, n0, p.N, p.b_cs, p.b_rs, lane);
+    // behind the first one, K's remainder or the part's first
+    const int begin = with_left ? from : from + 1, end = with_left ? full : to;
+    u32x4 ra[2][SA::N], rb[2][SB::N], la[SA::N], lb[SB::N];
+    auto fetch = [&](int d, int s) {
+#pragma unroll
+      for (int i = 0; i < SA::N; ++i) ra[d][i] = a.load(i, s);
+#pragma unroll
+      for (int i = 0; i < SB::N; ++i) rb[d][i] = b.load(i, s);
+    };
+    // (a wave's LDS operations complete in order; the fences keep the compiler from moving lanes' reads over other lanes' writes)
+    auto turn = [&](const u32x4* va, const u32x4* vb, auto&& next) {
+#pragma unroll
+      for (int i = 0; i < SA::N; ++i) *reinterpret_cast<u32x4*>(buf + a.lds_at[i]) = va[i];
+#pragma unroll
+      for (int i = 0; i < SB::N; ++i) *reinterpret_cast<u32x4*>(buf + SA::BYTES + b.lds_at[i]) = vb[i];
+      next();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      u32x4 fa[4], fb[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) fa[c] = SA::frag(buf, 0, c, lane), fb[c] = SB::frag(buf + SA::BYTES, 0, c, lane);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) mma(T(), fb[c], fa[c], acc);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    };
+    if (with_left && full > 0) {
+#pragma unroll
+      for (int i = 0; i < SA::N; ++i) la[i] = a.load_end(i, full, left, m0, p.M, lane);
+#pragma unroll
+      for (int i = 0; i < SB::N; ++i) lb[i] = b.load_end(i, full, left, n0, p.N, lane);
+    } else if (with_left) {
+#pragma unroll
+      for (int i = 0; i < SA::N; ++i) la[i] = a.load_last(i, full, left, m0, p.M, lane);
+#pragma unroll
+      for (int i = 0; i < SB::N; ++i) lb[i] = b.load_last(i, full, left, n0, p.N, lane);
+    } else {
+#pragma unroll
+      for (int i = 0; i < SA::N; ++i) la[i] = a.load(i, from);
+#pragma unroll
+      for (int i = 0; i < SB::N; ++i) lb[i] = b.load(i, from);
+    }
+    if (end > begin) {
+      fetch(0, begin);
+      __builtin_amdgcn_sched_barrier(0);  // (in this order: the loop counts on it)
+      fetch(1, min(begin + 1, end - 1));
+    }
+    if (with_left && full > 0) {
+#pragma unroll
+      for (int i = 0; i < SA::N; ++i) la[i] = SA::trimmed(la[i], i, left, lane);
+#pragma unroll
+      for (int i = 0; i < SB::N; ++i) lb[i] = SB::trimmed(lb[i], i, left, lane);
+    }
+    turn(la, lb, [] {});
+    auto step = [&](int d, int s) { turn(ra[d], rb[d], [&] { fetch(d, min(s + 2, end - 1)); }); };
+    int s = begin;
+    for (; s + 2 <= end; s += 2) step(0, s), step(1, s + 1);  // (no way out between the two: as in gemm_ragged)
+    if (s < end) step(0, s);
+  }
+  // quad g of lane l: row l % 32, columns 8 g + 4 (l / 32) and the next three.  Wave w finishes quad w, summed over the waves in the order of K.
+#pragma unroll
+  for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(buf + (g * 64 + lane) * 16) = f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+  __syncthreads();
+  f32x4 v = *reinterpret_cast<const f32x4*>(lds[0] + (wave * 64 + lane) * 16);
+#pragma unroll
+  for (int w = 1; w < 4; ++w) v += *reinterpret_cast<const f32x4*>(lds[w] + (wave * 64 + lane) * 16);
+  const int row = m0 + (lane & 31), col = n0 + 8 * wave + 4 * (lane >> 5);
+  if (row >= p.M) return;
+  typedef typename Result<T, SPLIT>::type R;
+  R* __restrict__ q = (SPLIT ? reinterpret_cast<R*>(ws + slab * slab_elems) : static_cast<R*>(p.c)) + (size_t)batch * p.c_bs + (size_t)row * p.N + col;
+  if (col + 4 <= p.N) {
+    store4(q, v);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (col + e < p.N) q[e] = (R)v[e];
+  }
+}
+
 // c = the slabs' sum, in their order
 template <typename T>
 __global__ void __launch_bounds__(256) gemm_ragged_fold(const float* __restrict__ ws, T* __restrict__ c, size_t elems, size_t slab_elems, int nsplit) {
@@ -299,8 +410,22 @@ hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, int nsplit,
   if (SPLIT) gemm_ragged_fold<T><<<(unsigned)((elems + 1023) / 1024), 256, 0, stream>>>(ws, static_cast<T*>(p.c), elems, slab, nsplit);
   return hipGetLastError();
 }
+template <typename T, bool SPLIT>
+hipError_t launch32(hipStream_t stream, const MMArgs& p, size_t batch, int nsplit, float* ws) {
+  const int tiles_m = (p.M + 31) / 32, tiles_n = (p.N + 31) / 32, ke = 128 / (int)sizeof(T), steps = (p.K + ke - 1) / ke, per = (steps + 4 * nsplit - 1) / (4 * nsplit);
+  const unsigned grid = (unsigned)((batch * tiles_m * tiles_n * nsplit + 7) / 8 * 8);
+  const size_t elems = batch * p.M * p.N, slab = (elems + 3) / 4 * 4;
+  const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
+  if (ak && bk) gemm_ragged32<T, true, true, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  else if (ak) gemm_ragged32<T, true, false, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  else if (bk) gemm_ragged32<T, false, true, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  else gemm_ragged32<T, false, false, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  if (SPLIT) gemm_ragged_fold<T><<<(unsigned)((elems + 1023) / 1024), 256, 0, stream>>>(ws, static_cast<T*>(p.c), elems, slab, nsplit);
+  return hipGetLastError();
+}
 template <typename T>
 hipError_t launch_plan(hipStream_t stream, const MMArgs& p, size_t batch, const RaggedPlan& pl, float* ws) {
+  if (pl.tile == 32) return pl.nsplit > 1 ? launch32<T, true>(stream, p, batch, pl.nsplit, ws) : launch32<T, false>(stream, p, batch, 1, nullptr);
   if (pl.nsplit > 1) return launch<T, 64, true>(stream, p, batch, pl.nsplit, ws);
   return pl.tile == 128 ? launch<T, 128, false>(stream, p, batch, 1, nullptr) : launch<T, 64, false>(stream, p, batch, 1, nullptr);
 }
@@ -332,41 +457,49 @@ static int tile_of(int dtype, const MMArgs& p, size_t big, size_t small) {
   return p.K > 64 || (p.K > 8 && big * 5 >= (big + 255) / 256 * 256 * 4) ? 128 : 64;
 }
 
-// Small tiles that leave CUs idle, or one round of the f32 matrix pipe nearly half empty, share a long sum: slabs of K in the workspace and a launch that adds them.
-// Priced by what a step takes alone on its CU (0.28 us, f32 0.58) or beside another tile (0.45, 1.1), the second launch (2.5 and 0.12 a slab) and
-// the slabs' way to memory and back.  Measured, us whole / as split: f32 1056 x 65 x 3317 63 / 17 (six), 26 x 777 x 2040 41 / 11 (sixteen), 139 x 2791 x 2962 58 / 40
-// (three), 511 x 1309 x 2341 48 / 35 (three), 1000 x 777 x 1531 32.6 / 33.9 (two: stays whole); f16 397 x 112 x 3459 19.4 / 9.0 (eight), 282 x 1004 x 2989 22.4 / 12.8 (three), 171 x
-// 2075 x 3227 23.9 / 17.2 (two), 443 x 498 x 784 7.1 / 7.5 (two: stays whole).  At most 32 MB of slabs, the least that the block of partial tiles
-// holds.
-static int split_of(int dtype, const MMArgs& p, size_t batch, size_t tiles) {
+// Fewer than 256 small tiles: 64 x 64 or, where that leaves most CUs without one, 32 x 32 with K over the workgroup's waves; and with a long sum slabs of K in the
+// workspace and a launch that adds them (2.5 us and 0.1 a slab, the slabs' way to memory and back, and 8.8 us at the least: a program's thread takes that for the two).
+//   64 x 64: a step takes 0.25 us and up to 0.16 more as the chip fills (f32: 0.56 and 0.06), 0.75 (1.1) beside another tile on its CU
+//   32 x 32: a quarter of the steps at 0.6 us (f32: 0.66, as many times as a CU has tiles); 16 bits wait for their 8 KB a step as well, 0.12 us and as much again when the chip is full
+// Measured, us 64 whole / 64 split / 32 whole / 32 split, the best split each: f32 300^3 9.0 / 8.7 / 6.3 / -, 625 x 319 x 353 10.3 / 9.7 / 6.3 / -, 15 of 19 x 18 x 640 14.8 / 9.1 /
+// 6.7 / 9.0, 700 x 700 x 500 13.0 / 12.5 / 10.2 / 14.9, 777 x 500 x 1500 30.6 / 20.8 / 19.2 / 22.8, 39 x 801 x 3001 56 / 12.9 / 18.2 / 11.5, 38 x 20 x 1920 37 / 11.0 / 12.3 / 9.1,
+// 1000 x 777 x 399 11.7 / 16.1 / 14.0 / -; f16 23 x 148 x 1355 8.4 / 8.9 / 6.2 / 8.9, 200 x 200 x 1000 7.2 / 8.6 / 6.0 / 8.8, 497 x 391 x 2100 13.4 / 10.6 / 10.0 / 14.4, 150 x 1000 x
+// 4001 21.7 / 11.7 / 15.6 / 15.1, 39 x 801 x 3001 15.1 / 9.0 / 10.8 / 9.0, 777 x 500 x 1500 10.2 / 10.4 / 11.1 / 16.7.  At most 32 MB of slabs, the least that the block of
+// partial tiles holds.
+static double few_tiles_us(int dtype, int tile, int steps, size_t tiles, int ns, size_t slab_bytes) {
   const bool f32 = dtype == UGHIP_F32;
-  const int ke = f32 ? 32 : 64, steps = (p.K + ke - 1) / ke;
-  const double alone = f32 ? 0.58 : 0.28, shared = f32 ? 1.1 : 0.45;
-  const size_t slab_bytes = (batch * p.M * p.N + 3) / 4 * 16;
-  if (tiles >= 256) return 1;
-  int best = 1;
-  double best_us = steps * alone * 0.95;
-  for (int ns = 2; ns <= 32 && ns * 2 <= steps && tiles * ns <= 512 && ns * slab_bytes <= RaggedPlan::MAX_WS; ++ns) {
-    const int per = (steps + ns - 1) / ns;
-    if ((steps + per - 1) / per != ns) continue;  // a slab would have no steps
-    const double us = per * (tiles * ns <= 256 ? alone : shared) + 2.5 + 0.12 * ns + (double)(ns + 1) * slab_bytes / 5e6;
-    if (us < best_us) best = ns, best_us = us;
-  }
-  return best;
+  const double share = (double)(tiles * ns) / 256;
+  const int per = (steps + ns - 1) / ns, part = (steps + 4 * ns - 1) / (4 * ns), on_cu = (int)((tiles * ns + 255) / 256);
+  double us = f32 ? 3.2 : 3.0;
+  if (tile == 32) us += 0.3 * on_cu + (f32 ? 0.66 * part * on_cu : std::max(0.6 * part, (0.12 + 0.12 * share) * per));
+  else us += per * (share > 1 ? (f32 ? 1.1 : 0.75) : f32 ? 0.56 + 0.06 * share : 0.25 + 0.16 * share);
+  return ns == 1 ? us : std::max(8.8, us + 2.5 + 0.1 * ns + (double)(ns + 1) * slab_bytes / 5e6);
 }
 
 RaggedPlan gemm_ragged_plan(int dtype, const MMArgs& p, size_t batch) {
   RaggedPlan pl;
   if (!supported(p, batch) || (dtype == UGHIP_F32 && p.K <= 16)) return pl;
-  const size_t big = batch * ((p.M + 127) / 128) * ((p.N + 127) / 128), small = batch * ((p.M + 63) / 64) * ((p.N + 63) / 64);
-  pl.tile = tile_of(dtype, p, big, small);
-  if (pl.tile == 64) pl.nsplit = split_of(dtype, p, batch, small);
-  if (pl.nsplit > 1) pl.ws_bytes = pl.nsplit * ((batch * p.M * p.N + 3) / 4 * 16);
+  auto tiles = [&](int t) { return batch * ((p.M + t - 1) / t) * ((p.N + t - 1) / t); };
+  const size_t small = tiles(64), slab_bytes = (batch * p.M * p.N + 3) / 4 * 16;
+  pl.tile = tile_of(dtype, p, tiles(128), small);
+  if (pl.tile == 128 || small >= 256) return pl;
+  const int ke = dtype == UGHIP_F32 ? 32 : 64, steps = (p.K + ke - 1) / ke;
+  double best = 0.95 * few_tiles_us(dtype, 64, steps, small, 1, slab_bytes);
+  for (int tile : {32, 64}) {
+    const size_t n = tiles(tile);
+    for (int ns = 1; ns <= 32 && ns * (tile == 32 ? 8 : 2) <= std::max(steps, 8) && (ns == 1 || (n * ns <= 512 && ns * slab_bytes <= RaggedPlan::MAX_WS)); ++ns) {
+      const int per = (steps + ns - 1) / ns;
+      if (tile == 64 && (ns == 1 || (steps + per - 1) / per != ns)) continue;  // (a slab would have no steps)
+      const double us = few_tiles_us(dtype, tile, steps, n, ns, slab_bytes);
+      if (us < best) best = us, pl.tile = tile, pl.nsplit = ns;
+    }
+  }
+  if (pl.nsplit > 1) pl.ws_bytes = pl.nsplit * slab_bytes;
   return pl;
 }
 
 hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, const RaggedPlan& pl, float* ws) {
-  if (!supported(p, batch) || (pl.tile != 64 && pl.tile != 128) || pl.nsplit < 1 || (pl.nsplit > 1 && (pl.tile != 64 || !ws))) return hipErrorInvalidValue;
+  if (!supported(p, batch) || (pl.tile != 32 && pl.tile != 64 && pl.tile != 128) || pl.nsplit < 1 || (pl.nsplit > 1 && (pl.tile == 128 || !ws))) return hipErrorInvalidValue;
   if (dtype == UGHIP_F32) return launch_plan<float>(stream, p, batch, pl, ws);
   return dtype == UGHIP_F16 ? launch_plan<_Float16>(stream, p, batch, pl, ws) : launch_plan<__bf16>(stream, p, batch, pl, ws);
 }

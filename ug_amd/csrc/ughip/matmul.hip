@@ -500,7 +500,7 @@ static Route matmul_route(int dtype, bool mixed, const MMArgs& p, size_t b, size
   return gemm_tiled_supported(dtype, p, b, mixed) ? ROUTE_TILED : ROUTE_ANY;
 }
 
-// The kernels behind ROUTE_ANY, in names: gemm_ragged's 64 x 64 and 128 x 128 tiles (gemm_ragged_plan), and the ones that go by element.
+// The kernels behind ROUTE_ANY, in names: gemm_ragged's tiles and splits of K (gemm_ragged_plan; the smaller two are not named), and the ones that go by element.
 static void any_name(const char* tn, const RaggedPlan& pl, char* out, size_t out_len) {
   if (pl.nsplit > 1) snprintf(out, out_len, "gemm_any<%s,splitK=%d>", tn, pl.nsplit);
   else snprintf(out, out_len, "gemm_any<%s%s>", tn, pl.tile == 128 ? ",128x128" : pl.tile ? "" : ",by element");
