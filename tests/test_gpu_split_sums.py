@@ -54,3 +54,15 @@ def test_last_step(hip, bmnk, dtype, rhs_nk, lhs_mk):
 @pytest.mark.parametrize("lhs_mk", [True, False], ids=["rows", "transposed"])
 def test_small_tiles(hip, bmnk, dtype, rhs_nk, lhs_mk):
     products.test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk)
+
+
+# aligned products of few tiles: on either side of where the kernel with larger tiles takes over (steps of K in all tiles; 32 tiles and K; 255 tiles and 256), small integers exactly
+@pytest.mark.parametrize("bmnk, small", [((1, 64, 64, 4096), True), ((1, 64, 64, 4128), False), ((1, 64, 2048, 2048), True), ((1, 64, 2112, 2048), False), ((8, 192, 64, 320), True),
+                                         ((1, 512, 512, 512), True), ((1, 576, 1600, 1024), True), ((1, 576, 1600, 1056), False), ((255, 64, 64, 64), True), ((256, 64, 64, 64), False)])
+@pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
+def test_aligned_products_of_few_tiles(hip, bmnk, small, rhs_nk):
+    b, m, n, k = bmnk
+    a, w = np.floor(products.rng.uniform_pm1(1, b * m * k) * 4).reshape(b, m, k), np.floor(products.rng.uniform_pm1(2, b * k * n) * 4).reshape(b, k, n)
+    got = products._raw_matmul(hip, ug_amd.F32, a, w, rhs_nk)
+    assert ug_amd.last_kernel().startswith("gemm_any<") == (small and not rhs_nk), ug_amd.last_kernel()
+    np.testing.assert_array_equal(got, np.matmul(a.astype(np.float32), w.astype(np.float32)))  # sums below 2^24: exact in any order

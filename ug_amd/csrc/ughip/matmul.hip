@@ -473,6 +473,19 @@ static int matmul_x6_plan(const MMArgs& p, size_t b, size_t lhs_offset, size_t r
   if (best && out) *out = q;
   return best;
 }
+// f32 products against a [k, n]-major rhs that gemm_tiled takes as well, but with tiles of 128 x 64 and more that leave most CUs idle or make it split K early:
+// gemm_ragged's 32 x 32 and 64 x 64 tiles are faster.  Measured, us gemm_tiled / gemm_ragged: 128^3 8.0 / 5.6, 256^3 10.2 / 5.5, 8 of 192 x 64 x 320 12.0 / 5.4, 384 x 832 x 576 14.0 /
+// 10.5, 512^3 12.6 / 6.3, 192 x 1024 x 1024 15.1 / 9.4, 1024 x 512 x 1024 20.1 / 13.8, 960 x 1024 x 768 25.5 / 18.0, 704 x 832 x 1536 29.3 / 26.1, 64 x 2048 x 4096 26.0 / 17.7, 64^2 x
+// 4096 19.0 / 10.4; 640 x 1280 x 4096 75.9 / 78.1: up to some 7000 steps of 32 in all tiles of 64 x 64, and with a long K few tiles only.  [n, k]-major products gain as much
+// but keep the order of their sums: the one with a bf16 matrix, which only gemm_tiled takes, has the same bits.
+static bool better_in_small_tiles(const MMArgs& p, size_t b) {
+  long long set = 0;
+  if (p.b_cs != 1 || p.b_rs == 1 || tune_get(TUNE_GEMM_SHAPE, &set) || tune_get(TUNE_GEMM_SPLIT, &set) || tune_on(TUNE_GEMM_4WAVES)) return false;
+  const size_t tiles = b * ((p.M + 63) / 64) * ((p.N + 63) / 64), steps = (p.K + 31) / 32;
+  if (tiles >= 256 || !gemm_ragged_plan(UGHIP_F32, p, b).tile) return false;
+  return p.K < 2048 ? tiles * steps <= 7200 : tiles <= 32 && p.K <= 4096;
+}
+
 static Route matmul_route(int dtype, bool mixed, const MMArgs& p, size_t b, size_t lhs_offset, size_t rhs_offset, int* dma_tile, bool allow_x6 = true) {
   const size_t m = (size_t)p.M, n = (size_t)p.N, k = (size_t)p.K;
   const bool f32 = dtype == UGHIP_F32;
@@ -497,7 +510,7 @@ static Route matmul_route(int dtype, bool mixed, const MMArgs& p, size_t b, size
       return ROUTE_X6;
     }
   if (f32 && !mixed && gemm_dma_f32_pick(p, b)) return ROUTE_DMA_F32;
-  return gemm_tiled_supported(dtype, p, b, mixed) ? ROUTE_TILED : ROUTE_ANY;
+  return gemm_tiled_supported(dtype, p, b, mixed) && !(f32 && !mixed && better_in_small_tiles(p, b)) ? ROUTE_TILED : ROUTE_ANY;
 }
 
 // The kernels behind ROUTE_ANY, in names: gemm_ragged's tiles and splits of K (gemm_ragged_plan; the smaller two are not named), and the ones that go by element.
