@@ -1618,10 +1618,16 @@ class Lowering {
     else o << pad << "const int ug_i = ug_g;\n";
   }
 
-  // The place of a load or store inside loop `l` that runs along the row; false: it does not step by one element there, or depends on other loops.
+  // The loops that run along the row: the column loop and the reductions'.
+  bool along_row(int l) const {
+    return l == cols_[0] || std::any_of(regions_.begin(), regions_.end(), [l](const Region& r) { return r.loop == l; });
+  }
+
+  // The place of a load or store inside loop `l`; false: that loop does not run along the row (a value per row, loaded in the row loop, may step by one
+  // there), the access does not step by one element in it, or it depends on other loops.
   bool place_of(int i, int l, Held* h) const {
     const Aff a = aff_of(I_[i].a);
-    if (!a.ok || guarded_[i]) return false;
+    if (!a.ok || guarded_[i] || !along_row(l)) return false;
     h->arg = arg_of_[I_[i].v];
     h->c = a.c;
     h->row.clear();
