@@ -178,10 +178,8 @@ int ughip_compile(ughip_device* dev, const ughip_ssa* ssa, const char* name, ugh
 /* Two row kernels that run one behind the other, as one launch: every row of `second` reads of the
  * result of `first` (its argument `link`) only its own row, and that row stays in registers.
  * shared[k], one per argument of `second`: the argument of `first` that is the same buffer, or -1.
- * out[0], the pair, takes the arguments of `first`, then those of `second` that are not shared; with
- * keep == 0 `link` is left out of them and never written.  out[0] is NULL when the kernels are not of
- * this form.  out[1] and out[2] are the two by themselves, as ughip_compile gives them, except that
- * beside a pair their code objects are made when they first run (a failure to do so is that run's).
+ * *out takes the arguments of `first`, then those of `second` that are not shared; with keep == 0 `link`
+ * is left out of them and never written.  It is NULL when the kernels are not of this form.
  * names: of the two, either may be NULL. */
 int ughip_compile_rows_pair(ughip_device* dev, const ughip_ssa* first, const ughip_ssa* second, const char* const* names, const int* shared, size_t n_shared, int link, int keep, ughip_func** out);
 /* The pair's HIP source, as ughip_codegen (no device needed); *out_len is 0 when there is none. */

@@ -5,6 +5,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import test_gpu_parity as parity
 import ug_amd
 from ug_amd import LazyBuffer as LB
 from ug_amd import Schedule
@@ -92,6 +93,33 @@ def test_what_others_see_of_the_buffer_between(hip, shape):
     e, out = _parts(x, w, dev=hip)
     Schedule.create([e, out]).compile().run()
     assert np.array_equal(kept, out.data_vec()) and e.realized()
+
+
+@pytest.mark.gpu
+def test_everything_is_compiled_when_compile_returns(hip):
+    """One of a pair's kernels by itself, on the cache that the pair was compiled with: its code is made by compile, not by run."""
+    objects, cache, x = lambda: parity.n_code_objects(hip), ug_amd.CompilationCache(), _x(8, 37, 1234)  # noqa: E731  (a shape of its own: nothing of it is compiled yet)
+    e, out = _parts(x, dev=hip)
+    del e
+    before = objects()
+    pair = Schedule.create_one(out).compile(cache)
+    assert objects() == before + 1 and len(cache) == 1
+    info = pair.funcs()
+    assert len(info) == 2 and all("ug_link" in f["source"] and f["info"]["strategy"] == "row_block" for f in info)
+    for alone in (lambda: _parts(x, dev=hip)[0], lambda: _quotient(hip, x)):
+        lb = alone()
+        cs = Schedule.create_one(lb).compile(cache)
+        compiled = objects()
+        cs.run()
+        assert objects() == compiled > before + 1
+    pair.run()
+    assert objects() == compiled
+    np.testing.assert_allclose(out.data_vec().reshape(x.shape), _softmax(x), rtol=60 * EPS32, atol=1e-30)
+
+
+def _quotient(dev, x):
+    e = LB.copy(np.exp(x), x.shape, dev)
+    return e.binary("div", e.reduce("sum", 1).broadcast(x.shape))
 
 
 @pytest.mark.gpu

@@ -572,7 +572,9 @@ void* ugh_cache_new(void) { return new CompilationCache(); }
 void ugh_cache_free(void* c) { delete static_cast<CompilationCache*>(c); }
 size_t ugh_cache_size(void* c) {
   CompilationCache* cc = static_cast<CompilationCache*>(c);
-  return cc->op_cache.size() + cc->ssa_cache.size();
+  size_t pairs = 0;
+  for (const auto& p : cc->pair_cache) pairs += p.second != nullptr;
+  return cc->op_cache.size() + cc->ssa_cache.size() + pairs;
 }
 int ugh_schedule_compile(void* s, void* cache, void** out) {
   return guard([&] {

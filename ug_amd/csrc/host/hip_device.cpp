@@ -42,13 +42,13 @@ std::shared_ptr<Func> HipDevice::compile(const ssa::Kernel& kernel, const std::s
   return std::make_shared<HipFunc>(f);
 }
 
-std::array<std::shared_ptr<Func>, 3> HipDevice::compile_rows_pair(const ssa::Kernel& first, const ssa::Kernel& second, const std::array<std::string, 2>& names,
-                                                                  const std::vector<int>& shared, int link, bool keep) {
+std::shared_ptr<Func> HipDevice::compile_rows_pair(const ssa::Kernel& first, const ssa::Kernel& second, const std::array<std::string, 2>& names,
+                                                   const std::vector<int>& shared, int link, bool keep) {
   ughip_ssa a = first.wire(), b = second.wire();
   const char* named[2] = {names[0].c_str(), names[1].c_str()};
-  ughip_func* f[3];
-  if (ughip_compile_rows_pair(d_, &a, &b, named, shared.data(), shared.size(), link, keep ? 1 : 0, f)) fail("compile");
-  return {f[0] ? std::make_shared<HipFunc>(f[0]) : nullptr, std::make_shared<HipFunc>(f[1]), std::make_shared<HipFunc>(f[2])};
+  ughip_func* f;
+  if (ughip_compile_rows_pair(d_, &a, &b, named, shared.data(), shared.size(), link, keep ? 1 : 0, &f)) fail("compile");
+  return f ? std::make_shared<HipFunc>(f) : nullptr;
 }
 
 static ughip_slice* raw_slice(const Slice& s) {

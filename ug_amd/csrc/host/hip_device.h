@@ -36,7 +36,7 @@ class HipDevice : public Device {
   void synchronize() override;
   std::shared_ptr<Func> compile(const ssa::Kernel& kernel, const std::string* name) override;
   bool joins_rows() const override { return true; }
-  std::array<std::shared_ptr<Func>, 3> compile_rows_pair(const ssa::Kernel& first, const ssa::Kernel& second, const std::array<std::string, 2>& names, const std::vector<int>& shared, int link, bool keep) override;
+  std::shared_ptr<Func> compile_rows_pair(const ssa::Kernel& first, const ssa::Kernel& second, const std::array<std::string, 2>& names, const std::vector<int>& shared, int link, bool keep) override;
   void run(Func& f, const std::vector<Slice*>& args) override;
   void matmul(Slice& dst, const Slice& lhs, const Slice& rhs, size_t b, size_t m, size_t n, size_t k, const Layout& lhs_l,
               const Layout& rhs_l) override;

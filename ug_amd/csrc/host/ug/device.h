@@ -34,11 +34,11 @@ struct Device {
   virtual std::unique_ptr<Slice> allocate_uninit(DType dtype, size_t len) = 0;
   virtual void synchronize() = 0;
   virtual std::shared_ptr<Func> compile(const ssa::Kernel& kernel, const std::string* name) = 0;
-  // Two kernels and, where the device can run them as one (ughip_compile_rows_pair), that one: {it or nullptr, first, second}.
+  // Two kernels as one launch (ughip_compile_rows_pair); nullptr: they stay two.
   virtual bool joins_rows() const { return false; }
-  virtual std::array<std::shared_ptr<Func>, 3> compile_rows_pair(const ssa::Kernel& first, const ssa::Kernel& second, const std::array<std::string, 2>& names, const std::vector<int>& shared, int link, bool keep) {
-    (void)shared, (void)link, (void)keep;
-    return {nullptr, compile(first, &names[0]), compile(second, &names[1])};
+  virtual std::shared_ptr<Func> compile_rows_pair(const ssa::Kernel& first, const ssa::Kernel& second, const std::array<std::string, 2>& names, const std::vector<int>& shared, int link, bool keep) {
+    (void)first, (void)second, (void)names, (void)shared, (void)link, (void)keep;
+    return nullptr;
   }
   virtual void run(Func& f, const std::vector<Slice*>& args) = 0;
   virtual void matmul(Slice& dst, const Slice& lhs, const Slice& rhs, size_t b, size_t m, size_t n, size_t k, const Layout& lhs_l,

@@ -154,9 +154,7 @@ struct CompiledFunc {
   size_t b = 0, m = 0, n = 0, k = 0;
   bool transpose = false;
   CustomF f;
-  // This kernel and the next as one launch (Device::compile_rows_pair): what run() dispatches in place of both.
-  std::shared_ptr<Func> pair;
-  Args pair_args;
+  bool in_pair = false;  // the second of two kernels that are one launch, which the first is (Device::compile_rows_pair): func and args are its, and run() leaves this one out
 };
 
 struct CompiledSchedule {

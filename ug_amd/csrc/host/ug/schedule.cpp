@@ -254,11 +254,18 @@ CompiledSchedule Schedule::compile_with_cache(CompilationCache& cache, bool pair
   for (size_t i = 0; i < items_.size(); ++i) {
     Args args;
     std::shared_ptr<Func> pair = pairs && device_->joins_rows() && i + 1 < items_.size() ? compile_pair(i, cache, &args) : nullptr;
-    out.funcs.push_back(compile_item(items_[i], cache));
-    if (!pair) continue;
-    out.funcs.back().pair = std::move(pair);
-    out.funcs.back().pair_args = std::move(args);
-    out.funcs.push_back(compile_item(items_[++i], cache));
+    if (!pair) {
+      out.funcs.push_back(compile_item(items_[i], cache));
+      continue;
+    }
+    // Neither kernel by itself is compiled or goes into the cache: a later schedule that has one alone compiles it then, and run() never does.
+    out.funcs.push_back({});
+    out.funcs.back().kind = CompiledFunc::Kernel;
+    out.funcs.back().func = pair;
+    out.funcs.back().args = std::move(args);
+    out.funcs.push_back(out.funcs.back());
+    out.funcs.back().in_pair = true;
+    ++i;
   }
   return out;
 }
@@ -330,10 +337,7 @@ std::shared_ptr<Func> Schedule::compile_pair(size_t first, CompilationCache& cac
   auto it = cache.pair_cache.find(key);
   if (it == cache.pair_cache.end()) {
     const std::array<std::string, 2> names{a.ops[0].name(), b.ops[0].name()};
-    auto funcs = device_->compile_rows_pair(a.optimize().lower(op::Opts()), b.optimize().lower(op::Opts()), names, shared, link, keep);
-    cache.op_cache.emplace(key_a, funcs[1]);
-    cache.op_cache.emplace(key_b, funcs[2]);
-    it = cache.pair_cache.emplace(key, funcs[0]).first;
+    it = cache.pair_cache.emplace(key, device_->compile_rows_pair(a.optimize().lower(op::Opts()), b.optimize().lower(op::Opts()), names, shared, link, keep)).first;
   }
   if (!it->second) return nullptr;
   for (size_t k = 0; k < n_first; ++k)
@@ -419,12 +423,8 @@ CompiledFunc Schedule::compile_item(const ScheduleItem& item, CompilationCache& 
 }
 
 void CompiledSchedule::allocate_all() const {
-  for (size_t i = 0; i < funcs.size(); ++i) {
-    const CompiledFunc& f = funcs[i];
-    if (f.pair) {
-      for (const auto& a : f.pair_args) a.second.maybe_allocate_uninit();
-      ++i;
-    } else if (f.kind == CompiledFunc::MatMul) {
+  for (const CompiledFunc& f : funcs) {
+    if (f.kind == CompiledFunc::MatMul) {
       f.dst.maybe_allocate_uninit();
       f.lhs.maybe_allocate_uninit();
       f.rhs.maybe_allocate_uninit();
@@ -435,30 +435,9 @@ void CompiledSchedule::allocate_all() const {
 }
 
 // schedule.rs:234-305
-// The slices of a launch's arguments, allocated where that is left to do.
-static void borrow(const Args& args, std::vector<Slice*>& bs) {
-  bs.clear();
-  for (const auto& a : args) {
-    a.second.maybe_allocate_uninit();
-    // RefCell::try_borrow_mut: a cell may appear once.
-    Slice* s = a.second.data()->slice.get();
-    for (Slice* seen : bs)
-      if (seen == s) bail("already borrowed: BorrowMutError");
-    bs.push_back(s);
-  }
-}
-
 void CompiledSchedule::run() const {
-  thread_local std::vector<Slice*> bs;
-  for (size_t i = 0; i < funcs.size(); ++i) {
-    if (!funcs[i].pair) {
-      run_one(funcs[i]);
-      continue;
-    }
-    borrow(funcs[i].pair_args, bs);
-    device->run(*funcs[i].pair, bs);
-    ++i;
-  }
+  for (const CompiledFunc& f : funcs)
+    if (!f.in_pair) run_one(f);
 }
 
 void CompiledSchedule::run_one(const CompiledFunc& f) const {
@@ -467,7 +446,15 @@ void CompiledSchedule::run_one(const CompiledFunc& f) const {
     switch (f.kind) {
       case CompiledFunc::Kernel:
       case CompiledFunc::Custom: {
-        borrow(f.args, bs);
+        bs.clear();
+        for (const auto& a : f.args) {
+          a.second.maybe_allocate_uninit();
+          // RefCell::try_borrow_mut: a cell may appear once.
+          Slice* s = a.second.data()->slice.get();
+          for (Slice* seen : bs)
+            if (seen == s) bail("already borrowed: BorrowMutError");
+          bs.push_back(s);
+        }
         if (f.kind == CompiledFunc::Kernel) device->run(*f.func, bs);
         else (*f.f)(bs);
         break;

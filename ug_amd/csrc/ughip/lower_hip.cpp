@@ -1731,16 +1731,17 @@ class Lowering {
 
 }  // namespace
 
-bool lower_rows_pair(const ughip_ssa& first, const ughip_ssa& second, const std::string entries[3], const int* shared, int link, bool keep, Lowered* out, Lowered parts[2]) {
+bool lower_rows_pair(const ughip_ssa& first, const ughip_ssa& second, const std::string& entry, const int* shared, int link, bool keep, Lowered* out) {
   for (const ughip_ssa* ssa : {&first, &second})
     if (!ssa->instrs || (!ssa->args && ssa->n_args)) throw std::runtime_error("ssa lowering: null instrs/args");
-  Lowering a(first, entries[1], false), b(second, entries[2], false);
-  parts[0] = a.run(), parts[1] = b.run();
-  const Lowered &la = parts[0], &lb = parts[1];
-  const std::string& entry = entries[0];
+  Lowering a(first, entry, false), b(second, entry, false);
+  const Lowered la = a.run();
+  const Lowering::RowsForm* fa = a.rows_form();
+  if (!fa) return false;
+  const Lowered lb = b.run();
+  const Lowering::RowsForm* fb = b.rows_form();
   b.rename("w");
-  const Lowering::RowsForm *fa = a.rows_form(), *fb = b.rows_form();
-  if (!fa || !fb || fa->nr != fb->nr || fa->width != fb->width || fa->trips != fb->trips || link < 0 || link >= (int)first.n_args || !la.arg_written[link]) return false;
+  if (!fb || fa->nr != fb->nr || fa->width != fb->width || fa->trips != fb->trips || link < 0 || link >= (int)first.n_args || !la.arg_written[link]) return false;
   int link_b = -1;
   for (size_t k = 0; k < second.n_args; ++k) {
     if (shared[k] < 0) continue;

@@ -36,8 +36,8 @@ Lowered lower_ssa(const ughip_ssa& ssa, const std::string& entry, bool as_writte
 // Two row kernels run one behind the other as one: every row of the second reads of the first's result only its own row, which stays in
 // registers.  shared[k]: the first kernel's argument that the second's k-th is, or -1; link: the first kernel's argument that lies between
 // them.  The arguments are the first kernel's, then those of the second's that are not shared; without keep the link is not among them and
-// never written.  false: the kernels are not of this form (nothing is wrong with them).  parts: the two as lower_ssa gives them, either way.
-bool lower_rows_pair(const ughip_ssa& first, const ughip_ssa& second, const std::string entries[3], const int* shared, int link, bool keep, Lowered* out, Lowered parts[2]);
+// never written.  false: the kernels are not of this form (nothing is wrong with them).
+bool lower_rows_pair(const ughip_ssa& first, const ughip_ssa& second, const std::string& entry, const int* shared, int link, bool keep, Lowered* out);
 
 const char* dtype_c_name(int dtype);
 size_t dtype_size(int dtype);

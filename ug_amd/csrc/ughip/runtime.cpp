@@ -55,8 +55,7 @@ using namespace ughip;
 struct ughip_func {
   ughip_device* dev = nullptr;
   Lowered low;
-  std::atomic<hipFunction_t> function{nullptr};  // set last: null until the code is compiled
-  hipFunction_t function2 = nullptr;
+  hipFunction_t function = nullptr, function2 = nullptr;
   void* scratch_part = nullptr;
 };
 
@@ -411,32 +410,28 @@ int ughip_rtc_check(const char* source, const char* arch, size_t* code_size) {
   return UGHIP_OK;
 }
 
-// The code object of a lowered func, compiled unless the device has it already.  The caller holds dev->mu.
-static int load_code(ughip_device* dev, ughip_func* f) {
-  auto it = dev->modules.find(f->low.source);
-  if (it == dev->modules.end()) {
-    std::vector<char> code;
-    if (int rc = rtc_compile(f->low.source, dev->arch, &code)) return rc;
-    CachedModule cm;
-    HIPCHK(hipModuleLoadData(&cm.module, code.data()));
-    hipError_t e = hipModuleGetFunction(&cm.function, cm.module, f->low.entry.c_str());
-    if (e == hipSuccess && !f->low.entry2.empty()) e = hipModuleGetFunction(&cm.function2, cm.module, f->low.entry2.c_str());
-    if (e != hipSuccess) {
-      hipModuleUnload(cm.module);
-      return set_error(UGHIP_ERR_HIP, "hipModuleGetFunction(%s): %s", f->low.entry.c_str(), hipGetErrorString(e));
-    }
-    it = dev->modules.emplace(f->low.source, cm).first;
-  }
-  f->function2 = it->second.function2;
-  f->function.store(it->second.function, std::memory_order_release);
-  return UGHIP_OK;
-}
-
-static int finish_func(ughip_device* dev, std::unique_ptr<ughip_func> f, bool deferred, ughip_func** out) {
+// A func for what `f->low` holds: its code object, compiled unless the device has it already, and its scratch.
+static int finish_func(ughip_device* dev, std::unique_ptr<ughip_func> f, ughip_func** out) {
+  f->dev = dev;
   if (f->low.grid == 0) f->low.empty_launch = true;
-  if (!f->low.empty_launch && !deferred) {
+  if (!f->low.empty_launch) {
     std::lock_guard<std::mutex> g(dev->mu);
-    if (int rc = load_code(dev, f.get())) return rc;
+    auto it = dev->modules.find(f->low.source);
+    if (it == dev->modules.end()) {
+      std::vector<char> code;
+      if (int rc = rtc_compile(f->low.source, dev->arch, &code)) return rc;
+      CachedModule cm;
+      HIPCHK(hipModuleLoadData(&cm.module, code.data()));
+      hipError_t e = hipModuleGetFunction(&cm.function, cm.module, f->low.entry.c_str());
+      if (e == hipSuccess && !f->low.entry2.empty()) e = hipModuleGetFunction(&cm.function2, cm.module, f->low.entry2.c_str());
+      if (e != hipSuccess) {
+        hipModuleUnload(cm.module);
+        return set_error(UGHIP_ERR_HIP, "hipModuleGetFunction(%s): %s", f->low.entry.c_str(), hipGetErrorString(e));
+      }
+      it = dev->modules.emplace(f->low.source, cm).first;
+    }
+    f->function = it->second.function;
+    f->function2 = it->second.function2;
   }
   if (f->low.scratch_part_bytes) HIPCHK(hipMalloc(&f->scratch_part, f->low.scratch_part_bytes));
   ughip_device_retain(dev);
@@ -448,18 +443,16 @@ int ughip_compile(ughip_device* dev, const ughip_ssa* ssa, const char* name, ugh
   if (!dev || !out) return set_error(UGHIP_ERR_INVALID, "null device/out");
   if (int rc = device_activate(dev)) return rc;
   std::unique_ptr<ughip_func> f(new ughip_func);
-  f->dev = dev;
   if (int rc = lower_checked(ssa, name, &f->low)) return rc;
-  return finish_func(dev, std::move(f), false, out);
+  return finish_func(dev, std::move(f), out);
 }
 
-static int lower_pair_checked(const ughip_ssa* first, const ughip_ssa* second, const char* const* names, const int* shared, size_t n_shared, int link, int keep, Lowered* low, Lowered parts[2], bool* taken) {
+static int lower_pair_checked(const ughip_ssa* first, const ughip_ssa* second, const char* const* names, const int* shared, size_t n_shared, int link, int keep, Lowered* low, bool* taken) {
   *taken = false;
   if (!first || !second || !names) return set_error(UGHIP_ERR_INVALID, "rows pair: null argument");
   if (n_shared != second->n_args || (n_shared && !shared)) return set_error(UGHIP_ERR_INVALID, "rows pair: the second kernel has %zu arguments, %zu given", second->n_args, n_shared);
   try {
-    const std::string a = sanitize_name(names[0]), b = sanitize_name(names[1]), entries[3] = {a + "_then_" + b, a, b};
-    *taken = lower_rows_pair(*first, *second, entries, shared, link, keep != 0, low, parts);
+    *taken = lower_rows_pair(*first, *second, sanitize_name(names[0]) + "_then_" + sanitize_name(names[1]), shared, link, keep != 0, low);
   } catch (const std::exception& e) {
     return set_error(UGHIP_ERR_COMPILE, "%s", e.what());
   }
@@ -467,9 +460,9 @@ static int lower_pair_checked(const ughip_ssa* first, const ughip_ssa* second, c
 }
 
 int ughip_codegen_rows_pair(const ughip_ssa* first, const ughip_ssa* second, const char* const* names, const int* shared, size_t n_shared, int link, int keep, char* buf, size_t buf_len, size_t* out_len) {
-  Lowered low, parts[2];
+  Lowered low;
   bool taken;
-  if (int rc = lower_pair_checked(first, second, names, shared, n_shared, link, keep, &low, parts, &taken)) return rc;
+  if (int rc = lower_pair_checked(first, second, names, shared, n_shared, link, keep, &low, &taken)) return rc;
   if (out_len) *out_len = low.source.size();
   if (buf && buf_len) {
     size_t n = std::min(buf_len - 1, low.source.size());
@@ -481,22 +474,12 @@ int ughip_codegen_rows_pair(const ughip_ssa* first, const ughip_ssa* second, con
 
 int ughip_compile_rows_pair(ughip_device* dev, const ughip_ssa* first, const ughip_ssa* second, const char* const* names, const int* shared, size_t n_shared, int link, int keep, ughip_func** out) {
   if (!dev || !out) return set_error(UGHIP_ERR_INVALID, "null device/out");
-  out[0] = out[1] = out[2] = nullptr;
+  *out = nullptr;
   if (int rc = device_activate(dev)) return rc;
-  std::unique_ptr<ughip_func> f[3];
-  for (auto& x : f) x.reset(new ughip_func), x->dev = dev;
-  Lowered parts[2];
+  std::unique_ptr<ughip_func> f(new ughip_func);
   bool taken;
-  if (int rc = lower_pair_checked(first, second, names, shared, n_shared, link, keep, &f[0]->low, parts, &taken)) return rc;
-  f[1]->low = std::move(parts[0]), f[2]->low = std::move(parts[1]);
-  for (int i = 0; i < 3; ++i) {
-    if (i == 0 && !taken) continue;
-    const int rc = finish_func(dev, std::move(f[i]), taken && i != 0, &out[i]);
-    if (rc == UGHIP_OK) continue;
-    for (int k = 0; k < i; ++k) ughip_func_release(out[k]), out[k] = nullptr;
-    return rc;
-  }
-  return UGHIP_OK;
+  if (int rc = lower_pair_checked(first, second, names, shared, n_shared, link, keep, &f->low, &taken)) return rc;
+  return taken ? finish_func(dev, std::move(f), out) : UGHIP_OK;
 }
 
 int ughip_compile_source(ughip_device* dev, const char* source, const char* entry, size_t n_args, const int* arg_dtypes, unsigned grid_dim,
@@ -538,7 +521,7 @@ int ughip_compile_source(ughip_device* dev, const char* source, const char* entr
       }
       it = dev->modules.emplace(key, cm).first;
     }
-    f->function.store(it->second.function);
+    f->function = it->second.function;
   }
   ughip_device_retain(dev);
   *out = f.release();
@@ -606,13 +589,8 @@ static int run_impl(ughip_device* dev, ughip_func* f, ughip_slice* const* args, 
   if (low.scratch_part_bytes) params[np++] = &f->scratch_part;
   if (!low.kparams.empty()) params[np++] = const_cast<int*>(low.kparams.data());
   if (int rc = device_activate(dev)) return rc;
-  if (!f->function.load(std::memory_order_acquire)) {  // (a part of a pair that has not run by itself yet)
-    std::lock_guard<std::mutex> g(dev->mu);
-    if (!f->function.load(std::memory_order_acquire))
-      if (int rc = load_code(dev, f)) return rc;
-  }
-  if (which != 2) HIPCHK(hipModuleLaunchKernel(f->function.load(std::memory_order_relaxed), low.grid, 1, 1, low.block, 1, 1, low.lds_bytes, dev->stream, params, nullptr));
-  if (!low.entry2.empty() && which != 1) HIPCHK(hipModuleLaunchKernel(f->function2, low.grid2, 1, 1, low.block2, 1, 1, 0, dev->stream, params, nullptr));
+  if (which != 2) HIPCHK(hipModuleLaunchKernel(f->function, low.grid, 1, 1, low.block, 1, 1, low.lds_bytes, dev->stream, params, nullptr));
+  if (f->function2 && which != 1) HIPCHK(hipModuleLaunchKernel(f->function2, low.grid2, 1, 1, low.block2, 1, 1, 0, dev->stream, params, nullptr));
   return UGHIP_OK;
 }
 
