@@ -31,6 +31,13 @@ def _parts(x, weight=None, dev=None):
     return e, out if weight is None else out.binary("mul", wide(LB.copy(weight, (1,) * (len(x.shape) - 1) + weight.shape, dev)))
 
 
+def _bare(*buffers):
+    """The same buffers without the operands that their Python objects hold: only the graph does then."""
+    for b in buffers:
+        b._keep = [k for k in b._keep if not isinstance(k, LB)]
+    return buffers
+
+
 def _joined(lb, keep=0):
     """The source of the first two items of a graph as one launch, '' where they stay two; needs no device."""
     s = Schedule.create_one(lb)
@@ -84,7 +91,7 @@ def test_what_others_see_of_the_buffer_between(hip, shape):
     assert e.realized()
     np.testing.assert_allclose(e.data_vec().reshape(shape), np.exp(x.astype(np.float64) - x.max(-1, keepdims=True)), rtol=40 * EPS32)
     kept = out.data_vec()
-    e, out = _parts(x, w, dev=hip)
+    e, out = _bare(*_parts(x, w, dev=hip))
     del e
     Schedule.create_one(out).compile().run()
     assert np.array_equal(kept, out.data_vec())
@@ -99,7 +106,7 @@ def test_what_others_see_of_the_buffer_between(hip, shape):
 def test_everything_is_compiled_when_compile_returns(hip):
     """One of a pair's kernels by itself, on the cache that the pair was compiled with: its code is made by compile, not by run."""
     objects, cache, x = lambda: parity.n_code_objects(hip), ug_amd.CompilationCache(), _x(8, 37, 1234)  # noqa: E731  (a shape of its own: nothing of it is compiled yet)
-    e, out = _parts(x, dev=hip)
+    e, out = _bare(*_parts(x, dev=hip))
     del e
     before = objects()
     pair = Schedule.create_one(out).compile(cache)
@@ -120,6 +127,87 @@ def test_everything_is_compiled_when_compile_returns(hip):
 def _quotient(dev, x):
     e = LB.copy(np.exp(x), x.shape, dev)
     return e.binary("div", e.reduce("sum", 1).broadcast(x.shape))
+
+
+def _reads(dev):
+    """Who may come to see the buffer between a softmax's kernels: name -> (what to schedule from (e, out), what holds it beside that, what it should
+    read of the exponentials)."""
+    shape, w = (5, 6), _x(9, 6, 3)
+    ones = LB.copy(np.ones(shape, np.float32), shape, dev)
+    return {
+        "a handle": (lambda e, out: [out], lambda e: e, lambda e: e),
+        "a sibling": (lambda e, out: [out], lambda e: e.binary("add", ones), lambda e: e + 1),
+        "a sibling's sibling": (lambda e, out: [out], lambda e: e.binary("mul", ones).unary("neg").reduce("sum", 1), lambda e: np.broadcast_to(-e.sum(1, keepdims=True), shape)),
+        "a reshape": (lambda e, out: [out], lambda e: e.reshape((30,)), lambda e: e.reshape(30)),
+        "a view": (lambda e, out: [out], lambda e: e.narrow(1, 2, 3), lambda e: e[:, 2:5]),
+        "an output": (lambda e, out: [e, out], None, None),
+        "a later kernel": (lambda e, out: [out, e.reduce("sum", 0)], None, None),
+        "a product": (lambda e, out: [out, e.matmul(LB.copy(w, w.shape, dev))], None, None),
+        "a product held elsewhere": (lambda e, out: [out], lambda e: e.matmul(LB.copy(w, w.shape, dev)), lambda e: e @ w),
+        "a custom op": (lambda e, out: [out, LB.custom(lambda s: s[1].copy_host_to_device(s[0].to_vec()), [e], shape, ug_amd.F32, dev)], None, None),
+        "another schedule": (lambda e, out: [out], lambda e: Schedule.create_one(e.binary("add", ones)), None),
+    }
+
+
+READS = ["a handle", "a sibling", "a sibling's sibling", "a reshape", "a view", "an output", "a later kernel", "a product", "a product held elsewhere", "a custom op", "another schedule"]
+
+
+def _read(dev, name):
+    make, hold, _ = _reads(dev)[name]
+    e, out = _parts(_x(6, 5, 6), dev=dev)
+    roots = make(e, out)
+    held = hold(e) if hold else None
+    _bare(*[b for b in [e, out, held, *roots] if isinstance(b, LB)])
+    if isinstance(held, Schedule):
+        _bare(*held._keep)
+        held._keep = []
+    del e
+    s = Schedule.create(roots)
+    return s, roots, held
+
+
+@pytest.mark.parametrize("name", READS)
+def test_a_buffer_that_somebody_can_reach_is_written(cpu, name):
+    s, roots, held = _read(cpu, name)
+    assert s.pair(0) is True
+
+
+def test_a_buffer_that_nobody_can_reach_is_not_written(cpu):
+    for weight in (None, _x(1, 6)):
+        e, out = _bare(*_parts(_x(6, 5, 6), weight, cpu))
+        del e
+        s = Schedule.create_one(out)
+        assert s.pair(0) is False and s.pair(1) is None
+        compiled = s.compile()
+        assert s.pair(0) is True    # (this device's two launches hold it)
+        del compiled
+        assert s.pair(0) is False
+    # one behind the other
+    [out] = _bare(ug_amd.llama.softmax(ug_amd.llama.softmax(LB.copy(_x(6, 5, 6), (5, 6), cpu))))
+    s = Schedule.create_one(out)
+    assert [s.pair(i) for i in range(len(s.items()))] == [False, False, False, None]
+    # kernels without a reduction are not row kernels
+    e = LB.copy(_x(1, 4, 8), (4, 8), cpu).unary("exp")
+    out = e.binary("mul", e)
+    s = Schedule.create_one(out)
+    assert [s.pair(i) for i in range(len(s.items()))] == [None] * len(s.items())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", READS)
+def test_everybody_sees_what_is_between(hip, name):
+    s, roots, held = _read(hip, name)
+    cs = s.compile()
+    assert "ug_link" in cs.funcs()[0]["source"]
+    cs.run()
+    x = _x(6, 5, 6).astype(np.float64)
+    e = np.exp(x - x.max(-1, keepdims=True))
+    want = {"an output": [e, _softmax(x)], "a later kernel": [_softmax(x), np.broadcast_to(e.sum(0), x.shape)], "a product": [_softmax(x), e @ _x(9, 6, 3)], "a custom op": [_softmax(x), e]}.get(name, [_softmax(x)])
+    for got, v in zip(roots, want):
+        np.testing.assert_allclose(got.data_vec().reshape(v.shape), v, rtol=1e-5, atol=1e-6)
+    if _reads(hip)[name][2]:
+        v = _reads(hip)[name][2](e)
+        np.testing.assert_allclose(held.data_vec().reshape(v.shape), v, rtol=1e-5, atol=1e-6)
 
 
 @pytest.mark.gpu

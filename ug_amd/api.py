@@ -655,6 +655,12 @@ class Schedule(_Handle):
         _chk(host_lib().ugh_schedule_item_ssa(_p(self.h), C.c_size_t(i), int(optimize), C.byref(out)))
         return SsaKernel(out.value)
 
+    def pair(self, i):
+        """Whether items i and i + 1 may be one launch as far as the graph says: None, or whether what lies between them would be written."""
+        may, keep = C.c_int(), C.c_int()
+        _chk(host_lib().ugh_schedule_pair(_p(self.h), C.c_size_t(i), C.byref(may), C.byref(keep)))
+        return bool(keep.value) if may.value else None
+
     def compile(self, cache=None):
         out = C.c_void_p()
         _chk(host_lib().ugh_schedule_compile(_p(self.h), _p(cache.h) if cache is not None else None, C.byref(out)))

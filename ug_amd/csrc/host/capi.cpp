@@ -568,12 +568,20 @@ int ugh_schedule_item_ssa(void* s, size_t i, int optimize, void** out) {
     *out = new ssa::Kernel(k.lower(op::Opts()));
   });
 }
+// Whether items i and i + 1 may be one launch as far as the graph says, and whether what lies between them would be written.
+int ugh_schedule_pair(void* s, size_t i, int* may, int* keep) {
+  return guard([&] {
+    const Schedule& sc = *static_cast<Schedule*>(s);
+    *may = sc.pair_at(i) ? 1 : 0;
+    *keep = *may && !sc.only_between(i, sc.holders()) ? 1 : 0;
+  });
+}
 void* ugh_cache_new(void) { return new CompilationCache(); }
 void ugh_cache_free(void* c) { delete static_cast<CompilationCache*>(c); }
 size_t ugh_cache_size(void* c) {
   CompilationCache* cc = static_cast<CompilationCache*>(c);
   size_t pairs = 0;
-  for (const auto& p : cc->pair_cache) pairs += p.second != nullptr;
+  for (const auto& p : cc->pair_cache) pairs += (p.second.func[0] != nullptr) + (p.second.func[1] != nullptr);
   return cc->op_cache.size() + cc->ssa_cache.size() + pairs;
 }
 int ugh_schedule_compile(void* s, void* cache, void** out) {

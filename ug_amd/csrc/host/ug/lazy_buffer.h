@@ -3,6 +3,7 @@
 #include <functional>
 #include <map>
 #include <memory>
+#include <optional>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -142,7 +143,12 @@ struct ScheduleItem {
 // cache.rs:74-101
 struct CompilationCache {
   std::unordered_map<std::string, std::shared_ptr<Func>> op_cache, ssa_cache;
-  std::unordered_map<std::string, std::shared_ptr<Func>> pair_cache;  // null: these two kernels do not run as one
+  // Two kernels as one launch, without and with what lies between them written; each made when it is first wanted.
+  struct Pair {
+    bool stays_two = false;
+    std::shared_ptr<Func> func[2];
+  };
+  std::unordered_map<std::string, Pair> pair_cache;
 };
 
 // schedule.rs:210-306
@@ -184,10 +190,25 @@ class Schedule {
   CompiledSchedule compile_and_run(CompilationCache& cache) const;
   const LazyBuffer& get_arg_id(ArgId id) const;
 
+  // Items `first` and `first + 1` as far as the graph says whether they may be one launch: row kernels of which the second reads what the first stores
+  // (its argument `link`); shared: per argument of the second the first's that is the same storage, or -1.
+  struct RowsPair {
+    int link = -1;
+    std::vector<int> shared;
+  };
+  std::optional<RowsPair> pair_at(size_t first) const;
+  // Handles per buffer, and the first and the last item that names it.
+  struct Holders {
+    std::unordered_map<const LazyBufferInner*, long> handles;
+    std::unordered_map<const LazyBufferInner*, std::pair<size_t, size_t>> items;
+  };
+  Holders holders() const;
+  bool only_between(size_t first, const Holders& h) const;
+
  private:
-  CompiledFunc compile_item(const ScheduleItem& item, CompilationCache& cache) const;
-  std::shared_ptr<Func> compile_pair(size_t first, CompilationCache& cache, Args* args) const;
-  bool only_between(const LazyBuffer& b, size_t first) const;
+  struct Prepared;
+  CompiledFunc compile_item(const ScheduleItem& item, CompilationCache& cache, Prepared* prepared) const;
+  bool compile_pair(size_t first, CompilationCache& cache, std::vector<Prepared>& prepared, std::optional<Holders>& held, CompiledFunc* out) const;
   std::vector<ScheduleItem> items_;
   std::map<size_t, LazyBuffer> per_arg_id_;
   DevicePtr device_;

@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <set>
 #include <unordered_map>
+#include <unordered_set>
 
 #include "lazy_buffer.h"
 
@@ -247,104 +248,155 @@ const LazyBuffer& Schedule::get_arg_id(ArgId id) const {
   return it->second;
 }
 
+// A kernel item's lowered forms, each made when it is first asked for.
+struct Schedule::Prepared {
+  std::optional<op::Kernel> kernel;
+  std::string key;
+  std::optional<ssa::Kernel> ssa;
+  void of(const ScheduleItem& item) {
+    if (kernel) return;
+    kernel = item.kernel.kernel();
+    key = normalized_kernel_key(*kernel);
+  }
+  const ssa::Kernel& serial() {
+    if (!ssa) ssa = kernel->optimize().lower(op::Opts());
+    return *ssa;
+  }
+};
+
 // schedule.rs:115-207
 CompiledSchedule Schedule::compile_with_cache(CompilationCache& cache, bool pairs) const {
   CompiledSchedule out;
   out.device = device_;
+  std::vector<Prepared> prepared(items_.size());
+  std::optional<Holders> holders;
   for (size_t i = 0; i < items_.size(); ++i) {
-    Args args;
-    std::shared_ptr<Func> pair = pairs && device_->joins_rows() && i + 1 < items_.size() ? compile_pair(i, cache, &args) : nullptr;
-    if (!pair) {
-      out.funcs.push_back(compile_item(items_[i], cache));
+    CompiledFunc pair;
+    if (!pairs || !device_->joins_rows() || !compile_pair(i, cache, prepared, holders, &pair)) {
+      out.funcs.push_back(compile_item(items_[i], cache, &prepared[i]));
       continue;
     }
     // Neither kernel by itself is compiled or goes into the cache: a later schedule that has one alone compiles it then, and run() never does.
-    out.funcs.push_back({});
-    out.funcs.back().kind = CompiledFunc::Kernel;
-    out.funcs.back().func = pair;
-    out.funcs.back().args = std::move(args);
-    out.funcs.push_back(out.funcs.back());
-    out.funcs.back().in_pair = true;
+    out.funcs.push_back(pair);
+    pair.in_pair = true;
+    out.funcs.push_back(std::move(pair));
     ++i;
   }
   return out;
 }
 
-// Whether nothing but items `first` and `first + 1` can ever ask for what is in `b`: no other item, no other buffer on the same storage, and
-// every holder of the handle is this schedule or the graph it was made from.  (Handles are only ever copied from handles, so nobody can come
-// by one later.)
-bool Schedule::only_between(const LazyBuffer& b, size_t first) const {
-  if (b.data().use_count() != 1) return false;
-  const LazyBufferInner* wanted = &b.inner();
-  long known = 0;
+// Every handle that this schedule and the graph it was made from hold, counted in one walk.  (Behind buffers that were there already nothing is
+// counted: a buffer that one of those holds is taken for somebody else's too, and written.)
+Schedule::Holders Schedule::holders() const {
+  Holders h;
   std::vector<const LazyBuffer*> todo;
-  std::set<const LazyBufferInner*> seen;
+  std::unordered_set<const LazyBufferInner*> results;
   auto note = [&](const LazyBuffer& x) {
-    if (!x.valid()) return;
-    if (&x.inner() == wanted) ++known;
-    if (seen.insert(&x.inner()).second) todo.push_back(&x);
+    if (x.valid() && ++h.handles[&x.inner()] == 1) todo.push_back(&x);
   };
   for (size_t i = 0; i < items_.size(); ++i) {
     const ScheduleItem& it = items_[i];
-    const long before = known;
-    for (const auto& a : it.kernel.args) note(a.second);
-    for (const auto& a : it.args) note(a.second);
-    for (const LazyBuffer* x : {&it.kernel.dst.second, &it.dst, &it.lhs, &it.rhs}) note(*x);
-    if (known != before && i != first && i != first + 1) return false;
+    auto named = [&](const LazyBuffer& x) {
+      if (!x.valid()) return;
+      note(x);
+      h.items.emplace(&x.inner(), std::make_pair(i, i)).first->second.second = i;
+    };
+    for (const auto& a : it.kernel.args) named(a.second);
+    for (const auto& a : it.args) named(a.second);
+    for (const LazyBuffer* x : {&it.kernel.dst.second, &it.dst, &it.lhs, &it.rhs}) named(*x);
+    for (const LazyBuffer* x : {&it.kernel.dst.second, &it.dst})
+      if (x->valid()) results.insert(&x->inner());
   }
   for (const auto& a : per_arg_id_) note(a.second);
   while (!todo.empty()) {
-    const Op& op = todo.back()->inner().op;
+    const LazyBuffer& x = *todo.back();
     todo.pop_back();
+    if (x.realized() && !results.count(&x.inner())) continue;
+    const Op& op = x.inner().op;
     note(op.arg);
     note(op.arg2);
     for (const LazyBuffer& a : op.args) note(a);
   }
-  return b.use_count() == known;
+  return h;
 }
 
-std::shared_ptr<Func> Schedule::compile_pair(size_t first, CompilationCache& cache, Args* args) const {
+// Whether nothing but items `first` and `first + 1` can ever ask for what the first one stores: no other item, no other buffer on the same storage,
+// and every holder of the handle is this schedule or the graph it was made from.  (Handles are only ever copied from handles, so nobody can come
+// by one later.)
+bool Schedule::only_between(size_t first, const Holders& h) const {
+  const LazyBuffer& b = items_[first].kernel.dst.second;
+  if (b.data().use_count() != 1) return false;
+  const auto at = h.items.find(&b.inner());
+  return at != h.items.end() && at->second.first >= first && at->second.second <= first + 1 && b.use_count() == h.handles.at(&b.inner());
+}
+
+static bool reduces(const op::Ast& a) {
+  switch (a.inner->kind) {
+    case op::AstInner::Reduce: return true;
+    case op::AstInner::Layout:
+    case op::AstInner::Unary: return reduces(a.inner->arg);
+    case op::AstInner::Binary: return reduces(a.inner->arg) || reduces(a.inner->rhs);
+    default: return false;
+  }
+}
+
+std::optional<Schedule::RowsPair> Schedule::pair_at(size_t first) const {
+  if (first + 1 >= items_.size()) return {};
   const ScheduleItem &x = items_[first], &y = items_[first + 1];
-  if (x.kind != ScheduleItem::Kernel || y.kind != ScheduleItem::Kernel || x.kernel.has_dst_layout || y.kernel.has_dst_layout) return nullptr;
+  if (x.kind != ScheduleItem::Kernel || y.kind != ScheduleItem::Kernel || x.kernel.has_dst_layout || y.kernel.has_dst_layout) return {};
   const LazyBuffer& between = x.kernel.dst.second;
-  if (between.elem_count() != y.kernel.dst.second.elem_count() || between.in_place_op() || y.kernel.dst.second.in_place_op()) return nullptr;
+  if (between.elem_count() != y.kernel.dst.second.elem_count() || between.in_place_op() || y.kernel.dst.second.in_place_op()) return {};
+  RowsPair p;
   // arguments by storage; a kernel that names one storage twice is refused when it runs, as ever
-  std::vector<const DataCell*> cells;
-  int link = -1;
-  for (const auto& a : x.kernel.args) {
-    const DataCell* c = a.second.data().get();
-    if (std::find(cells.begin(), cells.end(), c) != cells.end()) return nullptr;
-    if (c == between.data().get()) link = (int)cells.size();
-    cells.push_back(c);
+  const Args &xs = x.kernel.args, &ys = y.kernel.args;
+  const auto at = [](const Args& args, size_t end, const LazyBuffer& b) {
+    size_t i = 0;
+    while (i < end && args[i].second.data() != b.data()) ++i;
+    return i;
+  };
+  if (at(ys, ys.size(), between) == ys.size()) return {};
+  for (size_t i = 0; i < xs.size(); ++i)
+    if (at(xs, i, xs[i].second) < i) return {};
+  const size_t link = at(xs, xs.size(), between);
+  p.link = link < xs.size() ? (int)link : -1;
+  p.shared.reserve(ys.size());
+  for (size_t i = 0; i < ys.size(); ++i) {
+    if (at(ys, i, ys[i].second) < i) return {};
+    const size_t k = at(xs, xs.size(), ys[i].second);
+    p.shared.push_back(k < xs.size() ? (int)k : -1);
   }
-  const size_t n_first = cells.size();
-  std::vector<int> shared;
-  bool linked = false;
-  for (const auto& a : y.kernel.args) {
-    const DataCell* c = a.second.data().get();
-    const size_t at = std::find(cells.begin(), cells.end(), c) - cells.begin();
-    if (at < cells.size() && at >= n_first) return nullptr;
-    shared.push_back(at < n_first ? (int)at : -1);
-    linked |= (int)at == link;
-    if (at == cells.size()) cells.push_back(c);
+  // (row kernels reduce; asked last: it walks the expressions)
+  if (p.link < 0 || !reduces(x.kernel.ast) || !reduces(y.kernel.ast)) return {};
+  return p;
+}
+
+bool Schedule::compile_pair(size_t first, CompilationCache& cache, std::vector<Prepared>& prepared, std::optional<Holders>& held, CompiledFunc* out) const {
+  const std::optional<RowsPair> p = pair_at(first);
+  if (!p) return false;
+  Prepared &x = prepared[first], &y = prepared[first + 1];
+  x.of(items_[first]), y.of(items_[first + 1]);
+  std::string key;
+  key.reserve(x.key.size() + y.key.size() + 32);
+  key.append(x.key).append("\n").append(y.key).append("\n").append(std::to_string(p->link));
+  for (int s : p->shared) key += "," + std::to_string(s);
+  CompilationCache::Pair& known = cache.pair_cache[key];
+  if (known.stays_two) return false;
+  if (!held) held = holders();
+  const bool keep = !only_between(first, *held);
+  std::shared_ptr<Func>& func = known.func[keep];
+  if (!func) func = device_->compile_rows_pair(x.serial(), y.serial(), {x.kernel->ops[0].name(), y.kernel->ops[0].name()}, p->shared, p->link, keep);
+  if (!func) {
+    known.stays_two = true;
+    return false;
   }
-  if (link < 0 || !linked) return nullptr;
-  const bool keep = !only_between(between, first);
-  op::Kernel a = x.kernel.kernel(), b = y.kernel.kernel();
-  const std::string key_a = normalized_kernel_key(a), key_b = normalized_kernel_key(b);
-  std::string key = key_a + "\n" + key_b + "\n" + (keep ? "k" : "") + std::to_string(link);
-  for (int s : shared) key += "," + std::to_string(s);
-  auto it = cache.pair_cache.find(key);
-  if (it == cache.pair_cache.end()) {
-    const std::array<std::string, 2> names{a.ops[0].name(), b.ops[0].name()};
-    it = cache.pair_cache.emplace(key, device_->compile_rows_pair(a.optimize().lower(op::Opts()), b.optimize().lower(op::Opts()), names, shared, link, keep)).first;
-  }
-  if (!it->second) return nullptr;
-  for (size_t k = 0; k < n_first; ++k)
-    if (keep || (int)k != link) args->push_back({x.kernel.args[k].first, get_arg_id(x.kernel.args[k].first)});
-  for (size_t k = 0; k < shared.size(); ++k)
-    if (shared[k] < 0) args->push_back({y.kernel.args[k].first, get_arg_id(y.kernel.args[k].first)});
-  return it->second;
+  out->kind = CompiledFunc::Kernel;
+  out->func = func;
+  const Args &xs = items_[first].kernel.args, &ys = items_[first + 1].kernel.args;
+  for (size_t k = 0; k < xs.size(); ++k)
+    if (keep || (int)k != p->link) out->args.push_back({xs[k].first, get_arg_id(xs[k].first)});
+  for (size_t k = 0; k < ys.size(); ++k)
+    if (p->shared[k] < 0) out->args.push_back({ys[k].first, get_arg_id(ys[k].first)});
+  return true;
 }
 
 CompiledSchedule Schedule::compile_and_run(CompilationCache& cache) const {
@@ -352,13 +404,27 @@ CompiledSchedule Schedule::compile_and_run(CompilationCache& cache) const {
   out.device = device_;
   out.funcs.reserve(items_.size());
   for (const ScheduleItem& item : items_) {
-    out.funcs.push_back(compile_item(item, cache));
+    Prepared prepared;
+    out.funcs.push_back(compile_item(item, cache, &prepared));
     out.run_one(out.funcs.back());
   }
   return out;
 }
 
-CompiledFunc Schedule::compile_item(const ScheduleItem& item, CompilationCache& cache) const {
+// schedule.rs:162-188: grid heuristics, only for devices that ask for them.
+static ssa::Kernel on_a_grid(const op::Kernel& kernel) {
+  op::Opts opts;
+  if (kernel.ops.size() == 1 && kernel.ops[0].layout.rank() >= 1 && kernel.ops[0].layout.num_elements() >= 1) {
+    std::vector<std::pair<size_t, size_t>> dims;
+    for (size_t i = 0; i < kernel.ops[0].layout.rank(); ++i) dims.push_back({i, kernel.ops[0].layout.dims()[i]});
+    std::stable_sort(dims.begin(), dims.end(), [](const auto& a, const auto& b) { return a.second > b.second; });
+    if (dims.size() >= 2 && dims[1].second > 1) opts = op::Opts().with_block_axis(dims[0].first).with_thread_block(dims[1].first, 32);
+    else if (dims.size() > 1 && dims[0].second > 1) opts = op::Opts().with_global_axis(dims[0].first, 32);
+  }
+  return kernel.lower(opts);
+}
+
+CompiledFunc Schedule::compile_item(const ScheduleItem& item, CompilationCache& cache, Prepared* prepared) const {
   {
     CompiledFunc call;
     switch (item.kind) {
@@ -393,8 +459,9 @@ CompiledFunc Schedule::compile_item(const ScheduleItem& item, CompilationCache& 
       }
       case ScheduleItem::Kernel: {
         call.kind = CompiledFunc::Kernel;
-        op::Kernel kernel = item.kernel.kernel();
-        std::string key = normalized_kernel_key(kernel);
+        prepared->of(item);
+        const op::Kernel& kernel = *prepared->kernel;
+        const std::string& key = prepared->key;
         for (const Arg& a : kernel.args) call.args.push_back({a.id, get_arg_id(a.id)});
         auto it = cache.op_cache.find(key);
         if (it != cache.op_cache.end()) {
@@ -402,18 +469,9 @@ CompiledFunc Schedule::compile_item(const ScheduleItem& item, CompilationCache& 
           break;
         }
         std::string kernel_name = kernel.ops.empty() ? "" : kernel.ops[0].name();
-        kernel = kernel.optimize();
-        op::Opts opts;
-        // schedule.rs:162-188: grid heuristics, only for devices that ask for them.
-        if (device_->use_grid() && kernel.ops.size() == 1 && kernel.ops[0].layout.rank() >= 1 && kernel.ops[0].layout.num_elements() >= 1) {
-          std::vector<std::pair<size_t, size_t>> dims;
-          for (size_t i = 0; i < kernel.ops[0].layout.rank(); ++i) dims.push_back({i, kernel.ops[0].layout.dims()[i]});
-          std::stable_sort(dims.begin(), dims.end(), [](const auto& a, const auto& b) { return a.second > b.second; });
-          if (dims.size() >= 2 && dims[1].second > 1) opts = op::Opts().with_block_axis(dims[0].first).with_thread_block(dims[1].first, 32);
-          else if (dims.size() > 1 && dims[0].second > 1) opts = op::Opts().with_global_axis(dims[0].first, 32);
-        }
-        ssa::Kernel ssa = kernel.lower(opts);
-        call.func = device_->compile(ssa, kernel.ops.empty() ? nullptr : &kernel_name);
+        const std::string* name = kernel.ops.empty() ? nullptr : &kernel_name;
+        if (device_->use_grid()) call.func = device_->compile(on_a_grid(kernel.optimize()), name);
+        else call.func = device_->compile(prepared->serial(), name);
         cache.op_cache[key] = call.func;
         break;
       }

@@ -248,7 +248,7 @@ class Lowering {
   const ughip_instr* I_;
   int n_;
   std::string entry_;
-  bool as_written_ = false;
+  bool as_written_ = false, form_only_ = false;
   std::map<int, std::string> held_;  // loads whose element is in a register already, and what it is called
   mutable bool nt_loads_ = false;  // loads of the region being emitted bypass cache allocation
   bool nt_stores_ = false;         // stores to kernel arguments go past the cache (set while an elementwise kernel is emitted)
@@ -890,6 +890,7 @@ class Lowering {
   }
 
   void emit_literal(unsigned grid, unsigned block) {
+    if (form_only_) return;
     if (block > 1024) fail("block_dim > 1024");
     Text o;
     o << kPrelude << "\nextern \"C\" __global__ void __launch_bounds__(" << block << ") " << entry_ << "(" << signature(false) << ") {\n";
@@ -1244,6 +1245,7 @@ class Lowering {
   }
 
   void emit_elementwise(i64 total) {
+    if (form_only_) return;
     const int block = 256;
     i64 inner = chain_.empty() ? 1 : loops_[chain_.back()].trip;
     int vec = inner % 4 == 0 ? 4 : (inner % 2 == 0 ? 2 : 1);
@@ -1287,6 +1289,7 @@ class Lowering {
   }
 
   void emit_row_thread(const std::vector<int>& rows, const std::vector<int>& cols, i64 nr, i64 nc) {
+    if (form_only_) return;
     const int block = 256;
     uint64_t col_mask = 0;
     for (int l : cols) col_mask |= 1ull << l;
@@ -1332,11 +1335,12 @@ class Lowering {
     int block = tpr * rows_per_block;
     if (!grid_reduce) {
       find_rows_form(rows, cols, nr, nc, tpr, rows_per_block);
-      if (rows_ok_) {
+      if (rows_ok_ && !form_only_) {
         emit_rows();
         return;
       }
     }
+    if (form_only_) return;
     Text o;
     o << kPrelude << "\nextern \"C\" __global__ void __launch_bounds__(" << block << ") " << entry_ << "(" << signature(grid_reduce) << ") {\n";
     o << "  const int ug_t = (int)threadIdx.x % " << tpr << ";\n";
@@ -1465,6 +1469,8 @@ class Lowering {
   const std::vector<char>& written() const { return out_.arg_written; }
   const Lowered& lowered() const { return out_; }
   void rename(const std::string& prefix) { vp_ = prefix; }
+  // run() stops at the rows form: for a kernel whose own text nobody wants.
+  void want_form_only() { form_only_ = true; }
   // The one store of argument `arg` as a place; false: there are several, or it is not one element per column.
   bool stored_at(int arg, Held* at) const {
     int found = -1;
@@ -1735,6 +1741,7 @@ bool lower_rows_pair(const ughip_ssa& first, const ughip_ssa& second, const std:
   for (const ughip_ssa* ssa : {&first, &second})
     if (!ssa->instrs || (!ssa->args && ssa->n_args)) throw std::runtime_error("ssa lowering: null instrs/args");
   Lowering a(first, entry, false), b(second, entry, false);
+  a.want_form_only(), b.want_form_only();
   const Lowered la = a.run();
   const Lowering::RowsForm* fa = a.rows_form();
   if (!fa) return false;
