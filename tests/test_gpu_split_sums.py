@@ -47,6 +47,16 @@ def test_last_step(hip, bmnk, dtype, rhs_nk, lhs_mk):
     products.test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk)
 
 
+# one step of K or less on the large tile, whose form has no loop: a few elements, an odd number, a whole step
+@pytest.mark.parametrize("bmnk", [(16, 130, 1023, 9), (16, 130, 1023, 51), (16, 130, 1023, 64)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
+@pytest.mark.parametrize("lhs_mk", [True, False], ids=["rows", "transposed"])
+def test_one_step_on_the_large_tile(hip, bmnk, dtype, rhs_nk, lhs_mk):
+    products.test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk)
+    assert ug_amd.last_kernel() == f"gemm_any<{dtype},128x128>"
+
+
 # 32 x 32 tiles, a few and several to a CU: fewer steps of K than waves, as many, one more, uneven parts and a last wave without one; tiles over both edges; batches
 @pytest.mark.parametrize("bmnk", [(1, 100, 100, 65), (1, 33, 65, 120), (1, 300, 300, 300), (2, 31, 97, 257), (1, 330, 9, 350), (1, 625, 319, 353), (15, 19, 18, 640), (1, 23, 148, 1355), (8, 200, 200, 200)])
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])

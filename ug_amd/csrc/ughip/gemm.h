@@ -106,6 +106,7 @@ struct RaggedPlan {
   size_t ws_bytes = 0;
   static constexpr size_t MAX_WS = (size_t)32 << 20;
 };
+bool gemm_ragged_takes(int dtype, const MMArgs& p, size_t batch);  // whether that plan has a tile
 RaggedPlan gemm_ragged_plan(int dtype, const MMArgs& p, size_t batch);
 hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, const RaggedPlan& plan, float* workspace);
 

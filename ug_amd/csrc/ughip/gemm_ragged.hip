@@ -147,11 +147,15 @@ struct Result { typedef T type; };
 template <typename T>
 struct Result<T, true> { typedef float type; };
 
+// ONE: K is one step or less: loaded by element, one multiplication, no loop.  What bounds it: the launch.  (Going through the code for more steps, us before / so: f16
+// 777 x 1001 x 33 4.7 / 4.3, x 63 5.2 / 4.7, 40 of 130 x 130 x 40 5.7 / 5.2, 2001^2 x 33 9.3 / 8.5; f32 777 x 1001 x 30 5.0 / 4.7.)
 // SPLIT: slab s of nsplit has the steps per * s .. per * (s + 1) - 1 of K, the last one the remainder, and leaves its sums in ws, slab_elems apart.
-template <typename T, int BT, bool A_KC, bool B_KC, bool SPLIT>
+enum Form { ONE, WHOLE, SPLIT_K };
+template <typename T, int BT, bool A_KC, bool B_KC, Form FORM>
 __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int tiles_m, int tiles_n, int nsplit, int per, float* __restrict__ ws, size_t slab_elems) {
   typedef Side<T, BT, A_KC> SA;
   typedef Side<T, BT, B_KC> SB;
+  constexpr bool SPLIT = FORM == SPLIT_K;
   constexpr int MI = BT / 64, KE = SA::KE;
   __shared__ __attribute__((aligned(16))) char lds[2][SA::BYTES + SB::BYTES];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -205,48 +209,53 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
         for (int j = 0; j < MI; ++j) mma(T(), fb[j], fa[i], acc[i][j]);  // swapped: a lane holds columns of one row
     }
   };
-  if (with_left && full > 0) {
+  if constexpr (FORM == ONE) {
 #pragma unroll
-    for (int i = 0; i < SA::N; ++i) la[i] = a.load_end(i, full, left, m0, p.M, tid);
+    for (int i = 0; i < SA::N; ++i) la[i] = a.load_last(i, 0, left, m0, p.M, tid);
 #pragma unroll
-    for (int i = 0; i < SB::N; ++i) lb[i] = b.load_end(i, full, left, n0, p.N, tid);
-  } else if (with_left) {
-#pragma unroll
-    for (int i = 0; i < SA::N; ++i) la[i] = a.load_last(i, full, left, m0, p.M, tid);
-#pragma unroll
-    for (int i = 0; i < SB::N; ++i) lb[i] = b.load_last(i, full, left, n0, p.N, tid);
+    for (int i = 0; i < SB::N; ++i) lb[i] = b.load_last(i, 0, left, n0, p.N, tid);
+    put(lds[0], la, lb);
+    __syncthreads();
+    multiply(lds[0]);
   } else {
+    if (with_left) {
 #pragma unroll
-    for (int i = 0; i < SA::N; ++i) la[i] = a.load(i, begin - 1);
+      for (int i = 0; i < SA::N; ++i) la[i] = a.load_end(i, full, left, m0, p.M, tid);
 #pragma unroll
-    for (int i = 0; i < SB::N; ++i) lb[i] = b.load(i, begin - 1);
+      for (int i = 0; i < SB::N; ++i) lb[i] = b.load_end(i, full, left, n0, p.N, tid);
+    } else {
+#pragma unroll
+      for (int i = 0; i < SA::N; ++i) la[i] = a.load(i, begin - 1);
+#pragma unroll
+      for (int i = 0; i < SB::N; ++i) lb[i] = b.load(i, begin - 1);
+    }
+    if (end > begin) {
+      fetch(0, begin);
+      __builtin_amdgcn_sched_barrier(0);  // (in this order: the loop counts on it)
+      fetch(1, min(begin + 1, end - 1));
+    }
+    if (with_left) {
+#pragma unroll
+      for (int i = 0; i < SA::N; ++i) la[i] = SA::trimmed(la[i], i, left, tid);
+#pragma unroll
+      for (int i = 0; i < SB::N; ++i) lb[i] = SB::trimmed(lb[i], i, left, tid);
+    }
+    put(lds[0], la, lb);
+    __syncthreads();
+    multiply(lds[0]);
+    auto step = [&](int d, int s) {
+      char* buf = lds[d ^ 1];
+      put(buf, ra[d], rb[d]);
+      fetch(d, min(s + 2, end - 1));  // (without a branch, so that a step's loads can be waited for alone)
+      __syncthreads();                // one barrier a step: the buffer written next was read before it
+      multiply(buf);
+    };
+    // Two steps a turn and no way out between them: from there the compiler sees one back to the loop's head on which the loads wanted there are the latest,
+    // and waits for all of them there.  f16 900 x 1000 x 4001 29.2 -> 24.4 us, 1000 x 777 x 1531 14.2 -> 12.8; f32 497 x 391 x 2100 whole 45.3 -> 43.6.
+    int s = begin;
+    for (; s + 2 <= end; s += 2) step(0, s), step(1, s + 1);
+    if (s < end) step(0, s);
   }
-  if (end > begin) {
-    fetch(0, begin);
-    __builtin_amdgcn_sched_barrier(0);  // (in this order: the loop counts on it)
-    fetch(1, min(begin + 1, end - 1));
-  }
-  if (with_left && full > 0) {
-#pragma unroll
-    for (int i = 0; i < SA::N; ++i) la[i] = SA::trimmed(la[i], i, left, tid);
-#pragma unroll
-    for (int i = 0; i < SB::N; ++i) lb[i] = SB::trimmed(lb[i], i, left, tid);
-  }
-  put(lds[0], la, lb);
-  __syncthreads();
-  multiply(lds[0]);
-  auto step = [&](int d, int s) {
-    char* buf = lds[d ^ 1];
-    put(buf, ra[d], rb[d]);
-    fetch(d, min(s + 2, end - 1));  // (without a branch, so that a step's loads can be waited for alone)
-    __syncthreads();                // one barrier a step: the buffer written next was read before it
-    multiply(buf);
-  };
-  // Two steps a turn and no way out between them: from there the compiler sees one back to the loop's head on which the loads wanted there are the latest,
-  // and waits for all of them there.  f16 900 x 1000 x 4001 29.2 -> 24.4 us, 1000 x 777 x 1531 14.2 -> 12.8; f32 497 x 391 x 2100 whole 45.3 -> 43.6.
-  int s = begin;
-  for (; s + 2 <= end; s += 2) step(0, s), step(1, s + 1);
-  if (s < end) step(0, s);
 
   // element e of lane l of block (i, j): row l % 32, column 8 (e / 4) + 4 (l / 32) + e % 4
   typedef typename Result<T, SPLIT>::type R;
@@ -273,7 +282,7 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
 }
 
 // 32 x 32 tiles, for products of so few larger ones that most CUs would have none.  A wave has a block of its own parts of K, LDS of its own and no barriers
-// in its loop; the four waves' sums meet in LDS.  Part i (of 4 nsplit) has the steps per * i .. per * (i + 1) - 1, of which there may be none.
+// in its loop; the four waves' sums meet in LDS.  Part i (of 4 nsplit) has the steps per * i .. per * (i + 1) - 1, of which there may be none; K is more than one step.
 // What bounds it: launch and first bytes, then a wave's chain of steps (0.6 us, in 16 bits 8 KB of a CU's share of the caches).  f32 625 x 319 x 353 on 64 x 64 tiles 10.3 us, 6.3 so;
 // what it takes, and more figures: gemm_ragged_plan.
 template <typename T, bool A_KC, bool B_KC, bool SPLIT>
@@ -328,16 +337,11 @@ __global__ void __launch_bounds__(256) gemm_ragged32(MMArgs p, int batches, int 
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
     };
-    if (with_left && full > 0) {
+    if (with_left) {
 #pragma unroll
       for (int i = 0; i < SA::N; ++i) la[i] = a.load_end(i, full, left, m0, p.M, lane);
 #pragma unroll
       for (int i = 0; i < SB::N; ++i) lb[i] = b.load_end(i, full, left, n0, p.N, lane);
-    } else if (with_left) {
-#pragma unroll
-      for (int i = 0; i < SA::N; ++i) la[i] = a.load_last(i, full, left, m0, p.M, lane);
-#pragma unroll
-      for (int i = 0; i < SB::N; ++i) lb[i] = b.load_last(i, full, left, n0, p.N, lane);
     } else {
 #pragma unroll
       for (int i = 0; i < SA::N; ++i) la[i] = a.load(i, from);
@@ -349,7 +353,7 @@ __global__ void __launch_bounds__(256) gemm_ragged32(MMArgs p, int batches, int 
       __builtin_amdgcn_sched_barrier(0);  // (in this order: the loop counts on it)
       fetch(1, min(begin + 1, end - 1));
     }
-    if (with_left && full > 0) {
+    if (with_left) {
 #pragma unroll
       for (int i = 0; i < SA::N; ++i) la[i] = SA::trimmed(la[i], i, left, lane);
 #pragma unroll
@@ -397,17 +401,17 @@ __global__ void __launch_bounds__(256) gemm_ragged_fold(const float* __restrict_
   }
 }
 
-template <typename T, int BT, bool SPLIT>
+template <typename T, int BT, Form FORM>
 hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, int nsplit, float* ws) {
   const int tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BT - 1) / BT, ke = 128 / (int)sizeof(T), steps = (p.K + ke - 1) / ke, per = (steps + nsplit - 1) / nsplit;
   const unsigned grid = (unsigned)((batch * tiles_m * tiles_n * nsplit + 7) / 8 * 8);
   const size_t elems = batch * p.M * p.N, slab = (elems + 3) / 4 * 4;
   const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
-  if (ak && bk) gemm_ragged<T, BT, true, true, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  else if (ak) gemm_ragged<T, BT, true, false, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  else if (bk) gemm_ragged<T, BT, false, true, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  else gemm_ragged<T, BT, false, false, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  if (SPLIT) gemm_ragged_fold<T><<<(unsigned)((elems + 1023) / 1024), 256, 0, stream>>>(ws, static_cast<T*>(p.c), elems, slab, nsplit);
+  if (ak && bk) gemm_ragged<T, BT, true, true, FORM><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  else if (ak) gemm_ragged<T, BT, true, false, FORM><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  else if (bk) gemm_ragged<T, BT, false, true, FORM><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  else gemm_ragged<T, BT, false, false, FORM><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  if (FORM == SPLIT_K) gemm_ragged_fold<T><<<(unsigned)((elems + 1023) / 1024), 256, 0, stream>>>(ws, static_cast<T*>(p.c), elems, slab, nsplit);
   return hipGetLastError();
 }
 template <typename T, bool SPLIT>
@@ -426,8 +430,9 @@ hipError_t launch32(hipStream_t stream, const MMArgs& p, size_t batch, int nspli
 template <typename T>
 hipError_t launch_plan(hipStream_t stream, const MMArgs& p, size_t batch, const RaggedPlan& pl, float* ws) {
   if (pl.tile == 32) return pl.nsplit > 1 ? launch32<T, true>(stream, p, batch, pl.nsplit, ws) : launch32<T, false>(stream, p, batch, 1, nullptr);
-  if (pl.nsplit > 1) return launch<T, 64, true>(stream, p, batch, pl.nsplit, ws);
-  return pl.tile == 128 ? launch<T, 128, false>(stream, p, batch, 1, nullptr) : launch<T, 64, false>(stream, p, batch, 1, nullptr);
+  if (pl.nsplit > 1) return launch<T, 64, SPLIT_K>(stream, p, batch, pl.nsplit, ws);
+  if (p.K <= 128 / (int)sizeof(T)) return pl.tile == 128 ? launch<T, 128, ONE>(stream, p, batch, 1, nullptr) : launch<T, 64, ONE>(stream, p, batch, 1, nullptr);
+  return pl.tile == 128 ? launch<T, 128, WHOLE>(stream, p, batch, 1, nullptr) : launch<T, 64, WHOLE>(stream, p, batch, 1, nullptr);
 }
 
 }  // namespace
@@ -476,14 +481,17 @@ static double few_tiles_us(int dtype, int tile, int steps, size_t tiles, int ns,
   return ns == 1 ? us : std::max(8.8, us + 2.5 + 0.1 * ns + (double)(ns + 1) * slab_bytes / 5e6);
 }
 
+bool gemm_ragged_takes(int dtype, const MMArgs& p, size_t batch) { return supported(p, batch) && !(dtype == UGHIP_F32 && p.K <= 16); }
+
 RaggedPlan gemm_ragged_plan(int dtype, const MMArgs& p, size_t batch) {
   RaggedPlan pl;
-  if (!supported(p, batch) || (dtype == UGHIP_F32 && p.K <= 16)) return pl;
+  if (!gemm_ragged_takes(dtype, p, batch)) return pl;
   auto tiles = [&](int t) { return batch * ((p.M + t - 1) / t) * ((p.N + t - 1) / t); };
   const size_t small = tiles(64), slab_bytes = (batch * p.M * p.N + 3) / 4 * 16;
   pl.tile = tile_of(dtype, p, tiles(128), small);
   if (pl.tile == 128 || small >= 256) return pl;
   const int ke = dtype == UGHIP_F32 ? 32 : 64, steps = (p.K + ke - 1) / ke;
+  if (steps == 1) return pl;  // (nothing to share)
   double best = 0.95 * few_tiles_us(dtype, 64, steps, small, 1, slab_bytes);
   for (int tile : {32, 64}) {
     const size_t n = tiles(tile);
@@ -500,6 +508,7 @@ RaggedPlan gemm_ragged_plan(int dtype, const MMArgs& p, size_t batch) {
 
 hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, const RaggedPlan& pl, float* ws) {
   if (!supported(p, batch) || (pl.tile != 32 && pl.tile != 64 && pl.tile != 128) || pl.nsplit < 1 || (pl.nsplit > 1 && (pl.tile == 128 || !ws))) return hipErrorInvalidValue;
+  if ((pl.tile == 32 || pl.nsplit > 1) && p.K <= (dtype == UGHIP_F32 ? 32 : 64)) return hipErrorInvalidValue;
   if (dtype == UGHIP_F32) return launch_plan<float>(stream, p, batch, pl, ws);
   return dtype == UGHIP_F16 ? launch_plan<_Float16>(stream, p, batch, pl, ws) : launch_plan<__bf16>(stream, p, batch, pl, ws);
 }

@@ -482,7 +482,7 @@ static bool better_in_small_tiles(const MMArgs& p, size_t b) {
   long long set = 0;
   if (p.b_cs != 1 || p.b_rs == 1 || tune_get(TUNE_GEMM_SHAPE, &set) || tune_get(TUNE_GEMM_SPLIT, &set) || tune_on(TUNE_GEMM_4WAVES)) return false;
   const size_t tiles = b * ((p.M + 63) / 64) * ((p.N + 63) / 64), steps = (p.K + 31) / 32;
-  if (tiles >= 256 || !gemm_ragged_plan(UGHIP_F32, p, b).tile) return false;
+  if (tiles >= 256 || !gemm_ragged_takes(UGHIP_F32, p, b)) return false;
   return p.K < 2048 ? tiles * steps <= 7200 : tiles <= 32 && p.K <= 4096;
 }
 
@@ -514,9 +514,10 @@ static Route matmul_route(int dtype, bool mixed, const MMArgs& p, size_t b, size
 }
 
 // The kernels behind ROUTE_ANY, in names: gemm_ragged's tiles and splits of K (gemm_ragged_plan; the smaller two are not named), and the ones that go by element.
-static void any_name(const char* tn, const RaggedPlan& pl, char* out, size_t out_len) {
-  if (pl.nsplit > 1) snprintf(out, out_len, "gemm_any<%s,splitK=%d>", tn, pl.nsplit);
-  else snprintf(out, out_len, "gemm_any<%s%s>", tn, pl.tile == 128 ? ",128x128" : pl.tile ? "" : ",by element");
+template <typename F>
+static void any_name(const char* tn, const RaggedPlan& pl, F&& print) {
+  if (pl.nsplit > 1) print("gemm_any<%s,splitK=%d>", tn, pl.nsplit);
+  else print(pl.tile == 128 ? "gemm_any<%s,128x128>" : pl.tile ? "gemm_any<%s>" : "gemm_any<%s,by element>", tn);
 }
 
 static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* lhs, const ughip_slice* rhs, size_t b, size_t m, size_t n, size_t k,
@@ -631,9 +632,7 @@ static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* l
       ws = static_cast<float*>(dev->gemm_ws);
     }
     if (!ws) pl.nsplit = 1;  // no memory for the slabs: whole
-    char name[64];
-    any_name(tn, pl, name, sizeof name);
-    note_kernel("%s", name);
+    any_name(tn, pl, [](auto... text) { note_kernel(text...); });
     if (pl.tile) UGHIP_HIPCHK(gemm_ragged_launch(st, dst->dtype, p, b, pl, ws));
     else if (f32) gemm_f32_any<<<grid, 256, 0, st>>>(p);
     else if (dst->dtype == UGHIP_F16) gemm_half_any<_Float16><<<grid, 256, 0, st>>>(p);
@@ -1035,7 +1034,7 @@ extern "C" int ughip_matmul_plan(int dtype, int rhs_dtype, size_t b, size_t m, s
       break;
     }
     case ROUTE_TILED: gemm_tiled_name(dtype, p, b, mixed, nullptr, buf, buf_len); break;
-    default: any_name(tn, gemm_ragged_plan(dtype, p, b), buf, buf_len); break;
+    default: any_name(tn, gemm_ragged_plan(dtype, p, b), [&](auto... text) { snprintf(buf, buf_len, text...); }); break;
   }
   return UGHIP_OK;
 }
