@@ -48,7 +48,7 @@ def test_gated_columns(gpu, k, n):
     close(get(out, n), g / (1 + np.exp(-1.5 * g)) * (u + 1), 2 * bound(k))
 
 
-@pytest.mark.parametrize("k, parts", [(1024, 256), (1024, 128), (1024, 64), (1024, 4), (1024, 2), (2048, 2), (3072, 2), (1536, 2), (1536, 3), (8192, 8), (520, 1), (520, 65)])
+@pytest.mark.parametrize("k, parts", [(1024, 256), (1024, 128), (1024, 64), (1024, 4), (1024, 2), (2048, 2), (3072, 2), (1536, 2), (1536, 3), (8192, 8), (520, 1), (520, 65), (2560, 2), (3840, 3), (8192, 32), (768, 3), (8, 2), (520, 130), (8192, 2048)])
 @pytest.mark.parametrize("after", [False, True])
 def test_parts_of_the_row(gpu, k, parts, after):
     n = 33

@@ -389,20 +389,26 @@ __global__ void __launch_bounds__(1024) row_wide_kernel(RowArgs a) {
         for (int e = 0; e < 4; ++e) v[i][e] *= silu_f(y[i][e]);
     }
     if (!ok) v[0] = v[1] = zero;
-    if (a.norm) {
+    const int part = a.norm ? a.k / a.norm_groups : 0;
+    if (part == 4) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) v[i] = v[i] * (1.f / sqrtf((v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w) / 4.f + a.eps)) * nm[i];
+      if (!ok) v[0] = v[1] = zero;
+    } else if (part) {
       float ss = square(v[0], v[1]);
-      const int part = a.k / a.norm_groups;
       if (a.norm_groups == 1) {
         ss = any_block_sum(ss, red[1]);
-      } else if (part < 512) {  // 1, 2, 4, .. or 32 lanes (the host checks)
+      } else if (part < 256) {  // 1, 2, 4, 8 or 16 lanes (the host checks)
         for (int d = part >> 4; d; d >>= 1) ss += __shfl_xor(ss, d, 64);
-      } else {  // whole waves (the host checks)
-        ss = wave_sum(ss);
-        if (lane == 0) red[2][wave] = ss;
+      } else {  // whole waves, or whole halves of them (the host checks)
+        const int shift = part & 256 ? 5 : 6, mine = t >> shift, run = part >> (shift + 3), first = mine / run * run;
+        if (shift == 6) ss = wave_sum(ss);
+        else ss = row_sum16(ss), ss += __shfl_xor(ss, 16, 64);
+        float* sums = &red[1][0];  // 32 of them
+        if ((t & ((1 << shift) - 1)) == 0) sums[mine] = ss;
         __syncthreads();
-        const int run = part >> 9, first = wave / run * run;
         ss = 0.f;
-        for (int i = 0; i < run; ++i) ss += red[2][first + i];
+        for (int i = 0; i < run; ++i) ss += sums[first + i];
       }
       const float inv = 1.f / sqrtf(ss / (float)part + a.eps);
 #pragma unroll
@@ -474,24 +480,26 @@ hipError_t launch_any(hipStream_t st, const RowArgs& a, int route, bool up, size
 constexpr int WIDE_MAX = 8192;  // elements of the input row: eight to a thread
 
 // Columns per workgroup: the more, the fewer times the input row is read and made, but every CU wants a workgroup and some six waves to keep
-// enough of the matrix on its way (and past 16 matrix rows the last ones wait).  bf16, us by columns per workgroup 1 / 2 / 4 / 8 / 16, in a token's sequence:
-//   1024 of 1024 3.5 / 3.6 / 3.5 / 4.1 / 5.2, 3336 of 1024 6.5 / 5.9 / 5.0 / 5.2 / 6.2, gated 2816 of 1024 6.6 / 6.2 / 5.4 / 6.3 / 8.2, 1024 of 2816 3.6 / 3.7 / 3.7 / 4.3 / 5.3,
-//   6416 of 2048 15.4 / 11.5 / 9.9 / 9.1 / 8.1, gated 5632 of 2048 17.6 / 13.6 / 12.1 / 11.0 / 12.2, 2048 of 5632 7.4 / 6.4 / 6.0 / 6.0 / 7.2,
-//   32000 of 1024 28.6 / 17.4 / 13.5 / 12.5 / 13.8, of 2048 60 / 41 / 31 / 25 / 23
-int wide_columns(int cols, int threads, int matrices) {
+// enough of the matrix on its way (and past 16 matrix rows the last ones wait).  Weights from memory, us by columns per workgroup 1 / 2 / 4 / 8 / 16, bf16, then f32:
+//   1024 of 1024 4.5 / 4.1 / 4.2 / 5.0 / 5.9, 4.7 / 4.0 / 4.3 / 5.0 / 5.8; 3336 of 1024 6.7 / 5.8 / 4.9 / 5.1 / 6.0, 7.8 / 7.0 / 6.1 / 5.6 / 6.2; gated 2816 of 1024 7.2 / 6.7 / 5.8 / 6.3,
+//   9.2 / 7.7 / 7.9 / 8.0; 1024 of 2816 7.9 / 6.5 / 5.1 / 5.6 / 6.6, 8.5 / 7.2 / 6.1 / 7.1 / 10.0; 6416 of 2048 18.5 / 12.7 / 10.2 / 8.5 / 7.6, 24.2 / 18.1 / 14.8 / 14.1 / 13.6; gated 5632 of 2048
+//   20.4 / 15.5 / 12.9 / 11.3, 29.1 / 22.9 / 21.1 / 19.5; 2048 of 5632 23.0 / 14.2 / 10.5 / 8.7 / 9.5, 26.6 / 18.8 / 15.5 / 12.2 / 17.2; 8192 of 512 7.0 / 5.9 / 5.0 / 5.2 / 5.9, 7.8 / 7.0 / 6.2 / 5.9 / 6.2;
+//   32000 of 1024 31.5 / 20.8 / 15.9 / 14.4 / 13.7, 43.4 / 37.4 / 31.2 / 27.0 / 25.0 (in a reply, whose weights are partly cached, - / - / 16.6 / 14.7 / 14.0, - / - / 31.5 / 27.7 / 26.1);
+//   32000 of 2048 78 / 49 / 34 / 27 / 24, 111 / 77 / 59 / 52 / 49.
+int wide_columns(int cols, int threads, int matrices, int cus) {
   int most = 16 / matrices;
-  while (most > 1 && ((cols + most - 1) / most < 256 || (cols + most - 1) / most * (threads / 64) < 1400)) most /= 2;
+  while (most > 1 && ((cols + most - 1) / most < cus || (cols + most - 1) / most * (threads / 64) < cus * 11 / 2)) most /= 2;
   return most;
 }
 
 template <typename WT, int NM, int ROUTE, bool PLAIN>
-hipError_t launch_wide(hipStream_t st, const RowArgs& a, size_t lds) {
+hipError_t launch_wide(ughip_device* dev, const RowArgs& a, size_t lds) {
   const int total = (ROUTE == 2 ? a.segs : 1) * a.k, threads = (total / 8 + 63) / 64 * 64;
   auto go = [&](auto kernel, int columns) {
-    kernel<<<(unsigned)((a.cols + columns - 1) / columns), threads, lds, st>>>(a);
+    kernel<<<(unsigned)((a.cols + columns - 1) / columns), threads, lds, dev->stream>>>(a);
     return hipGetLastError();
   };
-  switch (wide_columns(a.cols, threads, NM)) {
+  switch (wide_columns(a.cols, threads, NM, dev->num_cus)) {
     case 1: return go(row_wide_kernel<WT, NM, 1, 1, ROUTE, PLAIN>, 1);
     case 2: return go(row_wide_kernel<WT, NM, 2, 1, ROUTE, PLAIN>, 2);
     case 4: return go(row_wide_kernel<WT, NM, 2, 2, ROUTE, PLAIN>, 4);
@@ -595,17 +603,17 @@ extern "C" int ughip_product_row(ughip_device* dev, const ughip_row_step* p) {
   const bool vec = p->k % 8 == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15) == 0;
   auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   const size_t part = p->k / norm_groups;
-  // pieces of eight elements, a thread each, and normed parts of whole waves or of whole powers of two of lanes
-  const bool parts_fit = !p->norm || norm_groups == 1 || part % 512 == 0 || (part >= 8 && part < 512 && (part & (part - 1)) == 0);
+  // pieces of eight elements, a thread each, and normed parts of whole halves of waves, of a power of two of lanes or of half a lane's
+  const bool parts_fit = !p->norm || norm_groups == 1 || part % 256 == 0 || (part >= 4 && part < 256 && (part & (part - 1)) == 0);
   if (vec && total <= (size_t)WIDE_MAX && parts_fit && a16(a.x) && a16(a.y) && a16(a.gate) && a16(a.x_out) && a16(a.extra)) {
     const size_t work = p->route == 1 ? (p->experts + (size_t)route_lds_floats(a.route.experts, a.route.groups) + 2 * p->top) * sizeof(float) : 0;
     const bool plain = !a.y && !a.gate && !a.norm;
     auto go = [&](auto type) {
       using WT = decltype(type);
-      if (p->route == 1) return launch_wide<WT, 2, 1, true>(dev->stream, a, work);
-      if (p->route == 2) return launch_wide<WT, 1, 2, true>(dev->stream, a, 0);
-      if (glu) return plain ? launch_wide<WT, 2, 0, true>(dev->stream, a, 0) : launch_wide<WT, 2, 0, false>(dev->stream, a, 0);
-      return plain ? launch_wide<WT, 1, 0, true>(dev->stream, a, 0) : launch_wide<WT, 1, 0, false>(dev->stream, a, 0);
+      if (p->route == 1) return launch_wide<WT, 2, 1, true>(dev, a, work);
+      if (p->route == 2) return launch_wide<WT, 1, 2, true>(dev, a, 0);
+      if (glu) return plain ? launch_wide<WT, 2, 0, true>(dev, a, 0) : launch_wide<WT, 2, 0, false>(dev, a, 0);
+      return plain ? launch_wide<WT, 1, 0, true>(dev, a, 0) : launch_wide<WT, 1, 0, false>(dev, a, 0);
     };
     UGHIP_HIPCHK(p->w->dtype == UGHIP_BF16 ? go(uint16_t()) : go(float()));
     return UGHIP_OK;
