@@ -3,9 +3,6 @@
 #include "llama.h"
 
 #include <atomic>
-#include <condition_variable>
-#include <deque>
-#include <functional>
 #include <mutex>
 #include <chrono>
 #include <cmath>
@@ -13,6 +10,7 @@
 
 #include "hip_device.h"
 #include "rng.h"
+#include "step_queue.h"
 #include "ug/block.h"
 #include "ug/safetensors.h"
 
@@ -1135,84 +1133,6 @@ struct PreparedStep {
   double build_ms = 0, gen_ms = 0, comp_ms = 0;
 };
 
-// Steps on their way to a thread that launches them in order.  Nothing is lost by an exception on either side: what the launches throw
-// comes out of push or finish, and the thread has ended when the queue is gone.
-class StepQueue {
- public:
-  explicit StepQueue(std::function<void(PreparedStep&)> run) : run_(std::move(run)), thread_([this] { loop(); }) {}
-  ~StepQueue() {
-    {
-      std::lock_guard<std::mutex> g(mu_);
-      waiting_.clear();  // (after finish there are none: these belong to a caller that gives up)
-    }
-    close();
-  }
-  // Waits while kAhead steps are.  Steps that have been launched end here: their buffers and graphs are the caller's thread's to free.
-  void push(PreparedStep&& st) {
-    std::deque<PreparedStep> launched;
-    {
-      std::unique_lock<std::mutex> g(mu_);
-      room_.wait(g, [this] { return waiting_.size() < kAhead || error_; });
-      if (error_) std::rethrow_exception(error_);
-      waiting_.push_back(std::move(st));
-      launched.swap(launched_);
-    }
-    some_.notify_one();
-  }
-  void finish() {
-    close();
-    if (error_) std::rethrow_exception(error_);
-  }
-
- private:
-  static constexpr size_t kAhead = 3;
-  void close() {
-    if (!thread_.joinable()) return;
-    {
-      std::lock_guard<std::mutex> g(mu_);
-      closed_ = true;
-    }
-    some_.notify_one();
-    thread_.join();
-  }
-  void loop() {
-    for (;;) {
-      PreparedStep st;
-      {
-        std::unique_lock<std::mutex> g(mu_);
-        some_.wait(g, [this] { return closed_ || !waiting_.empty(); });
-        if (waiting_.empty()) return;
-        st = std::move(waiting_.front());
-        waiting_.pop_front();
-      }
-      try {
-        run_(st);
-      } catch (...) {
-        std::lock_guard<std::mutex> g(mu_);
-        error_ = std::current_exception();
-        waiting_.clear();
-        closed_ = true;
-      }
-      {
-        std::lock_guard<std::mutex> g(mu_);
-        launched_.push_back(std::move(st));
-        if (error_) {
-          room_.notify_one();
-          return;
-        }
-      }
-      room_.notify_one();
-    }
-  }
-  std::function<void(PreparedStep&)> run_;
-  std::mutex mu_;
-  std::condition_variable room_, some_;
-  std::deque<PreparedStep> waiting_, launched_;
-  std::exception_ptr error_;
-  bool closed_ = false;
-  std::thread thread_;
-};
-
 double ms_between(std::chrono::steady_clock::time_point a, std::chrono::steady_clock::time_point b) {
   return std::chrono::duration<double, std::milli>(b - a).count();
 }
@@ -1298,7 +1218,7 @@ std::vector<int32_t> generate_greedy_queued(const Decoder& model, const std::vec
   // This thread builds the steps, the other one launches them, a few steps behind at most; both go on without waiting for each other (with a
   // thread per step that is joined before the next begins, a step took the slower half and 30 us: 0.17 ms beside 0.13).  A step's buffers go
   // back to the pool when its launches are out: the stream orders their reuse behind its kernels.
-  StepQueue queue([](PreparedStep& st) { st.compiled->run(); });
+  StepQueue<PreparedStep> queue([](PreparedStep& st) { st.compiled->run(); });
   for (size_t step = 1; step <= n_steps; ++step) {
     state->settle();
     PreparedStep next;
