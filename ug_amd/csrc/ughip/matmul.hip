@@ -11,6 +11,7 @@
 #include "bf16_split.h"
 #include "gemm.h"
 #include "internal.h"
+#include "scratch_block.h"
 #include "ughip.h"
 #include "wave_ops.h"
 
@@ -407,34 +408,36 @@ int matmul_scratch_setup(ughip_device* dev) {
 }
 }  // namespace ughip
 
-// The per-device block the split-K partial tiles go to, grown (never shrunk) to `bytes`.
-static int grow_gemm_ws(ughip_device* dev, size_t bytes) {
-  if (bytes <= dev->gemm_ws_bytes) return UGHIP_OK;
-  std::lock_guard<std::mutex> g(dev->mu);
-  UGHIP_HIPCHK(hipStreamSynchronize(dev->stream));  // earlier launches may still read the old block
-  if (dev->gemm_ws) (void)hipFree(dev->gemm_ws);
-  dev->gemm_ws = nullptr;
-  dev->gemm_ws_bytes = 0;
-  const size_t want = std::max<size_t>(bytes, (size_t)32 << 20);
-  UGHIP_HIPCHK(hipMalloc(&dev->gemm_ws, want));
-  dev->gemm_ws_bytes = want;
-  return UGHIP_OK;
-}
+namespace {
+struct HipBlocks {
+  hipStream_t stream;
+  bool went(hipError_t e, const char* what) { return e == hipSuccess ? true : (set_error(UGHIP_ERR_HIP, "%s: %s", what, hipGetErrorString(e)), false); }
+  bool synchronize() { return went(hipStreamSynchronize(stream), "hipStreamSynchronize before a block grows"); }
+  bool free(void* p) { return went(hipFree(p), "hipFree of a block that grows"); }
+  Grown allocate(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return went(e, "hipMalloc of a block") ? Grown::YES : Grown::FAILED;
+    (void)hipGetLastError();
+    return Grown::NO_MEMORY;
+  }
+};
+}  // namespace
 
-// The per-device block for what lies between the launches of one call on rows (normalised rows, the rows between the two
-// products of an MLP block); same life cycle.
-static int grow_rows_ws(ughip_device* dev, size_t bytes) {
-  if (bytes <= dev->rows_ws_bytes) return UGHIP_OK;
+// Grows (never shrinks) one of a device's blocks to `bytes`.  no_memory: where there is none, that is said there and the call succeeds.
+static int grow(ughip_device* dev, void** block, size_t* have, size_t bytes, size_t least, bool* no_memory) {
+  if (bytes <= *have) return UGHIP_OK;
   std::lock_guard<std::mutex> g(dev->mu);
-  UGHIP_HIPCHK(hipStreamSynchronize(dev->stream));
-  if (dev->rows_ws) (void)hipFree(dev->rows_ws);
-  dev->rows_ws = nullptr;
-  dev->rows_ws_bytes = 0;
-  const size_t want = std::max<size_t>(bytes, (size_t)16 << 20);
-  UGHIP_HIPCHK(hipMalloc(&dev->rows_ws, want));
-  dev->rows_ws_bytes = want;
+  const Grown grown = grow_block(HipBlocks{dev->stream}, block, have, bytes, least);
+  if (grown == Grown::FAILED) return UGHIP_ERR_HIP;
+  if (grown == Grown::YES) return UGHIP_OK;
+  if (!no_memory) return set_error(UGHIP_ERR_HIP, "hipMalloc of a block of %zu bytes: %s", std::max(bytes, least), hipGetErrorString(hipErrorOutOfMemory));
+  *no_memory = true;
   return UGHIP_OK;
 }
+// The per-device block the split-K partial tiles go to.
+static int grow_gemm_ws(ughip_device* dev, size_t bytes, bool* no_memory = nullptr) { return grow(dev, &dev->gemm_ws, &dev->gemm_ws_bytes, bytes, (size_t)32 << 20, no_memory); }
+// The per-device block for what lies between the launches of one call on rows (normalised rows, the rows between the two products of an MLP block).
+static int grow_rows_ws(ughip_device* dev, size_t bytes) { return grow(dev, &dev->rows_ws, &dev->rows_ws_bytes, bytes, (size_t)16 << 20, nullptr); }
 
 // Which kernel family a product goes to: decided from shapes, strides, offsets and alignment alone, so that the choice can be
 // asked for without a device (ughip_matmul_plan) and is the same one the launch makes.
@@ -628,8 +631,9 @@ static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* l
     static_assert(RaggedPlan::MAX_WS <= UGHIP_MATMUL_NOALLOC_SCRATCH_BYTES, "a product that could be taken whole is not refused for its slabs");
     float* ws = static_cast<float*>(dev->static_scratch);
     if (pl.nsplit > 1 && !no_alloc) {
-      if (grow_gemm_ws(dev, pl.ws_bytes)) (void)hipGetLastError();
-      ws = static_cast<float*>(dev->gemm_ws);
+      bool no_memory = false;
+      if (int rc = grow_gemm_ws(dev, pl.ws_bytes, &no_memory)) return rc;
+      ws = no_memory ? nullptr : static_cast<float*>(dev->gemm_ws);
     }
     if (!ws) pl.nsplit = 1;  // no memory for the slabs: whole
     any_name(tn, pl, [](auto... text) { note_kernel(text...); });
