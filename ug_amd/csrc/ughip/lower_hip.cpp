@@ -1450,8 +1450,7 @@ class Lowering {
   // moved back to end with the row; a group past the end is the last one again, folded and stored by nobody.
   // What bounds it: HBM for many rows, the launch for few.  Re-reading each loop's operands (and the softmax's exponentials through memory,
   // two launches) -> so, with stores through the cache: softmax [32, 1024] 6.3 -> 3.4 us, [16411, 1531] 77.3 -> 42.3 (4.7 TB/s of its 200 MB), [1472, 4113] 22.1 -> 13.8, [9994, 256] 8.4 -> 5.3;
-  // RMSNorm [1900, 2048] 7.3 -> 6.5.  At most 48 words a thread are held (rows of 49152, of
-  // 64-bit integers 24576: two kernels of 49152 of those went through scratch memory); longer rows go through memory as before.
+  // RMSNorm [1900, 2048] 7.3 -> 6.5.  At most 48 elements a thread are held (rows of 49152); longer rows go through memory as before.
  public:
   struct Held {  // a load's place: argument, offset = c + sum row[k] * (digit of row loop k) + unit * (index along the row)
     int arg = 0, unit = 0;
@@ -1496,12 +1495,11 @@ class Lowering {
     return any;
   }
 
-  static int words(int dtype) { return dtype_size(dtype) > 4 ? 2 : 1; }
   // Registers shared by the kernels of a source: the places in them, by the argument numbers of the source.
   struct Registers {
     std::vector<Held> at;
     std::vector<int> dtype;
-    int words_left = 48;  // per thread: at 1024 threads the compiler has 128
+    int floats_left = 48;  // per thread: at 1024 threads the compiler has 128
   };
   // Row decoding and the loads of everything that is held; link: this kernel's argument that is not loaded but found in ug_link.
   void emit_rows_head(Text& o, Registers& regs, const std::vector<int>& arg_number, int link) {
@@ -1518,9 +1516,8 @@ class Lowering {
       size_t k = std::find(regs.at.begin(), regs.at.end(), h) - regs.at.begin();
       const std::string name = "ug_h" + std::to_string(k);
       if (k == regs.at.size()) {
-        const int n = form_.per * form_.vec * words(I_[i].dtype);
-        if (regs.words_left < n) continue;
-        regs.words_left -= n;
+        if (regs.floats_left < form_.per * form_.vec) continue;
+        regs.floats_left -= form_.per * form_.vec;
         regs.at.push_back(h);
         regs.dtype.push_back(I_[i].dtype);
         o << "  " << dtype_c_name(I_[i].dtype) << " " << name << "[" << form_.per << "][" << form_.vec << "];\n";
@@ -1684,9 +1681,7 @@ class Lowering {
     form_.trips.clear();
     for (int r : rows)
       if (loops_[r].trip > 1) form_.trips.push_back(loops_[r].trip);
-    int widest = 1;
-    for (size_t a = 0; a < s_.n_args; ++a) widest = std::max(widest, words(s_.args[a].dtype));
-    rows_ok_ = form_.per * form_.vec * widest <= 48;
+    rows_ok_ = form_.per * form_.vec <= 48;
   }
 
   void emit_rows() {
@@ -1798,7 +1793,7 @@ bool lower_rows_pair(const ughip_ssa& first, const ughip_ssa& second, const std:
   Lowering::emit_rows_prologue(o, entry, sig, *fa);
   o << aliases << "  " << dtype_c_name(first.args[link].dtype) << " ug_link[" << fa->per << "][" << fa->vec << "];\n";
   Lowering::Registers regs;
-  regs.words_left -= fa->per * fa->vec * Lowering::words(first.args[link].dtype);
+  regs.floats_left -= fa->per * fa->vec;
   a.emit_rows_head(o, regs, number_a, -1);
   b.emit_rows_head(o, regs, number_b, link_b);
   o << "  {\n";
