@@ -38,6 +38,14 @@ def _bare(*buffers):
     return buffers
 
 
+def _whole_numbers(x, dev):
+    """(x - max) times the sum of that, row by row."""
+    wide = lambda r: r.broadcast(x.shape)  # noqa: E731
+    lx = LB.copy(x, x.shape, dev)
+    e = lx.binary("sub", wide(lx.reduce("max", 1)))
+    return _bare(e.binary("mul", wide(e.reduce("sum", 1))))[0]
+
+
 def _joined(lb, keep=0):
     """The source of the first two items of a graph as one launch, '' where they stay two; needs no device."""
     s = Schedule.create_one(lb)
@@ -79,6 +87,19 @@ def test_softmax_and_norm_of_any_width(hip, width, rows):
     got = ug_amd.llama.rms_norm(LB.copy(x, x.shape, hip), LB.copy(w, w.shape, hip), 1e-5).data_vec().reshape(x.shape)
     want = x / np.sqrt((x.astype(np.float64) ** 2).mean(-1, keepdims=True) + 1e-5) * w
     np.testing.assert_allclose(got, want, rtol=(10 + width / 1024 + np.log2(width)) * EPS32, atol=1e-30)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", [4, 5, 255, 256, 257, 4099, 24577, 49152, 49153])
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_rows_of_whole_numbers(hip, width, dtype):
+    x = np.random.default_rng(width).integers(-90, 90, (5, width)).astype(dtype)
+    out = _whole_numbers(x, hip)
+    cs = Schedule.create_one(out).compile()
+    assert ("ug_link" in cs.funcs()[0]["source"]) == (width <= 49152)
+    cs.run()
+    e = x - x.max(1, keepdims=True)
+    assert np.array_equal(out.data_vec().reshape(x.shape), e * e.sum(1, keepdims=True, dtype=dtype))
 
 
 @pytest.mark.gpu

@@ -1451,6 +1451,8 @@ class Lowering {
   // What bounds it: HBM for many rows, the launch for few.  Re-reading each loop's operands (and the softmax's exponentials through memory,
   // two launches) -> so, with stores through the cache: softmax [32, 1024] 6.3 -> 3.4 us, [16411, 1531] 77.3 -> 42.3 (4.7 TB/s of its 200 MB), [1472, 4113] 22.1 -> 13.8, [9994, 256] 8.4 -> 5.3;
   // RMSNorm [1900, 2048] 7.3 -> 6.5.  At most 48 elements a thread are held (rows of 49152); longer rows go through memory as before.
+  // Elements, not words: two kernels of 49152 64-bit integers go through 92 bytes of scratch memory a thread and still take 21 us a row, 28 as two through memory;
+  // counted in words, [60, 32768] of them 14.5 -> 27.8 us, [1000, 16384] 55 -> 62.
  public:
   struct Held {  // a load's place: argument, offset = c + sum row[k] * (digit of row loop k) + unit * (index along the row)
     int arg = 0, unit = 0;
