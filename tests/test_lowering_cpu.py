@@ -426,3 +426,10 @@ def test_forced_tiles_are_the_ones_that_their_numbers_name():
             assert _rows_plan(B, 1, 0, 1900, 2048, 2048) == auto, shape
     with ug_amd.tuning(X3_DMA=0):
         assert _rows_plan(B, 1, 0, 1900, 2048, 2048).startswith("gemm_tiled")
+
+
+@pytest.mark.parametrize("shape, past", [((32, 1024), False), ((1024, 1020), False), ((1024, 1024), True), ((1, 49152), False), ((700, 1531), True)])
+def test_row_results_go_past_the_cache_from_four_megabytes_on(cpu, shape, past):
+    s = Schedule.create_one(ug_amd.llama.rms_norm(LB.copy(np.ones(shape, np.float32), shape, cpu), LB.copy(np.ones(shape[1:], np.float32), shape[1:], cpu), 1e-5))
+    source, info = s.item_ssa(0).hip_code("norm")
+    assert info["strategy"] == "row_block" and ("__builtin_nontemporal_store" in source[source.index("__global__"):]) == past

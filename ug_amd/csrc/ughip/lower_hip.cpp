@@ -1587,10 +1587,12 @@ class Lowering {
       const std::string n = std::to_string(st);
       const std::string guard = masked ? "if (ug_g < " + std::to_string(form_.width) + ") " : "";
       Held h;
-      if (form_.vec == 4 && dtype_size(I_[st].dtype) == 4 && !ughip::tune_on(ughip::TUNE_NO_NT_STORES) && place_of(st, cols_[0], &h)) {
+      if (form_.vec == 4 && dtype_size(I_[st].dtype) == 4 && form_.nr * form_.width * 4 >= 4 << 20 && !ughip::tune_on(ughip::TUNE_NO_NT_STORES) && place_of(st, cols_[0], &h)) {
         // A whole group past the cache, as one vector at whatever element it starts (element by element the hint keeps the stores from
         // merging): the next kernel would find it in another XCD's L2 at best.  Softmax [16411, 1531] 43.1 -> 40.7 us, [957, 6560] 11.8 -> 9.8,
-        // [11392, 448] 9.7 -> 8.3; RMSNorm [1900, 2048] 6.5 -> 5.9; rows that fit a few workgroups as before.
+        // [11392, 448] 9.7 -> 8.3; RMSNorm [1900, 2048] 6.5 -> 5.9.  From 4 MB of results on: less than that is on its way out by itself before the launch
+        // ends, and a store past the cache is what the launch waits for.  x - max x, us through / past the cache: [60, 700] 2.3 / 2.6, [700, 300] 2.4 / 2.6 (0.8 MB), [700, 700]
+        // 2.6 / 2.8 (2.0), [5000, 200] 2.9 / 2.9 (4.0), [60, 24576] 4.2 / 4.0 (5.9), [700, 3000] 4.5 / 4.2 (8.4), [5000, 512] 4.2 / 3.4 (10.2).
         const std::string ty = dtype_c_name(I_[st].dtype), v = "ug_s" + n;
         o << "    " << guard << "{\n      typedef " << ty << " ug_4 __attribute__((ext_vector_type(4), aligned(4)));\n      __builtin_nontemporal_store(ug_4{" << v << "[0], " << v << "[1], " << v << "[2], " << v
           << "[3]}, (ug_4*)&" << var((int)I_[st].v) << "[ug_o" << n << "[0]]);\n    }\n";
