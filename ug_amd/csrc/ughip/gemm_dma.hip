@@ -520,7 +520,7 @@ static double ring_cost_us(size_t tiles, int kt, int tile, Operands from) {
 // the fold), us at 384 / 512 / 700 / 1024 / 1500 / 1900 / 2048 rows: 92 / 82 / 131 / 140 / 234 / 254 / 255 -> 76 / 74 / 116 / 126 / 205 / 238 / 240; k 1024, n 2 x 2816: 1500
 // 87 -> 68, 1900 92 -> 74; q | k | v of 1900 rows 80 -> 74 in two splits.  One plane of rows gains nothing (2048 x 11264 x 2048 from memory 97.6, 96.2 so).
 // UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 10 / 12 / 13 / 9 the ring's 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64, 0..2, 6 and 7 keep both out (tuning aid).
-double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
+double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile, bool beside_192) {
   const size_t tiles = tile_count(p, batch, tile);
   if (!tiles) return 1e30;
   const int kt = p.K / BK;
@@ -536,13 +536,13 @@ double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
     // 0.47 + 0.16 x busy, the next 256 fill the second slots (2048^3 24.7 us, 2304^3 31.3, 2816^3 45.5, 5120^2 x 1024 61)
     us += kt * 0.88 * (double)(tiles / 512) * layout;
     const size_t left = tiles % 512;
-    // (unsplit planes take as long with a few second slots filled as with most: 1900 x 2560 x 2048, 300 tiles, 78 us; 600 x 11264 x 2048, 440, 80)
-    if (left > 256) us += kt * (p.b_k_div == 3 && batch == 1 ? 0.82 : 0.63 + 0.25 * (double)(left - 256) / 256.0) * layout;
+    // (beside_192: unsplit planes take as long with a few second slots filled as with most: 1900 x 2560 x 2048, 300 tiles, 78 us; 600 x 11264 x 2048, 440, 80)
+    if (left > 256) us += kt * (beside_192 && batch == 1 ? 0.82 : 0.63 + 0.25 * (double)(left - 256) / 256.0) * layout;
     else if (left) us += kt * (0.47 + 0.16 * (double)left / 256.0) * layout;
     return us;
   }
-  // (256 x 128 with unsplit planes: 1900 x 2560 x 2048 81.5 us, and 74.5 in two splits of 256 x 192)
-  const double t0 = tile == 256 ? 0.9 : tile == 192 ? 0.76 : p.b_k_div == 3 && batch == 1 ? 0.68 : 0.62, t1 = tile == 256 ? 0.6 : tile == 192 ? 0.4 : 0.2;
+  // (beside_192: 256 x 128 with unsplit planes: 1900 x 2560 x 2048 81.5 us, and 74.5 in two splits of 256 x 192)
+  const double t0 = tile == 256 ? 0.9 : tile == 192 ? 0.76 : beside_192 && batch == 1 ? 0.68 : 0.62, t1 = tile == 256 ? 0.6 : tile == 192 ? 0.4 : 0.2;
   for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) {
     const double busy = (left < 256 ? (double)left : 256.0) / 256.0;
     us += kt * (t0 + t1 * busy) * layout;
