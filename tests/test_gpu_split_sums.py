@@ -68,7 +68,7 @@ def test_small_tiles(hip, bmnk, dtype, rhs_nk, lhs_mk):
 
 # aligned products of few tiles: on either side of where the kernel with larger tiles takes over (steps of K in all tiles; 32 tiles and K; 255 tiles and 256), small integers exactly
 @pytest.mark.parametrize("bmnk, small", [((1, 64, 64, 4096), True), ((1, 64, 64, 4128), False), ((1, 64, 2048, 2048), True), ((1, 64, 2112, 2048), False), ((8, 192, 64, 320), True),
-                                         ((1, 512, 512, 512), True), ((1, 576, 1600, 1024), True), ((1, 576, 1600, 1056), False), ((255, 64, 64, 64), True), ((256, 64, 64, 64), False)])
+                                         ((1, 512, 512, 512), True), ((1, 576, 1600, 1024), True), ((1, 576, 1600, 1056), False), ((255, 64, 64, 64), True), ((256, 64, 64, 64), False), ((1, 64, 384, 64), True), ((1, 64, 384, 32), False)])
 @pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
 def test_aligned_products_of_few_tiles(hip, bmnk, small, rhs_nk):
     b, m, n, k = bmnk

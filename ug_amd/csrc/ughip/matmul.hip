@@ -486,6 +486,7 @@ static bool better_in_small_tiles(const MMArgs& p, size_t b) {
   if (p.b_cs != 1 || p.b_rs == 1 || tune_get(TUNE_GEMM_SHAPE, &set) || tune_get(TUNE_GEMM_SPLIT, &set) || tune_on(TUNE_GEMM_4WAVES)) return false;
   const size_t tiles = b * ((p.M + 63) / 64) * ((p.N + 63) / 64), steps = (p.K + 31) / 32;
   if (tiles >= 256 || !gemm_ragged_takes(UGHIP_F32, p, b)) return false;
+  if (steps == 1) return false;  // (64 x 384 x 32 3.9 / 4.3, 32^3 3.5 / 3.7)
   return p.K < 2048 ? tiles * steps <= 7200 : tiles <= 32 && p.K <= 4096;
 }
 
