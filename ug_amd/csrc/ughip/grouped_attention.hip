@@ -508,7 +508,11 @@ int attend_few(ughip_device* dev, SplitArgs a) {
     if (g.t > 1) return go(attention_split_kernel<T, DQ, DV, NW, false, VEC, DV>);
     return across > 1 ? go(attention_split_kernel<T, DQ, DV, NW, true, VEC, 32>) : go(attention_split_kernel<T, DQ, DV, NW, true, VEC, DV>);
   };
-  UGHIP_HIPCHK(pieces_of_eight(g) ? with_vec(std::true_type()) : with_vec(std::false_type()));
+  // Queries staged eight elements at a time from 128 pieces on: fewer leave most waves idle, and a piece takes a lane longer than two elements do.  Several
+  // positions in bf16 behind 100, us by two / by eight: 32 heads of 64, 2 positions (16 pieces) 9.8 / 10.3, 8 (64) 10.3 / 10.5; 16 heads of 128, 2 (32) 12.1 / 12.5, 8 (128)
+  // 13.2 / 13.1; 64 heads of 128 on 8, 2 (256) 15.2 / 13.3.  One position comes with its key, and gains either way.
+  const bool eight = pieces_of_eight(g) && (g.t == 1 || live * (DQ / 8) >= 128);
+  UGHIP_HIPCHK(eight ? with_vec(std::true_type()) : with_vec(std::false_type()));
   if (splits > 1) {
     attention_merge_kernel<<<(unsigned)(g.kv_heads * a.rows), 256, 0, dev->stream>>>(a);
     UGHIP_HIPCHK(hipGetLastError());
