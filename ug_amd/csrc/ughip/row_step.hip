@@ -303,8 +303,8 @@ __global__ void __launch_bounds__(1024) row_wide_kernel(RowArgs a) {
   __shared__ int s_ids[64];
   __shared__ float s_wts[64];
   constexpr int NB = B < 2 ? B : 2;
-  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), waves = blockDim.x >> 6, e0 = t * 8;
-  const int total = (ROUTE == 2 ? a.segs : 1) * a.k;
+  const int total = (ROUTE == 2 ? a.segs : 1) * a.k, waves = (total + 511) >> 9;  // (blockDim is a trip to memory)
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), e0 = t * 8;
   const bool ok = e0 < total;
   const int at0 = ok ? e0 : 0;  // (a lane past the end reads the row's first elements and multiplies them with zeros)
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -323,7 +323,7 @@ __global__ void __launch_bounds__(1024) row_wide_kernel(RowArgs a) {
     if (t < 48) red[t >> 4][t & 15] = 0.f;
   if constexpr (ROUTE == 1) {  // which experts' matrices: before anything of them can be asked for
     float* lg = route_work;
-    for (int e = t; e < a.route.experts; e += blockDim.x) lg[e] = a.logits[e];
+    for (int e = t; e < a.route.experts; e += 64 * waves) lg[e] = a.logits[e];
     __syncthreads();
     if (wave == 0) {
       float* work = lg + a.route.experts;
