@@ -580,9 +580,10 @@ void* ugh_cache_new(void) { return new CompilationCache(); }
 void ugh_cache_free(void* c) { delete static_cast<CompilationCache*>(c); }
 size_t ugh_cache_size(void* c) {
   CompilationCache* cc = static_cast<CompilationCache*>(c);
-  size_t pairs = 0;
-  for (const auto& p : cc->pair_cache) pairs += (p.second.func[0] != nullptr) + (p.second.func[1] != nullptr);
-  return cc->op_cache.size() + cc->ssa_cache.size() + pairs;
+  size_t n = cc->ssa_cache.size();
+  for (const auto& k : cc->op_cache) n += k.second.func != nullptr;
+  for (const auto& p : cc->pair_cache) n += (p.second.func[0] != nullptr) + (p.second.func[1] != nullptr);
+  return n;
 }
 int ugh_schedule_compile(void* s, void* cache, void** out) {
   return guard([&] {

@@ -5,6 +5,7 @@
 #include <memory>
 #include <optional>
 #include <string>
+#include <tuple>
 #include <unordered_map>
 #include <vector>
 
@@ -142,13 +143,18 @@ struct ScheduleItem {
 
 // cache.rs:74-101
 struct CompilationCache {
-  std::unordered_map<std::string, std::shared_ptr<Func>> op_cache, ssa_cache;
+  // A kernel by its key, under which it is looked up once per schedule; null where nothing has wanted it by itself yet.
+  struct Entry {
+    std::shared_ptr<Func> func;
+  };
+  std::unordered_map<std::string, Entry> op_cache;
+  std::unordered_map<std::string, std::shared_ptr<Func>> ssa_cache;
   // Two kernels as one launch, without and with what lies between them written; each made when it is first wanted.
   struct Pair {
     bool stays_two = false;
     std::shared_ptr<Func> func[2];
   };
-  std::unordered_map<std::string, Pair> pair_cache;
+  std::map<std::tuple<const Entry*, const Entry*, int, std::vector<int>>, Pair> pair_cache;  // the kernels, the link, and what they share (Schedule::RowsPair)
 };
 
 // schedule.rs:210-306

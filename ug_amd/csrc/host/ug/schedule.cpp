@@ -248,15 +248,15 @@ const LazyBuffer& Schedule::get_arg_id(ArgId id) const {
   return it->second;
 }
 
-// A kernel item's lowered forms, each made when it is first asked for.
+// A kernel item's place in the cache and its serial form, each made when it is first asked for.
 struct Schedule::Prepared {
   std::optional<op::Kernel> kernel;
-  std::string key;
+  CompilationCache::Entry* entry = nullptr;
   std::optional<ssa::Kernel> ssa;
-  void of(const ScheduleItem& item) {
+  void of(const ScheduleItem& item, CompilationCache& cache) {
     if (kernel) return;
     kernel = item.kernel.kernel();
-    key = normalized_kernel_key(*kernel);
+    entry = &cache.op_cache[normalized_kernel_key(*kernel)];
   }
   const ssa::Kernel& serial() {
     if (!ssa) ssa = kernel->optimize().lower(op::Opts());
@@ -374,12 +374,8 @@ bool Schedule::compile_pair(size_t first, CompilationCache& cache, std::vector<P
   const std::optional<RowsPair> p = pair_at(first);
   if (!p) return false;
   Prepared &x = prepared[first], &y = prepared[first + 1];
-  x.of(items_[first]), y.of(items_[first + 1]);
-  std::string key;
-  key.reserve(x.key.size() + y.key.size() + 32);
-  key.append(x.key).append("\n").append(y.key).append("\n").append(std::to_string(p->link));
-  for (int s : p->shared) key += "," + std::to_string(s);
-  CompilationCache::Pair& known = cache.pair_cache[key];
+  x.of(items_[first], cache), y.of(items_[first + 1], cache);
+  CompilationCache::Pair& known = cache.pair_cache[{x.entry, y.entry, p->link, p->shared}];
   if (known.stays_two) return false;
   if (!held) held = holders();
   const bool keep = !only_between(first, *held);
@@ -459,20 +455,18 @@ CompiledFunc Schedule::compile_item(const ScheduleItem& item, CompilationCache& 
       }
       case ScheduleItem::Kernel: {
         call.kind = CompiledFunc::Kernel;
-        prepared->of(item);
+        prepared->of(item, cache);
         const op::Kernel& kernel = *prepared->kernel;
-        const std::string& key = prepared->key;
         for (const Arg& a : kernel.args) call.args.push_back({a.id, get_arg_id(a.id)});
-        auto it = cache.op_cache.find(key);
-        if (it != cache.op_cache.end()) {
-          call.func = it->second;
+        if (prepared->entry->func) {
+          call.func = prepared->entry->func;
           break;
         }
         std::string kernel_name = kernel.ops.empty() ? "" : kernel.ops[0].name();
         const std::string* name = kernel.ops.empty() ? nullptr : &kernel_name;
         if (device_->use_grid()) call.func = device_->compile(on_a_grid(kernel.optimize()), name);
         else call.func = device_->compile(prepared->serial(), name);
-        cache.op_cache[key] = call.func;
+        prepared->entry->func = call.func;
         break;
       }
     }
