@@ -10,8 +10,8 @@
 //
 // What bounds it: the steps of K on few tiles (0.3 us each in 16 bits, a CU's share of the caches; 0.6 in f32, the f32 matrix pipe two thirds of that; four steps ahead or more waves per tile change nothing), LDS and the f32
 // matrix pipe on many.  Against element-by-element
-// loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 12.2 us, f32 256 -> 32; 2001^3 f16 270 -> 37, f32 340 -> 135; 3999^2 x
-// 2000 f16 1204 -> 103, f32 1014 -> 520; 100^3 9.4 -> 5.4.  Which tile takes what and where K is split: gemm_ragged_plan.
+// loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 11.9 us, f32 256 -> 32; 2001^3 f16 270 -> 33, f32 340 -> 139; 3999^2 x
+// 2000 f16 1204 -> 103, f32 1014 -> 520; 100^3 9.4 -> 6.0.  Which tile takes what and where K is split: gemm_ragged_plan.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
