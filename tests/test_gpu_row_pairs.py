@@ -73,6 +73,18 @@ def test_which_neighbours_are_joined(cpu):
     assert _joined(t.binary("div", t.reduce("sum", 1).broadcast((64, 64)))) == ""  # another row's elements
 
 
+@pytest.mark.parametrize("each, joins", [(8, True), (30, True), (31, False), (40, False)])
+def test_a_pair_has_no_more_arguments_than_a_launch_takes(cpu, each, joins):
+    """Two kernels of 64 buffers at most each run; as one they would have up to twice that, which a launch refuses."""
+    x = _x(1, 3, 8)
+    more = lambda b: [b := b.binary("mul", LB.copy(x, x.shape, cpu)) for _ in range(each)][-1]  # noqa: E731
+    lx = LB.copy(x, x.shape, cpu)
+    e = more(lx.binary("sub", lx.reduce("max", 1).broadcast(x.shape)))
+    [out] = _bare(more(e.binary("div", e.reduce("sum", 1).broadcast(x.shape))))
+    args = [Schedule.create_one(out).item_ssa(i).wire().n_args for i in range(2)]
+    assert args == [each + 2, each + 2] and (_joined(out, keep=1) != "") == joins
+
+
 WIDTHS = [4, 5, 7, 63, 64, 65, 128, 255, 256, 257, 259, 260, 767, 768, 769, 1020, 1023, 1531, 4095, 4096, 4097, 8191, 8193, 16380, 49151, 49152, 49153]
 
 

@@ -1793,6 +1793,7 @@ bool lower_rows_pair(const ughip_ssa& first, const ughip_ssa& second, const std:
       aliases += "  " + b.arg_type(k) + " " + b.arg_name(k) + " = " + a.arg_name(shared[k]) + ";\n";
     }
   }
+  if (r.arg_dtype.size() > MAX_ARGS) return false;
   Text o;
   Lowering::emit_rows_prologue(o, entry, sig, *fa);
   o << aliases << "  " << dtype_c_name(first.args[link].dtype) << " ug_link[" << fa->per << "][" << fa->vec << "];\n";

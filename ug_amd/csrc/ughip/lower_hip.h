@@ -33,6 +33,8 @@ struct Lowered {
 // ug-cuda/src/code_gen.rs:68-186 emits) instead of re-parallelising it.
 Lowered lower_ssa(const ughip_ssa& ssa, const std::string& entry, bool as_written = false);
 
+constexpr size_t MAX_ARGS = 64;  // buffers that a launch takes
+
 // Two row kernels run one behind the other as one: every row of the second reads of the first's result only its own row, which stays in
 // registers.  shared[k]: the first kernel's argument that the second's k-th is, or -1; link: the first kernel's argument that lies between
 // them.  The arguments are the first kernel's, then those of the second's that are not shared; without keep the link is not among them and

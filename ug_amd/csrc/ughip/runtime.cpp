@@ -568,9 +568,9 @@ static int run_impl(ughip_device* dev, ughip_func* f, ughip_slice* const* args, 
   const Lowered& low = f->low;
   if (n_args != low.arg_dtype.size()) return set_error(UGHIP_ERR_INVALID, "kernel %s expects %zu args, got %zu", low.entry.c_str(), low.arg_dtype.size(), n_args);
   if (low.empty_launch) return UGHIP_OK;
-  void* ptrs[64];
-  void* params[66];
-  if (n_args > 64) return set_error(UGHIP_ERR_INVALID, "unsupported number of args for kernel %zu", n_args);
+  void* ptrs[MAX_ARGS];
+  void* params[MAX_ARGS + 2];
+  if (n_args > MAX_ARGS) return set_error(UGHIP_ERR_INVALID, "unsupported number of args for kernel %zu", n_args);
   for (size_t a = 0; a < n_args; ++a) {
     const ughip_slice* s = args[a];
     if (!s) return set_error(UGHIP_ERR_INVALID, "null slice for arg %zu", a);
