@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <cstdint>
 
 namespace ughip {
 
@@ -55,7 +56,11 @@ int gemm_dma_pick(int dtype, const MMArgs& p, size_t batch);
 // nsplit == 1: p.c [M, N] is written straight from the accumulators, residual [M, N] added when given.  nsplit > 1 (it
 // divides the K tiles, into a multiple of 3 and at least 4 each): workgroups share a tile's K range and leave nsplit
 // slabs [M, N] in p.c (scratch), for gemm_fold_f32 to add up.
-hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile, int nsplit, const float* residual, const char* note_tail);
+// gated, where _gates says that the tile can: the matrix is gate rows, then up rows, and silu(gate) * up goes to p.c [M, N / 2], or with
+// gated_planes (N / 2 % 64 == 0) there as the three planes of those rows.
+bool gemm_dma_planes3_gates(const MMArgs& p, int tile, int nsplit);
+hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile, int nsplit, const float* residual, const char* note_tail, bool gated = false,
+                                   uint16_t* gated_planes = nullptr);
 // f32 operands as three bf16 planes each (rows of 3 k elements, the planes of every 64 elements of k side by side; p.K = 6 k):
 // the product as six bf16 terms with an f32 result, on either rhs layout.
 bool gemm_dma_planes6_supported(const MMArgs& p, size_t batch, int tile);

@@ -29,6 +29,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "bf16_split.h"
 #include "gemm_dma.h"
 #include "internal.h"
 #include "ughip.h"
@@ -47,6 +48,18 @@ __device__ __forceinline__ void dma16_m0(unsigned lds_byte_addr, unsigned stage_
 }
 __device__ __forceinline__ void dma16_go(const void* base, unsigned voff) { asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base) : "memory"); }
 
+// z / (1 + exp(-z)) within a unit or two of the last place, as expf and a division give it, in a third of their instructions (an epilogue has nothing to hide
+// them behind): z log2(e) as a rounded product and its remainder, 2^t (1 + r ln 2), a reciprocal with one step of Newton's.  The limits stand for what the remainders
+// are where t is infinite or the reciprocal zero: they change no finite one.
+__device__ __forceinline__ float silu_32(float z) {
+  constexpr float L2E_HI = 1.44269502162933349609375f, L2E_LO = 1.925963033500011e-8f, LN2 = 0.693147182464599609375f;
+  const float t = -z * L2E_HI;
+  const float r = __builtin_fmaf(-z, L2E_LO, __builtin_fmaf(-z, L2E_HI, -t));
+  const float d = 1.f + __builtin_amdgcn_exp2f(t) * __builtin_fmaf(__builtin_amdgcn_fmed3f(r, -1e-3f, 1e-3f), LN2, 1.f);
+  const float q = __builtin_amdgcn_rcpf(d), left = __builtin_amdgcn_fmed3f(__builtin_fmaf(-d, q, 1.f), -1e-3f, 1e-3f);
+  return z * __builtin_fmaf(left, q, q);
+}
+
 // Lane l feeds row / column l % 16, k = 8 (l / 16) .. + 7 of a step of 32.  TWO: the schedule with two barriers per K tile.
 // F32OUT: the result leaves as f32 straight from the accumulators (+ residual when given) instead of as T through LDS.
 // BDIV > 1 ([n, k]-major rhs): K tile t of the lhs meets K tile t / BDIV of the rhs -- an lhs that holds BDIV planes of every
@@ -55,10 +68,13 @@ __device__ __forceinline__ void dma16_go(const void* base, unsigned voff) { asm 
 // by side, and K tile t of the loop is term t % 6 of k tile t / 6 of an f32 product taken as six bf16 ones -- (hi, lo),
 // (lo, hi), (mid, mid), (hi, mid), (mid, hi), (hi, hi), the small ones first; (mid, lo), (lo, mid) and (lo, lo) stay below
 // 2^-24 of the product and are left out.
-// ROWS (1, or 2 with SwiGLU): the lhs rows, the matrix and the result are those of DmaRows.
+// ROWS (1, or 2 with SwiGLU): the lhs rows, the matrix and the result are those of DmaRows.  ROWS 4: planes of rows against gate rows then up rows,
+// silu(gate) * up out (DmaRows: dst, n_out, dst_bf16 for the three planes of rows of n_out elements, else f32).
 template <typename T, int BM, int BN, bool B_KN, bool TWO, bool F32OUT = false, int BDIV = 1, int ROWS = 0>
 __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tiles_n, const float* __restrict__ residual, DmaRows rw) {
-  static_assert(ROWS == 0 || (BDIV == 1 && !B_KN && !F32OUT), "rows: one plane against an [n, k]-major rhs");
+  static_assert(ROWS == 0 || ROWS == 4 || (BDIV == 1 && !B_KN && !F32OUT), "rows: one plane against an [n, k]-major rhs");
+  static_assert(ROWS != 4 || (BDIV == 3 && BN == 192 && F32OUT), "gated planes: 96 columns of three planes are what LDS takes on the way out");
+  constexpr bool GATED = ROWS == 2 || ROWS == 4, BY_ROW = ROWS == 1 || ROWS == 2;
   static_assert(BDIV == 1 || BDIV == 6 || !B_KN, "planes of the lhs alone: against an [n, k]-major rhs only");
   static_assert(BN != 192 || (!B_KN && F32OUT), "192 columns: neither the swizzle of an n-contiguous tile nor the way out through LDS divides them");
   extern __shared__ u32x4 lds[];
@@ -75,7 +91,7 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   // block: its workgroups share few A and B panels in their XCD's L2.
   int bid = blockIdx.x;
   GroupTiles<BM> by_group{rw.group_end, rw.groups, p.M, lane};
-  if constexpr (ROWS != 0) {
+  if constexpr (BY_ROW) {
     if (rw.groups) {
       // how many tile rows there are is known here only: the workgroups past them leave before the runs are dealt
       const int rows = by_group.count();
@@ -102,11 +118,11 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   }
   int m0 = tm * BM, m_end = p.M, group = 0;
   const int n0 = tn * BN;
-  if (ROWS != 0 && rw.groups && !by_group.find(tm, group, m0, m_end)) return;  // the same for the whole workgroup
+  if (BY_ROW && rw.groups && !by_group.find(tm, group, m0, m_end)) return;  // the same for the whole workgroup
   const long long lda = p.a_rs, ldb = B_KN ? p.b_rs : p.b_cs;
-  const char* Ab = reinterpret_cast<const char*>(static_cast<const T*>(p.a) + (size_t)batch * p.a_bs + (ROWS ? 0 : (size_t)m0 * lda));
-  const char* Bb = reinterpret_cast<const char*>(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs + (ROWS ? (size_t)group * rw.w_group : 0) +
-                                                 (ROWS == 2 ? 0 : B_KN ? (size_t)n0 : (size_t)n0 * ldb));
+  const char* Ab = reinterpret_cast<const char*>(static_cast<const T*>(p.a) + (size_t)batch * p.a_bs + (BY_ROW ? 0 : (size_t)m0 * lda));
+  const char* Bb = reinterpret_cast<const char*>(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs + (BY_ROW ? (size_t)group * rw.w_group : 0) +
+                                                 (GATED ? 0 : B_KN ? (size_t)n0 : (size_t)n0 * ldb));
   const int KT = p.K / BK;
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
   const unsigned lds_addr = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds;
@@ -119,7 +135,7 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   for (int i = 0; i < NDA; ++i) {
     const int row = (i * 4 + wave) * 8 + (lane >> 3), cp = lane & 7;
     int src = min(row, m_last);
-    if constexpr (ROWS != 0) {
+    if constexpr (BY_ROW) {
       src += m0;
       if (rw.row_index) src = max(0, min(rw.row_index[src], rw.x_rows - 1));
     }
@@ -131,7 +147,7 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
     if (!B_KN) {
       const int row = g * 8 + (lane >> 3), cp = lane & 7;
       int src = min(row, n_left - 1);
-      if constexpr (ROWS == 2) {  // a wave's half of the tile: BN / 4 gate columns, then the same columns of up
+      if constexpr (GATED) {  // a wave's half of the tile: BN / 4 gate columns, then the same columns of up
         const int q = row % (BN / 2);
         src = min(tn * (BN / 2) + row / (BN / 2) * (BN / 4) + q % (BN / 4), rw.n_out - 1) + (q >= BN / 4 ? rw.n_out : 0);
       }
@@ -323,7 +339,63 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   tile(KT - 1, N_(), N_());
 
   // Register e of lane l of block (i, j): row wm + 16 i + l % 16, column wn + 16 j + 4 (l / 16) + e.
-  if constexpr (ROWS != 0) {
+  if constexpr (ROWS == 4) {
+    // As the fold of slabs has it: silu(gate) * up of the f32 sums, rounded to f32, then its three terms.  In registers it saves the f32 sums' way to memory and back and the
+    // launch that folds them: gate and up of 1900 rows, n 2 x 5632, k 2048, 218 us and a fold of 24 -> 228.  The ten are the vector instructions of two rounds of tiles, which a
+    // lone wave per SIMD has nothing to hide behind (19 with expf, a division and a store's place worked out for every piece).
+    constexpr int NC = NJ / 2, COLS = BN / 2;
+    auto gated = [&](int i, int j, int e) {
+      float y = silu_32(acc[i][j][e]) * acc[i][j + NC][e];
+      asm("" : "+v"(y));  // the terms of the f32 value, as if it had been stored
+      return y;
+    };
+    if (!rw.dst_bf16) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+          const int row = wm + i * 16 + (lane & 15), col = tn * COLS + (wave & 1) * (COLS / 2) + j * 16 + (lane >> 4) * 4;
+          if (row <= m_last && col < rw.n_out)
+            *reinterpret_cast<floatx4*>(static_cast<float*>(rw.dst) + (size_t)(m0 + row) * rw.n_out + col) = floatx4{gated(i, j, 0), gated(i, j, 1), gated(i, j, 2), gated(i, j, 3)};
+        }
+      return;
+    }
+    // rows of [hi | mid | lo], 96 columns each, through LDS: 16 rows of a wave's writes start in 16 different groups of four banks
+    constexpr int PITCH = 3 * COLS * 2 + 16, CHUNKS = COLS / 8;
+    char __attribute__((address_space(3)))* Cs = (char __attribute__((address_space(3)))*)lds;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        u32x2 hi, mid, lo;
+        unsigned h, m, l;
+        split3_pair(gated(i, j, 0), gated(i, j, 1), h, m, l);
+        hi.x = h, mid.x = m, lo.x = l;
+        split3_pair(gated(i, j, 2), gated(i, j, 3), h, m, l);
+        hi.y = h, mid.y = m, lo.y = l;
+        char __attribute__((address_space(3)))* at = Cs + (wm + i * 16 + (lane & 15)) * PITCH + ((wave & 1) * (COLS / 2) + j * 16 + (lane >> 4) * 4) * 2;
+        *(u32x2 __attribute__((address_space(3)))*)at = hi;
+        *(u32x2 __attribute__((address_space(3)))*)(at + COLS * 2) = mid;
+        *(u32x2 __attribute__((address_space(3)))*)(at + COLS * 4) = lo;
+      }
+    __syncthreads();
+    // three quarters of the threads, so that a pass is 16 whole rows of a plane and a thread's place in the row stays
+    const int c = tid % CHUNKS, r0 = tid / CHUNKS, col = tn * COLS + c * 8;
+    if (r0 >= 16 || col >= rw.n_out) return;  // n_out % 64 == 0: whole chunks
+    uint16_t* __restrict__ X3 = static_cast<uint16_t*>(rw.dst) + (size_t)(m0 + r0) * 3 * rw.n_out + col / 64 * 192 + col % 64;
+    const char __attribute__((address_space(3)))* from = Cs + r0 * PITCH + c * 16;
+#pragma unroll
+    for (int pass = 0; pass < BM / 16; ++pass) {
+      if (pass * 16 + r0 > m_last) break;
+#pragma unroll
+      for (int plane = 0; plane < 3; ++plane)
+        *reinterpret_cast<u32x4*>(X3 + plane * 64) = *(const u32x4 __attribute__((address_space(3)))*)(from + pass * 16 * PITCH + plane * COLS * 2);
+      X3 += (size_t)48 * rw.n_out;
+    }
+    return;
+  }
+  if constexpr (BY_ROW) {
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
     constexpr int NC = ROWS == 2 ? NJ / 2 : NJ;
 #pragma unroll
@@ -407,7 +479,7 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
 
 template <typename T, int BM, int BN, bool B_KN, bool F32OUT = false, int BDIV = 1, int ROWS = 0>
 hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, const float* residual = nullptr, const DmaRows& rw = DmaRows()) {
-  constexpr int STAGES = 2 * (BM + BN) * BK * 2, EPI = F32OUT || ROWS ? 0 : BM * (BN * 2 + 8);
+  constexpr int STAGES = 2 * (BM + BN) * BK * 2, EPI = ROWS == 4 ? BM * (3 * BN + 16) : F32OUT || ROWS ? 0 : BM * (BN * 2 + 8);
   constexpr int LDS_BYTES = STAGES > EPI ? STAGES : EPI;
   static std::atomic<unsigned long long> configured{0};  // one bit per device: the attribute is per device
   // the schedule with two barriers, except where it does not fit the registers (the transposing reads of the
@@ -632,8 +704,14 @@ void gemm_dma_planes3_name(int tile, int nsplit, const char* tail, char* out, si
   snprintf(out, out_len, "gemm_dma4<bf16,NT,%dx%d,%s,3 planes%s,f32 out%s>", bm, bn, waves_name(tile), split, tail ? tail : "");
 }
 
-hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile, int nsplit, const float* residual, const char* note_tail) {
-  if (p.b_k_div != 3 || !(p.b_rs == 1 && p.b_cs != 1) || !gemm_dma_planes3_split_ok(p, nsplit) || (nsplit > 1 && residual)) return hipErrorInvalidValue;
+// (the up rows of a tile lie n_out rows behind its gate rows, and both are reached from the matrix's first row with 32-bit offsets)
+bool gemm_dma_planes3_gates(const MMArgs& p, int tile, int nsplit) {
+  return tile == 192 && nsplit == 1 && p.N % 16 == 0 && (unsigned long long)p.b_cs * 2 * p.N < (1ull << 32);
+}
+
+hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile, int nsplit, const float* residual, const char* note_tail, bool gated, uint16_t* gated_planes) {
+  if (p.b_k_div != 3 || !(p.b_rs == 1 && p.b_cs != 1) || !gemm_dma_planes3_split_ok(p, nsplit) || (nsplit > 1 && residual) || (gated && !gemm_dma_planes3_gates(p, tile, nsplit)))
+    return hipErrorInvalidValue;
   MMArgs q = p;
   if (nsplit > 1) {
     q.K = p.K / nsplit;
@@ -646,6 +724,12 @@ hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile
   note_kernel("%s", name);
   if (ring_tile(tile)) return gemm_ring_launch(stream, UGHIP_BF16, DmaForm::PLANES3, q, (size_t)nsplit, tile, residual, DmaRows());
   if (tile == 256) return launch<__bf16, 256, 256, false, true, 3>(stream, q, (size_t)nsplit, residual);
+  if (tile == 192 && gated) {
+    DmaRows rw;
+    rw.dst = gated_planes ? static_cast<void*>(gated_planes) : p.c, rw.n_out = p.N / 2, rw.dst_bf16 = gated_planes != nullptr;
+    if (gated_planes && (rw.n_out % 64 || !aligned16(gated_planes))) return hipErrorInvalidValue;
+    return launch<__bf16, 256, 192, false, true, 3, 4>(stream, q, 1, nullptr, rw);
+  }
   if (tile == 192) return launch<__bf16, 256, 192, false, true, 3>(stream, q, (size_t)nsplit, residual);
   if (tile == 128) return launch<__bf16, 256, 128, false, true, 3>(stream, q, (size_t)nsplit, residual);
   return launch<__bf16, 128, 128, false, true, 3>(stream, q, (size_t)nsplit, residual);

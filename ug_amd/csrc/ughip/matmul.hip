@@ -907,7 +907,9 @@ static int linear_rows_core(ughip_device* dev, const char* what, const float* x,
     return UGHIP_OK;
   }
   const int dma_tile = route.dma_tile, dma_split = route.dma_split;
-  const bool dma_fold = dma_tile && (dma_split > 1 || kind == GemmEpilogue::SWIGLU);
+  const bool dma_gates = dma_tile && kind == GemmEpilogue::SWIGLU && gemm_dma_planes3_gates(p, dma_tile, dma_split);
+  const bool dma_fold = dma_tile && !dma_gates && (dma_split > 1 || kind == GemmEpilogue::SWIGLU);
+  const bool to_planes = dma_tile && kind == GemmEpilogue::SWIGLU && ar && ar->planes_out && out_cols % 64 == 0;
   const size_t ws_bytes = dma_tile ? (dma_fold ? ((size_t)dma_split * m * rows * sizeof(float) + 255) & ~(size_t)255 : 0)
                                    : (gemm_tiled_workspace_bytes(dtype, p, 1, &epi) + 255) & ~(size_t)255;
   const size_t x3_bytes = x3 && !planes_in ? m * 3 * k * sizeof(uint16_t) : 0;
@@ -928,7 +930,6 @@ static int linear_rows_core(ughip_device* dev, const char* what, const float* x,
   if (dma_tile) {
     if (dma_fold) {
       p.c = dev->gemm_ws;
-      const bool to_planes = kind == GemmEpilogue::SWIGLU && ar && ar->planes_out && out_cols % 64 == 0;
       UGHIP_HIPCHK(gemm_dma_launch_planes3(dev->stream, p, dma_tile, dma_split, nullptr, to_planes ? ",swiglu fold onto planes" : dma_planes_tail(kind, true, false)));
       if (to_planes) {
         const size_t elems = m * rows, n4 = elems / 8;
@@ -938,6 +939,10 @@ static int linear_rows_core(ughip_device* dev, const char* what, const float* x,
       } else {
         UGHIP_HIPCHK(gemm_fold_f32(dev->stream, static_cast<const float*>(dev->gemm_ws), dst, m, rows, dma_split, kind, epi.residual));
       }
+    } else if (dma_gates) {
+      UGHIP_HIPCHK(gemm_dma_launch_planes3(dev->stream, p, dma_tile, 1, nullptr, to_planes ? ",in-register swiglu fold onto planes" : ",in-register swiglu fold", true,
+                                           to_planes ? ar->planes_out : nullptr));
+      if (ar) ar->wrote_planes = to_planes;
     } else {
       UGHIP_HIPCHK(gemm_dma_launch_planes3(dev->stream, p, dma_tile, 1, epi.residual, dma_planes_tail(kind, false, epi.residual != nullptr)));
     }
@@ -1076,7 +1081,8 @@ extern "C" int ughip_linear_rows_plan(int w_dtype, int product, int form, size_t
     rows_x3_name(route.x3, kind, buf, buf_len);
   } else if (route.kind == RowsRoute::DMA_PLANES) {
     const bool fold = route.dma_split > 1 || kind == GemmEpilogue::SWIGLU;
-    gemm_dma_planes3_name(route.dma_tile, route.dma_split, dma_planes_tail(kind, fold, form == 1), buf, buf_len);
+    const bool gates = kind == GemmEpilogue::SWIGLU && gemm_dma_planes3_gates(p, route.dma_tile, route.dma_split);
+    gemm_dma_planes3_name(route.dma_tile, route.dma_split, gates ? ",in-register swiglu fold" : dma_planes_tail(kind, fold, form == 1), buf, buf_len);
   } else {
     gemm_tiled_name(dtype, p, 1, mixed, &epi, buf, buf_len);
   }
