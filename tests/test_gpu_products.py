@@ -188,6 +188,30 @@ def test_rows_by_group(hip, tune, groups, rows):
             close(out[: rows * n].reshape(rows, n), y, 2e-5)
 
 
+# groups of every height's first and last size, of none, one and two tiles and more; the shortest K loops and an odd one; columns that hang over the tile
+@pytest.mark.parametrize("n, k", [(96, 64), (200, 128), (264, 192), (136, 448)])
+@pytest.mark.parametrize("act", [NONE, SWIGLU])
+def test_tiles_as_high_as_their_groups(hip, tune, n, k, act):
+    """Every k order is the other tiles': the same bits, gathered rows and bf16 results too."""
+    sizes = [0, 1, 16, 17, 63, 64, 65, 0, 127, 128, 129, 191, 192, 193, 255, 256, 257, 300, 511, 512, 513, 770]
+    gpu, m, rows = Gpu(hip), sum(sizes), n if act == NONE else 2 * n
+    x, w = rand(1, m, k), rand(2, len(sizes), rows, k, std=k ** -0.5)
+    dx, dw = gpu.up(x, bf16=True), gpu.up(w, bf16=True)
+    src, end = gpu.up(np.random.default_rng(3).integers(0, m, m).astype(np.int32)), gpu.up(np.cumsum(sizes).astype(np.int32))
+    got = {}
+    for shape, tile in (("9", "64x64"), ("15", "256x192"), ("16", "256x128")):
+        tune.setenv("UGHIP_GEMM_SHAPE", shape)
+        dst = gpu.out(m * n + 8)
+        print("as high as their groups", n, k, act, tile, flush=True)
+        gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=BF16, act=act, row_index=src.raw(), group_end=end.raw(),
+                                                       groups=len(sizes), x_rows=m)))
+        assert f"{tile},512t,ring,rows" in ug_amd.last_kernel()
+        got[tile] = get(dst, m * n + 8)
+        assert np.all(np.isnan(got[tile][m * n :])) and np.all(np.isfinite(got[tile][: m * n]))
+    np.testing.assert_array_equal(got["256x192"], got["64x64"])
+    np.testing.assert_array_equal(got["256x128"], got["64x64"])
+
+
 @pytest.mark.parametrize("shape, kernel", [("3", "gemm_dma4<bf16,NT,256x256,256t,rows>"), ("4", "gemm_dma4<bf16,NT,256x128,512t,ring,rows>"), ("5", "gemm_dma4<bf16,NT,128x128,512t,ring,rows>"),
                                            ("0", "rows_product<bf16,none>"), ("6", "rows_product<bf16,none>"), ("7", "rows_product<bf16,none>")])
 def test_forced_tiles_of_rows(hip, tune, shape, kernel):

@@ -86,7 +86,8 @@ __device__ __forceinline__ int wave_scan(int v, F f) {
 // Rows sorted by group, ceil(rows / BM) tile rows to each: a lane per group, 64 at a time.  Every workgroup asks for it before its first load, one
 // that finds no tile of its own too, and mostly has its CU to itself: read one after the other by scalar loads the ends took it 0.1-0.15 us each
 // (64 groups, n = 2 x 552, k = 128, 1638 rows: 49 us so, on 64 x 128 tiles, 12.8 with a lane per group; 18.9 in rows_product).
-template <int BM>
+// EVEN: a group's rows in shares of equal size, whole 16s (BM % 16 == 0: no share is larger than BM, and as rows are more than (tiles - 1) BM, none is empty).
+template <int BM, bool EVEN = false>
 struct GroupTiles {
   const int* group_end;
   int groups, m, lane;
@@ -115,7 +116,13 @@ struct GroupTiles {
       if (!behind) continue;
       const int l = __builtin_ctzll(behind), first = __builtin_amdgcn_readlane(begin, l);
       group = base + l, m_end = __builtin_amdgcn_readlane(end, l);
-      m0 = first + (tile - __builtin_amdgcn_readlane(upto, l) + (m_end - first + BM - 1) / BM) * BM;
+      const int n = (m_end - first + BM - 1) / BM, at = tile - __builtin_amdgcn_readlane(upto, l) + n;
+      if constexpr (EVEN) {
+        const int share = ((m_end - first + n - 1) / n + 15) / 16 * 16;
+        m0 = first + at * share, m_end = min(m_end, m0 + share);
+      } else {
+        m0 = first + at * BM;
+      }
       return true;
     }
     return false;

@@ -24,6 +24,7 @@
 // issue slots, not waiting time -- warming L2 ahead of them or four stages of 32 k instead of two of 64 made it slower).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -506,11 +507,11 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 namespace {
 // tile codes of the entry points below: 256 = 256 x 256, 192 = 256 x 192 (three planes only), 128 = 256 x 128, 64 = 128 x 128; on gemm_ring 129 = 256 x 128, 65 = 128 x 128, 48 = 64 x 128,
-// 32 = 64 x 64 ([n, k]-major rhs only), 97 = 192 x 192 (rows only)
+// 32 = 64 x 64 ([n, k]-major rhs only), 97 = 192 x 192 (rows only), 193 / 130 = 256 x 192 / 256 x 128 and lower ones of that width (rows by group only)
 bool tile_dims(int tile, int* bm, int* bn) {
   if (tile == 256) *bm = 256, *bn = 256;
-  else if (tile == 192) *bm = 256, *bn = 192;
-  else if (tile == 128 || tile == 129) *bm = 256, *bn = 128;
+  else if (tile == 192 || tile == 193) *bm = 256, *bn = 192;
+  else if (tile == 128 || tile == 129 || tile == 130) *bm = 256, *bn = 128;
   else if (tile == 97) *bm = 192, *bn = 192;
   else if (tile == 64 || tile == 65) *bm = 128, *bn = 128;
   else if (tile == 48) *bm = 64, *bn = 128;
@@ -524,7 +525,8 @@ static size_t tile_count(const MMArgs& p, size_t batch, int tile) {  // 0: no su
   int bm, bn;
   return tile_dims(tile, &bm, &bn) ? batch * (size_t)((p.M + bm - 1) / bm) * (size_t)((p.N + bn - 1) / bn) : 0;
 }
-static bool ring_tile(int tile) { return tile == 129 || tile == 97 || tile == 65 || tile == 48 || tile == 32; }
+static bool by_height(int tile) { return tile == 193 || tile == 130; }  // rows by group: tiles of up to that height
+static bool ring_tile(int tile) { return tile == 129 || by_height(tile) || tile == 97 || tile == 65 || tile == 48 || tile == 32; }
 static int least_k(int tile) { return ring_tile(tile) ? BK : 4 * BK; }
 static const char* waves_name(int tile) { return ring_tile(tile) ? "512t,ring" : "256t"; }  // in the names of these kernels
 // (tuning aid) the tile code that GEMM_SHAPE names, 0: none of these kernels'
@@ -539,6 +541,8 @@ int gemm_dma_forced_tile(long long shape) {
     case 12: return 65;
     case 13: return 48;
     case 14: return 192;
+    case 15: return 193;
+    case 16: return 130;
   }
   return 0;
 }
@@ -550,7 +554,7 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || batch == 0) return false;
   if (p.a_cs != 1 || p.a_rs % 8 || (batch > 1 && (p.a_bs % 8 || p.b_bs % 8 || p.c_bs % 8))) return false;
   const bool nn = p.b_cs == 1 && p.b_rs != 1, nt = p.b_rs == 1 && p.b_cs != 1;
-  if (nn == nt || (nn && tile == 32) || tile == 97 || (tile == 192 && p.b_k_div != 3)) return false;
+  if (nn == nt || (nn && tile == 32) || tile == 97 || by_height(tile) || (tile == 192 && p.b_k_div != 3)) return false;
   const long long ldb = nn ? p.b_rs : p.b_cs;
   if (ldb % 8) return false;
   // per-lane offsets are 32-bit: the furthest row of a tile has to stay below 4 GiB from the tile's first byte
@@ -738,7 +742,8 @@ hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile
 
 bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int tile) {
   int bm, bn;
-  if (!tile_dims(tile, &bm, &bn) || (tile != 256 && !ring_tile(tile)) || ((tile == 256 || tile == 97) && act == RowsAct::LOOKUP)) return false;
+  if (!tile_dims(tile, &bm, &bn) || (tile != 256 && !ring_tile(tile)) || ((tile == 256 || tile == 97) && act == RowsAct::LOOKUP) || (by_height(tile) && (!r.groups || act == RowsAct::LOOKUP)))
+    return false;
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || p.a_cs != 1 || p.a_rs % 8 || p.b_rs != 1 || p.b_cs % 8) return false;
   if (r.n_out <= 0 || r.n_out % 4 || p.N != (act == RowsAct::GLU ? 2 * r.n_out : r.n_out) || r.dst_stride % 4 || r.w_group % 8) return false;
   // per-lane offsets are 32-bit: rows of x anywhere, matrix rows of a tile (of the whole matrix with SwiGLU)
@@ -746,6 +751,39 @@ bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int
   if (x_rows * p.a_rs * 2 >= (1ull << 31) || (unsigned long long)p.b_cs * 2 * (act == RowsAct::GLU ? p.N : bn) >= (1ull << 31)) return false;
   if (!aligned16(p.a) || !aligned16(p.b) || !aligned16(r.dst) || (r.bias && !aligned16(r.bias))) return false;
   return ((size_t)(p.M + bm - 1) / bm + r.groups) * (size_t)((p.N + bn - 1) / bn) < (1u << 24);
+}
+
+// What rows by group take.  How they are spread is not known here: eighths of the groups have SHARE of an even one's rows, as the shares of a router's experts come
+// out that differ by 40 % (taken as even, groups of 127 rows went to 192 x 192 tiles, of which one in eight is then two: 85 us where 59 are possible).  Every K tile brings a
+// matrix's columns from memory that at most a few workgroups share, 1.8 times the time that one matrix's tiles take.  Tiles by height (193, 130): a K tile by the
+// height in 64s; one round lasts for its highest tiles mostly, several go by the mean and leave one of the highest behind.
+// Fitted to 48 products of 16 groups (n 2 x 1408 and k 2048, n 2048 and k 1408, half of both; 512 to 8192 rows) on each of eight tiles: the choice is within 0.2 % of the best in the
+// mean, 5 % at most.  Gate and up, then down, of width 2048, us before and so: 768 rows 50.6 / 33.3 -> 47 / 25; 1280 50.6 / 47 -> 50 / 28; 1600 51 / 46 -> 51 / 30; 2036 84 / 37 -> 59 / 35;
+// 2560 67 / 59 -> 67 / 41; 3200 67 / 61 -> 67 / 47; 4096 80 / 55 -> 70 / 48; 8192 124 / 90 -> 124 / 83; of width 1024, 5200 rows 47 / 27 -> 36 / 27.
+static double grouped_cost_us(const MMArgs& p, int groups, int tile) {
+  static const double SHARE[8] = {0.50, 0.65, 0.76, 0.87, 0.98, 1.12, 1.32, 1.70};
+  static const double WIDE[4] = {1.0, 1.2, 1.5, 1.7}, NARROW[4] = {0.6, 0.83, 1.2, 1.3};  // us per K tile, 192 and 128 columns
+  int bm, bn;
+  tile_dims(tile, &bm, &bn);
+  const double even = (double)p.M / groups, columns = (p.N + bn - 1) / bn, kt = p.K / BK;
+  double tiles = 0, sum = 0, highest = 0;
+  for (double share : SHARE) {
+    const int rows = std::max(1, (int)(even * share + 0.999)), n = (rows + bm - 1) / bm;
+    const double count = groups / 8.0 * n * columns;
+    tiles += count;
+    if (!by_height(tile)) continue;
+    const int height = std::min(4, (((rows + n - 1) / n + 15) / 16 * 16 + 63) / 64);
+    const double us = (tile == 193 ? WIDE : NARROW)[height - 1];
+    sum += count * us, highest = std::max(highest, us);
+  }
+  if (by_height(tile)) return 5.0 + kt * (tiles <= 256 ? 0.8 * highest + 0.2 * sum / tiles : sum / 256 + 0.77 * highest);
+  if (tile == 256) {
+    double us = 6.0;
+    for (double left = tiles; left > 0; left -= 256) us += 1.66 * kt * (1.23 + 0.33 * std::min(left, 256.0) / 256.0);
+    return us;
+  }
+  const double fixed = ring_cost_us(0, (int)kt, tile, Operands::MEMORY);
+  return fixed + 1.8 * (ring_cost_us((size_t)(tiles + 0.5), (int)kt, tile, Operands::MEMORY) - fixed);
 }
 
 int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
@@ -756,28 +794,28 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
   // A model's products: the matrix comes from memory.  256 x 256 tiles of gemm_dma4 and the ring's, by what they are expected to take
   // (2048 positions: down 74 -> 51 us, gate and up 105 -> 89, output 26 -> 18, attention's input 37 -> 29; 509 positions: state-space output
   // 53 -> 19, input 43 -> 32, dense gate and up 40 -> 30; 700 positions' gate and up 52 -> 34; 33 rows of 11264 x 2048 31 -> 13).
-  // By group, how the rows are spread is not known here; the model takes them as even.  16 experts' gate and up (n = 2 x 1408, k = 2048) whose shares
-  // of the rows differ by 40 %, 256 x 256 / 256 x 128 / 192 x 192 / 128 x 128: 1000 rows 56 / 65 / 46 / 54 us, 2036 59 / 68 / 46 / 66, 2800 59 / 73 / 75 / 74, 4096
-  // 103 / 91 / 74 / 89; a router whose groups of 2036 rows run from 60 to 260 takes 52 to 72 on 192 x 192 (rows past 192 are a second round) and 70
-  // on 256 x 256.
-  const size_t groups = r.groups ? r.groups : 1;
-  const double m = (double)p.M / groups;  // rows as if they were spread evenly
   int best = 0;
   double best_us = 0;
+  if (r.groups > 1) {
+    for (int tile : {256, 129, 65, 48, 32, 97, 193, 130}) {
+      if (!gemm_dma_rows_supported(p, r, act, tile)) continue;
+      const double us = grouped_cost_us(p, r.groups, tile);
+      if (!best || us < best_us) best = tile, best_us = us;
+    }
+    return best;
+  }
   for (int tile : {256, 129, 65, 48, 32, 97}) {
     if (!gemm_dma_rows_supported(p, r, act, tile)) continue;
     int bm, bn;
     tile_dims(tile, &bm, &bn);
-    // tile rows: of groups near or above a tile's height every second one takes one more
-    const double rows = groups == 1 ? (p.M + bm - 1) / bm : m < 0.8 * bm ? groups : groups * (m / bm + 0.5);
-    const size_t tiles = (size_t)(rows + 0.5) * ((p.N + bn - 1) / bn);
+    const size_t tiles = (size_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
     const int kt = p.K / BK;
     double us = 6.0;
     if (tile == 256)
       for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (1.23 + 0.33 * (left < 256 ? (double)left : 256.0) / 256.0);
     else us = ring_cost_us(tiles, kt, tile, Operands::MEMORY);
-    // the larger tile on a near tie; 192 x 192 last: for one matrix where it clearly saves a round, by group from the same margin on as the others
-    if (!best || us < best_us * (tile == 97 && groups == 1 ? 0.9 : 0.97)) best = tile, best_us = us;
+    // the larger tile on a near tie; 192 x 192 last, where it clearly saves a round
+    if (!best || us < best_us * (tile == 97 ? 0.9 : 0.97)) best = tile, best_us = us;
   }
   return best;
 }

@@ -24,16 +24,18 @@
 namespace ughip {
 namespace {
 
-constexpr int stages(int bm) { return bm >= 192 ? 3 : 4; }
+constexpr int stages(int bm, int bn) { return bm == 256 && bn == 192 ? 2 : bm >= 192 || bm * bn > 128 * 128 ? 3 : 4; }
+constexpr int lds_bytes(int bm, int bn) { return stages(bm, bn) * (bm + bn) * BK * 2; }
 
+// One tile: rows [m0, m_end) (BM of them at most) and the columns of column tile tn, of one batch or group.
 // Template parameters and DmaRows as in gemm_dma4; ROWS 3: rows that leave as gelu(y) times an element of their token's row of a table.
 template <typename T, int BM, int BN, bool B_KN, bool F32OUT, int BDIV, int ROWS>
-__global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tiles_m, int tiles_n, const float* __restrict__ residual, DmaRows rw) {
+__device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group, int m0, int m_end, int tn, const float* __restrict__ residual, const DmaRows& rw) {
   static_assert(ROWS == 0 || (BDIV == 1 && !B_KN && !F32OUT), "rows: one plane against an [n, k]-major rhs");
   static_assert(BDIV == 1 || !B_KN, "planes of the lhs: against an [n, k]-major rhs only");
   static_assert(!B_KN || BN >= 128, "the swizzle of an n-contiguous tile wants eight 32-byte pieces per row");
   extern __shared__ u32x4 lds[];
-  constexpr int S = stages(BM);
+  constexpr int S = stages(BM, BN);
   constexpr int NI = BM / 64, NJ = BN / 32, NM = NI * NJ;  // 16-row and 16-column fragments and MFMAs of a wave and step of 32 k
   constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, STAGE_BYTES = A_BYTES + B_BYTES;
   constexpr int NDA = BM / 64, NDB = BN / 64, ND = NDA + NDB;   // loads per wave and K tile
@@ -41,32 +43,7 @@ __global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tile
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  // XCD-aware order of the tiles: as in gemm_dma4 (the grid is 8 more at least, the runs are of equal length)
-  int tiles = batches * tiles_m * tiles_n;
-  GroupTiles<BM> by_group{rw.group_end, rw.groups, p.M, lane};
-  if (ROWS != 0 && rw.groups) {
-    tiles_m = by_group.count();
-    tiles = tiles_m * tiles_n;
-  }
-  const int per = (tiles + 7) >> 3;
-  if ((int)blockIdx.x >= 8 * per) return;
-  const int bid = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
-  if (bid >= tiles) return;
-  const int tpb = tiles_m * tiles_n;
-  const int batch = bid / tpb;
-  const int t_in = bid - batch * tpb;
-  int tm, tn;
-  if ((tiles_m & 3) == 0) {
-    const int sr = t_in / (4 * tiles_n), rem = t_in - sr * 4 * tiles_n;
-    tm = sr * 4 + (rem & 3);
-    tn = rem >> 2;
-  } else {
-    tm = t_in / tiles_n;
-    tn = t_in - tm * tiles_n;
-  }
-  int m0 = tm * BM, m_end = p.M, group = 0;
   const int n0 = tn * BN;
-  if (ROWS != 0 && rw.groups && !by_group.find(tm, group, m0, m_end)) return;  // the same for the whole workgroup
   const long long lda = p.a_rs, ldb = B_KN ? p.b_rs : p.b_cs;
   const char* Ab = reinterpret_cast<const char*>(static_cast<const T*>(p.a) + (size_t)batch * p.a_bs + (ROWS ? 0 : (size_t)m0 * lda));
   const char* Bb = reinterpret_cast<const char*>(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs + (ROWS ? (size_t)group * rw.w_group : 0) +
@@ -187,10 +164,12 @@ __global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tile
 #pragma unroll
   for (int r = 0; r < R; ++r) read_frag(0, 0, r, 0);
   for (int kt = 0; kt < KT - S; ++kt) body(kt, CS());
-  if constexpr (S == 4) {
+  if constexpr (S > 3) {
     if (KT > 3) body(KT - 4, std::integral_constant<int, 3>());
   }
-  if (KT > 2) body(KT - 3, std::integral_constant<int, 2>());
+  if constexpr (S > 2) {
+    if (KT > 2) body(KT - 3, std::integral_constant<int, 2>());
+  }
   if (KT > 1) body(KT - 2, C1());
   body(KT - 1, C0());
 
@@ -283,22 +262,93 @@ __global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tile
   }
 }
 
+// The tiles of a launch, dealt to its workgroups.
 template <typename T, int BM, int BN, bool B_KN, bool F32OUT, int BDIV, int ROWS>
-hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, const float* residual, const DmaRows& rw) {
-  constexpr int LDS_BYTES = stages(BM) * (BM + BN) * BK * 2;  // the result's rows fit as well
-  static_assert(LDS_BYTES >= BM * (BN * 2 + 8));
-  static std::atomic<unsigned long long> configured{0};  // one bit per device: the attribute is per device
-  auto kernel = gemm_ring<T, BM, BN, B_KN, F32OUT, BDIV, ROWS>;
+__global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tiles_m, int tiles_n, const float* __restrict__ residual, DmaRows rw) {
+  const int lane = threadIdx.x & 63;
+  // XCD-aware order of the tiles: as in gemm_dma4 (the grid is 8 more at least, the runs are of equal length)
+  int tiles = batches * tiles_m * tiles_n;
+  GroupTiles<BM> by_group{rw.group_end, rw.groups, p.M, lane};
+  if (ROWS != 0 && rw.groups) {
+    tiles_m = by_group.count();
+    tiles = tiles_m * tiles_n;
+  }
+  const int per = (tiles + 7) >> 3;
+  if ((int)blockIdx.x >= 8 * per) return;
+  const int bid = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  if (bid >= tiles) return;
+  const int tpb = tiles_m * tiles_n;
+  const int batch = bid / tpb;
+  const int t_in = bid - batch * tpb;
+  int tm, tn;
+  if ((tiles_m & 3) == 0) {
+    const int sr = t_in / (4 * tiles_n), rem = t_in - sr * 4 * tiles_n;
+    tm = sr * 4 + (rem & 3);
+    tn = rem >> 2;
+  } else {
+    tm = t_in / tiles_n;
+    tn = t_in - tm * tiles_n;
+  }
+  int m0 = tm * BM, m_end = p.M, group = 0;
+  if (ROWS != 0 && rw.groups && !by_group.find(tm, group, m0, m_end)) return;  // the same for the whole workgroup
+  ring_tile<T, BM, BN, B_KN, F32OUT, BDIV, ROWS>(p, batch, group, m0, m_end, tn, residual, rw);
+}
+
+// Rows by group (bf16), each group's rows dealt evenly over as few tiles of at most 256 rows as hold them and every tile as high as its rows want, in steps of
+// 64.  What bounds such a product are its operands' bytes on their way to the CUs, in rounds of 256 workgroups: tiles of one height load and multiply
+// rows that nobody asked for, and a few groups above that height are a second round of nearly empty tiles.  16 groups, us on the best of the tiles of one height and so: n 2 x 1408,
+// k 2048, 768 rows 50.6 -> 47.1 (192 columns); n 2048, k 1408, 768 / 1024 / 1280 / 1600 rows 28.4 / 30.3 / 31.6 / 34.5 -> 25.1 / 26.3 / 28.1 / 30.4 (128 columns), 3200 / 4096 / 8192
+// rows 54.5 / 55 / 88 -> 47 / 48 / 83 (192 columns).
+template <int BN, int ROWS>
+__global__ void __launch_bounds__(512) gemm_ring_groups(MMArgs p, int tiles_n, DmaRows rw) {
+  GroupTiles<256, true> by_group{rw.group_end, rw.groups, p.M, (int)threadIdx.x & 63};
+  const int tiles_m = by_group.count(), tiles = tiles_m * tiles_n, per = (tiles + 7) >> 3;
+  if ((int)blockIdx.x >= 8 * per) return;
+  const int bid = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  if (bid >= tiles) return;
+  const int tm = bid / tiles_n, tn = bid - tm * tiles_n;
+  int m0, m_end, group;
+  if (!by_group.find(tm, group, m0, m_end)) return;
+  const int rows = m_end - m0;
+  if (rows <= 64) ring_tile<__bf16, 64, BN, false, false, 1, ROWS>(p, 0, group, m0, m_end, tn, nullptr, rw);
+  else if (rows <= 128) ring_tile<__bf16, 128, BN, false, false, 1, ROWS>(p, 0, group, m0, m_end, tn, nullptr, rw);
+  else if (rows <= 192) ring_tile<__bf16, 192, BN, false, false, 1, ROWS>(p, 0, group, m0, m_end, tn, nullptr, rw);
+  else ring_tile<__bf16, 256, BN, false, false, 1, ROWS>(p, 0, group, m0, m_end, tn, nullptr, rw);
+}
+
+template <typename K>
+hipError_t allow_lds(K kernel, int bytes, std::atomic<unsigned long long>& configured) {  // configured: one bit per device, the attribute is per device
   int dev = 0;
   if (hipError_t e = hipGetDevice(&dev)) return e;
   const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
-  if (!bit || !(configured.load(std::memory_order_relaxed) & bit)) {
-    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES)) return e;
-    configured.fetch_or(bit, std::memory_order_relaxed);
-  }
+  if (bit && (configured.load(std::memory_order_relaxed) & bit)) return hipSuccess;
+  if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes)) return e;
+  configured.fetch_or(bit, std::memory_order_relaxed);
+  return hipSuccess;
+}
+
+template <typename T, int BM, int BN, bool B_KN, bool F32OUT, int BDIV, int ROWS>
+hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, const float* residual, const DmaRows& rw) {
+  constexpr int LDS_BYTES = lds_bytes(BM, BN);  // the result's rows fit as well
+  static_assert(LDS_BYTES >= BM * (BN * 2 + 8));
+  static std::atomic<unsigned long long> configured{0};
+  auto kernel = gemm_ring<T, BM, BN, B_KN, F32OUT, BDIV, ROWS>;
+  if (hipError_t e = allow_lds(kernel, LDS_BYTES, configured)) return e;
   const int tiles_m = (p.M + BM - 1) / BM + rw.groups, tiles_n = (p.N + BN - 1) / BN;
   const size_t total = (batch * (size_t)tiles_m * tiles_n + 7) / 8 * 8 + (rw.groups ? 8 : 0);
   kernel<<<dim3((unsigned)total), dim3(512), LDS_BYTES, stream>>>(p, (int)batch, tiles_m, tiles_n, residual, rw);
+  return hipGetLastError();
+}
+
+template <int BN, int ROWS>
+hipError_t launch_groups(hipStream_t stream, const MMArgs& p, const DmaRows& rw) {
+  constexpr int A = lds_bytes(64, BN), B = lds_bytes(128, BN), C = lds_bytes(192, BN), D = lds_bytes(256, BN);
+  constexpr int AB = A > B ? A : B, CD = C > D ? C : D, LDS_BYTES = AB > CD ? AB : CD;
+  static std::atomic<unsigned long long> configured{0};
+  auto kernel = gemm_ring_groups<BN, ROWS>;
+  if (hipError_t e = allow_lds(kernel, LDS_BYTES, configured)) return e;
+  const int tiles_m = (p.M + 255) / 256 + rw.groups, tiles_n = (p.N + BN - 1) / BN;
+  kernel<<<dim3((unsigned)(((size_t)tiles_m * tiles_n + 7) / 8 * 8 + 8)), dim3(512), LDS_BYTES, stream>>>(p, tiles_n, rw);
   return hipGetLastError();
 }
 
@@ -308,6 +358,8 @@ hipError_t launch_nt(hipStream_t stream, const MMArgs& p, size_t batch, int tile
     if (tile == 129) return launch<T, 256, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
   }
   if constexpr (ROWS == 1 || ROWS == 2) {
+    if (tile == 193) return launch_groups<192, ROWS>(stream, p, rw);
+    if (tile == 130) return launch_groups<128, ROWS>(stream, p, rw);
     if (tile == 97) return launch<T, 192, 192, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
   }
   if (tile == 65) return launch<T, 128, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
