@@ -169,6 +169,26 @@ def test_grouped_attention_over_many_splits(gpu):
             close(got, want, 1e-4)
 
 
+# more workgroups than CUs, an odd and an even number of blocks of queries, the last one partial; results by fours and one by one; all positions in two cuts
+@pytest.mark.parametrize("sizes, cuts", [((16, 4, 64, 64, 0), (1075,)), ((16, 4, 64, 60, 0), (1100,)), ((18, 2, 128, 128, 0), (33, 1030)), ((16, 16, 192, 128, 0), (1090,))])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_grouped_attention_of_long_and_short_rows(gpu, sizes, cuts, bf16):
+    H, G, d, vd, _ = sizes
+    T, scale = sum(cuts), d ** -0.5
+    qkv = rng.bf16_round(rand(5, T, (H + G) * d + G * vd).astype(np.float32).ravel()).reshape(T, -1).astype(np.float64)
+    k, v = qkv[:, H * d : (H + G) * d].reshape(T, G, d), qkv[:, (H + G) * d :].reshape(T, G, vd)
+    q = qkv[:, : H * d].reshape(T, H, d)
+    want, spread = pt.grouped_attention(q, k, v, scale), pt.grouped_attention(q, k, np.abs(v), scale)
+    # bf16: a query times its scale is rounded once, so a score is off by at most 2^-9 of its terms' sizes, a weight by the power of twice that (both sums move)
+    off = np.stack([2.0 ** -9 * scale * (np.abs(q[:, h]) @ np.abs(k[:, h // (H // G)]).T).max(1) for h in range(H)], 1)
+    bound = 1e-4 * np.sqrt(np.mean(want ** 2)) + (np.expm1(2 * off)[:, :, None] * spread if bf16 else np.zeros_like(spread))
+    caches, pos = caches_for(gpu, G, d, vd, T, bf16), 0
+    for t in cuts:
+        got = attend(gpu, bf16, qkv, caches, T, t, pos, sizes, 0, scale, None, None)
+        assert np.all(np.abs(got - want[pos : pos + t]) <= bound[pos : pos + t])
+        pos += t
+
+
 # ---- delta rule --------------------------------------------------------------------------------------------------------------
 # (heads, kv_heads, dim, vdim, taps, decay rank, gate rank)
 DELTAS = [(1, 1, 1, 1, 1, 1, 1), (6, 2, 18, 21, 3, 7, 5), (4, 4, 64, 64, 4, 16, 8), (2, 1, 128, 128, 2, 24, 128), (3, 3, 100, 40, 5, 64, 136), (2, 2, 190, 24, 4, 8, 8), (1, 1, 256, 250, 3, 16, 16)]

@@ -458,12 +458,7 @@ int attend_many(ughip_device* dev, GroupedArgs g, AttRowsArgs r) {
   if (int rc = rows_scratch(dev, (size_t)g.heads * g.q_rows * DQ * sizeof(T), &g.qp)) return rc;
   if (int rc = place<T, DQ>(dev, g)) return rc;
   r.q = g.qp, r.q_rows = g.q_rows, r.k_rows = (int)g.cap;
-  constexpr int bytes = attention_rows_lds_bytes<T, DQ, DV>();
-  static_assert(bytes <= 160 * 1024, "tile does not fit LDS");
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_rows_kernel<T, DQ, DV>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  UGHIP_HIPCHK(attr);
-  attention_rows_kernel<T, DQ, DV><<<dim3((unsigned)g.heads, (unsigned)(g.q_rows / ATT_QT)), attention_rows_threads<T, DQ, DV>(), bytes, dev->stream>>>(r);
-  UGHIP_HIPCHK(hipGetLastError());
+  UGHIP_HIPCHK((attention_rows_launch<T, DQ, DV>(dev, r, g.heads)));
   return UGHIP_OK;
 }
 

@@ -112,10 +112,6 @@ __global__ void __launch_bounds__(256) latent_pack_kernel(PackArgs a) {
 
 template <typename T, int DQ, int DV>
 int launch_rows(ughip_device* dev, AttRowsArgs a, PackArgs pk) {
-  constexpr int bytes = attention_rows_lds_bytes<T, DQ, DV>();
-  static_assert(bytes <= 160 * 1024, "tile does not fit LDS");
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_rows_kernel<T, DQ, DV>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  UGHIP_HIPCHK(attr);
   pk.q_rows = (pk.t + ATT_QT - 1) / ATT_QT * ATT_QT, pk.k_rows = (pk.pos + pk.t + ATT_KT - 1) / ATT_KT * ATT_KT;
   const size_t q_bytes = (size_t)pk.heads * pk.q_rows * DQ * sizeof(T), k_bytes = (size_t)pk.heads * pk.k_rows * DQ * sizeof(T);
   void* ws = nullptr;
@@ -126,8 +122,7 @@ int launch_rows(ughip_device* dev, AttRowsArgs a, PackArgs pk) {
   const size_t pieces = (size_t)(pk.q_rows + pk.k_rows) * CH;
   latent_pack_kernel<T, DQ><<<dim3((unsigned)((pieces + 255) / 256), (unsigned)pk.heads), 256, 0, dev->stream>>>(pk);
   UGHIP_HIPCHK(hipGetLastError());
-  attention_rows_kernel<T, DQ, DV><<<dim3((unsigned)pk.heads, (unsigned)(pk.q_rows / ATT_QT)), attention_rows_threads<T, DQ, DV>(), bytes, dev->stream>>>(a);
-  UGHIP_HIPCHK(hipGetLastError());
+  UGHIP_HIPCHK((attention_rows_launch<T, DQ, DV>(dev, a, pk.heads)));
   return UGHIP_OK;
 }
 template <typename T>
