@@ -319,3 +319,28 @@ def test_one_row_elsewhere_is_rounded(hip, k, bias, offset):
     gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, offset, k), dst=view(dst, 0, n), w=dw.raw(), bias=db.raw() if bias else None, m=1, n=n, k=k, product=BF16, act=NONE)))
     assert "one row" not in ug_amd.last_kernel()
     close(get(dst, n), want, 2e-5)
+
+
+# f32 rows on 128 x 128, 64 x 128 and 64 x 64 tiles as the rounds of 256 have it; K of a step less and a step more, gated and plain, even and uneven groups
+@pytest.mark.parametrize("m, n, k, groups, act", [(70, 2050, 33, 0, SWIGLU), (129, 1040, 64, 0, SWIGLU), (300, 5632, 40, 0, SWIGLU), (513, 6592, 36, 0, NONE), (700, 6592, 31, 0, NONE), (1531, 2048, 24, 0, NONE),
+                                                  (150, 300, 20, 0, NONE), (1200, 1408, 28, 16, SWIGLU), (1200, 2048, 28, 16, NONE), (2036, 264, 20, 5, SWIGLU)])
+def test_f32_rows_of_every_tile(hip, m, n, k, groups, act):
+    gpu, rows, mats = Gpu(hip), n if act == NONE else 2 * n, max(1, groups)
+    gen = np.random.default_rng(6)
+    x, w = gen.standard_normal((m, k)).astype(np.float32), (gen.standard_normal((mats, rows, k)) / np.sqrt(k)).astype(np.float32)
+    kw, of = {}, np.zeros(m, int)
+    if groups:
+        end = np.sort(gen.integers(0, m + 1, groups)).astype(np.int32)
+        end[-1] = m
+        of = np.searchsorted(end, np.arange(m), side="right")
+        keep = gpu.up(np.arange(m, dtype=np.int32)), gpu.up(end)
+        kw = dict(row_index=keep[0].raw(), group_end=keep[1].raw(), groups=groups, x_rows=m)
+    y = np.concatenate([x[of == g].astype(np.float64) @ w[g].T.astype(np.float64) for g in range(mats)])
+    if act == SWIGLU:
+        y = y[:, :n] / (1 + np.exp(-y[:, :n])) * y[:, n:]
+    dx, dw, dst = gpu.up(x), gpu.up(w), gpu.out(m * n + 8)
+    print("f32 rows", m, n, k, groups, act, flush=True)
+    gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=F32, act=act, **kw)))
+    out = get(dst, m * n + 8)
+    assert np.all(np.isnan(out[m * n :])), "wrote past the end"
+    close(out[: m * n].reshape(m, n), y, 1e-5)  # k eps and the gate's few units, against sums of some standard deviations

@@ -753,22 +753,29 @@ bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int
   return ((size_t)(p.M + bm - 1) / bm + r.groups) * (size_t)((p.N + bn - 1) / bn) < (1u << 24);
 }
 
-// What rows by group take.  How they are spread is not known here: eighths of the groups have SHARE of an even one's rows, as the shares of a router's experts come
-// out that differ by 40 % (taken as even, groups of 127 rows went to 192 x 192 tiles, of which one in eight is then two: 85 us where 59 are possible).  Every K tile brings a
+// How rows by group are spread is not known where a product is planned: eighths of the groups have these shares of an even one's rows, as the shares of a router's experts come out that differ by 40 %.
+static const double SHARE[8] = {0.50, 0.65, 0.76, 0.87, 0.98, 1.12, 1.32, 1.70};
+static int share_rows(int m, int groups, double share) { return std::max(1, (int)((double)m / groups * share + 0.999)); }
+double grouped_tile_rows(int m, int groups, int bm) {
+  double n = 0;
+  for (double share : SHARE) n += groups / 8.0 * ((share_rows(m, groups, share) + bm - 1) / bm);
+  return n;
+}
+
+// What rows by group take, spread as SHARE says (taken as even, groups of 127 rows went to 192 x 192 tiles, of which one in eight is then two: 85 us where 59 are possible).  Every K tile brings a
 // matrix's columns from memory that at most a few workgroups share, 1.8 times the time that one matrix's tiles take.  Tiles by height (193, 130): a K tile by the
 // height in 64s; one round lasts for its highest tiles mostly, several go by the mean and leave one of the highest behind.
 // Fitted to 48 products of 16 groups (n 2 x 1408 and k 2048, n 2048 and k 1408, half of both; 512 to 8192 rows) on each of eight tiles: the choice is within 0.2 % of the best in the
 // mean, 5 % at most.  Gate and up, then down, of width 2048, us before and so: 768 rows 50.6 / 33.3 -> 47 / 25; 1280 50.6 / 47 -> 50 / 28; 1600 51 / 46 -> 51 / 30; 2036 84 / 37 -> 59 / 35;
 // 2560 67 / 59 -> 67 / 41; 3200 67 / 61 -> 67 / 47; 4096 80 / 55 -> 70 / 48; 8192 124 / 90 -> 124 / 83; of width 1024, 5200 rows 47 / 27 -> 36 / 27.
 static double grouped_cost_us(const MMArgs& p, int groups, int tile) {
-  static const double SHARE[8] = {0.50, 0.65, 0.76, 0.87, 0.98, 1.12, 1.32, 1.70};
   static const double WIDE[4] = {1.0, 1.2, 1.5, 1.7}, NARROW[4] = {0.6, 0.83, 1.2, 1.3};  // us per K tile, 192 and 128 columns
   int bm, bn;
   tile_dims(tile, &bm, &bn);
-  const double even = (double)p.M / groups, columns = (p.N + bn - 1) / bn, kt = p.K / BK;
+  const double columns = (p.N + bn - 1) / bn, kt = p.K / BK;
   double tiles = 0, sum = 0, highest = 0;
   for (double share : SHARE) {
-    const int rows = std::max(1, (int)(even * share + 0.999)), n = (rows + bm - 1) / bm;
+    const int rows = share_rows(p.M, groups, share), n = (rows + bm - 1) / bm;
     const double count = groups / 8.0 * n * columns;
     tiles += count;
     if (!by_height(tile)) continue;
@@ -799,6 +806,7 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
   if (r.groups > 1) {
     for (int tile : {256, 129, 65, 48, 32, 97, 193, 130}) {
       if (!gemm_dma_rows_supported(p, r, act, tile)) continue;
+      if (by_height(tile) && share_rows(p.M, r.groups, SHARE[7]) <= 64) continue;  // nothing to choose: the lowest tiles leave a CU several workgroups (216 rows 43.3, 44.0 by height)
       const double us = grouped_cost_us(p, r.groups, tile);
       if (!best || us < best_us) best = tile, best_us = us;
     }
