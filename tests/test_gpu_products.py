@@ -321,6 +321,34 @@ def test_one_row_elsewhere_is_rounded(hip, k, bias, offset):
     close(get(dst, n), want, 2e-5)
 
 
+# 32 x 32 tiles: one to nine K tiles (the ring has eight stages) and more, rows and columns that hang over, rows by group, a lookup behind, bf16 results
+@pytest.mark.parametrize("m, n, k", [(1, 8, 64), (33, 40, 128), (31, 72, 192), (65, 136, 448), (40, 24, 512), (32, 32, 576), (70, 264, 640), (100, 96, 1088)])
+@pytest.mark.parametrize("form", ["plain", "groups", "lookup", "bf16"])
+def test_smallest_ring_tile_gives_the_next_ones_bits(hip, tune, m, n, k, form):
+    gpu, gen = Gpu(hip), np.random.default_rng(7)
+    mats = 3 if form == "groups" else 1
+    dx, dw = gpu.up(rand(1, m, k), bf16=True), gpu.up(rand(2, mats, n, k, std=k ** -0.5), bf16=True)
+    keep, kw = [dx, dw, gpu.up(rand(3, n))], {}
+    if form == "plain":
+        kw = dict(bias=keep[2].raw())
+    if form == "groups":
+        keep += [gpu.up(gen.integers(0, m, m).astype(np.int32)), gpu.up(np.array([m // 3, m // 3, m], np.int32))]
+        kw = dict(row_index=keep[3].raw(), group_end=keep[4].raw(), groups=3, x_rows=m)
+    if form == "lookup":
+        keep += [gpu.up(rand(4, 50, n + 3)), gpu.up(gen.integers(0, 50, m).astype(np.int32))]
+        kw = dict(table=keep[3].raw(), ids=keep[4].raw(), table_rows=50, table_stride=n + 3, table_col=2)
+    got = {}
+    for shape, tile in (("9", "64x64,512t"), ("17", "32x32,256t")):
+        tune.setenv("UGHIP_GEMM_SHAPE", shape)
+        dst = gpu.out(m * n + 8, bf16=form == "bf16")
+        print("smallest ring tile", m, n, k, form, tile, flush=True)
+        gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=BF16, act=GELU_MUL if form == "lookup" else NONE, **kw)))
+        assert f"{tile},ring,rows" in ug_amd.last_kernel()
+        got[tile] = get(dst, m * n + 8)
+        assert np.all(np.isnan(got[tile][m * n :])) and np.all(np.isfinite(got[tile][: m * n]))
+    np.testing.assert_array_equal(got["64x64,512t"], got["32x32,256t"])
+
+
 # f32 rows on 128 x 128, 64 x 128 and 64 x 64 tiles as the rounds of 256 have it; K of a step less and a step more, gated and plain, even and uneven groups
 @pytest.mark.parametrize("m, n, k, groups, act", [(70, 2050, 33, 0, SWIGLU), (129, 1040, 64, 0, SWIGLU), (300, 5632, 40, 0, SWIGLU), (513, 6592, 36, 0, NONE), (700, 6592, 31, 0, NONE), (1531, 2048, 24, 0, NONE),
                                                   (150, 300, 20, 0, NONE), (1200, 1408, 28, 16, SWIGLU), (1200, 2048, 28, 16, NONE), (2036, 264, 20, 5, SWIGLU)])

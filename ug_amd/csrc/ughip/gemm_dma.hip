@@ -507,7 +507,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 namespace {
 // tile codes of the entry points below: 256 = 256 x 256, 192 = 256 x 192 (three planes only), 128 = 256 x 128, 64 = 128 x 128; on gemm_ring 129 = 256 x 128, 65 = 128 x 128, 48 = 64 x 128,
-// 32 = 64 x 64 ([n, k]-major rhs only), 97 = 192 x 192 (rows only), 193 / 130 = 256 x 192 / 256 x 128 and lower ones of that width (rows by group only)
+// 32 = 64 x 64 ([n, k]-major rhs only), 97 = 192 x 192 (rows only), 16 = 32 x 32 (rows only, not gated), 193 / 130 = 256 x 192 / 256 x 128 and lower ones of that width (rows by group only)
 bool tile_dims(int tile, int* bm, int* bn) {
   if (tile == 256) *bm = 256, *bn = 256;
   else if (tile == 192 || tile == 193) *bm = 256, *bn = 192;
@@ -516,6 +516,7 @@ bool tile_dims(int tile, int* bm, int* bn) {
   else if (tile == 64 || tile == 65) *bm = 128, *bn = 128;
   else if (tile == 48) *bm = 64, *bn = 128;
   else if (tile == 32) *bm = 64, *bn = 64;
+  else if (tile == 16) *bm = 32, *bn = 32;
   else return false;
   return true;
 }
@@ -526,9 +527,9 @@ static size_t tile_count(const MMArgs& p, size_t batch, int tile) {  // 0: no su
   return tile_dims(tile, &bm, &bn) ? batch * (size_t)((p.M + bm - 1) / bm) * (size_t)((p.N + bn - 1) / bn) : 0;
 }
 static bool by_height(int tile) { return tile == 193 || tile == 130; }  // rows by group: tiles of up to that height
-static bool ring_tile(int tile) { return tile == 129 || by_height(tile) || tile == 97 || tile == 65 || tile == 48 || tile == 32; }
+static bool ring_tile(int tile) { return tile == 129 || by_height(tile) || tile == 97 || tile == 65 || tile == 48 || tile == 32 || tile == 16; }
 static int least_k(int tile) { return ring_tile(tile) ? BK : 4 * BK; }
-static const char* waves_name(int tile) { return ring_tile(tile) ? "512t,ring" : "256t"; }  // in the names of these kernels
+static const char* waves_name(int tile) { return tile == 16 ? "256t,ring" : ring_tile(tile) ? "512t,ring" : "256t"; }  // in the names of these kernels
 // (tuning aid) the tile code that GEMM_SHAPE names, 0: none of these kernels'
 int gemm_dma_forced_tile(long long shape) {
   switch (shape) {
@@ -543,6 +544,7 @@ int gemm_dma_forced_tile(long long shape) {
     case 14: return 192;
     case 15: return 193;
     case 16: return 130;
+    case 17: return 16;
   }
   return 0;
 }
@@ -554,7 +556,7 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || batch == 0) return false;
   if (p.a_cs != 1 || p.a_rs % 8 || (batch > 1 && (p.a_bs % 8 || p.b_bs % 8 || p.c_bs % 8))) return false;
   const bool nn = p.b_cs == 1 && p.b_rs != 1, nt = p.b_rs == 1 && p.b_cs != 1;
-  if (nn == nt || (nn && tile == 32) || tile == 97 || by_height(tile) || (tile == 192 && p.b_k_div != 3)) return false;
+  if (nn == nt || (nn && tile == 32) || tile == 97 || tile == 16 || by_height(tile) || (tile == 192 && p.b_k_div != 3)) return false;
   const long long ldb = nn ? p.b_rs : p.b_cs;
   if (ldb % 8) return false;
   // per-lane offsets are 32-bit: the furthest row of a tile has to stay below 4 GiB from the tile's first byte
@@ -574,6 +576,8 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
 enum class Operands { MEMORY, CACHE, PLANES };
 static double ring_cost_us(size_t tiles, int kt, int tile, Operands from) {
   const bool memory = from == Operands::MEMORY, planes = from == Operands::PLANES;
+  // 32 x 32, two workgroups to a CU: 54 rows of 2048 x 5632 14.1, 228 of 2048 x 2048 9.8, 228 of 3072 x 768 7.6
+  if (tile == 16) return 2.3 + kt * (0.135 + (tiles > 256 ? 0.09 * std::min(1.0, (tiles - 256.0) / 256) : 0) + (tiles > 512 ? 0.2 * (tiles - 512.0) / 256 : 0));
   const double t0 = tile == 129 ? 0.64 : tile == 97 ? 0.62 : tile == 65 ? (memory ? 0.54 : 0.30) : tile == 48 ? (memory ? 0.40 : 0.21) : memory ? 0.255 : planes ? 0.11 : 0.14;
   const double t1 = tile == 129 ? 0.22 : tile == 97 ? 0.30 : memory ? 0 : tile == 65 ? 0.17 : tile == 48 ? 0.07 : planes ? 0.075 : 0.045;
   double us = tile == 129 || tile == 97 ? 5.0 : tile == 65 ? 4.0 : 3.3;
@@ -744,6 +748,7 @@ bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int
   int bm, bn;
   if (!tile_dims(tile, &bm, &bn) || (tile != 256 && !ring_tile(tile)) || ((tile == 256 || tile == 97) && act == RowsAct::LOOKUP) || (by_height(tile) && (!r.groups || act == RowsAct::LOOKUP)))
     return false;
+  if (tile == 16 && act == RowsAct::GLU) return false;
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || p.a_cs != 1 || p.a_rs % 8 || p.b_rs != 1 || p.b_cs % 8) return false;
   if (r.n_out <= 0 || r.n_out % 4 || p.N != (act == RowsAct::GLU ? 2 * r.n_out : r.n_out) || r.dst_stride % 4 || r.w_group % 8) return false;
   // per-lane offsets are 32-bit: rows of x anywhere, matrix rows of a tile (of the whole matrix with SwiGLU)
@@ -812,8 +817,9 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
     }
     return best;
   }
-  for (int tile : {256, 129, 65, 48, 32, 97}) {
+  for (int tile : {256, 129, 65, 48, 32, 16, 97}) {
     if (!gemm_dma_rows_supported(p, r, act, tile)) continue;
+    if (tile == 16 && p.K < 8 * BK) continue;  // shorter than its ring it gains nothing (54 rows of 2048 x 256 4.0 us on either)
     int bm, bn;
     tile_dims(tile, &bm, &bn);
     const size_t tiles = (size_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);

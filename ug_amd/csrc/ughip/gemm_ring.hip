@@ -2,6 +2,8 @@
 //
 //   Eight waves, 4 x 2, each BM / 4 x BN / 2 of the result in 16 x 16 accumulators (v_mfma_f32_16x16x32): a wave's waits are filled by the other
 //   one of its SIMD.  The k order of every sum is that of gemm_dma4 and gemm_tiled, so the results are theirs bit for bit.
+//   32 x 32, four waves and eight stages, for rows only: a CU has some 55 KB on its way whatever it is asked for, so where 64 x 64 tiles are few it is their bytes per CU that count (us on
+//   64 x 64 and so, weights from memory: 54 rows of 2048 x 2048 / 4096 / 5632 11.3 / 19.6 / 26.8 -> 6.7 / 10.6 / 14.1, 509 rows of 256 x 2048 8.9 -> 6.4, 228 of 2048 x 2048 11.3 -> 9.8).
 //   192 x 192 for rows only: 700 rows against 11264 x 2048 are 236 of them, one round (52 us with 256 x 256, 54 with 256 x 128, 34 so).
 //   A ring of four stages (three for the two largest tiles): the loads of a K tile go out (global_load_lds_dwordx4, as in gemm_dma4) when the tile that
 //   many in front of it has been read, so three (two) tiles are on their way while one is multiplied.  One barrier per K tile.
@@ -24,7 +26,8 @@
 namespace ughip {
 namespace {
 
-constexpr int stages(int bm, int bn) { return bm == 256 && bn == 192 ? 2 : bm >= 192 || bm * bn > 128 * 128 ? 3 : 4; }
+constexpr int waves(int bm) { return bm == 32 ? 4 : 8; }  // two to a row of them
+constexpr int stages(int bm, int bn) { return bm == 32 ? 8 : bm == 256 && bn == 192 ? 2 : bm >= 192 || bm * bn > 128 * 128 ? 3 : 4; }
 constexpr int lds_bytes(int bm, int bn) { return stages(bm, bn) * (bm + bn) * BK * 2; }
 
 // One tile: rows [m0, m_end) (BM of them at most) and the columns of column tile tn, of one batch or group.
@@ -36,9 +39,10 @@ __device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group,
   static_assert(!B_KN || BN >= 128, "the swizzle of an n-contiguous tile wants eight 32-byte pieces per row");
   extern __shared__ u32x4 lds[];
   constexpr int S = stages(BM, BN);
-  constexpr int NI = BM / 64, NJ = BN / 32, NM = NI * NJ;  // 16-row and 16-column fragments and MFMAs of a wave and step of 32 k
+  constexpr int W = waves(BM), WR = W / 2;  // waves, and rows of them
+  constexpr int NI = BM / (16 * WR), NJ = BN / 32, NM = NI * NJ;  // 16-row and 16-column fragments and MFMAs of a wave and step of 32 k
   constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, STAGE_BYTES = A_BYTES + B_BYTES;
-  constexpr int NDA = BM / 64, NDB = BN / 64, ND = NDA + NDB;   // loads per wave and K tile
+  constexpr int NDA = BM / (8 * W), NDB = BN / (8 * W), ND = NDA + NDB;   // loads per wave and K tile
   constexpr int R = NI + NJ;                                      // fragment reads per step
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -49,14 +53,14 @@ __device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group,
   const char* Bb = reinterpret_cast<const char*>(static_cast<const T*>(p.b) + (size_t)batch * p.b_bs + (ROWS ? (size_t)group * rw.w_group : 0) +
                                                  (ROWS == 2 ? 0 : B_KN ? (size_t)n0 : (size_t)n0 * ldb));
   const int KT = p.K / BK;
-  const int wm = (wave >> 1) * (BM / 4), wn = (wave & 1) * (BN / 2);
+  const int wm = (wave >> 1) * (BM / WR), wn = (wave & 1) * (BN / 2);
   const unsigned lds_addr = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds;
   // per-lane byte offsets of this wave's loads; rows past the end fetch the last row again (their results are not stored)
   unsigned voff[ND];
   const int m_last = m_end - 1 - m0, n_left = p.N - n0;
 #pragma unroll
   for (int i = 0; i < NDA; ++i) {
-    const int row = (i * 8 + wave) * 8 + (lane >> 3), cp = lane & 7;
+    const int row = (i * W + wave) * 8 + (lane >> 3), cp = lane & 7;
     int src = min(row, m_last);
     if constexpr (ROWS != 0) {
       src += m0;
@@ -66,7 +70,7 @@ __device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group,
   }
 #pragma unroll
   for (int i = 0; i < NDB; ++i) {
-    const int g = i * 8 + wave;
+    const int g = i * W + wave;
     if (!B_KN) {
       const int row = g * 8 + (lane >> 3), cp = lane & 7;
       int src = min(row, n_left - 1);
@@ -85,8 +89,8 @@ __device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group,
   const long long a_step = BK * 2, b_step = B_KN ? (long long)BK * ldb * 2 : BK * 2;
   auto dma = [&](int tile, int idx) {  // idx: compile-time after unrolling
     const unsigned st = lds_addr + (unsigned)tile % S * STAGE_BYTES;
-    if (idx < NDA) dma16(Ab + lhs_k_tile<BDIV>(tile) * a_step, voff[idx], st + (idx * 8 + wave) * 1024);
-    else dma16(Bb + rhs_k_tile<BDIV>(tile) * b_step, voff[idx], st + A_BYTES + ((idx - NDA) * 8 + wave) * 1024);
+    if (idx < NDA) dma16(Ab + lhs_k_tile<BDIV>(tile) * a_step, voff[idx], st + (idx * W + wave) * 1024);
+    else dma16(Bb + rhs_k_tile<BDIV>(tile) * b_step, voff[idx], st + A_BYTES + ((idx - NDA) * W + wave) * 1024);
   };
 
   floatx4 acc[NI][NJ];
@@ -164,13 +168,17 @@ __device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group,
 #pragma unroll
   for (int r = 0; r < R; ++r) read_frag(0, 0, r, 0);
   for (int kt = 0; kt < KT - S; ++kt) body(kt, CS());
-  if constexpr (S > 3) {
-    if (KT > 3) body(KT - 4, std::integral_constant<int, 3>());
-  }
-  if constexpr (S > 2) {
-    if (KT > 2) body(KT - 3, std::integral_constant<int, 2>());
-  }
-  if (KT > 1) body(KT - 2, C1());
+  auto left = [&](auto ahead) {
+    if constexpr (decltype(ahead)::value < S)
+      if (KT > decltype(ahead)::value) body(KT - 1 - decltype(ahead)::value, ahead);
+  };
+  left(std::integral_constant<int, 7>());
+  left(std::integral_constant<int, 6>());
+  left(std::integral_constant<int, 5>());
+  left(std::integral_constant<int, 4>());
+  left(std::integral_constant<int, 3>());
+  left(std::integral_constant<int, 2>());
+  left(C1());
   body(KT - 1, C0());
 
   // Register e of lane l of block (i, j): row wm + 16 i + l % 16, column wn + 16 j + 4 (l / 16) + e.
@@ -250,7 +258,7 @@ __device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group,
       *(u32x2 __attribute__((address_space(3)))*)(Cs + row * PITCH + col * 2) = __builtin_bit_cast(u32x2, v);
     }
   __syncthreads();
-  constexpr int CPR = BN / 8, RPP = 512 / CPR;
+  constexpr int CPR = BN / 8, RPP = 64 * W / CPR;
   T* __restrict__ C = static_cast<T*>(p.c) + (size_t)batch * p.c_bs + (size_t)m0 * p.N + n0;
   const int c = tid % CPR, r0 = tid / CPR;
 #pragma unroll
@@ -264,7 +272,7 @@ __device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group,
 
 // The tiles of a launch, dealt to its workgroups.
 template <typename T, int BM, int BN, bool B_KN, bool F32OUT, int BDIV, int ROWS>
-__global__ void __launch_bounds__(512) gemm_ring(MMArgs p, int batches, int tiles_m, int tiles_n, const float* __restrict__ residual, DmaRows rw) {
+__global__ void __launch_bounds__(64 * waves(BM)) gemm_ring(MMArgs p, int batches, int tiles_m, int tiles_n, const float* __restrict__ residual, DmaRows rw) {
   const int lane = threadIdx.x & 63;
   // XCD-aware order of the tiles: as in gemm_dma4 (the grid is 8 more at least, the runs are of equal length)
   int tiles = batches * tiles_m * tiles_n;
@@ -336,7 +344,7 @@ hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, const float
   if (hipError_t e = allow_lds(kernel, LDS_BYTES, configured)) return e;
   const int tiles_m = (p.M + BM - 1) / BM + rw.groups, tiles_n = (p.N + BN - 1) / BN;
   const size_t total = (batch * (size_t)tiles_m * tiles_n + 7) / 8 * 8 + (rw.groups ? 8 : 0);
-  kernel<<<dim3((unsigned)total), dim3(512), LDS_BYTES, stream>>>(p, (int)batch, tiles_m, tiles_n, residual, rw);
+  kernel<<<dim3((unsigned)total), dim3(64 * waves(BM)), LDS_BYTES, stream>>>(p, (int)batch, tiles_m, tiles_n, residual, rw);
   return hipGetLastError();
 }
 
@@ -361,6 +369,9 @@ hipError_t launch_nt(hipStream_t stream, const MMArgs& p, size_t batch, int tile
     if (tile == 193) return launch_groups<192, ROWS>(stream, p, rw);
     if (tile == 130) return launch_groups<128, ROWS>(stream, p, rw);
     if (tile == 97) return launch<T, 192, 192, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
+  }
+  if constexpr (ROWS == 1 || ROWS == 3) {
+    if (tile == 16) return launch<T, 32, 32, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
   }
   if (tile == 65) return launch<T, 128, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
   if (tile == 48) return launch<T, 64, 128, false, F32OUT, BDIV, ROWS>(stream, p, batch, residual, rw);
