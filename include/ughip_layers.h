@@ -124,6 +124,9 @@ int ughip_grouped_attention_cache(size_t kv_heads, size_t dim, size_t vdim, size
  * ughip_conv_ring_store: the step's last rows go into the ring (after everything that still reads the old ones). */
 int ughip_conv_silu_rows(ughip_device* dev, ughip_view x, const ughip_slice* taps, const ughip_slice* bias, size_t n_taps, const ughip_slice* ring, size_t pos,
                          size_t t, size_t channels, ughip_view dst);
+/* Both: the ring holds the step's last rows behind it. */
+int ughip_conv_silu_rows_and_store(ughip_device* dev, ughip_view x, const ughip_slice* taps, const ughip_slice* bias, size_t n_taps, ughip_slice* ring, size_t pos,
+                                   size_t t, size_t channels, ughip_view dst);
 int ughip_conv_ring_store(ughip_device* dev, ughip_view x, size_t n_taps, ughip_slice* ring, size_t pos, size_t t, size_t channels);
 /* xbc rows [heads vdim | groups state (B) | groups state (C)] (after the convolution), dt rows [heads] as projected:
  *   d = softplus(dt + dt_bias), S_h = exp(-exp(a_log_h) d_h) S_h + d_h B_g x_h^T, y_h = S_h^T C_g + skip_h x_h, g = h / (heads / groups)

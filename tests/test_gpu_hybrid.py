@@ -85,6 +85,48 @@ def test_products_of_rows_sorted_by_expert(gpu, m, n, k, experts, top, mode, act
     close(got[sl.ravel()], want, 2e-5)
 
 
+# runs of pairs that registers hold (8 and 32 to a thread), the first that they do not, none past the first threads
+@pytest.mark.parametrize("pairs, experts", [(1, 3), (255, 4), (2048, 16), (2049, 16), (8192, 5), (8193, 7)])
+def test_pairs_sorted_by_expert(gpu, pairs, experts):
+    ids = np.random.default_rng(pairs).integers(0, experts, pairs)
+    ids[ids == 1] = 2  # nobody's choice
+    d_ids, ri, sl, ge = gpu.up(ids.astype(np.int32)), gpu.ints(pairs), gpu.ints(pairs), gpu.ints(experts)
+    gpu.call("ughip_group_rows", p(d_ids), Z(pairs), Z(1), Z(experts), p(ri), p(sl), p(ge))
+    order = np.argsort(ids, kind="stable")
+    assert np.array_equal(ri.to_vec(), order) and np.array_equal(sl.to_vec()[order], np.arange(pairs))
+    assert np.array_equal(ge.to_vec(), np.cumsum(np.bincount(ids, minlength=experts)))
+
+
+# rows read 16 bytes at a time: fewer runs than waves, runs past the last one, one and several rounds of them, experts that end inside a tile
+@pytest.mark.parametrize("m, k, experts", [(1, 4, 2), (16, 60, 16), (17, 128, 5), (33, 1028, 16), (40, 2100, 12), (19, 2100, 17), (5, 576, 70)])
+def test_routing_by_whole_pieces(gpu, m, k, experts):
+    top = min(3, experts)
+    x, w, corr = rand(1, m, k), rand(2, experts, k, std=2 * k ** -0.5), rand(3, experts, std=0.4)
+    ids, wts = gpu.ints(m * top), gpu.out(m * top)
+    sx, sw, sc = gpu.up(x), gpu.up(w), gpu.up(corr)
+    gpu.call("ughip_route_rows", view(sx, 0, k), p(sw), p(sc), Z(m), Z(k), Z(experts), Z(1), Z(1), Z(top), p(ids), p(wts))
+    ids, wts = ids.to_vec().reshape(m, top), get(wts, (m, top))
+    rc = {"experts": experts, "top": top, "groups": {"count": 1, "keep": 1}}
+    for i in range(m):
+        chosen, weight = ph.route(x[i], {"router": w, "correction": corr}, rc)
+        assert ids[i].tolist() == chosen.tolist(), i
+        np.testing.assert_allclose(wts[i], weight, rtol=2e-5)
+
+
+# two to four taps by fours of channels, other counts one by one; steps shorter and longer than the ring, at its start and inside
+@pytest.mark.parametrize("taps, channels", [(2, 8), (3, 1028), (4, 12), (4, 6), (5, 8), (1, 4)])
+@pytest.mark.parametrize("t, pos", [(1, 0), (2, 3), (3, 1), (5, 0), (8, 9), (19, 6)])
+def test_convolution_that_leaves_its_ring(gpu, taps, channels, t, pos):
+    """As the convolution and the store behind it, bit for bit."""
+    x, w, old = gpu.up(rand(1, t, channels)), gpu.up(rand(2, channels, taps)), rand(3, taps, channels)
+    rings, out = [gpu.up(old), gpu.up(old)], [gpu.out(t * channels), gpu.out(t * channels)]
+    gpu.call("ughip_conv_silu_rows", view(x, 0, channels), p(w), None, Z(taps), p(rings[0]), Z(pos), Z(t), Z(channels), view(out[0], 0, channels))
+    gpu.call("ughip_conv_ring_store", view(x, 0, channels), Z(taps), p(rings[0]), Z(pos), Z(t), Z(channels))
+    gpu.call("ughip_conv_silu_rows_and_store", view(x, 0, channels), p(w), None, Z(taps), p(rings[1]), Z(pos), Z(t), Z(channels), view(out[1], 0, channels))
+    np.testing.assert_array_equal(get(out[0], t * channels), get(out[1], t * channels))
+    np.testing.assert_array_equal(rings[0].to_vec(), rings[1].to_vec())
+
+
 @pytest.mark.parametrize("experts, groups, keep, top", [(1, 1, 1, 1), (6, 3, 2, 2), (8, 4, 3, 3), (9, 9, 4, 4), (64, 8, 3, 6), (96, 4, 2, 7), (130, 13, 5, 5)])
 def test_routing(gpu, experts, groups, keep, top):
     m, k = 37, 75

@@ -62,11 +62,10 @@ struct ChannelDelta : Mixer {
     settle(c, s);
     LB p = stream_product(c, s, first);
     LB qkv = hip_op("conv_silu", {p, conv, ring}, {t, ch}, [=](ughip_device* d, const std::vector<ughip_slice*>& x, ughip_slice* out) {
-      return ughip_conv_silu_rows(d, {x[0], 0, wide}, x[1], nullptr, nt, x[2], pos, t, ch, {out, 0, ch});
+      return ughip_conv_silu_rows_and_store(d, {x[0], 0, wide}, x[1], nullptr, nt, x[2], pos, t, ch, {out, 0, ch});
     });
     LB a = product_rows({p, ch, wide}, t, {a2, LB(), hd, ra}), z = product_rows({p, ch + ra, wide}, t, {g2, LB(), I, rz});
-    LB y = hip_op("delta", {qkv, p, a, z, a_log, dt_bias, norm, S, ring}, {t, I}, [=](ughip_device* d, const std::vector<ughip_slice*>& x, ughip_slice* out) {
-      if (int rc = ughip_conv_ring_store(d, {x[1], 0, wide}, nt, x[8], pos, t, ch)) return rc;
+    LB y = hip_op("delta", {qkv, p, a, z, a_log, dt_bias, norm, S}, {t, I}, [=](ughip_device* d, const std::vector<ughip_slice*>& x, ughip_slice* out) {
       ughip_delta r = q;
       r.qkv = {x[0], 0, ch}, r.b = {x[1], ch + ra + rz, wide}, r.a = {x[2], 0, hd}, r.z = {x[3], 0, I}, r.dst = {out, 0, I};
       r.a_log = x[4], r.dt_bias = x[5], r.norm = x[6], r.s = x[7];

@@ -160,10 +160,9 @@ struct Mamba2 : Mixer {
     settle(c, s);
     LB p = stream_product(c, s, {in, LB(), wide, width});
     LB xbc = hip_op("conv_silu", {p, conv, conv_b, ring}, {t, ch}, [=](ughip_device* dev, const std::vector<ughip_slice*>& a, ughip_slice* out) {
-      return ughip_conv_silu_rows(dev, {a[0], I, wide}, a[1], a[2], nt, a[3], pos, t, ch, {out, 0, ch});
+      return ughip_conv_silu_rows_and_store(dev, {a[0], I, wide}, a[1], a[2], nt, a[3], pos, t, ch, {out, 0, ch});
     });
-    LB y = hip_op("ssm", {xbc, p, dt_bias, a_log, skip, S, ring}, {t, I}, [=](ughip_device* dev, const std::vector<ughip_slice*>& a, ughip_slice* out) {
-      if (int rc = ughip_conv_ring_store(dev, {a[1], I, wide}, nt, a[6], pos, t, ch)) return rc;
+    LB y = hip_op("ssm", {xbc, p, dt_bias, a_log, skip, S}, {t, I}, [=](ughip_device* dev, const std::vector<ughip_slice*>& a, ughip_slice* out) {
       return ughip_ssm_rows(dev, {a[0], 0, ch}, {a[1], I + ch, wide}, a[2], a[3], a[4], a[5], pos, t, H, vd, G, N, {out, 0, I});
     });
     LB yn = hip_op("gated_norm", {y, p, norm}, {t, I}, [=](ughip_device* dev, const std::vector<ughip_slice*>& a, ughip_slice* out) {

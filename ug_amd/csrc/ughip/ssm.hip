@@ -3,8 +3,7 @@
 //   S_t = exp(a_t) S_{t-1} + d_t B_t x_t^T,   y_t = S_t^T C_t + skip x_t,   a_t = -exp(a_log) d_t, d_t = softplus(dt_t + bias)
 //
 // Several positions run in chunks of Q.  With A_i = a_1 + .. + a_i inside a chunk:
-//   ssm_chunk_decays  d_i and A_i
-//   ssm_chunk_state   what a chunk adds to the state: sum_j B_j (exp(A_Q - A_j) d_j x_j)^T
+//   ssm_chunk_state   d_i and A_i, and what a chunk adds to the state: sum_j B_j (exp(A_Q - A_j) d_j x_j)^T
 //   ssm_chunk_scan    the state in front of every chunk, S <- exp(A_Q) S + that, in place              (elementwise, chunks in order)
 //   ssm_chunk_out     y_i = sum_{j <= i} exp(A_i - A_j) d_j (C_i . B_j) x_j + exp(A_i) S^T C_i + skip x_i
 // Every exponent is <= 0.  A workgroup takes a chunk and some heads of one group: B, C and the products C_i . B_j are the group's
@@ -39,7 +38,7 @@ struct SsmArgs {
 constexpr int ROWS_CONV = 8;
 template <int TAPS>
 __global__ void __launch_bounds__(256) conv_silu_rows4_kernel(const float* __restrict__ x, size_t x_stride, const float* __restrict__ taps, const float* __restrict__ bias,
-                                                              const float* __restrict__ ring, long long pos, int t, int channels, float* __restrict__ dst, size_t dst_stride) {
+                                                              float* ring, bool store, long long pos, int t, int channels, float* __restrict__ dst, size_t dst_stride) {
   const int c = (blockIdx.x * 256 + threadIdx.x) * 4, i0 = blockIdx.y * ROWS_CONV;
   if (c >= channels) return;
   auto row = [&](int r) -> f32x4_t {
@@ -68,6 +67,13 @@ __global__ void __launch_bounds__(256) conv_silu_rows4_kernel(const float* __res
     for (int e = 0; e < 4; ++e) v[e] = silu_f(v[e]);
     *reinterpret_cast<f32x4_t*>(dst + (size_t)(i0 + i) * dst_stride + c) = v;
   }
+  // (who has read these channels' old rows leaves the new ones: a launch of 4.6 us less for 0.8 more here)
+  static_assert(ROWS_CONV >= TAPS - 1, "the ring is read by the first rows' threads alone");
+  if (store && blockIdx.y == 0) {
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j)
+      if (const int i = t - 1 - j; i >= 0) *reinterpret_cast<f32x4_t*>(ring + (size_t)((pos + i) % TAPS) * channels + c) = *reinterpret_cast<const f32x4_t*>(x + (size_t)i * x_stride + c);
+  }
 }
 
 __global__ void __launch_bounds__(256) conv_silu_rows_kernel(const float* __restrict__ x, size_t x_stride, const float* __restrict__ taps, const float* __restrict__ bias,
@@ -94,21 +100,6 @@ __global__ void __launch_bounds__(256) conv_ring_store_kernel(const float* __res
   const int i = t - 1 - (int)blockIdx.y;
   if (c >= channels || i < 0) return;
   ring[(size_t)((pos + i) % n_taps) * channels + c] = x[(size_t)i * x_stride + c];
-}
-
-// One wave per chunk and head (q <= 64).
-__global__ void __launch_bounds__(256) ssm_chunk_decays_kernel(SsmArgs a) {
-  const int i = threadIdx.x & 63, h = blockIdx.y * 4 + (threadIdx.x >> 6), row0 = blockIdx.x * a.q;
-  if (h >= a.heads) return;
-  float dv = 0.f;
-  if (i < a.q && row0 + i < a.t) dv = softplus_f(a.dt[(size_t)(row0 + i) * a.dt_stride + h] + a.dt_bias[h]);
-  float s = -expf(a.a_log[h]) * dv;
-  for (int k = 1; k < 64; k <<= 1) {
-    const float o = __shfl_up(s, k, 64);
-    if (i >= k) s += o;
-  }
-  const size_t at = ((size_t)blockIdx.x * a.heads + h) * 64 + i;
-  a.cum[at] = s, a.step[at] = dv;
 }
 
 __device__ __forceinline__ f32x4_t mfma16(float x, float y, f32x4_t acc) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, acc, 0, 0, 0); }
@@ -210,9 +201,18 @@ __global__ void __launch_bounds__(256) ssm_chunk_state_kernel(SsmArgs a) {
   float weight = 0.f;  // of row `lane` (first wave)
   auto fetch = [&](int i) {
     x.load(xbc0 + (size_t)hw.head(i) * a.vdim + hw.col(i), a.xbc_stride, rows, min(PB, a.vdim - hw.col(i)), PB / 4, xt);
-    if (wave == 0) {
-      const size_t at = ((size_t)chunk * a.heads + hw.head(i)) * 64;
-      weight = a.step[at + lane] * expf(a.cum[at + 63] - a.cum[at + lane]);
+    if (wave == 0) {  // the head's d_i and A_i, for the launches behind this one too (q <= 64; a launch of 4.6 us by themselves)
+      const int h = hw.head(i);
+      float dv = 0.f;
+      if (lane < q && lane < rows) dv = softplus_f(a.dt[(size_t)(row0 + lane) * a.dt_stride + h] + a.dt_bias[h]);
+      float s = -expf(a.a_log[h]) * dv;
+      for (int d = 1; d < 64; d <<= 1) {
+        const float o = __shfl_up(s, d, 64);
+        if (lane >= d) s += o;
+      }
+      const size_t at = ((size_t)chunk * a.heads + h) * 64 + lane;
+      a.cum[at] = s, a.step[at] = dv;
+      weight = dv * expf(__shfl(s, 63, 64) - s);
     }
   };
   if (hw.items) fetch(0);
@@ -498,8 +498,9 @@ size_t out_lds_bytes(int q, int state) {
 
 }  // namespace
 
-extern "C" int ughip_conv_silu_rows(ughip_device* dev, ughip_view x, const ughip_slice* taps, const ughip_slice* bias, size_t n_taps, const ughip_slice* ring, size_t pos,
-                                    size_t t, size_t channels, ughip_view dst) {
+namespace {
+int conv_silu(ughip_device* dev, ughip_view x, const ughip_slice* taps, const ughip_slice* bias, size_t n_taps, const ughip_slice* ring, bool store, size_t pos, size_t t,
+              size_t channels, ughip_view dst) {
   if (!dev) return set_error(UGHIP_ERR_INVALID, "conv_silu_rows: null device");
   if (n_taps == 0 || n_taps > 1024) return set_error(UGHIP_ERR_INVALID, "conv_silu_rows: %zu taps", n_taps);
   if (int rc = check_view(dev, x, t, channels, UGHIP_F32, "conv_silu_rows x")) return rc;
@@ -514,7 +515,7 @@ extern "C" int ughip_conv_silu_rows(ughip_device* dev, ughip_view x, const ughip
   if (n_taps >= 2 && n_taps <= 4 && channels % 4 == 0 && x.stride % 4 == 0 && dst.stride % 4 == 0 && a16(view_ptr<float>(x)) && a16(view_ptr<float>(dst)) && t / ROWS_CONV < 65535) {
     const dim3 g4((unsigned)((channels / 4 + 255) / 256), (unsigned)((t + ROWS_CONV - 1) / ROWS_CONV));
     auto go = [&](auto kernel) {
-      kernel<<<g4, 256, 0, dev->stream>>>(view_ptr<float>(x), x.stride, buf_ptr<float>(taps), buf_ptr<float>(bias), buf_ptr<float>(ring), (long long)pos, (int)t, (int)channels,
+      kernel<<<g4, 256, 0, dev->stream>>>(view_ptr<float>(x), x.stride, buf_ptr<float>(taps), buf_ptr<float>(bias), static_cast<float*>(ring->ptr), store, (long long)pos, (int)t, (int)channels,
                                           view_ptr<float>(dst), dst.stride);
     };
     n_taps == 4 ? go(conv_silu_rows4_kernel<4>) : n_taps == 3 ? go(conv_silu_rows4_kernel<3>) : go(conv_silu_rows4_kernel<2>);
@@ -525,7 +526,19 @@ extern "C" int ughip_conv_silu_rows(ughip_device* dev, ughip_view x, const ughip
   conv_silu_rows_kernel<<<grid, 256, 0, dev->stream>>>(view_ptr<float>(x), x.stride, buf_ptr<float>(taps), buf_ptr<float>(bias), (int)n_taps, buf_ptr<float>(ring),
                                                        (long long)pos, (int)t, (int)channels, view_ptr<float>(dst), dst.stride);
   UGHIP_HIPCHK(hipGetLastError());
-  return UGHIP_OK;
+  return store ? ughip_conv_ring_store(dev, x, n_taps, const_cast<ughip_slice*>(ring), pos, t, channels) : UGHIP_OK;
+}
+}  // namespace
+
+extern "C" int ughip_conv_silu_rows(ughip_device* dev, ughip_view x, const ughip_slice* taps, const ughip_slice* bias, size_t n_taps, const ughip_slice* ring, size_t pos,
+                                    size_t t, size_t channels, ughip_view dst) {
+  return conv_silu(dev, x, taps, bias, n_taps, ring, false, pos, t, channels, dst);
+}
+
+extern "C" int ughip_conv_silu_rows_and_store(ughip_device* dev, ughip_view x, const ughip_slice* taps, const ughip_slice* bias, size_t n_taps, ughip_slice* ring, size_t pos,
+                                              size_t t, size_t channels, ughip_view dst) {
+  if (dst.s == ring || x.s == ring) return set_error(UGHIP_ERR_INVALID, "conv_silu_rows_and_store: the ring is a buffer of its own");
+  return conv_silu(dev, x, taps, bias, n_taps, ring, true, pos, t, channels, dst);
 }
 
 extern "C" int ughip_conv_ring_store(ughip_device* dev, ughip_view x, size_t n_taps, ughip_slice* ring, size_t pos, size_t t, size_t channels) {
@@ -579,7 +592,6 @@ extern "C" int ughip_ssm_rows(ughip_device* dev, ughip_view xbc, ughip_view dt, 
   }();
   UGHIP_HIPCHK(attr);
   const size_t lds_s = state_lds_bytes(q, (int)state), lds_o = out_lds_bytes(q, (int)state);
-  ssm_chunk_decays_kernel<<<dim3((unsigned)chunks, (unsigned)((heads + 3) / 4)), 256, 0, dev->stream>>>(a);
   if (vec) ssm_chunk_state_kernel<true><<<grid, 256, lds_s, dev->stream>>>(a);
   else ssm_chunk_state_kernel<false><<<grid, 256, lds_s, dev->stream>>>(a);
   ssm_chunk_scan_kernel<<<dim3((unsigned)((elems + 255) / 256), (unsigned)heads), 256, 0, dev->stream>>>(a);
