@@ -76,6 +76,7 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   static_assert(ROWS == 0 || ROWS == 4 || (BDIV == 1 && !B_KN && !F32OUT), "rows: one plane against an [n, k]-major rhs");
   static_assert(ROWS != 4 || (BDIV == 3 && BN == 192 && F32OUT), "gated planes: 96 columns of three planes are what LDS takes on the way out");
   constexpr bool GATED = ROWS == 2 || ROWS == 4, BY_ROW = ROWS == 1 || ROWS == 2;
+  static_assert(BDIV != 3 || TWO, "shared rhs tiles are scheduled with two barriers");
   static_assert(BDIV == 1 || BDIV == 6 || !B_KN, "planes of the lhs alone: against an [n, k]-major rhs only");
   static_assert(BN != 192 || (!B_KN && F32OUT), "192 columns: neither the swizzle of an n-contiguous tile nor the way out through LDS divides them");
   extern __shared__ u32x4 lds[];
@@ -83,6 +84,9 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   constexpr int NM = NI * NJ;                          // MFMAs per k32 step
   constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, STAGE_BYTES = A_BYTES + B_BYTES;
   constexpr int NDA = BM / 32, NDB = BN / 32, ND = NDA + NDB;  // DMA instructions per wave and K tile
+  // SHARED: the three planes of a lhs tile meet one rhs tile, which is loaded once for them, into a place of its own behind the lhs stages, and whose fragments stay in registers.
+  constexpr bool SHARED = BDIV == 3;
+  constexpr int A_STAGE = SHARED ? A_BYTES : STAGE_BYTES, B_AT = SHARED ? 2 * A_BYTES : A_BYTES, B_STAGE = SHARED ? 0 : STAGE_BYTES;
   constexpr int R = NI + NJ;                           // fragment reads per step
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -164,13 +168,12 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   }
   const long long a_step = BK * 2, b_step = B_KN ? (long long)BK * ldb * 2 : BK * 2;
   auto dma = [&](int tile, int idx) {  // idx: compile-time after unrolling
-    const unsigned st = lds_addr + (tile & 1) * STAGE_BYTES;
-    if (idx < NDA) dma16(Ab + lhs_k_tile<BDIV>(tile) * a_step, voff[idx], st + (idx * 4 + wave) * 1024);
-    else dma16(Bb + rhs_k_tile<BDIV>(tile) * b_step, voff[idx], st + A_BYTES + ((idx - NDA) * 4 + wave) * 1024);
+    if (idx < NDA) dma16(Ab + lhs_k_tile<BDIV>(tile) * a_step, voff[idx], lds_addr + (tile & 1) * A_STAGE + (idx * 4 + wave) * 1024);
+    else dma16(Bb + rhs_k_tile<BDIV>(tile) * b_step, voff[idx], lds_addr + (tile & 1) * B_STAGE + B_AT + ((idx - NDA) * 4 + wave) * 1024);
   };
   auto dma_m0 = [&](int tile, int idx) {
-    const unsigned in_stage = lds_addr + (idx < NDA ? (idx * 4 + wave) * 1024 : A_BYTES + ((idx - NDA) * 4 + wave) * 1024);  // loop invariant
-    dma16_m0(in_stage, (tile & 1) * STAGE_BYTES);
+    const unsigned in_stage = lds_addr + (idx < NDA ? (idx * 4 + wave) * 1024 : B_AT + ((idx - NDA) * 4 + wave) * 1024);  // loop invariant
+    dma16_m0(in_stage, (tile & 1) * (idx < NDA ? A_STAGE : B_STAGE));
     // the MFMA that follows in the source has to follow in the code: without this the compiler may hoist it above the
     // write of M0, and the load would then come right behind that write, without the wait state it needs
     __builtin_amdgcn_sched_barrier(0);
@@ -189,9 +192,9 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   u32x4 fa[2][NI], fb[2][NJ];
   auto read_frag = [&](int stage, int s, int idx, int set) {
     if (idx < NI) {
-      fa[set][idx] = lds[stage * (STAGE_BYTES / 16) + kc_idx(wm + idx * 16 + (lane & 15), 4 * s + (lane >> 4))];
+      fa[set][idx] = lds[stage * (A_STAGE / 16) + kc_idx(wm + idx * 16 + (lane & 15), 4 * s + (lane >> 4))];
     } else if (!B_KN) {
-      fb[set][idx - NI] = lds[stage * (STAGE_BYTES / 16) + A_BYTES / 16 + kc_idx(wn + (idx - NI) * 16 + (lane & 15), 4 * s + (lane >> 4))];
+      fb[set][idx - NI] = lds[stage * (B_STAGE / 16) + B_AT / 16 + kc_idx(wn + (idx - NI) * 16 + (lane & 15), 4 * s + (lane >> 4))];
     } else {
       // lane q + 4 e of a 16-lane group names row k0 + e, columns 4 q .. 4 q + 3 of the fragment's 16: lane i receives
       // k0 .. k0 + 3 of column i; group g takes k = 8 g .. 8 g + 7 of the step in two such reads
@@ -208,9 +211,10 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   // prologue: tiles 0 and 1 requested, tile 0 landed (tile 1 is waited for at the first barrier that publishes it)
 #pragma unroll
   for (int i = 0; i < ND; ++i) dma(0, i);
+  constexpr int ND1 = SHARED ? NDA : ND;  // (tile 1 meets tile 0's rhs)
 #pragma unroll
-  for (int i = 0; i < ND; ++i) dma(1, i);
-  wait_vmcnt<ND>();
+  for (int i = 0; i < ND1; ++i) dma(1, i);
+  wait_vmcnt<ND1>();
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int i = 0; i < R; ++i) read_frag(0, 0, i, 0);
@@ -329,15 +333,76 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
       }
     }
   };
+  // SHARED, with those two barriers: tile kt is plane P of its rhs tile.  The rhs fragments of step 1 are read with plane 0's first step and those of step 0 with plane 2's second one, where
+  // the registers of the rhs tile before have had their last use; from plane 0's barrier A on nobody reads that tile in LDS any more, and the next one's loads go out behind it, a half each with
+  // planes 0 and 1 (b).  Of loads and fragment reads it has three tenths less than tile by tile (10 loads a tile for 14, 20
+  // reads for 28 on 256 x 192), and the chip, held back by power, its clock: llama's gate and up of 1900 rows 228 -> 215 us, down 106 -> 99, q | k | v 63.7 -> 61.  The order of the sums is the same.
+  auto tile_shared = [&](int kt, auto plane, auto d, auto rn, auto b) {
+    constexpr int P = decltype(plane)::value;
+    constexpr bool D = decltype(d)::value, RN = decltype(rn)::value;
+    constexpr int R0 = NI + (P == 0 ? NJ : 0), R1 = RN ? NI + (P == 2 ? NJ : 0) : 0;
+    constexpr int NB0 = NDB / 2, B_FIRST = P == 1 ? NB0 : 0, NB = !decltype(b)::value || P == 2 ? 0 : P == 0 ? NB0 : NDB - NB0;
+    constexpr int NA = D ? NDA : 0, N = NA + NB;
+    constexpr int LOW = R0 + 4 > NM * 3 / 8 ? R0 + 4 : NM * 3 / 8, BAR = LOW < NM - 1 ? LOW : NM - 1;
+    constexpr int EARLY = N * (NM - BAR) / (2 * NM - BAR), LATE = N - EARLY, OPS = R1 + LATE;
+    static_assert(R0 <= NM && OPS <= NM && EARLY <= NM - BAR - 1, "at most one memory instruction per MFMA: M0 is written one MFMA ahead of its DMA");
+    const int cur = kt & 1, nxt = cur ^ 1;
+    // load e of this tile: the lhs of tile kt + 2 first, then its share of the next rhs tile
+    auto m0_of = [&](int e) { e < NA ? dma_m0(kt + 2, e) : dma_m0(kt + 3 - P, NDA + B_FIRST + e - NA); };
+    auto go_of = [&](int e) { e < NA ? dma_go(kt + 2, e) : dma_go(kt + 3 - P, NDA + B_FIRST + e - NA); };
+#pragma unroll
+    for (int g = 0; g < NM; ++g) {
+      if (g < R0) read_frag(cur, 1, g, 1);
+      if (g == BAR) {
+        wait_lgkmcnt0();
+        __builtin_amdgcn_s_barrier();
+      }
+      const int e = EARLY > 0 && g > BAR ? (g - BAR - 1) * EARLY / (NM - BAR - 1) : 0, e_next = EARLY > 0 && g > BAR ? (g - BAR) * EARLY / (NM - BAR - 1) : 0;
+      const bool load = e_next > e && e < EARLY;
+      if (load) m0_of(e);
+      acc[g / NJ][g % NJ] = mma16(T(), fb[0][g % NJ], fa[0][g / NJ], acc[g / NJ][g % NJ]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (load) go_of(e);
+    }
+    if (RN) {
+      wait_vmcnt<EARLY>();
+      __builtin_amdgcn_s_barrier();
+    }
+#pragma unroll
+    for (int g = 0; g < NM; ++g) {
+      const int t = (g * OPS + NM - 1) / NM, t_hi = ((g + 1) * OPS + NM - 1) / NM;
+      const int di = OPS ? t * LATE / OPS : 0, di_next = OPS ? (t + 1) * LATE / OPS : 0;
+      const bool load = t < t_hi && di_next > di;
+      if (load) m0_of(EARLY + di);
+      else if (t < t_hi) read_frag(nxt, 0, t - di, 0);
+      acc[g / NJ][g % NJ] = mma16(T(), fb[1][g % NJ], fa[1][g / NJ], acc[g / NJ][g % NJ]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (load) go_of(EARLY + di);
+    }
+  };
   auto tile = [&](int kt, auto d, auto rn) {
     if constexpr (TWO) tile_two(kt, d, rn);
     else tile_one(kt, d, rn);
   };
   using Y = std::true_type;
   using N_ = std::false_type;
-  for (int kt = 0; kt < KT - 2; ++kt) tile(kt, Y(), Y());
-  tile(KT - 2, N_(), Y());
-  tile(KT - 1, N_(), N_());
+  if constexpr (SHARED) {
+    using P0 = std::integral_constant<int, 0>;
+    using P1 = std::integral_constant<int, 1>;
+    using P2 = std::integral_constant<int, 2>;
+    for (int kt = 0; kt < KT - 3; kt += 3) {
+      tile_shared(kt, P0(), Y(), Y(), Y());
+      tile_shared(kt + 1, P1(), Y(), Y(), Y());
+      tile_shared(kt + 2, P2(), Y(), Y(), Y());
+    }
+    tile_shared(KT - 3, P0(), Y(), Y(), N_());
+    tile_shared(KT - 2, P1(), N_(), Y(), N_());
+    tile_shared(KT - 1, P2(), N_(), N_(), N_());
+  } else {
+    for (int kt = 0; kt < KT - 2; ++kt) tile(kt, Y(), Y());
+    tile(KT - 2, N_(), Y());
+    tile(KT - 1, N_(), N_());
+  }
 
   // Register e of lane l of block (i, j): row wm + 16 i + l % 16, column wn + 16 j + 4 (l / 16) + e.
   if constexpr (ROWS == 4) {
@@ -480,7 +545,7 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
 
 template <typename T, int BM, int BN, bool B_KN, bool F32OUT = false, int BDIV = 1, int ROWS = 0>
 hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, const float* residual = nullptr, const DmaRows& rw = DmaRows()) {
-  constexpr int STAGES = 2 * (BM + BN) * BK * 2, EPI = ROWS == 4 ? BM * (3 * BN + 16) : F32OUT || ROWS ? 0 : BM * (BN * 2 + 8);
+  constexpr int STAGES = (BDIV == 3 ? 2 * BM + BN : 2 * (BM + BN)) * BK * 2, EPI = ROWS == 4 ? BM * (3 * BN + 16) : F32OUT || ROWS ? 0 : BM * (BN * 2 + 8);
   constexpr int LDS_BYTES = STAGES > EPI ? STAGES : EPI;
   static std::atomic<unsigned long long> configured{0};  // one bit per device: the attribute is per device
   // the schedule with two barriers, except where it does not fit the registers (the transposing reads of the
