@@ -446,3 +446,15 @@ def test_rows_plan_beside_the_256x192_tile():
                       (2, 700, 5632, 2048): "256x192",        # 115 / 148 on 256 x 256
                       (1, 894, 10296, 1472): "256x192"}.items():  # 95 / 134 on 256 x 256
         assert _rows_plan(B, X3, *key).startswith(f"gemm_dma4<bf16,NT,{tile}"), (key, _rows_plan(B, X3, *key))
+
+
+@pytest.mark.parametrize("key, tile", [((2, 600, 2816, 1024), "128x128,512t,ring"),      # 33.0 us / 40.6 on gemm_tiled
+                                       ((1, 900, 4096, 4096), "128x128,512t,ring"),      # 85 / 101 on 256 x 128 in two parts
+                                       ((1, 1650, 1024, 2816), "64x128,512t,ring"),      # 40.0 / 45.2 on 256 x 128 in four
+                                       ((0, 1900, 2560, 2048), "64x128,512t,ring"),      # 600 tiles, past one round: 65 / 70 on 256 x 192 in two
+                                       ((2, 428, 1768, 640), "64x128,512t,ring"),        # 17.4 / 24.0 on gemm_tiled
+                                       ((0, 2048, 2560, 2048), "64x128,512t,ring"),      # 640 tiles
+                                       ((2, 384, 5632, 2048), "256x192,256t")])          # 67 / 74 on 64 x 128 in two parts of which each is past a round
+def test_three_planes_take_the_tile_priced_lowest(key, tile):
+    """Each us: the kernel named and the one that the prices of single planes named."""
+    assert _rows_plan(ug_amd.BF16, 1, *key).startswith(f"gemm_dma4<bf16,NT,{tile},3 planes"), _rows_plan(ug_amd.BF16, 1, *key)

@@ -633,18 +633,17 @@ bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile) {
 // What `tiles` tiles of the ring kernel take: a fixed part and, per round of 256 tiles, the K tiles.  The time of a K tile is mostly that of its
 // bytes on their way to a CU, some 100 bytes per ns from the memory-side cache and 60 from HBM however many are asked for at once (operands from
 // HBM: the kernel takes as long without its MFMAs), so it goes by where the operands come from.  MEMORY is a matrix nobody has read lately,
-// as the weights of a model's next layer are; CACHE what a product finds whose operands were written or read just before; PLANES an lhs of three
-// planes.  Fitted to (m x n x k, us): 2048^2 x 5632 from memory 51 (128 x 128) / 67 (256 x 128), 1024 x 2048 x
+// as the weights of a model's next layer are; CACHE what a product finds whose operands were written or read just before.  Fitted to (m x n x k, us): 2048^2 x 5632 from memory 51 (128 x 128) / 67 (256 x 128), 1024 x 2048 x
 // 5632 from memory 38 (64 x 128), 509 x 2048 x 5632 from memory 26 (64 x 64), 2048 x 11264 x 2048 from memory 89 (256 x 128), 700 x
 // 11264 x 2048 from memory 34 and 1500 x 11264 x 2048 68 (192 x 192); 2048^3 19.2 (128 x 128),
 // 1024 x 2048 x 4096 21.1 (64 x 128), 256 x 4096^2 14.7 (64 x 64), 584 x 360 x 6656 20.9 and 9 x 64 x 4416 13.2 (64 x 64).
-enum class Operands { MEMORY, CACHE, PLANES };
+enum class Operands { MEMORY, CACHE };
 static double ring_cost_us(size_t tiles, int kt, int tile, Operands from) {
-  const bool memory = from == Operands::MEMORY, planes = from == Operands::PLANES;
+  const bool memory = from == Operands::MEMORY;
   // 32 x 32, two workgroups to a CU: 54 rows of 2048 x 5632 14.1, 228 of 2048 x 2048 9.8, 228 of 3072 x 768 7.6
   if (tile == 16) return 2.3 + kt * (0.135 + (tiles > 256 ? 0.09 * std::min(1.0, (tiles - 256.0) / 256) : 0) + (tiles > 512 ? 0.2 * (tiles - 512.0) / 256 : 0));
-  const double t0 = tile == 129 ? 0.64 : tile == 97 ? 0.62 : tile == 65 ? (memory ? 0.54 : 0.30) : tile == 48 ? (memory ? 0.40 : 0.21) : memory ? 0.255 : planes ? 0.11 : 0.14;
-  const double t1 = tile == 129 ? 0.22 : tile == 97 ? 0.30 : memory ? 0 : tile == 65 ? 0.17 : tile == 48 ? 0.07 : planes ? 0.075 : 0.045;
+  const double t0 = tile == 129 ? 0.64 : tile == 97 ? 0.62 : tile == 65 ? (memory ? 0.54 : 0.30) : tile == 48 ? (memory ? 0.40 : 0.21) : memory ? 0.255 : 0.14;
+  const double t1 = tile == 129 ? 0.22 : tile == 97 ? 0.30 : memory ? 0 : tile == 65 ? 0.17 : tile == 48 ? 0.07 : 0.045;
   double us = tile == 129 || tile == 97 ? 5.0 : tile == 65 ? 4.0 : 3.3;
   for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (t0 + t1 * (left < 256 ? (double)left : 256.0) / 256.0);
   return us;
@@ -661,17 +660,14 @@ static double ring_cost_us(size_t tiles, int kt, int tile, Operands from) {
 // (3072 x 4096^2: 131 -> 91 us, 5120^2 x 1024: 77 -> 54, 1280 x 8192 x 2048: 64 -> 47, 2048 x 2560 x 2048: 35 -> 29,
 // 2304^3: 39 -> 35) and leaves those with about 128 tiles where they were (2048^2 x 5632: 56 us against 72).  The
 // 128 x 128 tile (two workgroups per CU) takes what neither fits: 2304^3 35 -> 31 us, 2048 x 2560 x 2048 29 -> 27.
-// 256 x 192, for three planes: what leaves 256 x 256 tiles a round and a half or a split.  Gate and up of a llama layer (k 2048, n 2 x 5632, with
-// the fold), us at 384 / 512 / 700 / 1024 / 1500 / 1900 / 2048 rows: 92 / 82 / 131 / 140 / 234 / 254 / 255 -> 76 / 74 / 116 / 126 / 205 / 238 / 240; k 1024, n 2 x 2816: 1500
-// 87 -> 68, 1900 92 -> 74; q | k | v of 1900 rows 80 -> 74 in two splits.  One plane of rows gains nothing (2048 x 11264 x 2048 from memory 97.6, 96.2 so).
 // UGHIP_GEMM_SHAPE=3 / 4 / 5 forces 256 x 256 / 256 x 128 / 128 x 128 where the kernel applies, 10 / 12 / 13 / 9 the ring's 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64, 0..2, 6 and 7 keep both out (tuning aid).
-double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile, bool beside_192) {
+double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile) {
   const size_t tiles = tile_count(p, batch, tile);
   if (!tiles) return 1e30;
   const int kt = p.K / BK;
   const bool nn = p.b_cs == 1 && p.b_rs != 1;
   if (ring_tile(tile))
-    return ring_cost_us(tiles, kt, tile, p.b_k_div == 3 ? Operands::PLANES : Operands::CACHE) * (nn ? 1.1 : 1.0) + (double)batch * p.M * p.N * 2 / 6.4e6;
+    return ring_cost_us(tiles, kt, tile, Operands::CACHE) * (nn ? 1.1 : 1.0) + (double)batch * p.M * p.N * 2 / 6.4e6;
   double us = 4.0 + (double)batch * p.M * p.N * 2 / 6.4e6;
   // (the figures below were fitted to the kernel on 32 x 32 x 16 MFMAs; on 16 x 16 x 32 and with the loads spread behind two
   // barriers every K tile takes 8 % less: 4096^3 97 us, 8 x 1024^3 18.8, 1024 x 4096^2 41 on 128 x 128 tiles)
@@ -681,13 +677,11 @@ double gemm_dma_cost_us(const MMArgs& p, size_t batch, int tile, bool beside_192
     // 0.47 + 0.16 x busy, the next 256 fill the second slots (2048^3 24.7 us, 2304^3 31.3, 2816^3 45.5, 5120^2 x 1024 61)
     us += kt * 0.88 * (double)(tiles / 512) * layout;
     const size_t left = tiles % 512;
-    // (beside_192: unsplit planes take as long with a few second slots filled as with most: 1900 x 2560 x 2048, 300 tiles, 78 us; 600 x 11264 x 2048, 440, 80)
-    if (left > 256) us += kt * (beside_192 && batch == 1 ? 0.82 : 0.63 + 0.25 * (double)(left - 256) / 256.0) * layout;
+    if (left > 256) us += kt * (0.63 + 0.25 * (double)(left - 256) / 256.0) * layout;
     else if (left) us += kt * (0.47 + 0.16 * (double)left / 256.0) * layout;
     return us;
   }
-  // (beside_192: 256 x 128 with unsplit planes: 1900 x 2560 x 2048 81.5 us, and 74.5 in two splits of 256 x 192)
-  const double t0 = tile == 256 ? 0.9 : tile == 192 ? 0.76 : beside_192 && batch == 1 ? 0.68 : 0.62, t1 = tile == 256 ? 0.6 : tile == 192 ? 0.4 : 0.2;
+  const double t0 = tile == 256 ? 0.9 : 0.62, t1 = tile == 256 ? 0.6 : 0.2;
   for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) {
     const double busy = (left < 256 ? (double)left : 256.0) / 256.0;
     us += kt * (t0 + t1 * busy) * layout;
@@ -767,6 +761,46 @@ bool gemm_dma_planes3_split_ok(const MMArgs& p, int nsplit) {
   if (nsplit < 1 || p.K % (BK * nsplit)) return false;
   const int kts = p.K / BK / nsplit;
   return kts % 3 == 0 && kts >= 4;
+}
+
+// What three planes against a matrix take on `tile` in `nsplit` parts of K, the result's way out with it (gated: 256 x 192 writes gated planes) but not a fold of slabs; < 0: not to be taken.
+// A fixed part (without the gap between two launches) and, per round of tiles, their K tiles (planes counted) at a time that grows with the share of the chip that is busy: with every workgroup that a CU holds (`per_cu`) a
+// new step and a slope.  Fitted to 107 products of 384 .. 4096 rows (3400 timed calls, each tile and 1, 2, 4, 8 parts): the choices by it are 1.1 % from the fastest in the mean; by the prices of one plane, with
+// 256 x 192 compared at a second price, they were 3.3 %.  us then -> now: 600 x 2 of 2816 x 1024 40.6 -> 33.0, 900 x 4096 x 4096 101 -> 85, 1650 x 1024 x 2816 45.2 -> 40.0, 450 x 2560 x 2048 32.6 -> 29.1, 509 x 2048 x 5632
+// 47.9 -> 45.3; llama's products of 1024 rows and more keep their tiles or gain up to a tenth.
+// The ring past one round: where a CU holds several workgroups their ends spread, and a little more than a round takes a quarter longer, not twice as long (1900 x 2560 x 2048, 600 tiles of 64 x 128: 65 us, 70 in two parts on 256 x 192);
+// below 48 K tiles such products keep the plans that callers hold them to (640 x 7600 x 640 31.5 us on 128 x 128, 27.9 so; 964 x 4928 x 256 19.6, 17.2).
+double gemm_dma_planes3_cost_us(const MMArgs& p, int tile, int nsplit, bool gated) {
+  static const struct Price {
+    int tile, per_cu;
+    double fixed, step[3], slope[3];
+  } prices[] = {
+      {256, 1, 3.3, {1.036}, {0.225}},
+      {192, 1, 3.2, {1.075}, {0}},
+      {128, 1, 3.4, {0.716}, {0.044}},
+      {64, 2, 2.95, {0.440, 0.144}, {0.142, 0.110}},
+      {65, 1, 4.1, {0.231}, {0.186}},
+      {48, 2, 4.25, {0.205, 0.152}, {0.015, 0.111}},
+      {32, 3, 3.95, {0.091, 0.065, 0.109}, {0.099, 0.027, 0.050}},
+  };
+  const size_t tiles = tile_count(p, (size_t)nsplit, tile);
+  for (const Price& c : prices) {
+    if (c.tile != tile) continue;
+    const size_t round = 256 * (size_t)c.per_cu;
+    const double kt = (double)(p.K / BK / nsplit);
+    double us = c.fixed + (double)p.M * p.N * 4 / 6.4e6 * (gated ? 0.25 : nsplit), rounds = (double)(tiles / round);
+    size_t last = tiles % round;
+    if (ring_tile(tile) && tiles > round) {
+      if (c.per_cu == 1 || nsplit > 1 || kt < 48) return -1.0;
+      rounds = std::max(1.25, (double)tiles / round), last = 0;
+    }
+    for (int j = 0; j < c.per_cu; ++j) {
+      const double left = std::min(256.0, std::max(0.0, (double)last - 256.0 * j));
+      us += kt * (rounds * (c.step[j] + c.slope[j]) + (left > 0 ? c.step[j] + c.slope[j] * left / 256 : 0.0));
+    }
+    return us;
+  }
+  return -1.0;
 }
 
 void gemm_dma_planes3_name(int tile, int nsplit, const char* tail, char* out, size_t out_len) {

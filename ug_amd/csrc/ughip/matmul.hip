@@ -813,30 +813,25 @@ static RowsRoute rows_route(const MMArgs& p, int dtype, bool x3, GemmEpilogue::K
     q.c = const_cast<void*>(dst);  // alignment of the result as f32
     const int named = x3_dma > 0 ? gemm_dma_forced_tile(x3_dma) : 0, forced_tile = named == 129 || named == 97 ? 0 : named;
     const int forced_split = (int)x3_split;
-    auto price = [&](int tile, int split, bool beside_192) {  // < 0: not taken
-      if ((forced_tile && tile != forced_tile) || (forced_split && split != forced_split) || !gemm_dma_planes3_split_ok(q, split)) return -1.0;
-      MMArgs qs = q;
-      if (split > 1) qs.K = q.K / split, qs.a_bs = qs.K, qs.b_bs = qs.K / 3, qs.c_bs = (long long)(m * rows);
-      if (!gemm_dma_supported(UGHIP_BF16, qs, (size_t)split, tile)) return -1.0;
-      // the kernel (its model counts 2 bytes per result element), the f32 result's other 2, and the fold where there is one:
-      // the slabs in, the result out, a launch
-      const bool fold = split > 1 || kind == GemmEpilogue::SWIGLU;
-      return gemm_dma_cost_us(qs, (size_t)split, tile, beside_192) + (double)split * m * rows * 2 / 6.4e6 + (fold ? 3.0 + (double)(split + 1) * m * rows * 4 / 6.4e6 : 0.0);
-    };
     double best = 0;
-    for (int tile : {256, 128, 65, 64, 48, 32})  // (codes 65, 48, 32: gemm_ring; 1900 x 2048 x 2048 64 -> 54 us, 512 x 2048 x 2048 32 -> 26)
-      for (int split : {1, 2, 4, 8})
-        if (const double us = price(tile, split, false); us >= 0 && (!r.dma_tile || us < best * 0.97)) r.dma_tile = tile, r.dma_split = split, best = us;
-    const double other = gemm_tiled_cost_us(dtype, p, 1);
-    // 64 x 64 tiles (code 32) whose long K is not split leave most CUs without one, and the others wait longer for each K tile than the model says: 1011 x 280
-    // x 2112 31.7 us, 25.2 on gemm_tiled; 740 x 512 x 2368 33.5 and 29.0; 3954 x 96 x 2368 43.7 and 39.5
-    if (r.dma_tile == 32 && r.dma_split == 1 && q.K >= 4096) best += 0.07 * (q.K / 64);
-    if (r.dma_tile && !forced_tile && other >= 0 && other < best * 1.05) r.dma_tile = 0;  // it has to be clearly cheaper: its model is the rougher one
-    // 256 x 192 against what these prices chose, at the price that products of this kind came to beside it.  (That price decides nothing else: choosing among the others
-    // by it, 964 x 4928 x 256 24.8 -> 33.3 us, 1683 x 2 of 2128 x 3008 131 -> 146, 640 x 7600 x 640 36.5 -> 41.8.)
-    best = r.dma_tile ? price(r.dma_tile, r.dma_split, true) : other;
-    for (int split : {1, 2, 4, 8})
-      if (const double us = price(192, split, true); us >= 0 && ((forced_tile && !r.dma_tile) || best < 0 || us < best * 0.97)) r.dma_tile = 192, r.dma_split = split, best = us;
+    for (int tile : {256, 192, 128, 65, 64, 48, 32})  // (codes 65, 48, 32: gemm_ring)
+      for (int split : {1, 2, 4, 8}) {
+        if ((forced_tile && tile != forced_tile) || (forced_split && split != forced_split) || !gemm_dma_planes3_split_ok(q, split)) continue;
+        MMArgs qs = q;
+        if (split > 1) qs.K = q.K / split, qs.a_bs = qs.K, qs.b_bs = qs.K / 3, qs.c_bs = (long long)(m * rows);
+        if (!gemm_dma_supported(UGHIP_BF16, qs, (size_t)split, tile)) continue;
+        const bool gates = kind == GemmEpilogue::SWIGLU && gemm_dma_planes3_gates(p, tile, split), fold = !gates && (split > 1 || kind == GemmEpilogue::SWIGLU);
+        double us = gemm_dma_planes3_cost_us(q, tile, split, gates);
+        if (us < 0 && !forced_tile) continue;
+        if (fold) us += 3.0 + (double)(split + 1) * m * rows * 4 / 6.4e6;  // the slabs in, the result out, a launch
+        // 64 x 64 tiles whose long K is not split leave most CUs without one, and the others wait longer for each K tile than the model says: 1011 x 280
+        // x 2112 31.7 us, 25.2 on gemm_tiled; 740 x 512 x 2368 33.5 and 29.0; 3954 x 96 x 2368 43.7 and 39.5
+        if (tile == 32 && split == 1 && q.K >= 4096) us += 0.07 * (q.K / 64);
+        if (!r.dma_tile || us < best) r.dma_tile = tile, r.dma_split = split, best = us;
+      }
+    double other = gemm_tiled_cost_us(dtype, p, 1);
+    if (kind == GemmEpilogue::SWIGLU && gemm_tiled_workspace_bytes(dtype, p, 1) == 0) other += 3.0 + 2.0 * m * rows * 4 / 6.4e6;  // its price of one part has no fold: 428 x 2 of 1768 x 640 24.0 us there, 17.4 on the ring
+    if (r.dma_tile && !forced_tile && other >= 0 && other < best * 1.05) r.dma_tile = 0, r.dma_split = 1;  // it has to be clearly cheaper: its model is the rougher one
   }
   if (r.dma_tile) r.kind = RowsRoute::DMA_PLANES;
   return r;
