@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "gemm.h"
+#include "layers.h"
 
 namespace ughip {
 
@@ -131,6 +132,99 @@ struct GroupTiles {
 
 // The products those kernels take, besides plain ones: see gemm_dma4.
 enum class DmaForm { PLAIN, PLANES3, ROWS, ROWS_GLU, ROWS_LOOKUP };
+// How a wave's NI x NJ fragments of rows leave (ROWS as in gemm_dma4, 3 as in gemm_ring): register e of fragment (i, j) is row row0 + 16 i of the tile's, column col0 + 16 j + e.
+// First everything that has to be loaded, then stores alone: a wait for a load behind a store is a wait for that store's way to memory as well, and with a bias or a table looked at
+// fragment by fragment each store was waited for before the next one went out, a lone wave per SIMD with nothing to do meanwhile: 256 x 256 tiles spent 26700 cycles here, gated ones
+// 23200; 20700 and 11800 so (2048 x 2 of 5632 x 2048 104 -> 94 us on them, 93 -> 92 on the ring's 256 x 128; 2048 x 8192 x 2048 62 -> 59).
+template <typename T, int ROWS, int NI, int NJ>
+__device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& rw, int m0, int m_last, int row0, int col0) {
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+  constexpr int NC = ROWS == 2 ? NJ / 2 : NJ;
+  floatx4 b[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) b[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (rw.bias) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) b[j] = *reinterpret_cast<const floatx4*>(rw.bias + (j < NC ? 0 : rw.n_out) + min(col0 + j % NC * 16, rw.n_out - 4));
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(b[j]));  // they are here from now on
+  if constexpr (ROWS == 3) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int id = rw.ids[m0 + min(row0 + i * 16, m_last)];
+      const bool known = id >= 0 && id < rw.table_rows;
+      const size_t at = (size_t)(known ? id : 0) * rw.table_stride + rw.table_col;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const size_t k = at + min(col0 + j * 16, rw.n_out - 4) + e;
+          const float f = rw.table_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(rw.table)[k]) : static_cast<const float*>(rw.table)[k];
+          acc[i][j][e] = gelu_tanh_f(acc[i][j][e] + b[j][e]) * (known ? f : __uint_as_float(0x7fc00000u));
+        }
+    }
+  }
+  auto value = [&](int i, int j) {
+    if constexpr (ROWS == 3) return acc[i][j];
+    floatx4 v = acc[i][j] + b[j];
+    if constexpr (ROWS == 2) {
+      floatx4 u = acc[i][j + NC] + b[j + NC];
+      if (rw.glu_limit > 0.f) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = v[e] > rw.glu_limit ? rw.glu_limit : v[e];
+          u[e] = u[e] > rw.glu_limit ? rw.glu_limit : u[e] < -rw.glu_limit ? -rw.glu_limit : u[e];
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = v[e] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * rw.glu_alpha * v[e])) * (u[e] + rw.glu_shift);
+    }
+    return v;
+  };
+  auto store = [&](auto* dst) {
+    auto* to = dst + (size_t)(m0 + row0) * rw.dst_stride + col0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      if (row0 + i * 16 <= m_last) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+          if (col0 + j * 16 < rw.n_out) {  // n_out % 4 == 0: a group of 4 columns exists whole or not at all
+            const floatx4 v = value(i, j);
+            if constexpr (sizeof(*dst) == 2) *reinterpret_cast<u32x2*>(to + j * 16) = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
+            else *reinterpret_cast<floatx4*>(to + j * 16) = v;
+          }
+      }
+      to += 16 * (size_t)rw.dst_stride;
+    }
+  };
+  if (rw.dst_bf16) store(static_cast<T*>(rw.dst));
+  else store(static_cast<float*>(rw.dst));
+}
+
+// How f32 sums leave, N % 8 == 0: rows of p.N from c on (+ residual where given, all of it loaded before the first store goes out, for the reason above).
+template <int NI, int NJ>
+__device__ __forceinline__ void sums_out(floatx4 (&acc)[NI][NJ], float* __restrict__ c, const float* __restrict__ residual, int n, int m_last, int n_left, int row0, int col0) {
+  if (residual) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const float* from = residual + (size_t)min(row0 + i * 16, m_last) * n;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] += *reinterpret_cast<const floatx4*>(from + min(col0 + j * 16, n_left - 4));
+    }
+  }
+  float* to = c + (size_t)row0 * n + col0;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    if (row0 + i * 16 <= m_last) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        if (col0 + j * 16 < n_left) *reinterpret_cast<floatx4*>(to + j * 16) = acc[i][j];  // a group of 4 columns exists whole or not at all
+    }
+    to += (size_t)16 * n;
+  }
+}
+
 // gemm_ring.hip: one of its tiles (codes 129, 97, 65, 48, 32: 256 x 128, 192 x 192, 128 x 128, 64 x 128, 64 x 64), operands as the _supported functions of gemm_dma.hip check them.
 hipError_t gemm_ring_launch(hipStream_t stream, int dtype, DmaForm form, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw);
 

@@ -462,56 +462,12 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
     return;
   }
   if constexpr (BY_ROW) {
-    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-    constexpr int NC = ROWS == 2 ? NJ / 2 : NJ;
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-      const int col = ROWS == 2 ? tn * (BN / 2) + (wave & 1) * (BN / 4) + j * 16 + (lane >> 4) * 4 : n0 + wn + j * 16 + (lane >> 4) * 4;
-      if (col >= rw.n_out) continue;  // n_out % 4 == 0: a group of 4 columns exists whole or not at all
-      floatx4 b = {0.f, 0.f, 0.f, 0.f}, bu = {0.f, 0.f, 0.f, 0.f};
-      if (rw.bias) {
-        b = *reinterpret_cast<const floatx4*>(rw.bias + col);
-        if (ROWS == 2) bu = *reinterpret_cast<const floatx4*>(rw.bias + rw.n_out + col);
-      }
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int row = wm + i * 16 + (lane & 15);
-        if (row > m_last) continue;
-        floatx4 v = acc[i][j] + b;
-        if constexpr (ROWS == 2) {
-          floatx4 u = acc[i][j + NC] + bu;
-          if (rw.glu_limit > 0.f) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              v[e] = v[e] > rw.glu_limit ? rw.glu_limit : v[e];
-              u[e] = u[e] > rw.glu_limit ? rw.glu_limit : u[e] < -rw.glu_limit ? -rw.glu_limit : u[e];
-            }
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = v[e] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * rw.glu_alpha * v[e])) * (u[e] + rw.glu_shift);
-        }
-        const size_t at = (size_t)(m0 + row) * rw.dst_stride + col;
-        if (rw.dst_bf16) *reinterpret_cast<u32x2*>(static_cast<T*>(rw.dst) + at) = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
-        else *reinterpret_cast<floatx4*>(static_cast<float*>(rw.dst) + at) = v;
-      }
-    }
+    rows_out<T, ROWS>(acc, rw, m0, m_last, wm + (lane & 15), (ROWS == 2 ? tn * (BN / 2) + (wave & 1) * (BN / 4) : n0 + wn) + (lane >> 4) * 4);
     return;
   }
   if constexpr (F32OUT) {
-    // four consecutive f32 per lane: 16-byte stores, 64 contiguous bytes per row and instruction
-    float* __restrict__ C = static_cast<float*>(p.c) + (size_t)batch * p.c_bs + (size_t)m0 * p.N + n0;
-    const float* __restrict__ Rz = residual ? residual + (size_t)batch * p.c_bs + (size_t)m0 * p.N + n0 : nullptr;
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int row = wm + i * 16 + (lane & 15), col = wn + j * 16 + (lane >> 4) * 4;
-        if (row <= m_last && col < n_left) {  // N % 8 == 0: a group of 4 columns exists whole or not at all
-          floatx4 v = acc[i][j];
-          if (Rz) v += *reinterpret_cast<const floatx4*>(Rz + (size_t)row * p.N + col);
-          *reinterpret_cast<floatx4*>(C + (size_t)row * p.N + col) = v;
-        }
-      }
+    const size_t at = (size_t)batch * p.c_bs + (size_t)m0 * p.N + n0;
+    sums_out(acc, static_cast<float*>(p.c) + at, residual ? residual + at : nullptr, p.N, m_last, n_left, wm + (lane & 15), wn + (lane >> 4) * 4);
     return;
   }
   // Epilogue through LDS.
