@@ -548,19 +548,29 @@ __global__ void __launch_bounds__(C * 4) delta_out_kernel(DeltaArgs a) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) ss[e] += o[v][e] * o[v][e];
   }
+  // Weights and gates all at once and in front of the first store: loaded one by one between the stores, each was waited for together with the store before it: 2048 rows, 16 heads of 128 columns 41 -> 31.5 us
+  float w[NV], z[NV][4];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int c = min(16 * v + j, a.vdim - 1);
+    w[v] = a.norm[c];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) z[v][e] = a.z[(size_t)(row0 + min(16 * I + 4 * kg + e, rows - 1)) * a.z_stride + (size_t)h * a.vdim + c];
+  }
   float inv[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) inv[e] = 1.f / sqrtf(row_sum16(ss[e]) / (float)a.vdim + a.eps);
 #pragma unroll
+  for (int v = 0; v < NV; ++v) asm volatile("" : "+v"(w[v]), "+v"(z[v][0]), "+v"(z[v][1]), "+v"(z[v][2]), "+v"(z[v][3]));  // here from now on
+#pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int c = 16 * v + j;
     if (c >= a.vdim) continue;
-    const float w = a.norm[c];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int r = 16 * I + 4 * kg + e;
       if (r >= rows) continue;
-      const float y = o[v][e] * inv[e] * w * sigmoid_f(a.z[(size_t)(row0 + r) * a.z_stride + (size_t)h * a.vdim + c]);
+      const float y = o[v][e] * inv[e] * w[v] * sigmoid_f(z[v][e]);
       const size_t to = (size_t)(row0 + r) * a.dst_stride + (size_t)h * a.vdim + c;
       if (a.dst_bf16) static_cast<uint16_t*>(a.dst)[to] = bf16_rne(y);
       else static_cast<float*>(a.dst)[to] = y;

@@ -260,6 +260,14 @@ __global__ void __launch_bounds__(256) rows_product_kernel(ProductArgs a) {
     }
    }
 
+  // (loaded here: a wait for a load between the stores is a wait for the stores before it)
+  float bias[2] = {0.f, 0.f};
+  if (a.bias) {
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+      bias[j] = ACT == UGHIP_ACT_SWIGLU ? a.bias[j * a.n + min(n0 + wn * 32 + (lane & 31), a.n - 1)] : a.bias[min(n0 + wn * 32 * NI + j * 32 + (lane & 31), a.n - 1)];
+  }
+  asm volatile("" : "+v"(bias[0]), "+v"(bias[1]));
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
 #pragma unroll
@@ -271,10 +279,10 @@ __global__ void __launch_bounds__(256) rows_product_kernel(ProductArgs a) {
         const int col = ACT == UGHIP_ACT_SWIGLU ? n0 + wn * 32 + (lane & 31) : n0 + wn * 32 * NI + j * 32 + (lane & 31);
         if (col >= a.n) continue;
         float v = acc[i][j][e];
-        if (a.bias) v += a.bias[col];
+        if (a.bias) v += bias[j];
         if constexpr (ACT == UGHIP_ACT_SWIGLU) {
           float u = acc[i][1][e];
-          if (a.bias) u += a.bias[a.n + col];
+          if (a.bias) u += bias[1];
           v = glu_f(v, u, a.glu);
         }
         if constexpr (ACT == UGHIP_ACT_GELU_MUL) v = gelu_tanh_f(v) * __uint_as_float(!there[i][e] ? 0x7fc00000u : a.table_bf16 ? factor[i][e][j] << 16 : factor[i][e][j]);

@@ -321,8 +321,9 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_out_kernel(SsmArgs a) {
   const int xt = q * PB / 4, st = np * PB / 4;
   TileRegs<4, VEC> x;
   TileRegs<8, VEC> s;
-  float decays = 0.f;  // A of row `lane` (first wave), d of it (second)
+  float decays = 0.f, next_skip = 0.f;  // A of row `lane` (first wave), d of it (second)
   auto fetch = [&](int i) {
+    next_skip = a.skip[hw.head(i)];
     const int pw = min(PB, a.vdim - hw.col(i));
     if (wave < 2) decays = (wave ? a.step : a.cum)[((size_t)chunk * a.heads + hw.head(i)) * 64 + lane];
     x.load(xbc0 + (size_t)hw.head(i) * a.vdim + hw.col(i), a.xbc_stride, rows, pw, PB / 4, xt);
@@ -373,6 +374,9 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_out_kernel(SsmArgs a) {
       tile_to_lds<VEC>(Ss + r0 * PS, PS, a.chunk_s + (((size_t)chunk * a.heads + h) * N + r0) * a.vdim + p0, a.vdim, N - r0, pw, PB / 4, min(2048, st - base));
     }
     if (wave < 2) (wave ? d : cum)[lane] = decays;
+    // here with the rest of the item: looked at between the stores below it would be waited for behind the next item's loads, and each store with them; 509 rows of 64 heads of 64, state 128: 23.6 -> 23.0 us
+    float skip = next_skip;
+    asm volatile("" : "+v"(skip));
     __syncthreads();
     if (it + 1 < hw.items) fetch(it + 1);
     if (wave >= tq) continue;  // q < 64: the waves without rows only move data
@@ -395,7 +399,6 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_out_kernel(SsmArgs a) {
         from_s[u] = mfma16(c.w, Ss[(k + 3) * PS + u * 16 + j], from_s[u]);
       }
     });
-    const float skip = a.skip[h];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int i = i0 + 4 * kg + e;
