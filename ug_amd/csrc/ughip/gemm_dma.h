@@ -136,8 +136,13 @@ enum class DmaForm { PLAIN, PLANES3, ROWS, ROWS_GLU, ROWS_LOOKUP };
 // First everything that has to be loaded, then stores alone: a wait for a load behind a store is a wait for that store's way to memory as well, and with a bias or a table looked at
 // fragment by fragment each store was waited for before the next one went out, a lone wave per SIMD with nothing to do meanwhile: 256 x 256 tiles spent 26700 cycles here, gated ones
 // 23200; 20700 and 11800 so (2048 x 2 of 5632 x 2048 104 -> 94 us on them, 93 -> 92 on the ring's 256 x 128; 2048 x 8192 x 2048 62 -> 59).
+// A store takes a CU's address unit a cycle for each lane that does not follow its neighbour in memory, and a lane of a fragment has a row to itself: 70 to 80 cycles where 16 would do.  So 16
+// rows at a time go through the wave's own piece of LDS (nobody reads operands any more; a wave's LDS instructions keep their order, so there is no barrier) and leave in 16-byte
+// pieces of whole rows, the next 16 on their way into a second piece: us, 2048 rows, weights from memory: f32 3072 x 2048
+// 47.8 -> 45.2 (256 x 256 tiles), 43.4 -> 41.8 (128 x 128); bf16 8192 x 2048 69.3 -> 66.5 (256 x 128), 86.3 -> 81.3 (128 x 128); gated 2 x 5632 92.2 -> 90.9, 116 -> 112.5.
 template <typename T, int ROWS, int NI, int NJ>
-__device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& rw, int m0, int m_last, int row0, int col0) {
+__device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& rw, int m0, int m_last, int row_base, int col_base, int wave, u32x4* lds) {
+  const int lane = threadIdx.x & 63, row0 = row_base + (lane & 15), col0 = col_base + (lane >> 4) * 4;
   typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
   constexpr int NC = ROWS == 2 ? NJ / 2 : NJ;
   floatx4 b[NJ];
@@ -182,7 +187,37 @@ __device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& 
     }
     return v;
   };
-  auto store = [&](auto* dst) {
+  auto out = [&](auto* dst) {
+    constexpr int E = sizeof(*dst), PER = 16 / E, CPR = NC * 16 / PER, RP = 64 / CPR, PITCH = NC * 16 * E + 16, PIECE = 16 * PITCH;  // elements of 16 bytes, those of a row, rows of a pass
+    typedef char __attribute__((address_space(3))) lds_char;
+    if (CPR >= 4 && (E == 4 || ((rw.n_out | rw.dst_stride) % 8 == 0 && ((size_t)rw.dst & 15) == 0))) {
+      lds_char* mine = (lds_char*)lds + wave * 2 * PIECE;
+      auto put = [&](int i) {
+        lds_char* to = mine + (i & 1) * PIECE + (lane & 15) * PITCH + (lane >> 4) * 4 * E;
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+          const floatx4 v = value(i, j);
+          if constexpr (E == 2) *(u32x2 __attribute__((address_space(3)))*)(to + j * 32) = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
+          else *(floatx4 __attribute__((address_space(3)))*)(to + j * 64) = v;
+        }
+        asm volatile("" ::: "memory");
+      };
+      put(0);
+      const int c = lane % CPR, r0 = lane / CPR, row = row_base + r0, col = col_base + c * PER;
+      const bool there = r0 < RP && col < rw.n_out;  // n_out % PER == 0: a piece exists whole or not at all
+      auto* to = dst + (size_t)(m0 + row) * rw.dst_stride + col;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        if (i + 1 < NI) put(i + 1);
+#pragma unroll
+        for (int r = 0; r < 16; r += RP) {
+          if (there && r + r0 < 16 && row + i * 16 + r <= m_last)
+            *reinterpret_cast<u32x4*>(to + (i * 16 + r) * (size_t)rw.dst_stride) = *(const u32x4 __attribute__((address_space(3)))*)(mine + (i & 1) * PIECE + (r + r0) * PITCH + c * 16);
+        }
+        asm volatile("" ::: "memory");
+      }
+      return;
+    }
     auto* to = dst + (size_t)(m0 + row0) * rw.dst_stride + col0;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
@@ -191,15 +226,15 @@ __device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& 
         for (int j = 0; j < NC; ++j)
           if (col0 + j * 16 < rw.n_out) {  // n_out % 4 == 0: a group of 4 columns exists whole or not at all
             const floatx4 v = value(i, j);
-            if constexpr (sizeof(*dst) == 2) *reinterpret_cast<u32x2*>(to + j * 16) = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
+            if constexpr (E == 2) *reinterpret_cast<u32x2*>(to + j * 16) = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
             else *reinterpret_cast<floatx4*>(to + j * 16) = v;
           }
       }
       to += 16 * (size_t)rw.dst_stride;
     }
   };
-  if (rw.dst_bf16) store(static_cast<T*>(rw.dst));
-  else store(static_cast<float*>(rw.dst));
+  if (rw.dst_bf16) out(static_cast<T*>(rw.dst));
+  else out(static_cast<float*>(rw.dst));
 }
 
 // How f32 sums leave, N % 8 == 0: rows of p.N from c on (+ residual where given, all of it loaded before the first store goes out, for the reason above).

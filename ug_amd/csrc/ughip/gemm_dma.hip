@@ -462,7 +462,8 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
     return;
   }
   if constexpr (BY_ROW) {
-    rows_out<T, ROWS>(acc, rw, m0, m_last, wm + (lane & 15), (ROWS == 2 ? tn * (BN / 2) + (wave & 1) * (BN / 4) : n0 + wn) + (lane >> 4) * 4);
+    static_assert(2 * STAGE_BYTES >= 4 * 2 * 16 * (BN / 2 * 4 + 16), "a wave's two pieces of 16 rows");
+    rows_out<T, ROWS>(acc, rw, m0, m_last, wm, ROWS == 2 ? tn * (BN / 2) + (wave & 1) * (BN / 4) : n0 + wn, wave, lds);
     return;
   }
   if constexpr (F32OUT) {

@@ -214,7 +214,8 @@ __device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group,
 
   // Register e of lane l of block (i, j): row wm + 16 i + l % 16, column wn + 16 j + 4 (l / 16) + e.
   if constexpr (ROWS != 0) {
-    rows_out<T, ROWS>(acc, rw, m0, m_last, wm + (lane & 15), (ROWS == 2 ? tn * (BN / 2) + (wave & 1) * (BN / 4) : n0 + wn) + (lane >> 4) * 4);
+    static_assert(S * STAGE_BYTES >= W * 2 * 16 * (BN / 2 * 4 + 16), "a wave's two pieces of 16 rows");
+    rows_out<T, ROWS>(acc, rw, m0, m_last, wm, ROWS == 2 ? tn * (BN / 2) + (wave & 1) * (BN / 4) : n0 + wn, wave, lds);
     return;
   }
   if constexpr (F32OUT) {
