@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "gemm.h"
 #include "layers.h"
 
@@ -142,7 +144,9 @@ enum class DmaForm { PLAIN, PLANES3, ROWS, ROWS_GLU, ROWS_LOOKUP };
 // 47.8 -> 45.2 (256 x 256 tiles), 43.4 -> 41.8 (128 x 128); bf16 8192 x 2048 69.3 -> 66.5 (256 x 128), 86.3 -> 81.3 (128 x 128); gated 2 x 5632 92.2 -> 90.9, 116 -> 112.5.
 template <typename T, int ROWS, int NI, int NJ>
 __device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& rw, int m0, int m_last, int row_base, int col_base, int wave, u32x4* lds) {
-  const int lane = threadIdx.x & 63, row0 = row_base + (lane & 15), col0 = col_base + (lane >> 4) * 4;
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));  // (not worked out in front of the products, where there is no register to keep it in)
+  const int row0 = row_base + (lane & 15), col0 = col_base + (lane >> 4) * 4;
   typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
   constexpr int NC = ROWS == 2 ? NJ / 2 : NJ;
   floatx4 b[NJ];
@@ -168,6 +172,7 @@ __device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& 
           const float f = rw.table_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(rw.table)[k]) : static_cast<const float*>(rw.table)[k];
           acc[i][j][e] = gelu_tanh_f(acc[i][j][e] + b[j][e]) * (known ? f : __uint_as_float(0x7fc00000u));
         }
+      asm volatile("" ::: "memory");  // (16 rows' table elements at a time: all of them at once are more than the registers hold)
     }
   }
   auto value = [&](int i, int j) {
@@ -188,10 +193,10 @@ __device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& 
     return v;
   };
   auto out = [&](auto* dst) {
-    constexpr int E = sizeof(*dst), PER = 16 / E, CPR = NC * 16 / PER, RP = 64 / CPR, PITCH = NC * 16 * E + 16, PIECE = 16 * PITCH;  // elements of 16 bytes, those of a row, rows of a pass
+    constexpr int E = sizeof(*dst), PER = 16 / E, CPR = NC * 16 / PER, RP = 64 / CPR, PITCH = NC * 16 * E + 16, PIECE = 16 * PITCH, PIECES = NI > 1 ? 2 : 1;  // elements of 16 bytes, those of a row, rows of a pass
     typedef char __attribute__((address_space(3))) lds_char;
     if (CPR >= 4 && (E == 4 || ((rw.n_out | rw.dst_stride) % 8 == 0 && ((size_t)rw.dst & 15) == 0))) {
-      lds_char* mine = (lds_char*)lds + wave * 2 * PIECE;
+      lds_char* mine = (lds_char*)lds + wave * PIECES * PIECE;
       auto put = [&](int i) {
         lds_char* to = mine + (i & 1) * PIECE + (lane & 15) * PITCH + (lane >> 4) * 4 * E;
 #pragma unroll
@@ -237,26 +242,45 @@ __device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& 
   else out(static_cast<float*>(rw.dst));
 }
 
-// How f32 sums leave, N % 8 == 0: rows of p.N from c on (+ residual where given, all of it loaded before the first store goes out, for the reason above).
+// How f32 sums leave, N % 8 == 0: rows of n from c on, by the same way.  A residual is added to them first, all of it loaded before the first store (but for
+// the tile whose sums leave no registers for that).
 template <int NI, int NJ>
-__device__ __forceinline__ void sums_out(floatx4 (&acc)[NI][NJ], float* __restrict__ c, const float* __restrict__ residual, int n, int m_last, int n_left, int row0, int col0) {
-  if (residual) {
+__device__ __forceinline__ void sums_out(floatx4 (&acc)[NI][NJ], float* __restrict__ c, const float* __restrict__ residual, int n, int m_last, int n_left, int row_base, int col_base,
+                                         int wave, u32x4* lds) {
+  constexpr int CPR = NJ * 4, RP = 64 / CPR, PITCH = NJ * 64 + 16, PIECE = 16 * PITCH, PIECES = NI > 1 ? 2 : 1;
+  typedef char __attribute__((address_space(3))) lds_char;
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));
+  if (NI * NJ < 64 && residual) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const float* from = residual + (size_t)min(row0 + i * 16, m_last) * n;
+      const float* from = residual + (size_t)min(row_base + i * 16 + (lane & 15), m_last) * n;
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[i][j] += *reinterpret_cast<const floatx4*>(from + min(col0 + j * 16, n_left - 4));
+      for (int j = 0; j < NJ; ++j) acc[i][j] += *reinterpret_cast<const floatx4*>(from + min(col_base + j * 16 + (lane >> 4) * 4, n_left - 4));
     }
   }
-  float* to = c + (size_t)row0 * n + col0;
+  const int r0 = lane / CPR, row = row_base + r0, col = col_base + lane % CPR * 4;
+  const bool there = r0 < RP && col < n_left;  // a piece exists whole or not at all
+  lds_char* mine = (lds_char*)lds + wave * PIECES * PIECE;
+  auto put = [&](int i) {
+    lds_char* to = mine + (i & 1) * PIECE + (lane & 15) * PITCH + (lane >> 4) * 16;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) *(floatx4 __attribute__((address_space(3)))*)(to + j * 64) = acc[i][j];
+    asm volatile("" ::: "memory");
+  };
+  float* to = c + (size_t)row * n + col;
+  put(0);
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    if (row0 + i * 16 <= m_last) {
+    if (i + 1 < NI) put(i + 1);
 #pragma unroll
-      for (int j = 0; j < NJ; ++j)
-        if (col0 + j * 16 < n_left) *reinterpret_cast<floatx4*>(to + j * 16) = acc[i][j];  // a group of 4 columns exists whole or not at all
-    }
-    to += (size_t)16 * n;
+    for (int r = 0; r < 16; r += RP)
+      if (there && r + r0 < 16 && row + i * 16 + r <= m_last) {
+        floatx4 v = *(const floatx4 __attribute__((address_space(3)))*)(mine + (i & 1) * PIECE + (r + r0) * PITCH + lane % CPR * 16);
+        if (NI * NJ == 64 && residual) v += *reinterpret_cast<const floatx4*>(residual + (size_t)(row + i * 16 + r) * n + col);
+        *reinterpret_cast<floatx4*>(to + (size_t)(i * 16 + r) * n) = v;
+      }
+    asm volatile("" ::: "memory");
   }
 }
 

@@ -461,14 +461,14 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
     }
     return;
   }
+  static_assert(2 * A_BYTES + (SHARED ? 1 : 2) * B_BYTES >= 4 * (NI > 1 ? 2 : 1) * 16 * (BN / 2 * 4 + 16), "what rows and f32 sums leave by: pieces of 16 rows of a wave's columns");
   if constexpr (BY_ROW) {
-    static_assert(2 * STAGE_BYTES >= 4 * 2 * 16 * (BN / 2 * 4 + 16), "a wave's two pieces of 16 rows");
     rows_out<T, ROWS>(acc, rw, m0, m_last, wm, ROWS == 2 ? tn * (BN / 2) + (wave & 1) * (BN / 4) : n0 + wn, wave, lds);
     return;
   }
   if constexpr (F32OUT) {
     const size_t at = (size_t)batch * p.c_bs + (size_t)m0 * p.N + n0;
-    sums_out(acc, static_cast<float*>(p.c) + at, residual ? residual + at : nullptr, p.N, m_last, n_left, wm + (lane & 15), wn + (lane >> 4) * 4);
+    sums_out(acc, static_cast<float*>(p.c) + at, residual ? residual + at : nullptr, p.N, m_last, n_left, wm, wn, wave, lds);
     return;
   }
   // Epilogue through LDS.

@@ -213,14 +213,14 @@ __device__ __forceinline__ void ring_tile(const MMArgs& p, int batch, int group,
   }
 
   // Register e of lane l of block (i, j): row wm + 16 i + l % 16, column wn + 16 j + 4 (l / 16) + e.
+  static_assert(S * A_BYTES + (SHARED ? 2 : S) * B_BYTES >= W * (NI > 1 ? 2 : 1) * 16 * (BN / 2 * 4 + 16), "what rows and f32 sums leave by: pieces of 16 rows of a wave's columns");
   if constexpr (ROWS != 0) {
-    static_assert(S * STAGE_BYTES >= W * 2 * 16 * (BN / 2 * 4 + 16), "a wave's two pieces of 16 rows");
     rows_out<T, ROWS>(acc, rw, m0, m_last, wm, ROWS == 2 ? tn * (BN / 2) + (wave & 1) * (BN / 4) : n0 + wn, wave, lds);
     return;
   }
   if constexpr (F32OUT) {
     const size_t at = (size_t)batch * p.c_bs + (size_t)m0 * p.N + n0;
-    sums_out(acc, static_cast<float*>(p.c) + at, residual ? residual + at : nullptr, p.N, m_last, n_left, wm + (lane & 15), wn + (lane >> 4) * 4);
+    sums_out(acc, static_cast<float*>(p.c) + at, residual ? residual + at : nullptr, p.N, m_last, n_left, wm, wn, wave, lds);
     return;
   }
   // 16-bit result through LDS, out in 16-byte pieces of whole rows past the cache.
