@@ -372,3 +372,25 @@ def test_f32_rows_of_every_tile(hip, m, n, k, groups, act):
     out = get(dst, m * n + 8)
     assert np.all(np.isnan(out[m * n :])), "wrote past the end"
     close(out[: m * n].reshape(m, n), y, 1e-5)  # k eps and the gate's few units, against sums of some standard deviations
+
+
+# Rows leave in 16-byte pieces through LDS where a bf16 row starts on one, else fragment by fragment: the same bits either way, edges of tiles and of pieces, nothing behind a row touched.
+@pytest.mark.parametrize("shape", ["3", "10", "11", "12", "13", "9", "17"])
+@pytest.mark.parametrize("m, n, act", [(300, 200, NONE), (257, 392, NONE), (16, 520, NONE), (271, 136, SWIGLU), (97, 200, SWIGLU)])
+def test_rows_leave_in_pieces_with_the_same_bits(hip, tune, shape, m, n, act):
+    if shape == "17" and act == SWIGLU:
+        pytest.skip("32 x 32 tiles are for plain rows")
+    gpu, k, rows = Gpu(hip), 512, 2 * n if act == SWIGLU else n
+    dx, dw, bias = gpu.up(rand(1, m, k), bf16=True), gpu.up(rand(2, rows, k, std=k ** -0.5), bf16=True), gpu.up(rand(3, rows))
+    tune.setenv("UGHIP_GEMM_SHAPE", shape)
+    got = {}
+    for bf16, gap in ((True, 8), (True, 4), (False, 8)):
+        print("rows out", shape, m, n, act, bf16, gap, flush=True)
+        dst = gpu.out(m * (n + gap), bf16=bf16)
+        gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n + gap), w=dw.raw(), bias=bias.raw(), m=m, n=n, k=k, product=BF16, act=act)))
+        assert "rows" in ug_amd.last_kernel() and "gemm_dma4" in ug_amd.last_kernel()
+        out = get(dst, m * (n + gap)).reshape(m, n + gap)
+        assert np.all(np.isnan(out[:, n:])) and np.all(np.isfinite(out[:, :n]))
+        got[bf16, gap] = out[:, :n]
+    np.testing.assert_array_equal(got[True, 8], got[True, 4])
+    np.testing.assert_array_equal(got[True, 8], rng.bf16_round(got[False, 8].ravel()).reshape(m, n))
