@@ -4,6 +4,7 @@ import ctypes as C
 import os
 import subprocess
 import sys
+import zlib
 
 import numpy as np
 import pytest
@@ -187,6 +188,33 @@ def test_grouped_attention_of_long_and_short_rows(gpu, sizes, cuts, bf16):
         got = attend(gpu, bf16, qkv, caches, T, t, pos, sizes, 0, scale, None, None)
         assert np.all(np.abs(got - want[pos : pos + t]) <= bound[pos : pos + t])
         pos += t
+
+
+# blocks of 64 and of 128 queries (192 elements), rows in one and two cuts, windows that start in either tile of a pair, results by fours and one by one
+@pytest.mark.parametrize("sizes, cuts, window, crc", [
+    ((16, 4, 128, 128, 0), (300,), 0, [1772602968]),
+    ((6, 2, 128, 90, 0), (70, 333), 0, [911175894, 3328899887]),
+    ((6, 2, 128, 90, 0), (70, 333), 333, [911175894, 1705608865]),
+    ((3, 3, 64, 64, 0), (1000, 513), 0, [955323054, 3587285614]),
+    ((3, 3, 64, 64, 0), (1000, 513), 333, [1205601681, 2264395259]),
+    ((2, 1, 60, 64, 0), (200,), 65, [1477877535]),
+    ((16, 16, 192, 128, 0), (509,), 0, [2093468606]),
+    ((16, 16, 192, 128, 0), (509,), 333, [3384680947]),
+    ((16, 16, 192, 128, 0), (2040,), 0, [3100763969]),
+    ((16, 16, 192, 128, 0), (2040,), 333, [1720511848]),
+    ((4, 2, 180, 100, 0), (77, 700), 0, [1699460730, 231609664]),
+    ((4, 2, 180, 100, 0), (77, 700), 333, [1699460730, 2151974969])])
+def test_attention_of_bf16_rows_keeps_its_order_of_sums(gpu, sizes, cuts, window, crc):
+    """The bits: a model's choices of experts and the last bits of its bf16 rows hang on them."""
+    H, G, d, vd, _ = sizes
+    T = sum(cuts)
+    qkv = np.random.default_rng(8).integers(-96, 97, (T, (H + G) * d + G * vd)) / 32.0
+    caches, pos, sums = caches_for(gpu, G, d, vd, T, True), 0, []
+    for t in cuts:
+        got = attend(gpu, True, qkv, caches, T, t, pos, sizes, window, d ** -0.5, None, None)
+        sums.append(zlib.crc32(got.astype(np.float32).tobytes()))
+        pos += t
+    assert sums == crc, sums
 
 
 # ---- delta rule --------------------------------------------------------------------------------------------------------------
