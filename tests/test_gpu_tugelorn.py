@@ -190,6 +190,20 @@ def test_grouped_attention_of_long_and_short_rows(gpu, sizes, cuts, bf16):
         pos += t
 
 
+# a window that makes most rows as long, in one round of blocks of 128 queries: whole tiles of keys to a wave
+@pytest.mark.parametrize("bf16, sizes", [(False, (16, 4, 128, 100, 0)), (False, (16, 2, 192, 128, 0)), (True, (16, 2, 256, 200, 0))])
+def test_grouped_attention_of_rows_as_long(gpu, bf16, sizes):
+    H, G, d, vd, _ = sizes
+    T, window, scale = 2040, 1000, d ** -0.5
+    qkv = rand(5, T, (H + G) * d + G * vd)
+    k, v, q = qkv[:, H * d : (H + G) * d].reshape(T, G, d), qkv[:, (H + G) * d :].reshape(T, G, vd), qkv[:, : H * d].reshape(T, H, d)
+    want, spread = pt.grouped_attention(q, k, v, scale, window), pt.grouped_attention(q, k, np.abs(v), scale, window)
+    off = np.stack([2.0 ** -9 * scale * (np.abs(q[:, h]) @ np.abs(k[:, h // (H // G)]).T).max(1) for h in range(H)], 1)  # as above
+    bound = 1e-4 * np.sqrt(np.mean(want ** 2)) + (np.expm1(2 * off)[:, :, None] * spread if bf16 else np.zeros_like(spread))
+    got = attend(gpu, bf16, qkv, caches_for(gpu, G, d, vd, T, bf16), T, T, 0, sizes, window, scale, None, None)
+    assert np.all(np.abs(got - want) <= bound)
+
+
 # blocks of 64 and of 128 queries (192 elements), rows in one and two cuts, windows that start in either tile of a pair, results by fours and one by one
 @pytest.mark.parametrize("sizes, cuts, window, crc", [
     ((16, 4, 128, 128, 0), (300,), 0, [1772602968]),

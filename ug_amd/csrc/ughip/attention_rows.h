@@ -7,7 +7,7 @@
 //   the same queries and other keys meet at the end.
 //   bf16 operands: v_mfma_f32_32x32x16_bf16, a weight as two bf16 terms (16 bits of it); f32: v_mfma_f32_32x32x2_f32.
 // bf16 heads of up to 192 elements: two groups of waves take every second tile of keys, by blocks of 128 queries, however many queries a workgroup has: a rounding in front of a product may turn a
-// router's choice or a bf16 row's last bit, so the order of these sums stays.  Otherwise a wave has a half of every tile.
+// router's choice or a bf16 row's last bit, so the order of these sums stays.  Otherwise a wave has a half of every tile (or, f32 in one round of workgroups, a tile).
 // What bounds it (bf16, 128 elements): the vector instructions of a wave's softmax and splits, 240 for 32 x 32 scores and 27 of 63 thousand cycles, 19 thousand of MFMA, and a wave's steps
 // one behind the other.  us with the launch that places queries and keys (11 to 16), 128 queries to a workgroup, then 64 queries and two workgroups to a CU: 16 heads of 128 on 4, 509 / 1024 / 2048 positions 25.3 / 39.0 /
 // 67.7 -> 21.6 / 33.3 / 59.9, 2048 behind a window of 1024 50.4 -> 50.9; 16 heads of 64 18.8 / 27.8 / 46.6 -> 16.8 / 24.3 / 42.6.  At 192 elements LDS has no room for two: 16 heads, 64 queries 30.6 / 46.3 / 86.5, 128 queries 33.3 /
@@ -16,6 +16,8 @@
 // of 128 85 / 301 -> 56 / 200, of 192 106 / 374 -> 70 / 251.
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "bf16_split.h"
 #include "layers.h"
@@ -349,15 +351,33 @@ hipError_t attention_rows_launch_as(ughip_device* dev, AttRowsArgs a, int heads)
   return hipGetLastError();
 }
 
+// Tiles of keys that the workgroup of the last but n-th block of queries goes through
+inline int attention_rows_tiles(const AttRowsArgs& a, int block, int n) {
+  const int q0 = std::max(0, (a.t + block - 1) / block - 1 - n) * block, last = a.pos + std::min(a.t, q0 + block);
+  return (last + ATT_KT - 1) / ATT_KT - (a.window ? std::max(0, a.pos + q0 - a.window + 1) / ATT_KT : 0);
+}
+// What the busiest CU of up to two rounds goes through, the longest rows first: the longest by itself, or the shortest of the first round and the longest of the second
+inline int attention_rows_busiest(const AttRowsArgs& a, int block, int heads, int cus) {
+  const int longest = attention_rows_tiles(a, block, 0);
+  if ((size_t)heads * ((a.t + block - 1) / block) <= (size_t)cus) return longest;
+  return std::max(longest, attention_rows_tiles(a, block, (cus - 1) / heads) + attention_rows_tiles(a, block, cus / heads));
+}
+
 // heads x blocks of queries; q_rows a multiple of ATT_QT
 template <typename T, int DQ, int DV>
 hipError_t attention_rows_launch(ughip_device* dev, AttRowsArgs a, int heads) {
   a.whole = a.vdim == DV && a.dst_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(a.dst) & (a.dst_bf16 ? 7 : 15)) == 0;
+  const size_t blocks = ((size_t)a.t + 127) / 128, cus = (size_t)dev->num_cus;
   if constexpr (sizeof(T) == 2 && DQ <= 192 && DV <= 128) {
     if constexpr (DQ == 192)
-      if ((size_t)heads * ((a.t + 127) / 128) >= (size_t)dev->num_cus) return attention_rows_launch_as<T, DQ, DV, 2, 1, 4>(dev, a, heads);
+      if (heads * blocks >= cus) return attention_rows_launch_as<T, DQ, DV, 2, 1, 4>(dev, a, heads);
     return attention_rows_launch_as<T, DQ, DV, 2, 1, 2>(dev, a, heads);
   } else {
+    // Halves of tiles and 64 queries, at 0.59 of the time of a whole tile with 128, unless those are one round and a window makes most rows as long: 16 heads over 2048 positions behind a window of 1024, 18 tiles against 17 + 16
+    // halves, us on halves and on whole tiles: f32 of 128 / 192 / 256 elements 193 / 243 / 432 and 183 / 228 / 395, bf16 of 256 133 and 113.  Over 1900 positions 178 and 184, without a window 199 and 302.
+    if constexpr (DQ >= 128)
+      if (heads * blocks <= cus && attention_rows_busiest(a, 128, heads, dev->num_cus) < 0.59 * attention_rows_busiest(a, 64, heads, dev->num_cus))
+        return attention_rows_launch_as<T, DQ, DV, 1, 1, 4>(dev, a, heads);
     return attention_rows_launch_as<T, DQ, DV, 1, 2, 2>(dev, a, heads);
   }
 }
