@@ -349,10 +349,12 @@ def test_smallest_ring_tile_gives_the_next_ones_bits(hip, tune, m, n, k, form):
     np.testing.assert_array_equal(got["64x64,512t"], got["32x32,256t"])
 
 
-# f32 rows on 128 x 128, 64 x 128 and 64 x 64 tiles as the rounds of 256 have it; K of a step less and a step more, gated and plain, even and uneven groups
-@pytest.mark.parametrize("m, n, k, groups, act", [(70, 2050, 33, 0, SWIGLU), (129, 1040, 64, 0, SWIGLU), (300, 5632, 40, 0, SWIGLU), (513, 6592, 36, 0, NONE), (700, 6592, 31, 0, NONE), (1531, 2048, 24, 0, NONE),
-                                                  (150, 300, 20, 0, NONE), (1200, 1408, 28, 16, SWIGLU), (1200, 2048, 28, 16, NONE), (2036, 264, 20, 5, SWIGLU)])
-def test_f32_rows_of_every_tile(hip, m, n, k, groups, act):
+# f32 rows on 128 x 128, 64 x 128 and 64 x 64 tiles as the rounds of 256 have it, a few tiles and one past a round too; K of a step less and a step more, gated and plain, even and uneven groups
+@pytest.mark.parametrize("m, n, k, groups, act, tile", [
+    (70, 2050, 33, 0, SWIGLU, "64x128"), (129, 1040, 64, 0, SWIGLU, "64x128"), (300, 5632, 40, 0, SWIGLU, "64x128"), (513, 6592, 36, 0, NONE, "64x128"), (700, 6592, 31, 0, NONE, "64x64"),
+    (1531, 2048, 24, 0, NONE, "128x128"), (150, 300, 20, 0, NONE, "64x64"), (1200, 1408, 28, 16, SWIGLU, "64x128"), (1200, 2048, 28, 16, NONE, "64x128"), (2036, 264, 20, 5, SWIGLU, "64x128"),
+    (128, 256, 72, 0, NONE, "64x64"), (256, 16, 65, 0, NONE, "64x64"), (100, 128, 40, 0, SWIGLU, "64x128"), (5504, 768, 20, 0, NONE, "64x128"), (2048, 2048, 20, 0, NONE, "128x128")])
+def test_f32_rows_of_every_tile(hip, m, n, k, groups, act, tile):
     gpu, rows, mats = Gpu(hip), n if act == NONE else 2 * n, max(1, groups)
     gen = np.random.default_rng(6)
     x, w = gen.standard_normal((m, k)).astype(np.float32), (gen.standard_normal((mats, rows, k)) / np.sqrt(k)).astype(np.float32)
@@ -369,6 +371,7 @@ def test_f32_rows_of_every_tile(hip, m, n, k, groups, act):
     dx, dw, dst = gpu.up(x), gpu.up(w), gpu.out(m * n + 8)
     print("f32 rows", m, n, k, groups, act, flush=True)
     gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=F32, act=act, **kw)))
+    assert ug_amd.last_kernel() == f"rows_product<f32,{'swiglu' if act == SWIGLU else 'none'}{',grouped' if groups else ''},{tile}>"
     out = get(dst, m * n + 8)
     assert np.all(np.isnan(out[m * n :])), "wrote past the end"
     close(out[: m * n].reshape(m, n), y, 1e-5)  # k eps and the gate's few units, against sums of some standard deviations

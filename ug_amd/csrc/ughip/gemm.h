@@ -101,7 +101,6 @@ struct DmaRows {
 };
 enum class RowsAct { NONE, GLU, LOOKUP };
 bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int tile);
-double grouped_tile_rows(int m, int groups, int bm);  // how many tiles of bm rows m rows by group are expected to be, a group's share being what a router makes it
 int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act);  // a tile code, 0: no tile takes it
 hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRows& r, RowsAct act, int tile);
 

@@ -33,6 +33,7 @@
 #include "bf16_split.h"
 #include "gemm_dma.h"
 #include "internal.h"
+#include "rows_prices.h"
 #include "ughip.h"
 
 namespace ughip {
@@ -812,15 +813,6 @@ bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int
   if (x_rows * p.a_rs * 2 >= (1ull << 31) || (unsigned long long)p.b_cs * 2 * (act == RowsAct::GLU ? p.N : bn) >= (1ull << 31)) return false;
   if (!aligned16(p.a) || !aligned16(p.b) || !aligned16(r.dst) || (r.bias && !aligned16(r.bias))) return false;
   return ((size_t)(p.M + bm - 1) / bm + r.groups) * (size_t)((p.N + bn - 1) / bn) < (1u << 24);
-}
-
-// How rows by group are spread is not known where a product is planned: eighths of the groups have these shares of an even one's rows, as the shares of a router's experts come out that differ by 40 %.
-static const double SHARE[8] = {0.50, 0.65, 0.76, 0.87, 0.98, 1.12, 1.32, 1.70};
-static int share_rows(int m, int groups, double share) { return std::max(1, (int)((double)m / groups * share + 0.999)); }
-double grouped_tile_rows(int m, int groups, int bm) {
-  double n = 0;
-  for (double share : SHARE) n += groups / 8.0 * ((share_rows(m, groups, share) + bm - 1) / bm);
-  return n;
 }
 
 // What rows by group take, spread as SHARE says (taken as even, groups of 127 rows went to 192 x 192 tiles, of which one in eight is then two: 85 us where 59 are possible).  Every K tile brings a

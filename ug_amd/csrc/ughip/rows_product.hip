@@ -9,11 +9,10 @@
 // F32, four v_mfma_f32_32x32x2_f32 per chunk (k taken chunk by chunk: lanes 0-31 the even, lanes 32-63 the odd one).
 #include <hip/hip_runtime.h>
 
-#include <cmath>
-
 #include "bf16_split.h"
 #include "gemm.h"
 #include "layers.h"
+#include "rows_prices.h"
 
 using namespace ughip;
 
@@ -304,29 +303,11 @@ hipError_t launch_tile(hipStream_t st, const ProductArgs& a, bool vec) {
   return hipGetLastError();
 }
 
-// f32: which of 128 x 128, 64 x 128 and 64 x 64 (22, 12, 11).  An f32 MFMA has its SIMD to itself, so a second tile on a CU takes as long again: a product lasts for as many rounds of 256 tiles
-// as it has, whole ones, at what a tile takes by itself (us per 2048 of K), and the larger tile's better rate is often less than the smaller one's fuller last round.  us on 22 / 12 / 11: gated
-// n 5632, k 2048, 100 rows 152 / 91, 300 rows 285 / 172, 509 296 / 258, 700 430 / 336, 1024 448 / 486; n 10304, k 2048, 509 rows 296 / 254 / 266; n 6592, 700 rows 290 / 246 / 231; n 2048,
-// 1531 rows 163 / 164 / 148; gated n 2816, k 1024, 300 rows 84 / 51, 700 151 / 91; 16 groups, gated n 1408, 1200 rows 296 / 251, 2036 rows 318 / 334.
-int f32_tile(const ProductArgs& a, bool gated) {
-  int best = 0;
-  double best_us = 0;
-  for (int tile : {22, 12, 11}) {
-    if (gated && tile == 11) continue;  // a tile's columns come in gate / up pairs
-    const int bm = tile == 22 ? 128 : 64, cols = (tile == 11 ? 64 : 128) / (gated ? 2 : 1);
-    // (by group a few tiles more than expected may be a round: 1200 rows on 128 x 128, n 2048 of k 1408, 201 us where 16 tile rows would be 108, 64 x 128 124)
-    const double rows = a.groups > 1 ? 1.06 * grouped_tile_rows(a.m, a.groups, bm) : (a.m + bm - 1) / bm, tiles = rows * ((a.n + cols - 1) / cols);
-    const double us = 4.0 + std::ceil(tiles / 256 - 0.01) * a.k / 2048.0 * (tile == 22 ? 144.0 : tile == 12 ? 81.0 : 45.5);
-    if (!best || us < best_us * 0.97) best = tile, best_us = us;
-  }
-  return best;
-}
-
 template <typename CT, typename XT, typename WT, int ACT>
 hipError_t launch_act(hipStream_t st, const ProductArgs& a, bool vec) {
   constexpr bool GATED = ACT == UGHIP_ACT_SWIGLU;
   if constexpr (sizeof(CT) == 4 && ACT != UGHIP_ACT_GELU_MUL) {
-    const int tile = f32_tile(a, GATED);
+    const int tile = f32_rows_tile(a.m, a.n, a.k, a.groups, GATED);
     if (tile == 22) return launch_tile<CT, XT, WT, 2, 2, ACT>(st, a, vec);
     if constexpr (!GATED)
       if (tile == 11) return launch_tile<CT, XT, WT, 1, 1, ACT>(st, a, vec);
@@ -452,6 +433,9 @@ extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
   else if (p->act == UGHIP_ACT_NONE) e = launch_act<__bf16, float, float, UGHIP_ACT_NONE>(dev->stream, a, vec);
   else return set_error(UGHIP_ERR_UNSUPPORTED, "%s: bf16 products with an activation take a BF16 matrix", what);
   UGHIP_HIPCHK(e);
-  note_kernel("rows_product<%s,%s%s>", f32 ? "f32" : "bf16", p->act == UGHIP_ACT_SWIGLU ? "swiglu" : p->act == UGHIP_ACT_GLU ? "glu" : p->act == UGHIP_ACT_GELU_MUL ? "gelu_mul" : "none", p->groups ? ",grouped" : "");
+  static const char* const tiles[] = {"", ",128x128", ",64x128", ",64x64"};
+  const int tile = f32 && act != UGHIP_ACT_GELU_MUL ? f32_rows_tile(a.m, a.n, a.k, a.groups, glu) : 0;
+  note_kernel("rows_product<%s,%s%s%s>", f32 ? "f32" : "bf16", p->act == UGHIP_ACT_SWIGLU ? "swiglu" : p->act == UGHIP_ACT_GLU ? "glu" : p->act == UGHIP_ACT_GELU_MUL ? "gelu_mul" : "none", p->groups ? ",grouped" : "",
+              tiles[tile == 22 ? 1 : tile == 12 ? 2 : tile == 11 ? 3 : 0]);
   return UGHIP_OK;
 }
