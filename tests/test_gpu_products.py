@@ -377,6 +377,16 @@ def test_f32_rows_of_every_tile(hip, m, n, k, groups, act, tile):
     close(out[: m * n].reshape(m, n), y, 1e-5)  # k eps and the gate's few units, against sums of some standard deviations
 
 
+def test_f32_rows_of_more_tile_rows_than_a_grid_has(hip):
+    """64-row tiles would be more than the 65535 that a grid's second dimension takes."""
+    gpu, m, n, k = Gpu(hip), 65535 * 64 + 1, 8, 8
+    gen = np.random.default_rng(3)
+    x, w = gen.standard_normal((m, k), np.float32), gen.standard_normal((n, k), np.float32)
+    dx, dw, dst = gpu.up(x), gpu.up(w), hip.allocate_uninit(ug_amd.F32, m * n)
+    gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=F32, act=NONE)))
+    np.testing.assert_allclose(dst.to_vec().reshape(m, n), x @ w.T, rtol=0, atol=2e-5)  # 8 products of normal deviates in f32 on either side
+
+
 # Rows leave in 16-byte pieces through LDS where a bf16 row starts on one, else fragment by fragment: the same bits either way, edges of tiles and of pieces, nothing behind a row touched.
 @pytest.mark.parametrize("shape", ["3", "10", "11", "12", "13", "9", "17"])
 @pytest.mark.parametrize("m, n, act", [(300, 200, NONE), (257, 392, NONE), (16, 520, NONE), (271, 136, SWIGLU), (97, 200, SWIGLU)])

@@ -14,6 +14,8 @@ TILES = {
     (64, 64, 2048, 0, 1): 12,
     # one tile past a round is a second one
     (5504, 768, 2048, 0, 0): 11, (5504, 384, 2048, 0, 1): 12,
+    # more tile rows than a grid has: the tile that has fewer, up to as many as that one has
+    (65535 * 64, 8, 8, 0, 0): 11, (65535 * 64 + 1, 8, 8, 0, 0): 22, (5000000, 8, 8, 0, 0): 22, (65535 * 128, 8, 8, 0, 0): 22, (5000000, 8, 8, 0, 1): 22, (65535 * 64 - 64, 8, 8, 1, 0): 11, (65535 * 64 - 63, 8, 8, 1, 0): 22,
     # as measured: the fuller last round
     (509, 5632, 2048, 0, 1): 12, (1024, 5632, 2048, 0, 1): 22, (509, 10304, 2048, 0, 0): 12, (700, 6592, 2048, 0, 0): 11, (1531, 2048, 2048, 0, 0): 11, (2036, 1408, 2048, 16, 1): 22,
     (1200, 1408, 2048, 16, 1): 12,

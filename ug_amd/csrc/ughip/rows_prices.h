@@ -25,6 +25,7 @@ inline int f32_rows_tile(int m, int n, int k, int groups, bool gated) {
   for (int tile : {22, 12, 11}) {
     if (gated && tile == 11) continue;  // a tile's columns come in gate / up pairs
     const int bm = tile == 22 ? 128 : 64, cols = (tile == 11 ? 64 : 128) / (gated ? 2 : 1);
+    if (best && (m + bm - 1) / bm + groups > 65535) continue;  // tile rows are a grid's second dimension
     // (by group a few tiles more than expected may be a round: 1200 rows on 128 x 128, n 2048 of k 1408, 201 us where 16 tile rows would be 108, 64 x 128 124)
     const double rows = groups > 1 ? 1.06 * grouped_tile_rows(m, groups, bm) : (m + bm - 1) / bm, tiles = rows * ((n + cols - 1) / cols);
     const double rounds = std::max(1.0, std::ceil(tiles / 256 - (groups > 1 ? 0.01 : 0.0)));
