@@ -16,7 +16,11 @@ def test_wide_tile(hip, tune, t, k, n, split):
 
 # gate and up columns of a tile gated in registers: 96 columns one short, exact and a bit; as planes, bit for bit what the f32 rows give
 @pytest.mark.parametrize("t,k,inter,n", [(513, 128, 192, 64), (511, 192, 64, 72), (512, 128, 128, 64), (400, 256, 1088, 136), (385, 128, 320, 64), (449, 448, 448, 64)])
-def test_wide_tile_gated(hip, tune, t, k, inter, n):
+def test_wide_tile_gated(hip, tune, monkeypatch, t, k, inter, n):
+    names, last = [], ug_amd.last_kernel
+    monkeypatch.setattr(ug_amd, "last_kernel", lambda: names.append(last()) or names[-1])
     tune.setenv("UGHIP_X3_DMA", "14")
     tune.setenv("UGHIP_X3_SPLIT", "1")
     parity.test_norm_and_mlp_folded_into_the_products_of_rows(hip, t, k, inter, n, 1, True)
+    tile = "gemm_dma4<bf16,NT,256x192,256t,3 planes,f32 out,in-register swiglu fold"
+    assert tile + ">" in names and any(tile + " onto planes> -> " in name for name in names), names
