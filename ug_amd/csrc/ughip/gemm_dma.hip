@@ -730,7 +730,8 @@ bool gemm_dma_planes3_split_ok(const MMArgs& p, int nsplit) {
 // 256 x 192 compared at a second price, they were 3.3 %.  us then -> now: 600 x 2 of 2816 x 1024 40.6 -> 33.0, 900 x 4096 x 4096 101 -> 85, 1650 x 1024 x 2816 45.2 -> 40.0, 450 x 2560 x 2048 32.6 -> 29.1, 509 x 2048 x 5632
 // 47.9 -> 45.3; llama's products of 1024 rows and more keep their tiles or gain up to a tenth.
 // The ring past one round: where a CU holds several workgroups their ends spread, and a little more than a round takes a quarter longer, not twice as long (1900 x 2560 x 2048, 600 tiles of 64 x 128: 65 us, 70 in two parts on 256 x 192);
-// below 48 K tiles such products keep the plans that callers hold them to (640 x 7600 x 640 31.5 us on 128 x 128, 27.9 so; 964 x 4928 x 256 19.6, 17.2).
+// below 48 K tiles that holds up to a round and a half: of 379 products of k 128 .. 960 that are priced so, the 301 within it take 0.95 to 1.8 times as long on the tiles priced next (1.12 in the mean; 640 x 7600 x 640 27.3 us, 29.1 on 128 x 128; 964 x
+// 4928 x 256 16.8 and 18.1; 1650 x 2472 x 512 23.1 and 34.6 on the register-staged kernel), those of more rounds 0.88 to 1.15 times (3107 x 5608 x 896 101.8 us, 89.8 on 128 x 128).
 double gemm_dma_planes3_cost_us(const MMArgs& p, int tile, int nsplit, bool gated) {
   static const struct Price {
     int tile, per_cu;
@@ -752,7 +753,7 @@ double gemm_dma_planes3_cost_us(const MMArgs& p, int tile, int nsplit, bool gate
     double us = c.fixed + (double)p.M * p.N * 4 / 6.4e6 * (gated ? 0.25 : nsplit), rounds = (double)(tiles / round);
     size_t last = tiles % round;
     if (ring_tile(tile) && tiles > round) {
-      if (c.per_cu == 1 || nsplit > 1 || kt < 48) return -1.0;
+      if (c.per_cu == 1 || nsplit > 1 || (kt < 48 && 2 * tiles > 3 * round)) return -1.0;
       rounds = std::max(1.25, (double)tiles / round), last = 0;
     }
     for (int j = 0; j < c.per_cu; ++j) {
