@@ -212,6 +212,19 @@ def test_tiles_as_high_as_their_groups(hip, tune, n, k, act):
     np.testing.assert_array_equal(got["256x128"], got["64x64"])
 
 
+# (groups, rows of one in the mean, n, k, act): us on the tile named and on the one that prices fitted to 16 groups of two matrices took, or that took them before
+@pytest.mark.parametrize("groups, per, n, k, act, tile", [(8, 1900, 8192, 4096, NONE, "256x256"),  # 820 .. 1016 / 1228 on 256 x 192
+                                                          (4, 1000, 1408, 2048, SWIGLU, "256x256"),  # 53 / 78 on 256 x 192
+                                                          (16, 260, 1408, 2048, SWIGLU, "192x192"),  # 72 / 57 .. 107 on 256 x 256, one round or two
+                                                          (16, 127, 1408, 2048, SWIGLU, "256x192")])  # 59 / 84 on 192 x 192
+def test_groups_take_the_tile_priced_lowest(hip, groups, per, n, k, act, tile):
+    gpu, m, rows = Gpu(hip), groups * per, n if act == NONE else 2 * n
+    dx, dw, dst = hip.allocate_uninit(ug_amd.BF16, m * k), hip.allocate_uninit(ug_amd.BF16, groups * rows * k), hip.allocate_uninit(ug_amd.BF16, m * n)
+    src, end = gpu.up(np.arange(m, dtype=np.int32)), gpu.up(np.arange(1, groups + 1, dtype=np.int32) * per)
+    gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=BF16, act=act, row_index=src.raw(), group_end=end.raw(), groups=groups, x_rows=m)))
+    assert f"NT,{tile}," in ug_amd.last_kernel(), ug_amd.last_kernel()
+
+
 @pytest.mark.parametrize("shape, kernel", [("3", "gemm_dma4<bf16,NT,256x256,256t,rows>"), ("4", "gemm_dma4<bf16,NT,256x128,512t,ring,rows>"), ("5", "gemm_dma4<bf16,NT,128x128,512t,ring,rows>"),
                                            ("0", "rows_product<bf16,none>"), ("6", "rows_product<bf16,none>"), ("7", "rows_product<bf16,none>")])
 def test_forced_tiles_of_rows(hip, tune, shape, kernel):

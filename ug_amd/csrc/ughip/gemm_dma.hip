@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <type_traits>
@@ -819,35 +820,51 @@ bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int
   return ((size_t)(p.M + bm - 1) / bm + r.groups) * (size_t)((p.N + bn - 1) / bn) < (1u << 24);
 }
 
-// What rows by group take, spread as SHARE says (taken as even, groups of 127 rows went to 192 x 192 tiles, of which one in eight is then two: 85 us where 59 are possible).  Every K tile brings a
-// matrix's columns from memory that at most a few workgroups share, 1.8 times the time that one matrix's tiles take.  Tiles by height (193, 130): a K tile by the
-// height in 64s; one round lasts for its highest tiles mostly, several go by the mean and leave one of the highest behind.
-// Fitted to 48 products of 16 groups (n 2 x 1408 and k 2048, n 2048 and k 1408, half of both; 512 to 8192 rows) on each of eight tiles: the choice is within 0.2 % of the best in the
-// mean, 5 % at most.  Gate and up, then down, of width 2048, us before and so: 768 rows 50.6 / 33.3 -> 47 / 25; 1280 50.6 / 47 -> 50 / 28; 1600 51 / 46 -> 51 / 30; 2036 84 / 37 -> 59 / 35;
-// 2560 67 / 59 -> 67 / 41; 3200 67 / 61 -> 67 / 47; 4096 80 / 55 -> 70 / 48; 8192 124 / 90 -> 124 / 83; of width 1024, 5200 rows 47 / 27 -> 36 / 27.
-static double grouped_cost_us(const MMArgs& p, int groups, int tile) {
-  static const double WIDE[4] = {1.0, 1.2, 1.5, 1.7}, NARROW[4] = {0.6, 0.83, 1.2, 1.3};  // us per K tile, 192 and 128 columns
+// What rows by group take, spread as SHARES says (taken as even, groups of 127 rows went to 192 x 192 tiles, of which one in eight is then two: 85 us where 59 are possible): a fixed part and, for every round of
+// 256 tiles, their K tiles, at a time that grows with the share of the chip that is busy; of a last round that is not full `tail` of the rest counts.  Tiles by height (193, 130): a K tile by the height in
+// 64s; one round lasts for its highest tiles mostly, several go by the mean and leave `last` of one of the highest behind.  Whether tiles near 256 are one round or two is seen by the router's rows alone: in between.
+// Fitted to 2000 products on each of the eight tiles (2 to 128 groups of 4 to 2048 rows, 18 matrices from 512 x 512 to 8192 x 4096, shares of the rows that differ by 20, 40 and 60 %, up to six draws of them): the choice is
+// 1.2 % from the fastest in the mean, 0.4 % for 16 groups of the decoders' matrices.  Prices fitted to those 16 groups alone, with every column of a matrix from memory once per tile, were 4.6 % and 2.8 % from it, and a tenth or
+// more slower than the best of the tiles of one height for 92 of the products, 14 so: 8 groups of 2048 rows, n 8192, k 4096 1295 us on 256 x 192 by height, 886 on 256 x 256; 32 of 800 rows 2200 and 1574; 8 of 200, n 2 x 4096, k 1024 54.7 and 37.8.
+struct GroupedRows {
+  double tiles[4] = {}, heights[4] = {};  // tile rows of 64, 128, 192 and 256 rows; those of up to 256 by their height in 64s
+  GroupedRows(int m, int groups) {
+    for (double share : SHARES) {
+      const int rows = share_rows(m, groups, share), n = (rows + 255) / 256;
+      tiles[0] += (rows + 63) / 64, tiles[1] += (rows + 127) / 128, tiles[2] += (rows + 191) / 192, tiles[3] += n;
+      heights[std::min(4, (((rows + n - 1) / n + 15) / 16 * 16 + 63) / 64) - 1] += n;
+    }
+    for (double* counts : {tiles, heights})
+      for (int i = 0; i < 4; ++i) counts[i] *= groups / 16.0;
+  }
+};
+static double grouped_cost_us(const MMArgs& p, const GroupedRows& rows, int tile) {
+  static const struct {
+    int tile;
+    double fixed, first, busy, tail;
+  } prices[] = {{256, 6.25, 1.214, 0.612, 0.78}, {129, 3.93, 1.055, 0.151, 0.4}, {97, 3.0, 1.013, 0.228, 0.645}, {65, 2.02, 0.429, 0.508, 0.78}, {48, 2.48, 0.339, 0.304, 1.0}, {32, 3.04, 0.047, 0.332, 0.285}};
+  static const struct {
+    double fixed, height[4], last;
+  } by_heights[] = {{2.63, {0.656, 0.839, 1.157, 1.612}, 0.70}, {2.99, {0.456, 0.636, 0.917, 1.087}, 0.61}};
+  constexpr double NEAR = 0.055;
   int bm, bn;
   tile_dims(tile, &bm, &bn);
-  const double columns = (p.N + bn - 1) / bn, kt = p.K / BK;
-  double tiles = 0, sum = 0, highest = 0;
-  for (double share : SHARE) {
-    const int rows = share_rows(p.M, groups, share), n = (rows + bm - 1) / bm;
-    const double count = groups / 8.0 * n * columns;
-    tiles += count;
-    if (!by_height(tile)) continue;
-    const int height = std::min(4, (((rows + n - 1) / n + 15) / 16 * 16 + 63) / 64);
-    const double us = (tile == 193 ? WIDE : NARROW)[height - 1];
-    sum += count * us, highest = std::max(highest, us);
+  const double columns = (p.N + bn - 1) / bn, kt = p.K / BK, tiles = rows.tiles[bm / 64 - 1] * columns, rounds = tiles / 256;
+  const double two = std::min(1.0, std::max(0.0, (rounds - (1 - NEAR)) / (2 * NEAR)));  // of one round and more
+  if (by_height(tile)) {
+    const auto& high = by_heights[tile == 193 ? 0 : 1];
+    double sum = 0, highest = 0;
+    for (int h = 0; h < 4; ++h)
+      if (rows.heights[h] > 0) sum += rows.heights[h] * columns * high.height[h], highest = high.height[h];
+    const double one = 0.89 * highest + 0.11 * sum / tiles, more = std::max(sum / 256 + high.last * highest, rounds < 1 + NEAR ? one : 0.0);
+    return high.fixed + kt * (one + (more - one) * two);
   }
-  if (by_height(tile)) return 5.0 + kt * (tiles <= 256 ? 0.8 * highest + 0.2 * sum / tiles : sum / 256 + 0.77 * highest);
-  if (tile == 256) {
-    double us = 6.0;
-    for (double left = tiles; left > 0; left -= 256) us += 1.66 * kt * (1.23 + 0.33 * std::min(left, 256.0) / 256.0);
-    return us;
-  }
-  const double fixed = ring_cost_us(0, (int)kt, tile, Operands::MEMORY);
-  return fixed + 1.8 * (ring_cost_us((size_t)(tiles + 0.5), (int)kt, tile, Operands::MEMORY) - fixed);
+  for (const auto& c : prices)
+    if (c.tile == tile) {
+      const double past = std::max(rounds, 1.001), more = past + c.tail * (std::ceil(past - 1e-9) - past);
+      return c.fixed + kt * (c.first + c.busy * std::min(1.0, rounds)) * (1 + (more - 1) * two);
+    }
+  return 1e30;
 }
 
 int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
@@ -861,10 +878,10 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
   int best = 0;
   double best_us = 0;
   if (r.groups > 1) {
+    const GroupedRows rows(p.M, r.groups);
     for (int tile : {256, 129, 65, 48, 32, 97, 193, 130}) {
       if (!gemm_dma_rows_supported(p, r, act, tile)) continue;
-      if (by_height(tile) && share_rows(p.M, r.groups, SHARE[7]) <= 64) continue;  // nothing to choose: the lowest tiles leave a CU several workgroups (216 rows 43.3, 44.0 by height)
-      const double us = grouped_cost_us(p, r.groups, tile);
+      const double us = grouped_cost_us(p, rows, tile);
       if (!best || us < best_us) best = tile, best_us = us;
     }
     return best;

@@ -5,13 +5,13 @@
 
 namespace ughip {
 
-// How rows by group are spread is not known where a product is planned: eighths of the groups have these shares of an even one's rows, as the shares of a router's experts come out that differ by 40 %.
-constexpr double SHARE[8] = {0.50, 0.65, 0.76, 0.87, 0.98, 1.12, 1.32, 1.70};
+// How rows by group are spread is not known where a product is planned: a router's experts come out with shares that differ by 40 % or so, the share of an even one's rows times one of these for a sixteenth of the groups each.
+constexpr double SHARES[16] = {.44, .55, .62, .68, .73, .79, .84, .90, .95, 1.02, 1.08, 1.16, 1.26, 1.38, 1.56, 1.94};
 inline int share_rows(int m, int groups, double share) { return std::max(1, (int)((double)m / groups * share + 0.999)); }
-// how many tiles of bm rows m rows by group are expected to be
+// how many tiles of bm rows m rows by group are expected to be, as the f32 prices below were fitted to it: by eighths
 inline double grouped_tile_rows(int m, int groups, int bm) {
   double n = 0;
-  for (double share : SHARE) n += groups / 8.0 * ((share_rows(m, groups, share) + bm - 1) / bm);
+  for (double share : {0.50, 0.65, 0.76, 0.87, 0.98, 1.12, 1.32, 1.70}) n += groups / 8.0 * ((share_rows(m, groups, share) + bm - 1) / bm);
   return n;
 }
 
