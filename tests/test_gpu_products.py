@@ -362,6 +362,35 @@ def test_smallest_ring_tile_gives_the_next_ones_bits(hip, tune, m, n, k, form):
     np.testing.assert_array_equal(got["64x64,512t"], got["32x32,256t"])
 
 
+@pytest.mark.parametrize("m, n, k", [(300, 264, 128), (257, 128, 64), (17, 392, 192)])
+@pytest.mark.parametrize("half", [False, True])
+def test_lookups_on_every_tile_of_the_ring(hip, tune, m, n, k, half):
+    """gelu(y) times the token's row of an f32 or a bf16 table, ids outside of it among them: the same bits on every tile, values against 64 bits."""
+    gpu, gen = Gpu(hip), np.random.default_rng(9)
+    x, w, bias, table, ids = rand(1, m, k), rand(2, n, k, std=k ** -0.5), rand(3, n), rand(4, 50, n + 3), gen.integers(0, 50, m)
+    ids[::7] = 50
+    ids[3::11] = -1
+    keep = [gpu.up(x, bf16=True), gpu.up(w, bf16=True), gpu.up(bias), gpu.up(table, bf16=half), gpu.up(ids.astype(np.int32))]
+    got = {}
+    for shape, tile in (("10", "256x128"), ("12", "128x128"), ("13", "64x128"), ("9", "64x64"), ("17", "32x32")):
+        tune.setenv("UGHIP_GEMM_SHAPE", shape)
+        dst = gpu.out(m * n + 8)
+        print("lookup", m, n, k, half, tile, flush=True)
+        gpu.call("ughip_product_rows", C.byref(Product(x=view(keep[0], 0, k), dst=view(dst, 0, n), w=keep[1].raw(), bias=keep[2].raw(), m=m, n=n, k=k, product=BF16, act=GELU_MUL, table=keep[3].raw(),
+                                                       ids=keep[4].raw(), table_rows=50, table_stride=n + 3, table_col=2)))
+        assert f"NT,{tile}," in ug_amd.last_kernel() and "ring,rows" in ug_amd.last_kernel()
+        out = get(dst, m * n + 8)
+        assert np.all(np.isnan(out[m * n :]))
+        got[tile] = out[: m * n].reshape(m, n)
+    known = (ids >= 0) & (ids < 50)
+    y = x @ w.T + bias
+    want = 0.5 * y * (1 + np.tanh(np.sqrt(2 / np.pi) * (y + 0.044715 * y ** 3))) * table[np.where(known, ids, 0), 2 : 2 + n]
+    for out in got.values():
+        np.testing.assert_array_equal(out, got["64x64"])
+    assert np.all(np.isnan(got["64x64"][~known]))
+    close(got["64x64"][known], want[known], 2e-5)
+
+
 # f32 rows on 128 x 128, 64 x 128 and 64 x 64 tiles as the rounds of 256 have it, a few tiles and one past a round too; K of a step less and a step more, gated and plain, even and uneven groups
 @pytest.mark.parametrize("m, n, k, groups, act, tile", [
     (70, 2050, 33, 0, SWIGLU, "64x128"), (129, 1040, 64, 0, SWIGLU, "64x128"), (300, 5632, 40, 0, SWIGLU, "64x128"), (513, 6592, 36, 0, NONE, "64x128"), (700, 6592, 31, 0, NONE, "64x64"),

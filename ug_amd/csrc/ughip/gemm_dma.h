@@ -164,15 +164,29 @@ __device__ __forceinline__ void rows_out(floatx4 (&acc)[NI][NJ], const DmaRows& 
       const int id = rw.ids[m0 + min(row0 + i * 16, m_last)];
       const bool known = id >= 0 && id < rw.table_rows;
       const size_t at = (size_t)(known ? id : 0) * rw.table_stride + rw.table_col;
+      // 16 rows' table elements at a time (all of them at once are more than the registers hold), the table's type asked for once: asked for each, every load was waited for by itself and the gates stayed, in
+      // part in scratch memory, until the last of them
+      float f[NJ][4];
+      auto load = [&](auto* table) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const auto v = table[at + min(col0 + j * 16, rw.n_out - 4) + e];
+            if constexpr (sizeof(v) == 2) f[j][e] = bf16_to_f32(v);
+            else f[j][e] = v;
+          }
+      };
+      if (rw.table_bf16) load(static_cast<const uint16_t*>(rw.table));
+      else load(static_cast<const float*>(rw.table));
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const size_t k = at + min(col0 + j * 16, rw.n_out - 4) + e;
-          const float f = rw.table_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(rw.table)[k]) : static_cast<const float*>(rw.table)[k];
-          acc[i][j][e] = gelu_tanh_f(acc[i][j][e] + b[j][e]) * (known ? f : __uint_as_float(0x7fc00000u));
+          acc[i][j][e] = gelu_tanh_f(acc[i][j][e] + b[j][e]) * (known ? f[j][e] : __uint_as_float(0x7fc00000u));
+          asm volatile("" : "+v"(acc[i][j][e]));
         }
-      asm volatile("" ::: "memory");  // (16 rows' table elements at a time: all of them at once are more than the registers hold)
+      asm volatile("" ::: "memory");
     }
   }
   auto value = [&](int i, int j) {
