@@ -430,11 +430,10 @@ def test_f32_rows_of_more_tile_rows_than_a_grid_has(hip):
 
 
 # Rows leave in 16-byte pieces through LDS where a bf16 row starts on one, else fragment by fragment: the same bits either way, edges of tiles and of pieces, nothing behind a row touched.
-@pytest.mark.parametrize("shape", ["3", "10", "11", "12", "13", "9", "17"])
-@pytest.mark.parametrize("m, n, act", [(300, 200, NONE), (257, 392, NONE), (16, 520, NONE), (271, 136, SWIGLU), (97, 200, SWIGLU)])
+# (17, 32 x 32 tiles: plain rows alone)
+@pytest.mark.parametrize("shape, m, n, act", [(shape, *size) for size in [(300, 200, NONE), (257, 392, NONE), (16, 520, NONE), (271, 136, SWIGLU), (97, 200, SWIGLU)]
+                                              for shape in ["3", "10", "11", "12", "13", "9"] + ["17"] * (size[2] == NONE)])
 def test_rows_leave_in_pieces_with_the_same_bits(hip, tune, shape, m, n, act):
-    if shape == "17" and act == SWIGLU:
-        pytest.skip("32 x 32 tiles are for plain rows")
     gpu, k, rows = Gpu(hip), 512, 2 * n if act == SWIGLU else n
     dx, dw, bias = gpu.up(rand(1, m, k), bf16=True), gpu.up(rand(2, rows, k, std=k ** -0.5), bf16=True), gpu.up(rand(3, rows))
     tune.setenv("UGHIP_GEMM_SHAPE", shape)

@@ -46,14 +46,14 @@ double gemm_tiled_cost_us(int dtype, const MMArgs& p, size_t batch);
 
 // 16-bit types, one wave per SIMD: 256 x 256, 256 x 192 (three planes only), 256 x 128 or 128 x 128 tiles (tile codes 256, 192, 128, 64), 4 waves laid out
 // 2 x 2 with the accumulators in the accumulation registers, loads that write LDS directly, rhs [n, k]- or [k, n]-major
-// (gemm_dma.hip), and a ring of four or three stages under eight waves with 256 x 128, 128 x 128, 64 x 128 and 64 x 64 tiles, 192 x 192 for rows (codes 129,
-// 65, 48, 32, 97; gemm_ring.hip).  Any M, N % 8 == 0, K % 64 == 0 (gemm_dma4: K >= 256), 16-byte aligned rows, contiguous [batch, M, N] result.
+// (gemm_dma.hip), and a ring of stages under eight waves with 256 x 128, 128 x 128, 64 x 128 and 64 x 64 tiles (codes 129, 65, 48, 32; gemm_ring.hip), for rows
+// also 192 x 192, 32 x 32 and, by group, tiles by height with 192 and 128 columns (97, 16, 193, 130).  Any M, N % 8 == 0, K % 64 == 0 (gemm_dma4: K >= 256), 16-byte aligned rows, contiguous [batch, M, N] result.
 bool gemm_dma_supported(int dtype, const MMArgs& p, size_t batch, int tile);
 hipError_t gemm_dma_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, int tile);
 // The tile code this kernel should take the problem with, 0 when another kernel should.
 int gemm_dma_pick(int dtype, const MMArgs& p, size_t batch);
 // The same kernel on three bf16 planes of f32 rows (p.K = 3 k, p.b_k_div = 3, [n, k]-major bf16 matrix), f32 result.
-// nsplit == 1: p.c [M, N] is written straight from the accumulators, residual [M, N] added when given.  nsplit > 1 (it
+// nsplit == 1: p.c [M, N] is written, residual [M, N] added when given.  nsplit > 1 (it
 // divides the K tiles, into a multiple of 3 and at least 4 each): workgroups share a tile's K range and leave nsplit
 // slabs [M, N] in p.c (scratch), for gemm_fold_f32 to add up.
 // gated, where _gates says that the tile can: the matrix is gate rows, then up rows, and silu(gate) * up goes to p.c [M, N / 2], or with

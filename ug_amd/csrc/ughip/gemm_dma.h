@@ -298,7 +298,7 @@ __device__ __forceinline__ void sums_out(floatx4 (&acc)[NI][NJ], float* __restri
   }
 }
 
-// gemm_ring.hip: one of its tiles (codes 129, 97, 65, 48, 32: 256 x 128, 192 x 192, 128 x 128, 64 x 128, 64 x 64), operands as the _supported functions of gemm_dma.hip check them.
+// gemm_ring.hip: one of its tiles (codes 129, 97, 65, 48, 32, 16: 256 x 128, 192 x 192, 128 x 128, 64 x 128, 64 x 64, 32 x 32; 193, 130: rows by group, tiles by height with 192 and 128 columns), operands as the _supported functions of gemm_dma.hip check them.
 hipError_t gemm_ring_launch(hipStream_t stream, int dtype, DmaForm form, const MMArgs& p, size_t batch, int tile, const float* residual, const DmaRows& rw);
 
 }  // namespace ughip

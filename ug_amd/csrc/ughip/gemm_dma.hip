@@ -67,9 +67,9 @@ __device__ __forceinline__ float silu_32(float z) {
 }
 
 // Lane l feeds row / column l % 16, k = 8 (l / 16) .. + 7 of a step of 32.  TWO: the schedule with two barriers per K tile.
-// F32OUT: the result leaves as f32 straight from the accumulators (+ residual when given) instead of as T through LDS.
+// F32OUT: the result leaves as f32 (+ residual when given) instead of as T, through LDS either way.
 // BDIV > 1 ([n, k]-major rhs): K tile t of the lhs meets K tile t / BDIV of the rhs -- an lhs that holds BDIV planes of every
-// 64 columns side by side (a row split into bf16 terms) against one matrix, whose tile then comes from cache for the other planes.
+// 64 columns side by side (a row split into bf16 terms) against one matrix, whose tile is loaded once for the three planes of one of the lhs (SHARED, below).
 // BDIV == 6 (either rhs layout): both operands hold three planes (hi, mid, lo: planes 0, 1, 2) of every 64 elements of k side
 // by side, and K tile t of the loop is term t % 6 of k tile t / 6 of an f32 product taken as six bf16 ones -- (hi, lo),
 // (lo, hi), (mid, mid), (hi, mid), (mid, hi), (hi, hi), the small ones first; (mid, lo), (lo, mid) and (lo, lo) stay below

@@ -5,8 +5,8 @@
 //   32 x 32, four waves and eight stages, for rows only: a CU has some 55 KB on its way whatever it is asked for, so where 64 x 64 tiles are few it is their bytes per CU that count (us on
 //   64 x 64 and so, weights from memory: 54 rows of 2048 x 2048 / 4096 / 5632 11.3 / 19.6 / 26.8 -> 6.7 / 10.6 / 14.1, 509 rows of 256 x 2048 8.9 -> 6.4, 228 of 2048 x 2048 11.3 -> 9.8).
 //   192 x 192 for rows only: 700 rows against 11264 x 2048 are 236 of them, one round (52 us with 256 x 256, 54 with 256 x 128, 34 so).
-//   A ring of four stages (three for the two largest tiles): the loads of a K tile go out (global_load_lds_dwordx4, as in gemm_dma4) when the tile that
-//   many in front of it has been read, so three (two) tiles are on their way while one is multiplied.  One barrier per K tile.
+//   A ring of four stages (three for 256 x 128, 192 x 192 and 192 columns of 128 rows, two for 256 x 192, eight for 32 x 32): the loads of a K tile go out (global_load_lds_dwordx4, as in gemm_dma4) when the tile
+//   that many in front of it has been read, so all but one of them are on their way while one is multiplied.  One barrier per K tile.
 //
 // What bounds it: the operands' way to a CU.  2048^2 x 5632 on 128 x 128 tiles, one to a CU, takes 42 us, 0.44 per K tile of 32 KB, with the operands in
 // the memory-side cache (matrix pipes busy 61 % of the time) and 54 us, 0.57, with both from HBM (42 %); gemm_dma4's two stages 58 and 75.  From HBM

@@ -847,7 +847,7 @@ struct RowsAround {
   float eps = 0.f;
   float* xn = nullptr;                  // ... into these m * k floats, unless the pass that writes the planes does it on its way
   const uint16_t* planes_in = nullptr;  // three-term product: the planes of x, already made (x is not read)
-  uint16_t* planes_out = nullptr;       // SwiGLU on a route that folds slabs: the result may go here as planes instead of to dst ...
+  uint16_t* planes_out = nullptr;       // SwiGLU on a route that folds slabs or gates in registers: the result may go here as planes instead of to dst ...
   bool wrote_planes = false;            // ... and this says whether it did
 };
 

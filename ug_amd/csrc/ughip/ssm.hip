@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_state_kernel(SsmArgs a) {
   float weight = 0.f;  // of row `lane` (first wave)
   auto fetch = [&](int i) {
     x.load(xbc0 + (size_t)hw.head(i) * a.vdim + hw.col(i), a.xbc_stride, rows, min(PB, a.vdim - hw.col(i)), PB / 4, xt);
-    if (wave == 0) {  // the head's d_i and A_i, for the launches behind this one too (q <= 64; a launch of 4.6 us by themselves)
+    if (wave == 0) {  // the head's d_i and A_i, for the launches behind this one too (q <= 64; a launch of 3.9 us by themselves)
       const int h = hw.head(i);
       float dv = 0.f;
       if (lane < q && lane < rows) dv = softplus_f(a.dt[(size_t)(row0 + lane) * a.dt_stride + h] + a.dt_bias[h]);
