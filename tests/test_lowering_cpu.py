@@ -455,7 +455,10 @@ def test_rows_plan_beside_the_256x192_tile():
                                        ((0, 1900, 2560, 2048), "64x128,512t,ring"),      # 600 tiles, past one round: 65 / 70 on 256 x 192 in two
                                        ((2, 428, 1768, 640), "64x128,512t,ring"),        # 17.4 / 24.0 on gemm_tiled
                                        ((0, 2048, 2560, 2048), "64x128,512t,ring"),      # 640 tiles
+                                       ((0, 1026, 3712, 128), "64x128,512t,ring"),       # 12.5 / 24.4 on gemm_tiled, whose price had no fold
+                                       ((0, 475, 1464, 1472), "64x64,512t,ring"),        # 19.6 / 23.4 on 64 x 128
+                                       ((1, 1819, 328, 1856), "64x64,512t,ring"),        # 26.4 / 31.3 on 64 x 128
                                        ((2, 384, 5632, 2048), "256x192,256t")])          # 67 / 74 on 64 x 128 in two parts of which each is past a round
 def test_three_planes_take_the_tile_priced_lowest(key, tile):
-    """Each us: the kernel named and the one that the prices of single planes named."""
+    """Each us: the kernel named and one that other prices named."""
     assert _rows_plan(ug_amd.BF16, 1, *key).startswith(f"gemm_dma4<bf16,NT,{tile},3 planes"), _rows_plan(ug_amd.BF16, 1, *key)

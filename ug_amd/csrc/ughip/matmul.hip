@@ -824,13 +824,15 @@ static RowsRoute rows_route(const MMArgs& p, int dtype, bool x3, GemmEpilogue::K
         double us = gemm_dma_planes3_cost_us(q, tile, split, gates);
         if (us < 0 && !forced_tile) continue;
         if (fold) us += 3.0 + (double)(split + 1) * m * rows * 4 / 6.4e6;  // the slabs in, the result out, a launch
-        // 64 x 64 tiles whose long K is not split leave most CUs without one, and the others wait longer for each K tile than the model says: 1011 x 280
-        // x 2112 31.7 us, 25.2 on gemm_tiled; 740 x 512 x 2368 33.5 and 29.0; 3954 x 96 x 2368 43.7 and 39.5
-        if (tile == 32 && split == 1 && q.K >= 4096) us += 0.07 * (q.K / 64);
+        // 64 x 64 tiles past a round wait longer for each K tile of a long K than the model says (1640 x 2560 x 2048 70.5 us, 63.9 on 64 x 128); within one they don't (475 x 1464 x 1472 19.6 and 23.4, 1819 x 328 x 1856 26.4 and 31.3)
+        if (tile == 32 && split == 1 && q.K >= 4096 && (m + 63) / 64 * ((rows + 63) / 64) > 768) us += 0.07 * (q.K / 64);
         if (!r.dma_tile || us < best) r.dma_tile = tile, r.dma_split = split, best = us;
       }
     double other = gemm_tiled_cost_us(dtype, p, 1);
-    if (kind == GemmEpilogue::SWIGLU && gemm_tiled_workspace_bytes(dtype, p, 1) == 0) other += 3.0 + 2.0 * m * rows * 4 / 6.4e6;  // its price of one part has no fold: 428 x 2 of 1768 x 640 24.0 us there, 17.4 on the ring
+    // few of them with a long K leave most CUs without one, where gemm_tiled splits it: 1011 x 280 x 2112 26.5 us, 24.8 there
+    if (r.dma_tile == 32 && r.dma_split == 1 && q.K >= 4096) best += 0.07 * (q.K / 64);
+    // Its price of one part has no fold, and there is one whatever `kind` is, the result being f32: 428 x 2 of 1768 x 640 24.0 us there, 17.4 on the ring; 1026 x 3712 x 128 24.4 and 12.5; 3564 x 4840 x 320 72 and 50 on 256 x 192
+    if (other >= 0 && gemm_tiled_workspace_bytes(dtype, p, 1) == 0) other += 3.0 + 2.0 * m * rows * 4 / 6.4e6;
     if (r.dma_tile && !forced_tile && other >= 0 && other < best * 1.05) r.dma_tile = 0, r.dma_split = 1;  // it has to be clearly cheaper: its model is the rougher one
   }
   if (r.dma_tile) r.kind = RowsRoute::DMA_PLANES;
