@@ -457,6 +457,8 @@ def test_rows_plan_beside_the_256x192_tile():
                                        ((0, 2048, 2560, 2048), "64x128,512t,ring"),      # 640 tiles
                                        ((0, 1026, 3712, 128), "64x128,512t,ring"),       # 12.5 / 24.4 on gemm_tiled, whose price had no fold
                                        ((0, 475, 1464, 1472), "64x64,512t,ring"),        # 19.6 / 23.4 on 64 x 128
+                                       ((0, 1849, 4616, 5312), "256x192,256t"),          # 244 / 275 on 64 x 128, past two rounds
+                                       ((2, 528, 5632, 2048), "128x128,256t"),           # 84 / 92 on 64 x 128, past a round and a half
                                        ((1, 1819, 328, 1856), "64x64,512t,ring"),        # 26.4 / 31.3 on 64 x 128
                                        ((2, 384, 5632, 2048), "256x192,256t")])          # 67 / 74 on 64 x 128 in two parts of which each is past a round
 def test_three_planes_take_the_tile_priced_lowest(key, tile):

@@ -730,21 +730,22 @@ bool gemm_dma_planes3_split_ok(const MMArgs& p, int nsplit) {
 // new step and a slope.  Fitted to 107 products of 384 .. 4096 rows (3400 timed calls, each tile and 1, 2, 4, 8 parts): the choices by it are 1.1 % from the fastest in the mean; by the prices of one plane, with
 // 256 x 192 compared at a second price, they were 3.3 %.  us then -> now: 600 x 2 of 2816 x 1024 40.6 -> 33.0, 900 x 4096 x 4096 101 -> 85, 1650 x 1024 x 2816 45.2 -> 40.0, 450 x 2560 x 2048 32.6 -> 29.1, 509 x 2048 x 5632
 // 47.9 -> 45.3; llama's products of 1024 rows and more keep their tiles or gain up to a tenth.
-// The ring past one round: where a CU holds several workgroups their ends spread, and a little more than a round takes a quarter longer, not twice as long (1900 x 2560 x 2048, 600 tiles of 64 x 128: 65 us, 70 in two parts on 256 x 192);
-// below 48 K tiles that holds up to a round and a half: of 379 products of k 128 .. 960 that are priced so, the 301 within it take 0.95 to 1.8 times as long on the tiles priced next (1.12 in the mean; 640 x 7600 x 640 27.3 us, 29.1 on 128 x 128; 964 x
-// 4928 x 256 16.8 and 18.1; 1650 x 2472 x 512 23.1 and 34.6 on the register-staged kernel), those of more rounds 0.88 to 1.15 times (3107 x 5608 x 896 101.8 us, 89.8 on 128 x 128).
+// The ring past one round: where a CU holds several workgroups their ends spread, and a little more than a round takes a quarter longer, not twice as long (1900 x 2560 x 2048, 600 tiles of 64 x 128: 65 us, 70 in two parts on 256 x 192).
+// That holds up to a round and a half: of 379 products of k 128 .. 960 that are priced so, the 301 within it take 0.95 to 1.8 times as long on the tiles priced next (1.12 in the mean; 640 x 7600 x 640 27.3 us, 29.1 on 128 x 128; 964 x
+// 4928 x 256 16.8 and 18.1; 1650 x 2472 x 512 23.1 and 34.6 on the register-staged kernel), those of more rounds 0.88 to 1.15 times (3107 x 5608 x 896 101.8 us, 89.8 on 128 x 128), and a long K loses there as well
+// (1849 x 4616 x 5312 275 us, 244 on 256 x 192).  `ends`: below 24 K tiles the large tiles' way in and out is not hidden by the K loop (k 128, us above the price without it: 256 x 256 9, 256 x 192 7, 256 x 128 6, 128 x 128 5.5, the ring's 4).
 double gemm_dma_planes3_cost_us(const MMArgs& p, int tile, int nsplit, bool gated) {
   static const struct Price {
-    int tile, per_cu;
+    int tile, per_cu, ends;
     double fixed, step[3], slope[3];
   } prices[] = {
-      {256, 1, 3.3, {1.036}, {0.225}},
-      {192, 1, 3.2, {1.075}, {0}},
-      {128, 1, 3.4, {0.716}, {0.044}},
-      {64, 2, 2.95, {0.440, 0.144}, {0.142, 0.110}},
-      {65, 1, 4.1, {0.231}, {0.186}},
-      {48, 2, 4.25, {0.205, 0.152}, {0.015, 0.111}},
-      {32, 3, 3.95, {0.091, 0.065, 0.109}, {0.099, 0.027, 0.050}},
+      {256, 1, 10, 3.3, {1.036}, {0.225}},
+      {192, 1, 6, 3.2, {1.075}, {0}},
+      {128, 1, 4, 3.4, {0.716}, {0.044}},
+      {64, 2, 3, 2.95, {0.440, 0.144}, {0.142, 0.110}},
+      {65, 1, 0, 4.1, {0.231}, {0.186}},
+      {48, 2, 0, 4.25, {0.205, 0.152}, {0.015, 0.111}},
+      {32, 3, 0, 3.95, {0.091, 0.065, 0.109}, {0.099, 0.027, 0.050}},
   };
   const size_t tiles = tile_count(p, (size_t)nsplit, tile);
   for (const Price& c : prices) {
@@ -752,9 +753,10 @@ double gemm_dma_planes3_cost_us(const MMArgs& p, int tile, int nsplit, bool gate
     const size_t round = 256 * (size_t)c.per_cu;
     const double kt = (double)(p.K / BK / nsplit);
     double us = c.fixed + (double)p.M * p.N * 4 / 6.4e6 * (gated ? 0.25 : nsplit), rounds = (double)(tiles / round);
+    us += 0.021 * c.ends * std::max(0.0, 24 - kt);
     size_t last = tiles % round;
     if (ring_tile(tile) && tiles > round) {
-      if (c.per_cu == 1 || nsplit > 1 || (kt < 48 && 2 * tiles > 3 * round)) return -1.0;
+      if (c.per_cu == 1 || nsplit > 1 || 2 * tiles > 3 * round) return -1.0;
       rounds = std::max(1.25, (double)tiles / round), last = 0;
     }
     for (int j = 0; j < c.per_cu; ++j) {
