@@ -59,7 +59,8 @@ def test_gates_of_every_size(hip, tune, inter):
         want = g64 / (1 + np.exp(-g64))
     whole = g > -88.72  # 1 + exp(-z) is finite in f32
     assert np.all(np.abs(got["14"][:many][~whole]) <= 2.7e-37)
-    units = {s: np.abs(v[:many].astype(np.float64) - want)[whole] / np.spacing(np.abs(want[whole]).astype(np.float32)) for s, v in got.items()}
+    unit = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(want[whole]), 2.0 ** -126))) - 23)
+    units = {s: np.abs(v[:many].astype(np.float64) - want)[whole] / unit for s, v in got.items()}
     print("units of the last place, in registers / fold: most %.2f / %.2f, rms %.3f / %.3f" % tuple(f(units[s]) for f in (np.max, lambda u: np.sqrt(np.mean(u * u))) for s in ("14", "3")), flush=True)
     # exp2, its product's rounding, the sum's, the quotient's: one unit and three halves, each up to twice that where the next binade begins
     assert np.max(units["14"]) <= 5
