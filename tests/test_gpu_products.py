@@ -156,6 +156,39 @@ def test_batches_of_products_of_any_size(hip, b, m, n, k, dtype, kernel, shared)
     assert np.all(np.abs(got[: b * m * n].reshape(exact.shape) - exact) <= bound * 1.001 + 1e-7)
 
 
+# tiles of 32, 64 and 128, whole and with K shared; K of one step and one element, of whole steps behind a remainder of 1, 63 and 64; slabs that begin behind K's first step
+@pytest.mark.parametrize("b, m, n, k", [(1, 40, 33, 65), (3, 31, 70, 129), (1, 65, 67, 191), (1, 1000, 777, 320), (2, 900, 130, 447), (1, 2001, 2050, 193), (1, 39, 801, 2113), (1, 392, 113, 3457)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rhs_nk", [True, False], ids=["NT", "NN"])
+def test_rows_that_start_inside_a_word(hip, b, m, n, k, dtype, rhs_nk):
+    """16-bit rows at odd elements, all of them or every second one, have the bits of the same rows at whole words; behind and between them is not-a-number."""
+    dt, enc = (ug_amd.F16, lambda v: v.astype(np.float16)) if dtype == "f16" else (ug_amd.BF16, rng.to_bf16_bits)
+    a, w = rounded(dtype, rng.uniform_pm1(1, b * m * k)).reshape(b, m, k), rounded(dtype, rng.uniform_pm1(2, b * k * n)).reshape(b, k, n)
+    lines = np.swapaxes(w, 1, 2) if rhs_nk else w
+
+    def placed(x, pitch, offset):
+        full = np.full(offset + x.shape[0] * x.shape[1] * pitch + 1, np.nan, np.float32)
+        full[offset:-1].reshape(x.shape[0], x.shape[1], pitch)[:, :, : x.shape[2]] = x
+        return hip.slice_from(enc(full)), pitch
+
+    def product(odd_a, odd_w, offset):
+        sa, pa = placed(a, k + 2 + (k + odd_a) % 2, offset)
+        sw, pw = placed(lines, lines.shape[2] + 2 + (lines.shape[2] + odd_w) % 2, offset)
+        dst = hip.allocate_uninit(dt, b * m * n)
+        hip.matmul(dst, sa, sw, (b, m, n, k), ((b, m, k), (m * pa, pa, 1), offset), ((b, k, n), (lines.shape[1] * pw, 1, pw) if rhs_nk else (k * pw, pw, 1), offset))
+        assert ug_amd.last_kernel().startswith("gemm_any<"), ug_amd.last_kernel()
+        return dst.to_vec().view(np.uint16)
+
+    print("inside a word", dtype, b, m, n, k, rhs_nk, flush=True)
+    want = product(0, 0, 0)
+    exact = np.matmul(a.astype(np.float64), w.astype(np.float64))
+    got = rng.from_bf16_bits(want) if dtype == "bf16" else want.view(np.float16)
+    bound = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype] * np.abs(exact) + (k + 1) * np.finfo(np.float32).eps * np.matmul(np.abs(a).astype(np.float64), np.abs(w).astype(np.float64))
+    assert np.all(np.abs(got.astype(np.float64).reshape(exact.shape) - exact) <= bound * 1.001 + 1e-7)
+    for odd_a, odd_w, offset in ((1, 1, 0), (1, 1, 1), (0, 0, 1), (1, 0, 1)):
+        assert np.array_equal(product(odd_a, odd_w, offset), want), (odd_a, odd_w, offset)
+
+
 # one group, a wave's 64 and one more, several rounds of them; groups without rows, ends in front of their predecessors' and behind the rows
 @pytest.mark.parametrize("groups", [1, 2, 63, 64, 65, 128, 300])
 @pytest.mark.parametrize("rows", [0, 3, 700])

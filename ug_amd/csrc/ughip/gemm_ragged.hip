@@ -8,13 +8,15 @@
 //   elements in front of K's end by vectors, with zeros for those that belong to the step before (a K of less than one step: element by element). It
 //   holds the only row of a [k, n]-major operand behind which nothing may be read.
 //
-// What bounds it: the steps of K on few tiles (0.3 us each in 16 bits, a CU's share of the caches; 0.6 in f32, the f32 matrix pipe two thirds of that; four steps ahead or more waves per tile change nothing), LDS and the f32
+// What bounds it: the steps of K on few tiles (0.2 us each in 16 bits with operands in L2 and 0.3 past it, a CU's share of the caches; 0.6 in f32, the f32 matrix pipe two thirds of that; four steps ahead, or a
+// tile's waves each on a part of K, change nothing), LDS and the f32
 // matrix pipe on many.  Against element-by-element
-// loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 11.9 us, f32 256 -> 32; 2001^3 f16 270 -> 33, f32 340 -> 139; 3999^2 x
+// loads between two barriers per 32 k (f32: 16), one box: 1000 x 777 x 1531 f16 196 -> 11.9 us (11.2 with chunks put together from words, Side), f32 256 -> 32; 2001^3 f16 270 -> 33, f32 340 -> 139; 3999^2 x
 // 2000 f16 1204 -> 103, f32 1014 -> 520; 100^3 9.4 -> 6.0.  Which tile takes what and where K is split: gemm_ragged_plan.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "gemm.h"
 #include "ughip.h"
@@ -60,8 +62,13 @@ __device__ __forceinline__ void mma(float, const u32x4& a, const u32x4& b, f32x1
 }
 
 // One operand's share of a workgroup's tile: `rows` (M or N) times k.  KC: contiguous along k.
-template <typename T, int B, bool KC, int THREADS = 256>
+// ODD (16 bits, KC): rows may start in the middle of a 4-byte word.  A 16-byte load there keeps a CU's address unit busy for 67 cycles, 44 in the mean where every
+// second row does, and 27 at any word (22 at 16 bytes; 256 workgroups, tiles in L2).  So chunks are loaded from the word behind a row's start on and put together
+// from two words each: the element in front is the last one of the chunk before, the lane below's or, for a row's first chunk, of the step before (`carry`).  A step
+// reads one element past its end, which is there: K's last elements are load_end's.  f16 1000 x 776 x 2057, both operands so, 15.3 -> 13.4 us.
+template <typename T, int B, bool KC, int THREADS = 256, bool ODD = false>
 struct Side {
+  static_assert(!ODD || (KC && sizeof(T) == 2));
   static constexpr int E = 16 / sizeof(T), KE = 8 * E;           // elements per chunk, k per step
   static constexpr int CPR = KC ? 8 : B / E;                     // chunks per row in LDS (a row: of k, or of the operand's rows at one k)
   static constexpr int PITCH = CPR * 16 + 16, LDS_ROWS = KC ? B : KE, BYTES = LDS_ROWS * PITCH;
@@ -69,6 +76,7 @@ struct Side {
   const T* at[N];
   long long step;  // elements from one K step to the next
   int lds_at[N];
+  unsigned odd[ODD ? N : 1], carry[ODD ? N : 1];
 
   __device__ void place(const T* base, int r0, int rows, long long rs, long long cs, int tid) {
     step = KC ? KE : KE * cs;
@@ -79,9 +87,28 @@ struct Side {
       // past the last row: any row (its results are not stored); a chunk that straddles the end runs on into the next k's row
       if (KC) at[i] = base + min(r0 + row, rows - 1) * rs + c * E;
       else at[i] = base + (long long)row * cs + (r0 + c * E < rows ? r0 + c * E : 0);
+      if constexpr (ODD) odd[i] = (unsigned)(reinterpret_cast<uintptr_t>(at[i]) >> 1) & 1u, at[i] += odd[i];  // (every step's: a step is 128 bytes)
     }
   }
-  __device__ u32x4 load(int i, int s) const { return load16(at[i] + s * step); }
+  __device__ u32x4 load(int i, int s) const {
+    if constexpr (ODD) return *reinterpret_cast<const u32x4_at4*>(at[i] + s * step);
+    else return load16(at[i] + s * step);
+  }
+  // ODD: chunks from step s on; the word that a row's first one wants of the step before
+  __device__ void begin_at(int s, int tid) {
+    if constexpr (ODD)
+#pragma unroll
+      for (int i = 0; i < N; ++i) carry[i] = *reinterpret_cast<const unsigned*>(at[i] - (tid & 7) * E + s * step - 2 * (int)odd[i]);
+  }
+  // The chunk that load's result stands for; ODD: step by step.
+  __device__ u32x4 chunk(u32x4 v, int i, int tid) {
+    if constexpr (!ODD) return v;
+    const unsigned below = __builtin_amdgcn_update_dpp(0u, v[3], 0x111, 0xf, 0xf, true);  // lane - 1's
+    const unsigned before = (tid & 7) == 0 ? carry[i] : below, pick = odd[i] ? 0x05040302u : 0x07060504u;
+    carry[i] = __builtin_amdgcn_update_dpp(0u, v[3], 0x107, 0xf, 0xf, true);              // lane + 7's
+    return u32x4{__builtin_amdgcn_perm(v[0], before, pick), __builtin_amdgcn_perm(v[1], v[0], pick), __builtin_amdgcn_perm(v[2], v[1], pick),
+                 __builtin_amdgcn_perm(v[3], v[2], pick)};
+  }
   // step s with `left` elements of k, by element; rows: of the operand behind r0
   __device__ u32x4 load_last(int i, int s, int left, int r0, int rows, int tid) const {
     const int id = tid + THREADS * i, row = id / CPR, c = id % CPR;
@@ -103,7 +130,7 @@ struct Side {
   // an element per thread kept a CU's address unit busy for a microsecond: f16 1000 x 777 x 1531 12.8 -> 12.2 us.)
   __device__ u32x4 load_end(int i, int s, int left, int r0, int rows, int tid) const {
     const int id = tid + THREADS * i, row = id / CPR, c = id % CPR, x = r0 + c * E < rows ? r0 + c * E : 0;
-    if (KC) return load16(at[i] + s * step - (KE - left));
+    if (KC) return load16(at[i] + s * step - (KE - left) - (ODD ? (int)odd[i] : 0));
     const T* q = at[i] + s * step - (KE - left) * (step / KE);
     if (row < KE - 1 || x + E <= rows) return load16(q);
     T t[E];  // behind the last row nothing may be read
@@ -151,10 +178,10 @@ struct Result<T, true> { typedef float type; };
 // 777 x 1001 x 33 4.7 / 4.3, x 63 5.2 / 4.7, 40 of 130 x 130 x 40 5.7 / 5.2, 2001^2 x 33 9.3 / 8.5; f32 777 x 1001 x 30 5.0 / 4.7.)
 // SPLIT: slab s of nsplit has the steps per * s .. per * (s + 1) - 1 of K, the last one the remainder, and leaves its sums in ws, slab_elems apart.
 enum Form { ONE, WHOLE, SPLIT_K };
-template <typename T, int BT, bool A_KC, bool B_KC, Form FORM>
+template <typename T, int BT, bool A_KC, bool B_KC, Form FORM, bool ODD>
 __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int tiles_m, int tiles_n, int nsplit, int per, float* __restrict__ ws, size_t slab_elems) {
-  typedef Side<T, BT, A_KC> SA;
-  typedef Side<T, BT, B_KC> SB;
+  typedef Side<T, BT, A_KC, 256, ODD && A_KC> SA;
+  typedef Side<T, BT, B_KC, 256, ODD && B_KC> SB;
   constexpr bool SPLIT = FORM == SPLIT_K;
   constexpr int MI = BT / 64, KE = SA::KE;
   __shared__ __attribute__((aligned(16))) char lds[2][SA::BYTES + SB::BYTES];
@@ -191,11 +218,11 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
 #pragma unroll
     for (int i = 0; i < SB::N; ++i) rb[d][i] = b.load(i, s);
   };
-  auto put = [&](char* buf, const u32x4* va, const u32x4* vb) {
+  auto put = [&](char* buf, const u32x4* va, const u32x4* vb, bool whole) {  // whole: chunks as they are
 #pragma unroll
-    for (int i = 0; i < SA::N; ++i) *reinterpret_cast<u32x4*>(buf + a.lds_at[i]) = va[i];
+    for (int i = 0; i < SA::N; ++i) *reinterpret_cast<u32x4*>(buf + a.lds_at[i]) = whole ? va[i] : a.chunk(va[i], i, tid);
 #pragma unroll
-    for (int i = 0; i < SB::N; ++i) *reinterpret_cast<u32x4*>(buf + SA::BYTES + b.lds_at[i]) = vb[i];
+    for (int i = 0; i < SB::N; ++i) *reinterpret_cast<u32x4*>(buf + SA::BYTES + b.lds_at[i]) = whole ? vb[i] : b.chunk(vb[i], i, tid);
   };
   auto multiply = [&](const char* buf) {
 #pragma unroll
@@ -214,10 +241,12 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
     for (int i = 0; i < SA::N; ++i) la[i] = a.load_last(i, 0, left, m0, p.M, tid);
 #pragma unroll
     for (int i = 0; i < SB::N; ++i) lb[i] = b.load_last(i, 0, left, n0, p.N, tid);
-    put(lds[0], la, lb);
+    put(lds[0], la, lb, true);
     __syncthreads();
     multiply(lds[0]);
   } else {
+    a.begin_at(with_left ? begin : begin - 1, tid);
+    b.begin_at(with_left ? begin : begin - 1, tid);
     if (with_left) {
 #pragma unroll
       for (int i = 0; i < SA::N; ++i) la[i] = a.load_end(i, full, left, m0, p.M, tid);
@@ -239,13 +268,16 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
       for (int i = 0; i < SA::N; ++i) la[i] = SA::trimmed(la[i], i, left, tid);
 #pragma unroll
       for (int i = 0; i < SB::N; ++i) lb[i] = SB::trimmed(lb[i], i, left, tid);
+      put(lds[0], la, lb, true);
+    } else {
+      put(lds[0], la, lb, false);
     }
-    put(lds[0], la, lb);
     __syncthreads();
     multiply(lds[0]);
     auto step = [&](int d, int s) {
       char* buf = lds[d ^ 1];
-      put(buf, ra[d], rb[d]);
+      if constexpr (ODD) __builtin_amdgcn_sched_barrier(0);  // (or both steps' chunks are put together here, behind all loads)
+      put(buf, ra[d], rb[d], false);
       fetch(d, min(s + 2, end - 1));  // (without a branch, so that a step's loads can be waited for alone)
       __syncthreads();                // one barrier a step: the buffer written next was read before it
       multiply(buf);
@@ -285,10 +317,10 @@ __global__ void __launch_bounds__(256) gemm_ragged(MMArgs p, int batches, int ti
 // in its loop; the four waves' sums meet in LDS.  Part i (of 4 nsplit) has the steps per * i .. per * (i + 1) - 1, of which there may be none; K is more than one step.
 // What bounds it: launch and first bytes, then a wave's chain of steps (0.6 us, in 16 bits 8 KB of a CU's share of the caches).  f32 625 x 319 x 353 on 64 x 64 tiles 10.3 us, 6.3 so;
 // what it takes, and more figures: gemm_ragged_plan.
-template <typename T, bool A_KC, bool B_KC, bool SPLIT>
+template <typename T, bool A_KC, bool B_KC, bool SPLIT, bool ODD>
 __global__ void __launch_bounds__(256) gemm_ragged32(MMArgs p, int batches, int tiles_m, int tiles_n, int nsplit, int per, float* __restrict__ ws, size_t slab_elems) {
-  typedef Side<T, 32, A_KC, 64> SA;
-  typedef Side<T, 32, B_KC, 64> SB;
+  typedef Side<T, 32, A_KC, 64, ODD && A_KC> SA;
+  typedef Side<T, 32, B_KC, 64, ODD && B_KC> SB;
   constexpr int KE = SA::KE, BUF = SA::BYTES + SB::BYTES;
   static_assert(BUF >= 4 * 1024);  // a wave's sums go where its operands were
   __shared__ __attribute__((aligned(16))) char lds[4][BUF];
@@ -321,11 +353,11 @@ __global__ void __launch_bounds__(256) gemm_ragged32(MMArgs p, int batches, int 
       for (int i = 0; i < SB::N; ++i) rb[d][i] = b.load(i, s);
     };
     // (a wave's LDS operations complete in order; the fences keep the compiler from moving lanes' reads over other lanes' writes)
-    auto turn = [&](const u32x4* va, const u32x4* vb, auto&& next) {
+    auto turn = [&](const u32x4* va, const u32x4* vb, bool whole, auto&& next) {  // whole: chunks as they are
 #pragma unroll
-      for (int i = 0; i < SA::N; ++i) *reinterpret_cast<u32x4*>(buf + a.lds_at[i]) = va[i];
+      for (int i = 0; i < SA::N; ++i) *reinterpret_cast<u32x4*>(buf + a.lds_at[i]) = whole ? va[i] : a.chunk(va[i], i, lane);
 #pragma unroll
-      for (int i = 0; i < SB::N; ++i) *reinterpret_cast<u32x4*>(buf + SA::BYTES + b.lds_at[i]) = vb[i];
+      for (int i = 0; i < SB::N; ++i) *reinterpret_cast<u32x4*>(buf + SA::BYTES + b.lds_at[i]) = whole ? vb[i] : b.chunk(vb[i], i, lane);
       next();
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -337,6 +369,8 @@ __global__ void __launch_bounds__(256) gemm_ragged32(MMArgs p, int batches, int 
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
     };
+    a.begin_at(from, lane);
+    b.begin_at(from, lane);
     if (with_left) {
 #pragma unroll
       for (int i = 0; i < SA::N; ++i) la[i] = a.load_end(i, full, left, m0, p.M, lane);
@@ -358,9 +392,14 @@ __global__ void __launch_bounds__(256) gemm_ragged32(MMArgs p, int batches, int 
       for (int i = 0; i < SA::N; ++i) la[i] = SA::trimmed(la[i], i, left, lane);
 #pragma unroll
       for (int i = 0; i < SB::N; ++i) lb[i] = SB::trimmed(lb[i], i, left, lane);
+      turn(la, lb, true, [] {});
+    } else {
+      turn(la, lb, false, [] {});
     }
-    turn(la, lb, [] {});
-    auto step = [&](int d, int s) { turn(ra[d], rb[d], [&] { fetch(d, min(s + 2, end - 1)); }); };
+    auto step = [&](int d, int s) {
+      if constexpr (ODD) __builtin_amdgcn_sched_barrier(0);
+      turn(ra[d], rb[d], false, [&] { fetch(d, min(s + 2, end - 1)); });
+    };
     int s = begin;
     for (; s + 2 <= end; s += 2) step(0, s), step(1, s + 1);  // (no way out between the two: as in gemm_ragged)
     if (s < end) step(0, s);
@@ -401,35 +440,39 @@ __global__ void __launch_bounds__(256) gemm_ragged_fold(const float* __restrict_
   }
 }
 
-template <typename T, int BT, Form FORM>
-hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, int nsplit, float* ws) {
-  const int tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BT - 1) / BT, ke = 128 / (int)sizeof(T), steps = (p.K + ke - 1) / ke, per = (steps + nsplit - 1) / nsplit;
-  const unsigned grid = (unsigned)((batch * tiles_m * tiles_n * nsplit + 7) / 8 * 8);
-  const size_t elems = batch * p.M * p.N, slab = (elems + 3) / 4 * 4;
-  const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
-  if (ak && bk) gemm_ragged<T, BT, true, true, FORM><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  else if (ak) gemm_ragged<T, BT, true, false, FORM><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  else if (bk) gemm_ragged<T, BT, false, true, FORM><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  else gemm_ragged<T, BT, false, false, FORM><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  if (FORM == SPLIT_K) gemm_ragged_fold<T><<<(unsigned)((elems + 1023) / 1024), 256, 0, stream>>>(ws, static_cast<T*>(p.c), elems, slab, nsplit);
-  return hipGetLastError();
+// Whether an operand's contiguous lines, `rows` of them, may start in the middle of a 4-byte word.
+bool odd_rows(const void* base, long long rows, long long pitch, size_t batch, long long batch_stride) {
+  return (reinterpret_cast<uintptr_t>(base) & 2) || (rows > 1 && (pitch & 1)) || (batch > 1 && (batch_stride & 1));
 }
-template <typename T, bool SPLIT>
-hipError_t launch32(hipStream_t stream, const MMArgs& p, size_t batch, int nsplit, float* ws) {
-  const int tiles_m = (p.M + 31) / 32, tiles_n = (p.N + 31) / 32, ke = 128 / (int)sizeof(T), steps = (p.K + ke - 1) / ke, per = (steps + 4 * nsplit - 1) / (4 * nsplit);
+// BT 32: gemm_ragged32
+template <typename T, int BT, Form FORM, bool ODD = false>
+hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, int nsplit, float* ws) {
+  const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
+  // ODD where both operands start anywhere and the address unit is what a step waits for; with one of them aligned putting chunks together takes as long as it saves.  us before /
+  // so: f16 1000 x 776 x 2057 [n, k]-major 15.3 / 13.3, 12 of 17 x 1728 x 3185 47.3 / 35.5, bf16 2692 x 1660 x 3123 (128 x 128) 74.0 / 64.7, [k, n]-major 1000 x 777 x 1531 12.6 / 11.9;
+  // x 776 x 2057, the lhs alone, 12.1 / 12.9 from L2, 13.3 / 13.2 past it.
+  if constexpr (sizeof(T) == 2 && FORM != ONE && !ODD)
+    if ((ak || bk) && odd_rows(p.a, ak ? p.M : p.K, ak ? p.a_rs : p.a_cs, batch, p.a_bs) && odd_rows(p.b, bk ? p.N : p.K, bk ? p.b_cs : p.b_rs, batch, p.b_bs))
+      return launch<T, BT, FORM, true>(stream, p, batch, nsplit, ws);
+  const int tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BT - 1) / BT, ke = 128 / (int)sizeof(T), steps = (p.K + ke - 1) / ke;
+  const int parts = BT == 32 ? 4 * nsplit : nsplit, per = (steps + parts - 1) / parts;
   const unsigned grid = (unsigned)((batch * tiles_m * tiles_n * nsplit + 7) / 8 * 8);
   const size_t elems = batch * p.M * p.N, slab = (elems + 3) / 4 * 4;
-  const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
-  if (ak && bk) gemm_ragged32<T, true, true, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  else if (ak) gemm_ragged32<T, true, false, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  else if (bk) gemm_ragged32<T, false, true, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  else gemm_ragged32<T, false, false, SPLIT><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
-  if (SPLIT) gemm_ragged_fold<T><<<(unsigned)((elems + 1023) / 1024), 256, 0, stream>>>(ws, static_cast<T*>(p.c), elems, slab, nsplit);
+  auto go = [&](auto a_kc, auto b_kc) {
+    constexpr bool odd = ODD && (a_kc() || b_kc());
+    if constexpr (BT == 32) gemm_ragged32<T, a_kc(), b_kc(), FORM == SPLIT_K, odd><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+    else gemm_ragged<T, BT, a_kc(), b_kc(), FORM, odd><<<grid, 256, 0, stream>>>(p, (int)batch, tiles_m, tiles_n, nsplit, per, ws, slab);
+  };
+  if (ak && bk) go(std::true_type(), std::true_type());
+  else if (ak) go(std::true_type(), std::false_type());
+  else if (bk) go(std::false_type(), std::true_type());
+  else go(std::false_type(), std::false_type());
+  if (FORM == SPLIT_K) gemm_ragged_fold<T><<<(unsigned)((elems + 1023) / 1024), 256, 0, stream>>>(ws, static_cast<T*>(p.c), elems, slab, nsplit);
   return hipGetLastError();
 }
 template <typename T>
 hipError_t launch_plan(hipStream_t stream, const MMArgs& p, size_t batch, const RaggedPlan& pl, float* ws) {
-  if (pl.tile == 32) return pl.nsplit > 1 ? launch32<T, true>(stream, p, batch, pl.nsplit, ws) : launch32<T, false>(stream, p, batch, 1, nullptr);
+  if (pl.tile == 32) return pl.nsplit > 1 ? launch<T, 32, SPLIT_K>(stream, p, batch, pl.nsplit, ws) : launch<T, 32, WHOLE>(stream, p, batch, 1, nullptr);
   if (pl.nsplit > 1) return launch<T, 64, SPLIT_K>(stream, p, batch, pl.nsplit, ws);
   if (p.K <= 128 / (int)sizeof(T)) return pl.tile == 128 ? launch<T, 128, ONE>(stream, p, batch, 1, nullptr) : launch<T, 64, ONE>(stream, p, batch, 1, nullptr);
   return pl.tile == 128 ? launch<T, 128, WHOLE>(stream, p, batch, 1, nullptr) : launch<T, 64, WHOLE>(stream, p, batch, 1, nullptr);
