@@ -77,6 +77,30 @@ def test_ring_rows(hip, tune, m, n, k, groups, act):
         close(out[: m * n].reshape(m, n), y, 2e-5)
 
 
+# columns of a last tile that hang over it (192; 96 gated), one row to three tiles of them; four K tiles, the fewest, and odd and even counts
+@pytest.mark.parametrize("m, n, k, groups", [(1, 8, 256, 0), (257, 192, 320, 0), (300, 200, 384, 0), (520, 392, 256, 0), (301, 104, 448, 4)])
+@pytest.mark.parametrize("act", [NONE, SWIGLU, GLU])
+@pytest.mark.parametrize("bf16_out", [False, True], ids=["f32", "bf16"])
+def test_rows_on_256x192_tiles(hip, tune, m, n, k, groups, act, bf16_out):
+    """Rows on 256 x 192 tiles with one wave per SIMD: the bits of the ring's 256 x 128 tiles, nothing behind the result."""
+    gpu, rows, mats = Gpu(hip), n if act == NONE else 2 * n, max(1, groups)
+    dx, dw, db = gpu.up(rand(1, m, k), bf16=True), gpu.up(rand(2, mats, rows, k, std=k ** -0.5), bf16=True), gpu.up(rand(3, rows, std=0.5))
+    idx = (gpu.up(np.random.default_rng(4).integers(0, m, m).astype(np.int32)), gpu.up(np.array([0, m // 3, m // 3, m], np.int32))) if groups else (None, None)
+    got = {}
+    for shape, name in (("14", "256x192,256t,rows"), ("10", "256x128,512t,ring,rows")):
+        tune.setenv("UGHIP_GEMM_SHAPE", shape)
+        dst = gpu.out(m * n + 8, bf16=bf16_out)
+        q = Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), bias=None if groups else db.raw(), m=m, n=n, k=k, product=BF16, act=act, row_index=idx[0].raw() if groups else None,
+                    group_end=idx[1].raw() if groups else None, groups=groups, x_rows=m if groups else 0, act_alpha=1.702 if act == GLU else 0, act_shift=1.0 if act == GLU else 0,
+                    act_limit=1.5 if act == GLU else 0)
+        print("256x192 rows", m, n, k, groups, act, shape, flush=True)
+        gpu.call("ughip_product_rows", C.byref(q))
+        assert name in ug_amd.last_kernel(), ug_amd.last_kernel()
+        got[shape] = get(dst, m * n + 8)
+        assert np.all(np.isnan(got[shape][m * n :])) and not np.any(np.isnan(got[shape][: m * n]))
+    np.testing.assert_array_equal(got["14"][: m * n], got["10"][: m * n])
+
+
 @pytest.mark.parametrize("m, n, k", [(385, 264, 256), (400, 136, 448)])
 def test_ring_planes(hip, tune, m, n, k):
     """Three bf16 terms on the ring's tiles, with a K split where it divides: the bound of an f32 sum."""

@@ -44,7 +44,7 @@ hipError_t gemm_tiled_launch(hipStream_t stream, int dtype, const MMArgs& p, siz
 // negative value when the kernel does not take the problem.  Used to decide between this kernel and gemm_dma4.
 double gemm_tiled_cost_us(int dtype, const MMArgs& p, size_t batch);
 
-// 16-bit types, one wave per SIMD: 256 x 256, 256 x 192 (three planes only), 256 x 128 or 128 x 128 tiles (tile codes 256, 192, 128, 64), 4 waves laid out
+// 16-bit types, one wave per SIMD: 256 x 256, 256 x 192 (three planes and rows), 256 x 128 or 128 x 128 tiles (tile codes 256, 192, 128, 64), 4 waves laid out
 // 2 x 2 with the accumulators in the accumulation registers, loads that write LDS directly, rhs [n, k]- or [k, n]-major
 // (gemm_dma.hip), and a ring of stages under eight waves with 256 x 128, 128 x 128, 64 x 128 and 64 x 64 tiles (codes 129, 65, 48, 32; gemm_ring.hip), for rows
 // also 192 x 192, 32 x 32 and, by group, tiles by height with 192 and 128 columns (97, 16, 193, 130).  Any M, N % 8 == 0, K % 64 == 0 (gemm_dma4: K >= 256), 16-byte aligned rows, contiguous [batch, M, N] result.

@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(256) gemm_dma4(MMArgs p, int tiles_m, int tile
   constexpr bool GATED = ROWS == 2 || ROWS == 4, BY_ROW = ROWS == 1 || ROWS == 2;
   static_assert(BDIV != 3 || TWO, "shared rhs tiles are scheduled with two barriers");
   static_assert(BDIV == 1 || BDIV == 6 || !B_KN, "planes of the lhs alone: against an [n, k]-major rhs only");
-  static_assert(BN != 192 || (!B_KN && F32OUT), "192 columns: neither the swizzle of an n-contiguous tile nor the way out through LDS divides them");
+  static_assert(BN != 192 || (!B_KN && (F32OUT || BY_ROW)), "192 columns: neither the swizzle of an n-contiguous tile nor the way out of whole tiles through LDS divides them");
   extern __shared__ u32x4 lds[];
   constexpr int NI = BM / 32, NJ = BN / 32;            // 16-row and 16-column fragments per wave
   constexpr int NM = NI * NJ;                          // MFMAs per k32 step
@@ -533,7 +533,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 }  // namespace
 
 namespace {
-// tile codes of the entry points below: 256 = 256 x 256, 192 = 256 x 192 (three planes only), 128 = 256 x 128, 64 = 128 x 128; on gemm_ring 129 = 256 x 128, 65 = 128 x 128, 48 = 64 x 128,
+// tile codes of the entry points below: 256 = 256 x 256, 192 = 256 x 192 (three planes and rows), 128 = 256 x 128, 64 = 128 x 128; on gemm_ring 129 = 256 x 128, 65 = 128 x 128, 48 = 64 x 128,
 // 32 = 64 x 64 ([n, k]-major rhs only), 97 = 192 x 192 (rows only), 16 = 32 x 32 (rows only, not gated), 193 / 130 = 256 x 192 / 256 x 128 and lower ones of that width (rows by group only)
 bool tile_dims(int tile, int* bm, int* bn) {
   if (tile == 256) *bm = 256, *bn = 256;
@@ -810,7 +810,7 @@ hipError_t gemm_dma_launch_planes3(hipStream_t stream, const MMArgs& p, int tile
 
 bool gemm_dma_rows_supported(const MMArgs& p, const DmaRows& r, RowsAct act, int tile) {
   int bm, bn;
-  if (!tile_dims(tile, &bm, &bn) || (tile != 256 && !ring_tile(tile)) || ((tile == 256 || tile == 97) && act == RowsAct::LOOKUP) || (by_height(tile) && (!r.groups || act == RowsAct::LOOKUP)))
+  if (!tile_dims(tile, &bm, &bn) || (tile != 256 && tile != 192 && !ring_tile(tile)) || ((tile == 256 || tile == 192 || tile == 97) && act == RowsAct::LOOKUP) || (by_height(tile) && (!r.groups || act == RowsAct::LOOKUP)))
     return false;
   if (tile == 16 && act == RowsAct::GLU) return false;
   if (p.M <= 0 || p.N <= 0 || p.N % 8 || p.K % BK || p.K < least_k(tile) || p.a_cs != 1 || p.a_rs % 8 || p.b_rs != 1 || p.b_cs % 8) return false;
@@ -874,9 +874,11 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
     const int tile = gemm_dma_forced_tile(s), forced = tile == 128 ? 129 : tile == 64 ? 65 : tile;  // (256 x 128 and 128 x 128 tiles of rows are the ring's)
     return forced && gemm_dma_rows_supported(p, r, act, forced) ? forced : 0;
   }
-  // A model's products: the matrix comes from memory.  256 x 256 tiles of gemm_dma4 and the ring's, by what they are expected to take
+  // A model's products: the matrix comes from memory.  256 x 256 and 256 x 192 tiles of gemm_dma4 and the ring's, by what they are expected to take
   // (2048 positions: down 74 -> 51 us, gate and up 105 -> 89, output 26 -> 18, attention's input 37 -> 29; 509 positions: state-space output
-  // 53 -> 19, input 43 -> 32, dense gate and up 40 -> 30; 700 positions' gate and up 52 -> 34; 33 rows of 11264 x 2048 31 -> 13).
+  // 53 -> 19, input 43 -> 32, dense gate and up 40 -> 30; 700 positions' gate and up 52 -> 34; 33 rows of 11264 x 2048 31 -> 13).  256 x 192 where they are nearly whole rounds: 256 x 256 / 256 x 192 / the best of
+  // the ring, us: 2048 x 2 of 5632 x 2048 98 / 86 / 91, 2048 x 2 of 2816 x 1024 29.5 / 26.9 / 34.4, 1544 x 2 of 3072 x 4160 90 / 78 / 100, 3305 x 6336 x 3328 134 / 125 / 132, 877 x 9984 x 2304 51 / 44 / 59; 2048 x 6592 x
+  // 2048, 208 tiles and 280, 48 / 71 / 59.  46 products of 300 to 4096 rows: what is taken by these prices is the fastest but for 4 % at most (3706 x 2 of 1152 x 512, 1.5 us, as before).
   int best = 0;
   double best_us = 0;
   if (r.groups > 1) {
@@ -888,7 +890,7 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
     }
     return best;
   }
-  for (int tile : {256, 129, 65, 48, 32, 16, 97}) {
+  for (int tile : {256, 192, 129, 65, 48, 32, 16, 97}) {
     if (!gemm_dma_rows_supported(p, r, act, tile)) continue;
     if (tile == 16 && p.K < 8 * BK) continue;  // shorter than its ring it gains nothing (54 rows of 2048 x 256 4.0 us on either)
     int bm, bn;
@@ -896,8 +898,8 @@ int gemm_dma_rows_pick(const MMArgs& p, const DmaRows& r, RowsAct act) {
     const size_t tiles = (size_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
     const int kt = p.K / BK;
     double us = 6.0;
-    if (tile == 256)
-      for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * (1.23 + 0.33 * (left < 256 ? (double)left : 256.0) / 256.0);
+    if (!ring_tile(tile))
+      for (size_t left = tiles; left > 0; left -= left < 256 ? left : 256) us += kt * ((tile == 256 ? 1.23 : 0.8) + (tile == 256 ? 0.33 : 0.47) * (left < 256 ? (double)left : 256.0) / 256.0);
     else us = ring_cost_us(tiles, kt, tile, Operands::MEMORY);
     // the larger tile on a near tie; 192 x 192 last, where it clearly saves a round
     if (!best || us < best_us * (tile == 97 ? 0.9 : 0.97)) best = tile, best_us = us;
@@ -911,6 +913,7 @@ hipError_t gemm_dma_launch_rows(hipStream_t stream, const MMArgs& p, const DmaRo
   tile_dims(tile, &bm, &bn);
   note_kernel("gemm_dma4<bf16,NT,%dx%d,%s,rows%s%s>", bm, bn, waves_name(tile), act == RowsAct::GLU ? ",swiglu" : act == RowsAct::LOOKUP ? ",lookup" : "", r.groups ? ",grouped" : "");
   if (ring_tile(tile)) return gemm_ring_launch(stream, UGHIP_BF16, act == RowsAct::GLU ? DmaForm::ROWS_GLU : act == RowsAct::LOOKUP ? DmaForm::ROWS_LOOKUP : DmaForm::ROWS, p, 1, tile, nullptr, r);
+  if (tile == 192) return act == RowsAct::GLU ? launch<__bf16, 256, 192, false, false, 1, 2>(stream, p, 1, nullptr, r) : launch<__bf16, 256, 192, false, false, 1, 1>(stream, p, 1, nullptr, r);
   return act == RowsAct::GLU ? launch<__bf16, 256, 256, false, false, 1, 2>(stream, p, 1, nullptr, r) : launch<__bf16, 256, 256, false, false, 1, 1>(stream, p, 1, nullptr, r);
 }
 
