@@ -476,6 +476,38 @@ def test_f32_rows_of_every_tile(hip, m, n, k, groups, act, tile):
     close(out[: m * n].reshape(m, n), y, 1e-5)  # k eps and the gate's few units, against sums of some standard deviations
 
 
+# K shared and whole, 32-, 64- and 128-row tiles and rows and columns that hang over them; bias, gates and lookups in the fold, results between other rows' elements
+@pytest.mark.parametrize("m, n, k", [(2, 8, 512), (17, 1032, 2048), (33, 136, 1056), (70, 520, 1024), (130, 264, 2048), (200, 1032, 2048)])
+@pytest.mark.parametrize("act, bias, gap", [(NONE, False, 0), (NONE, True, 0), (NONE, False, 3), (SWIGLU, True, 0), (GLU, False, 5), (GELU_MUL, False, 0), (GELU_MUL, True, 1)])
+def test_f32_rows_that_share_their_k(hip, m, n, k, act, bias, gap):
+    gpu, rows = Gpu(hip), 2 * n if act in (SWIGLU, GLU) else n
+    gen = np.random.default_rng(8)
+    x, w, b = gen.standard_normal((m, k), np.float32), (gen.standard_normal((rows, k)) / np.sqrt(k)).astype(np.float32), gen.standard_normal(rows).astype(np.float32)
+    table, ids = gen.standard_normal((50, n + 6)).astype(np.float32), gen.integers(-1, 51, m).astype(np.int32)
+    y = x.astype(np.float64) @ w.T.astype(np.float64) + (b if bias else 0)
+    if act in (SWIGLU, GLU):
+        limit, alpha, shift = (1.5, 1.702, 1.0) if act == GLU else (1e9, 1.0, 0.0)
+        g, u = np.minimum(y[:, :n], limit), np.clip(y[:, n:], -limit, limit)
+        y = g / (1 + np.exp(-alpha * g)) * (u + shift)
+    known = (ids >= 0) & (ids < 50)
+    if act == GELU_MUL:
+        y = 0.5 * y * (1 + np.tanh(np.sqrt(2 / np.pi) * (y + 0.044715 * y ** 3))) * table[np.where(known, ids, 0), 2 : 2 + n]
+    else:
+        known |= True
+    dx, dw, db, dt, di, dst = gpu.up(x), gpu.up(w), gpu.up(b), gpu.up(table), gpu.up(ids), gpu.out(m * (n + gap) + 8)
+    print("f32 rows, K shared", m, n, k, act, bias, gap, flush=True)
+    kw = dict(table=dt.raw(), ids=di.raw(), table_rows=50, table_stride=n + 6, table_col=2) if act == GELU_MUL else {}
+    gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n + gap), w=dw.raw(), bias=db.raw() if bias else None, m=m, n=n, k=k, product=F32, act=act,
+                                                   act_alpha=1.702 if act == GLU else 0, act_shift=1.0 if act == GLU else 0, act_limit=1.5 if act == GLU else 0, **kw)))
+    assert ug_amd.last_kernel().startswith("gemm_tiled<f32,NT,"), ug_amd.last_kernel()
+    out = get(dst, m * (n + gap) + 8)
+    assert np.all(np.isnan(out[m * (n + gap) :]))
+    out = out[: m * (n + gap)].reshape(m, n + gap)
+    assert np.all(np.isnan(out[:, n:])) and np.all(np.isnan(out[~known, :n]))
+    # sums of 2048 are off by 8e-7 of their spread in the mean square, five times that at most here; in a gated unit times the other factor, of up to 4.5
+    close(out[known, :n], y[known], 5 * 8e-7 * 4.5 if act != NONE else 1e-5)
+
+
 def test_f32_rows_of_more_tile_rows_than_a_grid_has(hip):
     """64-row tiles would be more than the 65535 that a grid's second dimension takes."""
     gpu, m, n, k = Gpu(hip), 65535 * 64 + 1, 8, 8

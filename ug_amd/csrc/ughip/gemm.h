@@ -31,10 +31,23 @@ struct MMArgs {
 bool gemm_tiled_supported(int dtype, const MMArgs& p, size_t batch, bool rhs_bf16 = false);
 // What the fold of the partial tiles does on its way out (f32 products only).  With an epilogue the product always goes
 // through the scratch block, even unsplit, and p.c is the epilogue's output.
+struct RowsOut {
+  enum Form { PLAIN = 0, GATED = 1, LOOKUP = 2 } form = PLAIN;
+  const float* bias = nullptr;  // N values
+  float* dst = nullptr;         // rows of N (GATED: N / 2) elements, stride apart
+  size_t stride = 0;
+  float alpha = 1.f, shift = 0.f, limit = 0.f;  // GATED: the gated unit of gate rows, then up rows
+  const void* table = nullptr;                  // LOOKUP: gelu(y) times element (ids[row], table_col + column) of a table, f32 or bf16
+  const int* ids = nullptr;
+  size_t table_stride = 0, table_col = 0;
+  int table_rows = 0;
+  bool table_bf16 = false;
+};
 struct GemmEpilogue {
-  enum Kind { NONE = 0, ADD = 1, SWIGLU = 2 } kind;
+  enum Kind { NONE = 0, ADD = 1, SWIGLU = 2, ROWS = 3 } kind;
   const float* residual;  // ADD: c[m, n] = product + residual[m, n].  SWIGLU: c[m, n / 2] = silu(product[:, :n/2]) * product[:, n/2:]
   bool out_f32 = false;   // a 16-bit product whose fold writes f32 (p.c is then a float buffer)
+  const RowsOut* rows = nullptr;  // ROWS: (p.c is not written)
 };
 // Bytes of f32 scratch the launch needs (split-K partial tiles for skinny products; 0 for most without an epilogue).
 size_t gemm_tiled_workspace_bytes(int dtype, const MMArgs& p, size_t batch, const GemmEpilogue* epi = nullptr);
@@ -42,7 +55,7 @@ hipError_t gemm_tiled_launch(hipStream_t stream, int dtype, const MMArgs& p, siz
                              const GemmEpilogue* epi = nullptr);
 // What the launch above is expected to take (us), from the same per-tile figures that choose its tile and K split; a
 // negative value when the kernel does not take the problem.  Used to decide between this kernel and gemm_dma4.
-double gemm_tiled_cost_us(int dtype, const MMArgs& p, size_t batch);
+double gemm_tiled_cost_us(int dtype, const MMArgs& p, size_t batch, bool always_fold = false);
 
 // 16-bit types, one wave per SIMD: 256 x 256, 256 x 192 (three planes and rows), 256 x 128 or 128 x 128 tiles (tile codes 256, 192, 128, 64), 4 waves laid out
 // 2 x 2 with the accumulators in the accumulation registers, loads that write LDS directly, rhs [n, k]- or [k, n]-major

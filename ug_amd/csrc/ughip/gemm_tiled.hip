@@ -25,6 +25,7 @@
 
 #include "gemm.h"
 #include "internal.h"
+#include "layers.h"
 #include "ughip.h"
 
 namespace ughip {
@@ -442,6 +443,45 @@ __global__ void __launch_bounds__(256) gemm_split_reduce(const float* __restrict
   o[3] = (T)s.w;
 }
 
+// The fold that makes rows of sums what a product of rows leaves: bias, then the gated unit or the gated lookup, four columns of a row to a thread.  What bounds it: a launch and the slabs' way from the caches.
+template <int FORM>
+__global__ void __launch_bounds__(256) gemm_rows_fold(const float* __restrict__ ws, size_t n4, size_t slab_elems, int nsplit, int n, RowsOut o) {
+  const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (g >= n4) return;
+  const int cols = FORM == RowsOut::GATED ? n / 2 : n;
+  const size_t r = g / (cols / 4), at = r * n;
+  const int col = (int)(g - r * (cols / 4)) * 4;
+  f32x4 v[2];
+#pragma unroll
+  for (int h = 0; h < (FORM == RowsOut::GATED ? 2 : 1); ++h) {
+    const float* from = ws + at + col + h * cols;
+    v[h] = *reinterpret_cast<const f32x4*>(from);
+    for (int k = 1; k < nsplit; ++k) v[h] += *reinterpret_cast<const f32x4*>(from + k * slab_elems);
+    if (o.bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[h][e] += o.bias[col + h * cols + e];
+    }
+  }
+  if constexpr (FORM == RowsOut::GATED) {
+    const GluForm glu{o.alpha, o.shift, o.limit};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[0][e] = glu_f(v[0][e], v[1][e], glu);
+  }
+  if constexpr (FORM == RowsOut::LOOKUP) {
+    const int id = o.ids[r];
+    const bool there = id >= 0 && id < o.table_rows;
+    const size_t from = (size_t)(there ? id : 0) * o.table_stride + o.table_col + col;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float f = o.table_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(o.table)[from + e]) : static_cast<const float*>(o.table)[from + e];
+      v[0][e] = gelu_tanh_f(v[0][e]) * (there ? f : __uint_as_float(0x7fc00000u));
+    }
+  }
+  float* to = o.dst + r * o.stride + col;  // (rows may start anywhere)
+#pragma unroll
+  for (int e = 0; e < 4; ++e) to[e] = v[0][e];
+}
+
 // Raises the kernel's dynamic LDS limit once per device (`done`: one bit per device ordinal; devices past 63 pay the call every launch).
 hipError_t allow_lds(const void* kernel, int lds_bytes, std::atomic<unsigned long long>& done) {
   int dev = 0;
@@ -476,7 +516,12 @@ hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, int nsplit,
         gemm_split_reduce<float, GemmEpilogue::ADD><<<grid, dim3(256), 0, stream>>>(ws, c, elems / 4, elems, nsplit, epi->residual, p.N);
       else if (epi && epi->kind == GemmEpilogue::SWIGLU)
         gemm_split_reduce<float, GemmEpilogue::SWIGLU><<<half_grid, dim3(256), 0, stream>>>(ws, c, elems / 8, elems, nsplit, nullptr, p.N);
-      else
+      else if (epi && epi->kind == GemmEpilogue::ROWS) {
+        const RowsOut& o = *epi->rows;
+        if (o.form == RowsOut::GATED) gemm_rows_fold<RowsOut::GATED><<<half_grid, dim3(256), 0, stream>>>(ws, elems / 8, elems, nsplit, p.N, o);
+        else if (o.form == RowsOut::LOOKUP) gemm_rows_fold<RowsOut::LOOKUP><<<grid, dim3(256), 0, stream>>>(ws, elems / 4, elems, nsplit, p.N, o);
+        else gemm_rows_fold<RowsOut::PLAIN><<<grid, dim3(256), 0, stream>>>(ws, elems / 4, elems, nsplit, p.N, o);
+      } else
         gemm_split_reduce<float, 0><<<grid, dim3(256), 0, stream>>>(ws, c, elems / 4, elems, nsplit, nullptr, p.N);
     } else {
       if (epi) return hipErrorInvalidValue;
@@ -617,12 +662,12 @@ hipError_t gemm_fold_f32(hipStream_t stream, const float* slabs, float* c, size_
   return hipGetLastError();
 }
 
-double gemm_tiled_cost_us(int dtype, const MMArgs& p, size_t batch) {
+double gemm_tiled_cost_us(int dtype, const MMArgs& p, size_t batch, bool always_fold) {
   if (!gemm_tiled_supported(dtype, p, batch)) return -1.0;
-  const int s = pick_shape(p, batch, dtype);
+  const int s = pick_shape(p, batch, dtype, always_fold);
   const size_t tiles = tile_count(p, batch, s);
   const double launch_us = 4.0;
-  if (tiles < 256) return launch_us + pick_split(dtype, p, batch, s).cost_us;
+  if (tiles < 256 || always_fold) return launch_us + pick_split(dtype, p, batch, s, always_fold).cost_us;
   // many tiles: a last, partly filled round of workgroups costs a third of a full one plus its share of the rest
   // (16-bit products of 1900..5120 rows with 300, 320, 324, 384, 484 and 800 tiles: within 10 %)
   const double whole = pick_split(dtype, p, batch, s).cost_us / (double)((tiles + 255) / 256);
@@ -649,7 +694,7 @@ void gemm_tiled_name(int dtype, const MMArgs& p, size_t batch, bool rhs_bf16, co
   const bool ragged = s != 0 && (p.M % kShapes[s][0] || p.N % kShapes[s][1]);
   char split[48] = "";
   if (nsplit > 1 || epi)
-    snprintf(split, sizeof split, ",splitK=%d%s%s", nsplit, !epi ? "" : epi->kind == GemmEpilogue::ADD ? ",+residual" : epi->kind == GemmEpilogue::SWIGLU ? ",swiglu" : "",
+    snprintf(split, sizeof split, ",splitK=%d%s%s", nsplit, !epi ? "" : epi->kind == GemmEpilogue::ADD ? ",+residual" : epi->kind == GemmEpilogue::SWIGLU ? ",swiglu" : epi->kind == GemmEpilogue::ROWS ? ",rows" : "",
              epi && epi->out_f32 ? ",f32 out" : "");
   snprintf(out, out_len, "gemm_tiled<%s,%s,%dx%d,%dt%s%s>", tn, nt ? "NT" : "NN", kShapes[s][0], kShapes[s][1], s == 0 && !tune_on(TUNE_GEMM_4WAVES) ? 512 : 256,
            ragged ? ",ragged" : "", split);

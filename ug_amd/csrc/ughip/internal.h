@@ -67,6 +67,8 @@ int rows_add_product_from(ughip_device* dev, const char* what, const float* x, c
 // dst [m, n] = x w^T on dense f32 rows and a BF16 matrix through the kernels of ughip_linear_rows: up to 32 rows on the f32 pipe, up to
 // 128 as three bf16 terms.  false: not their shapes (nothing is launched).
 bool few_rows_product_fits(const ughip_slice* w, const float* x, const float* dst, size_t m, size_t n, size_t k);
+// The device's block for partial tiles, dev->gemm_ws, at least `bytes` long.  no_memory: set, and no error, where there is none.
+int gemm_workspace(ughip_device* dev, size_t bytes, bool* no_memory);
 int few_rows_product(ughip_device* dev, const char* what, const float* x, const ughip_slice* w, float* dst, size_t m, size_t n, size_t k);
 const char* dtype_name(int dt);
 

@@ -1141,6 +1141,8 @@ bool few_rows_product_fits(const ughip_slice* w, const float* x, const float* ds
   return gemm_tiled_supported(x3 ? UGHIP_BF16 : UGHIP_F32, rows_args(x, w->ptr, const_cast<float*>(dst), m, n, k, x3), 1, !x3);
 }
 
+int gemm_workspace(ughip_device* dev, size_t bytes, bool* no_memory) { return grow_gemm_ws(dev, bytes, no_memory); }
+
 int few_rows_product(ughip_device* dev, const char* what, const float* x, const ughip_slice* w, float* dst, size_t m, size_t n, size_t k) {
   return linear_rows_core(dev, what, x, w, nullptr, dst, m, n, k, GemmEpilogue::NONE, m > 32 ? UGHIP_PRODUCT_BF16X3 : UGHIP_PRODUCT_F32, nullptr);
 }

@@ -19,7 +19,7 @@ inline double grouped_tile_rows(int m, int groups, int bm) {
 // as it has, whole ones and one at least, at what a tile takes by itself (us per 2048 of K), and the larger tile's better rate is often less than the smaller one's fuller last round.  us on 22 / 12 / 11: gated
 // n 5632, k 2048, 100 rows 152 / 91, 300 rows 285 / 172, 509 296 / 258, 700 430 / 336, 1024 448 / 486; n 10304, k 2048, 509 rows 296 / 254 / 266; n 6592, 700 rows 290 / 246 / 231; n 2048,
 // 1531 rows 163 / 164 / 148; gated n 2816, k 1024, 300 rows 84 / 51, 700 151 / 91; 16 groups, gated n 1408, 1200 rows 296 / 251, 2036 rows 318 / 334.
-inline int f32_rows_tile(int m, int n, int k, int groups, bool gated) {
+inline int f32_rows_tile(int m, int n, int k, int groups, bool gated, double* price_us = nullptr) {
   int best = 0;
   double best_us = 0;
   for (int tile : {22, 12, 11}) {
@@ -32,6 +32,7 @@ inline int f32_rows_tile(int m, int n, int k, int groups, bool gated) {
     const double us = 4.0 + rounds * k / 2048.0 * (tile == 22 ? 144.0 : tile == 12 ? 81.0 : 45.5);
     if (!best || us < best_us * 0.97) best = tile, best_us = us;
   }
+  if (price_us) *price_us = best_us;
   return best;
 }
 

@@ -332,6 +332,44 @@ hipError_t launch_types(hipStream_t st, const ProductArgs& a, int act, bool vec)
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// f32 rows against an f32 matrix on gemm_tiled, whose tiles go down to 32 rows and whose K is shared where the tiles leave CUs idle: bias, gated unit and lookup are the fold's.  Which of the two kernels a product takes goes
+// by their prices, with 2 us for the other's longer way in (2 to 64 rows of 2048 x 128: 6.9 / 8.4).  us here / there, n x k: 16 rows of 2048 x 2048 48.2 / 14.2, 2048 x 5632 125 / 19.3, gated 2 x 5632 x 2048 83.5 / 29.1, 256 x
+// 2048 with a lookup 48.3 / 13.5; 64 rows 49.0 / 14.7, 126 / 24.0, 85.1 / 45.1; 256 rows 48.7 / 27.7, 126 / 53.8, 151 / 113; 1024 rows 85.4 / 72.5, 225 / 186, 417 / 383; 2048 rows 151 / 130, 401 / 346, 821 / 716; 400 of
+// 6592 x 2048 125 / 128.  Against 64 bits: 2048 rows of 2048 x 5632 1.34e-6 on either, 16 rows 1.33e-6 / 3.4e-7 (shorter sums).
+// done: whether it was launched, else the product is the caller's.
+int tiled_rows(ughip_device* dev, const ProductArgs& a, int act, bool* done) {
+  const bool gated = act == UGHIP_ACT_SWIGLU, lookup = act == UGHIP_ACT_GELU_MUL;
+  *done = false;
+  MMArgs p;
+  p.a = a.x, p.b = a.w, p.M = a.m, p.N = gated ? 2 * a.n : a.n, p.K = a.k;
+  p.a_rs = (long long)a.x_stride, p.a_cs = 1, p.b_rs = 1, p.b_cs = (long long)a.w_stride;
+  p.a_bs = p.b_bs = p.c_bs = 0;
+  p.c = reinterpret_cast<void*>(uintptr_t(1) << 20);  // (a fold's result has a place of its own)
+  const bool fold = gated || lookup || a.bias || a.dst_stride != (size_t)a.n || !aligned16(a.dst);
+  if (!fold) p.c = a.dst;
+  if (a.groups || a.m < 2 || p.N % 8 || a.n % 4 || (long long)a.m * p.N % 8) return UGHIP_OK;
+  const double us = gemm_tiled_cost_us(UGHIP_F32, p, 1, fold);
+  double here = 0;
+  f32_rows_tile(a.m, a.n, a.k, 0, gated, &here);
+  if (us < 0 || us + 2.0 >= 0.97 * here) return UGHIP_OK;
+  RowsOut out;
+  out.form = gated ? RowsOut::GATED : lookup ? RowsOut::LOOKUP : RowsOut::PLAIN;
+  out.bias = a.bias, out.dst = static_cast<float*>(a.dst), out.stride = a.dst_stride;
+  out.alpha = a.glu.alpha, out.shift = a.glu.shift, out.limit = a.glu.limit;
+  out.table = a.table, out.ids = a.ids, out.table_stride = a.table_stride, out.table_col = a.table_col, out.table_rows = a.table_rows, out.table_bf16 = a.table_bf16;
+  GemmEpilogue epi{GemmEpilogue::ROWS, nullptr};
+  epi.rows = &out;
+  const GemmEpilogue* e = fold ? &epi : nullptr;
+  const size_t bytes = gemm_tiled_workspace_bytes(UGHIP_F32, p, 1, e);
+  bool no_memory = false;
+  if (bytes)
+    if (int rc = gemm_workspace(dev, bytes, &no_memory)) return rc;
+  if (no_memory) return UGHIP_OK;
+  UGHIP_HIPCHK(gemm_tiled_launch(dev->stream, UGHIP_F32, p, 1, bytes ? static_cast<float*>(dev->gemm_ws) : nullptr, false, e));
+  *done = true;
+  return UGHIP_OK;
+}
+
 }  // namespace
 
 extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
@@ -424,6 +462,11 @@ extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
       UGHIP_HIPCHK(gemm_dma_launch_rows(dev->stream, q, r, form, tile));
       return UGHIP_OK;
     }
+  }
+  if (f32 && vec) {
+    bool done = false;
+    if (int rc = tiled_rows(dev, a, act, &done)) return rc;
+    if (done) return UGHIP_OK;
   }
   hipError_t e;
   if (f32) e = launch_types<float, float, float>(dev->stream, a, act, vec);
