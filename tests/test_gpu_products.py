@@ -476,6 +476,33 @@ def test_f32_rows_of_every_tile(hip, m, n, k, groups, act, tile):
     close(out[: m * n].reshape(m, n), y, 1e-5)  # k eps and the gate's few units, against sums of some standard deviations
 
 
+# rows a little further apart than they are long, behind others; gathered and by group (with rows that nobody asks for)
+@pytest.mark.parametrize("m, n, k, groups, act", [(*size, 0, act) for size in [(1, 8, 64), (16, 264, 512), (33, 136, 128), (70, 520, 320)] for act in (SWIGLU, GLU, GELU_MUL)] +
+                         [(40, 136, 576, 3, act) for act in (NONE, SWIGLU, GLU)])
+def test_f32_rows_of_a_bf16_product_have_the_bits_of_rounded_ones(hip, m, n, k, groups, act):
+    gpu, rows, mats, rx = Gpu(hip), 2 * n if act in (SWIGLU, GLU) else n, max(1, groups), m + 3
+    gen = np.random.default_rng(8)
+    x = gen.standard_normal((rx, k + 8)).astype(np.float32)
+    dx, db = gpu.up(np.concatenate([np.full(4, np.nan, np.float32), x.ravel()])), gpu.up(np.concatenate([np.full(8, np.nan, np.float32), x.ravel()]), bf16=True)
+    dw, dt, di = gpu.up(rand(2, mats, rows, k, std=k ** -0.5), bf16=True), gpu.up(rand(3, 50, n)), gpu.up(gen.integers(-1, 51, m).astype(np.int32))
+    kw = {}
+    if groups:
+        idx, end = gpu.up(gen.integers(0, rx, m).astype(np.int32)), gpu.up(np.array([0, m // 3, m], np.int32))
+        kw = dict(row_index=idx.raw(), group_end=end.raw(), groups=groups, x_rows=rx)
+    if act == GELU_MUL:
+        kw = dict(table=dt.raw(), ids=di.raw(), table_rows=50, table_stride=n)
+    got = []
+    for rows_of, offset in ((dx, 4), (db, 8)):
+        dst = gpu.out(m * n + 8)
+        print("rounded rows", m, n, k, groups, act, flush=True)
+        gpu.call("ughip_product_rows", C.byref(Product(x=view(rows_of, offset, k + 8), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=BF16, act=act, act_alpha=1.702 if act == GLU else 0,
+                                                       act_shift=1.0 if act == GLU else 0, act_limit=1.5 if act == GLU else 0, **kw)))
+        assert ug_amd.last_kernel().startswith("gemm_dma4<bf16,NT,"), ug_amd.last_kernel()
+        got.append(get(dst, m * n + 8))
+    np.testing.assert_array_equal(got[0], got[1])
+    assert np.all(np.isnan(got[0][m * n :])) and np.any(np.isfinite(got[0][: m * n]))
+
+
 # K shared and whole, 32-, 64- and 128-row tiles and rows and columns that hang over them; bias, gates and lookups in the fold, results between other rows' elements
 @pytest.mark.parametrize("m, n, k", [(2, 8, 512), (17, 1032, 2048), (33, 136, 1056), (70, 520, 1024), (130, 264, 2048), (200, 1032, 2048)])
 @pytest.mark.parametrize("act, bias, gap", [(NONE, False, 0), (NONE, True, 0), (NONE, False, 3), (SWIGLU, True, 0), (GLU, False, 5), (GELU_MUL, False, 0), (GELU_MUL, True, 1)])
