@@ -478,7 +478,7 @@ def test_f32_rows_of_every_tile(hip, m, n, k, groups, act, tile):
 
 # rows a little further apart than they are long, behind others; gathered and by group (with rows that nobody asks for)
 @pytest.mark.parametrize("m, n, k, groups, act", [(*size, 0, act) for size in [(1, 8, 64), (16, 264, 512), (33, 136, 128), (70, 520, 320)] for act in (SWIGLU, GLU, GELU_MUL)] +
-                         [(40, 136, 576, 3, act) for act in (NONE, SWIGLU, GLU)])
+                         [(40, 136, 576, 3, act) for act in (NONE, SWIGLU, GLU)] + [(140, 136, 1024, 0, NONE)])
 def test_f32_rows_of_a_bf16_product_have_the_bits_of_rounded_ones(hip, m, n, k, groups, act):
     gpu, rows, mats, rx = Gpu(hip), 2 * n if act in (SWIGLU, GLU) else n, max(1, groups), m + 3
     gen = np.random.default_rng(8)
