@@ -127,33 +127,3 @@ def test_mask_then_softmax_row_zero_is_one_hot(cpu, cpu_ops):
     p = cpu_ops.custom_softmax(cpu_ops.causal_mask(LB.copy(x, shape, cpu))).data_vec().reshape(shape)
     np.testing.assert_array_equal(p[..., 0, :], np.broadcast_to(np.eye(9, dtype=np.float32)[0], (1, 2, 9)))
     assert np.all(np.triu(p, 1) == 0)
-
-
-@pytest.mark.parametrize("rank", [1, 2, 3, 4, 5])
-def test_device_matmul_takes_its_numbers_as_it_took_them(cpu, rank):
-    """Every rank, ints of either kind, strides of a transposed operand and offsets reach the device as given; a layout
-    of uneven lists, a float and a rank that the device refuses stay errors."""
-    m, n, k = (1, 5, 3) if rank == 1 else (4, 5, 3)
-    a, w = rng.normal(7, m * k + 2), rng.normal(8, n * k + 1)
-    sa, sw, out = cpu.slice_from(a), cpu.slice_from(w), cpu.allocate_uninit(ug_amd.F32, m * n)
-    ones = (1,) * max(0, rank - 2)
-    left, right = (ones + (m, k), (m * k,) * len(ones) + (k, 1), 2), (ones + (k, n), (k * n,) * len(ones) + (1, k), 1)
-    if rank == 1:
-        left, right = ((k,), (1,), 2), ((n,), (1,), 1)
-
-    def run(cast):
-        turned = [(tuple(map(cast, d)), [cast(x) for x in s], cast(o)) for d, s, o in (left, right)]
-        cpu.matmul(out, sa, sw, tuple(map(cast, (1, m, n, k))), *turned)
-        return out.to_vec()
-
-    if rank in (1, 5):
-        with pytest.raises(ug_amd.UgError):
-            run(int)
-    else:
-        want = a[2:].reshape(m, k).astype(np.float64) @ w[1:].reshape(n, k).T.astype(np.float64)
-        np.testing.assert_allclose(run(int).reshape(m, n), want, rtol=0, atol=k * EPS32 * float(np.abs(a).max() * np.abs(w).max()))
-        np.testing.assert_array_equal(run(int), run(np.int64))
-    with pytest.raises((TypeError, ValueError)):
-        run(float)
-    with pytest.raises(IndexError):
-        cpu.matmul(out, sa, sw, (1, m, n, k), (left[0], left[1] + (1,), 0), right)

@@ -4,7 +4,6 @@ read like the reference's own (ug-core/tests/lb_tests.rs, ug-core/src/common_tes
 import contextlib
 import ctypes as C
 import os
-import struct
 
 import numpy as np
 
@@ -100,8 +99,6 @@ class LlamaConfig(C.Structure):
         return self.hidden_size // self.num_attention_heads
 
 
-_MATMUL_SIZES = {rank: struct.Struct(f"{7 + 4 * rank}Q") for rank in range(1, 5)}  # size_t: b, m, n, k, rank, both offsets, then dims and strides of either operand
-
 CUSTOM_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.POINTER(C.c_void_p), C.c_size_t)
 
 
@@ -122,7 +119,6 @@ def host_lib():
                   "ugh_compiled_free", "ugh_llama_ops_free", "ugh_llama_model_free", "ugh_lb_dims", "ugh_ssa_set_launch",
                   "ugh_decoder_free", "ugh_decoder_state_free"):
             getattr(lib, f).restype = None
-        lib.ugh_device_matmul_packed.argtypes = [C.c_void_p] * 4 + [C.c_char_p]
         _host = lib
     return _host
 
@@ -325,16 +321,6 @@ class Device(_Handle):
         """lhs_l / rhs_l: (dims, strides, offset) as in ug::Layout."""
         b, m, n, k = bmnk
         rank = len(lhs_l[0])
-        # All sizes as one packed argument: a dozen ctypes objects took longer than a small product (16 x 16 x 16 back to back: 4.8 to 5.2 us a call, 3.75 packed).
-        # What does not pack (another rank, lists of uneven lengths, a negative number) is for the other call to take or refuse.
-        try:
-            ld, ls, rd, rs = lhs_l[0], lhs_l[1], rhs_l[0], rhs_l[1]
-            sizes = _MATMUL_SIZES[rank].pack(b, m, n, k, rank, lhs_l[2], rhs_l[2], *ld, *ls, *rd, *rs) if len(ls) == len(rd) == len(rs) == rank else None
-        except (KeyError, TypeError, struct.error):
-            sizes = None
-        if sizes is not None:
-            _chk(host_lib().ugh_device_matmul_packed(self.h, dst.h, lhs.h, rhs.h, sizes))
-            return
         sz = C.c_size_t * rank
         _chk(host_lib().ugh_device_matmul(_p(self.h), _p(dst.h), _p(lhs.h), _p(rhs.h), C.c_size_t(b), C.c_size_t(m), C.c_size_t(n),
                                           C.c_size_t(k), C.c_size_t(rank), sz(*lhs_l[0]), sz(*lhs_l[1]), C.c_size_t(lhs_l[2]),

@@ -146,17 +146,6 @@ int ugh_device_matmul(void* d, void* dst, void* lhs, void* rhs, size_t b, size_t
   });
 }
 
-// The same with every number in one array: b, m, n, k, rank (1 .. 4), lhs and rhs offset, lhs dims and strides, rhs dims and strides.
-int ugh_device_matmul_packed(void* d, void* dst, void* lhs, void* rhs, const char* packed) {
-  size_t v[7 + 4 * 4];
-  memcpy(v, packed, 7 * sizeof(size_t));
-  const size_t rank = v[4];
-  if (rank < 1 || rank > 4) return guard([&] { bail("matmul: rank " + std::to_string(rank)); });
-  memcpy(v, packed, (7 + 4 * rank) * sizeof(size_t));
-  const size_t* at = v + 7;
-  return ugh_device_matmul(d, dst, lhs, rhs, v[0], v[1], v[2], v[3], rank, at, at + rank, v[5], at + 2 * rank, at + 3 * rank, v[6]);
-}
-
 // ---- ssa kernels --------------------------------------------------------------------------------
 int ugh_sample_ssa(const char* name, size_t p0, size_t p1, size_t p2, void** out) {
   return guard([&] {
