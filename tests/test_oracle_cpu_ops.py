@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import ug_amd
-from ug_amd import LazyBuffer as LB, rng
+from ug_amd import LazyBuffer as LB, Schedule, rng
 
 EPS32 = float(np.finfo(np.float32).eps)
 
@@ -127,3 +127,33 @@ def test_mask_then_softmax_row_zero_is_one_hot(cpu, cpu_ops):
     p = cpu_ops.custom_softmax(cpu_ops.causal_mask(LB.copy(x, shape, cpu))).data_vec().reshape(shape)
     np.testing.assert_array_equal(p[..., 0, :], np.broadcast_to(np.eye(9, dtype=np.float32)[0], (1, 2, 9)))
     assert np.all(np.triu(p, 1) == 0)
+
+
+@pytest.mark.parametrize("first", ["nothing", "the call's result", "everything"])
+def test_a_custom_calls_result_as_argument_operand_and_result(cpu, first):
+    """A call's result that another call, an expression and the caller ask for: one call whichever of them is scheduled first, and the same once it exists."""
+    x = np.arange(12, dtype=np.float32).reshape(3, 4) - 5
+    calls = []
+
+    def add_one(slices):
+        calls.append("add")
+        slices[1].copy_host_to_device(slices[0].to_vec() + np.float32(1))
+
+    def difference(slices):
+        calls.append("difference")
+        slices[2].copy_host_to_device(slices[0].to_vec() - slices[1].to_vec())
+
+    buf = LB.copy(x, (3, 4), cpu)
+    y = LB.custom(add_one, [buf], (3, 4), ug_amd.F32, cpu)
+    doubled = y.binary("mul", y).binary("add", buf)
+    z = LB.custom(difference, [doubled, y], (3, 4), ug_amd.F32, cpu)
+    if first == "the call's result":
+        Schedule.create_one(y).compile().run()
+    if first == "everything":
+        Schedule.create([y, doubled, z]).compile().run()
+    Schedule.create([z, y, doubled, y]).compile().run()
+    want = (x + 1) * (x + 1) + x
+    np.testing.assert_array_equal(np.reshape(y.data_vec(), (3, 4)), x + 1)
+    np.testing.assert_array_equal(np.reshape(doubled.data_vec(), (3, 4)), want)
+    np.testing.assert_array_equal(np.reshape(z.data_vec(), (3, 4)), want - (x + 1))
+    assert calls == ["add", "difference"]

