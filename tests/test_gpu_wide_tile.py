@@ -65,3 +65,10 @@ def test_gates_of_every_size(hip, tune, inter):
     # exp2, its product's rounding, the sum's, the quotient's: one unit and three halves, each up to twice that where the next binade begins
     assert np.max(units["14"]) <= 5
     assert np.sqrt(np.mean(units["14"] ** 2)) <= 1.02 * np.sqrt(np.mean(units["3"] ** 2))
+
+
+# up to 64 rows the split inside the product has tiles of 64: rows one tile, one short and the fewest, columns that hang over, fewer units than the ring has stages, as many and more, runs that begin
+# and end anywhere in a column tile and a last one that hangs over behind a whole one
+@pytest.mark.parametrize("t,k,n,units", [(64, 64, 8, None), (63, 320, 392, "7"), (64, 384, 136, "6"), (33, 448, 264, "5"), (64, 1024, 640, "16"), (50, 2048, 11264, None), (64, 5632, 1000, None), (40, 640, 2056, "11")])
+def test_split_inside_the_product_on_64_rows(hip, tune, t, k, n, units):
+    parity.test_three_bf16_terms_split_inside_the_product(hip, tune, t, k, n, units)

@@ -1,7 +1,8 @@
 // 33 .. 128 f32 rows against a bf16 matrix [n, k] as three bf16 terms per row element, on the bf16 matrix pipe, with the split done
 // inside the product: x [m, k] f32 is read as it is, no planes go through memory.
 //
-//   unit      = one k tile (64) of one column tile (128 columns): 128 x 128 x 64 x 3 terms, 96 MFMAs of 16 x 16 x 32 per wave
+//   unit      = one k tile (64) of one column tile (128 columns): 128 x 128 x 64 x 3 terms, 96 MFMAs of 16 x 16 x 32 per wave.  Up to 64 rows (BM 64) half of
+//               that, waves 0-3 with 16 rows each: the products of rows that nobody has were the longer half of a unit's time.
 //   workgroup = 8 waves, takes `units` consecutive units of the (column tile, k tile) order -- a stream-K split: with 11264
 //               columns and k = 2048 that is 2816 units, 11 for each of 256 workgroups, where whole tiles would leave 80 CUs idle
 //               (88 tiles x 2) or need a second round (88 x 3).  A workgroup whose units cross into the next column tile stores one
@@ -10,7 +11,7 @@
 //   waves 0-3 : the products.  Wave w owns rows 32 w .. 32 w + 31 and all 128 columns: 16 accumulators.  The matrix tile's
 //               fragments (16 x 128 bits) are read from LDS once per unit and meet the three planes in turn; the row fragments
 //               come from LDS plane by plane.  These waves also send the matrix tiles on their way: global -> LDS
-//               (global_load_lds_dwordx4), three units ahead in a ring of four stages, four instructions per wave and unit.
+//               (global_load_lds_dwordx4), three units ahead in a ring of four stages (BM 64: five in six), four instructions per wave and unit.
 //   waves 4-7 : the rows.  Each loads its part of the 128 x 64 f32 tile of the next unit but one (16-byte loads, rows 256 bytes
 //               apart in memory: whole lines), splits every element into hi + mid + lo (v_cvt_pk_bf16_f32 rounds to nearest
 //               even; the remainders are exact) and writes the three planes into one of two LDS stages in the layout the
@@ -19,11 +20,14 @@
 //   barrier t : in front of the last plane of unit t - 1.  Says that tile t and planes t are in LDS and that nobody reads the LDS
 //               of unit t - 1 any more (its fragments are in registers by then); the last plane of unit t - 1 then runs while the
 //               fragments of unit t arrive, so the matrix pipe does not wait behind the barrier.
-//   LDS       : 4 x 16 KiB matrix stages + 2 x 48 KiB plane stages = 160 KiB, one workgroup per CU.
+//   LDS       : 4 x 16 KiB matrix stages + 2 x 48 KiB plane stages = 160 KiB (BM 64: 6 x 16 + 2 x 24 = 144), one workgroup per CU.
 //
-// What bounds it: the matrix pipe at the rate the power limit allows with random operands (1.7-1.8 PFLOP/s: 0.96 us per unit with
+// What bounds it: with 128 rows the matrix pipe at the rate the power limit allows with random operands (1.7-1.8 PFLOP/s: 0.96 us per unit with
 // every CU busy), plus 4 us of launch, first tile and slab stores; barriers and LDS traffic add a quarter, the conversions and
-// the rows' loads (32 KiB per unit and CU from L2, where planes written by a kernel in front would be 48) a tenth each.
+// the rows' loads (32 KiB per unit and CU from L2, where planes written by a kernel in front would be 48) a tenth each.  With 64 rows a unit is 0.32 us of products and takes 1.0 to 1.1 us, most of it
+// what the four waves of products issue besides; the matrix alone would be 0.8 us a unit from HBM.  So nothing is divided per unit, and no read hangs on a branch between two products.  llama's products of
+// 50 rows in a prompt of width 2048 (gate and up, down, q | k | v, output), us, on 128 rows and so: 27.0, 19.0, 13.1, 12.4 -> 18.7, 14.0, 9.4, 8.7; of width 1024, 64 rows 13.4, 11.5, 8.5, 7.2 -> 9.6, 8.3, 6.6, 5.5.
+// Row loads three units ahead instead of one made nothing faster.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -62,9 +66,11 @@ __device__ __forceinline__ void dma16(const void* base, unsigned voff, unsigned 
 // (16 rows x 4 chunks per instruction) then meet every bank once
 __device__ __forceinline__ int kc_idx(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
 
-constexpr int BN = 128, BM = 128;
-constexpr int NB = 4;  // stages of the matrix ring
-constexpr int B_STAGE = BN * 64 * 2, B_BYTES = NB * B_STAGE, PLANE = BM * 64 * 2, A_STAGE = 3 * PLANE, LDS_TOTAL = B_BYTES + 2 * A_STAGE;
+constexpr int BN = 128, MOST = 128;
+constexpr int stages(int bm) { return bm == 64 ? 6 : 4; }  // of the matrix ring
+constexpr int B_STAGE = BN * 64 * 2;
+constexpr int lds_total(int bm) { return stages(bm) * B_STAGE + 2 * 3 * bm * 64 * 2; }
+inline int tile_rows(size_t m) { return m <= 64 ? 64 : 128; }
 
 // x = hi + mid + lo, every term a bf16 (round to nearest even of what the terms before left: the remainders are exact, so
 // |x - (hi + mid + lo)| <= 2^-25 |x|).  An infinity (given, or reached when |x| rounds up past the largest bf16) is all in hi: its
@@ -83,18 +89,20 @@ __device__ __forceinline__ void split_pair(float x0, float x1, unsigned& hi, uns
   hi = h, mid = m, lo = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{q0, q1}, bf16x2));
 }
 
-// x: [m][k] f32, m <= 128; w: [n][k] bf16; slabs: [S][m][n] f32.  Unit u = T * KT + kt (T: column tile, kt: k tile);
+// x: [m][k] f32, m <= BM; w: [n][k] bf16; slabs: [S][m][n] f32.  Unit u = T * KT + kt (T: column tile, kt: k tile);
 // workgroup g takes units [g U, min(g U + U, total)) and writes slab g - (T KT) / U of every tile T it touches.
+template <int BM>
 __global__ void __launch_bounds__(512) rows_x3_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w, float* __restrict__ slabs, int m, int n, int k, int KT,
                                                       int U, int total) {
+  constexpr int NB = stages(BM), B_BYTES = NB * B_STAGE, PLANE = BM * 64 * 2, A_STAGE = 3 * PLANE, NI = BM / 64;
   extern __shared__ u32x4 lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int u0 = blockIdx.x * U, nU = min(U, total - u0);
   if (wave >= 4) {
-    // 32 instructions of 64 lanes x 4 floats cover the 128 x 64 tile; this wave takes instructions c, c + 4, ...
+    // BM / 4 instructions of 64 lanes x 4 floats cover the BM x 64 tile; this wave takes instructions c, c + 4, ...
     const int c = wave - 4;
-    constexpr int NQ = 8;
+    constexpr int NQ = BM / 16;
     f32x4 raw[2][NQ];
     unsigned goff[NQ];  // byte offset of the lane's 4 floats inside x, without the k tile (rows past the end read the last row: not stored)
     unsigned loff[NQ];  // byte offset inside a plane of the stage
@@ -104,11 +112,12 @@ __global__ void __launch_bounds__(512) rows_x3_kernel(const float* __restrict__ 
       goff[i] = (unsigned)min(row, m - 1) * (unsigned)k * 4u + kq * 16;
       loff[i] = (unsigned)(kc_idx(row, kq >> 1) * 16 + (kq & 1) * 8);
     }
-    auto load = [&](int set, int t) __attribute__((always_inline)) {
-      const int kt = (u0 + min(t, nU - 1)) % KT;  // past the last unit: the last one again, unused
-      const char* base = reinterpret_cast<const char*>(x) + (size_t)kt * 256;
+    int kt_next = u0 % KT, left = nU;  // units are loaded in order: no division for each of them
+    auto load = [&](int set) __attribute__((always_inline)) {
+      const char* base = reinterpret_cast<const char*>(x) + (size_t)kt_next * 256;
 #pragma unroll
       for (int i = 0; i < NQ; ++i) raw[set][i] = *reinterpret_cast<const f32x4*>(base + goff[i]);
+      if (--left > 0) kt_next = kt_next + 1 == KT ? 0 : kt_next + 1;  // past the last unit: the last one again, unused
     };
     auto convert = [&](int set, int t) __attribute__((always_inline)) {
       char __attribute__((address_space(3)))* dst = (char __attribute__((address_space(3)))*)lds + B_BYTES + (t & 1) * A_STAGE;
@@ -133,18 +142,18 @@ __global__ void __launch_bounds__(512) rows_x3_kernel(const float* __restrict__ 
       }
 #undef UGHIP_ROWS_X3_CONVERT
     };
-    load(0, 0);
-    load(1, 1);
+    load(0);
+    load(1);
     convert(0, 0);
     wait_lgkmcnt0();  // the planes are in LDS
     __builtin_amdgcn_s_barrier();  // barrier 0
     for (int t = 1; t < nU; t += 2) {
-      load(0, t + 1);
+      load(0);
       convert(1, t);
       wait_lgkmcnt0();
       __builtin_amdgcn_s_barrier();  // barrier t
       if (t + 1 < nU) {
-        load(1, t + 2);
+        load(1);
         convert(0, t + 1);
         wait_lgkmcnt0();
         __builtin_amdgcn_s_barrier();  // barrier t + 1
@@ -153,33 +162,51 @@ __global__ void __launch_bounds__(512) rows_x3_kernel(const float* __restrict__ 
     return;
   }
   const unsigned lds_addr = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds;
-  auto issue = [&](int t) {
-    const int u = u0 + t, T = u / KT, kt = u - T * KT;
-    const int n_left = n - T * BN;  // a last tile may hang over the end of n: rows past the end fetch the last row again, their columns are not stored
-    const char* base = reinterpret_cast<const char*>(w) + ((size_t)T * BN * k + (size_t)kt * 64) * 2;
+  // Tiles are sent for and finished in order: where that stands is counted up.  (With three divisions and four products of an offset for every unit gate and up of 50 rows of width 2048 took 20.6 us for 19.4.)
+  struct At {
+    int T, kt;
+  };
+  At sent{u0 / KT, u0 % KT}, done = sent;
+  auto step = [&](At& at) {
+    if (++at.kt == KT) at.kt = 0, ++at.T;
+  };
+  unsigned vo[4];
+  auto offsets = [&]() {
+    const int n_left = n - sent.T * BN;  // a last tile may hang over the end of n: rows past the end fetch the last row again, their columns are not stored
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int q = wave + 4 * i, row = q * 8 + (lane >> 3), cp = lane & 7;
-      const unsigned vo = (unsigned)(min(row, n_left - 1) * k * 2 + ((cp ^ ((row >> 1) & 7)) << 4));
-      dma16(base, vo, lds_addr + (t % NB) * B_STAGE + q * 1024);
+      const int row = (wave + 4 * i) * 8 + (lane >> 3), cp = lane & 7;
+      vo[i] = (unsigned)(min(row, n_left - 1) * k * 2 + ((cp ^ ((row >> 1) & 7)) << 4));
     }
   };
-  int issued = 0;
+  offsets();
+  int issued = 0, stage = 0;
+  auto issue = [&]() {
+    const char* base = reinterpret_cast<const char*>(w) + ((size_t)sent.T * BN * k + (size_t)sent.kt * 64) * 2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16(base, vo[i], lds_addr + stage * B_STAGE + (wave + 4 * i) * 1024);
+    ++issued;
+    if (++stage == NB) stage = 0;
+    step(sent);
+    if (sent.kt == 0 && n - sent.T * BN < BN && issued < nU) offsets();
+  };
   // This wave's part of tile t has landed: loads return in order, so with `ahead` younger tiles on their way at most 4 * ahead
   // loads may be outstanding.  (The slab stores of a tile boundary retire in no fixed order against loads, but they can only add
   // to the count: a tile that has not landed keeps every younger load outstanding as well.)
   auto wait_tile = [&](int t) {
     const int ahead = issued - 1 - t;
-    if (ahead >= 2) wait_vmcnt<8>();
+    if (NB > 4 && ahead >= 4) wait_vmcnt<16>();
+    else if (NB > 4 && ahead == 3) wait_vmcnt<12>();
+    else if (ahead >= 2) wait_vmcnt<8>();
     else if (ahead == 1) wait_vmcnt<4>();
     else wait_vmcnt<0>();
   };
-  const int r_base = wave * 32;
-  u32x4 fa[2][2][2], bf[2][8];
-  f32x4 acc[2][8];
+  const int r_base = wave * (BM / 4);
+  u32x4 fa[2][NI][2], bf[2][8];
+  f32x4 acc[NI][8];
   auto zero = [&]() {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
@@ -187,7 +214,7 @@ __global__ void __launch_bounds__(512) rows_x3_kernel(const float* __restrict__ 
   // lane l feeds row / column l % 16, k = 8 (l / 16) .. + 7 of a step of 32
   auto read_a = [&](int set, int t, int p) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int s = 0; s < 2; ++s) fa[set][i][s] = lds[(B_BYTES + (t & 1) * A_STAGE + p * PLANE) / 16 + kc_idx(r_base + 16 * i + (lane & 15), 4 * s + (lane >> 4))];
   };
@@ -198,16 +225,17 @@ __global__ void __launch_bounds__(512) rows_x3_kernel(const float* __restrict__ 
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i][j] = mma16(bf[s][j], fa[set][i][s], acc[i][j]);  // operands swapped: a lane holds 4 consecutive columns of one row
+        for (int i = 0; i < NI; ++i) acc[i][j] = mma16(bf[s][j], fa[set][i][s], acc[i][j]);  // operands swapped: a lane holds 4 consecutive columns of one row
   };
   // Register e of lane l of block (i, j): row r_base + 16 i + l % 16, column 16 j + 4 (l / 16) + e.
   auto finish = [&](int t) {
-    const int u = u0 + t, T = u / KT;
-    if (t + 1 >= nU || (u + 1) / KT != T) {
+    const int T = done.T;
+    step(done);
+    if (t + 1 >= nU || done.T != T) {
       const int slab = blockIdx.x - (T * KT) / U;
       float* out = slabs + (size_t)slab * m * n + (size_t)T * BN;
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < NI; ++i)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const int row = r_base + 16 * i + (lane & 15), col = 16 * j + (lane >> 4) * 4;
@@ -216,13 +244,10 @@ __global__ void __launch_bounds__(512) rows_x3_kernel(const float* __restrict__ 
       zero();
     }
   };
-  for (; issued < min(nU, NB - 1); ++issued) issue(issued);
+  while (issued < min(nU, NB - 1)) issue();
   wait_tile(0);
   __builtin_amdgcn_s_barrier();  // barrier 0
-  if (issued < nU) {
-    issue(issued);
-    ++issued;
-  }
+  if (issued < nU) issue();
   read_a(0, 0, 0);
 #pragma unroll
   for (int s = 0; s < 2; ++s)
@@ -240,19 +265,16 @@ __global__ void __launch_bounds__(512) rows_x3_kernel(const float* __restrict__ 
       wait_tile(t + 1);
       wait_lgkmcnt0();  // this unit's last fragments are in registers: its LDS may be written again behind the barrier
       __builtin_amdgcn_s_barrier();  // barrier t + 1
-      if (issued < nU) {  // into the stage of tile t - 1, whose fragments were read in front of barrier t
-        issue(issued);
-        ++issued;
-      }
-      read_a(P ^ 1, t + 1, 0);
+      if (issued < nU) issue();  // into the stage of tile t, whose fragments were read in front of this barrier
     }
+    read_a(P ^ 1, t + 1, 0);
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i][j] = mma16(bf[s][j], fa[P][i][s], acc[i][j]);
-        if (more) read_b(t + 1, s, j);  // behind the last use of this unit's fragment
+        for (int i = 0; i < NI; ++i) acc[i][j] = mma16(bf[s][j], fa[P][i][s], acc[i][j]);
+        read_b(t + 1, s, j);  // behind the last use of this unit's fragment (behind the last unit: what lies there, unused; with a branch around each of them 19.4 us for 18.7)
       }
     finish(t);
   };
@@ -309,7 +331,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 bool rows_x3_supported(const void* x, const void* w, const void* c, const void* residual, size_t m, size_t n, size_t k) {
   // (the unit count and the byte offsets inside one column tile's rows are held in 32 bits)
-  return m >= 1 && m <= (size_t)BM && n >= 8 && n % 8 == 0 && k >= 64 && k % 64 == 0 && k <= (1u << 20) && n <= (1u << 24) && n * k <= (1ull << 31) && aligned16(x) &&
+  return m >= 1 && m <= (size_t)MOST && n >= 8 && n % 8 == 0 && k >= 64 && k % 64 == 0 && k <= (1u << 20) && n <= (1u << 24) && n * k <= (1ull << 31) && aligned16(x) &&
          aligned16(w) && aligned16(c) && aligned16(residual);
 }
 
@@ -355,13 +377,15 @@ hipError_t rows_x3_launch(hipStream_t stream, const float* x, const void* w, flo
   if (hipError_t e = hipGetDevice(&dev)) return e;
   const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
   if (!bit || !(configured.load(std::memory_order_relaxed) & bit)) {
-    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(rows_x3_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_TOTAL)) return e;
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(rows_x3_kernel<128>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_total(128))) return e;
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(rows_x3_kernel<64>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_total(64))) return e;
     configured.fetch_or(bit, std::memory_order_relaxed);
   }
   const int KT = (int)(k / 64), tiles = (int)((n + BN - 1) / BN), total = tiles * KT;
   // one slab per tile and nothing for the fold to do: the slab is the result
   const bool direct = pl.max_slabs == 1 && kind == GemmEpilogue::NONE;
-  rows_x3_kernel<<<dim3((unsigned)pl.groups), dim3(512), LDS_TOTAL, stream>>>(x, static_cast<const uint16_t*>(w), direct ? c : ws, (int)m, (int)n, (int)k, KT, pl.units, total);
+  auto kernel = tile_rows(m) == 64 ? rows_x3_kernel<64> : rows_x3_kernel<128>;
+  kernel<<<dim3((unsigned)pl.groups), dim3(512), lds_total(tile_rows(m)), stream>>>(x, static_cast<const uint16_t*>(w), direct ? c : ws, (int)m, (int)n, (int)k, KT, pl.units, total);
   if (hipError_t e = hipGetLastError()) return e;
   if (direct) {
     char name[160];
