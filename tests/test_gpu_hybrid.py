@@ -273,6 +273,23 @@ def test_latent_attention_both_ways(gpu, heads, dim, rot, vdim, rank, pos, t, bf
     close(get(dst, want.shape), want, 0.12 if bf16 else 1e-4)
 
 
+@pytest.mark.parametrize("lo, hi", [(-0.1, 0.1), (-1, 1), (-20, -1), (1, 21), (-86, 21)])
+def test_softplus_against_64_bits(gpu, lo, hi):
+    """log(1 + e^z) of a decay's step, one position of a state of one element that starts at zero: y = d * B * x * C with all of them 1."""
+    heads = 32768
+    z = np.random.default_rng(3).uniform(lo, hi, heads).astype(np.float32)
+    z[:4] = lo, hi, (lo + hi) / 2, np.clip(20.0, lo, hi)
+    one, zero, dst = gpu.up(np.ones(heads + 2)), gpu.up(np.zeros(heads)), gpu.out(heads)
+    sz, S = gpu.up(z), gpu.out(heads)
+    gpu.call("ughip_ssm_rows", view(one, 0, heads + 2), view(sz, 0, heads), p(zero), p(zero), p(zero), p(S), Z(0), Z(1), Z(heads), Z(1), Z(1), Z(1), view(dst, 0, heads))
+    want, e = np.logaddexp(0, z.astype(np.float64)), np.exp(np.float64(z))
+    # two functions, each correct to 0.6 of a unit of its result (0.5 is what rounding leaves): the exponential's error, times the logarithm's slope, and the logarithm's own
+    bound = 0.6 * np.spacing(want.astype(np.float32)) + 0.6 * np.spacing(e.astype(np.float32)) / (1 + e)
+    off = np.abs(get(dst, (heads,)) - want) / bound
+    print("softplus", lo, hi, "of the bound", off.max())
+    assert off.max() <= 1
+
+
 @pytest.mark.parametrize("heads, vdim, groups, state, taps", [(1, 1, 1, 1, 1), (6, 21, 3, 19, 3), (4, 64, 2, 128, 4), (2, 70, 1, 40, 4), (3, 16, 3, 200, 2), (8, 4, 4, 8, 5)])
 @pytest.mark.parametrize("cuts", [(1, 1, 1, 1, 1, 1), (150,), (64, 64), (65, 2, 3, 1, 63), (2, 2, 5), (17, 1, 130)])
 def test_state_space_rows_and_steps(gpu, heads, vdim, groups, state, taps, cuts):

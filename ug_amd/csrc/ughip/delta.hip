@@ -112,8 +112,8 @@ constexpr int prepare_threads() {
 }
 // PAIR: two workgroups to a CU.  The queries stay in memory, read where they are used, times their rows' factors (77 KB are left in LDS of 64 rows of
 // 128 channels), and A is read again for every tile of the solve; bound by vector instructions and by what waits for memory between barriers.  2048 positions of 16 heads: 69 us with
-// one workgroup to a CU, 62 us so, 52 with queries asked for ahead of their use, left operands stored in rows and a shorter softplus (10 of the 39 us of a workgroup had been the
-// decays' logarithms).  64 and 200 positions of 8 and 16 heads 27.0 and 28.4 -> 24.0 and 24.9.  Up to one workgroup per CU the queries lie in LDS and A in registers; all three launches of the rows with it, against
+// one workgroup to a CU, 62.6 us so, 59.9 with queries asked for ahead of their use and left operands stored in rows (10 of the 39 us of a workgroup are the
+// decays' logarithms).  Up to one workgroup per CU the queries lie in LDS and A in registers; all three launches of the rows with it, against
 // PAIR there: 989 positions of 4 heads 86.8 and 90.0 us, 898 of 16 (100 channels) 71.9 and 74.8, 3 of 16 (vdim 64) 22.2 and 23.0.
 template <int C, bool VEC, bool PAIR>
 __global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_prepare_kernel(DeltaArgs a) {
