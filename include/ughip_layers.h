@@ -48,7 +48,8 @@ int ughip_gather_rows(ughip_device* dev, const ughip_slice* table, size_t table_
  *                       chosen by the row's token.
  * groups > 0: w holds `groups` matrices one after the other and the m rows come sorted by group: rows
  * group_end[g - 1] .. group_end[g] - 1 meet matrix g, and row r reads x row row_index[r] (NULL: r); what ughip_group_rows
- * writes.  No bias then. */
+ * writes.  No bias then.  An index outside 0 .. x_rows - 1 reads nothing outside x: for F32 rows it stands for a row of zeros, for BF16
+ * rows it is the caller's mistake and what row r of dst holds then is not said (the 16-bit kernels take the nearest row). */
 enum { UGHIP_PRODUCT_BF16 = 2 };
 enum { UGHIP_ACT_NONE = 0, UGHIP_ACT_SWIGLU = 1, UGHIP_ACT_GELU_MUL = 2, UGHIP_ACT_GLU = 3 };
 typedef struct ughip_product {

@@ -503,6 +503,35 @@ def test_f32_rows_of_a_bf16_product_have_the_bits_of_rounded_ones(hip, m, n, k, 
     assert np.all(np.isnan(got[0][m * n :])) and np.any(np.isfinite(got[0][: m * n]))
 
 
+# tiles of bf16 rows and, K no multiple of 64, the kernel of any size; many more rows than are asked for, of which one that nobody asks for is not-a-number
+@pytest.mark.parametrize("k", [1024, 2048, 1020])
+@pytest.mark.parametrize("act", [NONE, SWIGLU])
+def test_f32_rows_by_group_that_name_no_row_are_zeros(hip, k, act):
+    gpu, m, n, rx, groups = Gpu(hip), 70, 136, 5000, 3
+    rows = 2 * n if act else n
+    gen = np.random.default_rng(5)
+    idx = gen.integers(0, rx - 1, m).astype(np.int32)
+    idx[[0, 7, 30, 69]] = -1, rx, 0x7fffffff, -0x80000000
+    x = gen.standard_normal((rx, k)).astype(np.float32)
+    x[rx - 1] = np.nan
+    x[0] = np.nan  # (what an index below would be taken for)
+    idx[idx == 0] = 1
+    w = rand(2, groups, rows, k, std=k ** -0.5)
+    dx, dw, di, de, dst = gpu.up(x), gpu.up(w, bf16=True), gpu.up(idx), gpu.up(np.array([20, 21, m], np.int32)), gpu.out(m * n + 8)
+    print("rows that are none", k, act, flush=True)
+    gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), m=m, n=n, k=k, product=BF16, act=act, row_index=di.raw(), group_end=de.raw(), groups=groups,
+                                                   x_rows=rx)))
+    assert ug_amd.last_kernel().startswith("rows_product<" if k % 64 else "gemm_dma4<bf16,NT,"), ug_amd.last_kernel()
+    got, there = get(dst, m * n + 8), (idx >= 0) & (idx < rx)
+    assert np.all(np.isnan(got[m * n :]))
+    got = got[: m * n].reshape(m, n)
+    assert np.all(got[~there] == 0)
+    y = np.stack([rng.bf16_round(x[idx[r] if there[r] else 1]).astype(np.float64) @ w[0 if r < 20 else 1 if r < 21 else 2].T for r in range(m)])
+    if act:
+        y = y[:, :n] / (1 + np.exp(-y[:, :n])) * y[:, n:]
+    close(got[there], y[there], 2e-5)
+
+
 # K shared and whole, 32-, 64- and 128-row tiles and rows and columns that hang over them; bias, gates and lookups in the fold, results between other rows' elements
 @pytest.mark.parametrize("m, n, k", [(2, 8, 512), (17, 1032, 2048), (33, 136, 1056), (70, 520, 1024), (130, 264, 2048), (200, 1032, 2048)])
 @pytest.mark.parametrize("act, bias, gap", [(NONE, False, 0), (NONE, True, 0), (NONE, False, 3), (SWIGLU, True, 0), (GLU, False, 5), (GELU_MUL, False, 0), (GELU_MUL, True, 1)])

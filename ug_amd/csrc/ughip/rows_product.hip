@@ -330,13 +330,16 @@ hipError_t launch_types(hipStream_t st, const ProductArgs& a, int act, bool vec)
   return launch_act<CT, XT, WT, UGHIP_ACT_NONE>(st, a, vec);
 }
 
-// Rows as bf16, dense, rounded as Raw has it; a thread eight elements.
-__global__ void __launch_bounds__(256) round_rows_kernel(const float* __restrict__ x, uint16_t* __restrict__ out, size_t chunks, unsigned per_row, size_t stride) {
+// Row r, or row index[r] and zeros where there is no such row, as bf16, dense, rounded as Raw has it; a thread eight elements.
+__global__ void __launch_bounds__(256) round_rows_kernel(const float* __restrict__ x, const int* __restrict__ index, int x_rows, uint16_t* __restrict__ out, size_t chunks, unsigned per_row,
+                                                         size_t stride) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= chunks) return;
   const size_t r = i / per_row, c = i - r * per_row;
-  const f32x4_t* from = reinterpret_cast<const f32x4_t*>(x + r * stride + c * 8);
-  *reinterpret_cast<u32x4_t*>(out + i * 8) = Raw<__bf16, float>{from[0], from[1], true}.pack();
+  const int src = index ? index[r] : (int)r;
+  const bool there = src >= 0 && src < x_rows;
+  const f32x4_t* from = reinterpret_cast<const f32x4_t*>(x + (size_t)(there ? src : 0) * stride + c * 8);
+  *reinterpret_cast<u32x4_t*>(out + i * 8) = Raw<__bf16, float>{from[0], from[1], there}.pack();
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -453,7 +456,7 @@ extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
   if (!f32 && !xb && wb && !a.dst_bf16 && p->act == UGHIP_ACT_NONE && !a.bias && !a.groups && p->x.stride == p->k && p->dst.stride == p->n && w_stride == p->k &&
       few_rows_product_fits(p->w, static_cast<const float*>(a.x), static_cast<const float*>(a.dst), p->m, p->n, p->k))
     return few_rows_product(dev, what, static_cast<const float*>(a.x), p->w, static_cast<float*>(a.dst), p->m, p->n, p->k);
-  // f32 rows that a bf16 product rounds: rounded ahead of it by a launch of their own, for those tiles (us here / so: 16 rows gated 2 x 5632 x 2048 29.2 / 15.3, 256 x 2048 with a lookup 17.6 / 11.1, 16 groups of
+  // f32 rows that a bf16 product rounds: rounded (and gathered: those that are asked for, zeros where an index names none) ahead of it by a launch of their own, for those tiles (us here / so: 16 rows gated 2 x 5632 x 2048 29.2 / 15.3, 256 x 2048 with a lookup 17.6 / 11.1, 16 groups of
   // 64 rows in all, n 2 x 704, k 1024 17.9 / 14.0; 509 rows 51 / 34, 19.0 / 11.0, 20.2 / 15.5; plain with a bias 16 x 2048 x 5632 41.5 / 13, 509 x 2048 x 512 8.1 / 11.1)
   const bool rounded = !f32 && !xb && wb && vec && (act != UGHIP_ACT_NONE || a.groups || p->k >= 1024);
   // bf16 rows and matrices: tiles of the kernels whose loads write LDS, from one row up (17 rows of 10304 x 2048 12.6 us against 17.6 here, 5 gated
@@ -470,17 +473,18 @@ extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
     r.glu_alpha = a.glu.alpha, r.glu_shift = a.glu.shift, r.glu_limit = a.glu.limit;
     r.table = a.table, r.ids = a.ids, r.table_stride = (long long)a.table_stride, r.table_col = (long long)a.table_col, r.table_rows = a.table_rows, r.table_bf16 = a.table_bf16;
     const RowsAct form = glu ? RowsAct::GLU : act == UGHIP_ACT_GELU_MUL ? RowsAct::LOOKUP : RowsAct::NONE;
-    if (rounded) q.a = reinterpret_cast<const void*>(uintptr_t(1) << 20), q.a_rs = a.k;
+    if (rounded) q.a = reinterpret_cast<const void*>(uintptr_t(1) << 20), q.a_rs = a.k, r.row_index = nullptr, r.x_rows = a.m;  // (rows are gathered where they are rounded)
     int tile = gemm_dma_rows_pick(q, r, form);
     if (tile && rounded) {
       bool no_memory = false;
-      if (int rc = gemm_workspace(dev, x_rows * p->k * 2, &no_memory)) return rc;
+      if (int rc = gemm_workspace(dev, p->m * p->k * 2, &no_memory)) return rc;
       if (no_memory) tile = 0;
       else q.a = dev->gemm_ws;
     }
     if (tile && rounded) {
-      const size_t chunks = x_rows * p->k / 8;
-      round_rows_kernel<<<(unsigned)((chunks + 255) / 256), 256, 0, dev->stream>>>(static_cast<const float*>(a.x), static_cast<uint16_t*>(dev->gemm_ws), chunks, (unsigned)(p->k / 8), a.x_stride);
+      const size_t chunks = p->m * p->k / 8;
+      round_rows_kernel<<<(unsigned)((chunks + 255) / 256), 256, 0, dev->stream>>>(static_cast<const float*>(a.x), a.row_index, a.x_rows, static_cast<uint16_t*>(dev->gemm_ws), chunks,
+                                                                                  (unsigned)(p->k / 8), a.x_stride);
       UGHIP_HIPCHK(hipGetLastError());
     }
     if (tile) {
