@@ -477,8 +477,8 @@ def test_f32_rows_of_every_tile(hip, m, n, k, groups, act, tile):
 
 
 # rows a little further apart than they are long, behind others; gathered and by group (with rows that nobody asks for)
-@pytest.mark.parametrize("m, n, k, groups, act", [(*size, 0, act) for size in [(1, 8, 64), (16, 264, 512), (33, 136, 128), (70, 520, 320)] for act in (SWIGLU, GLU, GELU_MUL)] +
-                         [(40, 136, 576, 3, act) for act in (NONE, SWIGLU, GLU)] + [(140, 136, 1024, 0, NONE)])
+@pytest.mark.parametrize("m, n, k, groups, act", [(*size, 0, act) for size in [(1, 8, 640), (16, 264, 512), (33, 136, 384), (70, 520, 320)] for act in (SWIGLU, GLU, GELU_MUL)] +
+                         [(40, 136, 576, 3, act) for act in (SWIGLU, GLU)] + [(40, 136, 832, 3, NONE), (40, 136, 64, 70, NONE), (140, 136, 1024, 0, NONE), (33, 8, 768, 0, NONE)])
 def test_f32_rows_of_a_bf16_product_have_the_bits_of_rounded_ones(hip, m, n, k, groups, act):
     gpu, rows, mats, rx = Gpu(hip), 2 * n if act in (SWIGLU, GLU) else n, max(1, groups), m + 3
     gen = np.random.default_rng(8)
@@ -487,7 +487,7 @@ def test_f32_rows_of_a_bf16_product_have_the_bits_of_rounded_ones(hip, m, n, k, 
     dw, dt, di = gpu.up(rand(2, mats, rows, k, std=k ** -0.5), bf16=True), gpu.up(rand(3, 50, n)), gpu.up(gen.integers(-1, 51, m).astype(np.int32))
     kw = {}
     if groups:
-        idx, end = gpu.up(gen.integers(0, rx, m).astype(np.int32)), gpu.up(np.array([0, m // 3, m], np.int32))
+        idx, end = gpu.up(gen.integers(0, rx, m).astype(np.int32)), gpu.up(np.array([0, m // 3] + [m] * (groups - 2), np.int32))
         kw = dict(row_index=idx.raw(), group_end=end.raw(), groups=groups, x_rows=rx)
     if act == GELU_MUL:
         kw = dict(table=dt.raw(), ids=di.raw(), table_rows=50, table_stride=n)

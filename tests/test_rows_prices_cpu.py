@@ -39,3 +39,34 @@ def test_f32_rows_take_the_tile_whose_rounds_are_shortest(tmp_path):
     asked = "\n".join(" ".join(map(str, key)) for key in TILES)
     out = subprocess.run([str(tmp_path / "tiles")], input=asked, capture_output=True, text=True, timeout=60)
     assert out.returncode == 0 and dict(zip(TILES, map(int, out.stdout.split()))) == TILES
+
+
+# (m, n, k, groups, gated, lookup) -> rounded ahead of the product, as either was measured (us on the way / ahead)
+AHEAD = {
+    (2, 64, 64, 0, 1, 0): 0, (2, 64, 512, 0, 1, 0): 1, (2, 64, 2048, 0, 1, 0): 1,                 # 3.3 / 6.2, 6.8 / 5.9, 19.9 / 9.3
+    (130, 64, 64, 0, 1, 0): 1, (32, 704, 128, 0, 1, 0): 0,                                        # 6.7 / 5.9, 5.4 / 6.1
+    (2, 704, 128, 0, 0, 1): 0, (2, 704, 512, 0, 0, 1): 1, (64, 64, 64, 0, 0, 1): 1,               # 5.0 / 6.0, 7.2 / 5.9, 7.1 / 5.9
+    (32, 704, 128, 4, 0, 0): 0, (32, 704, 1024, 4, 0, 0): 1, (64, 64, 64, 64, 0, 0): 1,           # 4.3 / 6.4, 9.1 / 8.2, 9.6 / 6.0
+    (16, 2048, 384, 0, 0, 0): 0, (16, 2048, 768, 0, 0, 0): 1, (16, 2048, 1024, 0, 0, 0): 1,       # 5.7 / 6.0, 7.7 / 6.9, 9.1 / 6.7
+    (300, 2048, 640, 0, 0, 0): 0, (16, 2048, 320, 16, 1, 0): 0, (16, 5632, 2048, 0, 1, 0): 1,     # 8.0 / 8.8, 9.2 / 13.5, 29.2 / 15.3
+    (64, 704, 1024, 16, 1, 0): 1, (64, 1408, 1024, 16, 1, 0): 1, (64, 2048, 1024, 16, 1, 0): 0,   # 17.2 / 12.9, 20.8 / 18.8, 22.7 / 26.9
+}
+AHEAD_PROGRAM = r"""
+#include "rows_prices.h"
+
+#include <cstdio>
+
+int main() {
+  int m, n, k, groups, gated, lookup;
+  while (scanf("%d %d %d %d %d %d", &m, &n, &k, &groups, &gated, &lookup) == 6) printf("%d\n", ughip::rows_rounded_ahead(m, n, k, groups, gated != 0, lookup != 0));
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
+def test_rows_are_rounded_ahead_of_a_product_where_that_pays_for_the_launch(tmp_path):
+    (tmp_path / "main.cpp").write_text(AHEAD_PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I" + os.path.join(ROOT, "ug_amd", "csrc", "ughip"), str(tmp_path / "main.cpp"), "-o", str(tmp_path / "ahead")], check=True)
+    asked = "\n".join(" ".join(map(str, key)) for key in AHEAD)
+    out = subprocess.run([str(tmp_path / "ahead")], input=asked, capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0 and dict(zip(AHEAD, map(int, out.stdout.split()))) == AHEAD

@@ -36,4 +36,35 @@ inline int f32_rows_tile(int m, int n, int k, int groups, bool gated, double* pr
   return best;
 }
 
+// bf16 products of f32 rows: rows_product, which rounds on its way to LDS and has one chain of steps, or a launch that rounds the rows ahead (k % 64 == 0) and the tiles of bf16 rows, two launches of 5.7 us before
+// anything else.  What either takes, us: fitted to 2500 products whose matrices come from caches and 240 from memory (2 to 3000 rows; plain, gated, with a lookup, 2 to 64 groups; n 32 to 6000, k 64 to 5632), 13 and 10 % off
+// in the mean square.
+inline double rounded_on_the_way_us(int m, int n, int k, int groups, bool gated, bool lookup) {
+  const int rows = groups ? (m + groups - 1) / groups : m, met = groups ? std::min(groups, m) : 1;  // matrices that rows meet
+  const long long big = (long long)((m + 127) / 128) * ((n + 127) / 128);
+  const int tile = gated ? (rows > 64 ? 22 : 12) : rows > 64 && big >= 192 ? 22 : 11, bm = tile == 22 ? 128 : 64, cols = (tile == 11 ? 64 : 128) / (gated ? 2 : 1);
+  static const struct {
+    double fixed, height, step, past_step, past, mb;  // height: of a tile's, that rows fill; past: for every round of 256 tiles behind the first; mb: of the matrices
+  } prices[] = {{2.89, 1.39, 0.775, 0.629, 1.9, 0.0}, {2.37, 2.67, 0.578, 0.168, 1.1, 0.059}, {5.69, 0.99, 0.917, 0.706, 3.2, 0.012}};
+  const auto& p = prices[tile == 11 ? 0 : tile == 12 ? 1 : 2];
+  const double high = (double)std::min(rows, bm) / bm, past = std::max(0.0, (double)met * ((rows + bm - 1) / bm) * ((n + cols - 1) / cols) / 256 - 1);
+  const int steps = tile == 11 ? (k + 127) / 128 : (k + 63) / 64;
+  // (a lookup's rows of the table are scattered: 128 x 128 of its elements are asked for by each tile)
+  return p.fixed + p.height * high + steps * (p.step + p.past_step * past) + p.past * past + p.mb * 2e-6 * met * (gated ? 2.0 : 1.0) * n * k + 0.095 * groups +
+         (!lookup ? 0 : tile == 22 ? 23.0 : 1.47 + 1.18 * high);
+}
+inline double rounded_ahead_us(int m, int n, int k, int groups, bool gated) {
+  const int rows = groups ? (m + groups - 1) / groups : m, met = groups ? std::min(groups, m) : 1;
+  const double columns = (gated ? 2.0 : 1.0) * n, past = std::max(0.0, (double)met * ((rows + 127) / 128) * std::ceil(columns / 128) / 256 - 1);  // as tiles of 128 x 128
+  const double us = 5.69 + k / 64 * (0.086 + 0.159 * past) + 1.15 * past + 0.106e-6 * (2.0 * met * columns * k) + 0.169e-6 * (6.0 * m * k) + 0.184e-6 * (4.0 * m * n) + 0.65e-9 * (m * columns * k);
+  return std::max(5.8, us);
+}
+// Ahead where it is clearly the faster one: of the products from caches 1.1 % from the faster one in the mean, 7 of them 4 % and more (13 % at most) slower than on the way; from memory 1.9 %, none.  us on the way / ahead: gated, 2
+// rows, n 64, k 64 3.3 / 6.2, k 512 6.8 / 5.9, k 2048 19.9 / 9.3; 130 rows, k 64 6.7 / 5.9; lookups, 2 rows, n 704, k 128 5.0 / 6.0, k 512 7.2 / 5.9; 4 groups, 32 rows, n 704, k 128 4.3 / 6.4, k 1024 9.1 / 8.2; 64 groups, 64
+// rows, n 64, k 64 9.6 / 6.0; 16 groups, 64 rows, gated, k 1024, n 704 17.2 / 12.9, n 1408 20.8 / 18.8, n 2048 22.7 / 26.9; plain with a bias, n 2048, 16 rows k 384 5.7 / 6.0, k 768 7.7 / 6.9, k 1024 9.1 / 6.7, 300 rows k
+// 640 8.0 / 8.8.
+inline bool rows_rounded_ahead(int m, int n, int k, int groups, bool gated, bool lookup) {
+  return rounded_on_the_way_us(m, n, k, groups, gated, lookup) > 1.06 * rounded_ahead_us(m, n, k, groups, gated);
+}
+
 }  // namespace ughip

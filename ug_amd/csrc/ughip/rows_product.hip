@@ -456,9 +456,9 @@ extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
   if (!f32 && !xb && wb && !a.dst_bf16 && p->act == UGHIP_ACT_NONE && !a.bias && !a.groups && p->x.stride == p->k && p->dst.stride == p->n && w_stride == p->k &&
       few_rows_product_fits(p->w, static_cast<const float*>(a.x), static_cast<const float*>(a.dst), p->m, p->n, p->k))
     return few_rows_product(dev, what, static_cast<const float*>(a.x), p->w, static_cast<float*>(a.dst), p->m, p->n, p->k);
-  // f32 rows that a bf16 product rounds: rounded (and gathered: those that are asked for, zeros where an index names none) ahead of it by a launch of their own, for those tiles (us here / so: 16 rows gated 2 x 5632 x 2048 29.2 / 15.3, 256 x 2048 with a lookup 17.6 / 11.1, 16 groups of
-  // 64 rows in all, n 2 x 704, k 1024 17.9 / 14.0; 509 rows 51 / 34, 19.0 / 11.0, 20.2 / 15.5; plain with a bias 16 x 2048 x 5632 41.5 / 13, 509 x 2048 x 512 8.1 / 11.1)
-  const bool rounded = !f32 && !xb && wb && vec && (act != UGHIP_ACT_NONE || a.groups || p->k >= 1024);
+  // f32 rows that a bf16 product rounds: rounded (and gathered: those that are asked for, zeros where an index names none) ahead of it by a launch of their own, for those tiles, where that pays for the launch
+  // (rows_rounded_ahead; us on the way / ahead: 16 rows gated 2 x 5632 x 2048 29.2 / 15.3, 256 x 2048 with a lookup 17.6 / 11.1, plain with a bias 2048 x 5632 41.5 / 13)
+  const bool rounded = !f32 && !xb && wb && vec && p->k % 64 == 0 && rows_rounded_ahead(a.m, a.n, a.k, a.groups, glu, act == UGHIP_ACT_GELU_MUL);
   // bf16 rows and matrices: tiles of the kernels whose loads write LDS, from one row up (17 rows of 10304 x 2048 12.6 us against 17.6 here, 5 gated
   // rows of 11264 x 2048 12.4 against 28.5; 509 rows of 256 x 2048 times a lookup 14.2 against 20.2, 2048 rows of 2048 x 128 8.4 against 12.3)
   if ((xb && wb) || rounded) {
