@@ -564,6 +564,21 @@ def test_f32_rows_that_share_their_k(hip, m, n, k, act, bias, gap):
     close(out[known, :n], y[known], 5 * 8e-7 * 4.5 if act != NONE else 1e-5)
 
 
+# sums of 131 MB and of 137; rows rounded to 128 MiB and to a row more
+@pytest.mark.parametrize("m, n, k, kind, kernel", [(5000, 6592, 1024, F32, "gemm_tiled<f32,NT,"), (5200, 6592, 1024, F32, "rows_product<f32,"), (16384, 1024, 4096, BF16, "gemm_dma4<bf16,NT,"),
+                                                   (16385, 1024, 4096, BF16, "rows_product<bf16,")])
+def test_rows_take_a_share_of_the_devices_block_at_most(hip, m, n, k, kind, kernel):
+    gpu = Gpu(hip)
+    x, w, b = rng.normal(1, m * k, 1.0).reshape(m, k), rand(2, n, k, std=k ** -0.5), rand(3, n)
+    dx, dw, db, dst = gpu.up(x), gpu.up(w, bf16=kind == BF16), gpu.up(b), gpu.out(m * n)
+    print("the block's share", m, n, k, flush=True)
+    gpu.call("ughip_product_rows", C.byref(Product(x=view(dx, 0, k), dst=view(dst, 0, n), w=dw.raw(), bias=db.raw(), m=m, n=n, k=k, product=kind, act=NONE)))
+    assert ug_amd.last_kernel().startswith(kernel), ug_amd.last_kernel()
+    some = [0, 1, 255, m // 2, m - 130, m - 1]
+    rows = rng.bf16_round(x[some]) if kind == BF16 else x[some]
+    close(get(dst, (m, n))[some], rows.astype(np.float64) @ w.T + b, 1e-5)
+
+
 def test_f32_rows_of_more_tile_rows_than_a_grid_has(hip):
     """64-row tiles would be more than the 65535 that a grid's second dimension takes."""
     gpu, m, n, k = Gpu(hip), 65535 * 64 + 1, 8, 8

@@ -70,3 +70,30 @@ def test_rows_are_rounded_ahead_of_a_product_where_that_pays_for_the_launch(tmp_
     asked = "\n".join(" ".join(map(str, key)) for key in AHEAD)
     out = subprocess.run([str(tmp_path / "ahead")], input=asked, capture_output=True, text=True, timeout=60)
     assert out.returncode == 0 and dict(zip(AHEAD, map(int, out.stdout.split()))) == AHEAD
+
+
+# (us on the tiles, us on rows_product, bytes between the tiles and their fold) -> on the tiles
+ON_TILES = {
+    (771.0, 868.0, 2048 * 11264 * 4): 1, (771.0, 868.0, 1 << 27): 1, (771.0, 868.0, (1 << 27) + 1): 0, (6105.2, 6340.0, 16384 * 11264 * 4): 0, (771.0, 868.0, 0): 1,
+    (-1.0, 868.0, 0): 0, (840.0, 868.0, 0): 0,
+}
+ON_TILES_PROGRAM = r"""
+#include "rows_prices.h"
+
+#include <cstdio>
+
+int main() {
+  double tiles, other;
+  size_t bytes;
+  while (scanf("%lf %lf %zu", &tiles, &other, &bytes) == 3) printf("%d\n", ughip::f32_rows_on_tiles(tiles, other, bytes));
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
+def test_f32_rows_take_no_more_of_the_devices_block_than_its_share(tmp_path):
+    (tmp_path / "main.cpp").write_text(ON_TILES_PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I" + os.path.join(ROOT, "ug_amd", "csrc", "ughip"), str(tmp_path / "main.cpp"), "-o", str(tmp_path / "on_tiles")], check=True)
+    asked = "\n".join(" ".join(map(str, key)) for key in ON_TILES)
+    out = subprocess.run([str(tmp_path / "on_tiles")], input=asked, capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0 and dict(zip(ON_TILES, map(int, out.stdout.split()))) == ON_TILES

@@ -2,8 +2,13 @@
 #pragma once
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 
 namespace ughip {
+
+// What a product of rows takes at most of the device's block, which stays as large as the largest call made it, where it can do without: 128 MiB are the sums of 2978 rows of 2 x 5632, and of a product with more the tiles
+// of 32 to 128 rows would gain 9 % at most (6144 rows of 5632 x 2048 1185 us for 1300 by the prices, 16384 of 2 x 5632 4 %, with 738 MB).
+constexpr size_t ROWS_BLOCK_MOST = (size_t)128 << 20;
 
 // How rows by group are spread is not known where a product is planned: a router's experts come out with shares that differ by 40 % or so, the share of an even one's rows times one of these for a sixteenth of the groups each.
 constexpr double SHARES[16] = {.44, .55, .62, .68, .73, .79, .84, .90, .95, 1.02, 1.08, 1.16, 1.26, 1.38, 1.56, 1.94};
@@ -35,6 +40,9 @@ inline int f32_rows_tile(int m, int n, int k, int groups, bool gated, double* pr
   if (price_us) *price_us = best_us;
   return best;
 }
+
+// f32 rows against an f32 matrix: gemm_tiled's tiles, at their price (negative: they do not take it) and with `bytes` for what lies between them and the fold, or rows_product's.  2 us are the tiles' longer way in.
+inline bool f32_rows_on_tiles(double tiles_us, double rows_product_us, size_t bytes) { return tiles_us >= 0 && tiles_us + 2.0 < 0.97 * rows_product_us && bytes <= ROWS_BLOCK_MOST; }
 
 // bf16 products of f32 rows: rows_product, which rounds on its way to LDS and has one chain of steps, or a launch that rounds the rows ahead (k % 64 == 0) and the tiles of bf16 rows, two launches of 5.7 us before
 // anything else.  What either takes, us: fitted to 2500 products whose matrices come from caches and 240 from memory (2 to 3000 rows; plain, gated, with a lookup, 2 to 64 groups; n 32 to 6000, k 64 to 5632), 13 and 10 % off

@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(256) round_rows_kernel(const float* __restrict
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // f32 rows against an f32 matrix on gemm_tiled, whose tiles go down to 32 rows and whose K is shared where the tiles leave CUs idle: bias, gated unit and lookup are the fold's.  Which of the two kernels a product takes goes
-// by their prices, with 2 us for the other's longer way in (2 to 64 rows of 2048 x 128: 6.9 / 8.4).  us here / there, n x k: 16 rows of 2048 x 2048 48.2 / 14.2, 2048 x 5632 125 / 19.3, gated 2 x 5632 x 2048 83.5 / 29.1, 256 x
+// by their prices (f32_rows_on_tiles; 2 to 64 rows of 2048 x 128: 6.9 / 8.4) and by what the fold's sums need.  us here / there, n x k: 16 rows of 2048 x 2048 48.2 / 14.2, 2048 x 5632 125 / 19.3, gated 2 x 5632 x 2048 83.5 / 29.1, 256 x
 // 2048 with a lookup 48.3 / 13.5; 64 rows 49.0 / 14.7, 126 / 24.0, 85.1 / 45.1; 256 rows 48.7 / 27.7, 126 / 53.8, 151 / 113; 1024 rows 85.4 / 72.5, 225 / 186, 417 / 383; 2048 rows 151 / 130, 401 / 346, 821 / 716; 400 of
 // 6592 x 2048 125 / 128.  Against 64 bits: 2048 rows of 2048 x 5632 1.34e-6 on either, 16 rows 1.33e-6 / 3.4e-7 (shorter sums).
 // done: whether it was launched, else the product is the caller's.
@@ -363,16 +363,16 @@ int tiled_rows(ughip_device* dev, const ProductArgs& a, int act, bool* done) {
   const double us = gemm_tiled_cost_us(UGHIP_F32, p, 1, fold);
   double here = 0;
   f32_rows_tile(a.m, a.n, a.k, 0, gated, &here);
-  if (us < 0 || us + 2.0 >= 0.97 * here) return UGHIP_OK;
+  GemmEpilogue epi{GemmEpilogue::ROWS, nullptr};
+  const GemmEpilogue* e = fold ? &epi : nullptr;
+  const size_t bytes = us < 0 ? 0 : gemm_tiled_workspace_bytes(UGHIP_F32, p, 1, e);
+  if (!f32_rows_on_tiles(us, here, bytes)) return UGHIP_OK;
   RowsOut out;
   out.form = gated ? RowsOut::GATED : lookup ? RowsOut::LOOKUP : RowsOut::PLAIN;
   out.bias = a.bias, out.dst = static_cast<float*>(a.dst), out.stride = a.dst_stride;
   out.alpha = a.glu.alpha, out.shift = a.glu.shift, out.limit = a.glu.limit;
   out.table = a.table, out.ids = a.ids, out.table_stride = a.table_stride, out.table_col = a.table_col, out.table_rows = a.table_rows, out.table_bf16 = a.table_bf16;
-  GemmEpilogue epi{GemmEpilogue::ROWS, nullptr};
   epi.rows = &out;
-  const GemmEpilogue* e = fold ? &epi : nullptr;
-  const size_t bytes = gemm_tiled_workspace_bytes(UGHIP_F32, p, 1, e);
   bool no_memory = false;
   if (bytes)
     if (int rc = gemm_workspace(dev, bytes, &no_memory)) return rc;
@@ -458,7 +458,7 @@ extern "C" int ughip_product_rows(ughip_device* dev, const ughip_product* p) {
     return few_rows_product(dev, what, static_cast<const float*>(a.x), p->w, static_cast<float*>(a.dst), p->m, p->n, p->k);
   // f32 rows that a bf16 product rounds: rounded (and gathered: those that are asked for, zeros where an index names none) ahead of it by a launch of their own, for those tiles, where that pays for the launch
   // (rows_rounded_ahead; us on the way / ahead: 16 rows gated 2 x 5632 x 2048 29.2 / 15.3, 256 x 2048 with a lookup 17.6 / 11.1, plain with a bias 2048 x 5632 41.5 / 13)
-  const bool rounded = !f32 && !xb && wb && vec && p->k % 64 == 0 && rows_rounded_ahead(a.m, a.n, a.k, a.groups, glu, act == UGHIP_ACT_GELU_MUL);
+  const bool rounded = !f32 && !xb && wb && vec && p->k % 64 == 0 && p->m * p->k * 2 <= ROWS_BLOCK_MOST && rows_rounded_ahead(a.m, a.n, a.k, a.groups, glu, act == UGHIP_ACT_GELU_MUL);
   // bf16 rows and matrices: tiles of the kernels whose loads write LDS, from one row up (17 rows of 10304 x 2048 12.6 us against 17.6 here, 5 gated
   // rows of 11264 x 2048 12.4 against 28.5; 509 rows of 256 x 2048 times a lookup 14.2 against 20.2, 2048 rows of 2048 x 128 8.4 against 12.3)
   if ((xb && wb) || rounded) {
