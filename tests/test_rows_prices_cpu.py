@@ -97,3 +97,31 @@ def test_f32_rows_take_no_more_of_the_devices_block_than_its_share(tmp_path):
     asked = "\n".join(" ".join(map(str, key)) for key in ON_TILES)
     out = subprocess.run([str(tmp_path / "on_tiles")], input=asked, capture_output=True, text=True, timeout=60)
     assert out.returncode == 0 and dict(zip(ON_TILES, map(int, out.stdout.split()))) == ON_TILES
+
+
+# (rows, vdim, CUs) -> results of a workgroup
+MERGED = {
+    (16, 128, 256): 16, (32, 128, 256): 16, (33, 128, 256): 32, (64, 128, 256): 32, (65, 128, 256): 64, (128, 128, 256): 64, (129, 128, 256): 128, (256, 128, 256): 128, (2048, 128, 256): 128,
+    (128, 64, 256): 32, (129, 64, 256): 64, (512, 64, 256): 64, (2048, 16, 256): 16, (2048, 8, 256): 16, (2048, 17, 256): 32, (128, 32, 256): 16, (129, 32, 256): 32, (64, 200, 256): 64, (512, 200, 256): 128,
+    (512, 1, 256): 16, (128, 128, 64): 128,
+}
+MERGED_PROGRAM = r"""
+#include "rows_prices.h"
+
+#include <cstdio>
+
+int main() {
+  size_t rows, vdim;
+  int cus;
+  while (scanf("%zu %zu %d", &rows, &vdim, &cus) == 3) printf("%d\n", ughip::latent_merge_results(rows, vdim, cus));
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
+def test_latent_merge_leaves_no_cu_idle_and_makes_no_more_than_there_is(tmp_path):
+    (tmp_path / "main.cpp").write_text(MERGED_PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I" + os.path.join(ROOT, "ug_amd", "csrc", "ughip"), str(tmp_path / "main.cpp"), "-o", str(tmp_path / "merged")], check=True)
+    asked = "\n".join(" ".join(map(str, key)) for key in MERGED)
+    out = subprocess.run([str(tmp_path / "merged")], input=asked, capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0 and dict(zip(MERGED, map(int, out.stdout.split()))) == MERGED

@@ -12,6 +12,7 @@
 #include "attention_rows.h"
 #include "bf16_split.h"
 #include "layers.h"
+#include "rows_prices.h"
 
 using namespace ughip;
 
@@ -357,8 +358,8 @@ __global__ void __launch_bounds__(64 * SPLIT_WAVES) latent_split_kernel(SplitArg
   }
 }
 
-// The parts of one (position, head) added up, then MERGE_V elements of the head's result through the values' up-projection: 16 where that is what gives every CU something to do, more where
-// there are rows enough, as every workgroup adds all parts up.  us with 16 and so, 16 heads of 128 elements, rank 512: 16 positions 27.8 -> 16.5, 64 87.9 -> 38.4.
+// The parts of one (position, head) added up, then MERGE_V elements of the head's result through the values' up-projection (how many: latent_merge_results).  us for all
+// three launches with 16 always and so, 16 heads of 128 elements, rank 512, bf16 matrices: 4 positions 18.7 -> 16.4, 16 36.8 -> 24.4, 64 110.7 -> 58.1.
 constexpr int MERGE_WAVES = 16, MERGE_THREADS = 64 * MERGE_WAVES, SPLITS_MAX = 128;
 template <typename WT, bool V4, int MERGE_V>
 __global__ void __launch_bounds__(MERGE_THREADS) latent_merge_kernel(const float* __restrict__ acc, const float* __restrict__ ml, const WT* __restrict__ w, float* __restrict__ dst,
@@ -570,8 +571,10 @@ extern "C" int ughip_latent_attention_absorbed(ughip_device* dev, ughip_view q, 
                                                                                                                   (int)rank, (int)vdim);
   };
   auto merge = [&](auto* w, auto vec) {
-    if (rows < 128) merge_some(w, vec, integral_constant<int, 16>{});
-    else if (rows < 512) merge_some(w, vec, integral_constant<int, 64>{});
+    const int some = latent_merge_results(rows, vdim, dev->num_cus);
+    if (some == 16) merge_some(w, vec, integral_constant<int, 16>{});
+    else if (some == 32) merge_some(w, vec, integral_constant<int, 32>{});
+    else if (some == 64) merge_some(w, vec, integral_constant<int, 64>{});
     else merge_some(w, vec, integral_constant<int, 128>{});
   };
   if (bf && v4) merge(buf_ptr<uint16_t>(w_uv), std::true_type{});

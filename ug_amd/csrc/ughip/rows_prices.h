@@ -75,4 +75,13 @@ inline bool rows_rounded_ahead(int m, int n, int k, int groups, bool gated, bool
   return rounded_on_the_way_us(m, n, k, groups, gated, lookup) > 1.06 * rounded_ahead_us(m, n, k, groups, gated);
 }
 
+// How many of a head's vdim results a workgroup of latent_merge makes, of 16, 32, 64 and 128 (latent_attention.hip): every one adds all parts of its row up, so as few workgroups to a row as leave no CU idle, the least number of
+// results that is one round of them, and no more than there are.  us for all three launches on 16 / 32 / 64 / 128, f32, rank 512: vdim 128, 64 rows 18.4 / 16.1 / 16.7 / 19.0, 96 21.2 / 19.2 / 17.2 / 19.4, 128 24.2 / 20.0 / 18.1 /
+// 20.5, 256 35.2 / 27.3 / 23.5 / 22.4, 2048 192 / 128 / 97 / 87; vdim 64, 128 rows 19.3 / 17.1 / 17.6 / 18.6, 192 22.9 / 20.8 / 18.8 / 19.7; vdim 16, 1024 rows 37.0 / 37.1 / 37.7 / 40.3.
+inline int latent_merge_results(size_t rows, size_t vdim, int cus) {
+  int v = 16;
+  while (v < 128 && (size_t)v < vdim && rows * ((vdim + v - 1) / v) > (size_t)cus) v *= 2;
+  return v;
+}
+
 }  // namespace ughip
