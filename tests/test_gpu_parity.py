@@ -1691,7 +1691,7 @@ def test_projections_of_several_rows_as_three_bf16_terms(hip, t, k, n):
         assert kern3.startswith("gemm_tiled<f32xbf16,NT,"), kern3
         lin3, add3, glu3, kern3 = run_c_abi()
     if 32 < t <= 128:
-        assert kern3.startswith("rows_x3<128x128,3 terms split in the kernel,"), kern3   # the split happens inside the product
+        assert kern3.startswith(f"rows_x3<{64 if t <= 64 else 128}x128,3 terms split in the kernel,"), kern3   # the split happens inside the product
     else:
         assert kern3.startswith("gemm_tiled<bf16,NT,") and "f32 out" in kern3, kern3   # (fewer than 384 rows in every case here)
     assert kern1.startswith("gemm_tiled<f32xbf16,NT,"), kern1
@@ -1785,7 +1785,7 @@ def test_three_bf16_terms_split_inside_the_product(hip, tune, t, k, n, units):
         tune.setenv("UGHIP_X3_ROWS", units)
     (lin, add, glu), kerns = run(x, w, wgu)
     for kn, word in zip(kerns, ("fold>", "+residual in the fold", "swiglu fold")):   # ("no fold" where every tile has one slab: it is the result)
-        assert kn.startswith("rows_x3<128x128,3 terms split in the kernel,") and word in kn, kn
+        assert kn.startswith(f"rows_x3<{64 if t <= 64 else 128}x128,3 terms split in the kernel,") and word in kn, kn
     if units and -(-n // 128) * (k // 64) <= 256 * int(units):
         assert f",{units} units x " in kerns[0], kerns[0]
     if (t, k, n) == (128, 2048, 11264):

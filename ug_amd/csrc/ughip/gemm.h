@@ -142,7 +142,7 @@ void gemm_dma_f32_name(const MMArgs& p, char* out, size_t out_len);
 // (rows_x3.hip): partial sums of `units` consecutive (column tile, k tile) units per workgroup go to f32 slabs in `ws`, a fold adds
 // them in a fixed order and applies the epilogue.  n % 8 == 0, k % 64 == 0, 16-byte aligned buffers.
 struct RowsX3Plan {
-  int units = 0, groups = 0, max_slabs = 0;
+  int tile_rows = 128, units = 0, groups = 0, max_slabs = 0;  // tile_rows: 64 or 128, of 128 columns
   size_t ws_bytes = 0;
 };
 bool rows_x3_supported(const void* x, const void* w, const void* c, const void* residual, size_t m, size_t n, size_t k);

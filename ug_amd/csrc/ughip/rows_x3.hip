@@ -8,11 +8,11 @@
 //               (88 tiles x 2) or need a second round (88 x 3).  A workgroup whose units cross into the next column tile stores one
 //               slab of partial sums per tile it touches; slab s of a tile is the s-th workgroup that touches it, and the fold
 //               adds them in that order, so the result does not depend on timing.
-//   waves 0-3 : the products.  Wave w owns rows 32 w .. 32 w + 31 and all 128 columns: 16 accumulators.  The matrix tile's
+//   waves 0-3 : the products.  Wave w owns rows 32 w .. 32 w + 31 (BM 64: 16 w .. 16 w + 15) and all 128 columns: 16 accumulators (8).  The matrix tile's
 //               fragments (16 x 128 bits) are read from LDS once per unit and meet the three planes in turn; the row fragments
 //               come from LDS plane by plane.  These waves also send the matrix tiles on their way: global -> LDS
 //               (global_load_lds_dwordx4), three units ahead in a ring of four stages (BM 64: five in six), four instructions per wave and unit.
-//   waves 4-7 : the rows.  Each loads its part of the 128 x 64 f32 tile of the next unit but one (16-byte loads, rows 256 bytes
+//   waves 4-7 : the rows.  Each loads its part of the BM x 64 f32 tile of the next unit but one (16-byte loads, rows 256 bytes
 //               apart in memory: whole lines), splits every element into hi + mid + lo (v_cvt_pk_bf16_f32 rounds to nearest
 //               even; the remainders are exact) and writes the three planes into one of two LDS stages in the layout the
 //               fragment reads want.  Their VALU work shares the SIMDs with the MFMAs of waves 0-3, which leave the issue
@@ -70,7 +70,6 @@ constexpr int BN = 128, MOST = 128;
 constexpr int stages(int bm) { return bm == 64 ? 6 : 4; }  // of the matrix ring
 constexpr int B_STAGE = BN * 64 * 2;
 constexpr int lds_total(int bm) { return stages(bm) * B_STAGE + 2 * 3 * bm * 64 * 2; }
-inline int tile_rows(size_t m) { return m <= 64 ? 64 : 128; }
 
 // x = hi + mid + lo, every term a bf16 (round to nearest even of what the terms before left: the remainders are exact, so
 // |x - (hi + mid + lo)| <= 2^-25 |x|).  An infinity (given, or reached when |x| rounds up past the largest bf16) is all in hi: its
@@ -121,7 +120,7 @@ __global__ void __launch_bounds__(512) rows_x3_kernel(const float* __restrict__ 
     };
     auto convert = [&](int set, int t) __attribute__((always_inline)) {
       char __attribute__((address_space(3)))* dst = (char __attribute__((address_space(3)))*)lds + B_BYTES + (t & 1) * A_STAGE;
-      // an element that is, or rounds to, an infinity is rare: one test for the wave's 2048 elements chooses the code that looks for them
+      // an element that is, or rounds to, an infinity is rare: one test for the wave's 2048 elements (BM 64: 1024) chooses the code that looks for them
       float big = 0.f;
 #pragma unroll
       for (int i = 0; i < NQ; ++i) big = fmaxf(big, fmaxf(fmaxf(fabsf(raw[set][i][0]), fabsf(raw[set][i][1])), fmaxf(fabsf(raw[set][i][2]), fabsf(raw[set][i][3]))));
@@ -336,13 +335,15 @@ bool rows_x3_supported(const void* x, const void* w, const void* c, const void* 
 }
 
 // Units per workgroup: every CU busy in one round, and past that as few slabs as the units' time allows -- a unit costs a
-// microsecond of a workgroup's time, a slab (64 KiB written, read once by the fold) about half a microsecond of everybody's.
+// microsecond of a workgroup's time, a slab (64 KiB written, read once by the fold) a thirtieth of one of everybody's.  Half as large a
+// slab, of tiles of 64 rows, goes by the same price: 18 products of 50 and 64 rows had the fastest number of units so, or one within 0.2 us of it (50 rows of 2048 x 5632 on 6 / 8 / 12 units 15.3 / 15.5 / 17.3 us,
+// of 2560 x 2048 on 3 / 4 / 6 12.5 / 11.3 / 12.1).
 RowsX3Plan rows_x3_plan(size_t m, size_t n, size_t k, int forced_units, int num_cus) {
   RowsX3Plan pl;
   const int KT = (int)(k / 64), tiles = (int)((n + BN - 1) / BN), total = tiles * KT;
   const int cus = num_cus > 0 ? num_cus : 256;
   auto fill = [&](int U, RowsX3Plan* out) {
-    out->units = U, out->groups = (total + U - 1) / U, out->max_slabs = 0;
+    out->tile_rows = m <= 64 ? 64 : 128, out->units = U, out->groups = (total + U - 1) / U, out->max_slabs = 0;
     int segments = 0;
     for (int g = 0; g < out->groups; ++g) segments += (std::min(g * U + U, total) - 1) / KT - (g * U) / KT + 1;
     for (int T = 0; T < tiles; ++T) out->max_slabs = std::max(out->max_slabs, (T * KT + KT - 1) / U - (T * KT) / U + 1);
@@ -366,7 +367,7 @@ RowsX3Plan rows_x3_plan(size_t m, size_t n, size_t k, int forced_units, int num_
 }
 
 void rows_x3_name(const RowsX3Plan& pl, GemmEpilogue::Kind kind, char* out, size_t out_len) {
-  snprintf(out, out_len, "rows_x3<128x128,3 terms split in the kernel,%d units x %d workgroups,%d slabs%s>", pl.units, pl.groups, pl.max_slabs,
+  snprintf(out, out_len, "rows_x3<%dx128,3 terms split in the kernel,%d units x %d workgroups,%d slabs%s>", pl.tile_rows, pl.units, pl.groups, pl.max_slabs,
            kind == GemmEpilogue::SWIGLU ? ",swiglu fold" : kind == GemmEpilogue::ADD ? ",+residual in the fold" : pl.max_slabs == 1 ? ",no fold" : ",fold");
 }
 
@@ -384,8 +385,9 @@ hipError_t rows_x3_launch(hipStream_t stream, const float* x, const void* w, flo
   const int KT = (int)(k / 64), tiles = (int)((n + BN - 1) / BN), total = tiles * KT;
   // one slab per tile and nothing for the fold to do: the slab is the result
   const bool direct = pl.max_slabs == 1 && kind == GemmEpilogue::NONE;
-  auto kernel = tile_rows(m) == 64 ? rows_x3_kernel<64> : rows_x3_kernel<128>;
-  kernel<<<dim3((unsigned)pl.groups), dim3(512), lds_total(tile_rows(m)), stream>>>(x, static_cast<const uint16_t*>(w), direct ? c : ws, (int)m, (int)n, (int)k, KT, pl.units, total);
+  if (m > (size_t)pl.tile_rows) return hipErrorInvalidValue;
+  auto kernel = pl.tile_rows == 64 ? rows_x3_kernel<64> : rows_x3_kernel<128>;
+  kernel<<<dim3((unsigned)pl.groups), dim3(512), lds_total(pl.tile_rows), stream>>>(x, static_cast<const uint16_t*>(w), direct ? c : ws, (int)m, (int)n, (int)k, KT, pl.units, total);
   if (hipError_t e = hipGetLastError()) return e;
   if (direct) {
     char name[160];
