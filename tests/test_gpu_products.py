@@ -154,8 +154,8 @@ def test_products_of_any_size(hip, bmnk, dtype, rhs_nk, lhs_mk):
 
 
 # products of one tile, of several, of tiles of both sizes, in batches; f32 on both sides of one step by element
-@pytest.mark.parametrize("b, m, n, k, dtype, kernel", [(300, 33, 17, 40, "f32", "gemm_any<f32>"), (17, 9, 70, 65, "f16", "gemm_any<f16>"), (9, 65, 129, 130, "bf16", "gemm_any<bf16>"),
-                                                       (3, 1155, 1155, 130, "bf16", "gemm_any<bf16,128x128>"), (5, 70, 130, 16, "f32", "gemm_any<f32,by element>"),
+@pytest.mark.parametrize("b, m, n, k, dtype, kernel", [(300, 33, 17, 40, "f32", "gemm_any<f32>"), (17, 9, 70, 65, "f16", "gemm_any<f16>"), (9, 65, 129, 130, "bf16", "gemm_any<bf16,words>"),
+                                                       (3, 1155, 1155, 130, "bf16", "gemm_any<bf16,128x128,words>"), (5, 70, 130, 16, "f32", "gemm_any<f32,by element>"),
                                                        (5, 70, 131, 17, "f32", "gemm_any<f32>"), (2, 20, 7, 100, "f16", "gemm_any<f16,by element>")])
 @pytest.mark.parametrize("shared", [False, True], ids=["batched", "one lhs"])
 def test_batches_of_products_of_any_size(hip, b, m, n, k, dtype, kernel, shared):
@@ -200,7 +200,8 @@ def test_rows_that_start_inside_a_word(hip, b, m, n, k, dtype, rhs_nk):
         sw, pw = placed(lines, lines.shape[2] + 2 + (lines.shape[2] + odd_w) % 2, offset)
         dst = hip.allocate_uninit(dt, b * m * n)
         hip.matmul(dst, sa, sw, (b, m, n, k), ((b, m, k), (m * pa, pa, 1), offset), ((b, k, n), (lines.shape[1] * pw, 1, pw) if rhs_nk else (k * pw, pw, 1), offset))
-        assert ug_amd.last_kernel().startswith("gemm_any<"), ug_amd.last_kernel()
+        name = ug_amd.last_kernel()
+        assert name.startswith("gemm_any<") and name.endswith(",words>") == bool(odd_a and odd_w or offset), name
         return dst.to_vec().view(np.uint16)
 
     print("inside a word", dtype, b, m, n, k, rhs_nk, flush=True)

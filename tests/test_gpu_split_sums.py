@@ -26,7 +26,7 @@ def test_split_sums(hip, bmnk, dtype, rhs_nk, lhs_mk):
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_three_and_four_tiles_to_a_cu(hip, bmnk, large, dtype):
     products.test_products_of_any_size(hip, bmnk, dtype, True, True)
-    assert ug_amd.last_kernel() == f"gemm_any<{dtype}{',128x128' if large else ''}>"
+    assert ug_amd.last_kernel() == f"gemm_any<{dtype}{',128x128' if large else ''},words>"
 
 
 @pytest.mark.parametrize("dtype", [ug_amd.F32, ug_amd.BF16], ids=["f32", "bf16"])

@@ -373,11 +373,11 @@ def test_plans_of_products_of_any_size():
     F, H, B = ug_amd.F32, ug_amd.F16, ug_amd.BF16
     want = {
         (F, F, 300, 33, 17, 129, 0): "gemm_any<f32>",
-        (H, H, 300, 33, 17, 129, 0): "gemm_any<f16>",                  # 300 tiles of 128 x 128, nine tenths of them padding
+        (H, H, 300, 33, 17, 129, 0): "gemm_any<f16,words>",            # rows of both operands at odd elements; 300 tiles of 128 x 128, nine tenths of them padding
         (H, H, 100, 9, 700, 333, 0): "gemm_any<f16>",
-        (H, H, 1, 2001, 2001, 1001, 0): "gemm_any<f16,128x128>",
+        (H, H, 1, 2001, 2001, 1001, 0): "gemm_any<f16,128x128,words>",
         (B, B, 200, 70, 130, 333, 0): "gemm_any<bf16,128x128>",        # a quarter padding
-        (B, B, 1, 2001, 2001, 65, 0): "gemm_any<bf16,128x128>",
+        (B, B, 1, 2001, 2001, 65, 0): "gemm_any<bf16,128x128,words>",
         (B, B, 1, 2001, 2001, 63, 0): "gemm_any<bf16,128x128>",        # one full round
         (B, B, 1, 3001, 3001, 63, 0): "gemm_any<bf16>",
         (F, F, 1, 2001, 2001, 1001, 0): "gemm_any<f32>",

@@ -126,6 +126,7 @@ struct RaggedPlan {
   static constexpr size_t MAX_WS = (size_t)32 << 20;
 };
 bool gemm_ragged_takes(int dtype, const MMArgs& p, size_t batch);  // whether that plan has a tile
+bool gemm_ragged_words(int dtype, const MMArgs& p, size_t batch, const RaggedPlan& plan);  // whether that plan's kernel loads rows that start inside a word by words
 RaggedPlan gemm_ragged_plan(int dtype, const MMArgs& p, size_t batch);
 hipError_t gemm_ragged_launch(hipStream_t stream, int dtype, const MMArgs& p, size_t batch, const RaggedPlan& plan, float* workspace);
 

@@ -444,15 +444,19 @@ __global__ void __launch_bounds__(256) gemm_ragged_fold(const float* __restrict_
 bool odd_rows(const void* base, long long rows, long long pitch, size_t batch, long long batch_stride) {
   return (reinterpret_cast<uintptr_t>(base) & 2) || (rows > 1 && (pitch & 1)) || (batch > 1 && (batch_stride & 1));
 }
+// ODD where both operands start anywhere and the address unit is what a step waits for; with one of them aligned putting chunks together takes as long as it saves.  us before /
+// so: f16 1000 x 776 x 2057 [n, k]-major 15.3 / 13.3, 12 of 17 x 1728 x 3185 47.3 / 35.5, bf16 2692 x 1660 x 3123 (128 x 128) 74.0 / 64.7, [k, n]-major 1000 x 777 x 1531 12.6 / 11.9;
+// x 776 x 2057, the lhs alone, 12.1 / 12.9 from L2, 13.3 / 13.2 past it.
+bool by_words(const MMArgs& p, size_t batch) {
+  const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
+  return (ak || bk) && odd_rows(p.a, ak ? p.M : p.K, ak ? p.a_rs : p.a_cs, batch, p.a_bs) && odd_rows(p.b, bk ? p.N : p.K, bk ? p.b_cs : p.b_rs, batch, p.b_bs);
+}
 // BT 32: gemm_ragged32
 template <typename T, int BT, Form FORM, bool ODD = false>
 hipError_t launch(hipStream_t stream, const MMArgs& p, size_t batch, int nsplit, float* ws) {
   const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
-  // ODD where both operands start anywhere and the address unit is what a step waits for; with one of them aligned putting chunks together takes as long as it saves.  us before /
-  // so: f16 1000 x 776 x 2057 [n, k]-major 15.3 / 13.3, 12 of 17 x 1728 x 3185 47.3 / 35.5, bf16 2692 x 1660 x 3123 (128 x 128) 74.0 / 64.7, [k, n]-major 1000 x 777 x 1531 12.6 / 11.9;
-  // x 776 x 2057, the lhs alone, 12.1 / 12.9 from L2, 13.3 / 13.2 past it.
   if constexpr (sizeof(T) == 2 && FORM != ONE && !ODD)
-    if ((ak || bk) && odd_rows(p.a, ak ? p.M : p.K, ak ? p.a_rs : p.a_cs, batch, p.a_bs) && odd_rows(p.b, bk ? p.N : p.K, bk ? p.b_cs : p.b_rs, batch, p.b_bs))
+    if (by_words(p, batch))
       return launch<T, BT, FORM, true>(stream, p, batch, nsplit, ws);
   const int tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BT - 1) / BT, ke = 128 / (int)sizeof(T), steps = (p.K + ke - 1) / ke;
   const int parts = BT == 32 ? 4 * nsplit : nsplit, per = (steps + parts - 1) / parts;
@@ -523,6 +527,8 @@ static double few_tiles_us(int dtype, int tile, int steps, size_t tiles, int ns,
   else us += per * (share > 1 ? (f32 ? 1.1 : 0.75) : f32 ? 0.56 + 0.06 * share : 0.25 + 0.16 * share);
   return ns == 1 ? us : std::max(8.8, us + 2.5 + 0.1 * ns + (double)(ns + 1) * slab_bytes / 5e6);
 }
+
+bool gemm_ragged_words(int dtype, const MMArgs& p, size_t batch, const RaggedPlan& plan) { return plan.tile && dtype != UGHIP_F32 && p.K > 64 && by_words(p, batch); }
 
 bool gemm_ragged_takes(int dtype, const MMArgs& p, size_t batch) { return supported(p, batch) && !(dtype == UGHIP_F32 && p.K <= 16); }
 

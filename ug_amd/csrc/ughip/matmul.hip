@@ -517,11 +517,12 @@ static Route matmul_route(int dtype, bool mixed, const MMArgs& p, size_t b, size
   return gemm_tiled_supported(dtype, p, b, mixed) && !(f32 && !mixed && better_in_small_tiles(p, b)) ? ROUTE_TILED : ROUTE_ANY;
 }
 
-// The kernels behind ROUTE_ANY, in names: gemm_ragged's tiles and splits of K (gemm_ragged_plan; the smaller two are not named), and the ones that go by element.
+// The kernels behind ROUTE_ANY, in names: gemm_ragged's tiles and splits of K (gemm_ragged_plan; the smaller two are not named), rows that start inside a word loaded by words, and the ones that go by element.
 template <typename F>
-static void any_name(const char* tn, const RaggedPlan& pl, F&& print) {
-  if (pl.nsplit > 1) print("gemm_any<%s,splitK=%d>", tn, pl.nsplit);
-  else print(pl.tile == 128 ? "gemm_any<%s,128x128>" : pl.tile ? "gemm_any<%s>" : "gemm_any<%s,by element>", tn);
+static void any_name(const char* tn, const RaggedPlan& pl, bool words, F&& print) {
+  const char* by = words ? ",words" : "";
+  if (pl.nsplit > 1) print("gemm_any<%s,splitK=%d%s>", tn, pl.nsplit, by);
+  else print(pl.tile == 128 ? "gemm_any<%s,128x128%s>" : pl.tile ? "gemm_any<%s%s>" : "gemm_any<%s,by element%s>", tn, by);
 }
 
 static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* lhs, const ughip_slice* rhs, size_t b, size_t m, size_t n, size_t k,
@@ -637,7 +638,7 @@ static int matmul_impl(ughip_device* dev, ughip_slice* dst, const ughip_slice* l
       ws = no_memory ? nullptr : static_cast<float*>(dev->gemm_ws);
     }
     if (!ws) pl.nsplit = 1;  // no memory for the slabs: whole
-    any_name(tn, pl, [](auto... text) { note_kernel(text...); });
+    any_name(tn, pl, gemm_ragged_words(dst->dtype, p, b, pl), [](auto... text) { note_kernel(text...); });
     if (pl.tile) UGHIP_HIPCHK(gemm_ragged_launch(st, dst->dtype, p, b, pl, ws));
     else if (f32) gemm_f32_any<<<grid, 256, 0, st>>>(p);
     else if (dst->dtype == UGHIP_F16) gemm_half_any<_Float16><<<grid, 256, 0, st>>>(p);
@@ -1044,7 +1045,7 @@ extern "C" int ughip_matmul_plan(int dtype, int rhs_dtype, size_t b, size_t m, s
       break;
     }
     case ROUTE_TILED: gemm_tiled_name(dtype, p, b, mixed, nullptr, buf, buf_len); break;
-    default: any_name(tn, gemm_ragged_plan(dtype, p, b), [&](auto... text) { snprintf(buf, buf_len, text...); }); break;
+    default: any_name(tn, gemm_ragged_plan(dtype, p, b), gemm_ragged_words(dtype, p, b, gemm_ragged_plan(dtype, p, b)), [&](auto... text) { snprintf(buf, buf_len, text...); }); break;
   }
   return UGHIP_OK;
 }
