@@ -125,3 +125,28 @@ def test_latent_merge_leaves_no_cu_idle_and_makes_no_more_than_there_is(tmp_path
     asked = "\n".join(" ".join(map(str, key)) for key in MERGED)
     out = subprocess.run([str(tmp_path / "merged")], input=asked, capture_output=True, text=True, timeout=60)
     assert out.returncode == 0 and dict(zip(MERGED, map(int, out.stdout.split()))) == MERGED
+
+
+# (m, n, k) -> us that an f32 product with a lookup takes on the tile it has, as measured; n 5632 and 1024 rows are 352 tiles of 128 x 128, where 64 x 64 would be priced lower
+LOOKUPS = {(1024, 5632, 512): 103.4, (1024, 5632, 128): 50.0, (2000, 5632, 128): 74.8, (100, 64, 512): 17.1, (200, 1024, 512): 17.4}
+LOOKUPS_PROGRAM = r"""
+#include "rows_prices.h"
+
+#include <cstdio>
+
+int main() {
+  int m, n, k;
+  while (scanf("%d %d %d", &m, &n, &k) == 3) printf("%f\n", ughip::f32_lookup_us(m, n, k));
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
+def test_f32_lookups_are_priced_on_the_tile_they_have(tmp_path):
+    (tmp_path / "main.cpp").write_text(LOOKUPS_PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I" + os.path.join(ROOT, "ug_amd", "csrc", "ughip"), str(tmp_path / "main.cpp"), "-o", str(tmp_path / "lookups")], check=True)
+    asked = "\n".join(" ".join(map(str, key)) for key in LOOKUPS)
+    out = subprocess.run([str(tmp_path / "lookups")], input=asked, capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0
+    for key, us in zip(LOOKUPS, map(float, out.stdout.split())):
+        assert abs(us - LOOKUPS[key]) <= 0.2 * LOOKUPS[key], (key, us)  # a price: what the formula leaves out is within a fifth

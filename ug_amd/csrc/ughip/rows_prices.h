@@ -41,6 +41,15 @@ inline int f32_rows_tile(int m, int n, int k, int groups, bool gated, double* pr
   return best;
 }
 
+// The tile of what is not gated where f32_rows_tile does not choose it, in bf16 and with a lookup.  rows: of a group, or m
+inline int rows_tile(int m, int n, int rows) { return rows > 64 && (long long)((m + 127) / 128) * ((n + 127) / 128) >= 192 ? 22 : 11; }
+// f32 products with a lookup on that tile: what a product without one takes there, and the table's scattered elements, by rounds of the large tile (us, k 128: 1024 rows of n 5632 50, 2000 75; 100 of n 64, k 512 17.1, without a lookup 14.6)
+inline double f32_lookup_us(int m, int n, int k) {
+  const int tile = rows_tile(m, n, m), t = tile == 22 ? 128 : 64;
+  const double rounds = std::max(1.0, std::ceil((double)((m + t - 1) / t) * ((n + t - 1) / t) / 256));
+  return 4.0 + rounds * k / 2048.0 * (tile == 22 ? 144.0 : 45.5) + (tile == 22 ? 14.0 * rounds : 2.5);
+}
+
 // f32 rows against an f32 matrix: gemm_tiled's tiles, at their price (negative: they do not take it) and with `bytes` for what lies between them and the fold, or rows_product's.  2 us are the tiles' longer way in.
 inline bool f32_rows_on_tiles(double tiles_us, double rows_product_us, size_t bytes) { return tiles_us >= 0 && tiles_us + 2.0 < 0.97 * rows_product_us && bytes <= ROWS_BLOCK_MOST; }
 
@@ -49,8 +58,7 @@ inline bool f32_rows_on_tiles(double tiles_us, double rows_product_us, size_t by
 // in the mean square.
 inline double rounded_on_the_way_us(int m, int n, int k, int groups, bool gated, bool lookup) {
   const int rows = groups ? (m + groups - 1) / groups : m, met = groups ? std::min(groups, m) : 1;  // matrices that rows meet
-  const long long big = (long long)((m + 127) / 128) * ((n + 127) / 128);
-  const int tile = gated ? (rows > 64 ? 22 : 12) : rows > 64 && big >= 192 ? 22 : 11, bm = tile == 22 ? 128 : 64, cols = (tile == 11 ? 64 : 128) / (gated ? 2 : 1);
+  const int tile = gated ? (rows > 64 ? 22 : 12) : rows_tile(m, n, rows), bm = tile == 22 ? 128 : 64, cols = (tile == 11 ? 64 : 128) / (gated ? 2 : 1);
   static const struct {
     double fixed, height, step, past_step, past, mb;  // height: of a tile's, that rows fill; past: for every round of 256 tiles behind the first; mb: of the matrices
   } prices[] = {{2.89, 1.39, 0.775, 0.629, 1.9, 0.0}, {2.37, 2.67, 0.578, 0.168, 1.1, 0.059}, {5.69, 0.99, 0.917, 0.706, 3.2, 0.012}};

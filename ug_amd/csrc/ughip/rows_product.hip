@@ -317,8 +317,7 @@ hipError_t launch_act(hipStream_t st, const ProductArgs& a, bool vec) {
   if constexpr (GATED) {  // a tile's columns come in gate / up pairs
     return rows > 64 ? launch_tile<CT, XT, WT, 2, 2, ACT>(st, a, vec) : launch_tile<CT, XT, WT, 1, 2, ACT>(st, a, vec);
   } else {
-    const long long big = (long long)((a.m + 127) / 128) * ((a.n + 127) / 128);
-    if (rows > 64 && big >= 192) return launch_tile<CT, XT, WT, 2, 2, ACT>(st, a, vec);
+    if (rows_tile(a.m, a.n, rows) == 22) return launch_tile<CT, XT, WT, 2, 2, ACT>(st, a, vec);
     return launch_tile<CT, XT, WT, 1, 1, ACT>(st, a, vec);
   }
 }
@@ -362,7 +361,8 @@ int tiled_rows(ughip_device* dev, const ProductArgs& a, int act, bool* done) {
   if (a.groups || a.m < 2 || p.N % 8 || a.n % 4 || (long long)a.m * p.N % 8) return UGHIP_OK;
   const double us = gemm_tiled_cost_us(UGHIP_F32, p, 1, fold);
   double here = 0;
-  f32_rows_tile(a.m, a.n, a.k, 0, gated, &here);
+  if (lookup) here = f32_lookup_us(a.m, a.n, a.k);
+  else f32_rows_tile(a.m, a.n, a.k, 0, gated, &here);
   GemmEpilogue epi{GemmEpilogue::ROWS, nullptr};
   const GemmEpilogue* e = fold ? &epi : nullptr;
   const size_t bytes = us < 0 ? 0 : gemm_tiled_workspace_bytes(UGHIP_F32, p, 1, e);
