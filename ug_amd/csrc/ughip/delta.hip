@@ -48,14 +48,6 @@ __device__ __forceinline__ void mfma16x16_each(const f32x4_t (&x)[N], const f32x
 }
 // Where element (row, k) of a left operand lies in its tile, and a tile's lane.
 __device__ __forceinline__ int left_at(int row, int k) { return ((k >> 2) * 16 + row) * 4 + (k & 3); }
-// A result (lane l: column l % 16, rows 4 (l / 16) .. + 3) as a left operand's tile: a quad of lanes turns its 4 x 4 elements, and what was four stores to 16 places each is one of 1 KB in a row.
-__device__ __forceinline__ void store_left(float* tile, const f32x4_t& v, int lane) {
-  const bool odd = lane & 1, high = lane & 2;
-  const float a = dpp_move<0xB1>(odd ? v.x : v.y), b = dpp_move<0xB1>(odd ? v.z : v.w);  // quad_perm: lane ^ 1
-  const f32x4_t p = {odd ? a : v.x, odd ? v.y : a, odd ? b : v.z, odd ? v.w : b};
-  const float c = dpp_move<0x4E>(high ? p.x : p.z), d = dpp_move<0x4E>(high ? p.y : p.w);  // lane ^ 2
-  *reinterpret_cast<f32x4_t*>(tile + ((lane >> 2 & 3) * 16 + (lane >> 4) * 4 + (lane & 3)) * 4) = f32x4_t{high ? c : p.x, high ? d : p.y, high ? p.z : c, high ? p.w : d};
-}
 __device__ __forceinline__ float* tile_at(float* tiles, size_t tile, int lane) { return tiles + (tile * 64 + lane) * 4; }
 __device__ __forceinline__ f32x4_t tile_of(const float* tiles, size_t tile, int lane) { return *reinterpret_cast<const f32x4_t*>(tiles + (tile * 64 + lane) * 4); }
 __device__ __forceinline__ float exact_sigmoid(float z) { return 1.f / (1.f + expf(-z)); }
@@ -111,9 +103,8 @@ constexpr int prepare_threads() {
   return C == 64 ? 512 : 256;
 }
 // PAIR: two workgroups to a CU.  The queries stay in memory, read where they are used, times their rows' factors (77 KB are left in LDS of 64 rows of
-// 128 channels), and A is read again for every tile of the solve; bound by vector instructions and by what waits for memory between barriers.  2048 positions of 16 heads: 69 us with
-// one workgroup to a CU, 62.6 us so, 59.9 with queries asked for ahead of their use and left operands stored in rows (10 of the 39 us of a workgroup are the
-// decays' logarithms).  Up to one workgroup per CU the queries lie in LDS and A in registers; all three launches of the rows with it, against
+// 128 channels), and A is read again for every tile of the solve; bound by vector instructions.  2048 positions of 16 heads: 69 us with
+// one workgroup to a CU, 62 us so.  Up to one workgroup per CU the queries lie in LDS and A in registers; all three launches of the rows with it, against
 // PAIR there: 989 positions of 4 heads 86.8 and 90.0 us, 898 of 16 (100 channels) 71.9 and 74.8, 3 of 16 (vdim 64) 22.2 and 23.0.
 template <int C, bool VEC, bool PAIR>
 __global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_prepare_kernel(DeltaArgs a) {
@@ -131,17 +122,6 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_
   const int d4 = dp / 4;
   const float neg = -expf(a.a_log[h]) * LOG2E;
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  constexpr int TURNS = C / (4 * NW);  // rows of a lane where rows become unit vectors
-  f32x4_t asked[PAIR ? TURNS : 1][2];  // PAIR: its pieces of these queries (128 channels at most)
-  if constexpr (PAIR) {
-#pragma unroll
-    for (int n = 0; n < TURNS; ++n)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int c = j * 4 + 64 * u;
-        asked[n][u] = c < d ? four<VEC>(a.qkv + (size_t)(row0 + min((n * NW + wave) * 4 + kg, rows - 1)) * a.qkv_stride + (size_t)g * d + c, d - c) : zero;
-      }
-  }
   constexpr int AT_ONCE = 4;  // pieces of a thread on their way together: the decays' logarithms are long, and a load behind them would come late
   for (int e0 = threadIdx.x; e0 < C * d4; e0 += AT_ONCE * NT) {
     f32x4_t k[AT_ONCE], l[AT_ONCE], bias[AT_ONCE], q[PAIR ? 1 : AT_ONCE];
@@ -179,13 +159,11 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_
   };
   // unit vectors: 16 lanes per row
   const float q_scale = 1.f / sqrtf((float)d);
-#pragma unroll
-  for (int n = 0; n < TURNS; ++n) {
-    const int r = (n * NW + wave) * 4 + kg;
+  for (int r = wave * 4 + kg; r < C; r += 4 * NW) {
     float* row = K + r * ds;
     float ss = 0.f, sq = 0.f;
     for (int c = j * 4; c < dp; c += 64) {
-      const f32x4_t q = PAIR ? asked[n][c >= 64 ? 1 : 0] : query(r, c), v = *reinterpret_cast<const f32x4_t*>(row + c);
+      const f32x4_t q = query(r, c), v = *reinterpret_cast<const f32x4_t*>(row + c);
       ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
       sq += q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
     }
@@ -221,25 +199,10 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_
       for (J = n - NB; J >= I; ++I) J -= I;
     }
     const float uq = PAIR ? unit[16 * I + j] : 1.f;
-    // PAIR: queries come from memory, an iteration ahead (waited for where they are used they were half of this phase's time)
-    f32x4_t next[2];
-    auto ask = [&](int c) {
-      if constexpr (PAIR) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) next[u] = query(16 * I + j, min(c, dp - 32 + 4 * kg) + 16 * u);
-      }
-    };
-    auto asked_or = [&](int u, int c) {
-      if constexpr (PAIR) return next[u] * uq;
-      else return query(16 * I + j, c);
-    };
-    ask(4 * kg);
     if (J < I) {
       f32x4_t acc[4] = {zero, zero, zero, zero};
       for (int c = 4 * kg; c < dp; c += 32) {
         f32x4_t x[4], y[4];
-        const f32x4_t q[2] = {asked_or(0, c), asked_or(1, c + 16)};
-        ask(c + 32);
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const int cc = c + 16 * u;  // dp is a multiple of 64
@@ -248,13 +211,17 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_
           for (int M = J + 1; M < I; ++M) rest += row4(B, 16 * M + 15, cc);
           y[2 * u] = y[2 * u + 1] = row4(K, 16 * J + j, cc) * exp2_4(rest);
           x[2 * u] = row4(K, 16 * I + j, cc) * left;
-          x[2 * u + 1] = q[u] * left;
+          x[2 * u + 1] = unit_query(16 * I + j, cc, uq) * left;
         }
         mfma16x16_each(x, y, acc);
       }
       const f32x4_t ak = acc[0] + acc[2], aq = acc[1] + acc[3];
-      store_left(tile_a(I, J), ak * *reinterpret_cast<const f32x4_t*>(beta + 16 * I + 4 * kg), lane);
-      store_left(P + (I * NB + J) * 256, aq, lane);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 16 * I + 4 * kg + e;
+        tile_a(I, J)[left_at(4 * kg + e, j)] = ak[e] * beta[i];
+        P[(I * NB + J) * 256 + left_at(4 * kg + e, j)] = aq[e];
+      }
       continue;
     }
 
@@ -265,27 +232,23 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_
       f32x4_t acc[4] = {zero, zero, zero, zero};
       for (int c = 4 * kg; c < dp; c += 32) {
         f32x4_t x[4], y[4];
-        const f32x4_t q[2] = {asked_or(0, c), asked_or(1, c + 16)};
-        ask(c + 32);
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const int cc = c + 16 * u;
           const f32x4_t l = row4(B, 16 * I + j, cc), k = row4(K, 16 * I + j, cc), left = exp2_4(l);
           y[2 * u] = y[2 * u + 1] = k * exp2_4(-l);
           x[2 * u] = k * left;
-          x[2 * u + 1] = q[u] * left;
+          x[2 * u + 1] = unit_query(16 * I + j, cc, uq) * left;
         }
         mfma16x16_each(x, y, acc);
       }
-      f32x4_t ak = acc[0] + acc[2], aq = acc[1] + acc[3];
+      const f32x4_t ak = acc[0] + acc[2], aq = acc[1] + acc[3];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int i = 4 * kg + e;
-        ak[e] = j < i ? ak[e] * beta[16 * I + i] : 0.f;
-        aq[e] = j <= i ? aq[e] : 0.f;
+        const int i = 4 * kg + e, row = 16 * I + i;
+        tile_a(I, I)[left_at(i, j)] = j < i ? ak[e] * beta[row] : 0.f;
+        P[(I * NB + I) * 256 + left_at(i, j)] = j <= i ? aq[e] : 0.f;
       }
-      store_left(tile_a(I, I), ak, lane);
-      store_left(P + (I * NB + I) * 256, aq, lane);
       continue;
     }
     // row 16 I + j against rows 16 I + 4 kg ..
@@ -397,7 +360,8 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_
         for (int J = 0; J < I; ++J) x[I] -= acc[J];
         x[I] = mfma16x16(mi[I], x[I], zero);
         if (tile < kt) {
-          store_left(W + (I * kt + tile) * 256, x[I], lane);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) W[(I * kt + tile) * 256 + left_at(4 * kg + e, j)] = x[I][e];
         } else {
           *reinterpret_cast<f32x4_t*>(tile_at(V, (tile - kt) * NB + I, lane)) = x[I];
         }
@@ -406,27 +370,11 @@ __global__ void __launch_bounds__((prepare_threads<C>()), (PAIR ? 4 : 1)) delta_
   }
   // G q, and G_C / G k
   float* QG = a.qg + at * C * dp;
-  for (int e0 = threadIdx.x; e0 < C * d4; e0 += 2 * NT) {
-    f32x4_t q[2];
-    auto at_of = [&](int e, int& r, int& c) {
-      const int tile = e / 64;
-      r = tile / (dp / 16) * 16 + (e & 15), c = tile % (dp / 16) * 16 + (e >> 4 & 3) * 4;
-    };
-    int r, c;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {  // (PAIR: both on their way together)
-      at_of(min(e0 + u * NT, C * d4 - 1), r, c);
-      q[u] = unit_query(r, c, PAIR ? unit[r] : 1.f);
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int e = e0 + u * NT;
-      if (e >= C * d4) break;
-      at_of(e, r, c);
-      f32x4_t l = row4(B, r, c);
-      for (int M = 0; M < r / 16; ++M) l += row4(B, 16 * M + 15, c);
-      *reinterpret_cast<f32x4_t*>(QG + 4 * e) = q[u] * exp2_4(l);
-    }
+  for (int e = threadIdx.x; e < C * d4; e += NT) {
+    const int tile = e / 64, r = tile / (dp / 16) * 16 + (e & 15), c = tile % (dp / 16) * 16 + (e >> 4 & 3) * 4;
+    f32x4_t l = row4(B, r, c);
+    for (int M = 0; M < r / 16; ++M) l += row4(B, 16 * M + 15, c);
+    *reinterpret_cast<f32x4_t*>(QG + 4 * e) = unit_query(r, c, PAIR ? unit[r] : 1.f) * exp2_4(l);
   }
   float* KD = a.kd + at * C * dp;
   for (int e = threadIdx.x; e < C * d4; e += NT) {
