@@ -38,7 +38,9 @@ int ughip_gather_rows(ughip_device* dev, const ughip_slice* table, size_t table_
  *                       elements apart, by ughip_gemv_multi, which keeps those of an F32 matrix too.)
  * x, w and dst may each be F32 or BF16 (F32 only for UGHIP_PRODUCT_F32).  BF16 rows and matrices with k % 64 == 0 and 16-byte aligned
  * rows take the 16-bit kernels of ughip_matmul whose loads write LDS (256 x 256 tiles, or the ring of stages with smaller ones), the
- * rest one that takes any size (ughip_last_kernel names it).
+ * rest one that takes any size (ughip_last_kernel names it), or where that is expected to be faster: F32 rows of a bf16 product
+ * rounded by a launch ahead, for those kernels, and F32 products on the tiles of ughip_matmul.  Both take up to 128 MiB of the
+ * device's block for partial tiles, and go the other way where there is no memory for it.
  * `act`:
  *   UGHIP_ACT_NONE      dst[m, n] = y;
  *   UGHIP_ACT_SWIGLU    w is [2 n, k], gate rows then up rows (and bias 2 n values): dst = silu(y_gate) * y_up;

@@ -29,8 +29,7 @@ struct MMArgs {
 // stores only what exists.
 // rhs_bf16: the rhs is stored as bf16 under an f32 product ([n, k] row-major only) and widened on its way into LDS.
 bool gemm_tiled_supported(int dtype, const MMArgs& p, size_t batch, bool rhs_bf16 = false);
-// What the fold of the partial tiles does on its way out (f32 products only).  With an epilogue the product always goes
-// through the scratch block, even unsplit, and p.c is the epilogue's output.
+// What a product of rows leaves (ughip_product_rows), from its sums: bias, then nothing, the gated unit or the gated lookup.
 struct RowsOut {
   enum Form { PLAIN = 0, GATED = 1, LOOKUP = 2 } form = PLAIN;
   const float* bias = nullptr;  // N values
@@ -43,6 +42,8 @@ struct RowsOut {
   int table_rows = 0;
   bool table_bf16 = false;
 };
+// What the fold of the partial tiles does on its way out (f32 products only).  With an epilogue the product always goes
+// through the scratch block, even unsplit, and p.c is the epilogue's output.
 struct GemmEpilogue {
   enum Kind { NONE = 0, ADD = 1, SWIGLU = 2, ROWS = 3 } kind;
   const float* residual;  // ADD: c[m, n] = product + residual[m, n].  SWIGLU: c[m, n / 2] = silu(product[:, :n/2]) * product[:, n/2:]
