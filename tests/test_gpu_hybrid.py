@@ -283,8 +283,12 @@ def test_softplus_against_64_bits(gpu, lo, hi):
     sz, S = gpu.up(z), gpu.out(heads)
     gpu.call("ughip_ssm_rows", view(one, 0, heads + 2), view(sz, 0, heads), p(zero), p(zero), p(zero), p(S), Z(0), Z(1), Z(heads), Z(1), Z(1), Z(1), view(dst, 0, heads))
     want, e = np.logaddexp(0, z.astype(np.float64)), np.exp(np.float64(z))
+
+    def unit(v):  # in 64 bits: 32-bit units of such sums may be subnormal, which a process may have switched off
+        return 2.0 ** (np.floor(np.log2(v)) - 23)
+
     # two functions, each correct to 0.6 of a unit of its result (0.5 is what rounding leaves): the exponential's error, times the logarithm's slope, and the logarithm's own
-    bound = 0.6 * np.spacing(want.astype(np.float32)) + 0.6 * np.spacing(e.astype(np.float32)) / (1 + e)
+    bound = 0.6 * unit(want) + 0.6 * unit(e) / (1 + e)
     off = np.abs(get(dst, (heads,)) - want) / bound
     print("softplus", lo, hi, "of the bound", off.max())
     assert off.max() <= 1
